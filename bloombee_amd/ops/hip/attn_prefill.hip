@@ -3,217 +3,330 @@
 // Replaces the reference's mha_llama prefill path
 // (flexgen_utils/pytorch_backend.py:665-731), reading K/V directly from the
 // paged cache (new tokens are kv_write'n first, then attended — one code path
-// for first-prefill, multi-turn continuation and chunked prefill).
+// for first-prefill, multi-turn continuation, chunked prefill and the tree
+// steps of speculative decoding).
 //
-// Structure (v2): grid = (ceil(Tq/128), B*Hq); block = 512 (8 waves), each
-//   wave owns 16 q rows — 128 rows per workgroup halves the KV re-streaming
-//   of the 64-row v1 (every staged tile feeds twice the MFMA work).
-//   KV tiles of 32 keys stage through LDS
-//   (K row-major padded +16 B -> conflict-free 16-lane ds_read_b128;
-//    V transposed [d][key] at 80 B row stride — same property)
-//   QK^T and P.V on v_mfma_f32_16x16x32_bf16; online softmax in f32
-//   (exp2 domain, scale folded), P round-trips LDS to reach A-fragment
-//   layout.
+// Rows are (token, head of the group) pairs, so that a K/V tile serves all heads
+// that share it; a wave owns 32 rows, a workgroup 128. Tiles of 64 keys go to LDS
+// without passing through registers, double-buffered.
+//
+// Both products run transposed on v_mfma_f32_32x32x16_bf16: S^T = K Q^T, then
+// O^T = V^T P^T. The keys of a tile lie in LDS in an order (bits 2 and 3 of a key's
+// number swapped) in which the 16 scores a lane gets are the eight consecutive keys
+// it must hand to each of two value products: the weights never leave registers, a
+// row's maximum takes one exchange between the halves of a wave, and its sum none
+// until the end.
+//
+// The matrix cores bound long prompts (a tile is 32 products of 32 clocks a wave,
+// and its softmax about as many clocks on the vector units, which two waves a SIMD
+// overlap); the chain of tiles bounds short ones, so there the keys are split over
+// workgroups and a second kernel folds the parts.
+//
+// Measured, 32 heads on 8 of 128: four prompts of 4096 672 us (820 TF/s of the
+// visible half; 3808 us with 16-row tiles of one head each, staged through
+// registers, weights through LDS), one of 333 behind 1201 37 us (163), a tree of 25
+// behind 1500 20 us (168).
 //
 // Numerics: fp32 softmax/accum; bf16 operands — matches reference tolerance
 // class (test_block_exact_match.py atol 1e-4 forward on fp32 inputs).
 
 #include "common.h"
 
-
-static constexpr int KVBLK = 32;
-
+struct PrefillArgs {
+  const unsigned short* q;        // (b, token, head) at the strides below
+  const unsigned short* k_pages;  // (np, Hkv, P, D)
+  const unsigned short* v_pages;  // (np, Hkv, D, P)
+  const int* page_table;          // (B, maxp)
+  const int* q_start;             // (B,)
+  const float* alibi;             // (Hq,) slopes or null
+  const unsigned char* tree_mask; // (B, Tq, Tq) bool or null: spec-verify ancestor
+                                  // mask over the NEW tokens (ref
+                                  // backend.py:944-1047); committed positions
+                                  // < q_start stay fully visible
+  unsigned short* out;
+  float* pml;                     // splits: (n_split, B * Hkv, Tq * G, 2)
+  float* pacc;                    // (n_split, B * Hkv, Tq * G, D)
+  int B, Hkv, G, Tq, p_log2, maxp, window, n_split;
+  float scale;
+  long q_sb, q_st, q_sh, o_sb, o_st, o_sh;
+};
 
 template <int D>
-__global__ __launch_bounds__(512) void attn_prefill_kernel(
-    const unsigned short* __restrict__ q,        // (B, Hq, Tq, D)
-    const unsigned short* __restrict__ k_pages,  // (np, Hkv, P, D)
-    const unsigned short* __restrict__ v_pages,
-    const int* __restrict__ page_table,          // (B, maxp)
-    const int* __restrict__ q_start,             // (B,)
-    const float* __restrict__ alibi,             // (Hq,) slopes or null
-    const unsigned char* __restrict__ tree_mask, // (B, Tq, Tq) bool or null:
-                                                 // spec-verify ancestor mask
-                                                 // over the NEW tokens (ref
-                                                 // backend.py:944-1047);
-                                                 // committed positions < qs
-                                                 // stay fully visible
-    unsigned short* __restrict__ out,            // (B, Hq, Tq, D)
-    int B, int Hq, int G, int Tq, int P, int maxp, int window, float scale,
-    long q_sb, long q_st, long q_sh, long o_sb, long o_st, long o_sh) {
-  // q element (b, h, row, d) at b*q_sb + row*q_st + h*q_sh + d (same for
-  // out) — reads the q section of a fused (B, T, X, D) QKV output directly.
-  constexpr int KROW_B = D * 2 + 16;  // K LDS row stride (pad kills conflicts)
-  constexpr int VROW_B = KVBLK * 2 + 16;  // V^T LDS row stride (80 B)
-  constexpr int PROW_B = KVBLK * 2 + 16;
-  constexpr int NKK = D / 32;   // QK^T k-slices
-  constexpr int NDT = D / 16;   // PV d-tiles
+struct PrefillTile {
+  static constexpr int KT = 64, RC = D / 8;       // 16 B pieces of a key row
+  static constexpr int KB = KT * D * 2;           // bytes of K, and of V
+  static constexpr int BYTES = 2 * KB;
+  static constexpr int NI = KB / 1024 / 4;        // loads of a wave, K or V
+  // piece c of LDS row r lies at c ^ swizzle(r): 16 rows read at one piece cover
+  // all banks
+  DEVINL static int swizzle(int r) {
+    return RC >= 16 ? r & 15 : RC == 8 ? (r >> 1) & 7 : (r >> 2) & 3;
+  }
+};
 
-  __shared__ __attribute__((aligned(16))) unsigned char lds[
-      KVBLK * KROW_B + D * VROW_B + 8 * 16 * PROW_B];
-  unsigned short* k_lds = (unsigned short*)lds;
-  unsigned short* v_lds = (unsigned short*)(lds + KVBLK * KROW_B);
-  unsigned short* p_lds = (unsigned short*)(lds + KVBLK * KROW_B + D * VROW_B);
+// GENERAL: slopes, tree masks, scales that are not positive.
+template <int D, bool GENERAL>
+__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
+    PrefillArgs a) {
+  using Tile = PrefillTile<D>;
+  constexpr int KT = Tile::KT, RC = Tile::RC, NI = Tile::NI;
+  constexpr int NKK = D / 16, ND = D / 32;
+  static_assert(NI >= 1, "tile smaller than the workgroup");
+  extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
 
-  const int qtile = blockIdx.x;
-  const int bh = blockIdx.y;
-  const int b = bh / Hq, h = bh % Hq;
-  const int kvh = h / G;
-  const int qbase = qtile * 128;
+  // consecutive workgroups take different (sequence, head group, split) units, so
+  // that the row tiles of one unit meet in one XCD's L2 (units are a multiple of 8
+  // where the heads are); late rows see the most keys and go first
+  const int units = a.B * a.Hkv;
+  const int unit = blockIdx.x % units, split = blockIdx.x / units;
+  const int b = unit / a.Hkv, g = unit % a.Hkv;
+  const int G = a.G, R = a.Tq * G;
+  const int base = (int)(gridDim.y - 1 - blockIdx.y) * 128;
   const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = tid & (WAVE - 1);
-  const int li = lane & 15;      // fragment row/col index
-  const int hi = lane >> 4;      // fragment k-quad
-  const int qs = q_start[b];
-  const int ctx = qs + Tq;
-  const float sc2 = scale * LOG2E;
-  const float aslope = (alibi != nullptr) ? alibi[h] * LOG2E : 0.f;
+  const int li = lane & 31, hi = lane >> 5;
+  const int qs = a.q_start[b];
+  const bool tree = GENERAL && a.tree_mask != nullptr;
+  const int plog = a.p_log2, pmask = (1 << plog) - 1;
+  const int* table = a.page_table + (long)b * a.maxp;
 
-  // ---- Q fragments (load once): row = li, k = hi*8 + j (+32*kk) ----
-  const int my_qrow = min(qbase + wave * 16 + li, Tq - 1);
-  bf16x8 qfrag[NKK];
+  // this lane's row (column of S^T)
+  const int row = base + wave * 32 + li;
+  const int r = min(row, R - 1);
+  const int tok = r / G, head = g * G + r % G, qpos = qs + tok;
+  const unsigned short* qp =
+      a.q + (long)b * a.q_sb + (long)tok * a.q_st + (long)head * a.q_sh + hi * 8;
+  bf16x8 qf[NKK];
 #pragma unroll
-  for (int kk = 0; kk < NKK; ++kk) {
-    qfrag[kk] = as_bf16x8(*reinterpret_cast<const short8*>(
-        q + (long)b * q_sb + (long)my_qrow * q_st + (long)h * q_sh + hi * 8 + 32 * kk));
+  for (int kk = 0; kk < NKK; ++kk)
+    qf[kk] = as_bf16x8(*reinterpret_cast<const short8*>(qp + kk * 16));
+  const float sc2 = a.scale * LOG2E;
+  const float slope2 = GENERAL && a.alibi ? a.alibi[head] * LOG2E : 0.f;
+  const unsigned char* mask =
+      tree ? a.tree_mask + ((long)b * a.Tq + tok) * a.Tq : nullptr;
+
+  // keys the workgroup and this wave see; tree nodes may see any new token
+  const int last = min(base + 128, R) - 1;
+  const int kend = tree ? qs + a.Tq : qs + last / G + 1;
+  const int kbeg =
+      a.window > 0 ? max(0, qs + base / G - a.window + 1) & ~(KT - 1) : 0;
+  const int w0 = base + wave * 32, w1 = min(w0 + 31, R - 1);
+  const int wlast = w0 >= R ? -1 : tree ? kend - 1 : qs + w1 / G;
+  const int wfirst = a.window > 0 ? qs + w0 / G - a.window + 1 : 0;
+  // tiles in [ilo, ihi] need no mask
+  const int ihi = tree ? qs - 1 : qs + w0 / G;
+  const int ilo = a.window > 0 ? qs + w1 / G - a.window + 1 : 0;
+  const int sees = a.window > 0 ? a.window : 0x7fffffff;
+
+  const int tiles = (kend - kbeg + KT - 1) / KT;
+  const int per = (tiles + a.n_split - 1) / a.n_split;
+  const int t0 = kbeg + split * per * KT;
+  const int t1 = min(kend, t0 + per * KT);
+
+  // where this lane's pieces come from
+  int kkey[NI], kcol[NI], vkey[NI], vrow[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int at = (wave + i * 4) * 64 + lane;
+    const int lr = at / RC;
+    kcol[i] = ((at % RC) ^ Tile::swizzle(lr)) * 8;
+    kkey[i] = (lr & ~12) | ((lr & 4) << 1) | ((lr & 8) >> 1);
+    vkey[i] = at / (2 * D) * 16 + (at & 1) * 8;   // groups of 16 keys, (d, octet)
+    vrow[i] = at % (2 * D) / 2;
   }
-
-  // online-softmax state: this lane's 4 C-rows (r = hi*4 + reg)
-  float m2[4], l[4];
-  f32x4 acc_o[NDT];
+  int kpage[NI], vpage[NI];
+  auto look_up = [&](int kb) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) { m2[r] = NEG_BIG; l[r] = 0.f; }
-#pragma unroll
-  for (int n = 0; n < NDT; ++n) acc_o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  // key range this q-tile can see: [lo_min, kmax). Tree queries are not
-  // causal among themselves — every node may see any masked-visible node.
-  const int qpos_max = qs + min(qbase + 127, Tq - 1);
-  const int kmax = (tree_mask != nullptr) ? ctx : min(ctx, qpos_max + 1);
-  int kstart = 0;
-  if (window > 0) kstart = max(0, ((qs + qbase) - window + 1) / KVBLK * KVBLK);
-
-  for (int kbase = kstart; kbase < kmax; kbase += KVBLK) {
-    __syncthreads();  // everyone done reading previous tile
-    // ---- stage K tile (row-major, padded) ----
-    for (int idx = tid; idx < KVBLK * (D / 8); idx += 512) {
-      const int t = idx / (D / 8);
-      const int d8 = (idx % (D / 8)) * 8;
-      const int kpos = kbase + t;
-      short8 kv{};
-      if (kpos < ctx) {
-        const int page = page_table[b * maxp + kpos / P];
-        const long off =
-            (((long)page * (long)(Hq / G) + kvh) * P + (kpos % P)) * D + d8;
-        kv = *reinterpret_cast<const short8*>(k_pages + off);
-      }
-      *reinterpret_cast<short8*>((unsigned char*)k_lds + t * KROW_B + d8 * 2) = kv;
+    for (int i = 0; i < NI; ++i) {
+      kpage[i] = table[min(kb + kkey[i], kend - 1) >> plog];
+      vpage[i] = table[min(kb + vkey[i], kend - 1) >> plog];
     }
-    // ---- stage V tile: pool is d-major (np, Hkv, D, P), so an 8-position
-    // piece at fixed d is one contiguous 16 B load AND one contiguous 16 B
-    // LDS store (kbase is KVBLK-aligned => each octet sits in one page) ----
-    for (int idx = tid; idx < D * (KVBLK / 8); idx += 512) {
-      const int d = idx / (KVBLK / 8);
-      const int o8 = (idx % (KVBLK / 8)) * 8;
-      const int kpos = kbase + o8;
-      short8 vv{};
-      if (kpos < ctx) {
-        const int page = page_table[b * maxp + kpos / P];
-        vv = *reinterpret_cast<const short8*>(
-            v_pages + (((long)page * (long)(Hq / G) + kvh) * D + d) * P +
-            (kpos % P));
-      }
-      *reinterpret_cast<short8*>((unsigned char*)v_lds + d * VROW_B + o8 * 2) = vv;
+  };
+  auto issue = [&](int kb, unsigned char* buf) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int pos = min(kb + kkey[i], kend - 1) & pmask;
+      copy16_to_lds(a.k_pages +
+                        ((((long)kpage[i] * a.Hkv + g) << plog) + pos) * D + kcol[i],
+                    buf + (wave + i * 4) * 1024);
     }
-    __syncthreads();
-
-    // ---- S = Q K^T over this tile: 2 n-tiles of 16 keys ----
-    f32x4 s[KVBLK / 16];
 #pragma unroll
-    for (int n = 0; n < KVBLK / 16; ++n) {
-      s[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < NKK; ++kk) {
-        bf16x8 bfrag = as_bf16x8(*reinterpret_cast<const short8*>(
-            (unsigned char*)k_lds + (li + 16 * n) * KROW_B + hi * 16 + 64 * kk));
-        s[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qfrag[kk], bfrag, s[n], 0, 0, 0);
-      }
+    for (int i = 0; i < NI; ++i) {
+      const int pos = min(kb + vkey[i], (kend - 1) & ~7) & pmask;
+      copy16_to_lds(a.v_pages +
+                        ((((long)vpage[i] * a.Hkv + g) * D + vrow[i]) << plog) + pos,
+                    buf + Tile::KB + (wave + i * 4) * 1024);
     }
+  };
 
-    // ---- mask + online softmax (C layout: row=hi*4+reg, col=li+16n) ----
-    float p[KVBLK / 16][4];
+  float m = NEG_BIG, l = 0.f;   // maximum of the unscaled scores, this half's sum
+  f32x16 acc[ND];
 #pragma unroll
-    for (int reg = 0; reg < 4; ++reg) {
-      const int qrow = qbase + wave * 16 + hi * 4 + reg;
-      const int qpos = qs + qrow;
-      float rm = NEG_BIG;
+  for (int n = 0; n < ND; ++n) acc[n] = f32x16{};
+  const int sw = Tile::swizzle(li);
+  const int krow = li * (D * 2);
+
+  auto compute = [&](int kb, const unsigned char* kt) {
+    f32x16 s[2];
+    s[0] = s[1] = f32x16{};
 #pragma unroll
-      for (int n = 0; n < KVBLK / 16; ++n) {
-        const int kpos = kbase + li + 16 * n;
-        float sv = s[n][reg] * sc2 + aslope * (float)kpos;
-        bool dead = (qrow >= Tq) | (kpos >= ctx);
-        if (!dead) {
-          if (tree_mask != nullptr) {
-            if (kpos >= qs)
-              dead = !tree_mask[((long)b * Tq + qrow) * Tq + (kpos - qs)];
+    for (int kk = 0; kk < NKK; ++kk)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const bf16x8 kf = as_bf16x8(*reinterpret_cast<const short8*>(
+            kt + n * (32 * D * 2) + krow + (((kk * 2 + hi) ^ sw) << 4)));
+        s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s[n], 0, 0, 0);
+      }
+    // s[n][j] is key kb + n * 32 + (j & 8) * 2 + hi * 8 + (j & 7)
+    if (GENERAL) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          s[n][j] = s[n][j] * sc2 +
+                    slope2 * (float)(kb + n * 32 + (j & 8) * 2 + hi * 8 + (j & 7));
+    }
+    if (kb < ilo || kb + KT - 1 > ihi) {
+      const int d0 = qpos - kb - hi * 8;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int off = n * 32 + (j & 8) * 2 + (j & 7);
+          bool dead;
+          if (tree) {
+            const int k = kb + hi * 8 + off - qs;
+            dead = k >= a.Tq || (k >= 0 && !mask[k]);
           } else {
-            dead = (kpos > qpos) |
-                   (window > 0 && kpos <= qpos - window);
+            const int dist = d0 - off;
+            dead = dist < 0 || dist >= sees;
           }
+          if (dead) s[n][j] = NEG_BIG;
         }
-        sv = dead ? NEG_BIG : sv;
-        p[n][reg] = sv;
-        rm = fmaxf(rm, sv);
-      }
-      rm = group16_reduce_max(rm);
-      const float mn = fmaxf(m2[reg], rm);
-      const float corr = fast_exp2(m2[reg] - mn);
-      float psum = 0.f;
-#pragma unroll
-      for (int n = 0; n < KVBLK / 16; ++n) {
-        p[n][reg] = fast_exp2(p[n][reg] - mn);
-        psum += p[n][reg];
-      }
-      psum = group16_reduce_sum(psum);
-      l[reg] = l[reg] * corr + psum;
-      m2[reg] = mn;
-#pragma unroll
-      for (int n = 0; n < NDT; ++n) acc_o[n][reg] *= corr;
     }
-
-    // ---- P -> LDS (C layout scatter), read back as A fragments ----
-    unsigned char* pw = (unsigned char*)p_lds + wave * 16 * PROW_B;
+    float mx = m;
 #pragma unroll
-    for (int n = 0; n < KVBLK / 16; ++n)
+    for (int n = 0; n < 2; ++n)
 #pragma unroll
-      for (int reg = 0; reg < 4; ++reg)
-        *(unsigned short*)(pw + (hi * 4 + reg) * PROW_B + (li + 16 * n) * 2) =
-            f2bf(p[n][reg]);
-    // wave-local LDS; per-wave ds ordering is enforced by lgkmcnt waits
-
-    bf16x8 pfrag = as_bf16x8(
-        *reinterpret_cast<const short8*>(pw + li * PROW_B + hi * 16));
-
-    // ---- acc_o += P V : NDT n-tiles of 16 d-cols ----
+      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[n][j]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float f = GENERAL ? 1.f : sc2;
+    if (__builtin_amdgcn_ballot_w64(mx > m)) {
+      const float corr = fast_exp2((m - mx) * f);
+      l *= corr;
 #pragma unroll
-    for (int n = 0; n < NDT; ++n) {
-      bf16x8 vfrag = as_bf16x8(*reinterpret_cast<const short8*>(
-          (unsigned char*)v_lds + (li + 16 * n) * VROW_B + hi * 16));
-      acc_o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pfrag, vfrag, acc_o[n], 0, 0, 0);
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[n][j] *= corr;
+      m = mx;
+    }
+    // a row that has seen nothing yet keeps weights of zero
+    const float ref = m > 0.5f * NEG_BIG ? m * f : 0.f;
+    bf16x8 pf[4];
+    float ps[2] = {0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const float p = fast_exp2(fmaf(s[n][j], f, -ref));
+        ps[n] += p;
+        pf[n * 2 + (j >> 3)][j & 7] = (__bf16)p;
+      }
+    l += ps[0] + ps[1];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int n = 0; n < ND; ++n) {
+        const bf16x8 vf = as_bf16x8(*reinterpret_cast<const short8*>(
+            kt + Tile::KB + j * (D * 32) + (n * 32 + li) * 32 + hi * 16));
+        acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[j], acc[n], 0, 0, 0);
+      }
+  };
+
+  if (t0 < t1) {
+    // page numbers are looked up a tile ahead of the loads that need them
+    look_up(t0);
+    issue(t0, prefill_lds);
+    look_up(t0 + KT);
+    __syncthreads();
+    int buf = 0;
+    for (int kb = t0; kb < t1; kb += KT) {
+      if (kb + KT < t1) {
+        issue(kb + KT, prefill_lds + (buf ^ 1) * Tile::BYTES);
+        look_up(kb + 2 * KT);
+      }
+      if (kb <= wlast && kb + KT > wfirst)
+        compute(kb, prefill_lds + buf * Tile::BYTES);
+      __syncthreads();
+      buf ^= 1;
     }
   }
 
-  // ---- epilogue: normalize and store ----
-#pragma unroll
-  for (int reg = 0; reg < 4; ++reg) {
-    const int qrow = qbase + wave * 16 + hi * 4 + reg;
-    if (qrow >= Tq) continue;
-    const float inv = (l[reg] > 0.f) ? 1.f / l[reg] : 0.f;
-#pragma unroll
-    for (int n = 0; n < NDT; ++n) {
-      out[(long)b * o_sb + (long)qrow * o_st + (long)h * o_sh + li + 16 * n] =
-          f2bf(acc_o[n][reg] * inv);
+  // a row's values are spread over the two lanes of its column
+  l += __shfl_xor(l, 32);
+  if (row >= R) return;
+  if (a.n_split > 1) {
+    const long at = ((long)split * units + unit) * R + r;
+    if (hi == 0) {
+      a.pml[at * 2] = GENERAL ? m : m * sc2;
+      a.pml[at * 2 + 1] = l;
     }
+    if (l > 0.f) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *reinterpret_cast<f32x4*>(a.pacc + at * D + n * 32 + j * 8 + hi * 4) =
+              f32x4{acc[n][j * 4], acc[n][j * 4 + 1], acc[n][j * 4 + 2],
+                    acc[n][j * 4 + 3]};
+    }
+    return;
   }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  unsigned short* op =
+      a.out + (long)b * a.o_sb + (long)tok * a.o_st + (long)head * a.o_sh + hi * 4;
+#pragma unroll
+  for (int n = 0; n < ND; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      short4v o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (short)f2bf(acc[n][j * 4 + e] * inv);
+      *reinterpret_cast<short4v*>(op + n * 32 + j * 8) = o;
+    }
+}
+
+// Folds the splits of a row: a wave a row, grid rows of all units / 4. A split that
+// saw nothing has a sum of zero and left its values unwritten.
+template <int D>
+__global__ __launch_bounds__(256) void attn_prefill_fold_kernel(PrefillArgs a) {
+  constexpr int V = D >= 128 ? D / 64 : 1;   // columns of a lane
+  const int units = a.B * a.Hkv, R = a.Tq * a.G;
+  const long rows = (long)units * R;
+  const long at = (long)blockIdx.x * 4 + threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1);
+  if (at >= rows || lane * V >= D) return;
+  float m = NEG_BIG;
+  for (int s = 0; s < a.n_split; ++s)
+    m = fmaxf(m, a.pml[(s * rows + at) * 2]);
+  float l = 0.f, o[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) o[e] = 0.f;
+  for (int s = 0; s < a.n_split; ++s) {
+    const float ls = a.pml[(s * rows + at) * 2 + 1];
+    if (!(ls > 0.f)) continue;
+    const float w = fast_exp2(a.pml[(s * rows + at) * 2] - m);
+    l += w * ls;
+    const float* p = a.pacc + (s * rows + at) * D + lane * V;
+#pragma unroll
+    for (int e = 0; e < V; ++e) o[e] += w * p[e];
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int unit = (int)(at / R), r = (int)(at % R);
+  unsigned short* op = a.out + (long)(unit / a.Hkv) * a.o_sb +
+                       (long)(r / a.G) * a.o_st +
+                       (long)(unit % a.Hkv * a.G + r % a.G) * a.o_sh + lane * V;
+#pragma unroll
+  for (int e = 0; e < V; ++e) op[e] = f2bf(o[e] * inv);
 }

@@ -9,6 +9,7 @@
 typedef __attribute__((ext_vector_type(8))) short short8;   // 8 x bf16 = 16 B
 typedef __attribute__((ext_vector_type(4))) short short4v;  // 4 x bf16 = 8 B
 typedef __attribute__((ext_vector_type(4))) float f32x4;    // MFMA 16x16 accum
+typedef __attribute__((ext_vector_type(16))) float f32x16;  // MFMA 32x32 accum
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 
 static constexpr int WAVE = 64;  // CDNA wavefront (guide §1: not 32)
@@ -80,6 +81,15 @@ DEVINL float group16_reduce_max(float x) {
 DEVINL float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 DEVINL float fast_expf(float x) { return __builtin_amdgcn_exp2f(x * LOG2E); }
+
+// 16 B a lane from memory to LDS without registers; l is the wave's, lane i's piece
+// lands i * 16 behind it.
+typedef const __attribute__((address_space(1))) void* gptr_t;
+typedef __attribute__((address_space(3))) void* lptr_t;
+
+DEVINL void copy16_to_lds(const unsigned short* g, unsigned char* l) {
+  __builtin_amdgcn_global_load_lds((gptr_t)g, (lptr_t)l, 16, 0, 0);
+}
 
 DEVINL long ldiv_up(long a, long b) { return (a + b - 1) / b; }
 

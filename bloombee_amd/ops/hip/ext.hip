@@ -366,6 +366,59 @@ torch::Tensor attn_decode_qkv(torch::Tensor qkv, long Hq, torch::Tensor k_pages,
       .view({B, 1, Hq * D});
 }
 
+// Launches attention of a.Tq tokens a sequence; a's tensors and strides are set.
+static void launch_attn_prefill(PrefillArgs a, int D, int P,
+                                const torch::TensorOptions& f32) {
+  TORCH_CHECK(P > 0 && (P & (P - 1)) == 0, "page size must be a power of two");
+  a.p_log2 = __builtin_ctz(P);
+  const long rows = (long)a.Tq * a.G, units = (long)a.B * a.Hkv;
+  if (rows == 0 || units == 0) return;
+  const long row_tiles = (rows + 127) / 128;
+  // A workgroup walks its keys in a chain of tiles, about 1.7 us each at D = 128
+  // when it has the CU to itself. Where row tiles alone leave CUs idle the keys are
+  // split until every CU has a workgroup, and until it has two where the chains
+  // stay long; no split is shorter than two tiles of the longest context the table
+  // can name. Measured with 32 heads on 8, splits as written against none / against
+  // twice as many: 25 tokens behind 1500 20 / 41 / 20 us, 64 behind 8000
+  // 38 / 195 / 51, 333 behind 1201 37 / 42 / 39, 500 behind 7000 (four splits)
+  // 95 / 184 / 106, 1000 behind 4000 (two) 114 / 127 / 125.
+  const long base = row_tiles * units, room = (long)a.maxp * P;
+  long splits = std::max<long>(1, 256 / base);
+  if (room > splits * 24 * 64) splits = std::max<long>(1, 512 / base);
+  a.n_split = (int)std::max<long>(1, std::min({splits, room / 128, 32L}));
+  torch::Tensor part;
+  if (a.n_split > 1) {
+    part = torch::empty({(long)a.n_split * units * rows * (D + 2)}, f32);
+    a.pacc = part.data_ptr<float>();
+    a.pml = a.pacc + (long)a.n_split * units * rows * D;
+  }
+  const bool general = a.alibi || a.tree_mask || !(a.scale > 0.f);
+  const dim3 grid(units * a.n_split, row_tiles);
+  auto launch = [&](auto d, auto gen) {
+    constexpr int DD = decltype(d)::value;
+    auto kernel = attn_prefill_kernel<DD, decltype(gen)::value>;
+    constexpr int lds = 2 * PrefillTile<DD>::BYTES;
+    if (lds > 64 * 1024)
+      TORCH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      lds) == hipSuccess,
+                  "cannot reserve ", lds, " bytes of LDS");
+    kernel<<<grid, 256, lds, cur_stream()>>>(a);
+    if (a.n_split > 1)
+      attn_prefill_fold_kernel<DD>
+          <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
+  };
+  auto by_dim = [&](auto gen) {
+    if (D == 128) launch(std::integral_constant<int, 128>{}, gen);
+    else if (D == 64) launch(std::integral_constant<int, 64>{}, gen);
+    else if (D == 256) launch(std::integral_constant<int, 256>{}, gen);
+    else if (D == 32) launch(std::integral_constant<int, 32>{}, gen);
+    else TORCH_CHECK(false, "unsupported head_dim ", D);
+  };
+  if (general) by_dim(std::true_type{});
+  else by_dim(std::false_type{});
+}
+
 torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
                            torch::Tensor v_pages, torch::Tensor page_table,
                            torch::Tensor q_start, double scale, long window,
@@ -377,13 +430,11 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
   TORCH_CHECK(q.dim() == 4, "attn_prefill expects (B, Hq, Tq, D)");
   const int B = q.size(0), Hq = q.size(1), Tq = q.size(2), D = q.size(3);
   const int Hkv = k_pages.size(1), P = k_pages.size(2), maxp = page_table.size(1);
-  const int G = Hq / Hkv;
-  const float* alibi_ptr = nullptr;
+  PrefillArgs a{};
   if (alibi.has_value()) {
     TORCH_CHECK(alibi->scalar_type() == at::kFloat && alibi->numel() == Hq);
-    alibi_ptr = alibi->data_ptr<float>();
+    a.alibi = alibi->data_ptr<float>();
   }
-  const unsigned char* tm_ptr = nullptr;
   if (tree_mask.has_value()) {
     TORCH_CHECK(tree_mask->scalar_type() == at::kBool &&
                 tree_mask->is_contiguous() &&
@@ -392,24 +443,23 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
     TORCH_CHECK(window == 0, "tree_mask + sliding window: use the torch path");
     CHECK_DEV((*tree_mask));
     // kBool tensors dispatch data_ptr<bool>, not <unsigned char> (Byte)
-    tm_ptr = reinterpret_cast<const unsigned char*>(
+    a.tree_mask = reinterpret_cast<const unsigned char*>(
         tree_mask->data_ptr<bool>());
   }
   auto out = torch::empty_like(q);
-  dim3 grid((Tq + 127) / 128, B * Hq);
-  auto launch = [&](auto d) {
-    attn_prefill_kernel<decltype(d)::value><<<grid, 512, 0, cur_stream()>>>(
-        bf_ptr(q), bf_ptr(k_pages), bf_ptr(v_pages), page_table.data_ptr<int>(),
-        q_start.data_ptr<int>(), alibi_ptr, tm_ptr, bf_ptr_mut(out), B, Hq, G,
-        Tq, P, maxp, (int)window, (float)scale,
-        (long)Hq * Tq * D, (long)D, (long)Tq * D,
-        (long)Hq * Tq * D, (long)D, (long)Tq * D);
-  };
-  if (D == 128) launch(std::integral_constant<int, 128>{});
-  else if (D == 64) launch(std::integral_constant<int, 64>{});
-  else if (D == 256) launch(std::integral_constant<int, 256>{});
-  else if (D == 32) launch(std::integral_constant<int, 32>{});
-  else TORCH_CHECK(false, "unsupported head_dim ", D);
+  a.q = bf_ptr(q);
+  a.k_pages = bf_ptr(k_pages);
+  a.v_pages = bf_ptr(v_pages);
+  a.page_table = page_table.data_ptr<int>();
+  a.q_start = q_start.data_ptr<int>();
+  a.out = bf_ptr_mut(out);
+  a.B = B; a.Hkv = Hkv; a.G = Hq / Hkv; a.Tq = Tq; a.maxp = maxp;
+  a.window = (int)window;
+  a.scale = (float)scale;
+  a.q_sb = a.o_sb = (long)Hq * Tq * D;
+  a.q_st = a.o_st = D;
+  a.q_sh = a.o_sh = (long)Tq * D;
+  launch_attn_prefill(a, D, P, q.options().dtype(at::kFloat));
   return out;
 }
 
@@ -427,22 +477,23 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
   const int B = qkv.size(0), Tq = qkv.size(1);
   const int X = Hq + 2 * Hkv;
   TORCH_CHECK(qkv.dim() == 3 && qkv.size(2) == (long)X * D, "bad fused qkv shape");
-  const int G = Hq / Hkv;
   auto out = torch::empty({B, Tq, (long)Hq * D}, qkv.options());
-  dim3 grid((Tq + 127) / 128, B * Hq);
-  auto launch = [&](auto d) {
-    attn_prefill_kernel<decltype(d)::value><<<grid, 512, 0, cur_stream()>>>(
-        bf_ptr(qkv), bf_ptr(k_pages), bf_ptr(v_pages), page_table.data_ptr<int>(),
-        q_start.data_ptr<int>(), nullptr, nullptr, bf_ptr_mut(out), B, Hq, G,
-        Tq, P, maxp, (int)window, (float)scale,
-        (long)Tq * X * D, (long)X * D, (long)D,
-        (long)Tq * Hq * D, (long)Hq * D, (long)D);
-  };
-  if (D == 128) launch(std::integral_constant<int, 128>{});
-  else if (D == 64) launch(std::integral_constant<int, 64>{});
-  else if (D == 256) launch(std::integral_constant<int, 256>{});
-  else if (D == 32) launch(std::integral_constant<int, 32>{});
-  else TORCH_CHECK(false, "unsupported head_dim ", D);
+  PrefillArgs a{};
+  a.q = bf_ptr(qkv);
+  a.k_pages = bf_ptr(k_pages);
+  a.v_pages = bf_ptr(v_pages);
+  a.page_table = page_table.data_ptr<int>();
+  a.q_start = q_start.data_ptr<int>();
+  a.out = bf_ptr_mut(out);
+  a.B = B; a.Hkv = Hkv; a.G = Hq / Hkv; a.Tq = Tq; a.maxp = maxp;
+  a.window = (int)window;
+  a.scale = (float)scale;
+  a.q_sb = (long)Tq * X * D;
+  a.q_st = (long)X * D;
+  a.q_sh = a.o_sh = D;
+  a.o_sb = (long)Tq * Hq * D;
+  a.o_st = (long)Hq * D;
+  launch_attn_prefill(a, D, P, qkv.options().dtype(at::kFloat));
   return out;
 }
 

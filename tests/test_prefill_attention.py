@@ -1,0 +1,92 @@
+"""Prompt attention over paged caches at the edges of its tiles: rows are (token,
+head of the group) pairs, 128 a workgroup, keys come in tiles of 64 and are split
+over workgroups where the rows leave the device idle."""
+import pytest
+import torch
+
+from bloombee_amd import ops
+from bloombee_amd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def paged(B, Hkv, D, P, lengths, room, seed):
+    """Pages in random order, with large values beyond each sequence's end."""
+    gen = torch.Generator().manual_seed(seed)
+    maxp = -(-room // P)
+    n = B * maxp + 3
+    kp = torch.randn(n, Hkv, P, D, generator=gen).bfloat16()
+    vp = torch.randn(n, Hkv, D, P, generator=gen).bfloat16()
+    table = torch.randperm(n, generator=gen)[:B * maxp].view(B, maxp).int()
+    for b, length in enumerate(lengths):
+        for pos in range(length, maxp * P):
+            page = int(table[b, pos // P])
+            kp[page, :, pos % P] = 50.0
+            vp[page, :, :, pos % P] = 50.0
+    return kp, vp, table
+
+
+CASES = [
+    # B, Hq, Hkv, D, P, tokens, starts, room, window
+    (1, 4, 2, 128, 16, 2, (0,), 16, 0),            # the smallest prompt
+    (2, 8, 2, 128, 16, 25, (1500, 3), 1600, 0),    # split keys, one side short
+    (1, 8, 8, 64, 16, 65, (63,), 128, 0),          # one row over a tile
+    (1, 4, 1, 128, 16, 33, (95,), 128, 0),         # rows of 33 tokens, 132
+    (1, 6, 2, 128, 8, 43, (21,), 64, 0),           # a group of three, small pages
+    (2, 4, 4, 32, 32, 129, (0, 31), 160, 0),
+    (1, 2, 1, 256, 16, 70, (130,), 256, 0),
+    (8, 32, 8, 128, 16, 127, (0, 1, 2, 63, 64, 65, 7, 0), 192, 0),  # no splits
+    (2, 8, 2, 128, 16, 100, (300, 0), 512, 64),    # a window of one tile
+    (1, 4, 2, 64, 16, 90, (200,), 400, 33),
+    (1, 71, 1, 64, 16, 5, (40,), 64, 0),           # a wide group
+]
+
+
+def close(got, want):
+    # weights enter the value product in bf16 and the result is bf16: 2^-9 of the
+    # largest value (4.5 standard deviations) each
+    err = (got.cpu().float() - want.float()).abs().max()
+    assert err <= 2 * 4.5 * 2.0 ** -9, err
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c[:6])))
+@pytest.mark.parametrize("form", ["plain", "alibi", "tree"])
+def test_prompt_attention(case, form):
+    B, Hq, Hkv, D, P, T, starts, room, window = case
+    if form == "tree" and window:
+        pytest.skip("tree steps have no window")
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=T)
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    slopes = ops.alibi_slopes_for(Hq) if form == "alibi" else None
+    tree = None
+    if form == "tree":
+        tree = torch.rand(B, T, T, generator=gen) < 0.3
+        tree |= torch.eye(T, dtype=torch.bool)
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long(),
+                          sliding_window=window or None, alibi_slopes=slopes,
+                          tree_mask=tree)
+    dev = [t.to(DEV) for t in (q, kp, vp, table, qs)]
+    got = ops.attn_paged(*dev, window=window, alibi_slopes=slopes,
+                         tree_mask=None if tree is None else tree.to(DEV))
+    close(got, want)
+
+
+@pytest.mark.parametrize("case", CASES[1:5], ids=lambda c: "-".join(map(str, c[:6])))
+def test_queries_of_a_fused_projection(case):
+    """Queries read from [q | k | v] rows, results in rows of heads; infinite keys
+    beyond the context do no harm."""
+    B, Hq, Hkv, D, P, T, starts, room, window = case
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=T)
+    kp[kp == 50.0] = float("inf")
+    gen = torch.Generator().manual_seed(3)
+    qkv = torch.randn(B, T, (Hq + 2 * Hkv) * D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    want = ops.attn_paged_qkv(qkv.float(), Hq, Hkv, kp.float(), vp.float(), table,
+                              qs)
+    got = ops.attn_paged_qkv(qkv.to(DEV), Hq, Hkv, kp.to(DEV), vp.to(DEV),
+                             table.to(DEV), qs.to(DEV))
+    close(got, want)
