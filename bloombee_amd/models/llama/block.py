@@ -30,6 +30,7 @@ import torch.nn.functional as F
 from bloombee_amd import ops
 from bloombee_amd.kv.paged import SessionHandle
 from bloombee_amd.models.base import ModelConfig
+from bloombee_amd.ops import training
 
 
 class RopeTables:
@@ -299,15 +300,7 @@ class LlamaBlock(torch.nn.Module):
     # training path (differentiable; full sequence, no KV cache)
     # ------------------------------------------------------------------
     def forward_train(self, hidden: torch.Tensor, start_pos: int = 0) -> torch.Tensor:
-        B, T, H = hidden.shape
-        Hq, Hkv, D = self.Hq, self.Hkv, self.D
-        cfg = self.config
-        G = Hq // Hkv
-
-        def rms(x, w):
-            xf = x.float()
-            return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + cfg.rms_norm_eps)
-                    ).to(x.dtype) * w
+        eps = self.config.rms_norm_eps
 
         def lin(x_, w, name):
             # training path honors active LoRA adapters too (the inference
@@ -320,34 +313,14 @@ class LlamaBlock(torch.nn.Module):
                     y = y + d
             return y
 
-        x = rms(hidden, self.input_norm_w)
-        qkv = lin(x, self.qkv_w, "qkv_w").view(B, T, Hq + 2 * Hkv, D).permute(0, 2, 1, 3)
-        q, k, v = qkv.split([Hq, Hkv, Hkv], dim=1)
+        hidden, x = training.norm(hidden, self.input_norm_w, eps)
         cos, sin = self.rope.get(hidden.device)
-        pos = torch.arange(start_pos, start_pos + T, device=hidden.device)
-        c = cos[pos].view(1, 1, T, D // 2).float()
-        s = sin[pos].view(1, 1, T, D // 2).float()
-
-        def rot(t):
-            tf = t.float()
-            t1, t2 = tf[..., : D // 2], tf[..., D // 2:]
-            return torch.cat([t1 * c - t2 * s, t2 * c + t1 * s], -1).to(t.dtype)
-
-        q, k = rot(q), rot(k)
-        k = k.repeat_interleave(G, dim=1)
-        v = v.repeat_interleave(G, dim=1)
-        scores = torch.matmul(q.float(), k.float().transpose(-1, -2)) * self.scale
-        mask = torch.ones(T, T, dtype=torch.bool, device=hidden.device).tril()
-        scores = scores.masked_fill(~mask, float("-inf"))
-        p = torch.softmax(scores, dim=-1)
-        attn = torch.matmul(p, v.float()).to(hidden.dtype)
-        attn = attn.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
-        h2 = hidden + lin(attn, self.o_w, "o_w")
-        y = rms(h2, self.post_norm_w)
-        gu = F.linear(y, self.gate_up_w)
-        g, u = gu.split([self.I, self.I], dim=-1)
-        m = F.linear(F.silu(g.float()).to(u.dtype) * u, self.down_w)
-        return h2 + m
+        attn = training.rope_attention(lin(x, self.qkv_w, "qkv_w"), cos, sin,
+                                       self.Hq, self.Hkv, start_pos, self.scale)
+        h2, y = training.add_norm(lin(attn, self.o_w, "o_w"), hidden,
+                                  self.post_norm_w, eps)
+        m = training.swiglu(F.linear(y, self.gate_up_w))
+        return h2 + F.linear(m, self.down_w)
 
     def forward(self, *args, **kw):
         return self.forward_inference(*args, **kw)

@@ -1,0 +1,548 @@
+// Causal attention of whole sequences with its gradients, rotations included.
+//
+//  rope_rows_kernel        rotates queries and keys of a fused [q | k | v] projection
+//                          into a buffer of their own.
+//  attn_train_kernel       the attention; keeps the 32-bit result and each row's
+//                          log-sum for the gradients.
+//  attn_train_dq_kernel    gradients of the queries, turned back; a row's
+//                          sum(dO * O) on the way, for the next kernel.
+//  attn_train_dkv_kernel   gradients of keys (turned back) and values, summed over
+//                          the heads of a group in registers.
+//
+// Rows are (token, head of the group) pairs. All products are
+// v_mfma_f32_32x32x16_bf16. Scores and weights never reach memory: the gradient
+// kernels make them anew, the first with a row a lane (S^T, what it adds up is over
+// keys), the second with a key a lane (S, what it adds up is over rows), so that each
+// finds its second products' operand in its registers: the keys (rows) of a product
+// are taken in an order, bits 2 and 3 of their number swapped, in which the 16
+// results of a lane are the eight consecutive ones it hands to each of two products.
+// The other operand has to be read by columns, which the transposing LDS reads do.
+// No atomics; every sum has a fixed order.
+//
+// Weights and their gradients are 32-bit. They enter the second products as a sum of
+// two bf16 (the value and what its rounding lost); queries, keys, values and dO are
+// bf16 already. So a product loses no more than 2^-17 of a term.
+//
+// The matrix cores bound all three: 3, 4 and 6 products of 32 x 32 x D a tile. Two
+// sequences of 1999, 32 heads on 8 of 128: 136, 166 and 401 us (721, 788 and 490
+// TF/s of the visible half); as float32 torch operations a layer's attention took
+// 9.2 ms both ways.
+
+#pragma once
+#include "common.h"
+
+struct TrainAttnArgs {
+  const unsigned short* qk;    // (B, T, Hq + Hkv, D) rotated
+  const unsigned short* qkv;   // (B, T, Hq + 2 Hkv, D)
+  const unsigned short* dout;  // (B, T, Hq, D)
+  const float* cos_t;          // (positions, D / 2)
+  const float* sin_t;
+  unsigned short* out;         // (B, T, Hq, D)
+  float* out32;                // the same, or null: no gradients wanted
+  float* lse;                  // (B * Hkv, T * G) log2 units
+  float* delta;                // (B * Hkv, T * G)
+  unsigned short* dqkv;        // (B, T, Hq + 2 Hkv, D)
+  int B, T, Hkv, G, start;
+  float scale;
+};
+
+template <int D>
+struct TrainTile {
+  static constexpr int RC = D / 8;                // 16 B pieces of a row
+  static constexpr int BYTES = 64 * D * 2;        // 64 rows
+  static constexpr int NI = BYTES / 1024 / 4;     // loads of a wave
+  // piece c of row r lies at c ^ swizzle(r). Sixteen rows read at one piece, and
+  // four rows read at four consecutive pieces, cover all banks.
+  DEVINL static int swizzle(int r) {
+    return RC >= 16 ? ((r & 3) << 2) | ((r >> 2) & 3)
+                    : ((r & 2) << 1) | ((r >> 2) & 3);
+  }
+};
+
+typedef __attribute__((address_space(3))) short4v train_lds4;
+
+// MFMA row -> row of the tile it stands for.
+DEVINL int swap23(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
+
+// Eight elements of row `row` from kk * 16 + hi * 8.
+template <int D>
+DEVINL bf16x8 row_frag(const unsigned char* tile, int row, int kk, int hi) {
+  return as_bf16x8(*reinterpret_cast<const short8*>(
+      tile + row * (D * 2) + (((kk * 2 + hi) ^ TrainTile<D>::swizzle(row)) << 4)));
+}
+
+// Column n * 32 + (lane & 31) of rows r0 + (lane >> 5) * 8 .. +7; r0 % 16 == 0.
+template <int D>
+DEVINL bf16x8 col_frag(const unsigned char* tile, int r0, int n, int lane) {
+  const int i = lane & 15, row = r0 + (lane >> 5) * 8 + (i >> 2);
+  const int piece = n * 4 + ((lane >> 4) & 1) * 2 + ((i >> 1) & 1);
+  short8 v;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int r = row + q * 4;
+    const short4v c = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (train_lds4*)(tile + r * (D * 2) +
+                      ((piece ^ TrainTile<D>::swizzle(r)) << 4) + (i & 1) * 8));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[q * 4 + e] = c[e];
+  }
+  return as_bf16x8(v);
+}
+
+DEVINL void split_pair(const float* p, bf16x8& hi, bf16x8& lo) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    hi[j] = (__bf16)p[j];
+    lo[j] = (__bf16)(p[j] - (float)hi[j]);
+  }
+}
+
+// Rows of two (token, head) tensors that a workgroup's kernels read.
+struct RowMap {
+  const unsigned short* base;
+  long ld;      // of a token
+  int G;        // heads taken in turns
+  DEVINL const unsigned short* at(int row, int D) const {
+    return base + (long)(row / G) * ld + row % G * D;
+  }
+};
+
+// 64 rows from r0 to LDS, rows beyond `last` repeat it.
+template <int D>
+DEVINL void stage_rows(const RowMap& m, int r0, int last, unsigned char* tile,
+                       int wave, int lane) {
+  using Tile = TrainTile<D>;
+#pragma unroll
+  for (int i = 0; i < Tile::NI; ++i) {
+    const int at = (wave + i * 4) * 64 + lane;
+    const int r = at / Tile::RC, c = (at % Tile::RC) ^ Tile::swizzle(r);
+    copy16_to_lds(m.at(min(r0 + r, last), D) + c * 8, tile + (wave + i * 4) * 1024);
+  }
+}
+
+// grid: ceil(B * T * (Hq + Hkv) * D / 16 / 256); a thread turns eight pairs
+__global__ __launch_bounds__(256) void rope_rows_kernel(
+    const unsigned short* __restrict__ qkv, unsigned short* __restrict__ qk,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t, long tokens,
+    int T, int heads, int X, int D, int start) {
+  const int per = D / 16;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= tokens * heads * per) return;
+  const int c = (int)(i % per) * 8;
+  const int h = (int)(i / per % heads);
+  const long t = i / per / heads;
+  const unsigned short* src = qkv + (t * X + h) * D + c;
+  unsigned short* dst = qk + (t * heads + h) * D + c;
+  const long p = (long)(start + (int)(t % T)) * (D / 2) + c;
+  float x[8], y[8], u[8], v[8];
+  load_bf16x8(src, x);
+  load_bf16x8(src + D / 2, y);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float cs = cos_t[p + j], sn = sin_t[p + j];
+    u[j] = x[j] * cs - y[j] * sn;
+    v[j] = y[j] * cs + x[j] * sn;
+  }
+  store_bf16x8(dst, u);
+  store_bf16x8(dst + D / 2, v);
+}
+
+// grid (B * Hkv, row tiles of 128); four waves of 32 rows
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_train_kernel(TrainAttnArgs a) {
+  using Tile = TrainTile<D>;
+  constexpr int KT = 64, NKK = D / 16, ND = D / 32;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * Tile::BYTES];
+  const int b = blockIdx.x / a.Hkv, g = blockIdx.x % a.Hkv;
+  const int G = a.G, R = a.T * G, Hq = a.Hkv * G;
+  const int base = (int)(gridDim.y - 1 - blockIdx.y) * 128;  // long rows first
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int li = lane & 31, hi = lane >> 5;
+  const long ldq = (long)(Hq + a.Hkv) * D, ldx = (long)(Hq + 2 * a.Hkv) * D;
+  const unsigned short* qb = a.qk + (long)b * a.T * ldq;
+  const RowMap keys{qb + (long)(Hq + g) * D, ldq, 1};
+  const RowMap vals{a.qkv + (long)b * a.T * ldx + (long)(Hq + a.Hkv + g) * D, ldx, 1};
+  const RowMap rows{qb + (long)g * G * D, ldq, G};
+
+  const int row = base + wave * 32 + li;
+  const int r = min(row, R - 1), tok = r / G;
+  bf16x8 qf[NKK];
+  const unsigned short* qp = rows.at(r, D) + hi * 8;
+#pragma unroll
+  for (int kk = 0; kk < NKK; ++kk)
+    qf[kk] = as_bf16x8(*reinterpret_cast<const short8*>(qp + kk * 16));
+  const float sc2 = a.scale * LOG2E;
+  const int kend = (min(base + 128, R) - 1) / G + 1;
+  const int w0 = base + wave * 32;
+  const int wlast = w0 >= R ? -1 : min(w0 + 31, R - 1) / G;
+  const int wfull = w0 / G;    // keys up to here are seen by all rows of the wave
+  const int krow = swap23(li);
+
+  float m = NEG_BIG, l = 0.f;
+  f32x16 acc[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n) acc[n] = f32x16{};
+
+  stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
+  stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
+  __syncthreads();
+  int buf = 0;
+  for (int kb = 0; kb < kend; kb += KT) {
+    if (kb + KT < kend) {
+      unsigned char* next = lds + (buf ^ 1) * 2 * Tile::BYTES;
+      stage_rows<D>(keys, kb + KT, kend - 1, next, wave, lane);
+      stage_rows<D>(vals, kb + KT, kend - 1, next + Tile::BYTES, wave, lane);
+    }
+    const unsigned char* kt = lds + buf * 2 * Tile::BYTES;
+    if (kb <= wlast) {
+      f32x16 s[2];
+      s[0] = s[1] = f32x16{};
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk)
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+          s[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              row_frag<D>(kt, n * 32 + krow, kk, hi), qf[kk], s[n], 0, 0, 0);
+      // s[n][j] is key kb + n * 32 + (j & 8) * 2 + hi * 8 + (j & 7)
+      if (kb + KT - 1 > wfull) {
+        const int d0 = tok - kb - hi * 8;
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (n * 32 + (j & 8) * 2 + (j & 7) > d0) s[n][j] = NEG_BIG;
+      }
+      float mx = m;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) mx = fmaxf(mx, s[n][j]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (__builtin_amdgcn_ballot_w64(mx > m)) {
+        const float corr = fast_exp2((m - mx) * sc2);
+        l *= corr;
+#pragma unroll
+        for (int n = 0; n < ND; ++n)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) acc[n][j] *= corr;
+        m = mx;
+      }
+      const float ref = m > 0.5f * NEG_BIG ? m * sc2 : 0.f;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          float p[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            p[e] = fast_exp2(fmaf(s[n][j * 8 + e], sc2, -ref));
+            l += p[e];
+          }
+          bf16x8 ph, pl;
+          split_pair(p, ph, pl);
+#pragma unroll
+          for (int d = 0; d < ND; ++d) {
+            const bf16x8 vf =
+                col_frag<D>(kt + Tile::BYTES, n * 32 + j * 16, d, lane);
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph, acc[d], 0, 0, 0);
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl, acc[d], 0, 0, 0);
+          }
+        }
+    }
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  l += __shfl_xor(l, 32);
+  if (row >= R) return;
+  const float inv = 1.f / l;
+  const long at = (((long)b * a.T + tok) * Hq + g * G + r % G) * D + hi * 4;
+  if (a.out32 && hi == 0)
+    a.lse[(long)blockIdx.x * R + r] = m * sc2 + __log2f(l);
+#pragma unroll
+  for (int n = 0; n < ND; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4 o;
+      short4v u;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        o[e] = acc[n][j * 4 + e] * inv;
+        u[e] = (short)f2bf(o[e]);
+      }
+      *reinterpret_cast<short4v*>(a.out + at + n * 32 + j * 8) = u;
+      if (a.out32) *reinterpret_cast<f32x4*>(a.out32 + at + n * 32 + j * 8) = o;
+    }
+}
+
+// grid and rows as above
+template <int D>
+__global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) {
+  using Tile = TrainTile<D>;
+  constexpr int KT = 64, NKK = D / 16, ND = D / 32;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * Tile::BYTES];
+  const int b = blockIdx.x / a.Hkv, g = blockIdx.x % a.Hkv;
+  const int G = a.G, R = a.T * G, Hq = a.Hkv * G;
+  const int base = (int)(gridDim.y - 1 - blockIdx.y) * 128;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int li = lane & 31, hi = lane >> 5;
+  const long ldq = (long)(Hq + a.Hkv) * D, ldx = (long)(Hq + 2 * a.Hkv) * D;
+  const unsigned short* qb = a.qk + (long)b * a.T * ldq;
+  const RowMap keys{qb + (long)(Hq + g) * D, ldq, 1};
+  const RowMap vals{a.qkv + (long)b * a.T * ldx + (long)(Hq + a.Hkv + g) * D, ldx, 1};
+  const RowMap rows{qb + (long)g * G * D, ldq, G};
+
+  const int row = base + wave * 32 + li;
+  const int r = min(row, R - 1), tok = r / G;
+  const long at = (((long)b * a.T + tok) * Hq + g * G + r % G) * D;
+  bf16x8 qf[NKK], of[NKK];
+  const unsigned short* qp = rows.at(r, D) + hi * 8;
+  float del = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NKK; ++kk) {
+    qf[kk] = as_bf16x8(*reinterpret_cast<const short8*>(qp + kk * 16));
+    const long c = at + kk * 16 + hi * 8;
+    of[kk] = as_bf16x8(*reinterpret_cast<const short8*>(a.dout + c));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) del += (float)of[kk][e] * a.out32[c + e];
+  }
+  del += __shfl_xor(del, 32);
+  const float lse = a.lse[(long)blockIdx.x * R + r];
+  if (hi == 0 && row < R) a.delta[(long)blockIdx.x * R + r] = del;
+  const float sc2 = a.scale * LOG2E;
+  const int kend = (min(base + 128, R) - 1) / G + 1;
+  const int w0 = base + wave * 32;
+  const int wlast = w0 >= R ? -1 : min(w0 + 31, R - 1) / G;
+  const int wfull = w0 / G;
+  const int krow = swap23(li);
+
+  f32x16 acc[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n) acc[n] = f32x16{};
+
+  stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
+  stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
+  __syncthreads();
+  int buf = 0;
+  for (int kb = 0; kb < kend; kb += KT) {
+    if (kb + KT < kend) {
+      unsigned char* next = lds + (buf ^ 1) * 2 * Tile::BYTES;
+      stage_rows<D>(keys, kb + KT, kend - 1, next, wave, lane);
+      stage_rows<D>(vals, kb + KT, kend - 1, next + Tile::BYTES, wave, lane);
+    }
+    const unsigned char* kt = lds + buf * 2 * Tile::BYTES;
+    if (kb <= wlast) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        f32x16 s = f32x16{}, dp = f32x16{};
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+          s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              row_frag<D>(kt, n * 32 + krow, kk, hi), qf[kk], s, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              row_frag<D>(kt + Tile::BYTES, n * 32 + krow, kk, hi), of[kk], dp, 0, 0,
+              0);
+        }
+        const int d0 = tok - kb - hi * 8;
+        const bool edge = kb + KT - 1 > wfull;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          float ds[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float p = fast_exp2(fmaf(s[j * 8 + e], sc2, -lse));
+            ds[e] = p * (dp[j * 8 + e] - del);
+            if (edge && n * 32 + j * 16 + e > d0) ds[e] = 0.f;
+          }
+          bf16x8 dh, dl;
+          split_pair(ds, dh, dl);
+#pragma unroll
+          for (int d = 0; d < ND; ++d) {
+            const bf16x8 kf = col_frag<D>(kt, n * 32 + j * 16, d, lane);
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, dh, acc[d], 0, 0, 0);
+            acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, dl, acc[d], 0, 0, 0);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  if (row >= R) return;
+  // back through the rotation: element d turned with element d + D / 2
+  unsigned short* dq = a.dqkv + ((long)b * a.T + tok) * ldx +
+                       (long)(g * G + r % G) * D + hi * 4;
+  const long p = (long)(a.start + tok) * (D / 2) + hi * 4;
+#pragma unroll
+  for (int n = 0; n < ND / 2; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      short4v x, y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float cs = a.cos_t[p + n * 32 + j * 8 + e];
+        const float sn = a.sin_t[p + n * 32 + j * 8 + e];
+        const float u = acc[n][j * 4 + e] * a.scale;
+        const float v = acc[n + ND / 2][j * 4 + e] * a.scale;
+        x[e] = (short)f2bf(u * cs + v * sn);
+        y[e] = (short)f2bf(v * cs - u * sn);
+      }
+      *reinterpret_cast<short4v*>(dq + n * 32 + j * 8) = x;
+      *reinterpret_cast<short4v*>(dq + D / 2 + n * 32 + j * 8) = y;
+    }
+}
+
+// grid (B * Hkv, tiles of 64 keys); waves 0 and 1 own 32 keys each, waves 2 and 3 the
+// same keys: the two pairs take the two halves of a tile of 64 rows and add up at the
+// end. 192 accumulator and operand registers leave room for one wave a SIMD; tiles of
+// 64 keys and not 128 make twice as many workgroups with half as long a chain.
+template <int D>
+__global__ __launch_bounds__(256, 1) void attn_train_dkv_kernel(TrainAttnArgs a) {
+  using Tile = TrainTile<D>;
+  constexpr int NKK = D / 16, ND = D / 32;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * Tile::BYTES];
+  __shared__ __attribute__((aligned(16))) float stat[2][2][64];
+  const int b = blockIdx.x / a.Hkv, g = blockIdx.x % a.Hkv;
+  const int G = a.G, R = a.T * G, Hq = a.Hkv * G;
+  const int k0 = blockIdx.y * 64;                // early keys are seen most
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int li = lane & 31, hi = lane >> 5;
+  const int half = (wave >> 1) * 32;
+  const long ldq = (long)(Hq + a.Hkv) * D, ldx = (long)(Hq + 2 * a.Hkv) * D;
+  const unsigned short* qb = a.qk + (long)b * a.T * ldq;
+  const RowMap rows{qb + (long)g * G * D, ldq, G};
+  const RowMap outs{a.dout + ((long)b * a.T * Hq + (long)g * G) * D, (long)Hq * D, G};
+  const float* lse = a.lse + (long)blockIdx.x * R;
+  const float* delta = a.delta + (long)blockIdx.x * R;
+
+  const int key = k0 + (wave & 1) * 32 + li;
+  bf16x8 kf[NKK], vf[NKK];
+  {
+    const long t = (long)b * a.T + min(key, a.T - 1);
+    const unsigned short* kp = a.qk + t * ldq + (long)(Hq + g) * D + hi * 8;
+    const unsigned short* vp = a.qkv + t * ldx + (long)(Hq + a.Hkv + g) * D + hi * 8;
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+      kf[kk] = as_bf16x8(*reinterpret_cast<const short8*>(kp + kk * 16));
+      vf[kk] = as_bf16x8(*reinterpret_cast<const short8*>(vp + kk * 16));
+    }
+  }
+  const float sc2 = a.scale * LOG2E;
+  const int first = key * G;                     // rows from here on see the key
+  const int full = (k0 + (wave & 1) * 32 + 31) * G;   // ... all keys of the wave
+  const int qrow = half + swap23(li);
+
+  f32x16 dk[ND], dv[ND];
+#pragma unroll
+  for (int n = 0; n < ND; ++n) dk[n] = dv[n] = f32x16{};
+
+  const int r0 = (k0 * G) & ~63;
+  float mine = 0.f;
+  auto fetch = [&](int rb) {
+    if (tid < 64) mine = lse[min(rb + tid, R - 1)];
+    else if (tid < 128) mine = delta[min(rb + tid - 64, R - 1)];
+  };
+  auto keep = [&](int bf) {
+    if (tid < 128) stat[bf][tid >> 6][tid & 63] = mine;
+  };
+  stage_rows<D>(rows, r0, R - 1, lds, wave, lane);
+  stage_rows<D>(outs, r0, R - 1, lds + Tile::BYTES, wave, lane);
+  fetch(r0);
+  keep(0);
+  __syncthreads();
+  int buf = 0;
+  for (int rb = r0; rb < R; rb += 64) {
+    const bool more = rb + 64 < R;
+    if (more) {
+      unsigned char* next = lds + (buf ^ 1) * 2 * Tile::BYTES;
+      stage_rows<D>(rows, rb + 64, R - 1, next, wave, lane);
+      stage_rows<D>(outs, rb + 64, R - 1, next + Tile::BYTES, wave, lane);
+      fetch(rb + 64);
+    }
+    const unsigned char* qt = lds + buf * 2 * Tile::BYTES;
+    const unsigned char* ot = qt + Tile::BYTES;
+    const int w0 = rb + half;
+    if (w0 < R && w0 + 31 >= (k0 + (wave & 1) * 32) * G) {
+      f32x16 s = f32x16{}, dp = f32x16{};
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk) {
+        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(qt, qrow, kk, hi),
+                                                    kf[kk], s, 0, 0, 0);
+        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(ot, qrow, kk, hi),
+                                                     vf[kk], dp, 0, 0, 0);
+      }
+      // element j of a lane is row w0 + (j & 8) * 2 + hi * 8 + (j & 7)
+      const bool edge = w0 < full || w0 + 31 >= R;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float p[8], ds[8];
+        const int rr = half + j * 16 + hi * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          p[e] = fast_exp2(fmaf(s[j * 8 + e], sc2, -stat[buf][0][rr + e]));
+          const int q = rb + rr + e;
+          if (edge && (q < first || q >= R)) p[e] = 0.f;
+          ds[e] = p[e] * (dp[j * 8 + e] - stat[buf][1][rr + e]);
+        }
+        bf16x8 ph, pl, dh, dl;
+        split_pair(p, ph, pl);
+        split_pair(ds, dh, dl);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          const bf16x8 oc = col_frag<D>(ot, half + j * 16, d, lane);
+          const bf16x8 qc = col_frag<D>(qt, half + j * 16, d, lane);
+          dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ph, oc, dv[d], 0, 0, 0);
+          dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dh, qc, dk[d], 0, 0, 0);
+          dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pl, oc, dv[d], 0, 0, 0);
+          dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dl, qc, dk[d], 0, 0, 0);
+        }
+      }
+    }
+    if (more) keep(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  // the second pair's sums go through LDS, values and keys one after the other
+  float* sums = reinterpret_cast<float*>(lds) + (wave & 1) * 32 * D;
+  auto join = [&](f32x16 (&x)[ND]) {
+    if (wave >> 1) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sums[(n * 16 + j) * 64 + lane] = x[n][j];
+    }
+    __syncthreads();
+    if (!(wave >> 1)) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[n][j] += sums[(n * 16 + j) * 64 + lane];
+    }
+    __syncthreads();
+  };
+  join(dv);
+  join(dk);
+  if (wave >> 1) return;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int t = k0 + (wave & 1) * 32 + (j & 3) + (j >> 2) * 8 + hi * 4;
+    if (t >= a.T) continue;
+    unsigned short* kx = a.dqkv + ((long)b * a.T + t) * ldx + (long)(Hq + g) * D + li;
+    unsigned short* vx = kx + (long)a.Hkv * D;
+    const long p = (long)(a.start + t) * (D / 2) + li;
+#pragma unroll
+    for (int n = 0; n < ND; ++n) vx[n * 32] = f2bf(dv[n][j]);
+#pragma unroll
+    for (int n = 0; n < ND / 2; ++n) {
+      const float cs = a.cos_t[p + n * 32], sn = a.sin_t[p + n * 32];
+      const float u = dk[n][j] * a.scale, v = dk[n + ND / 2][j] * a.scale;
+      kx[n * 32] = f2bf(u * cs + v * sn);
+      kx[D / 2 + n * 32] = f2bf(v * cs - u * sn);
+    }
+  }
+}

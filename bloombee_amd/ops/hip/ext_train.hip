@@ -1,0 +1,180 @@
+// Torch bindings of the training path's kernels.
+
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
+
+#include "attn_train.hip"
+#include "train_rows.hip"
+
+using torch::Tensor;
+using OptTensor = c10::optional<Tensor>;
+
+static hipStream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+#define CHECK_T(x, st)                                                        \
+  TORCH_CHECK((x).is_cuda() && (x).is_contiguous() &&                         \
+                  (x).scalar_type() == (st),                                  \
+              #x " must be a contiguous device tensor of ", toString(st))
+
+static void check_launch() {
+  const hipError_t e = hipGetLastError();
+  TORCH_CHECK(e == hipSuccess, "kernel launch: ", hipGetErrorString(e));
+}
+
+static const unsigned short* in(const Tensor& t) {
+  return reinterpret_cast<const unsigned short*>(t.data_ptr());
+}
+static unsigned short* out(const Tensor& t) {
+  return reinterpret_cast<unsigned short*>(t.data_ptr());
+}
+
+// Sizes of a fused projection (B, T, (Hq + 2 Hkv) * D), positions from `start`.
+static TrainAttnArgs attn_args(const Tensor& qkv, long Hq, long Hkv,
+                               const Tensor& cos_t, const Tensor& sin_t, long start,
+                               double scale) {
+  CHECK_T(qkv, at::kBFloat16);
+  CHECK_T(cos_t, at::kFloat);
+  CHECK_T(sin_t, at::kFloat);
+  TORCH_CHECK(Hkv > 0 && Hq > 0 && Hq % Hkv == 0, "heads: ", Hq, " on ", Hkv);
+  TORCH_CHECK(qkv.dim() == 3 && qkv.size(2) % (Hq + 2 * Hkv) == 0 &&
+                  qkv.numel() > 0,
+              "bad fused qkv shape");
+  const long D = qkv.size(2) / (Hq + 2 * Hkv);
+  TORCH_CHECK(D == 64 || D == 128, "unsupported head_dim ", D);
+  TORCH_CHECK(cos_t.dim() == 2 && cos_t.size(1) == D / 2 &&
+                  cos_t.sizes() == sin_t.sizes(),
+              "bad rotation tables");
+  TORCH_CHECK(start >= 0 && start + qkv.size(1) <= cos_t.size(0),
+              "positions beyond the rotation tables");
+  TORCH_CHECK(qkv.size(1) * (Hq / Hkv) < (1L << 30), "too many rows");
+  TORCH_CHECK(scale > 0, "scale must be positive");
+  TrainAttnArgs a{};
+  a.qkv = in(qkv);
+  a.cos_t = cos_t.data_ptr<float>();
+  a.sin_t = sin_t.data_ptr<float>();
+  a.B = qkv.size(0);
+  a.T = qkv.size(1);
+  a.Hkv = Hkv;
+  a.G = Hq / Hkv;
+  a.start = start;
+  a.scale = scale;
+  return a;
+}
+
+template <typename F>
+static void by_head(long D, F f) {
+  if (D == 128) f(std::integral_constant<int, 128>{});
+  else f(std::integral_constant<int, 64>{});
+}
+
+// (result, rotated queries and keys, 32-bit result, log-sums); without `grad` the
+// last two are empty.
+std::vector<Tensor> rope_attention(Tensor qkv, long Hq, long Hkv, Tensor cos_t,
+                                   Tensor sin_t, long start, double scale,
+                                   bool grad) {
+  TrainAttnArgs a = attn_args(qkv, Hq, Hkv, cos_t, sin_t, start, scale);
+  const long D = qkv.size(2) / (Hq + 2 * Hkv), B = a.B, T = a.T;
+  Tensor qk = torch::empty({B, T, (Hq + Hkv) * D}, qkv.options());
+  Tensor o = torch::empty({B, T, Hq * D}, qkv.options());
+  const auto f32 = qkv.options().dtype(at::kFloat);
+  Tensor o32 = torch::empty({grad ? B : 0, T, Hq * D}, f32);
+  Tensor lse = torch::empty({grad ? B * Hkv : 0, T * a.G}, f32);
+  a.qk = in(qk);
+  a.out = out(o);
+  if (grad) {
+    a.out32 = o32.data_ptr<float>();
+    a.lse = lse.data_ptr<float>();
+  }
+  const long pairs = B * T * (Hq + Hkv) * D / 16;
+  rope_rows_kernel<<<(pairs + 255) / 256, 256, 0, stream()>>>(
+      a.qkv, out(qk), a.cos_t, a.sin_t, B * T, T, Hq + Hkv, Hq + 2 * Hkv, D, start);
+  by_head(D, [&](auto d) {
+    attn_train_kernel<decltype(d)::value>
+        <<<dim3(B * Hkv, (T * a.G + 127) / 128), 256, 0, stream()>>>(a);
+  });
+  check_launch();
+  return {o, qk, o32, lse};
+}
+
+Tensor rope_attention_grad(Tensor gout, Tensor qkv, Tensor qk, Tensor o32,
+                           Tensor lse, long Hq, long Hkv, Tensor cos_t, Tensor sin_t,
+                           long start, double scale) {
+  TrainAttnArgs a = attn_args(qkv, Hq, Hkv, cos_t, sin_t, start, scale);
+  const long D = qkv.size(2) / (Hq + 2 * Hkv), B = a.B, T = a.T;
+  CHECK_T(gout, at::kBFloat16);
+  CHECK_T(qk, at::kBFloat16);
+  CHECK_T(o32, at::kFloat);
+  CHECK_T(lse, at::kFloat);
+  TORCH_CHECK(gout.numel() == B * T * Hq * D && o32.numel() == gout.numel() &&
+                  qk.numel() == B * T * (Hq + Hkv) * D &&
+                  lse.numel() == B * T * Hq,
+              "gradient of another shape");
+  Tensor delta = torch::empty_like(lse);
+  Tensor dqkv = torch::empty_like(qkv);
+  a.qk = in(qk);
+  a.dout = in(gout);
+  a.out32 = o32.data_ptr<float>();
+  a.lse = lse.data_ptr<float>();
+  a.delta = delta.data_ptr<float>();
+  a.dqkv = out(dqkv);
+  by_head(D, [&](auto d) {
+    constexpr int DD = decltype(d)::value;
+    attn_train_dq_kernel<DD>
+        <<<dim3(B * Hkv, (T * a.G + 127) / 128), 256, 0, stream()>>>(a);
+    attn_train_dkv_kernel<DD>
+        <<<dim3(B * Hkv, (T + 63) / 64), 256, 0, stream()>>>(a);
+  });
+  check_launch();
+  return dqkv;
+}
+
+Tensor rms_norm_grad(Tensor x, Tensor w, Tensor gy, OptTensor gx, double eps) {
+  CHECK_T(x, at::kBFloat16);
+  CHECK_T(w, at::kBFloat16);
+  CHECK_T(gy, at::kBFloat16);
+  const long H = x.size(-1);
+  TORCH_CHECK(H % 8 == 0 && H <= 16384 && w.numel() == H &&
+                  gy.numel() == x.numel(),
+              "bad norm shapes");
+  if (gx.has_value()) {
+    CHECK_T((*gx), at::kBFloat16);
+    TORCH_CHECK(gx->numel() == x.numel());
+  }
+  Tensor dx = torch::empty_like(x);
+  if (x.numel() == 0) return dx;
+  auto launch = [&](auto it) {
+    rms_norm_grad_kernel<decltype(it)::value>
+        <<<x.numel() / H, 256, 0, stream()>>>(
+            in(x), in(w), in(gy), gx.has_value() ? in(*gx) : nullptr, out(dx), H,
+            (float)eps);
+  };
+  if (H <= 2048) launch(std::integral_constant<int, 1>{});
+  else if (H <= 4096) launch(std::integral_constant<int, 2>{});
+  else if (H <= 8192) launch(std::integral_constant<int, 4>{});
+  else launch(std::integral_constant<int, 8>{});
+  check_launch();
+  return dx;
+}
+
+Tensor swiglu_grad(Tensor gu, Tensor gm) {
+  CHECK_T(gu, at::kBFloat16);
+  CHECK_T(gm, at::kBFloat16);
+  const long I = gm.size(-1);
+  TORCH_CHECK(I % 8 == 0 && gu.size(-1) == 2 * I && gu.numel() == 2 * gm.numel(),
+              "bad product shapes");
+  Tensor dgu = torch::empty_like(gu);
+  if (gm.numel() == 0) return dgu;
+  const long N = gm.numel() / I;
+  swiglu_grad_kernel<<<std::min<long>((N * I / 8 + 255) / 256, 4096), 256, 0,
+                       stream()>>>(in(gu), in(gm), out(dgu), N, I);
+  check_launch();
+  return dgu;
+}
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("rope_attention", &rope_attention);
+  m.def("rope_attention_grad", &rope_attention_grad);
+  m.def("rms_norm_grad", &rms_norm_grad);
+  m.def("swiglu_grad", &swiglu_grad);
+}

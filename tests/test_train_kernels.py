@@ -1,0 +1,190 @@
+"""Fused steps of the training path against their plain forms: both are compared with
+the plain form in 64 bits, and the fused one may be no further away."""
+import pytest
+import torch
+
+from bloombee_amd import ops
+from bloombee_amd.ops import training
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def draw(*shape, seed=0, scale=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=gen) * scale).to(torch.bfloat16).to(DEV)
+
+
+def away(x, exact):
+    return float((x.double() - exact).norm() / exact.norm().clamp_min(1e-30))
+
+
+def check(fused, plain, exact):
+    """Both round their results to bf16; a tenth more covers another order of
+    rounding, 1e-6 results that are exact."""
+    for f, p, e in zip(fused, plain, exact):
+        assert f.shape == p.shape and f.dtype == p.dtype
+        assert away(f, e) <= 1.1 * away(p, e) + 1e-6, (away(f, e), away(p, e))
+
+
+def grads(f, xs, gs, dtype=None):
+    xs = [x.detach().to(dtype or x.dtype).requires_grad_(True) for x in xs]
+    out = f(*xs)
+    out = out if isinstance(out, tuple) else (out,)
+    return [*out, *torch.autograd.grad(out, xs, [g.to(o.dtype) for g, o
+                                                 in zip(gs, out)])]
+
+
+def attention(Hq, Hkv, D, T, start):
+    cos, sin = ops.rope_cos_sin(D, start + T + 3)
+    cos, sin = cos.to(DEV), sin.to(DEV)
+    scale = D ** -0.5
+    fused = lambda x: training.rope_attention(x, cos, sin, Hq, Hkv, start, scale)
+    plain = lambda x: training._attention(x, cos, sin, Hq, Hkv, start, scale)
+
+    def exact(x):
+        B, X = x.shape[0], Hq + 2 * Hkv
+        q, k, v = x.view(B, T, X, D).split([Hq, Hkv, Hkv], 2)
+        c, s = (t[start:start + T, None].double() for t in (cos, sin))
+
+        def rot(t):
+            a, b = t.chunk(2, -1)
+            return torch.cat([a * c - b * s, b * c + a * s], -1)
+
+        q, k = rot(q), rot(k).repeat_interleave(Hq // Hkv, 2)
+        v = v.repeat_interleave(Hq // Hkv, 2)
+        sc = torch.einsum("bthd,bshd->bhts", q, k) * scale
+        i = torch.arange(T, device=DEV)
+        p = torch.softmax(sc.masked_fill(i > i[:, None], float("-inf")), -1)
+        return torch.einsum("bhts,bshd->bthd", p, v).reshape(B, T, Hq * D)
+
+    return fused, plain, exact
+
+
+@pytest.mark.parametrize("case", [
+    # B, Hq, Hkv, D, T, start: rows (token, head of the group) go in tiles of 128
+    # and 64, keys in tiles of 64 and 32
+    (1, 4, 4, 128, 1, 0), (1, 4, 1, 128, 2, 0), (2, 8, 2, 128, 31, 5),
+    (1, 8, 2, 128, 32, 0), (3, 8, 2, 128, 33, 0), (1, 2, 2, 64, 63, 0),
+    (2, 6, 2, 64, 64, 7), (1, 4, 2, 128, 65, 0), (1, 4, 4, 64, 128, 0),
+    (1, 4, 4, 128, 129, 1), (2, 12, 4, 128, 200, 0), (1, 32, 8, 128, 515, 0),
+], ids=lambda c: "-".join(map(str, c)))
+def test_attention(case):
+    B, Hq, Hkv, D, T, start = case
+    x = draw(B, T, (Hq + 2 * Hkv) * D, seed=T)
+    g = draw(B, T, Hq * D, seed=T + 1)
+    fused, plain, exact = attention(Hq, Hkv, D, T, start)
+    assert training._fused(x)
+    check(grads(fused, [x], [g]), grads(plain, [x], [g]),
+          grads(exact, [x], [g], torch.float64))
+    with torch.no_grad():
+        assert torch.equal(fused(x), fused(x.clone().requires_grad_(True)))
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (3, 5, 256), (7, 2056), (2, 3, 4096),
+                                   (5, 16384)], ids=str)
+def test_norms(shape):
+    x, a = draw(*shape, seed=1), draw(*shape, seed=2)
+    w = draw(shape[-1], seed=3, scale=0.2) + 1
+    gh, gy = draw(*shape, seed=4), draw(*shape, seed=5)
+
+    def add_norm(f):
+        return lambda a, x: f(a, x, w, 1e-5)
+
+    def plain(a, x):
+        h = x + a
+        return h, training._rms(h, w, 1e-5)
+
+    def exact(a, x):
+        h = (x + a)
+        h = h + (h.bfloat16().double() - h).detach()   # the sum is a bf16 result
+        return h, h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+
+    check(grads(add_norm(training.add_norm), [a, x], [gh, gy]),
+          grads(plain, [a, x], [gh, gy]), grads(exact, [a, x], [gh, gy], torch.float64))
+    one = grads(lambda t: training.norm(t, w, 1e-5), [x], [gh, gy])
+    two = grads(lambda t: training.add_norm(torch.zeros_like(t), t, w, 1e-5), [x],
+                [gh, gy])
+    for u, v in zip(one, two):
+        assert torch.equal(u, v)
+
+
+@pytest.mark.parametrize("shape", [(1, 16), (5, 3, 528), (33, 28672)], ids=str)
+def test_swiglu(shape):
+    x = draw(*shape, seed=1, scale=2.0)
+    g = draw(*shape[:-1], shape[-1] // 2, seed=2)
+
+    def exact(t):
+        a, b = t.chunk(2, -1)
+        return torch.nn.functional.silu(a) * b
+
+    check(grads(training.swiglu, [x], [g]), grads(training._swiglu, [x], [g]),
+          grads(exact, [x], [g], torch.float64))
+
+
+def steps():
+    """Every fused step as a function of one bf16 tensor."""
+    w = draw(768, seed=9, scale=0.2) + 1
+    fused, plain, _ = attention(4, 1, 128, 9, 0)
+    x = draw(2, 9, 768, seed=3)
+    return {"attention": (fused, plain, x),
+            "norm": (lambda t: sum(training.norm(t, w, 1e-5)),
+                     lambda t: t + training._rms(t, w, 1e-5), x),
+            "swiglu": (training.swiglu, training._swiglu, x)}
+
+
+@pytest.mark.parametrize("name", ["attention", "norm", "swiglu"])
+def test_watched_operations_stay_plain(name):
+    """What looks into the operations gets the plain form's answer."""
+    fused, plain, x = steps()[name]
+    t = draw(*x.shape, seed=4)
+
+    def same(a, b):
+        # both bf16, a value of another order of rounding apart
+        assert a.shape == b.shape
+        assert away(a.float(), b.double()) < 0.02
+
+    # gradients of gradients
+    def twice(f):
+        y = x.clone().requires_grad_(True)
+        g, = torch.autograd.grad(f(y).float().square().sum(), y, create_graph=True)
+        return torch.autograd.grad((g.float() * t.float()).sum(), y)[0]
+    same(twice(fused), twice(plain))
+    # a batch of gradients at once
+    def batch(f):
+        y = x.clone().requires_grad_(True)
+        out = f(y)
+        gs = torch.stack([draw(*out.shape, seed=s) for s in (5, 6)])
+        return torch.autograd.grad(out, y, gs, is_grads_batched=True)[0]
+    same(batch(fused), batch(plain))
+    # forward mode, function transforms
+    with torch.autograd.forward_ad.dual_level():
+        d = [torch.autograd.forward_ad.unpack_dual(
+            f(torch.autograd.forward_ad.make_dual(x, t))).tangent
+            for f in (fused, plain)]
+    same(*d)
+    same(torch.func.vmap(fused)(x[None])[0], plain(x))
+    same(*[torch.func.grad(lambda y: f(y).float().sum())(x) for f in (fused, plain)])
+    # tracing
+    same(torch.jit.trace(fused, x, check_trace=False)(x), plain(x))
+    # saved tensors can be moved and come back
+    y = x.clone().requires_grad_(True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda v: v.cpu(),
+                                                  lambda v: v.to(DEV)):
+        out = fused(y)
+    z = x.clone().requires_grad_(True)
+    ref = fused(z)
+    g = draw(*out.shape, seed=7)
+    assert torch.equal(torch.autograd.grad(out, y, g)[0],
+                       torch.autograd.grad(ref, z, g)[0])
+    # rows that do not lie one after the other
+    wide = torch.cat([x, t], -1)[..., :x.shape[-1]]
+    assert torch.equal(fused(wide), fused(x))
+
+
+def test_trained_norm_weights_get_their_gradients():
+    x, w = draw(3, 256), (draw(256, seed=1) + 1).requires_grad_(True)
+    assert not training._fused(x, w)
+    h, y = training.norm(x, w, 1e-5)
+    assert torch.autograd.grad(y.sum(), w)[0].abs().sum() > 0
