@@ -119,6 +119,35 @@ class LlamaBlock(torch.nn.Module):
                                       device=device)
             self._ss_hidden = torch.empty_like(self._ss_h2)
 
+    def _input_stats(self, hidden, fuse_norm: bool):
+        """(row statistics of `hidden` for its fused norm or None, whether the
+        fused norm can run): a first block of many rows has no producer."""
+        if not fuse_norm:
+            return None, False
+        if not ops.row_stats_wanted(hidden):
+            return None, True
+        pb = getattr(self, "prev_block", None)
+        if pb is not None and getattr(pb, "_ss_valid", False):
+            return pb._ss_hidden, True
+        return None, False
+
+    def _fused_tail(self, hidden, attn) -> torch.Tensor:
+        """h2 = hidden + o(attn) via the GEMM's residual epilogue, which also
+        emits row sum-of-squares where the next norm wants them; the
+        post-attention rmsnorm and the gated product ride gate_up. down-proj
+        leaves the stats for the NEXT block's input norm."""
+        eps = self.config.rms_norm_eps
+        if not ops.row_stats_wanted(hidden):
+            h2 = ops.linear(attn, self.o_w, residual=hidden)
+            return ops.linear(ops.linear_swiglu(h2, self.gate_up_w, eps),
+                              self.down_w, residual=h2)
+        self._ensure_ss_bufs(hidden.device)
+        h2 = ops.linear(attn, self.o_w, residual=hidden, ss_out=self._ss_h2)
+        m = ops.linear_swiglu(h2, self.gate_up_w, eps, ss_in=self._ss_h2)
+        out = ops.linear(m, self.down_w, residual=h2, ss_out=self._ss_hidden)
+        self._ss_valid = True
+        return out
+
     @torch.no_grad()
     def fold_norm_weights(self):
         """Reparameterize for the fused-norm decode path: qkv_w <- qkv_w *
@@ -214,26 +243,18 @@ class LlamaBlock(torch.nn.Module):
         cfg = self.config
 
         # Decode-shaped GPU steps fold both per-layer rmsnorms into the
-        # skinny GEMM's A-operand stage (ops.linear norm=...): two fewer
-        # launches + elementwise passes per layer. The row sum-of-squares
-        # the norm needs is produced by the PRECEDING GEMM's epilogue
-        # (ss buffers chained block-to-block via prev_block; re-streaming
-        # A instead costs +18-60 us/GEMM — profiles/r02 §13). W4/LoRA
-        # blocks and prefill keep the separate-norm path.
+        # skinny GEMMs, the rotation with the K/V write into the first one and
+        # the gated product into the third: a launch there costs more than
+        # most of these steps do. Up to ops.STREAM_ROWS rows a GEMM sums up
+        # the squares its norm needs; beyond, they are produced by the
+        # PRECEDING GEMM's epilogue (ss buffers chained block-to-block via
+        # prev_block; re-streaming A instead costs +18-60 us/GEMM —
+        # profiles/r02 §13). W4/LoRA blocks and prefill keep the separate
+        # steps.
         fuse_norm = self._fuse_norm_gate(hidden)
         self._ss_valid = False
         if fuse_norm and not getattr(self, "_norm_folded", False):
             self.fold_norm_weights()   # one-time reparameterization
-        pb = getattr(self, "prev_block", None)
-        if fuse_norm and pb is not None and getattr(pb, "_ss_valid", False):
-            # previous block's down-proj left sum-of-squares for `hidden`;
-            # norm weight is folded into qkv_w -> invr-only norm (mode 2)
-            qkv = ops.linear(hidden, self.qkv_w,
-                             norm=(None, cfg.rms_norm_eps),
-                             ss_in=pb._ss_hidden)
-        else:
-            x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
-            qkv = self._lin(x, self.qkv_w, "qkv_w")        # (B, T, (Hq+2Hkv)D)
         cos, sin = self.rope.get(hidden.device)
         kp = kv.k_pages(self.layer_index)
         vp = kv.v_pages(self.layer_index)
@@ -246,10 +267,18 @@ class LlamaBlock(torch.nn.Module):
             position_ids = (start_pos.view(B, 1) + off
                             + torch.arange(T, device=hidden.device)
                             .view(1, T)).int()
-        # fused RoPE + paged KV write on the raw GEMM output, then attention
+        # fused RoPE + paged KV write on the GEMM output, then attention
         # reads q in place and emits the O-projection input — no transposes
-        ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
-                           start_pos)
+        ss, ok = self._input_stats(hidden, fuse_norm)
+        if ok:
+            qkv = ops.linear_rope_kv(hidden, self.qkv_w, cfg.rms_norm_eps, ss,
+                                     Hq, Hkv, cos, sin, position_ids, kp, vp,
+                                     pt, start_pos)
+        else:
+            x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
+            qkv = self._lin(x, self.qkv_w, "qkv_w")    # (B, T, (Hq+2Hkv)D)
+            ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp,
+                               pt, start_pos)
         hp = (kv.host_prefix(self.layer_index)
               if hasattr(kv, "host_prefix") else None)
         if hp is not None:
@@ -262,32 +291,12 @@ class LlamaBlock(torch.nn.Module):
             attn = ops.attn_paged_mixed(q, kp, vp, pt, start_pos + T,
                                         hp[0], hp[1], self.scale)
             attn = attn.permute(0, 2, 1, 3).reshape(B, T, Hq * D_)
-        elif tree_mask is not None:
-            # tree-structured verify step (spec decoding): unfused q view +
-            # the tree-mask attention path
-            q = (qkv[..., : Hq * D].view(B, T, Hq, D)
-                 .permute(0, 2, 1, 3).contiguous())
-            attn = ops.attn_paged(q, kp, vp, pt, start_pos.long(), self.scale,
-                                  tree_mask=tree_mask)
-            attn = attn.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
         else:
+            # tree_mask: tree-structured verify step (spec decoding)
             attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos,
-                                      self.scale)
+                                      self.scale, tree_mask=tree_mask)
         if fuse_norm:
-            # h2 = hidden + o(attn) via the GEMM's residual epilogue, which
-            # also emits row sum-of-squares; the post-attention rmsnorm
-            # folds into the gate_up A-stage consuming them. down-proj
-            # leaves the stats for the NEXT block's input norm.
-            self._ensure_ss_bufs(hidden.device)
-            h2 = ops.linear(attn, self.o_w, residual=hidden,
-                            ss_out=self._ss_h2)
-            gu = ops.linear(h2, self.gate_up_w,
-                            norm=(None, cfg.rms_norm_eps),
-                            ss_in=self._ss_h2)
-            out = ops.linear(ops.swiglu(gu), self.down_w, residual=h2,
-                             ss_out=self._ss_hidden)
-            self._ss_valid = True
-            return out
+            return self._fused_tail(hidden, attn)
         a = self._lin(attn, self.o_w, "o_w")
 
         # h2 = hidden + a fused into the post-attention norm

@@ -41,22 +41,13 @@ class Qwen3Block(LlamaBlock):
         self._ss_valid = False
         if fuse_norm and not getattr(self, "_norm_folded", False):
             self.fold_norm_weights()
-        pb = getattr(self, "prev_block", None)
-        if fuse_norm and pb is not None and getattr(pb, "_ss_valid", False):
+        ss, ok = self._input_stats(hidden, fuse_norm)
+        if ok:
             qkv = ops.linear(hidden, self.qkv_w,
-                             norm=(None, cfg.rms_norm_eps),
-                             ss_in=pb._ss_hidden)
+                             norm=(None, cfg.rms_norm_eps), ss_in=ss)
         else:
             x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
             qkv = self._lin(x, self.qkv_w, "qkv_w")
-        # per-head q/k RMS norm on the fused buffer (contiguous D-sized rows)
-        qk = qkv[..., :(Hq + Hkv) * D]
-        q_flat = qkv[..., :Hq * D].reshape(-1, D)
-        k_flat = qkv[..., Hq * D:(Hq + Hkv) * D].reshape(-1, D)
-        qkv[..., :Hq * D] = ops.rms_norm(q_flat, self.q_norm_w,
-                                         cfg.rms_norm_eps).view(B, T, Hq * D)
-        qkv[..., Hq * D:(Hq + Hkv) * D] = ops.rms_norm(
-            k_flat, self.k_norm_w, cfg.rms_norm_eps).view(B, T, Hkv * D)
         cos, sin = self.rope.get(hidden.device)
         kp = kv.k_pages(self.layer_index)
         vp = kv.v_pages(self.layer_index)
@@ -68,8 +59,10 @@ class Qwen3Block(LlamaBlock):
             position_ids = (start_pos.view(B, 1) + off
                             + torch.arange(T, device=hidden.device)
                             .view(1, T)).int()
+        # the per-head q/k norms run ahead of the rotation in its launch
         ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
-                           start_pos)
+                           start_pos, head_norms=(self.q_norm_w, self.k_norm_w,
+                                                  cfg.rms_norm_eps))
         hp = (kv.host_prefix(self.layer_index)
               if hasattr(kv, "host_prefix") else None)
         if hp is not None:
@@ -82,15 +75,7 @@ class Qwen3Block(LlamaBlock):
             attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos,
                                       self.scale)
         if fuse_norm:
-            self._ensure_ss_bufs(hidden.device)
-            h2 = ops.linear(attn, self.o_w, residual=hidden,
-                            ss_out=self._ss_h2)
-            gu = ops.linear(h2, self.gate_up_w,
-                            norm=(None, cfg.rms_norm_eps), ss_in=self._ss_h2)
-            out = ops.linear(ops.swiglu(gu), self.down_w, residual=h2,
-                             ss_out=self._ss_hidden)
-            self._ss_valid = True
-            return out
+            return self._fused_tail(hidden, attn)
         a = self._lin(attn, self.o_w, "o_w")
         h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
         return self._lin(ops.swiglu(self._lin(y, self.gate_up_w, "gate_up_w")),

@@ -19,6 +19,8 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     kv_write,
     layer_norm,
     linear,
+    linear_rope_kv,
+    linear_swiglu,
     linear_w4,
     mfma_selftest,
     moe_gemm_grouped,
@@ -29,6 +31,7 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     rope_apply_,
     rope_kv_write_,
     rope_cos_sin,
+    row_stats_wanted,
     set_attn_sparsity,
     swiglu,
 )

@@ -55,44 +55,61 @@ DEVINL void store_bf16_e(unsigned short* p, const float* in) {
 }
 
 
-// Combine n_split partials. grid = (B*Hkv), block = G*16 (<= 128 threads).
+// Combine n_split partials: a wave a row (unit, head of the chunk), grid
+// ceil(units * maxg / 4). Lanes read the splits' maxima and sums at once and share
+// out the weights, so that the loads of the values do not wait for one another
+// (32 splits: 15 us in a decode step when they did, about 5 now, which is a launch).
 template <int D>
-__global__ void attn_decode_combine_kernel(
+__global__ __launch_bounds__(256) void attn_decode_combine_kernel(
     const float* __restrict__ part_ml, const float* __restrict__ part_acc,
-    unsigned short* __restrict__ out, int Hkv, int G, int nch, int maxg,
+    unsigned short* __restrict__ out, int units, int Hkv, int G, int nch, int maxg,
     int n_split, long out_sb, long out_sh) {
-  constexpr int E = D / 16;
-  const int bh = blockIdx.x;           // (b, kvh, chunk)
+  constexpr int E = D >= 128 ? D / 64 : 1;   // columns of a lane
+  const int row = blockIdx.x * 4 + threadIdx.x / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int bh = row / maxg, g = row % maxg;   // bh: (b, kvh, chunk)
+  if (bh >= units) return;
   const int b = bh / (Hkv * nch);
   const int rem = bh % (Hkv * nch);
   const int kvh = rem / nch;
   const int g0 = (rem % nch) * maxg;
-  const int g = threadIdx.x / 16;
-  const int li = threadIdx.x & 15;
-  if (g0 + g >= G || g >= maxg) return;
-  float m2 = NEG_BIG, l = 0.f, acc[E];
+  if (g0 + g >= G) return;
+  const float* ml = part_ml + ((long)bh * n_split * maxg + g) * 2;
+  float m = NEG_BIG;
+  for (int s = lane; s < n_split; s += WAVE)
+    if (ml[(long)s * maxg * 2 + 1] != 0.f) m = fmaxf(m, ml[(long)s * maxg * 2]);
+  m = wave_reduce_max(m);
+  float l = 0.f, acc[E];
 #pragma unroll
   for (int j = 0; j < E; ++j) acc[j] = 0.f;
-  for (int s = 0; s < n_split; ++s) {
-    const long pbase = (long)bh * n_split + s;
-    const float mo = part_ml[(pbase * maxg + g) * 2 + 0];
-    const float lo = part_ml[(pbase * maxg + g) * 2 + 1];
-    if (lo == 0.f) continue;
-    const float mn = fmaxf(m2, mo);
-    const float c1f = fast_exp2(m2 - mn);
-    const float c2f = fast_exp2(mo - mn);
-    l = l * c1f + lo * c2f;
+  const int col = min(lane * E, D - E);
+  const float* pa = part_acc + ((long)bh * n_split * maxg + g) * D + col;
+  for (int s0 = 0; s0 < n_split; s0 += WAVE) {
+    const int s = s0 + lane;
+    float w = 0.f;
+    if (s < n_split) {
+      const float ls = ml[(long)s * maxg * 2 + 1];
+      // splits beyond the context have no sum; their values are zero
+      if (ls != 0.f) {
+        w = fast_exp2(ml[(long)s * maxg * 2] - m);
+        l += w * ls;
+      }
+    }
+    const int n = min(WAVE, n_split - s0);
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) {
+      const float wi = __shfl(w, i);
 #pragma unroll
-    for (int j = 0; j < E; ++j)
-      acc[j] = acc[j] * c1f + part_acc[(pbase * maxg + g) * D + li * E + j] * c2f;
-    m2 = mn;
+      for (int j = 0; j < E; ++j)
+        acc[j] += wi * pa[(long)(s0 + i) * maxg * D + j];
+    }
   }
-  float o[E];
+  l = wave_reduce_sum(l);
+  if (lane * E >= D) return;
   const float inv = (l > 0.f) ? 1.f / l : 0.f;
+  unsigned short* o = out + (long)b * out_sb + (kvh * G + g0 + g) * out_sh + col;
 #pragma unroll
-  for (int j = 0; j < E; ++j) o[j] = acc[j] * inv;
-  store_bf16_e<E>(out + (long)b * out_sb + (kvh * G + g0 + g) * out_sh + li * E,
-                  o);
+  for (int j = 0; j < E; ++j) o[j] = f2bf(acc[j] * inv);
 }
 
 // Pure-streaming probe: same grid/walk/loads as attn_decode_kernel but no

@@ -76,7 +76,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
     float* __restrict__ part_ml,                 // (B*Hkv*nch*n_split, MAXG, 2)
     float* __restrict__ part_acc,                // (..., MAXG, D)
     int B, int Hkv, int G, int nch, int P, int maxp, int n_split, int window,
-    float scale, long q_sb, long q_sh, long out_sb, long out_sh) {
+    float scale, long q_sb, long q_sh, long out_sb, long out_sh, int ctx_add,
+    int share) {
   constexpr int NKK = D / 32;   // QK^T k-slices
   constexpr int NDT = D / 16;   // PV d-tiles
   constexpr int NPT = DKVBLK / 16;  // position tiles per KV tile
@@ -89,10 +90,12 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
   const int kvh = rem / nch;
   const int g0 = (rem % nch) * MAXG;   // this chunk's first group col
   const int Gl = min(G - g0, MAXG);    // live head cols in this chunk
-  const int ctx = ctx_lens[b];
+  const int ctx = ctx_lens[b] + ctx_add;
 
   const int pages_total = (ctx + P - 1) / P;
-  const int pages_per_split = (pages_total + n_split - 1) / n_split;
+  // no split shorter than `share` tokens: a short context takes fewer splits
+  const int parts = min(n_split, max(1, (ctx + share - 1) / share));
+  const int pages_per_split = (pages_total + parts - 1) / parts;
   const int c0 = split * pages_per_split * P;
   const int c1 = min(ctx, c0 + pages_per_split * P);
   int lo = 0;
@@ -450,7 +453,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_wide_kernel(
     const float* __restrict__ alibi, unsigned short* __restrict__ out,
     float* __restrict__ part_ml, float* __restrict__ part_acc,
     int B, int Hkv, int G, int nch, int P, int maxp, int n_split, int window,
-    float scale, long q_sb, long q_sh, long out_sb, long out_sh) {
+    float scale, long q_sb, long q_sh, long out_sb, long out_sh, int ctx_add,
+    int share) {
   constexpr int D = 512;
   constexpr int NKK_W = 4;          // QK k-slices per wave (128 d)
   constexpr int NDT_W = 8;          // PV d-tiles per wave (128 d)
@@ -464,10 +468,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_wide_kernel(
   const int kvh = rem / nch;
   const int g0 = (rem % nch) * MAXG;
   const int Gl = min(G - g0, MAXG);
-  const int ctx = ctx_lens[b];
+  const int ctx = ctx_lens[b] + ctx_add;
 
   const int pages_total = (ctx + P - 1) / P;
-  const int pages_per_split = (pages_total + n_split - 1) / n_split;
+  const int parts = min(n_split, max(1, (ctx + share - 1) / share));
+  const int pages_per_split = (pages_total + parts - 1) / parts;
   const int c0 = split * pages_per_split * P;
   const int c1 = min(ctx, c0 + pages_per_split * P);
   int lo = 0;

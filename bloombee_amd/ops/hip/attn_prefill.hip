@@ -306,27 +306,36 @@ __global__ __launch_bounds__(256) void attn_prefill_fold_kernel(PrefillArgs a) {
   const long rows = (long)units * R;
   const long at = (long)blockIdx.x * 4 + threadIdx.x / WAVE;
   const int lane = threadIdx.x & (WAVE - 1);
-  if (at >= rows || lane * V >= D) return;
-  float m = NEG_BIG;
-  for (int s = 0; s < a.n_split; ++s)
-    m = fmaxf(m, a.pml[(s * rows + at) * 2]);
-  float l = 0.f, o[V];
+  if (at >= rows) return;
+  // lanes read the splits' maxima and sums at once and share out the weights
+  // (n_split <= 32), so that the loads of the values do not wait for one another
+  float m = NEG_BIG, l = 0.f, w = 0.f;
+  if (lane < a.n_split) {
+    m = a.pml[(lane * rows + at) * 2];
+    l = a.pml[(lane * rows + at) * 2 + 1];
+    if (!(l > 0.f)) m = NEG_BIG;
+  }
+  const float top = wave_reduce_max(m);
+  if (l > 0.f) w = fast_exp2(m - top);
+  l = wave_reduce_sum(w * l);
+  const int col = min(lane * V, D - V);
+  float o[V];
 #pragma unroll
   for (int e = 0; e < V; ++e) o[e] = 0.f;
+#pragma unroll 8
   for (int s = 0; s < a.n_split; ++s) {
-    const float ls = a.pml[(s * rows + at) * 2 + 1];
-    if (!(ls > 0.f)) continue;
-    const float w = fast_exp2(a.pml[(s * rows + at) * 2] - m);
-    l += w * ls;
-    const float* p = a.pacc + (s * rows + at) * D + lane * V;
+    const float ws = __shfl(w, s);
+    if (ws == 0.f) continue;
+    const float* p = a.pacc + (s * rows + at) * D + col;
 #pragma unroll
-    for (int e = 0; e < V; ++e) o[e] += w * p[e];
+    for (int e = 0; e < V; ++e) o[e] += ws * p[e];
   }
+  if (lane * V >= D) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
   const int unit = (int)(at / R), r = (int)(at % R);
   unsigned short* op = a.out + (long)(unit / a.Hkv) * a.o_sb +
                        (long)(r / a.G) * a.o_st +
-                       (long)(unit % a.Hkv * a.G + r % a.G) * a.o_sh + lane * V;
+                       (long)(unit % a.Hkv * a.G + r % a.G) * a.o_sh + col;
 #pragma unroll
   for (int e = 0; e < V; ++e) op[e] = f2bf(o[e] * inv);
 }

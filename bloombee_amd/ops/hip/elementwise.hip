@@ -225,6 +225,7 @@ __global__ void add_kernel(const unsigned short* __restrict__ a,
 // q heads: rotary in place. k heads: rotary -> k_pages (never written back).
 // v heads: straight copy -> v_pages. One launch replaces rope + kv_write and
 // removes every transpose copy between the QKV GEMM and attention.
+// q_norm, k_norm: weights of an RMS norm of every head ahead of its rotation, or null.
 // grid: (B*T, Hq+2Hkv), block: 64.
 // ---------------------------------------------------------------------------
 
@@ -233,7 +234,9 @@ __global__ void rope_kv_write_kernel(
     const float* __restrict__ sin_t, const int* __restrict__ pos,
     unsigned short* __restrict__ k_pages, unsigned short* __restrict__ v_pages,
     const int* __restrict__ page_table, const int* __restrict__ start_pos,
-    int B, int Hq, int Hkv, int T, int D, int P, int maxp, int max_pos) {
+    int B, int Hq, int Hkv, int T, int D, int P, int maxp, int max_pos,
+    const unsigned short* __restrict__ q_norm,
+    const unsigned short* __restrict__ k_norm, float eps) {
   const int bt = blockIdx.x;
   const int b = bt / T, t = bt % T;
   const int h = blockIdx.y;
@@ -259,8 +262,22 @@ __global__ void rope_kv_write_kernel(
     const int page = page_table[b * maxp + abspos / P];
     dst = k_pages + (((long)page * Hkv + hk) * P + (abspos % P)) * D;
   }
+  const unsigned short* nw = h < Hq ? q_norm : k_norm;
+  float r = 1.f;
+  if (nw) {
+    float sq = 0.f;
+    for (int i = threadIdx.x; i < D; i += blockDim.x) {
+      const float x = bf2f(base[i]);
+      sq += x * x;
+    }
+    r = rsqrtf(wave_reduce_sum(sq) / (float)D + eps);
+  }
   for (int i = threadIdx.x; i < D / 2; i += blockDim.x) {
     float x1 = bf2f(base[i]), x2 = bf2f(base[i + D / 2]);
+    if (nw) {
+      x1 *= r * bf2f(nw[i]);
+      x2 *= r * bf2f(nw[i + D / 2]);
+    }
     float cc = c[i], ss = s[i];
     dst[i] = f2bf(x1 * cc - x2 * ss);
     dst[i + D / 2] = f2bf(x2 * cc + x1 * ss);

@@ -17,6 +17,7 @@
 #include "attn_decode_mfma.hip"
 #include "attn_prefill.hip"
 #include "gemm_skinny.hip"
+#include "gemm_stream.hip"
 #include "moe_gemm.hip"
 #include "w4_gemm.hip"
 #include "mfma_selftest.hip"
@@ -203,7 +204,8 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
                                torch::Tensor& pml, torch::Tensor& pacc, int B,
                                int Hkv, int G, int nch, int P, int maxp,
                                int n_split, int window, float scale, long q_off,
-                               long q_sb, long q_sh, long out_sb, long out_sh) {
+                               long q_sb, long q_sh, long out_sb, long out_sh,
+                               int ctx_add, int share) {
   dim3 grid(B * Hkv * nch, n_split);
   const int maxg = (G <= 4 && nch == 1) ? 4 : 16;
   // paired-tile variant (NT=2): 2x KV bytes in flight per wave — the
@@ -231,37 +233,42 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
               bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
               ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
               pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
-              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh);
+              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
+              share);
     } else if (D <= 128 && pf) {
       attn_decode_mfma_kernel<D, decltype(mg)::value, 1, 1>
           <<<grid, 256, 0, cur_stream()>>>(
               bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
               ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
               pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
-              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh);
+              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
+              share);
     } else if (D <= 128 && nt2) {
       attn_decode_mfma_kernel<D, decltype(mg)::value, 2>
           <<<grid, 256, 0, cur_stream()>>>(
               bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
               ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
               pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
-              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh);
+              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
+              share);
     } else {
       attn_decode_mfma_kernel<D, decltype(mg)::value, 1>
           <<<grid, 256, 0, cur_stream()>>>(
               bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
               ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
               pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
-              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh);
+              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
+              share);
     }
   };
   if (maxg == 4) launch_mfma(std::integral_constant<int, 4>{});
   else launch_mfma(std::integral_constant<int, 16>{});
   if (n_split > 1) {
+    const int units = B * Hkv * nch;
     attn_decode_combine_kernel<D>
-        <<<B * Hkv * nch, maxg * 16, 0, cur_stream()>>>(
+        <<<(units * maxg + 3) / 4, 256, 0, cur_stream()>>>(
             pml.data_ptr<float>(), pacc.data_ptr<float>(), bf_ptr_mut(out),
-            Hkv, G, nch, maxg, n_split, out_sb, out_sh);
+            units, Hkv, G, nch, maxg, n_split, out_sb, out_sh);
   }
 }
 
@@ -271,7 +278,7 @@ static torch::Tensor attn_decode_core(
     const torch::Tensor& ctx_lens, const c10::optional<torch::Tensor>& alibi,
     double scale, long window, long n_split_req,
     int B, int Hq, int D, long q_off, long q_sb, long q_sh,
-    torch::Tensor out, long out_sb, long out_sh) {
+    torch::Tensor out, long out_sb, long out_sh, int ctx_add = 0) {
   const int Hkv = k_pages.size(1), P = k_pages.size(2), maxp = page_table.size(1);
   const int G = Hq / Hkv;
   TORCH_CHECK(Hq % Hkv == 0);
@@ -283,6 +290,7 @@ static torch::Tensor attn_decode_core(
     alibi_ptr = alibi->data_ptr<float>();
   }
   int n_split = (int)n_split_req;
+  int share = n_split > 0 ? 1 : 128;   // least tokens of a split
   if (n_split <= 0) {
     // measured optimum (benchmarks/bench_kernels.py attn_decode): size the
     // grid for full residency — NT=1 runs 118 VGPRs -> 4 WGs/CU (1024 WGs),
@@ -300,8 +308,19 @@ static torch::Tensor attn_decode_core(
     // (measured: B32 ns=2 50 us / 5.4 TB/s vs 59 at 768-1024 WGs)
     const long target = (pf_env0 && D <= 128) ? 512
                         : (nt_env0 >= 2 && D <= 128) ? 768 : 1024;
-    n_split = (int)std::max<long>(
-        1, std::min<long>(32, target / std::max(1, B * Hkv * nch)));
+    const long units = std::max(1, B * Hkv * nch), room = (long)maxp * P;
+    if (units > target) {
+      // More units than fit at once: contexts of a large batch differ, and a
+      // workgroup with a long one outlasts the rest. Shares of 1024 tokens even it
+      // out (97 sequences of 64 to 4000 tokens, 8 heads of 128: 183 us unsplit,
+      // 152 us so).
+      share = 1024;
+      n_split = (int)std::min(32L, (room + share - 1) / share);
+    } else {
+      // a wave takes 32 tokens at a time, a workgroup 128: shorter splits idle
+      // most of its waves
+      n_split = (int)std::max(1L, std::min({32L, target / units, room / share}));
+    }
   }
   const int maxg = (G <= 4 && nch == 1) ? 4 : 16;
   auto fopt = torch::TensorOptions().device(q.device()).dtype(at::kFloat);
@@ -317,7 +336,7 @@ static torch::Tensor attn_decode_core(
     attn_decode_launch<decltype(d)::value>(
         q, k_pages, v_pages, page_table, ctx_lens, alibi_ptr, out, pml, pacc,
         B, Hkv, G, nch, P, maxp, n_split, (int)window, (float)scale, q_off,
-        q_sb, q_sh, out_sb, out_sh);
+        q_sb, q_sh, out_sb, out_sh, ctx_add, share);
   };
   if (D == 128) go(std::integral_constant<int, 128>{});
   else if (D == 64) go(std::integral_constant<int, 64>{});
@@ -346,11 +365,12 @@ torch::Tensor attn_decode(torch::Tensor q, torch::Tensor k_pages,
 }
 
 // Fused-QKV decode: q section of qkv (B, 1, (Hq+2Hkv)*D) read in place,
-// out (B, 1, Hq*D) ready for the O-projection GEMM — zero transposes.
+// out (B, 1, Hq*D) ready for the O-projection GEMM — zero transposes. A context is
+// ctx_lens + ctx_add tokens.
 torch::Tensor attn_decode_qkv(torch::Tensor qkv, long Hq, torch::Tensor k_pages,
                               torch::Tensor v_pages, torch::Tensor page_table,
                               torch::Tensor ctx_lens, double scale, long window,
-                              long n_split_req) {
+                              long n_split_req, long ctx_add) {
   CHECK_DEV(qkv); CHECK_BF16(qkv); CHECK_CONTIG(qkv);
   CHECK_DEV_ALL3(k_pages, page_table, ctx_lens);
   const int Hkv = k_pages.size(1);
@@ -362,7 +382,7 @@ torch::Tensor attn_decode_qkv(torch::Tensor qkv, long Hq, torch::Tensor k_pages,
   return attn_decode_core(qkv, k_pages, v_pages, page_table, ctx_lens,
                           c10::nullopt, scale, window, n_split_req, B, (int)Hq,
                           D, /*q_off*/ 0, (long)(Hq + 2 * Hkv) * D, (long)D,
-                          out, (long)Hq * D, (long)D)
+                          out, (long)Hq * D, (long)D, (int)ctx_add)
       .view({B, 1, Hq * D});
 }
 
@@ -419,6 +439,18 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   else by_dim(std::false_type{});
 }
 
+static void set_tree_mask(PrefillArgs& a, const c10::optional<torch::Tensor>& mask,
+                          int B, int Tq, long window) {
+  if (!mask.has_value()) return;
+  TORCH_CHECK(mask->scalar_type() == at::kBool && mask->is_contiguous() &&
+                  mask->sizes() == (at::IntArrayRef{B, Tq, Tq}),
+              "tree_mask must be contiguous bool (B, Tq, Tq)");
+  TORCH_CHECK(window == 0, "tree_mask + sliding window: use the torch path");
+  CHECK_DEV((*mask));
+  // kBool tensors dispatch data_ptr<bool>, not <unsigned char> (Byte)
+  a.tree_mask = reinterpret_cast<const unsigned char*>(mask->data_ptr<bool>());
+}
+
 torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
                            torch::Tensor v_pages, torch::Tensor page_table,
                            torch::Tensor q_start, double scale, long window,
@@ -435,17 +467,7 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
     TORCH_CHECK(alibi->scalar_type() == at::kFloat && alibi->numel() == Hq);
     a.alibi = alibi->data_ptr<float>();
   }
-  if (tree_mask.has_value()) {
-    TORCH_CHECK(tree_mask->scalar_type() == at::kBool &&
-                tree_mask->is_contiguous() &&
-                tree_mask->sizes() == (at::IntArrayRef{B, Tq, Tq}),
-                "tree_mask must be contiguous bool (B, Tq, Tq)");
-    TORCH_CHECK(window == 0, "tree_mask + sliding window: use the torch path");
-    CHECK_DEV((*tree_mask));
-    // kBool tensors dispatch data_ptr<bool>, not <unsigned char> (Byte)
-    a.tree_mask = reinterpret_cast<const unsigned char*>(
-        tree_mask->data_ptr<bool>());
-  }
+  set_tree_mask(a, tree_mask, B, Tq, window);
   auto out = torch::empty_like(q);
   a.q = bf_ptr(q);
   a.k_pages = bf_ptr(k_pages);
@@ -468,7 +490,8 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
 torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
                                torch::Tensor k_pages, torch::Tensor v_pages,
                                torch::Tensor page_table, torch::Tensor q_start,
-                               double scale, long window) {
+                               double scale, long window,
+                               c10::optional<torch::Tensor> tree_mask) {
   CHECK_DEV(qkv); CHECK_BF16(qkv); CHECK_CONTIG(qkv);
   CHECK_DEV_ALL3(k_pages, page_table, q_start);
   const int Hkv = k_pages.size(1), P = k_pages.size(2), D = k_pages.size(3);
@@ -479,6 +502,7 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
   TORCH_CHECK(qkv.dim() == 3 && qkv.size(2) == (long)X * D, "bad fused qkv shape");
   auto out = torch::empty({B, Tq, (long)Hq * D}, qkv.options());
   PrefillArgs a{};
+  set_tree_mask(a, tree_mask, B, Tq, window);
   a.q = bf_ptr(qkv);
   a.k_pages = bf_ptr(k_pages);
   a.v_pages = bf_ptr(v_pages);
@@ -501,7 +525,9 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
 void rope_kv_write_(torch::Tensor qkv, long Hq_, long Hkv_, torch::Tensor cos_t,
                     torch::Tensor sin_t, c10::optional<torch::Tensor> pos,
                     torch::Tensor k_pages, torch::Tensor v_pages,
-                    torch::Tensor page_table, torch::Tensor start_pos) {
+                    torch::Tensor page_table, torch::Tensor start_pos,
+                    c10::optional<torch::Tensor> q_norm,
+                    c10::optional<torch::Tensor> k_norm, double eps) {
   CHECK_DEV(qkv); CHECK_BF16(qkv); CHECK_CONTIG(qkv);
   CHECK_DEV_ALL3(k_pages, page_table, start_pos);
   CHECK_DEV_ALL2(cos_t, sin_t);
@@ -516,12 +542,22 @@ void rope_kv_write_(torch::Tensor qkv, long Hq_, long Hkv_, torch::Tensor cos_t,
     TORCH_CHECK(pos->scalar_type() == at::kInt);
     pos_ptr = pos->data_ptr<int>();
   }
+  const unsigned short* norms[2] = {nullptr, nullptr};
+  const c10::optional<torch::Tensor>* given[2] = {&q_norm, &k_norm};
+  for (int i = 0; i < 2; ++i)
+    if (given[i]->has_value()) {
+      const torch::Tensor& w = **given[i];
+      TORCH_CHECK(w.is_cuda() && w.scalar_type() == at::kBFloat16 &&
+                      w.is_contiguous() && w.numel() == D,
+                  "head norm weights must be contiguous bf16 of length D");
+      norms[i] = bf_ptr(w);
+    }
   dim3 grid(B * T, Hq + 2 * Hkv);
   rope_kv_write_kernel<<<grid, 64, 0, cur_stream()>>>(
       bf_ptr_mut(qkv), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), pos_ptr,
       bf_ptr_mut(k_pages), bf_ptr_mut(v_pages), page_table.data_ptr<int>(),
       start_pos.data_ptr<int>(), B, Hq, Hkv, T, D, P, maxp,
-      (int)cos_t.size(0));
+      (int)cos_t.size(0), norms[0], norms[1], (float)eps);
 }
 
 
@@ -687,6 +723,180 @@ torch::Tensor gemm_w4(torch::Tensor A, torch::Tensor Wq, torch::Tensor scale,
 // ---------------------------------------------------------------------------
 // skinny-M GEMM (decode projections)
 // ---------------------------------------------------------------------------
+
+// Rows up to which the one-launch kernel (gemm_stream.hip) is the faster one: every
+// workgroup of it reads all of A, which eight rows keep small beside its 16 rows of W.
+// 4096 x 4096 9.1 us at 1 row, 11.0 at 16, 16.5 at 32 (split GEMM and its fold: 13.9,
+// 14.9, 15.1), 14336 x 4096 25, 35, 51 (30, 31, 32).
+static constexpr int STREAM_ROWS = 8;
+
+static StreamArgs stream_args(const torch::Tensor& A, const torch::Tensor& W) {
+  CHECK_DEV(A); CHECK_BF16(A); CHECK_CONTIG(A);
+  CHECK_DEV(W); CHECK_BF16(W); CHECK_CONTIG(W);
+  StreamArgs a{};
+  a.K = A.size(-1);
+  a.M = A.numel() / a.K;
+  a.N = W.size(0);
+  TORCH_CHECK(W.dim() == 2 && W.size(1) == a.K, "A/W K mismatch");
+  TORCH_CHECK(a.M >= 1 && a.M <= 32, "1 to 32 rows, got ", a.M);
+  a.A = bf_ptr(A);
+  a.W = bf_ptr(W);
+  return a;
+}
+
+static void check_stream(const StreamArgs& a) {
+  TORCH_CHECK(a.M <= STREAM_ROWS && a.K % 128 == 0, "up to ", STREAM_ROWS,
+              " rows and K%128 required");
+}
+
+// C(M,N) = A @ W^T [* 1/rms of A's rows] [+ bias] [+ residual], M <= STREAM_ROWS;
+// eps < 0: no norm.
+torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
+                          c10::optional<torch::Tensor> residual,
+                          c10::optional<torch::Tensor> bias, double eps) {
+  StreamArgs a = stream_args(A, W);
+  check_stream(a);
+  TORCH_CHECK(a.N % 16 == 0, "N%16 required");
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N;
+  auto C = torch::empty(sizes, A.options());
+  a.C = bf_ptr_mut(C);
+  a.eps = eps;
+  if (residual.has_value()) {
+    TORCH_CHECK(residual->is_cuda() && residual->scalar_type() == at::kBFloat16 &&
+                residual->is_contiguous() &&
+                residual->numel() == (long)a.M * a.N, "bad residual");
+    a.R = bf_ptr(*residual);
+  }
+  if (bias.has_value()) {
+    TORCH_CHECK(bias->is_cuda() && bias->scalar_type() == at::kBFloat16 &&
+                bias->is_contiguous() && bias->numel() == a.N, "bad bias");
+    a.bias = bf_ptr(*bias);
+  }
+  if (eps >= 0)
+    gemm_stream_kernel<EPI_SUM, 1, 1, true, 8, 4>
+        <<<a.N / 16, 512, 0, cur_stream()>>>(a);
+  else
+    gemm_stream_kernel<EPI_SUM, 1, 1, false, 8, 4>
+        <<<a.N / 16, 512, 0, cur_stream()>>>(a);
+  return C;
+}
+
+// Unsplit or split v2 GEMM of the fused forms below, norm mode 2.
+template <bool SWIGLU>
+static void launch_skinny_fused(const StreamArgs& a, const float* ss, int nstripes,
+                                int kchunk, int ksplit, float* part) {
+  const dim3 grid(a.N / 64, ksplit);
+  auto launch = [&](auto mt) {
+    gemm_skinny_v2_kernel<decltype(mt)::value, false, SWIGLU>
+        <<<grid, 256, 0, cur_stream()>>>(a.A, a.W, nullptr, nullptr, a.C, part, a.M,
+                                         a.N, a.K, kchunk, ksplit, nullptr, a.eps, 2,
+                                         ss, nstripes, nullptr);
+  };
+  if (a.M <= 16) launch(std::integral_constant<int, 1>{});
+  else launch(std::integral_constant<int, 2>{});
+}
+
+static const float* row_stats(const c10::optional<torch::Tensor>& ss, int* nstripes) {
+  if (!ss.has_value()) return nullptr;
+  TORCH_CHECK(ss->is_cuda() && ss->is_contiguous() &&
+              ss->scalar_type() == at::kFloat && ss->numel() % 32 == 0,
+              "ss_in must be f32 (nstripes,32)");
+  *nstripes = (int)(ss->numel() / 32);
+  return ss->data_ptr<float>();
+}
+
+// silu(gate) * up of [gate | up] = rms(A) @ W^T, norm weight folded into W; ss_in as
+// in gemm_skinny (used beyond STREAM_ROWS).
+torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps,
+                          c10::optional<torch::Tensor> ss_in) {
+  StreamArgs a = stream_args(A, W);
+  TORCH_CHECK(a.K % 256 == 0 && a.N % 64 == 0, "K%256, N%64 required");
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N / 2;
+  auto C = torch::empty(sizes, A.options());
+  a.C = bf_ptr_mut(C);
+  a.eps = eps;
+  int nstripes = 0;
+  const float* ss = row_stats(ss_in, &nstripes);
+  if (a.M <= STREAM_ROWS)
+    gemm_stream_kernel<EPI_SWIGLU, 2, 1, true, 4, 3>
+        <<<a.N / 32, 256, 0, cur_stream()>>>(a);
+  else
+    launch_skinny_fused<true>(a, ss, nstripes, a.K, 1, nullptr);
+  return C;
+}
+
+// [q | k | v] = rms(A) @ W^T with q turned in the result and k, v in their page slots
+// (their columns of the result stay unwritten). A (B, T, K), norm weight folded in.
+torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps,
+                           c10::optional<torch::Tensor> ss_in, long Hq, long Hkv,
+                           torch::Tensor cos_t, torch::Tensor sin_t,
+                           c10::optional<torch::Tensor> pos, torch::Tensor k_pages,
+                           torch::Tensor v_pages, torch::Tensor page_table,
+                           torch::Tensor start_pos) {
+  StreamArgs a = stream_args(A, W);
+  TORCH_CHECK(A.dim() == 3 && a.K % 256 == 0 && a.N % 64 == 0,
+              "(B, T, K) rows, K%256, N%64 required");
+  CHECK_DEV_ALL3(k_pages, v_pages, page_table);
+  CHECK_DEV_ALL3(cos_t, sin_t, start_pos);
+  CHECK_BF16(k_pages); CHECK_BF16(v_pages);
+  CHECK_CONTIG(k_pages); CHECK_CONTIG(v_pages); CHECK_CONTIG(page_table);
+  a.T = A.size(1);
+  a.Hq = Hq; a.Hkv = Hkv;
+  a.P = k_pages.size(2); a.D = k_pages.size(3);
+  a.maxp = page_table.size(1);
+  TORCH_CHECK(a.D % 32 == 0 && a.N == (Hq + 2 * Hkv) * a.D &&
+              k_pages.size(1) == Hkv && v_pages.sizes() ==
+                  (at::IntArrayRef{k_pages.size(0), Hkv, a.D, a.P}),
+              "bad fused qkv shape");
+  TORCH_CHECK(page_table.scalar_type() == at::kInt &&
+              page_table.size(0) >= A.size(0) &&
+              start_pos.scalar_type() == at::kInt &&
+              start_pos.numel() >= A.size(0), "bad page table or positions");
+  TORCH_CHECK(cos_t.scalar_type() == at::kFloat && cos_t.is_contiguous() &&
+              sin_t.scalar_type() == at::kFloat && sin_t.is_contiguous() &&
+              cos_t.dim() == 2 && cos_t.size(1) == a.D / 2 &&
+              cos_t.sizes() == sin_t.sizes(), "bad rotation tables");
+  if (pos.has_value()) {
+    CHECK_DEV((*pos));
+    TORCH_CHECK(pos->scalar_type() == at::kInt && pos->is_contiguous() &&
+                pos->numel() == a.M, "bad position ids");
+    a.pos = pos->data_ptr<int>();
+  }
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N;
+  auto C = torch::empty(sizes, A.options());
+  a.C = bf_ptr_mut(C);
+  a.eps = eps;
+  a.cos_t = cos_t.data_ptr<float>();
+  a.sin_t = sin_t.data_ptr<float>();
+  a.max_pos = cos_t.size(0);
+  a.table = page_table.data_ptr<int>();
+  a.start = start_pos.data_ptr<int>();
+  a.k_pages = bf_ptr_mut(k_pages);
+  a.v_pages = bf_ptr_mut(v_pages);
+  if (a.M <= STREAM_ROWS) {
+    gemm_stream_kernel<EPI_ROPE, 2, 1, true, 4, 3>
+        <<<a.N / 32, 256, 0, cur_stream()>>>(a);
+    return C;
+  }
+  // the split of gemm_skinny's small-N shapes; the fold turns and stores
+  int nstripes = 0;
+  const float* ss = row_stats(ss_in, &nstripes);
+  const int stages = a.K / 256;
+  int ksplit = std::min<int>(
+      std::max(1, a.K / 512), std::max(1, std::min(8, 1024 / (a.N / 64))));
+  const int per = (stages + ksplit - 1) / ksplit;
+  ksplit = (stages + per - 1) / per;
+  auto part = torch::empty({(long)ksplit, (long)a.M, (long)a.N},
+                           A.options().dtype(at::kFloat));
+  launch_skinny_fused<false>(a, ss, nstripes, per * 256, ksplit,
+                             part.data_ptr<float>());
+  rope_kv_fold_kernel<<<(a.M * (a.N / 2) + 255) / 256, 256, 0, cur_stream()>>>(
+      a, part.data_ptr<float>(), ksplit);
+  return C;
+}
 
 // C(M,N) = A(M,K) @ W(N,K)^T [+ residual (M,N)] [+ bias (N,)], M <= 32.
 torch::Tensor gemm_skinny(torch::Tensor A, torch::Tensor W,
@@ -910,6 +1120,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_decode_qkv", &attn_decode_qkv);
   m.def("attn_prefill_qkv", &attn_prefill_qkv);
   m.def("rope_kv_write_", &rope_kv_write_);
+  m.def("gemm_stream", &gemm_stream);
+  m.def("gemm_swiglu", &gemm_swiglu);
+  m.def("gemm_rope_kv", &gemm_rope_kv);
+  m.attr("STREAM_ROWS") = STREAM_ROWS;
   m.def("attn_prefill", &attn_prefill);
   m.def("gemm_skinny", &gemm_skinny, py::arg("A"), py::arg("W"),
         py::arg("residual") = c10::nullopt, py::arg("bias") = c10::nullopt,

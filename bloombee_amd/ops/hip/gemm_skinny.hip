@@ -118,7 +118,11 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(
 // Host guarantees (k1 - k0) % 256 == 0 so the set pairing needs no tail.
 // STAGE_NORM: norm mode 1 as an instantiation of its own — its per-element
 // scaling, though never run, slows the other modes' pipeline by 7%.
-template <int MT, bool STAGE_NORM = false>
+// SWIGLU: W is a fused [gate | up] projection; waves 0 and 1 take 32 gate rows, 2 and
+// 3 the up rows that go with them, and C (M, N/2) is silu(gate) * up: the product's
+// own launch (4.8 us at 32 x 14336) and a round trip of both through memory go.
+// Unsplit, norm mode 2.
+template <int MT, bool STAGE_NORM = false, bool SWIGLU = false>
 __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
     const unsigned short* __restrict__ A,   // (M, K) bf16
     const unsigned short* __restrict__ W,   // (N, K) bf16
@@ -164,7 +168,8 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
     if (nwg >= 8)
       tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig8;
   }
-  const int n0 = tile * 64 + wave * 16;
+  const int n0 = SWIGLU ? (wave >> 1) * (N / 2) + tile * 32 + (wave & 1) * 16
+                        : tile * 64 + wave * 16;
   const int split = blockIdx.y;
   const int k0 = split * kchunk;
   const int k1 = min(K, k0 + kchunk);
@@ -324,6 +329,33 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
   }
 
   if (norm_mode == 2) reduce_invr();
+
+  if constexpr (SWIGLU) {
+    float* up = reinterpret_cast<float*>(atile);   // (MT * 16, 32): atile is dead
+    __syncthreads();
+    if (wave >= 2) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg)
+          up[(t * 16 + hi * 4 + reg) * 32 + (wave & 1) * 16 + li] = acc[t][reg];
+    }
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg) {
+          const int m = t * 16 + hi * 4 + reg;
+          if (m >= M) continue;
+          const float r = norm_mode == 2 ? invr[m] : 1.f;
+          const float v = acc[t][reg] * r;
+          const float u = up[m * 32 + wave * 16 + li] * r;
+          C[(long)m * (N / 2) + n0 + li] = f2bf(v / (1.f + fast_expf(-v)) * u);
+        }
+    }
+    return;
+  }
 
   if (Cpart == nullptr) {
     if (ssout == nullptr) {

@@ -188,22 +188,29 @@ def attn_prefill(
 
 
 def rope_kv_write_(qkv, Hq: int, Hkv: int, cos, sin, position_ids,
-                   k_pages, v_pages, page_table, start_pos):
+                   k_pages, v_pages, page_table, start_pos,
+                   head_norms: Optional[tuple] = None):
     """Fused RoPE + paged KV write on the raw QKV GEMM output.
 
     qkv: (B, T, (Hq+2Hkv)*D) — q section roped in place; k roped -> pages;
     v copied -> pages. position_ids None => start_pos[b] + t.
+    head_norms=(q weight, k weight, eps): an RMS norm of every q and k head
+    ahead of the rotation.
     """
+    qw, kw, eps = head_norms or (None, None, 0.0)
     if _on_gpu(qkv):
         _require_ext()
         hip_ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin,
                                position_ids.int() if position_ids is not None else None,
-                               k_pages, v_pages, page_table, start_pos.int())
+                               k_pages, v_pages, page_table, start_pos.int(),
+                               qw, kw, eps)
         return
     B, T, _ = qkv.shape
     D = k_pages.shape[3]
     q = qkv[..., : Hq * D].view(B, T, Hq, D).permute(0, 2, 1, 3)
     k = qkv[..., Hq * D:(Hq + Hkv) * D].view(B, T, Hkv, D).permute(0, 2, 1, 3)
+    if head_norms is not None:
+        q, k = ref.rms_norm(q, qw, eps), ref.rms_norm(k, kw, eps)
     v = qkv[..., (Hq + Hkv) * D:].view(B, T, Hkv, D).permute(0, 2, 1, 3)
     if position_ids is None:
         position_ids = start_pos.view(B, 1).long() + torch.arange(T).view(1, T)
@@ -213,11 +220,12 @@ def rope_kv_write_(qkv, Hq: int, Hkv: int, cos, sin, position_ids,
 
 
 def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
-                   q_start, scale=None, window: int = 0):
+                   q_start, scale=None, window: int = 0, tree_mask=None):
     """Attention reading q straight from the fused QKV buffer.
 
     qkv: (B, T, (Hq+2Hkv)*D) with the q section already roped and the new
-    tokens' K/V already in the pages (rope_kv_write_ first).
+    tokens' K/V already in the pages (rope_kv_write_ first). tree_mask: as in
+    attn_paged.
     Returns (B, T, Hq*D) — the O-projection GEMM input, no transposes.
     """
     B, T, _ = qkv.shape
@@ -225,16 +233,25 @@ def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     if _on_gpu(qkv):
-        _require_ext()
-        if T == 1:
-            ctx = q_start + 1
-            return hip_ops.attn_decode_qkv(qkv, Hq, k_pages, v_pages, page_table,
-                                           ctx.int(), scale, window, 0)
-        return hip_ops.attn_prefill_qkv(qkv, Hq, k_pages, v_pages, page_table,
-                                        q_start.int(), scale, window)
+        if tree_mask is None or (_TREE_KERNEL and window == 0 and D <= 256):
+            _require_ext()
+            if T == 1 and tree_mask is None:
+                return hip_ops.attn_decode_qkv(qkv, Hq, k_pages, v_pages,
+                                               page_table, q_start.int(), scale,
+                                               window, 0, 1)
+            if tree_mask is not None:
+                tree_mask = tree_mask.to(qkv.device).contiguous().bool()
+            return hip_ops.attn_prefill_qkv(qkv, Hq, k_pages, v_pages,
+                                            page_table, q_start.int(), scale,
+                                            window, tree_mask)
     q = qkv[..., : Hq * D].view(B, T, Hq, D).permute(0, 2, 1, 3).contiguous()
-    out = ref.attn_paged(q, k_pages, v_pages, page_table, q_start.long(), scale,
-                         sliding_window=window if window > 0 else None)
+    if tree_mask is not None:
+        out = attn_paged(q, k_pages, v_pages, page_table, q_start.long(), scale,
+                         window, tree_mask=tree_mask)
+    else:
+        out = ref.attn_paged(q, k_pages, v_pages, page_table, q_start.long(),
+                             scale,
+                             sliding_window=window if window > 0 else None)
     return out.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
 
 
@@ -299,6 +316,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
     if (_on_gpu(x) and M <= 32 and x.dtype == torch.bfloat16
             and K % 256 == 0 and N % 64 == 0):
         _require_ext()
+        if (M <= hip_ops.STREAM_ROWS and ss_out is None
+                and (norm is None or norm[0] is None)):
+            return hip_ops.gemm_stream(x.contiguous(), w, residual, bias,
+                                       -1.0 if norm is None else float(norm[1]))
         if norm is not None or ss_out is not None:
             nw = None
             eps = 0.0
@@ -342,6 +363,34 @@ def fuse_norm_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (_FUSE_NORM and _on_gpu(x) and x.numel() // K <= 32
             and x.dtype == torch.bfloat16 and K % 256 == 0
             and w.shape[0] % 64 == 0 and HAVE_HIP_OPS)
+
+
+def row_stats_wanted(x: torch.Tensor) -> bool:
+    """Whether a fused norm of these rows reads the statistics its producer
+    leaves (ss_out): a few rows are summed up by the GEMM that reads them."""
+    return x.numel() // x.shape[-1] > hip_ops.STREAM_ROWS
+
+
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor, eps: float,
+                  ss_in: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """swiglu(rmsnorm(x) @ w^T) of a fused [gate | up] projection whose norm
+    weight is folded in, in one launch. Callers gate on fuse_norm_linear_ok."""
+    _require_ext()
+    return hip_ops.gemm_swiglu(x.contiguous(), w, eps, ss_in)
+
+
+def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, eps: float,
+                   ss_in: Optional[torch.Tensor], Hq: int, Hkv: int, cos, sin,
+                   position_ids, k_pages, v_pages, page_table,
+                   start_pos) -> torch.Tensor:
+    """rope_kv_write_ of rmsnorm(x) @ w^T: returns (B, T, (Hq+2Hkv)*D) with the
+    turned queries; keys and values are in the pages only. Callers gate on
+    fuse_norm_linear_ok."""
+    _require_ext()
+    return hip_ops.gemm_rope_kv(
+        x.contiguous(), w, eps, ss_in, Hq, Hkv, cos, sin,
+        position_ids.int().contiguous() if position_ids is not None else None,
+        k_pages, v_pages, page_table, start_pos.int())
 
 
 def attn_paged_mixed(q, k_pages, v_pages, page_table, ctx_lens,

@@ -1,0 +1,141 @@
+"""Decode GEMMs that take what follows them along, and the split of decode attention,
+at the edges of their rules: rows up to which one launch does a GEMM, tiles of 16 and
+32 columns, pieces of 128 columns of K shared out over eight or four waves."""
+import pytest
+import torch
+
+from bloombee_amd import ops
+from bloombee_amd.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+ROWS = [1, 2, 7, 8, 9, 16, 17, 25, 32]
+
+
+def draw(*shape, seed=0, scale=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=gen) * scale).bfloat16().to(DEV)
+
+
+def close(got, want, scale=1.0):
+    """Results are one bf16 rounding of 32-bit sums, 2^-9 of a value; another 2^-8 of
+    the result's scale for hardware exponentials and reciprocals."""
+    err = (got.double() - want).abs()
+    assert bool((err <= 2.0 ** -8 * want.abs() + 2.0 ** -8 * scale).all()), err.max()
+
+
+def rms(x, eps):
+    x = x.double()
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps)
+
+
+@pytest.mark.parametrize("M", [1, 2, 7, 8])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 1152), (80, 2944)])
+def test_stream(M, N, K):
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    b, r = draw(N, seed=3), draw(M, N, seed=4)
+    want = x.double() @ w.double().T
+    close(ops.hip_ops.gemm_stream(x, w, None, None, -1.0), want)
+    close(ops.hip_ops.gemm_stream(x, w, r, b, -1.0), want + b.double() + r.double())
+    close(ops.hip_ops.gemm_stream(x, w, r, None, 1e-5),
+          rms(x, 1e-5) @ w.double().T + r.double())
+
+
+def test_stream_refuses_what_it_cannot_do():
+    for M, N, K in ((9, 16, 128), (1, 24, 128), (1, 16, 192)):
+        with pytest.raises(RuntimeError):
+            ops.hip_ops.gemm_stream(draw(M, K), draw(N, K), None, None, -1.0)
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("I,K", [(32, 256), (96, 768), (1024, 512)])
+def test_gated_product(M, I, K):
+    x, w = draw(M, K, seed=1), draw(2 * I, K, seed=2, scale=K ** -0.5)
+    z = rms(x, 1e-5) @ w.double().T
+    want = torch.nn.functional.silu(z[:, :I]) * z[:, I:]
+    assert ops.fuse_norm_linear_ok(x, w)
+    close(ops.linear_swiglu(x, w, 1e-5), want)
+    if ops.row_stats_wanted(x):
+        # squares of the rows as a producer of four stripes leaves them
+        ss = torch.zeros(4, 32, device=DEV)
+        ss[:, :M] = x.float().view(M, 4, -1).pow(2).sum(-1).T
+        close(ops.linear_swiglu(x, w, 1e-5, ss_in=ss.flatten()), want)
+
+
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("Hq,Hkv,D,P,K", [(4, 2, 64, 16, 256), (2, 1, 128, 8, 512),
+                                          (8, 2, 32, 16, 1024)])
+@pytest.mark.parametrize("ids", [False, True])
+def test_rotations_and_pages(M, Hq, Hkv, D, P, K, ids):
+    B = 1 if M % 2 else 2
+    T = M // B
+    x = draw(B, T, K, seed=1)
+    w = draw((Hq + 2 * Hkv) * D, K, seed=2, scale=K ** -0.5)
+    start = torch.tensor([5, 2 * P - 1][:B], dtype=torch.int32, device=DEV)
+    room = int(start.max()) + T
+    maxp = -(-room // P) + 1
+    table = torch.randperm(B * maxp, generator=torch.Generator().manual_seed(3))
+    table = table.view(B, maxp).int().to(DEV)
+    kp, vp = draw(B * maxp, Hkv, P, D, seed=4), draw(B * maxp, Hkv, D, P, seed=5)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(D, 128))
+    pos = None
+    if ids:
+        pos = torch.arange(M, device=DEV, dtype=torch.int32).view(B, T) % 7 + 3
+    # the same in steps: plain projection, then the CPU form of the pages' writer
+    z = (rms(x, 1e-5) @ w.double().T).float().cpu()
+    kw, vw = kp.float().cpu(), vp.float().cpu()
+    ops.rope_kv_write_(z, Hq, Hkv, cos.cpu(), sin.cpu(),
+                       pos.cpu() if ids else None, kw, vw, table.cpu(), start.cpu())
+    got = ops.linear_rope_kv(x, w, 1e-5, None, Hq, Hkv, cos, sin, pos, kp, vp, table,
+                             start)
+    close(got[..., :Hq * D].cpu(), z[..., :Hq * D].double())
+    close(kp.cpu(), kw.double())
+    close(vp.cpu(), vw.double())
+
+
+def test_head_norms_ride_the_rotation():
+    B, T, Hq, Hkv, D, P = 2, 3, 4, 2, 128, 16
+    z = draw(B, T, (Hq + 2 * Hkv) * D, seed=1)
+    qw, kw = draw(D, seed=2) + 1, draw(D, seed=3) + 1
+    table = torch.arange(4, dtype=torch.int32, device=DEV).view(B, 2)
+    start = torch.tensor([0, 15], dtype=torch.int32, device=DEV)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(D, 64))
+    pages = [torch.zeros(4, Hkv, *s, dtype=torch.bfloat16, device=DEV)
+             for s in ((P, D), (D, P))]
+    want = z.float().cpu()
+    wp = [p.float().cpu() for p in pages]
+    norms = (qw, kw, 1e-6)
+    ops.rope_kv_write_(want, Hq, Hkv, cos.cpu(), sin.cpu(), None, *wp, table.cpu(),
+                       start.cpu(), head_norms=(qw.float().cpu(), kw.float().cpu(),
+                                                1e-6))
+    ops.rope_kv_write_(z, Hq, Hkv, cos, sin, None, *pages, table, start,
+                       head_norms=norms)
+    close(z[..., :Hq * D].cpu(), want[..., :Hq * D].double(), 4.0)
+    for p, q in zip(pages, wp):
+        close(p.cpu(), q.double(), 4.0)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,room,lengths", [
+    (1, 4, 1, 128, 128, [1]),                 # one split, one token
+    (1, 4, 2, 128, 300, [300]),               # two splits
+    (2, 8, 2, 128, 4096, [5, 4096]),          # a short context in a wide table
+    (1, 71, 1, 64, 2000, [777]),              # a group in five chunks
+    (65, 8, 8, 64, 2100, None),               # more units than fit: even shares
+])
+def test_decode_attention_splits(B, Hq, Hkv, D, room, lengths):
+    P = 16
+    gen = torch.Generator().manual_seed(B)
+    if lengths is None:
+        lengths = torch.randint(1, room + 1, (B,), generator=gen).tolist()
+    maxp = -(-room // P)
+    kp, vp = draw(B * maxp, Hkv, P, D, seed=1), draw(B * maxp, Hkv, D, P, seed=2)
+    table = torch.randperm(B * maxp, generator=gen).view(B, maxp).int().to(DEV)
+    qkv = draw(B, 1, (Hq + 2 * Hkv) * D, seed=3)
+    start = torch.tensor([n - 1 for n in lengths], dtype=torch.int32, device=DEV)
+    q = qkv[..., :Hq * D].view(B, 1, Hq, D).transpose(1, 2)
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, start.long())
+    got = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, table, start)
+    # weights enter the value product in bf16: 2^-9 of the largest value
+    err = (got.view(B, Hq, D).float() - want[:, :, 0]).abs().max()
+    assert err <= 2 * 4.5 * 2.0 ** -9, err
