@@ -1,11 +1,10 @@
 """Server-side Mixtral block (parity: reference models/mixtral/block.py
 WrappedMixtralBlock :13-137): LLaMA-style GQA attention + top-2 MoE MLP.
 
-MoE execution (MI-native): tokens are gathered per selected expert and each
-expert's gate_up/down run as skinny-M GEMMs — at decode batch sizes every
-expert's token group is M <= 32, exactly the shape gemm_skinny.hip is built
-for (BASELINE.json config 4's "MoE grouped GEMM"); the scatter-add back is a
-single index_add per expert."""
+MoE execution (MI-native): on the device norm, routing and the grouped expert
+GEMMs of all experts run without a host sync (ops.routed_mlp). The loop over
+experts is the CPU form, and that of an expert-parallel rank, which holds some
+of them."""
 from __future__ import annotations
 
 import math
@@ -63,38 +62,23 @@ class MixtralBlock(torch.nn.Module):
         return self
 
     # -- MoE MLP ----------------------------------------------------------
+    def _grouped(self, y: torch.Tensor) -> bool:
+        """This rank holds all experts and the grouped kernels take them."""
+        return (getattr(self, "ep_range", (0, self.E)) == (0, self.E)
+                and not getattr(self, "moe_loop", False)
+                and ops.routed_mlp_ok(y, self.expert_gate_up_w,
+                                      self.expert_down_w, self.topk))
+
     def _moe(self, y: torch.Tensor) -> torch.Tensor:
+        if self._grouped(y):
+            return ops.routed_mlp(y, self.router_w, self.expert_gate_up_w,
+                                  self.expert_down_w, self.topk)
         B, T, H = y.shape
         flat = y.reshape(-1, H)
         logits = ops.linear(flat, self.router_w).float()
         weights, experts = logits.topk(self.topk, dim=-1)
         weights = torch.softmax(weights, dim=-1).to(y.dtype)
         e0, e1 = getattr(self, "ep_range", (0, self.E))
-        if (flat.is_cuda and ops.HAVE_HIP_OPS
-                and flat.dtype == torch.bfloat16
-                and (e0, e1) == (0, self.E) and flat.shape[0] <= 1024
-                and not getattr(self, "moe_loop", False)):
-            # grouped decode path: expert-sort the (token, choice) slots on
-            # device and run BOTH expert GEMMs as single grouped launches
-            # (ops/hip/moe_gemm.hip) — no per-expert host sync, no
-            # per-expert kernel launches
-            Tk = flat.shape[0] * self.topk
-            fe = experts.reshape(-1)
-            order = fe.argsort(stable=True)
-            counts = torch.bincount(fe, minlength=self.E)
-            off = torch.zeros(self.E + 1, dtype=torch.int32,
-                              device=flat.device)
-            off[1:] = counts.cumsum(0).int()
-            tok = (order // self.topk).int()
-            wsorted = weights.reshape(-1)[order].float()
-            mch = (flat.shape[0] + 31) // 32
-            gu = ops.moe_gemm_grouped(flat, self.expert_gate_up_w, off,
-                                      rowmap=tok, S=Tk, mchunks=mch)
-            dn = ops.moe_gemm_grouped(ops.swiglu(gu), self.expert_down_w,
-                                      off, scale=wsorted, S=Tk, mchunks=mch)
-            out = torch.zeros_like(flat)
-            out.index_add_(0, tok.long(), dn)
-            return out.view(B, T, H)
         out = torch.zeros_like(flat)
         # expert-parallel mode (parallel/expert.py): this rank holds only
         # experts [e0, e1); partial sums cross ranks via one all-reduce
@@ -121,15 +105,19 @@ class MixtralBlock(torch.nn.Module):
         Hq, Hkv = self.Hq, self.Hkv
         cfg = self.config
         x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
-        qkv = ops.linear(x, self.qkv_w)
         cos, sin = self.rope.get(hidden.device)
         kp = kv.k_pages(self.layer_index)
         vp = kv.v_pages(self.layer_index)
         pt = kv.page_table()
+        qkv = ops.linear(x, self.qkv_w)
         ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
                            start_pos)
         attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale)
         a = ops.linear(attn, self.o_w)
+        if self._grouped(hidden):
+            return ops.routed_mlp(a, self.router_w, self.expert_gate_up_w,
+                                  self.expert_down_w, self.topk, hidden,
+                                  (self.post_norm_w, cfg.rms_norm_eps))
         h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
         return h2 + self._moe(y)
 

@@ -31,6 +31,8 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     rope_apply_,
     rope_kv_write_,
     rope_cos_sin,
+    routed_mlp,
+    routed_mlp_ok,
     row_stats_wanted,
     set_attn_sparsity,
     swiglu,

@@ -19,6 +19,7 @@
 #include "gemm_skinny.hip"
 #include "gemm_stream.hip"
 #include "moe_gemm.hip"
+#include "moe_route.hip"
 #include "w4_gemm.hip"
 #include "mfma_selftest.hip"
 #include "quant4.hip"
@@ -560,6 +561,57 @@ void rope_kv_write_(torch::Tensor qkv, long Hq_, long Hkv_, torch::Tensor cos_t,
       (int)cos_t.size(0), norms[0], norms[1], (float)eps);
 }
 
+
+// (a + res, its RMS norm, chosen experts (N, top) int32, their weights f32) of rows
+// a, res (N, H); without res and norm_w the first two are a itself.
+std::vector<torch::Tensor> norm_route(torch::Tensor a,
+                                      c10::optional<torch::Tensor> res,
+                                      c10::optional<torch::Tensor> norm_w,
+                                      torch::Tensor router, long top, double eps) {
+  CHECK_DEV_ALL2(a, router); CHECK_BF16(a); CHECK_BF16(router);
+  CHECK_CONTIG(a); CHECK_CONTIG(router);
+  TORCH_CHECK(a.dim() == 2 && router.dim() == 2, "(N, H) rows, (E, H) router");
+  const long N = a.size(0), H = a.size(1), E = router.size(0);
+  TORCH_CHECK(router.size(1) == H && H % 8 == 0 && E <= ROUTE_MAX_E && top >= 1 &&
+                  top <= E && res.has_value() == norm_w.has_value(),
+              "bad router shapes");
+  const bool norm = norm_w.has_value();
+  if (norm) {
+    CHECK_DEV_ALL2((*res), (*norm_w)); CHECK_BF16((*res)); CHECK_BF16((*norm_w));
+    CHECK_CONTIG((*res)); CHECK_CONTIG((*norm_w));
+    TORCH_CHECK(res->numel() == a.numel() && norm_w->numel() == H, "bad norm shapes");
+  }
+  auto h = norm ? torch::empty_like(a) : a, y = norm ? torch::empty_like(a) : a;
+  auto ids = torch::empty({N, top}, a.options().dtype(at::kInt));
+  auto wts = torch::empty({N, top}, a.options().dtype(at::kFloat));
+  if (N == 0) return {h, y, ids, wts};
+  dispatch_iters(H, [&](auto iters) {
+    norm_route_kernel<decltype(iters)::value><<<N, 256, 0, cur_stream()>>>(
+        bf_ptr(a), norm ? bf_ptr(*res) : nullptr, norm ? bf_ptr(*norm_w) : nullptr,
+        bf_ptr(router), bf_ptr_mut(h), bf_ptr_mut(y), ids.data_ptr<int>(),
+        wts.data_ptr<float>(), H, E, top, (float)eps);
+  });
+  return {h, y, ids, wts};
+}
+
+// h (N, W), if any, + the sum over the experts of y (N, top, W).
+torch::Tensor add_experts(c10::optional<torch::Tensor> h, torch::Tensor y) {
+  CHECK_DEV(y); CHECK_BF16(y); CHECK_CONTIG(y);
+  TORCH_CHECK(y.dim() == 3 && y.size(2) % 8 == 0, "bad expert rows");
+  if (h.has_value()) {
+    CHECK_DEV((*h)); CHECK_BF16((*h)); CHECK_CONTIG((*h));
+    TORCH_CHECK(h->dim() == 2 && y.size(0) == h->size(0) && y.size(2) == h->size(1),
+                "bad expert rows");
+  }
+  auto out = torch::empty({y.size(0), y.size(2)}, y.options());
+  const long n = out.numel();
+  if (n == 0) return out;
+  add_experts_kernel<<<std::min<long>((n / 8 + 255) / 256, 4096), 256, 0,
+                       cur_stream()>>>(h.has_value() ? bf_ptr(*h) : nullptr,
+                                       bf_ptr(y), bf_ptr_mut(out), n, y.size(2),
+                                       y.size(1));
+  return out;
+}
 
 // C(S,N) = A[row(s)] @ W[expert(s)]^T — grouped decode MoE (moe_gemm.hip).
 // off: (E+1,) int32 exclusive prefix sums of per-expert slot counts;
@@ -1120,6 +1172,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attn_decode_qkv", &attn_decode_qkv);
   m.def("attn_prefill_qkv", &attn_prefill_qkv);
   m.def("rope_kv_write_", &rope_kv_write_);
+  m.def("norm_route", &norm_route);
+  m.def("add_experts", &add_experts);
   m.def("gemm_stream", &gemm_stream);
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);

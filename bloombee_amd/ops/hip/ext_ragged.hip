@@ -802,10 +802,12 @@ void attn_ragged(Tensor q, Tensor kp, OptTensor vp, Tensor table,
 // h (N, K), up (E, planes, F, K), down (E, Wp, F), ids/wts (N, top)
 // -> y (N, top, Wp); rows of skipped choices are not written. Two planes:
 // gated activation (limit, slope, shift), one: relu(up)^2. win: the weight
-// multiplies the expert's input, else its output.
+// multiplies the expert's input, else its output. stepwise: silu(gate) * up of
+// rounded products.
 Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
-                   bool win, double limit, double slope, double shift) {
-  const GluConst glu{(float)limit, (float)slope, (float)shift};
+                   bool win, double limit, double slope, double shift,
+                   bool stepwise) {
+  const GluConst glu{(float)limit, (float)slope, (float)shift, stepwise};
   check_act(h);
   const auto ta = h.scalar_type();
   for (const Tensor& t : {h, up, down})

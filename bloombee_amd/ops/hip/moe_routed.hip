@@ -34,9 +34,16 @@ static constexpr int MOE_MAX_E = 1024;
 
 struct GluConst {
   float limit, slope, shift;
+  // gate and up are rounded to bf16 ahead of silu(gate) * up, as where the two
+  // products and the activation are steps of their own: same bits as those
+  bool stepwise;
 };
 
 DEVINL float gated(const GluConst& c, float g, float u) {
+  if (c.stepwise) {
+    g = bf2f(f2bf(g));
+    return g / (1.f + fast_expf(-g)) * bf2f(f2bf(u));
+  }
   g = fminf(g, c.limit);
   u = fminf(fmaxf(u, -c.limit), c.limit) + c.shift;
   return g * sigmoid_f(c.slope * g) * u;

@@ -404,6 +404,41 @@ def attn_paged_mixed(q, k_pages, v_pages, page_table, ctx_lens,
                                 host_k, host_v, scale)
 
 
+def routed_mlp_ok(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
+                  top: int) -> bool:
+    """routed_mlp's kernels take these: gate_up (E, 2I, H), down (E, H, I)."""
+    E, H, I = down.shape
+    return (_on_gpu(x) and x.dtype == torch.bfloat16 and x.numel() > 0
+            and E <= 64 and 1 <= top <= E and H % 64 == 0 and I % 64 == 0
+            and H <= 16384 and gate_up.is_contiguous() and down.is_contiguous())
+
+
+def routed_mlp(a: torch.Tensor, router_w: torch.Tensor, gate_up: torch.Tensor,
+               down: torch.Tensor, top: int,
+               residual: Optional[torch.Tensor] = None,
+               norm: Optional[tuple] = None) -> torch.Tensor:
+    """Sum of the chosen experts of the rows a: the top router logits choose, a
+    softmax over them weighs. With a residual and norm=(weight, eps): h +
+    experts(rmsnorm(h)), h = a + residual. Norm and routing are one launch, the
+    experts two weight streams up to 32 rows and a sort with two tiled GEMMs
+    beyond (moe_routed.hip); nothing waits for the host. Callers gate on
+    routed_mlp_ok."""
+    _require_ext()
+    from bloombee_amd.ops import ragged
+
+    E, H, I = down.shape
+    w, eps = norm or (None, 0.0)
+    h, y, ids, wts = hip_ops.norm_route(
+        a.reshape(-1, H).contiguous(),
+        None if residual is None else residual.reshape(-1, H).contiguous(), w,
+        router_w, top, eps)
+    # every step's results are bf16, as in a loop over the experts: the choices
+    # of later layers hang on near ties, and are to be the loop's
+    rows = ragged.moe_experts(y, gate_up.view(E, 2, I, H), down,
+                              ragged.Routing(ids, wts, None), stepwise=True)
+    return hip_ops.add_experts(None if residual is None else h, rows).view(a.shape)
+
+
 def moe_gemm_grouped(A: torch.Tensor, W: torch.Tensor, off: torch.Tensor,
                      rowmap: Optional[torch.Tensor] = None,
                      scale: Optional[torch.Tensor] = None,
@@ -416,8 +451,7 @@ def moe_gemm_grouped(A: torch.Tensor, W: torch.Tensor, off: torch.Tensor,
     the int32 exclusive prefix sum ON DEVICE (no host sync — hipGraph-safe,
     unlike the per-expert nonzero() loop). S = total slots, mchunks = host
     upper bound on ceil(max rows per expert / 32) (worst case: every token
-    routed to one expert). Replaces the per-expert skinny GEMM loop for
-    Mixtral decode (BASELINE config 4 "MoE grouped GEMM").
+    routed to one expert).
     """
     E, N, K = W.shape
     if S is None:

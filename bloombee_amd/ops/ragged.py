@@ -629,15 +629,16 @@ SILU = GluSpec()
 
 def moe_experts(h: torch.Tensor, up: torch.Tensor, down: torch.Tensor,
                 rt: Routing, weight_input: bool = False,
-                act: GluSpec = SILU) -> torch.Tensor:
+                act: GluSpec = SILU, stepwise: bool = False) -> torch.Tensor:
     """(N, top, W) weighted outputs of the chosen experts; the rows of
     identity choices are not defined. up (E, 2, F, K): the gated activation act,
     or (E, 1, F, K): relu(up)^2; down (E, W, F); K, F and W padded to 64. The
-    weight multiplies an expert's output, or its input."""
+    weight multiplies an expert's output, or its input. stepwise (silu(gate) * up
+    only): gate and up are rounded to the activation type first."""
     consts = (act.limit, act.slope, act.shift)
     if h.is_cuda:
         return _ext().moe_experts(h, up, down, rt.ids, rt.wts, weight_input,
-                                  *consts)
+                                  *consts, stepwise)
     return ref.moe_experts(h, up, down, rt.ids, rt.wts, weight_input, *consts)
 
 

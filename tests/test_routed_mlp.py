@@ -1,0 +1,92 @@
+"""Routing ahead of the experts and their sum behind them, at the edges: one expert,
+64, all of them chosen, equal and missing logits, rows of either path (two weight
+streams up to 32 rows, sorted tiles beyond)."""
+import pytest
+import torch
+
+from bloombee_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def draw(*shape, seed=0, scale=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=gen) * scale).bfloat16().to(DEV)
+
+
+def rms(x, w, eps):
+    x = x.double()
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps) * w.double()
+
+
+@pytest.mark.parametrize("N,H,E,top", [(1, 8, 1, 1), (5, 264, 8, 2), (33, 4096, 8, 8),
+                                       (3, 2048, 64, 6), (2, 16384, 5, 3)])
+def test_norm_and_routing(N, H, E, top):
+    a, r = draw(N, H, seed=1), draw(N, H, seed=2)
+    w, router = draw(H, seed=3, scale=0.1) + 1, draw(E, H, seed=4, scale=H ** -0.5)
+    h, y, ids, wts = ops.hip_ops.norm_route(a, r, w, router, top, 1e-5)
+    assert torch.equal(h, a + r)
+    want = rms(h, w, 1e-5)
+    # one rounding to bf16
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-6).all())
+    # from its own norm on: logits are bf16 results of 32-bit sums
+    logits = y.double() @ router.double().T
+    got = logits.gather(1, ids.long())
+    step = 2.0 ** -8 * logits.abs().amax(1, keepdim=True) + 1e-6
+    kth = logits.topk(top, -1).values
+    assert bool(((got - kth).abs() <= 2 * step).all())
+    assert all(len(set(row)) == top for row in ids.tolist())
+    soft = torch.softmax(got, -1)
+    # the weights are bf16 themselves
+    assert bool(((wts.double() - soft).abs() <= 4 * step + 2.0 ** -9).all())
+
+
+def test_equal_and_missing_logits_choose_distinct_experts():
+    a = draw(3, 64, seed=1)
+    router = draw(6, 64, seed=2)
+    router[2] = router[4]
+    a[1] = 0.0                               # all equal
+    a[2, 5] = float("nan")                   # none there
+    _, y, ids, wts = ops.hip_ops.norm_route(a, None, None, router, 3, 0.0)
+    assert y.data_ptr() == a.data_ptr()
+    assert all(len(set(row)) == 3 and 0 <= min(row) and max(row) < 6
+               for row in ids.tolist())
+    assert ids[1].tolist() == [0, 1, 2]      # the first of equal ones
+    assert bool(((wts[:2].sum(1) - 1).abs() <= 3 * 2.0 ** -10).all())
+    assert bool(wts[2].isnan().all())
+
+
+@pytest.mark.parametrize("N", [1, 31, 32, 33, 200])
+@pytest.mark.parametrize("E,top,H,I", [(4, 2, 256, 320), (1, 1, 64, 64),
+                                       (8, 3, 192, 128)])
+def test_routed_mlp(N, E, top, H, I):
+    a, r = draw(N, H, seed=1), draw(N, H, seed=2)
+    w, router = draw(H, seed=3, scale=0.1) + 1, draw(E, H, seed=4)
+    up = draw(E, 2 * I, H, seed=5, scale=H ** -0.5)
+    down = draw(E, H, I, seed=6, scale=I ** -0.5)
+    assert ops.routed_mlp_ok(a, up, down, top)
+    h, y, ids, wts = ops.hip_ops.norm_route(a, r, w, router, top, 1e-5)
+    want = torch.zeros(N, H, dtype=torch.float64, device=DEV)
+    tol = torch.zeros_like(want)
+    for n in range(N):
+        for c in range(top):
+            e, wt = int(ids[n, c]), float(wts[n, c])
+            g, u = (y[n].double() @ up[e].double().T).chunk(2)
+            act = torch.nn.functional.silu(g) * u
+            row = wt * (act @ down[e].double().T)
+            want[n] += row
+            # an expert's row and the sums over them are bf16, 2^-9 of them; so
+            # are gate, up and activation, whose roundings add up like random
+            # ones (five deviations, three roundings)
+            tol[n] += 2.0 ** -9 * ((1 + top) * row.abs() + 15 * wt * (
+                act.square() @ down[e].double().square().T).sqrt())
+    got = ops.routed_mlp(y, router, up, down, top)
+    # hardware exponentials stay far below
+    assert bool(((got.double() - want).abs()
+                 <= tol + 2.0 ** -8 * want.abs() + 1e-6).all())
+    got = ops.routed_mlp(a, router, up, down, top, r, (w, 1e-5))
+    want = want + h.double()
+    assert bool(((got.double() - want).abs()
+                 <= tol + 2.0 ** -8 * want.abs() + 1e-6).all())
