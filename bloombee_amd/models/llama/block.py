@@ -76,12 +76,6 @@ class LlamaBlock(torch.nn.Module):
         self.gate_up_w = p(2 * I, H)              # fused gate|up
         self.down_w = p(H, I)
         self.rope = rope if rope is not None else RopeTables(config)
-        # fused-norm chain state (forward_inference fuse_norm path):
-        # per-stripe row sum-of-squares buffers, (H/64, 32) f32, written by
-        # the o/down GEMM epilogues and consumed by the next fused rmsnorm
-        self._ss_h2 = None
-        self._ss_hidden = None
-        self._ss_valid = False
 
     @torch.no_grad()
     def init_random(self, seed: Optional[int] = None):
@@ -102,9 +96,8 @@ class LlamaBlock(torch.nn.Module):
         return self
 
     def _fuse_norm_gate(self, hidden) -> bool:
-        """All four decode GEMMs must hit the v2 kernel (K%256) with
-        stripe-aligned N so the fused-norm ss chain stays on-device;
-        W4/LoRA blocks keep the separate-norm path."""
+        """All four decode GEMMs must be decode-shaped (<= 32 rows, K%256,
+        N%64); W4/LoRA blocks keep the separate-norm path."""
         return (getattr(self, "_w4", None) is None
                 and getattr(self, "lora_delta", None) is None
                 and ops.fuse_norm_linear_ok(hidden, self.qkv_w)
@@ -112,41 +105,13 @@ class LlamaBlock(torch.nn.Module):
                 and (self.Hq * self.D) % 256 == 0
                 and self.config.hidden_size % 64 == 0)
 
-    def _ensure_ss_bufs(self, device) -> None:
-        if self._ss_h2 is None or self._ss_h2.device != device:
-            st = self.config.hidden_size // 64
-            self._ss_h2 = torch.empty(st * 32, dtype=torch.float32,
-                                      device=device)
-            self._ss_hidden = torch.empty_like(self._ss_h2)
-
-    def _input_stats(self, hidden, fuse_norm: bool):
-        """(row statistics of `hidden` for its fused norm or None, whether the
-        fused norm can run): a first block of many rows has no producer."""
-        if not fuse_norm:
-            return None, False
-        if not ops.row_stats_wanted(hidden):
-            return None, True
-        pb = getattr(self, "prev_block", None)
-        if pb is not None and getattr(pb, "_ss_valid", False):
-            return pb._ss_hidden, True
-        return None, False
-
     def _fused_tail(self, hidden, attn) -> torch.Tensor:
-        """h2 = hidden + o(attn) via the GEMM's residual epilogue, which also
-        emits row sum-of-squares where the next norm wants them; the
-        post-attention rmsnorm and the gated product ride gate_up. down-proj
-        leaves the stats for the NEXT block's input norm."""
-        eps = self.config.rms_norm_eps
-        if not ops.row_stats_wanted(hidden):
-            h2 = ops.linear(attn, self.o_w, residual=hidden)
-            return ops.linear(ops.linear_swiglu(h2, self.gate_up_w, eps),
-                              self.down_w, residual=h2)
-        self._ensure_ss_bufs(hidden.device)
-        h2 = ops.linear(attn, self.o_w, residual=hidden, ss_out=self._ss_h2)
-        m = ops.linear_swiglu(h2, self.gate_up_w, eps, ss_in=self._ss_h2)
-        out = ops.linear(m, self.down_w, residual=h2, ss_out=self._ss_hidden)
-        self._ss_valid = True
-        return out
+        """What follows attention in a decode-shaped step: h2 = hidden + o(attn)
+        via the GEMM's residual epilogue; the post-attention rmsnorm and the
+        gated product ride gate_up."""
+        h2 = ops.linear(attn, self.o_w, residual=hidden)
+        m = ops.linear_swiglu(h2, self.gate_up_w, self.config.rms_norm_eps)
+        return ops.linear(m, self.down_w, residual=h2)
 
     @torch.no_grad()
     def fold_norm_weights(self):
@@ -245,14 +210,9 @@ class LlamaBlock(torch.nn.Module):
         # Decode-shaped GPU steps fold both per-layer rmsnorms into the
         # skinny GEMMs, the rotation with the K/V write into the first one and
         # the gated product into the third: a launch there costs more than
-        # most of these steps do. Up to ops.STREAM_ROWS rows a GEMM sums up
-        # the squares its norm needs; beyond, they are produced by the
-        # PRECEDING GEMM's epilogue (ss buffers chained block-to-block via
-        # prev_block; re-streaming A instead costs +18-60 us/GEMM —
-        # profiles/r02 §13). W4/LoRA blocks and prefill keep the separate
+        # most of these steps do. W4/LoRA blocks and prefill keep the separate
         # steps.
         fuse_norm = self._fuse_norm_gate(hidden)
-        self._ss_valid = False
         if fuse_norm and not getattr(self, "_norm_folded", False):
             self.fold_norm_weights()   # one-time reparameterization
         cos, sin = self.rope.get(hidden.device)
@@ -269,11 +229,10 @@ class LlamaBlock(torch.nn.Module):
                             .view(1, T)).int()
         # fused RoPE + paged KV write on the GEMM output, then attention
         # reads q in place and emits the O-projection input — no transposes
-        ss, ok = self._input_stats(hidden, fuse_norm)
-        if ok:
-            qkv = ops.linear_rope_kv(hidden, self.qkv_w, cfg.rms_norm_eps, ss,
-                                     Hq, Hkv, cos, sin, position_ids, kp, vp,
-                                     pt, start_pos)
+        if fuse_norm:
+            qkv = ops.linear_rope_kv(hidden, self.qkv_w, cfg.rms_norm_eps, Hq,
+                                     Hkv, cos, sin, position_ids, kp, vp, pt,
+                                     start_pos)
         else:
             x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
             qkv = self._lin(x, self.qkv_w, "qkv_w")    # (B, T, (Hq+2Hkv)D)

@@ -34,17 +34,14 @@ class Qwen3Block(LlamaBlock):
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
         cfg = self.config
 
-        # fused-norm chain (see llama/block.py): both rmsnorms ride the
-        # GEMMs; the per-head q/k norms below act on the GEMM OUTPUT and
-        # are unaffected by the input-norm weight fold
+        # both rmsnorms ride the GEMMs (see llama/block.py); the per-head q/k
+        # norms below act on the GEMM OUTPUT and are unaffected by the
+        # input-norm weight fold
         fuse_norm = self._fuse_norm_gate(hidden)
-        self._ss_valid = False
         if fuse_norm and not getattr(self, "_norm_folded", False):
             self.fold_norm_weights()
-        ss, ok = self._input_stats(hidden, fuse_norm)
-        if ok:
-            qkv = ops.linear(hidden, self.qkv_w,
-                             norm=(None, cfg.rms_norm_eps), ss_in=ss)
+        if fuse_norm and ops.streams_weights(hidden, self.qkv_w):
+            qkv = ops.linear(hidden, self.qkv_w, norm=(None, cfg.rms_norm_eps))
         else:
             x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
             qkv = self._lin(x, self.qkv_w, "qkv_w")

@@ -33,7 +33,7 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     rope_cos_sin,
     routed_mlp,
     routed_mlp_ok,
-    row_stats_wanted,
     set_attn_sparsity,
+    streams_weights,
     swiglu,
 )

@@ -776,11 +776,15 @@ torch::Tensor gemm_w4(torch::Tensor A, torch::Tensor Wq, torch::Tensor scale,
 // skinny-M GEMM (decode projections)
 // ---------------------------------------------------------------------------
 
-// Rows up to which the one-launch kernel (gemm_stream.hip) is the faster one: every
-// workgroup of it reads all of A, which eight rows keep small beside its 16 rows of W.
-// 4096 x 4096 9.1 us at 1 row, 11.0 at 16, 16.5 at 32 (split GEMM and its fold: 13.9,
-// 14.9, 15.1), 14336 x 4096 25, 35, 51 (30, 31, 32).
-static constexpr int STREAM_ROWS = 8;
+// Where the one-launch kernel (gemm_stream.hip) is the faster one. Every workgroup of it
+// reads all of A, twice the bytes of its W at 32 rows: beyond 16 rows that outweighs the
+// launch it saves once W is large. 4096 x 4096 8.8 us at 1 row, 10.1 at 16, 11.9 at 32
+// (split GEMM and its fold: 14.0, 14.6, 15.3), 14336 x 4096 24.8, 28.5, 35.0 (29.7,
+// 30.7, 32.0), [gate | up] of 4096 x 14336 with its product 46.9, 51.7, 58.9 (55.3, 52,
+// 55).
+static bool stream_rows(long M, long N, long K) {
+  return M <= 16 || (M <= 32 && N * K <= (32L << 20));
+}
 
 static StreamArgs stream_args(const torch::Tensor& A, const torch::Tensor& W) {
   CHECK_DEV(A); CHECK_BF16(A); CHECK_CONTIG(A);
@@ -796,19 +800,21 @@ static StreamArgs stream_args(const torch::Tensor& A, const torch::Tensor& W) {
   return a;
 }
 
-static void check_stream(const StreamArgs& a) {
-  TORCH_CHECK(a.M <= STREAM_ROWS && a.K % 128 == 0, "up to ", STREAM_ROWS,
-              " rows and K%128 required");
+// f(rows of A / 16, loads of four of its rows)
+template <typename F>
+static void by_rows(int M, F f) {
+  if (M <= 4) f(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{});
+  else if (M <= 16) f(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+  else f(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
 }
 
-// C(M,N) = A @ W^T [* 1/rms of A's rows] [+ bias] [+ residual], M <= STREAM_ROWS;
-// eps < 0: no norm.
+// C(M,N) = A @ W^T [* 1/rms of A's rows] [+ bias] [+ residual], M <= 32; eps < 0: no
+// norm.
 torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
                           c10::optional<torch::Tensor> residual,
                           c10::optional<torch::Tensor> bias, double eps) {
   StreamArgs a = stream_args(A, W);
-  check_stream(a);
-  TORCH_CHECK(a.N % 16 == 0, "N%16 required");
+  TORCH_CHECK(a.N % 16 == 0 && a.K % 128 == 0, "N%16, K%128 required");
   auto sizes = A.sizes().vec();
   sizes.back() = a.N;
   auto C = torch::empty(sizes, A.options());
@@ -825,43 +831,36 @@ torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
                 bias->is_contiguous() && bias->numel() == a.N, "bad bias");
     a.bias = bf_ptr(*bias);
   }
-  if (eps >= 0)
-    gemm_stream_kernel<EPI_SUM, 1, 1, true, 8, 4>
-        <<<a.N / 16, 512, 0, cur_stream()>>>(a);
-  else
-    gemm_stream_kernel<EPI_SUM, 1, 1, false, 8, 4>
-        <<<a.N / 16, 512, 0, cur_stream()>>>(a);
+  by_rows(a.M, [&](auto mt, auto xn) {
+    constexpr int MT = decltype(mt)::value, XN = decltype(xn)::value;
+    constexpr int DP = MT == 1 ? 4 : 1;
+    if (eps >= 0)
+      gemm_stream_kernel<EPI_SUM, 1, MT, XN, true, 8, DP>
+          <<<a.N / 16, 512, 0, cur_stream()>>>(a);
+    else
+      gemm_stream_kernel<EPI_SUM, 1, MT, XN, false, 8, DP>
+          <<<a.N / 16, 512, 0, cur_stream()>>>(a);
+  });
   return C;
 }
 
-// Unsplit or split v2 GEMM of the fused forms below, norm mode 2.
+// Split or unsplit v2 GEMM of the fused forms below; squares of the rows on the way.
 template <bool SWIGLU>
-static void launch_skinny_fused(const StreamArgs& a, const float* ss, int nstripes,
-                                int kchunk, int ksplit, float* part) {
+static void launch_skinny_fused(const StreamArgs& a, int kchunk, int ksplit,
+                                float* part, float* squares) {
   const dim3 grid(a.N / 64, ksplit);
   auto launch = [&](auto mt) {
-    gemm_skinny_v2_kernel<decltype(mt)::value, false, SWIGLU>
+    gemm_skinny_v2_kernel<decltype(mt)::value, false, SWIGLU, true>
         <<<grid, 256, 0, cur_stream()>>>(a.A, a.W, nullptr, nullptr, a.C, part, a.M,
-                                         a.N, a.K, kchunk, ksplit, nullptr, a.eps, 2,
-                                         ss, nstripes, nullptr);
+                                         a.N, a.K, kchunk, ksplit, nullptr, a.eps, 0,
+                                         nullptr, 0, squares);
   };
   if (a.M <= 16) launch(std::integral_constant<int, 1>{});
   else launch(std::integral_constant<int, 2>{});
 }
 
-static const float* row_stats(const c10::optional<torch::Tensor>& ss, int* nstripes) {
-  if (!ss.has_value()) return nullptr;
-  TORCH_CHECK(ss->is_cuda() && ss->is_contiguous() &&
-              ss->scalar_type() == at::kFloat && ss->numel() % 32 == 0,
-              "ss_in must be f32 (nstripes,32)");
-  *nstripes = (int)(ss->numel() / 32);
-  return ss->data_ptr<float>();
-}
-
-// silu(gate) * up of [gate | up] = rms(A) @ W^T, norm weight folded into W; ss_in as
-// in gemm_skinny (used beyond STREAM_ROWS).
-torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps,
-                          c10::optional<torch::Tensor> ss_in) {
+// silu(gate) * up of [gate | up] = rms(A) @ W^T, norm weight folded into W.
+torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   StreamArgs a = stream_args(A, W);
   TORCH_CHECK(a.K % 256 == 0 && a.N % 64 == 0, "K%256, N%64 required");
   auto sizes = A.sizes().vec();
@@ -869,20 +868,22 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps,
   auto C = torch::empty(sizes, A.options());
   a.C = bf_ptr_mut(C);
   a.eps = eps;
-  int nstripes = 0;
-  const float* ss = row_stats(ss_in, &nstripes);
-  if (a.M <= STREAM_ROWS)
-    gemm_stream_kernel<EPI_SWIGLU, 2, 1, true, 4, 3>
-        <<<a.N / 32, 256, 0, cur_stream()>>>(a);
-  else
-    launch_skinny_fused<true>(a, ss, nstripes, a.K, 1, nullptr);
+  if (!stream_rows(a.M, a.N, a.K)) {
+    launch_skinny_fused<true>(a, a.K, 1, nullptr, nullptr);
+    return C;
+  }
+  by_rows(a.M, [&](auto mt, auto xn) {
+    constexpr int MT = decltype(mt)::value, NW = MT == 1 ? 8 : 4;
+    gemm_stream_kernel<EPI_SWIGLU, 2, MT, decltype(xn)::value, true, NW, 3 - MT>
+        <<<a.N / 32, NW * 64, 0, cur_stream()>>>(a);
+  });
   return C;
 }
 
 // [q | k | v] = rms(A) @ W^T with q turned in the result and k, v in their page slots
 // (their columns of the result stay unwritten). A (B, T, K), norm weight folded in.
-torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps,
-                           c10::optional<torch::Tensor> ss_in, long Hq, long Hkv,
+torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq,
+                           long Hkv,
                            torch::Tensor cos_t, torch::Tensor sin_t,
                            c10::optional<torch::Tensor> pos, torch::Tensor k_pages,
                            torch::Tensor v_pages, torch::Tensor page_table,
@@ -928,25 +929,26 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps,
   a.start = start_pos.data_ptr<int>();
   a.k_pages = bf_ptr_mut(k_pages);
   a.v_pages = bf_ptr_mut(v_pages);
-  if (a.M <= STREAM_ROWS) {
-    gemm_stream_kernel<EPI_ROPE, 2, 1, true, 4, 3>
-        <<<a.N / 32, 256, 0, cur_stream()>>>(a);
+  if (stream_rows(a.M, a.N, a.K)) {
+    by_rows(a.M, [&](auto mt, auto xn) {
+      constexpr int MT = decltype(mt)::value;
+      gemm_stream_kernel<EPI_ROPE, 2, MT, decltype(xn)::value, true, 4, 4 - MT>
+          <<<a.N / 32, 256, 0, cur_stream()>>>(a);
+    });
     return C;
   }
-  // the split of gemm_skinny's small-N shapes; the fold turns and stores
-  int nstripes = 0;
-  const float* ss = row_stats(ss_in, &nstripes);
+  // the split of gemm_skinny's small-N shapes; the fold norms, turns and stores
   const int stages = a.K / 256;
   int ksplit = std::min<int>(
       std::max(1, a.K / 512), std::max(1, std::min(8, 1024 / (a.N / 64))));
   const int per = (stages + ksplit - 1) / ksplit;
   ksplit = (stages + per - 1) / per;
-  auto part = torch::empty({(long)ksplit, (long)a.M, (long)a.N},
-                           A.options().dtype(at::kFloat));
-  launch_skinny_fused<false>(a, ss, nstripes, per * 256, ksplit,
-                             part.data_ptr<float>());
+  const long n = (long)ksplit * a.M * a.N;
+  auto part = torch::empty({n + ksplit * 32}, A.options().dtype(at::kFloat));
+  float* pp = part.data_ptr<float>();
+  launch_skinny_fused<false>(a, per * 256, ksplit, pp, pp + n);
   rope_kv_fold_kernel<<<(a.M * (a.N / 2) + 255) / 256, 256, 0, cur_stream()>>>(
-      a, part.data_ptr<float>(), ksplit);
+      a, pp, pp + n, ksplit);
   return C;
 }
 
@@ -1177,7 +1179,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_stream", &gemm_stream);
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);
-  m.attr("STREAM_ROWS") = STREAM_ROWS;
+  m.def("stream_rows", &stream_rows);
   m.def("attn_prefill", &attn_prefill);
   m.def("gemm_skinny", &gemm_skinny, py::arg("A"), py::arg("W"),
         py::arg("residual") = c10::nullopt, py::arg("bias") = c10::nullopt,

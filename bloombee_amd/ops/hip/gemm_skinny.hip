@@ -121,8 +121,12 @@ __global__ __launch_bounds__(256) void gemm_skinny_kernel(
 // SWIGLU: W is a fused [gate | up] projection; waves 0 and 1 take 32 gate rows, 2 and
 // 3 the up rows that go with them, and C (M, N/2) is silu(gate) * up: the product's
 // own launch (4.8 us at 32 x 14336) and a round trip of both through memory go.
-// Unsplit, norm mode 2.
-template <int MT, bool STAGE_NORM = false, bool SWIGLU = false>
+// Unsplit.
+// GRAM: the rows' sums of squares come off the matrix cores, as the diagonal of A A^T,
+// for norm weights that are folded into W. With SWIGLU they scale the sums; where Cpart
+// takes unscaled parts, the first column tile of each split leaves its own in ssout,
+// (ksplit, 32), for the fold.
+template <int MT, bool STAGE_NORM = false, bool SWIGLU = false, bool GRAM = false>
 __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
     const unsigned short* __restrict__ A,   // (M, K) bf16
     const unsigned short* __restrict__ W,   // (N, K) bf16
@@ -176,9 +180,9 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
 
   const unsigned short* wrow = W + (long)(n0 + li) * K;
 
-  f32x4 acc[MT];
+  f32x4 acc[MT], sq[MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < MT; ++t) acc[t] = sq[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   // ---- A staging: the whole workgroup copies A[0:M][ks:ks+256] with
   // full-line loads; rows beyond M-1 are clamped (their C rows are dropped).
@@ -239,6 +243,9 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
             atile + (t * 16 + li) * RSTRIDE + half * 128 + u * 32 + hi * 8));
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bB[u], acc[t],
                                                          0, 0, 0);
+        if (GRAM)
+          sq[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, afrag, sq[t],
+                                                          0, 0, 0);
       }
   };
 
@@ -328,7 +335,20 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
     }
   }
 
-  if (norm_mode == 2) reduce_invr();
+  if constexpr (GRAM) {
+    if (wave == 0) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg)
+          if (hi * 4 + reg == li) {
+            if (SWIGLU) invr[t * 16 + li] = rsqrtf(sq[t][reg] / K + eps);
+            else if (tile == 0) ssout[split * 32 + t * 16 + li] = sq[t][reg];
+          }
+    }
+  } else {
+    if (norm_mode == 2) reduce_invr();
+  }
 
   if constexpr (SWIGLU) {
     float* up = reinterpret_cast<float*>(atile);   // (MT * 16, 32): atile is dead
@@ -348,7 +368,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
         for (int reg = 0; reg < 4; ++reg) {
           const int m = t * 16 + hi * 4 + reg;
           if (m >= M) continue;
-          const float r = norm_mode == 2 ? invr[m] : 1.f;
+          const float r = invr[m];
           const float v = acc[t][reg] * r;
           const float u = up[m * 32 + wave * 16 + li] * r;
           C[(long)m * (N / 2) + n0 + li] = f2bf(v / (1.f + fast_expf(-v)) * u);

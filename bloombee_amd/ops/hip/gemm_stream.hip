@@ -6,13 +6,18 @@
 // and with the RMS norm of the rows ahead of them (its weight folded into W).
 //
 // The weights are streamed once and bound it. A workgroup owns 16 rows of W (two sets
-// of 16 where the epilogue pairs columns) over all of K: its eight waves take every
-// eighth piece of 128 columns and add up in LDS, so that no partial sums go through
-// memory and nothing has to be folded by another launch. In a decode step a launch
-// costs about 5 us whatever it does (code, arguments and first loads miss caches that
-// the weights swept), which is why the layer's small steps ride here.
-// Every wave keeps DP pieces of W in flight in registers; rows of A come from L2 in
-// fragments, W being the wider of the two streams.
+// of 16 where the epilogue pairs columns) over all of K: its waves take pieces of 128
+// columns in turns and add up in LDS, so that no partial sums go through memory and
+// nothing has to be folded by another launch. In a decode step a launch costs about
+// 5 us whatever it does (code, arguments and first loads miss caches that the weights
+// swept), which is why the layer's small steps ride here.
+//
+// W goes straight to registers, DP pieces ahead. All of A is read by every workgroup, as
+// many bytes as of W at 16 rows: it comes from L2 to a piece of LDS of the wave's own,
+// in whole lines and without registers on the way (fragments straight from L2 took
+// 51 us where this takes 35: 32 rows, 14336 x 4096).
+// Loads of W as nontemporal cost 15% (29.5 us for 25.6: one row, 14336 x 4096).
+//
 // A row's sum of squares for the norm is the diagonal of A A^T, made by the matrix
 // cores from the fragments at hand.
 
@@ -63,31 +68,39 @@ DEVINL void rope_kv_store(const StreamArgs& a, int h, int d, int m, float v, flo
   dst[a.D / 2] = f2bf(u * cs + v * sn);
 }
 
-// Folds the splits of such a projection, (ksplit, M, N) f32: a thread a pair of
-// columns, grid M * N / 2 / 256.
+// Folds the splits of such a projection, (ksplit, M, N) f32, and the rows' squares,
+// (ksplit, 32): a thread a pair of columns, grid M * N / 2 / 256.
 __global__ __launch_bounds__(256) void rope_kv_fold_kernel(
-    StreamArgs a, const float* __restrict__ part, int ksplit) {
+    StreamArgs a, const float* __restrict__ part, const float* __restrict__ squares,
+    int ksplit) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= a.M * (a.N / 2)) return;
   const int m = i / (a.N / 2), c = i % (a.N / 2);
   const int h = c / (a.D / 2), d = c % (a.D / 2);
   const float* p = part + (long)m * a.N + h * a.D + d;
   const long step = (long)a.M * a.N;
-  float v = 0.f, u = 0.f;
+  float v = 0.f, u = 0.f, sq = 0.f;
 #pragma unroll 8
   for (int s = 0; s < ksplit; ++s) {
     v += p[s * step];
     u += p[s * step + a.D / 2];
+    sq += squares[s * 32 + m];
   }
-  rope_kv_store(a, h, d, m, v, u);
+  const float r = rsqrtf(sq / a.K + a.eps);
+  rope_kv_store(a, h, d, m, v * r, u * r);
 }
 
-// NW waves; RT sets of 16 rows of W (EPI_SUM: side by side), MT of 16 rows of A.
-template <int EPI, int RT, int MT, bool NORM, int NW, int DP>
+// NW waves; RT sets of 16 rows of W (EPI_SUM: side by side), MT of 16 rows of A, of
+// which XN * 4 are there.
+template <int EPI, int RT, int MT, int XN, bool NORM, int NW, int DP>
 __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs a) {
   static_assert(EPI == EPI_SUM || RT == 2, "pairs");
-  __shared__ __attribute__((aligned(16))) float sums[NW][RT * MT * 256];
+  static_assert(XN <= MT * 4, "rows");
+  constexpr int XB = MT * 4096;        // bytes of a piece of A
+  constexpr int XT = NW * DP * XB, ST = NW * RT * MT * 1024;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[XT > ST ? XT : ST];
   __shared__ float squares[NW][MT * 16];
+  float* sums = reinterpret_cast<float*>(lds);   // [NW][RT * MT * 256]
   const int tid = threadIdx.x, lane = tid & (WAVE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int li = lane & 15, hi = lane >> 4;
@@ -114,17 +127,20 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs
 
   // a lane's place: 32-bit byte offsets to uniform bases, which move along K
   const unsigned wofs = (unsigned)(li * a.K + hi * 8) * 2;
-  unsigned xofs[MT];
+  // load t of a piece of A is rows 4 t .. +3, 16 B pieces c of row r at c ^ r: sixteen
+  // rows read at one piece cover all banks
+  unsigned xofs[XN];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-    xofs[t] = (unsigned)(min(t * 16 + li, a.M - 1) * a.K + hi * 8) * 2;
-  auto load = [](const unsigned short* base, unsigned ofs, bool once) {
-    const short8* p =
-        reinterpret_cast<const short8*>(reinterpret_cast<const char*>(base) + ofs);
-    return as_bf16x8(once ? __builtin_nontemporal_load(p) : *p);
+  for (int t = 0; t < XN; ++t) {
+    const int row = t * 4 + (lane >> 4), col = (lane & 15) ^ (row & 15);
+    xofs[t] = (unsigned)(min(row, a.M - 1) * a.K + col * 8) * 2;
+  }
+  auto at_byte = [](const unsigned short* base, unsigned ofs) {
+    return reinterpret_cast<const unsigned short*>(
+        reinterpret_cast<const char*>(base) + ofs);
   };
 
-  bf16x8 w[DP][RT][4], x[DP][MT][4];
+  bf16x8 w[DP][RT][4];
   f32x4 acc[RT][MT], sq[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
@@ -133,44 +149,74 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs
     for (int t = 0; t < RT; ++t) acc[t][m] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   const int count = (a.K / 128 - wave + NW - 1) / NW;
+  unsigned char* mine = lds + wave * (DP * XB);
   auto issue = [&](int d, int i) {
     const int k = (i * NW + wave) * 128;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int t = 0; t < XN; ++t)
+      copy16_to_lds(at_byte(a.A + k, xofs[t]), mine + d * XB + t * 1024);
+    // ahead of W in every respect: whoever has waited for W has waited for these
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int t = 0; t < RT; ++t)
-        w[d][t][u] = load(a.W + (long)row0[t] * a.K + k, wofs + u * 64, true);
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        x[d][m][u] = load(a.A + k, xofs[m] + u * 64, false);
-    }
+        w[d][t][u] = as_bf16x8(*reinterpret_cast<const short8*>(
+            at_byte(a.W + (long)row0[t] * a.K + k, wofs + u * 64)));
+    __builtin_amdgcn_sched_barrier(0);
   };
+  auto consume = [&](int d) {
+    // W arrives here, and with it the rows of A that were asked for before it: loads of
+    // a wave return in order
 #pragma unroll
-  for (int d = 0; d < DP; ++d)
-    if (d < count) issue(d, d);
-  for (int i = 0; i < count; i += DP) {
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-    for (int d = 0; d < DP; ++d) {
-      if (i + d < count) {
+      for (int t = 0; t < RT; ++t) asm volatile("" : "+v"(w[d][t][u]));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
+      for (int m = 0; m < MT; ++m) {
+        const bf16x8 x = as_bf16x8(*reinterpret_cast<const short8*>(
+            mine + d * XB + (m * 16 + li) * 256 + (((u * 4 + hi) ^ li) << 4)));
 #pragma unroll
-            for (int t = 0; t < RT; ++t)
-              acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  w[d][t][u], x[d][m][u], acc[t][m], 0, 0, 0);
-            if (NORM)
-              sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  x[d][m][u], x[d][m][u], sq[m], 0, 0, 0);
-          }
-        // keep the loads that follow above the next piece's products
-        __builtin_amdgcn_sched_barrier(0);
-        if (i + d + DP < count) issue(d, i + d + DP);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int t = 0; t < RT; ++t)
+          acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[d][t][u], x,
+                                                              acc[t][m], 0, 0, 0);
+        if (NORM)
+          sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, x, sq[m], 0, 0, 0);
       }
-    }
+    // the loads that take this piece's place stay behind its products
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // The steady part has no conditions on the way, so that the wait for a piece counts
+  // the loads behind it and leaves them in flight.
+  int i = 0;
+  if (count >= 2 * DP) {
+#pragma unroll
+    for (int d = 0; d < DP; ++d) issue(d, d);
+    for (; i + 2 * DP <= count; i += DP)
+#pragma unroll
+      for (int d = 0; d < DP; ++d) {
+        consume(d);
+        issue(d, i + d + DP);
+      }
+  } else {
+#pragma unroll
+    for (int d = 0; d < DP; ++d)
+      if (d < count) issue(d, d);
   }
+  for (; i < count; i += DP)
+#pragma unroll
+    for (int d = 0; d < DP; ++d)
+      if (i + d < count) {
+        consume(d);
+        if (i + d + DP < count) issue(d, i + d + DP);
+      }
+  __syncthreads();   // the sums take the place of the rows
 
   // acc[t][m] holds W rows hi * 4 .. +3 of A row li
 #pragma unroll
@@ -178,7 +224,7 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs
 #pragma unroll
     for (int m = 0; m < MT; ++m)
       *reinterpret_cast<f32x4*>(
-          &sums[wave][(t * MT + m) * 256 + li * 16 + hi * 4]) = acc[t][m];
+          &sums[(wave * RT * MT + t * MT + m) * 256 + li * 16 + hi * 4]) = acc[t][m];
   if (NORM) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -188,9 +234,9 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs
   }
   __syncthreads();
   auto total = [&](int at) {
-    float v = sums[0][at];
+    float v = sums[at];
 #pragma unroll
-    for (int i = 1; i < NW; ++i) v += sums[i][at];
+    for (int i = 1; i < NW; ++i) v += sums[i * RT * MT * 256 + at];
     return v;
   };
   constexpr int OUT = (EPI == EPI_SUM ? RT : 1) * MT * 256;

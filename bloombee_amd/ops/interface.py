@@ -316,8 +316,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
     if (_on_gpu(x) and M <= 32 and x.dtype == torch.bfloat16
             and K % 256 == 0 and N % 64 == 0):
         _require_ext()
-        if (M <= hip_ops.STREAM_ROWS and ss_out is None
-                and (norm is None or norm[0] is None)):
+        if (ss_in is None and ss_out is None
+                and (norm is None or norm[0] is None)
+                and hip_ops.stream_rows(M, N, K)):
             return hip_ops.gemm_stream(x.contiguous(), w, residual, bias,
                                        -1.0 if norm is None else float(norm[1]))
         if norm is not None or ss_out is not None:
@@ -352,43 +353,37 @@ _FUSE_NORM = os.environ.get("BBAMD_FUSE_NORM", "1") != "0"
 
 
 def fuse_norm_linear_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """True when linear(norm=...) will take the fused-kernel path (so the
-    caller can skip emitting a separate rms_norm). Default ON
-    (BBAMD_FUSE_NORM=0 reverts): +2.9% on the flagship decode bench
-    (5289 vs 5140 tok/s) once the row stats ride the producer GEMM's
-    epilogue and the norm weights are folded into the projections
-    (profiles/r02 §13; the naive per-WG A-restream variant measured 16%
-    SLOWER — the chain is what makes it pay)."""
+    """True where a decode GEMM can take its input's rmsnorm along
+    (linear_rope_kv, linear_swiglu), so that the caller need not emit it.
+    Default ON (BBAMD_FUSE_NORM=0 reverts)."""
     K = x.shape[-1]
     return (_FUSE_NORM and _on_gpu(x) and x.numel() // K <= 32
             and x.dtype == torch.bfloat16 and K % 256 == 0
             and w.shape[0] % 64 == 0 and HAVE_HIP_OPS)
 
 
-def row_stats_wanted(x: torch.Tensor) -> bool:
-    """Whether a fused norm of these rows reads the statistics its producer
-    leaves (ss_out): a few rows are summed up by the GEMM that reads them."""
-    return x.numel() // x.shape[-1] > hip_ops.STREAM_ROWS
+def streams_weights(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether linear() of rows that pass fuse_norm_linear_ok sums up the
+    squares of a folded norm itself; elsewhere that takes a pass over x."""
+    return hip_ops.stream_rows(x.numel() // x.shape[-1], *w.shape)
 
 
-def linear_swiglu(x: torch.Tensor, w: torch.Tensor, eps: float,
-                  ss_in: Optional[torch.Tensor] = None) -> torch.Tensor:
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
     """swiglu(rmsnorm(x) @ w^T) of a fused [gate | up] projection whose norm
     weight is folded in, in one launch. Callers gate on fuse_norm_linear_ok."""
     _require_ext()
-    return hip_ops.gemm_swiglu(x.contiguous(), w, eps, ss_in)
+    return hip_ops.gemm_swiglu(x.contiguous(), w, eps)
 
 
-def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, eps: float,
-                   ss_in: Optional[torch.Tensor], Hq: int, Hkv: int, cos, sin,
-                   position_ids, k_pages, v_pages, page_table,
-                   start_pos) -> torch.Tensor:
+def linear_rope_kv(x: torch.Tensor, w: torch.Tensor, eps: float, Hq: int,
+                   Hkv: int, cos, sin, position_ids, k_pages, v_pages,
+                   page_table, start_pos) -> torch.Tensor:
     """rope_kv_write_ of rmsnorm(x) @ w^T: returns (B, T, (Hq+2Hkv)*D) with the
     turned queries; keys and values are in the pages only. Callers gate on
     fuse_norm_linear_ok."""
     _require_ext()
     return hip_ops.gemm_rope_kv(
-        x.contiguous(), w, eps, ss_in, Hq, Hkv, cos, sin,
+        x.contiguous(), w, eps, Hq, Hkv, cos, sin,
         position_ids.int().contiguous() if position_ids is not None else None,
         k_pages, v_pages, page_table, start_pos.int())
 

@@ -10,7 +10,7 @@ from bloombee_amd.ops import reference as ref
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
-ROWS = [1, 2, 7, 8, 9, 16, 17, 25, 32]
+ROWS = [1, 2, 4, 5, 16, 17, 25, 32]
 
 
 def draw(*shape, seed=0, scale=1.0):
@@ -30,8 +30,8 @@ def rms(x, eps):
     return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps)
 
 
-@pytest.mark.parametrize("M", [1, 2, 7, 8])
-@pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 1152), (80, 2944)])
+@pytest.mark.parametrize("M", ROWS)
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 256), (64, 1152), (80, 8064)])
 def test_stream(M, N, K):
     x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
     b, r = draw(N, seed=3), draw(M, N, seed=4)
@@ -43,7 +43,7 @@ def test_stream(M, N, K):
 
 
 def test_stream_refuses_what_it_cannot_do():
-    for M, N, K in ((9, 16, 128), (1, 24, 128), (1, 16, 192)):
+    for M, N, K in ((33, 16, 128), (1, 24, 128), (1, 16, 192)):
         with pytest.raises(RuntimeError):
             ops.hip_ops.gemm_stream(draw(M, K), draw(N, K), None, None, -1.0)
 
@@ -56,11 +56,32 @@ def test_gated_product(M, I, K):
     want = torch.nn.functional.silu(z[:, :I]) * z[:, I:]
     assert ops.fuse_norm_linear_ok(x, w)
     close(ops.linear_swiglu(x, w, 1e-5), want)
-    if ops.row_stats_wanted(x):
-        # squares of the rows as a producer of four stripes leaves them
-        ss = torch.zeros(4, 32, device=DEV)
-        ss[:, :M] = x.float().view(M, 4, -1).pow(2).sum(-1).T
-        close(ops.linear_swiglu(x, w, 1e-5, ss_in=ss.flatten()), want)
+
+
+@pytest.mark.parametrize("M", [17, 32])
+def test_large_weights_keep_the_split_gemm(M):
+    """Beyond 16 rows and 2^25 weights: the split forms, with the rows' squares."""
+    K = 4096
+    x = draw(M, K, seed=1)
+    w = draw(8256, K, seed=2, scale=K ** -0.5)
+    assert not ops.streams_weights(x, w) and ops.streams_weights(x[:16], w)
+    assert ops.streams_weights(x, w[:8192])
+    z = rms(x, 1e-5) @ w.double().T
+    want = torch.nn.functional.silu(z[:, :4128]) * z[:, 4128:]
+    close(ops.linear_swiglu(x, w, 1e-5), want)
+    kp, vp = draw(4, 43, 16, 64, seed=4), draw(4, 43, 64, 16, seed=5)
+    table = torch.arange(4, device=DEV, dtype=torch.int32).view(1, 4)
+    start = torch.tensor([9], dtype=torch.int32, device=DEV)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(64, 128))
+    z = z.view(1, M, -1).float().cpu()
+    kw, vw = kp.float().cpu(), vp.float().cpu()
+    ops.rope_kv_write_(z, 43, 43, cos.cpu(), sin.cpu(), None, kw, vw, table.cpu(),
+                       start.cpu())
+    got = ops.linear_rope_kv(x[None], w, 1e-5, 43, 43, cos, sin, None, kp, vp, table,
+                             start)
+    close(got[..., :43 * 64].cpu(), z[..., :43 * 64].double())
+    close(kp.cpu(), kw.double())
+    close(vp.cpu(), vw.double())
 
 
 @pytest.mark.parametrize("M", ROWS)
@@ -87,7 +108,7 @@ def test_rotations_and_pages(M, Hq, Hkv, D, P, K, ids):
     kw, vw = kp.float().cpu(), vp.float().cpu()
     ops.rope_kv_write_(z, Hq, Hkv, cos.cpu(), sin.cpu(),
                        pos.cpu() if ids else None, kw, vw, table.cpu(), start.cpu())
-    got = ops.linear_rope_kv(x, w, 1e-5, None, Hq, Hkv, cos, sin, pos, kp, vp, table,
+    got = ops.linear_rope_kv(x, w, 1e-5, Hq, Hkv, cos, sin, pos, kp, vp, table,
                              start)
     close(got[..., :Hq * D].cpu(), z[..., :Hq * D].double())
     close(kp.cpu(), kw.double())
