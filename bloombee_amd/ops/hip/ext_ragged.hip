@@ -864,7 +864,7 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
   auto iopt = ids.options();
   auto off = torch::empty({E + 1}, iopt);
   auto sorted = torch::empty({S}, iopt);
-  auto tiles = torch::empty({max_tiles + 1, 2}, iopt);
+  auto tiles = torch::empty({max_tiles + 1, 4}, iopt);
   int* offp = off.data_ptr<int>();
   int* sp = sorted.data_ptr<int>();
   int* tp = tiles.data_ptr<int>();

@@ -31,6 +31,7 @@
 #include "rows.hip"
 
 static constexpr int MOE_MAX_E = 1024;
+static constexpr int MOE_GROUP = 8;
 
 struct GluConst {
   float limit, slope, shift;
@@ -59,8 +60,9 @@ DEVINL int xcd_order(int id, int n) {
 // sort: one workgroup of 1024
 // ---------------------------------------------------------------------------
 
-// off (E+1), sorted (S) slots, tiles (max_tiles + 1, 2): expert (-1 = unused)
-// and first sorted position of every BM-row tile; then the number of tiles.
+// off (E+1), sorted (S) slots, tiles (max_tiles + 1, 4): expert (-1 = unused), first
+// sorted position, group's first tile and number of tiles of every BM-row tile; then
+// the number of tiles. A group is a share of one expert's tiles, at most MOE_GROUP.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     const int* __restrict__ ids, int* __restrict__ off,
     int* __restrict__ sorted, int* __restrict__ tiles, int S, int E, int BM,
@@ -89,18 +91,22 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   const int first = scan[tid] - c;
   if (tid < E) {
     off[tid] = first;
+    const int t0 = tscan[tid] - nt, groups = (nt + MOE_GROUP - 1) / MOE_GROUP;
+    const int per = nt ? (nt + groups - 1) / groups : 1;
     for (int k = 0; k < nt; ++k) {
-      const int at = tscan[tid] - nt + k;
+      const int at = t0 + k, g = k / per * per;
       if (at < max_tiles) {
-        tiles[2 * at] = tid;
-        tiles[2 * at + 1] = first + k * BM;
+        tiles[4 * at] = tid;
+        tiles[4 * at + 1] = first + k * BM;
+        tiles[4 * at + 2] = t0 + g;
+        tiles[4 * at + 3] = min(per, min(nt, max_tiles - t0) - g);
       }
     }
   }
   if (tid == E - 1) off[E] = scan[tid];
-  if (tid == 0) tiles[2 * max_tiles] = min(tscan[MOE_MAX_E - 1], max_tiles);
+  if (tid == 0) tiles[4 * max_tiles] = min(tscan[MOE_MAX_E - 1], max_tiles);
   for (int i = tscan[MOE_MAX_E - 1] + tid; i < max_tiles; i += 1024)
-    tiles[2 * i] = -1;
+    tiles[4 * i] = -1;
   cnt[tid] = first;
   __syncthreads();
   for (int i = tid; i < S; i += 1024) {
@@ -255,15 +261,32 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(
 // tile: grid of column tiles * row tiles; K % 64 == 0
 // ---------------------------------------------------------------------------
 
+// Place of 16 B piece c of a row of four: the lanes that read together (four rows each
+// of 0, 3 at one piece and 1, 2 at the next, by fours) cover all banks.
+DEVINL int moe_piece(int r, int c) {
+  const int g = (r >> 2) & 3;
+  return c ^ ((g & 1) << 1) ^ ((g >> 1) * 3);
+}
+
 // UP: A row = sorted slot / top, out row = sorted position, N = activations
 //     (two planes: 128 per tile, 128 gate rows and 128 up rows of W; one: 256).
 // else: A row = sorted position, out row = slot, 256 columns per tile.
 //
 // A BM x 256 tile per workgroup; each of the four waves holds all BM rows of
 // 64 columns, so a W fragment read from LDS feeds BM / 16 MFMAs. LDS rows are
-// 64 B (32 of K) in four 16 B pieces, piece c of row r at c ^ (r / 4 % 4).
+// 64 B (32 of K) in four 16 B pieces, piece c of row r at moe_piece(r, c).
+//
+// Every expert's weights come from memory once at best; what bounds it is how often
+// they come again. Hence the order of the tiles below: an expert's row tiles take one
+// column after the other together and find W in their XCD's L2. Tiles of several
+// experts in a group of eight: 1430 us for both products at 1400 tokens, two of eight
+// experts, 4096 x 14336, now 1229 (5000 tokens: 4421, 4101).
+// Few rows an expert (BM 64) are a stream of weights: two of three buffers are on
+// their way while the third is computed with (64 tokens: 737 -> 615 us, 4.6 TB/s). At
+// BM 128 that much ahead costs more in L2 than it hides (1340 us for 1229), as does a
+// start of K that differs between columns; tiles of 32 x 32 are slower, too (1289).
 template <int BM, int UP>
-__global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_tile_kernel(
+__global__ __launch_bounds__(256, 2) void moe_tile_kernel(
     const unsigned short* __restrict__ A, const unsigned short* __restrict__ W,
     const int* __restrict__ off, const int* __restrict__ sorted,
     const int* __restrict__ tiles, const float* __restrict__ wts,
@@ -271,20 +294,19 @@ __global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_tile_kernel(
     int K, int lda, int ldc, GluConst glu) {
   constexpr int BK = 32, RB = BK * 2, BN = 256, HN = BN / 2;
   constexpr int AI = BM * 4 / 256, BI = BN * 4 / 256;  // 16 B pieces per thread
-  constexpr int MT = BM / 16, NT = 4;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2][(BM + BN) * RB];
+  constexpr int MT = BM / 16, NT = 4, NB = BM > 64 ? 2 : 3;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NB][(BM + BN) * RB];
 
-  // eight row tiles by all column tiles at a time: the workgroups that run
-  // together share both operands
-  const int nrt = tiles[2 * max_tiles];
+  // an expert's row tiles side by side, column after column: they read the same W
+  // within the time that L2 keeps it
+  const int nrt = tiles[4 * max_tiles];
   const int total = nrt * ntn;
   if ((int)blockIdx.x >= total) return;
   const int id = xcd_order(blockIdx.x, total);
-  const int grp = id / (8 * ntn), in_grp = id % (8 * ntn);
-  const int gsz = min(8, nrt - grp * 8);
-  const int rt = grp * 8 + in_grp % gsz, nt = in_grp / gsz;
-  const int e = tiles[2 * rt];
-  const int p0 = tiles[2 * rt + 1];
+  const int first = tiles[4 * (id / ntn) + 2], gsz = tiles[4 * (id / ntn) + 3];
+  const int rt = first + (id - first * ntn) % gsz, nt = (id - first * ntn) / gsz;
+  const int e = tiles[4 * rt];
+  const int p0 = tiles[4 * rt + 1];
   const int cnt = min(BM, off[e + 1] - p0);
   const int n0 = nt * (UP == 2 ? HN : BN);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -296,14 +318,14 @@ __global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_tile_kernel(
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
     const int ch = (i * 4 + wave) * 64 + lane;
-    const int r = ch / 4, c = (ch % 4) ^ ((r >> 2) & 3);
+    const int r = ch / 4, c = moe_piece(r, ch % 4);
     const int p = p0 + min(r, cnt - 1);
     ap[i] = A + (long)(UP ? sorted[p] / top : p) * lda + c * 8;
   }
 #pragma unroll
   for (int i = 0; i < BI; ++i) {
     const int ch = (i * 4 + wave) * 64 + lane;
-    const int r = ch / 4, c = (ch % 4) ^ ((r >> 2) & 3);
+    const int r = ch / 4, c = moe_piece(r, ch % 4);
     const long wrow =
         UP == 2 ? ((long)e * 2 + r / HN) * N + min(n0 + r % HN, N - 1)
                 : (long)e * N + min(n0 + r, N - 1);
@@ -331,27 +353,39 @@ __global__ __launch_bounds__(256, BM > 64 ? 2 : 3) void moe_tile_kernel(
     for (int n = 0; n < NT; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   issue(0, 0);
-  __syncthreads();
-  int buf = 0;
+  if (NB == 3) issue(BK, 1);  // K >= 64
+  int buf = 0, to = NB - 1;
   for (int k = 0; k < K; k += BK) {
-    if (k + BK < K) issue(k + BK, buf ^ 1);
+    if (NB == 2) {
+      __syncthreads();
+    } else {
+      // this step's loads have landed, the next one's stay on their way
+      if (k + BK < K)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AI + BI) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      // and everyone's; the buffer of the last step is free
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    if (k + (NB - 1) * BK < K) issue(k + (NB - 1) * BK, to);
     bf16x8 wf[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
       wf[n] = as_bf16x8(*reinterpret_cast<const short8*>(
-          lds[buf] + (BM + brow[n]) * RB + ((hi ^ ((brow[n] >> 2) & 3)) * 16)));
+          lds[buf] + (BM + brow[n]) * RB + moe_piece(brow[n], hi) * 16));
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int r = m * 16 + li;
       const bf16x8 af = as_bf16x8(*reinterpret_cast<const short8*>(
-          lds[buf] + r * RB + ((hi ^ ((r >> 2) & 3)) * 16)));
+          lds[buf] + r * RB + moe_piece(r, hi) * 16));
 #pragma unroll
       for (int n = 0; n < NT; ++n)
         acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], af,
                                                             acc[m][n], 0, 0, 0);
     }
-    __syncthreads();
-    buf ^= 1;
+    buf = buf == NB - 1 ? 0 : buf + 1;
+    to = to == NB - 1 ? 0 : to + 1;
   }
 
   // a lane holds columns hi*4..hi*4+3 of row li in every tile
@@ -402,9 +436,9 @@ __global__ __launch_bounds__(256) void moe_simple_kernel(
     GluConst glu) {
   constexpr int NW = UP ? UP : 1, BK = 16;
   __shared__ float al[BK][64 + 4], wl[NW][BK][64 + 4];
-  const int e = tiles[2 * blockIdx.y];
+  const int e = tiles[4 * blockIdx.y];
   if (e < 0) return;
-  const int p0 = tiles[2 * blockIdx.y + 1];
+  const int p0 = tiles[4 * blockIdx.y + 1];
   const int cnt = min(64, off[e + 1] - p0);
   const int n0 = blockIdx.x * 64;
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from bloombee_amd import ops
+from bloombee_amd.ops import ragged
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +91,35 @@ def test_routed_mlp(N, E, top, H, I):
     want = want + h.double()
     assert bool(((got.double() - want).abs()
                  <= tol + 2.0 ** -8 * want.abs() + 1e-6).all())
+
+
+@pytest.mark.parametrize("counts,K,F,W", [
+    ([40, 0, 1, 64, 65], 64, 64, 320),               # tiles of 64 rows, two steps each
+    ([129, 1, 300, 0, 127], 192, 192, 64),           # tiles of 128
+    ([0, 1030, 128, 2, 2400], 128, 320, 64),         # groups of 5 and 4, of 7, 6 and 6
+])
+@pytest.mark.parametrize("planes", [1, 2])
+def test_order_of_tiles(counts, K, F, W, planes):
+    """Experts of none to many row tiles, columns that end within a tile."""
+    E, N = len(counts), sum(counts)
+    gen = torch.Generator().manual_seed(1)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    ids = ids[torch.randperm(N, generator=gen)].to(DEV)
+    wts = torch.rand(N, generator=gen).to(DEV) + 0.5
+    h = draw(N, K, seed=2)
+    up = draw(E, planes, F, K, seed=3, scale=K ** -0.5)
+    down = draw(E, W, F, seed=4, scale=F ** -0.5)
+    rt = ragged.Routing(ids.int()[:, None], wts[:, None], None)
+    got = ragged.moe_experts(h, up, down, rt)[:, 0]
+    for e in range(E):
+        at = ids == e
+        z = torch.einsum("nk,pfk->pnf", h[at].double(), up[e].double())
+        act = (torch.nn.functional.silu(z[0]) * z[1] if planes == 2
+               else z[0].clamp(min=0) ** 2)
+        w = wts[at].double()[:, None]
+        want = act @ down[e].double().T * w
+        # the result's rounding, 2^-9, and that of activations, whose exponentials
+        # and reciprocals take as much again
+        tol = 2.0 ** -8 * want.abs() + 2.0 ** -8 * w * (act.abs()
+                                                      @ down[e].double().abs().T)
+        assert bool(((got[at].double() - want).abs() <= tol + 1e-6).all())
