@@ -156,7 +156,7 @@ void residual_norm(Tensor x, OptTensor parts, OptTensor routed, OptTensor ids,
     a.nw = nw->data_ptr<float>();
     a.h = h->data_ptr();
     a.ldh = h->size(1);
-    vec = vec && a.ldh % 4 == 0;
+    vec = vec && a.ldh % 4 == 0 && (size_t)a.nw % 16 == 0;
   }
   if (other.has_value()) {
     rows_f32(*other);
@@ -598,10 +598,13 @@ Tensor router_gemm(Tensor A, Tensor W) {
   const int M = A.size(0), N = W.size(0), K = A.size(1);
   auto C = torch::empty({1, M, N}, A.options().dtype(at::kFloat));
   if (M == 0) return C;
-  router_gemm_kernel<<<dim3((N + 63) / 64, (M + 31) / 32), 256, 0,
-                       cur_stream()>>>(
-      (const bf16_bits*)A.data_ptr(), (const bf16_bits*)W.data_ptr(),
-      C.data_ptr<float>(), M, N, K);
+  by_bool(N > 16, [&](auto many) {
+    constexpr int NT = decltype(many)::value ? 4 : 1;
+    router_gemm_kernel<NT><<<dim3((N + NT * 16 - 1) / (NT * 16), (M + 15) / 16), 512, 0,
+                             cur_stream()>>>(
+        (const bf16_bits*)A.data_ptr(), (const bf16_bits*)W.data_ptr(),
+        C.data_ptr<float>(), M, N, K);
+  });
   check_launch();
   return C;
 }
