@@ -137,6 +137,35 @@ def test_head_norms_ride_the_rotation():
         close(p.cpu(), q.double(), 4.0)
 
 
+@pytest.mark.parametrize("B,T", [(1, 63), (1, 64), (64, 1), (3, 23), (2, 100), (9, 8)])
+@pytest.mark.parametrize("Hq,Hkv,D,P", [(4, 2, 128, 16), (3, 1, 64, 8), (2, 1, 32, 32),
+                                        (2, 2, 256, 16)])
+@pytest.mark.parametrize("norms", [False, True])
+def test_octets_of_tokens(B, T, Hq, Hkv, D, P, norms):
+    """Many tokens: octets that begin or end within a sequence, one token each; the
+    slots around them stay as they are."""
+    qkv = draw(B, T, (Hq + 2 * Hkv) * D, seed=1)
+    start = (torch.arange(B, dtype=torch.int32) * 5 + 3).to(DEV)
+    maxp = -(-(int(start.max()) + T) // P)
+    gen = torch.Generator().manual_seed(3)
+    table = torch.randperm(B * maxp, generator=gen).view(B, maxp).int().to(DEV)
+    kp, vp = draw(B * maxp, Hkv, P, D, seed=4), draw(B * maxp, Hkv, D, P, seed=5)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(D, 256))
+    pos = (torch.arange(B * T, dtype=torch.int32, device=DEV).view(B, T) % 200
+           if T % 2 else None)
+    hn = (draw(D, seed=6) + 1, draw(D, seed=7) + 1, 1e-6) if norms else None
+    want, kw, vw = qkv.float().cpu(), kp.float().cpu(), vp.float().cpu()
+    ops.rope_kv_write_(want, Hq, Hkv, cos.cpu(), sin.cpu(),
+                       None if pos is None else pos.cpu(), kw, vw, table.cpu(),
+                       start.cpu(), head_norms=hn and (hn[0].float().cpu(),
+                                                       hn[1].float().cpu(), 1e-6))
+    ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, pos, kp, vp, table, start, head_norms=hn)
+    scale = 4.0 if norms else 1.0
+    close(qkv[..., :Hq * D].cpu(), want[..., :Hq * D].double(), scale)
+    close(kp.cpu(), kw.double(), scale)
+    assert torch.equal(vp.cpu().float(), vw)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,room,lengths", [
     (1, 4, 1, 128, 128, [1]),                 # one split, one token
     (1, 4, 2, 128, 300, [300]),               # two splits
