@@ -25,7 +25,6 @@ import math
 from typing import Optional, Tuple
 
 import torch
-import torch.nn.functional as F
 
 from bloombee_amd import ops
 from bloombee_amd.kv.paged import SessionHandle
@@ -273,7 +272,7 @@ class LlamaBlock(torch.nn.Module):
         def lin(x_, w, name):
             # training path honors active LoRA adapters too (the inference
             # path routes through self._lin; keep both consistent)
-            y = F.linear(x_, w)
+            y = training.linear(x_, w)
             ld = getattr(self, "lora_delta", None)
             if ld is not None:
                 d = ld(name, x_)
@@ -287,8 +286,8 @@ class LlamaBlock(torch.nn.Module):
                                        self.Hq, self.Hkv, start_pos, self.scale)
         h2, y = training.add_norm(lin(attn, self.o_w, "o_w"), hidden,
                                   self.post_norm_w, eps)
-        m = training.swiglu(F.linear(y, self.gate_up_w))
-        return h2 + F.linear(m, self.down_w)
+        m = training.swiglu(training.linear(y, self.gate_up_w))
+        return h2 + training.linear(m, self.down_w)
 
     def forward(self, *args, **kw):
         return self.forward_inference(*args, **kw)

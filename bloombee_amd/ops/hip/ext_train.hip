@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "attn_train.hip"
+#include "gemm_grad.hip"
 #include "train_rows.hip"
 
 using torch::Tensor;
@@ -172,7 +173,47 @@ Tensor swiglu_grad(Tensor gu, Tensor gm) {
   return dgu;
 }
 
+// g (M, N) @ w (N, K) -> (M, K); splits <= 0: as many as the sizes want.
+Tensor linear_grad(Tensor g, Tensor w, long splits) {
+  CHECK_T(g, at::kBFloat16);
+  CHECK_T(w, at::kBFloat16);
+  TORCH_CHECK(g.dim() == 2 && w.dim() == 2 && g.size(1) == w.size(0) &&
+                  g.size(0) < (1L << 30) && w.size(0) % 32 == 0 &&
+                  w.size(1) % 256 == 0 && w.numel() > 0 && w.numel() < (1L << 40),
+              "need (M, N) @ (N, K), N % 32 == 0, K % 256 == 0");
+  TORCH_CHECK((size_t)g.data_ptr() % 16 == 0 && (size_t)w.data_ptr() % 16 == 0,
+              "rows must be aligned to 16 bytes");
+  GemmGradArgs a{};
+  a.A = in(g);
+  a.W = in(w);
+  a.M = g.size(0);
+  a.N = w.size(0);
+  a.K = w.size(1);
+  Tensor c = torch::empty({g.size(0), w.size(1)}, g.options());
+  if (a.M == 0) return c;
+  const long tiles = ((a.M + 127) / 128) * (a.K / 256);
+  if (splits <= 0) splits = std::min<long>(32, 512 / std::max<long>(1, tiles));
+  a.splits = (int)std::max<long>(1, std::min<long>(splits, a.N / 256));
+  Tensor part;
+  if (a.splits > 1) {
+    part = torch::empty({a.splits, g.size(0), w.size(1)},
+                        g.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+  } else {
+    a.C = out(c);
+  }
+  gemm_grad_kernel<<<tiles * a.splits, 256, 0, stream()>>>(a);
+  check_launch();
+  if (a.splits > 1) {
+    gemm_grad_fold_kernel<<<(c.numel() / 8 + 255) / 256, 256, 0, stream()>>>(
+        a.part, out(c), c.numel(), a.splits);
+    check_launch();
+  }
+  return c;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("linear_grad", &linear_grad);
   m.def("rope_attention", &rope_attention);
   m.def("rope_attention_grad", &rope_attention_grad);
   m.def("rms_norm_grad", &rms_norm_grad);

@@ -1,5 +1,6 @@
 """Steps of the training path, differentiable: rotary causal attention of whole
-sequences on a fused projection, RMS norms around the residual, the gated product.
+sequences on a fused projection, RMS norms around the residual, the gated product,
+gradients of frozen projections.
 
 Each has a plain torch form, which every tensor can take, and a fused one with
 gradient kernels (module _hip_train) for bf16 tensors on the device. The fused form
@@ -242,3 +243,52 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
     if _fused(gu) and gu.shape[-1] % 16 == 0:
         return _SwiGlu.apply(gu)
     return _swiglu(gu)
+
+
+# ---------------------------------------------------------------------------
+# frozen projections
+# ---------------------------------------------------------------------------
+
+def _few_rows(M: int, N: int, K: int) -> bool:
+    """Whether a split sum along N beats the library's GEMM for the gradient,
+    (M, N) @ (N, K): that one leaves most of the chip idle where the result has
+    few tiles. us, split and library, N x K:
+    28672 x 4096: 33 rows 53, 164; 128 67, 145; 450 156, 279; 1024 296, 360;
+        2000 554, 414
+    20480 x 5120: 300 rows 127, 137; 900 277, 268 (160 tiles)
+    57344 x 8192: 128 rows 192, 298; 300 481, 398
+    6144 x 4096:  33 rows 21, 25; 128 31, 46; 450 50, 48
+    4096 x 4096:  33 rows 17, 22; 128 24, 34; 200 32, 26"""
+    if N % 32 or K % 256:
+        return False
+    tiles = -(-M // 128) * (K // 256)
+    return (M <= 128 and N >= K
+            or M <= 1024 and N >= 4 * K and K <= 5120 and tiles <= 128)
+
+
+class _Linear(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(w)
+        return F.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        w, = ctx.saved_tensors
+        if _again(g) or not _plain(w):
+            return g.matmul(w), None
+        rows, w = g.reshape(-1, g.shape[-1]).contiguous(), w.contiguous()
+        if rows.data_ptr() % 16 or w.data_ptr() % 16:
+            return g.matmul(w), None
+        dx = _ext().linear_grad(rows, w, 0)
+        return dx.view(*g.shape[:-1], w.shape[1]), None
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w^T; w is frozen where the gradient kernel is to take part."""
+    if (torch.is_grad_enabled() and x.requires_grad and _fused(x, w)
+            and w.dim() == 2 and x.dim() >= 2 and x.shape[-1] == w.shape[1]
+            and w.is_contiguous()
+            and _few_rows(x.numel() // x.shape[-1], *w.shape)):
+        return _Linear.apply(x, w)
+    return F.linear(x, w)

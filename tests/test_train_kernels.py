@@ -128,13 +128,54 @@ def steps():
     w = draw(768, seed=9, scale=0.2) + 1
     fused, plain, _ = attention(4, 1, 128, 9, 0)
     x = draw(2, 9, 768, seed=3)
+    m = draw(1024, 768, seed=10, scale=768 ** -0.5)
     return {"attention": (fused, plain, x),
             "norm": (lambda t: sum(training.norm(t, w, 1e-5)),
                      lambda t: t + training._rms(t, w, 1e-5), x),
-            "swiglu": (training.swiglu, training._swiglu, x)}
+            "swiglu": (training.swiglu, training._swiglu, x),
+            "linear": (lambda t: training.linear(t, m),
+                       lambda t: torch.nn.functional.linear(t, m), x)}
 
 
-@pytest.mark.parametrize("name", ["attention", "norm", "swiglu"])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (33, 1056, 256), (127, 4096, 512),
+                                   (128, 256, 256), (129, 2080, 512), (300, 3104, 768)])
+@pytest.mark.parametrize("splits", [0, 1, 2, 7])
+def test_gradient_of_a_projection(M, N, K, splits):
+    """Rows that end within a tile, steps that do not share out evenly."""
+    g, w = draw(M, N, seed=1), draw(N, K, seed=2, scale=N ** -0.5)
+    got = training._ext().linear_grad(g, w, splits)
+    want = g.double() @ w.double()
+    # one rounding to bf16, eight significant bits: half a unit of the last one is
+    # 2^-9 of the next power of two, up to 2^-8 of the value; products are exact in 32
+    # bits, whose sums round N times
+    tol = 2.0 ** -8 * want.abs() + N * 2.0 ** -24 * (g.double().abs()
+                                                     @ w.double().abs())
+    assert bool(((got.double() - want).abs() <= tol).all())
+
+
+def test_projections_at_the_rule():
+    for M, N, K in ((128, 256, 256), (129, 256, 256), (130, 1024, 256),
+                    (1025, 1024, 256), (64, 256, 512), (64, 264, 256)):
+        x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+        g = draw(M, N, seed=3)
+        taken = "_Linear" in type(training.linear(x.requires_grad_(True), w).grad_fn
+                                  ).__name__
+        assert taken == ((M <= 128 or (M == 130)) and N >= K and N % 32 == 0)
+        f, p, e = (grads(fn, [x], [g], dt) for fn, dt in (
+            (lambda t: training.linear(t, w), None),
+            (lambda t: torch.nn.functional.linear(t, w), None),
+            (lambda t: torch.nn.functional.linear(t, w.double()), torch.float64)))
+        check(f, p, e)
+    # gradients whose rows are not aligned, trained weights
+    x, w = draw(4, 256).requires_grad_(True), draw(256, 256, seed=1)
+    y = training.linear(x, w)
+    off = draw(4 * 256 + 1, seed=2)[1:].view(4, 256)
+    assert torch.equal(torch.autograd.grad(y, x, off)[0], off @ w)
+    w.requires_grad_(True)
+    assert torch.autograd.grad(training.linear(x, w).sum(), w)[0].shape == w.shape
+
+
+@pytest.mark.parametrize("name", ["attention", "norm", "swiglu", "linear"])
 def test_watched_operations_stay_plain(name):
     """What looks into the operations gets the plain form's answer."""
     fused, plain, x = steps()[name]
