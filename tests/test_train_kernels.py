@@ -129,12 +129,15 @@ def steps():
     fused, plain, _ = attention(4, 1, 128, 9, 0)
     x = draw(2, 9, 768, seed=3)
     m = draw(1024, 768, seed=10, scale=768 ** -0.5)
+    p = draw(4, 768, seed=11)
     return {"attention": (fused, plain, x),
             "norm": (lambda t: sum(training.norm(t, w, 1e-5)),
                      lambda t: t + training._rms(t, w, 1e-5), x),
             "swiglu": (training.swiglu, training._swiglu, x),
             "linear": (lambda t: training.linear(t, m),
-                       lambda t: torch.nn.functional.linear(t, m), x)}
+                       lambda t: torch.nn.functional.linear(t, m), x),
+            "prompts": (lambda t: training.add_prompts(t, p),
+                        lambda t: training._add_prompts(t, p), x)}
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 32, 256), (33, 1056, 256), (127, 4096, 512),
@@ -175,7 +178,8 @@ def test_projections_at_the_rule():
     assert torch.autograd.grad(training.linear(x, w).sum(), w)[0].shape == w.shape
 
 
-@pytest.mark.parametrize("name", ["attention", "norm", "swiglu", "linear"])
+@pytest.mark.parametrize("name", ["attention", "norm", "swiglu", "linear",
+                                  "prompts"])
 def test_watched_operations_stay_plain(name):
     """What looks into the operations gets the plain form's answer."""
     fused, plain, x = steps()[name]
@@ -229,3 +233,12 @@ def test_trained_norm_weights_get_their_gradients():
     assert not training._fused(x, w)
     h, y = training.norm(x, w, 1e-5)
     assert torch.autograd.grad(y.sum(), w)[0].abs().sum() > 0
+
+
+@pytest.mark.parametrize("B,T,n", [(1, 1, 1), (3, 7, 7), (2, 9, 4), (2, 5, 0)])
+def test_prompts(B, T, n):
+    x, p, g = draw(B, T, 264, seed=1), draw(n, 264, seed=2), draw(B, T, 264, seed=3)
+    f, q, e = (grads(fn, [x, p], [g], dt) for fn, dt in (
+        (training.add_prompts, None), (training._add_prompts, None),
+        (training._add_prompts, torch.float64)))
+    check(f, q, e)
