@@ -57,13 +57,12 @@ DEVINL float quad16_reduce_sum(float x) {
 // short splits.
 // PIPE=1 (NT must be 1): register double-buffered software pipeline — the
 // next tile's K AND V loads are issued before the current tile's MFMA/
-// softmax consume their buffers, so a full iteration of compute covers each
-// load's latency. The r02 PMC diagnosis (WAIT_ANY 82%, ACTIVE 12%, no DRAM
-// credit stalls, and n_split>0 makes things WORSE) shows the kernel is
-// per-wave-latency-bound, not occupancy- or bandwidth-bound: the serial
-// K-wait -> softmax -> PV chain leaves ~2.5 us/iter of HBM idle per wave.
-// Costs ~96 VGPRs of double buffers — free at this grid (B*Hkv WGs = 1
-// WG/CU: occupancy is grid-bound, not VGPR-bound).
+// softmax consume their buffers, and stay in flight behind it: the waits count
+// them (see load_tile below for what that takes). The chain of tiles of a wave bounds
+// short grids: one context of 8000 tokens on 8 workgroups takes 112 us, 192 where
+// every tile's loads were waited for ahead of the one before it. 32 contexts of 2048
+// 54.5 -> 50.1 us, of 8000 184 -> 172 (6.1 TB/s), 97 of 64 to 4000 182 -> 157.
+// Costs ~96 VGPRs of double buffers.
 template <int D, int MAXG, int NT, int PIPE = 0>
 __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
     const unsigned short* __restrict__ q,        // strided, see q_sb/q_sh
@@ -149,26 +148,38 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
     static_assert(NT == 1, "PIPE implies NT==1");
     bf16x8 vb0[NDT], vb1[NDT];
     bf16x8 kb0[NPT][NKK], kb1[NPT][NKK];
-    auto load_tile = [&](bf16x8 (&vb)[NDT], bf16x8 (&kb)[NPT][NKK], int tb) {
-      const int vpos = tb + hi * 8;
-      int vpage = -1;
-      if (vpos < c1) vpage = page_table[b * maxp + vpos / P];
-      const long vrow = ((long)vpage * Hkv + kvh) * D;
+    // Page numbers are looked up two tiles ahead and asked for before the tile in
+    // between, so that waiting for them leaves its loads in flight; nothing is loaded
+    // under a condition, for a wait behind one has to assume that the loads did not
+    // happen and drains everything. Beyond the split's end the last keys and values
+    // are loaded again: weights of zero meet them.
+    const bool pow2 = (P & (P - 1)) == 0;
+    const int plog = 31 - __builtin_clz(P);
+    auto page_of = [&](int pos) { return pow2 ? pos >> plog : pos / P; };
+    const int* table = page_table + (long)b * maxp;
+    const int vlast = (c1 - 1) & ~7;
+    struct Pages { int v, k[NPT]; };
+    auto look_up = [&](Pages& p, int tb) {
+      p.v = table[page_of(min(tb + hi * 8, vlast))];
 #pragma unroll
-      for (int n = 0; n < NDT; ++n) {
-        vb[n] = as_bf16x8(short8{});
-        if (vpage >= 0)
-          vb[n] = as_bf16x8(__builtin_nontemporal_load(
-              reinterpret_cast<const short8*>(
-                  v_pages + (vrow + li + 16 * n) * P + (vpos % P))));
-      }
+      for (int n = 0; n < NPT; ++n)
+        p.k[n] = table[page_of(min(tb + li + 16 * n, c1 - 1))];
+    };
+    auto load_tile = [&](bf16x8 (&vb)[NDT], bf16x8 (&kb)[NPT][NKK], int tb,
+                         const Pages& p) {
+      const int vpos = min(tb + hi * 8, vlast);
+      const unsigned short* vrow = v_pages + ((long)p.v * Hkv + kvh) * D * P +
+                                   (long)li * P + (vpos - page_of(vpos) * P);
+#pragma unroll
+      for (int n = 0; n < NDT; ++n)
+        vb[n] = as_bf16x8(__builtin_nontemporal_load(
+            reinterpret_cast<const short8*>(vrow + 16 * n * P)));
 #pragma unroll
       for (int n = 0; n < NPT; ++n) {
-        const int pos = tb + li + 16 * n;
-        const int cpos = min(pos, c1 - 1);
-        const int page = page_table[b * maxp + cpos / P];
-        const unsigned short* krow = k_pages + ((long)page * Hkv) * P * D +
-                                     head_slab_k + (long)(cpos % P) * D;
+        const int pos = min(tb + li + 16 * n, c1 - 1);
+        const unsigned short* krow = k_pages + (long)p.k[n] * Hkv * P * D +
+                                     head_slab_k +
+                                     (long)(pos - page_of(pos) * P) * D;
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk)
           kb[n][kk] = as_bf16x8(__builtin_nontemporal_load(
@@ -232,15 +243,27 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
         acc_o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[n], pfrag,
                                                            acc_o[n], 0, 0, 0);
     };
-    if (tbs < c1) load_tile(vb0, kb0, tbs);
-    for (int tb = tbs; tb < c1; tb += 2 * TSTRIDE) {
-      if (tb + TSTRIDE < c1) load_tile(vb1, kb1, tb + TSTRIDE);
+    if (tbs < c1) {
+      Pages pa, pb;
+      look_up(pa, tbs);
+      look_up(pb, tbs + TSTRIDE);
+      load_tile(vb0, kb0, tbs, pa);
       __builtin_amdgcn_sched_barrier(0);
-      compute_tile(vb0, kb0, tb);
-      if (tb + TSTRIDE >= c1) break;
-      if (tb + 2 * TSTRIDE < c1) load_tile(vb0, kb0, tb + 2 * TSTRIDE);
-      __builtin_amdgcn_sched_barrier(0);
-      compute_tile(vb1, kb1, tb + TSTRIDE);
+      int tb = tbs;
+      while (true) {
+        look_up(pa, tb + 2 * TSTRIDE);
+        load_tile(vb1, kb1, tb + TSTRIDE, pb);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_tile(vb0, kb0, tb);
+        tb += TSTRIDE;
+        if (tb >= c1) break;
+        look_up(pb, tb + 2 * TSTRIDE);
+        load_tile(vb0, kb0, tb + TSTRIDE, pa);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_tile(vb1, kb1, tb);
+        tb += TSTRIDE;
+        if (tb >= c1) break;
+      }
     }
   } else {
   // wave w owns NT adjacent tiles starting at tile w*NT, stride 4*NT tiles

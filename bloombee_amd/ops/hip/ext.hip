@@ -217,9 +217,9 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
     return e ? std::atoi(e) : 2;
   }();
   // Software-pipelined variant (next tile's K+V double-buffered in
-  // registers; r02 WAIT_ANY diagnosis): DEFAULT — 50 us / 5.4 TB/s at B32
-  // ctx2048 and 6.3 TB/s (achievable-HBM ceiling) at ctx8192 vs 59-62 us
-  // for the NT variants. BBAMD_ATTN_PF=0 reverts to the NT path.
+  // registers, its loads in flight behind this tile's): DEFAULT — 50 us /
+  // 5.4 TB/s at B32 ctx2048 and 6.1 TB/s at ctx 8000 vs 59-62 us
+  // for the NT variants at ctx2048. BBAMD_ATTN_PF=0 reverts to the NT path.
   static const bool pf_env = [] {
     const char* e = std::getenv("BBAMD_ATTN_PF");
     return !e || std::atoi(e) != 0;
@@ -305,16 +305,15 @@ static torch::Tensor attn_decode_core(
       const char* e = std::getenv("BBAMD_ATTN_PF");
       return !e || std::atoi(e) != 0;
     }();
-    // pipelined variant: 254 VGPRs -> 2 waves/SIMD -> 512 WGs fill the chip
-    // (measured: B32 ns=2 50 us / 5.4 TB/s vs 59 at 768-1024 WGs)
+    // pipelined variant: 244 VGPRs -> 2 waves/SIMD -> 512 WGs fill the chip
     const long target = (pf_env0 && D <= 128) ? 512
                         : (nt_env0 >= 2 && D <= 128) ? 768 : 1024;
     const long units = std::max(1, B * Hkv * nch), room = (long)maxp * P;
     if (units > target) {
       // More units than fit at once: contexts of a large batch differ, and a
       // workgroup with a long one outlasts the rest. Shares of 1024 tokens even it
-      // out (97 sequences of 64 to 4000 tokens, 8 heads of 128: 183 us unsplit,
-      // 152 us so).
+      // out (97 sequences of 64 to 4000 tokens, 8 heads of 128: 168 us unsplit,
+      // 157 us so).
       share = 1024;
       n_split = (int)std::min(32L, (room + share - 1) / share);
     } else {

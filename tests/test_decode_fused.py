@@ -173,8 +173,8 @@ def test_octets_of_tokens(B, T, Hq, Hkv, D, P, norms):
     (1, 71, 1, 64, 2000, [777]),              # a group in five chunks
     (65, 8, 8, 64, 2100, None),               # more units than fit: even shares
 ])
-def test_decode_attention_splits(B, Hq, Hkv, D, room, lengths):
-    P = 16
+@pytest.mark.parametrize("P", [8, 16, 24])        # 24: pages found by division
+def test_decode_attention_splits(B, Hq, Hkv, D, room, lengths, P):
     gen = torch.Generator().manual_seed(B)
     if lengths is None:
         lengths = torch.randint(1, room + 1, (B,), generator=gen).tolist()
