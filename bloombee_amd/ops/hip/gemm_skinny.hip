@@ -318,22 +318,27 @@ __global__ __launch_bounds__(256) void gemm_skinny_v2_kernel(
     store_a();
     __syncthreads();
   }
-  for (int k = k0; k < k1; k += KSTEP) {
+  auto stage = [&](int k, auto more) {
     // the barriers keep the scheduler from sinking a set's loads down to
     // their first use
-    if (k + KSTEP < k1) load_a(k + KSTEP);
+    if constexpr (decltype(more)::value) load_a(k + KSTEP);
     issue1(k + 128);
     __builtin_amdgcn_sched_barrier(0);
     mfma_set(bB0, 0);
-    if (k + KSTEP < k1) issue0(k + KSTEP);
+    if constexpr (decltype(more)::value) issue0(k + KSTEP);
     __builtin_amdgcn_sched_barrier(0);
     mfma_set(bB1, 1);
-    if (k + KSTEP < k1) {
+    if constexpr (decltype(more)::value) {
       __syncthreads();  // everyone done reading stage s
       store_a();
       __syncthreads();
     }
-  }
+  };
+  // the last stage apart: a wait behind loads under a condition has to assume that
+  // they were not issued, and drains them
+  int k = k0;
+  for (; k + KSTEP < k1; k += KSTEP) stage(k, std::true_type{});
+  if (k < k1) stage(k, std::false_type{});
 
   if constexpr (GRAM) {
     if (wave == 0) {

@@ -227,21 +227,25 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(
   load_w(b0, 0);
   store_a();
   __syncthreads();
-  for (int k = 0; k < K; k += KSTEP) {
-    const bool more = k + KSTEP < K;
-    if (more) load_a(k + KSTEP);
+  auto stage = [&](int k, auto more) {
+    if constexpr (decltype(more)::value) load_a(k + KSTEP);
     load_w(b1, k + 128);
     __builtin_amdgcn_sched_barrier(0);
     mma(b0, 0);
-    if (more) load_w(b0, k + KSTEP);
+    if constexpr (decltype(more)::value) load_w(b0, k + KSTEP);
     __builtin_amdgcn_sched_barrier(0);
     mma(b1, 1);
-    if (more) {
+    if constexpr (decltype(more)::value) {
       __syncthreads();
       store_a();
       __syncthreads();
     }
-  }
+  };
+  // the last stage apart: a wait behind loads under a condition has to assume that
+  // they were not issued, and drains them
+  int k = 0;
+  for (; k + KSTEP < K; k += KSTEP) stage(k, std::true_type{});
+  stage(k, std::false_type{});
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
