@@ -255,8 +255,7 @@ def _layer_numbers(model: str, args) -> dict:
         kv.page_table()
         step = lambda: stack.forward_inference(x, kv, pos)
         step()
-        # mixtral's routing (bincount) cannot be captured: it runs eagerly
-        if on_gpu and cfg.model_type != "mixtral":
+        if on_gpu:
             step()
             sync()
             graph = torch.cuda.CUDAGraph()

@@ -801,10 +801,10 @@ torch::Tensor gemm_w4(torch::Tensor A, torch::Tensor Wq, torch::Tensor scale,
 
 // Where the one-launch kernel (gemm_stream.hip) is the faster one. Every workgroup of it
 // reads all of A, twice the bytes of its W at 32 rows: beyond 16 rows that outweighs the
-// launch it saves once W is large. 4096 x 4096 8.8 us at 1 row, 10.1 at 16, 11.9 at 32
-// (split GEMM and its fold: 14.0, 14.6, 15.3), 14336 x 4096 24.8, 28.5, 35.0 (29.7,
-// 30.7, 32.0), [gate | up] of 4096 x 14336 with its product 46.9, 51.7, 58.9 (55.3, 52,
-// 55).
+// launch it saves once W is large. us, one launch and split GEMM with its fold:
+// 4096 x 4096 1 row 8.2, 12.2; 16 rows 10.4, 13.0; 32 rows 12.6, 14.2; 14336 x 4096
+// 23.8, 28.5; 30.1, 29.8; 37.6, 31.5; [gate | up] of 4096 x 14336 with its product, which
+// is not split, at 16 rows 51.3, 49.9; at 32 58.9, 53.8.
 static bool stream_rows(long M, long N, long K) {
   return M <= 16 || (M <= 32 && N * K <= (32L << 20));
 }
