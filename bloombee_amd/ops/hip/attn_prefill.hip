@@ -272,7 +272,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
       a.pml[at * 2] = GENERAL ? m : m * sc2;
       a.pml[at * 2 + 1] = l;
     }
-    if (l > 0.f) {
+    if (l != 0.f) {   // NaN sums, too: the fold is to see them
 #pragma unroll
       for (int n = 0; n < ND; ++n)
 #pragma unroll
@@ -283,7 +283,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     }
     return;
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l != 0.f ? 1.f / l : 0.f;
   unsigned short* op =
       a.out + (long)b * a.o_sb + (long)tok * a.o_st + (long)head * a.o_sh + hi * 4;
 #pragma unroll
@@ -298,7 +298,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
 }
 
 // Folds the splits of a row: a wave a row, grid rows of all units / 4. A split that
-// saw nothing has a sum of zero and left its values unwritten.
+// saw nothing has a sum of zero and left its values unwritten; a NaN in a split makes
+// the row NaN.
 template <int D>
 __global__ __launch_bounds__(256) void attn_prefill_fold_kernel(PrefillArgs a) {
   constexpr int V = D >= 128 ? D / 64 : 1;   // columns of a lane
@@ -313,10 +314,10 @@ __global__ __launch_bounds__(256) void attn_prefill_fold_kernel(PrefillArgs a) {
   if (lane < a.n_split) {
     m = a.pml[(lane * rows + at) * 2];
     l = a.pml[(lane * rows + at) * 2 + 1];
-    if (!(l > 0.f)) m = NEG_BIG;
+    if (l == 0.f) m = NEG_BIG;
   }
   const float top = wave_reduce_max(m);
-  if (l > 0.f) w = fast_exp2(m - top);
+  if (l != 0.f) w = fast_exp2(m - top);
   l = wave_reduce_sum(w * l);
   const int col = min(lane * V, D - V);
   float o[V];
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(256) void attn_prefill_fold_kernel(PrefillArgs a) {
     for (int e = 0; e < V; ++e) o[e] += ws * p[e];
   }
   if (lane * V >= D) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l != 0.f ? 1.f / l : 0.f;
   const int unit = (int)(at / R), r = (int)(at % R);
   unsigned short* op = a.out + (long)(unit / a.Hkv) * a.o_sb +
                        (long)(r / a.G) * a.o_st +

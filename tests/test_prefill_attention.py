@@ -90,3 +90,30 @@ def test_queries_of_a_fused_projection(case):
     got = ops.attn_paged_qkv(qkv.to(DEV), Hq, Hkv, kp.to(DEV), vp.to(DEV),
                              table.to(DEV), qs.to(DEV))
     close(got, want)
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[7]], ids=["split", "unsplit"])
+@pytest.mark.parametrize("form", ["plain", "alibi"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")], ids=str)
+@pytest.mark.parametrize("where", ["key", "query"])
+def test_rows_without_a_finite_result_say_so(case, form, bad, where):
+    """A row that meets a NaN or an infinite score is NaN whether its keys are split
+    or not; rows that do not are as they were."""
+    B, Hq, Hkv, D, P, T, starts, room, _ = case
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=T)
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    if where == "key":                       # of one head, seen from the tenth token on
+        pos = starts[0] + 9
+        kp[int(table[0, pos // P]), 0, pos % P, 5] = bad
+    else:
+        q[0, 1, 7, 3] = bad
+    qs = torch.tensor(starts, dtype=torch.int32)
+    slopes = ops.alibi_slopes_for(Hq) if form == "alibi" else None
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long(),
+                          alibi_slopes=slopes)
+    assert bool(want.isnan().any()) and bool(want.isfinite().any())
+    got = ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)],
+                         alibi_slopes=slopes).cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    close(got.nan_to_num(0), want.nan_to_num(0))
