@@ -18,6 +18,12 @@ static hipStream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
                   (x).scalar_type() == (st),                                  \
               #x " must be a contiguous device tensor of ", toString(st))
 
+// Rows that are read 16 bytes at a time, by the kernels or by copies to LDS.
+#define CHECK_ROWS(x)                                                         \
+  CHECK_T(x, at::kBFloat16);                                                  \
+  TORCH_CHECK((size_t)(x).data_ptr() % 16 == 0,                               \
+              #x " must be aligned to 16 bytes")
+
 static void check_launch() {
   const hipError_t e = hipGetLastError();
   TORCH_CHECK(e == hipSuccess, "kernel launch: ", hipGetErrorString(e));
@@ -34,7 +40,7 @@ static unsigned short* out(const Tensor& t) {
 static TrainAttnArgs attn_args(const Tensor& qkv, long Hq, long Hkv,
                                const Tensor& cos_t, const Tensor& sin_t, long start,
                                double scale) {
-  CHECK_T(qkv, at::kBFloat16);
+  CHECK_ROWS(qkv);
   CHECK_T(cos_t, at::kFloat);
   CHECK_T(sin_t, at::kFloat);
   TORCH_CHECK(Hkv > 0 && Hq > 0 && Hq % Hkv == 0, "heads: ", Hq, " on ", Hkv);
@@ -103,8 +109,8 @@ Tensor rope_attention_grad(Tensor gout, Tensor qkv, Tensor qk, Tensor o32,
                            long start, double scale) {
   TrainAttnArgs a = attn_args(qkv, Hq, Hkv, cos_t, sin_t, start, scale);
   const long D = qkv.size(2) / (Hq + 2 * Hkv), B = a.B, T = a.T;
-  CHECK_T(gout, at::kBFloat16);
-  CHECK_T(qk, at::kBFloat16);
+  CHECK_ROWS(gout);
+  CHECK_ROWS(qk);
   CHECK_T(o32, at::kFloat);
   CHECK_T(lse, at::kFloat);
   TORCH_CHECK(gout.numel() == B * T * Hq * D && o32.numel() == gout.numel() &&
@@ -131,15 +137,15 @@ Tensor rope_attention_grad(Tensor gout, Tensor qkv, Tensor qk, Tensor o32,
 }
 
 Tensor rms_norm_grad(Tensor x, Tensor w, Tensor gy, OptTensor gx, double eps) {
-  CHECK_T(x, at::kBFloat16);
-  CHECK_T(w, at::kBFloat16);
-  CHECK_T(gy, at::kBFloat16);
+  CHECK_ROWS(x);
+  CHECK_ROWS(w);
+  CHECK_ROWS(gy);
   const long H = x.size(-1);
   TORCH_CHECK(H % 8 == 0 && H <= 16384 && w.numel() == H &&
                   gy.numel() == x.numel(),
               "bad norm shapes");
   if (gx.has_value()) {
-    CHECK_T((*gx), at::kBFloat16);
+    CHECK_ROWS((*gx));
     TORCH_CHECK(gx->numel() == x.numel());
   }
   Tensor dx = torch::empty_like(x);
@@ -159,8 +165,8 @@ Tensor rms_norm_grad(Tensor x, Tensor w, Tensor gy, OptTensor gx, double eps) {
 }
 
 Tensor swiglu_grad(Tensor gu, Tensor gm) {
-  CHECK_T(gu, at::kBFloat16);
-  CHECK_T(gm, at::kBFloat16);
+  CHECK_ROWS(gu);
+  CHECK_ROWS(gm);
   const long I = gm.size(-1);
   TORCH_CHECK(I % 8 == 0 && gu.size(-1) == 2 * I && gu.numel() == 2 * gm.numel(),
               "bad product shapes");
@@ -175,14 +181,12 @@ Tensor swiglu_grad(Tensor gu, Tensor gm) {
 
 // g (M, N) @ w (N, K) -> (M, K); splits <= 0: as many as the sizes want.
 Tensor linear_grad(Tensor g, Tensor w, long splits) {
-  CHECK_T(g, at::kBFloat16);
-  CHECK_T(w, at::kBFloat16);
+  CHECK_ROWS(g);
+  CHECK_ROWS(w);
   TORCH_CHECK(g.dim() == 2 && w.dim() == 2 && g.size(1) == w.size(0) &&
                   g.size(0) < (1L << 30) && w.size(0) % 32 == 0 &&
                   w.size(1) % 256 == 0 && w.numel() > 0 && w.numel() < (1L << 40),
               "need (M, N) @ (N, K), N % 32 == 0, K % 256 == 0");
-  TORCH_CHECK((size_t)g.data_ptr() % 16 == 0 && (size_t)w.data_ptr() % 16 == 0,
-              "rows must be aligned to 16 bytes");
   GemmGradArgs a{};
   a.A = in(g);
   a.W = in(w);

@@ -59,6 +59,12 @@ def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
                     for t in (x, *weights)))
 
 
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """t as the kernels read it: contiguous, and 16 bytes at a time."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _again(*grads: torch.Tensor) -> bool:
     """The gradient is itself recorded, or taken for a batch at once."""
     return torch.is_grad_enabled() or not all(_plain(g) for g in grads)
@@ -106,7 +112,7 @@ def _attention(qkv, cos, sin, Hq, Hkv, start, scale):
 class _Attention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, qkv, cos, sin, Hq, Hkv, start, scale, keep):
-        x = qkv.contiguous()
+        x = _rows(qkv)
         out, qk, out32, lse = _ext().rope_attention(x, Hq, Hkv, cos, sin, start,
                                                     scale, keep)
         if keep:
@@ -122,7 +128,7 @@ class _Attention(torch.autograd.Function):
             dx = _vjp(lambda x: _attention(x, cos, sin, *ctx.sizes), qkv, g)
         else:
             dx = _ext().rope_attention_grad(
-                g.contiguous(), qkv.contiguous(), qk, out32, lse, Hq, Hkv, cos, sin,
+                _rows(g), _rows(qkv), qk, out32, lse, Hq, Hkv, cos, sin,
                 start, scale)
         return dx, None, None, None, None, None, None, None
 
@@ -159,8 +165,7 @@ def _norm_grad(h, w, eps, gh, gy):
     """Of h and its norm together."""
     if _again(gh, gy):
         return gh + _vjp(lambda t: _rms(t, w, eps), h, gy)
-    return _ext().rms_norm_grad(h.contiguous(), w.contiguous(), gy.contiguous(),
-                                gh.contiguous(), eps)
+    return _ext().rms_norm_grad(_rows(h), _rows(w), _rows(gy), _rows(gh), eps)
 
 
 class _Norm(torch.autograd.Function):
@@ -168,7 +173,7 @@ class _Norm(torch.autograd.Function):
     def forward(ctx, x, w, eps):
         ctx.save_for_backward(x, w)
         ctx.eps = eps
-        return x.view_as(x), interface.rms_norm(x, w, eps)
+        return x.view_as(x), interface.rms_norm(_rows(x), _rows(w), eps)
 
     @staticmethod
     def backward(ctx, gx, gy):
@@ -179,7 +184,7 @@ class _Norm(torch.autograd.Function):
 class _AddNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, x, w, eps):
-        h, y = interface.rms_norm_residual(a, x, w, eps)
+        h, y = interface.rms_norm_residual(_rows(a), _rows(x), _rows(w), eps)
         ctx.save_for_backward(h, w)
         ctx.eps = eps
         return h, y
@@ -228,14 +233,14 @@ class _SwiGlu(torch.autograd.Function):
     @staticmethod
     def forward(ctx, gu):
         ctx.save_for_backward(gu)
-        return interface.swiglu(gu)
+        return interface.swiglu(_rows(gu))
 
     @staticmethod
     def backward(ctx, gm):
         gu, = ctx.saved_tensors
         if _again(gm):
             return _vjp(_swiglu, gu, gm)
-        return _ext().swiglu_grad(gu.contiguous(), gm.contiguous())
+        return _ext().swiglu_grad(_rows(gu), _rows(gm))
 
 
 def swiglu(gu: torch.Tensor) -> torch.Tensor:

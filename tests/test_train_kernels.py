@@ -242,3 +242,40 @@ def test_prompts(B, T, n):
         (training.add_prompts, None), (training._add_prompts, None),
         (training._add_prompts, torch.float64)))
     check(f, q, e)
+
+
+@pytest.mark.parametrize("name", ["attention", "norm", "swiglu", "linear",
+                                  "prompts"])
+def test_rows_at_any_address(name):
+    """Tensors that begin at two bytes into a line are read as they are elsewhere."""
+    fused, _, x = steps()[name]
+
+    def off(t):
+        wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        wide[1:].copy_(t.reshape(-1))
+        return wide[1:].view(t.shape)
+
+    y = x.clone().requires_grad_(True)
+    z = off(x).requires_grad_(True)
+    assert z.data_ptr() % 16 == 2 and z.is_contiguous()
+    a, b = fused(y), fused(z)
+    g = draw(*a.shape, seed=7)
+    assert torch.equal(a, b)
+    want, = torch.autograd.grad(a, y, g)
+    got, = torch.autograd.grad(b, z, off(g))
+    # an unaligned gradient may take the library's product
+    assert away(got, want.double()) < 2.0 ** -8
+
+
+def test_bindings_refuse_unaligned_rows():
+    ext = training._ext()
+    _, _, x = steps()["attention"]
+    wide = torch.empty(x.numel() + 1, dtype=x.dtype, device=DEV)
+    odd = wide[1:].view(x.shape)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(128, 16))
+    with pytest.raises(RuntimeError, match="aligned"):
+        ext.rope_attention(odd, 4, 1, cos, sin, 0, 1.0, True)
+    out, qk, o32, lse = ext.rope_attention(x, 4, 1, cos, sin, 0, 1.0, True)
+    off = torch.empty(out.numel() + 1, dtype=x.dtype, device=DEV)[1:].view(out.shape)
+    with pytest.raises(RuntimeError, match="aligned"):
+        ext.rope_attention_grad(off, x, qk, o32, lse, 4, 1, cos, sin, 0, 1.0)
