@@ -809,9 +809,12 @@ static bool stream_rows(long M, long N, long K) {
   return M <= 16 || (M <= 32 && N * K <= (32L << 20));
 }
 
-static StreamArgs stream_args(const torch::Tensor& A, const torch::Tensor& W) {
+// A's rows go to LDS by 16-byte copies: a view that does not begin at 16 bytes is copied
+// first. W is read by loads to registers, which any address of an element suits.
+static StreamArgs stream_args(torch::Tensor& A, const torch::Tensor& W) {
   CHECK_DEV(A); CHECK_BF16(A); CHECK_CONTIG(A);
   CHECK_DEV(W); CHECK_BF16(W); CHECK_CONTIG(W);
+  if ((size_t)A.data_ptr() % 16 != 0) A = A.clone();
   StreamArgs a{};
   a.K = A.size(-1);
   a.M = A.numel() / a.K;

@@ -189,3 +189,32 @@ def test_decode_attention_splits(B, Hq, Hkv, D, room, lengths, P):
     # weights enter the value product in bf16: 2^-9 of the largest value
     err = (got.view(B, Hq, D).float() - want[:, :, 0]).abs().max()
     assert err <= 2 * 4.5 * 2.0 ** -9, err
+
+
+def off(t):
+    """The same at two bytes into a line."""
+    wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+    wide[1:].copy_(t.reshape(-1))
+    assert wide[1:].data_ptr() % 16 == 2
+    return wide[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("M", [1, 5, 16, 17, 32])
+def test_rows_at_any_address(M):
+    x, w, r = draw(M, 512, seed=1), draw(64, 512, seed=2, scale=0.05), draw(M, 64)
+    assert torch.equal(ops.linear(off(x), w, residual=r), ops.linear(x, w, residual=r))
+    assert torch.equal(ops.linear(x, off(w)), ops.linear(x, w))
+    assert torch.equal(ops.linear_swiglu(off(x), w, 1e-5), ops.linear_swiglu(x, w, 1e-5))
+    table = torch.arange(4, device=DEV, dtype=torch.int32).view(1, 4)
+    start = torch.tensor([9], dtype=torch.int32, device=DEV)
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(32, 128))
+    w = draw(128, 512, seed=2, scale=0.05)
+    outs = []
+    for rows in (x, off(x)):
+        kp, vp = (torch.zeros(4, 1, *s, dtype=torch.bfloat16, device=DEV)
+                  for s in ((16, 32), (32, 16)))
+        q = ops.linear_rope_kv(rows[None], w, 1e-5, 2, 1, cos, sin, None, kp, vp, table,
+                               start)
+        outs.append((q[..., :64], kp, vp))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
