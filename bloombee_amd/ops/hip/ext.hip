@@ -817,10 +817,10 @@ static StreamArgs stream_args(torch::Tensor& A, const torch::Tensor& W) {
   if ((size_t)A.data_ptr() % 16 != 0) A = A.clone();
   StreamArgs a{};
   a.K = A.size(-1);
+  TORCH_CHECK(W.dim() == 2 && W.size(1) == a.K && a.K > 0, "A/W K mismatch");
   a.M = A.numel() / a.K;
   a.N = W.size(0);
-  TORCH_CHECK(W.dim() == 2 && W.size(1) == a.K, "A/W K mismatch");
-  TORCH_CHECK(a.M >= 1 && a.M <= 32, "1 to 32 rows, got ", a.M);
+  TORCH_CHECK(a.M <= 32, "at most 32 rows, got ", a.M);
   a.A = bf_ptr(A);
   a.W = bf_ptr(W);
   return a;
@@ -857,6 +857,7 @@ torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
                 bias->is_contiguous() && bias->numel() == a.N, "bad bias");
     a.bias = bf_ptr(*bias);
   }
+  if (a.M == 0) return C;
   by_rows(a.M, [&](auto mt, auto xn) {
     constexpr int MT = decltype(mt)::value, XN = decltype(xn)::value;
     constexpr int DP = MT == 1 ? 4 : 1;
@@ -894,6 +895,7 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   auto C = torch::empty(sizes, A.options());
   a.C = bf_ptr_mut(C);
   a.eps = eps;
+  if (a.M == 0) return C;
   if (!stream_rows(a.M, a.N, a.K)) {
     launch_skinny_fused<true>(a, a.K, 1, nullptr, nullptr);
     return C;
@@ -947,6 +949,7 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq
   sizes.back() = a.N;
   auto C = torch::empty(sizes, A.options());
   a.C = bf_ptr_mut(C);
+  if (a.M == 0) return C;
   a.eps = eps;
   a.cos_t = cos_t.data_ptr<float>();
   a.sin_t = sin_t.data_ptr<float>();
@@ -1029,6 +1032,7 @@ torch::Tensor gemm_skinny(torch::Tensor A, torch::Tensor W,
   auto sizes = A.sizes().vec();
   sizes.back() = N;
   auto C = torch::empty(sizes, A.options());
+  if (M == 0) return C;   // missing rows repeat row M - 1
   const unsigned short* rp = nullptr;
   if (residual.has_value()) {
     TORCH_CHECK(residual->is_contiguous() && residual->numel() == (long)M * N);

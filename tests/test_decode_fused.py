@@ -218,3 +218,10 @@ def test_rows_at_any_address(M):
         outs.append((q[..., :64], kp, vp))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+def test_no_rows():
+    x, w = draw(0, 512), draw(64, 512)
+    for rows in (x, x.view(0, 1, 512), x.view(1, 0, 512)):
+        assert ops.linear(rows, w).shape == (*rows.shape[:-1], 64)
+        assert ops.linear_swiglu(rows, w, 1e-5).shape == (*rows.shape[:-1], 32)
