@@ -599,6 +599,8 @@ std::vector<torch::Tensor> norm_route(torch::Tensor a,
                   top <= E && res.has_value() == norm_w.has_value(),
               "bad router shapes");
   const bool norm = norm_w.has_value();
+  // rows that are handed on as they are go to LDS by 16-byte copies in the experts
+  if (!norm && (size_t)a.data_ptr() % 16 != 0) a = a.clone();
   if (norm) {
     CHECK_DEV_ALL2((*res), (*norm_w)); CHECK_BF16((*res)); CHECK_BF16((*norm_w));
     CHECK_CONTIG((*res)); CHECK_CONTIG((*norm_w));

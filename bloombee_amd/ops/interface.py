@@ -405,7 +405,10 @@ def routed_mlp_ok(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
     E, H, I = down.shape
     return (_on_gpu(x) and x.dtype == torch.bfloat16 and x.numel() > 0
             and E <= 64 and 1 <= top <= E and H % 64 == 0 and I % 64 == 0
-            and H <= 16384 and gate_up.is_contiguous() and down.is_contiguous())
+            and H <= 16384
+            # read by 16-byte copies to LDS
+            and all(w.is_contiguous() and w.data_ptr() % 16 == 0
+                    for w in (gate_up, down)))
 
 
 def routed_mlp(a: torch.Tensor, router_w: torch.Tensor, gate_up: torch.Tensor,

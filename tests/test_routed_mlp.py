@@ -123,3 +123,24 @@ def test_order_of_tiles(counts, K, F, W, planes):
         tol = 2.0 ** -8 * want.abs() + 2.0 ** -8 * w * (act.abs()
                                                       @ down[e].double().abs().T)
         assert bool(((got[at].double() - want).abs() <= tol + 1e-6).all())
+
+
+@pytest.mark.parametrize("N", [3, 40])
+def test_rows_at_any_address(N):
+    """Views that begin at two bytes into a line: rows are copied, weights are left to
+    the loop over the experts."""
+    E, top, H, I = 4, 2, 128, 64
+    a, router = draw(N, H, seed=1), draw(E, H, seed=4)
+    up = draw(E, 2 * I, H, seed=5, scale=H ** -0.5)
+    down = draw(E, H, I, seed=6, scale=I ** -0.5)
+
+    def off(t):
+        wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        wide[1:].copy_(t.reshape(-1))
+        return wide[1:].view(t.shape)
+
+    assert torch.equal(ops.routed_mlp(off(a), router, up, down, top),
+                       ops.routed_mlp(a, router, up, down, top))
+    assert ops.routed_mlp_ok(off(a), up, down, top)
+    assert not ops.routed_mlp_ok(a, off(up), down, top)
+    assert not ops.routed_mlp_ok(a, up, off(down), top)
