@@ -46,7 +46,8 @@ struct PrefillArgs {
   unsigned short* out;
   float* pml;                     // splits: (n_split, B * Hkv, Tq * G, 2)
   float* pacc;                    // (n_split, B * Hkv, Tq * G, D)
-  int B, Hkv, G, Tq, p_log2, maxp, window, n_split;
+  int B, Hkv, G, Tq, P, maxp, window, n_split;
+  int p_log2;                     // of P where it is a power of two
   float scale;
   long q_sb, q_st, q_sh, o_sb, o_st, o_sh;
 };
@@ -65,7 +66,9 @@ struct PrefillTile {
 };
 
 // GENERAL: slopes, tree masks, scales that are not positive.
-template <int D, bool GENERAL>
+// DIVIDE: pages that do not hold a power of two of keys; a form of its own, since even
+// the choice costs where pages are found by shifts (0.75 us of a tree's 20).
+template <int D, bool GENERAL, bool DIVIDE>
 __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     PrefillArgs a) {
   using Tile = PrefillTile<D>;
@@ -89,6 +92,9 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int qs = a.q_start[b];
   const bool tree = GENERAL && a.tree_mask != nullptr;
   const int plog = a.p_log2, pmask = (1 << plog) - 1;
+  auto page_of = [&](int pos) { return DIVIDE ? pos / a.P : pos >> plog; };
+  auto slot_of = [&](int pos) { return DIVIDE ? pos % a.P : pos & pmask; };
+  auto first_of = [&](long page) { return DIVIDE ? page * a.P : page << plog; };
   const int* table = a.page_table + (long)b * a.maxp;
 
   // this lane's row (column of S^T)
@@ -139,23 +145,23 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   auto look_up = [&](int kb) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      kpage[i] = table[min(kb + kkey[i], kend - 1) >> plog];
-      vpage[i] = table[min(kb + vkey[i], kend - 1) >> plog];
+      kpage[i] = table[page_of(min(kb + kkey[i], kend - 1))];
+      vpage[i] = table[page_of(min(kb + vkey[i], kend - 1))];
     }
   };
   auto issue = [&](int kb, unsigned char* buf) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int pos = min(kb + kkey[i], kend - 1) & pmask;
+      const int pos = slot_of(min(kb + kkey[i], kend - 1));
       copy16_to_lds(a.k_pages +
-                        ((((long)kpage[i] * a.Hkv + g) << plog) + pos) * D + kcol[i],
+                        (first_of((long)kpage[i] * a.Hkv + g) + pos) * D + kcol[i],
                     buf + (wave + i * 4) * 1024);
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int pos = min(kb + vkey[i], (kend - 1) & ~7) & pmask;
+      const int pos = slot_of(min(kb + vkey[i], (kend - 1) & ~7));
       copy16_to_lds(a.v_pages +
-                        ((((long)vpage[i] * a.Hkv + g) * D + vrow[i]) << plog) + pos,
+                        first_of(((long)vpage[i] * a.Hkv + g) * D + vrow[i]) + pos,
                     buf + Tile::KB + (wave + i * 4) * 1024);
     }
   };

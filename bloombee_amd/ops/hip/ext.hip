@@ -389,8 +389,11 @@ torch::Tensor attn_decode_qkv(torch::Tensor qkv, long Hq, torch::Tensor k_pages,
 // Launches attention of a.Tq tokens a sequence; a's tensors and strides are set.
 static void launch_attn_prefill(PrefillArgs a, int D, int P,
                                 const torch::TensorOptions& f32) {
-  TORCH_CHECK(P > 0 && (P & (P - 1)) == 0, "page size must be a power of two");
+  // eight values of a page's row are read at once
+  TORCH_CHECK(P > 0 && P % 8 == 0, "page size must be a multiple of eight");
+  a.P = P;
   a.p_log2 = __builtin_ctz(P);
+  const bool divide = (P & (P - 1)) != 0;
   const long rows = (long)a.Tq * a.G, units = (long)a.B * a.Hkv;
   if (rows == 0 || units == 0) return;
   const long row_tiles = (rows + 127) / 128;
@@ -412,11 +415,12 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
     a.pacc = part.data_ptr<float>();
     a.pml = a.pacc + (long)a.n_split * units * rows * D;
   }
-  const bool general = a.alibi || a.tree_mask || !(a.scale > 0.f);
+  const bool general = divide || a.alibi || a.tree_mask || !(a.scale > 0.f);
   const dim3 grid(units * a.n_split, row_tiles);
-  auto launch = [&](auto d, auto gen) {
+  auto launch = [&](auto d, auto gen, auto div) {
     constexpr int DD = decltype(d)::value;
-    auto kernel = attn_prefill_kernel<DD, decltype(gen)::value>;
+    auto kernel =
+        attn_prefill_kernel<DD, decltype(gen)::value, decltype(div)::value>;
     constexpr int lds = 2 * PrefillTile<DD>::BYTES;
     if (lds > 64 * 1024)
       TORCH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -428,15 +432,16 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
       attn_prefill_fold_kernel<DD>
           <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
   };
-  auto by_dim = [&](auto gen) {
-    if (D == 128) launch(std::integral_constant<int, 128>{}, gen);
-    else if (D == 64) launch(std::integral_constant<int, 64>{}, gen);
-    else if (D == 256) launch(std::integral_constant<int, 256>{}, gen);
-    else if (D == 32) launch(std::integral_constant<int, 32>{}, gen);
+  auto by_dim = [&](auto gen, auto div) {
+    if (D == 128) launch(std::integral_constant<int, 128>{}, gen, div);
+    else if (D == 64) launch(std::integral_constant<int, 64>{}, gen, div);
+    else if (D == 256) launch(std::integral_constant<int, 256>{}, gen, div);
+    else if (D == 32) launch(std::integral_constant<int, 32>{}, gen, div);
     else TORCH_CHECK(false, "unsupported head_dim ", D);
   };
-  if (general) by_dim(std::true_type{});
-  else by_dim(std::false_type{});
+  if (divide) by_dim(std::true_type{}, std::true_type{});
+  else if (general) by_dim(std::true_type{}, std::false_type{});
+  else by_dim(std::false_type{}, std::false_type{});
 }
 
 static void set_tree_mask(PrefillArgs& a, const c10::optional<torch::Tensor>& mask,

@@ -133,6 +133,12 @@ def set_attn_sparsity(frac: float) -> None:
     _attn_sparsity = float(frac)
 
 
+def _kernel_pages(k_pages: torch.Tensor) -> bool:
+    """The kernels read values eight keys of a page at a time; pages that do not hold
+    a multiple of that go through the torch composition."""
+    return k_pages.shape[2] % 8 == 0
+
+
 def attn_decode(
     q, k_pages, v_pages, page_table, ctx_lens, scale: Optional[float] = None,
     window: int = 0, n_split: int = 0, alibi_slopes=None,
@@ -146,7 +152,7 @@ def attn_decode(
                                    alibi_slopes=alibi_slopes)
     if _on_gpu(q):
         _require_ext()
-        if q.shape[-1] > 256 and q.shape[-1] != 512:
+        if (q.shape[-1] > 256 and q.shape[-1] != 512) or not _kernel_pages(k_pages):
             # odd wide head dims: gather-based torch composition on-device
             # (D=512 runs attn_decode_wide_kernel — d split across waves)
             return ref.attn_paged(q, k_pages, v_pages, page_table,
@@ -173,7 +179,7 @@ def attn_prefill(
         scale = 1.0 / math.sqrt(q.shape[-1])
     if _on_gpu(q):
         _require_ext()
-        if q.shape[-1] > 256:
+        if q.shape[-1] > 256 or not _kernel_pages(k_pages):
             return ref.attn_paged(q, k_pages, v_pages, page_table,
                                   q_start.long(), scale,
                                   sliding_window=window if window > 0 else None,
@@ -232,7 +238,7 @@ def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
     D = k_pages.shape[3]
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    if _on_gpu(qkv):
+    if _on_gpu(qkv) and _kernel_pages(k_pages):
         if tree_mask is None or (_TREE_KERNEL and window == 0 and D <= 256):
             _require_ext()
             if T == 1 and tree_mask is None:
@@ -268,7 +274,7 @@ def attn_paged(q, k_pages, v_pages, page_table, q_start, scale=None, window: int
     if tree_mask is not None:
         if scale is None:
             scale = 1.0 / math.sqrt(q.shape[-1])
-        if (_on_gpu(q) and _TREE_KERNEL and window == 0
+        if (_on_gpu(q) and _TREE_KERNEL and window == 0 and _kernel_pages(k_pages)
                 and q.shape[-1] <= 256 and alibi_slopes is None):
             # fused tree-mask prefill kernel (spec verify) — the default
             # GPU path (tests/test_treekernel.py parity on MI355X)

@@ -117,3 +117,42 @@ def test_rows_without_a_finite_result_say_so(case, form, bad, where):
                          alibi_slopes=slopes).cpu()
     assert torch.equal(got.isnan(), want.isnan())
     close(got.nan_to_num(0), want.nan_to_num(0))
+
+
+@pytest.mark.parametrize("P", [24, 40, 4, 12])
+@pytest.mark.parametrize("form", ["plain", "window", "alibi", "tree"])
+@pytest.mark.parametrize("start", [3, 1500])
+def test_pages_of_other_sizes(P, form, start):
+    """Pages of eight times any number of keys, and others, for prompts and for one
+    token."""
+    B, Hq, Hkv, D, T = 2, 4, 2, 64, 37
+    starts = (start, 17)
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], 1600, seed=P)
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    slopes = ops.alibi_slopes_for(Hq) if form == "alibi" else None
+    tree = None
+    if form == "tree":
+        tree = torch.rand(B, T, T, generator=gen) < 0.3
+        tree |= torch.eye(T, dtype=torch.bool)
+    window = 50 if form == "window" else 0
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long(),
+                          sliding_window=window or None, alibi_slopes=slopes,
+                          tree_mask=tree)
+    got = ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)], window=window,
+                         alibi_slopes=slopes,
+                         tree_mask=None if tree is None else tree.to(DEV))
+    close(got, want)
+    if tree is None:
+        last = [t.to(DEV) for t in (q[:, :, -1:], kp, vp, table, qs + T - 1)]
+        close(ops.attn_paged(*last, window=window, alibi_slopes=slopes),
+              want[:, :, -1:])
+    # and with queries of a fused projection
+    if form != "alibi":
+        qkv = torch.zeros(B, T, (Hq + 2 * Hkv) * D, dtype=torch.bfloat16)
+        qkv[..., :Hq * D] = q.transpose(1, 2).reshape(B, T, -1)
+        got = ops.attn_paged_qkv(qkv.to(DEV), Hq, Hkv, kp.to(DEV), vp.to(DEV),
+                                 table.to(DEV), qs.to(DEV), window=window,
+                                 tree_mask=None if tree is None else tree.to(DEV))
+        close(got.view(B, T, Hq, D).transpose(1, 2), want)
