@@ -444,6 +444,14 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   else by_dim(std::false_type{}, std::false_type{});
 }
 
+// Pages go to LDS by 16-byte copies: a view that does not begin at 16 bytes is copied.
+static void set_pages(PrefillArgs& a, torch::Tensor& k, torch::Tensor& v) {
+  for (torch::Tensor* t : {&k, &v})
+    if ((size_t)t->data_ptr() % 16 != 0) *t = t->clone();
+  a.k_pages = bf_ptr(k);
+  a.v_pages = bf_ptr(v);
+}
+
 static void set_tree_mask(PrefillArgs& a, const c10::optional<torch::Tensor>& mask,
                           int B, int Tq, long window) {
   if (!mask.has_value()) return;
@@ -475,8 +483,7 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
   set_tree_mask(a, tree_mask, B, Tq, window);
   auto out = torch::empty_like(q);
   a.q = bf_ptr(q);
-  a.k_pages = bf_ptr(k_pages);
-  a.v_pages = bf_ptr(v_pages);
+  set_pages(a, k_pages, v_pages);
   a.page_table = page_table.data_ptr<int>();
   a.q_start = q_start.data_ptr<int>();
   a.out = bf_ptr_mut(out);
@@ -509,8 +516,7 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
   PrefillArgs a{};
   set_tree_mask(a, tree_mask, B, Tq, window);
   a.q = bf_ptr(qkv);
-  a.k_pages = bf_ptr(k_pages);
-  a.v_pages = bf_ptr(v_pages);
+  set_pages(a, k_pages, v_pages);
   a.page_table = page_table.data_ptr<int>();
   a.q_start = q_start.data_ptr<int>();
   a.out = bf_ptr_mut(out);

@@ -156,3 +156,22 @@ def test_pages_of_other_sizes(P, form, start):
                                  table.to(DEV), qs.to(DEV), window=window,
                                  tree_mask=None if tree is None else tree.to(DEV))
         close(got.view(B, T, Hq, D).transpose(1, 2), want)
+
+
+def test_pages_at_any_address():
+    """Pages that begin at two bytes into a line are read as they are elsewhere."""
+    B, Hq, Hkv, D, P, T, starts, room, _ = CASES[1]
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=T)
+    q = torch.randn(B, Hq, T, D, generator=torch.Generator().manual_seed(3)).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+
+    def off(t):
+        wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=DEV)
+        wide[1:].copy_(t.reshape(-1))
+        assert wide[1:].data_ptr() % 16 == 2
+        return wide[1:].view(t.shape)
+
+    q, kp, vp, table, qs = (t.to(DEV) for t in (q, kp, vp, table, qs))
+    want = ops.attn_paged(q, kp, vp, table, qs)
+    assert torch.equal(ops.attn_paged(q, off(kp), off(vp), table, qs), want)
+    assert torch.equal(ops.attn_paged(off(q), kp, vp, table, qs), want)
