@@ -44,8 +44,10 @@ def _plain(t: torch.Tensor) -> bool:
 
 
 def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
-    """The kernels take these: weights are frozen."""
+    """The kernels take these: weights are frozen. They are launched on the current
+    device's stream: tensors of another device are left to torch, which switches."""
     return (x.is_cuda and x.numel() > 0
+            and x.device.index == torch.cuda.current_device()
             and all(t.dtype == torch.bfloat16 and _plain(t)
                     for t in (x, *weights))
             and all(w.device == x.device and not w.requires_grad

@@ -279,3 +279,20 @@ def test_bindings_refuse_unaligned_rows():
     off = torch.empty(out.numel() + 1, dtype=x.dtype, device=DEV)[1:].view(out.shape)
     with pytest.raises(RuntimeError, match="aligned"):
         ext.rope_attention_grad(off, x, qk, o32, lse, 4, 1, cos, sin, 0, 1.0)
+
+
+def test_another_device_than_the_current_one(monkeypatch):
+    """The kernels go to the current device's stream: a tensor of another one takes
+    the torch operations, which switch devices themselves."""
+    forms = steps()
+    assert all(f(x.clone().requires_grad_(True)).grad_fn is not None
+               and training._fused(x) for f, _, x in forms.values())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    for fused, plain, x in forms.values():
+        assert not training._fused(x)
+        y, z = (x.clone().requires_grad_(True) for _ in range(2))
+        a, b = fused(y), plain(z)
+        g = draw(*a.shape, seed=7)
+        assert torch.equal(a, b)
+        assert torch.equal(*(torch.autograd.grad(o, t, g)[0]
+                             for o, t in ((a, y), (b, z))))
