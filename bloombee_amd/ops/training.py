@@ -5,9 +5,9 @@ gradients of frozen projections, prompts added to the first tokens.
 Each has a plain torch form, which every tensor can take, and a fused one with
 gradient kernels (module _hip_train) for bf16 tensors on the device. The fused form
 is an autograd node: it is passed by wherever something watches or replaces the torch
-operations themselves (tracing, function transforms, forward-mode, dispatch modes,
-autocast, tensor subclasses), and gradients that are differentiated again or taken in
-batches go through the plain form.
+operations themselves (tracing, function transforms, forward-mode, dispatch and
+function modes, autocast, tensor subclasses), and gradients that are differentiated
+again or taken in batches go through the plain form.
 """
 from __future__ import annotations
 
@@ -16,6 +16,7 @@ from typing import Tuple
 
 import torch
 import torch.nn.functional as F
+from torch.utils._device import DeviceContext
 
 from bloombee_amd.ops import interface
 
@@ -43,6 +44,14 @@ def _plain(t: torch.Tensor) -> bool:
             and not torch._C._functorch.is_legacy_batchedtensor(t))
 
 
+def _no_function_mode() -> bool:
+    """No mode sees torch's functions but that of a default device, which places
+    what factories make."""
+    return (torch._C._len_torch_function_stack() == 0
+            or all(type(m) is DeviceContext
+                   for m in torch.overrides._get_current_function_mode_stack()))
+
+
 def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     """The kernels take these: weights are frozen. They are launched on the current
     device's stream: tensors of another device are left to torch, which switches."""
@@ -56,6 +65,7 @@ def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
             and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling()
             and torch._C._len_torch_dispatch_stack() == 0
+            and _no_function_mode()
             and torch._C._functorch.peek_interpreter_stack() is None
             and all(torch.autograd.forward_ad.unpack_dual(t).tangent is None
                     for t in (x, *weights)))

@@ -296,3 +296,22 @@ def test_another_device_than_the_current_one(monkeypatch):
         assert torch.equal(a, b)
         assert torch.equal(*(torch.autograd.grad(o, t, g)[0]
                              for o, t in ((a, y), (b, z))))
+
+
+def test_function_modes_see_the_operations():
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    for name, (fused, plain, x) in steps().items():
+        seen = []
+        with Watch():
+            fused(x)
+        with Watch():
+            mid, seen = seen, []
+            plain(x)
+        assert set(seen) <= set(mid), name
+    # a default device replaces nothing
+    with torch.device(DEV):
+        assert training._fused(x)
