@@ -96,9 +96,13 @@ class LlamaBlock(torch.nn.Module):
 
     def _fuse_norm_gate(self, hidden) -> bool:
         """All four decode GEMMs must be decode-shaped (<= 32 rows, K%256,
-        N%64); W4/LoRA blocks keep the separate-norm path."""
+        N%64); W4/LoRA blocks keep the separate-norm path, as do blocks whose
+        weights are streamed in as they were stored (offload/weights.py): what
+        is folded into those is lost with the next binding."""
         return (getattr(self, "_w4", None) is None
                 and getattr(self, "lora_delta", None) is None
+                and (getattr(self, "_norm_folded", False)
+                     or not getattr(self, "streamed", False))
                 and ops.fuse_norm_linear_ok(hidden, self.qkv_w)
                 and self.I % 256 == 0 and (2 * self.I) % 64 == 0
                 and (self.Hq * self.D) % 256 == 0

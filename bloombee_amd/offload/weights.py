@@ -135,6 +135,8 @@ class OffloadedBlockStack:
                                        device=self.device) for _ in range(2)]
             # drop offloaded device copies
             for i in range(self.resident, n):
+                # from here on its weights are the host copies, in their form
+                stack.blocks[i].streamed = True
                 self._bind(i, 0)  # placeholder binding
             logger.info("offload: %d/%d blocks resident, %d on disk, "
                         "compress=%s", self.resident, n, ndisk,

@@ -228,3 +228,41 @@ def test_mixed_device_decode_qwen3_pattern():
     kv.close()
     got = torch.stack(got, 1)
     assert torch.equal(got, expect), (got, expect)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["llama-mini-gpu", "qwen3-0.6b"])
+def test_offloaded_decode_keeps_the_norm_weights(model):
+    """Decode steps on the device, where norm weights are folded into resident
+    projections: a block whose weights are bound anew for every step keeps both as
+    they are stored."""
+    from bloombee_amd.models.base import resolve_config
+
+    cfg = resolve_config(model)
+    stacks = [BlockStack(cfg, 0, 3, device="cuda:0", seed=3) for _ in range(2)]
+    for stack in stacks:
+        gen = torch.Generator(device="cuda:0").manual_seed(7)
+        for blk in stack.blocks:
+            for n, p in blk.named_parameters():
+                if n.endswith("norm_w"):
+                    p.data.copy_(torch.randn(p.shape, generator=gen, device="cuda:0")
+                                 .exp())
+                else:
+                    p.data.copy_(torch.randn(p.shape, generator=gen, device="cuda:0")
+                                 * p.shape[-1] ** -0.5)
+    off = OffloadedBlockStack(stacks[1], OffloadPolicy(weight_gpu_percent=0.0))
+    x = torch.randn(2, 5, cfg.hidden_size,
+                    generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    outs = []
+    for stack in (stacks[0], off):
+        kv = stack.make_kv(256).allocate(2, 16)
+        kv.extend(5)
+        outs.append([stack.forward_inference(
+            x[:, t:t + 1].contiguous(), kv,
+            torch.full((2,), t, dtype=torch.int32, device="cuda:0"))
+            for t in range(5)])
+        kv.close()
+    for t, (want, got) in enumerate(zip(*outs)):
+        # both round to bf16 at each of some ten steps of three layers, 2^-9 each
+        away = (got.float() - want.float()).norm() / want.float().norm()
+        assert away < 30 * 2.0 ** -9, (t, away)
