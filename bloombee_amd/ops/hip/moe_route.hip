@@ -80,13 +80,17 @@ __global__ __launch_bounds__(256) void norm_route_kernel(
   }
   __syncthreads();
   if (wave != 0) return;
-  // a lane an expert; larger keys win, NaN above all, of equal ones the first
+  // a lane an expert; larger keys win, NaN of either sign above all, of equal ones (both
+  // zeros are) the first
   float logit = 0.f;
   unsigned long long key = 0;   // taken, or no expert
   if (lane < E) {
     logit = bf2f(f2bf(dots[0][lane] + dots[1][lane] + dots[2][lane] + dots[3][lane]));
     const unsigned b = __float_as_uint(logit);
-    const unsigned u = (b >> 31) ? ~b : b | 0x80000000u;
+    const unsigned u = logit != logit ? 0xffffffffu
+                       : logit == 0.f ? 0x80000000u
+                       : (b >> 31)    ? ~b
+                                      : b | 0x80000000u;
     key = ((unsigned long long)u + 1) << 8 | (unsigned)(ROUTE_MAX_E - lane);
   }
   float first = 0.f, mine = 0.f, sum = 0.f;

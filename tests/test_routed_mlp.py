@@ -144,3 +144,22 @@ def test_rows_at_any_address(N):
     assert ops.routed_mlp_ok(off(a), up, down, top)
     assert not ops.routed_mlp_ok(a, off(up), down, top)
     assert not ops.routed_mlp_ok(a, up, off(down), top)
+
+
+@pytest.mark.parametrize("bits", [0x7fc0, 0xffc0 - 0x10000], ids=["nan", "-nan"])
+def test_order_of_unusual_logits(bits):
+    """NaN of either sign above all numbers, both zeros equal, infinities in place."""
+    a = torch.zeros(1, 64, dtype=torch.bfloat16, device=DEV)
+    a[0, 0] = 1.0
+    router = torch.zeros(6, 64, dtype=torch.bfloat16, device=DEV)
+    router[:, 0] = torch.tensor([1.0, float("inf"), -float("inf"), 3.0, 0.0, 2.0])
+    router.view(torch.int16)[4, 0] = bits
+    _, _, ids, wts = ops.hip_ops.norm_route(a, None, None, router, 5, 0.0)
+    assert ids[0].tolist() == [4, 1, 3, 5, 0]
+    assert bool(wts.isnan().all())
+    # products that vanish in bf16 keep their sign
+    a[0, 0] = 2.0 ** -100
+    router[:, 0] = torch.tensor([-2.0 ** -40, 2.0 ** -40, -1.0, 0.0, -1.0, -1.0])
+    _, _, ids, wts = ops.hip_ops.norm_route(a, None, None, router, 5, 0.0)
+    assert ids[0].tolist() == [0, 1, 3, 2, 4]
+    assert bool(((wts - 0.2).abs() <= 2.0 ** -10).all())
