@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
               reinterpret_cast<const short8*>(krow + hi * 8 + 32 * kk)));
       }
     };
-    auto compute_tile = [&](const bf16x8 (&vb)[NDT],
+    auto compute_tile = [&](bf16x8 (&vb)[NDT],
                             const bf16x8 (&kb)[NPT][NKK], int tb) {
       f32x4 st[NPT];
 #pragma unroll
@@ -238,6 +238,13 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
                              (16 * n + hi * 4 + reg) * 2) = f2bf(p[n][reg]);
       bf16x8 pfrag = as_bf16x8(
           *reinterpret_cast<const short8*>(p_lds + li * PROW_B + hi * 16));
+      // octets beyond the end repeat the last one: weights of zero meet them, but an
+      // infinite value takes no part twice
+      if (tb + DKVBLK > c1) {
+#pragma unroll
+        for (int n = 0; n < NDT; ++n)
+          if (tb + hi * 8 >= c1) vb[n] = as_bf16x8(short8{});
+      }
 #pragma unroll
       for (int n = 0; n < NDT; ++n)
         acc_o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[n], pfrag,

@@ -262,6 +262,16 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
         issue(kb + KT, prefill_lds + (buf ^ 1) * Tile::BYTES);
         look_up(kb + 2 * KT);
       }
+      if (kb + KT > kend) {
+        // octets beyond the end repeat the last one: weights of zero meet them, but an
+        // infinite value takes no part twice
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          if (kb + vkey[i] >= kend)
+            *reinterpret_cast<short8*>(prefill_lds + buf * Tile::BYTES + Tile::KB +
+                                       (wave + i * 4) * 1024 + lane * 16) = short8{};
+        __syncthreads();
+      }
       if (kb <= wlast && kb + KT > wfirst)
         compute(kb, prefill_lds + buf * Tile::BYTES);
       __syncthreads();

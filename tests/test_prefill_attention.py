@@ -175,3 +175,26 @@ def test_pages_at_any_address():
     want = ops.attn_paged(q, kp, vp, table, qs)
     assert torch.equal(ops.attn_paged(q, off(kp), off(vp), table, qs), want)
     assert torch.equal(ops.attn_paged(off(q), kp, vp, table, qs), want)
+
+
+@pytest.mark.parametrize("Hkv,D,room,tokens,start", [
+    (2, 128, 64, 1, 36), (2, 128, 2000, 1, 1500),      # one token: one split, several
+    (2, 64, 64, 25, 12), (2, 128, 2000, 25, 1476),     # a prompt: the same
+    (8, 128, 64, 600, 5), (1, 256, 64, 3, 40),
+])
+def test_infinite_values_of_the_last_key(Hkv, D, room, tokens, start):
+    """Places beyond the context take no part, also where an infinite value is near:
+    whoever sees it has an infinite result."""
+    room = max(room, start + tokens + 3)
+    kp, vp, table = paged(1, Hkv, D, 16, [start + tokens], room, seed=5)
+    last = start + tokens - 1
+    vp[int(table[0, last // 16]), 0, 7, last % 16] = float("inf")
+    q = torch.randn(1, 2 * Hkv, tokens, D,
+                    generator=torch.Generator().manual_seed(3)).bfloat16()
+    qs = torch.tensor([start], dtype=torch.int32)
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long())[:, :, -1]
+    assert int(want.isinf().sum()) == 2 and not bool(want.isnan().any())
+    got = ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)]).cpu()[:, :, -1]
+    assert torch.equal(got.float().isinf(), want.isinf())
+    seen = want.isfinite()
+    close(got[seen], want[seen])
