@@ -812,14 +812,71 @@ torch::Tensor gemm_w4(torch::Tensor A, torch::Tensor Wq, torch::Tensor scale,
 // skinny-M GEMM (decode projections)
 // ---------------------------------------------------------------------------
 
-// Where the one-launch kernel (gemm_stream.hip) is the faster one. Every workgroup of it
-// reads all of A, twice the bytes of its W at 32 rows: beyond 16 rows that outweighs the
-// launch it saves once W is large. us, one launch and split GEMM with its fold:
-// 4096 x 4096 1 row 8.2, 12.2; 16 rows 10.4, 13.0; 32 rows 12.6, 14.2; 14336 x 4096
-// 23.8, 28.5; 30.1, 29.8; 37.6, 31.5; [gate | up] of 4096 x 14336 with its product, which
-// is not split, at 16 rows 51.3, 49.9; at 32 58.9, 53.8.
+// Where the one-launch kernel (gemm_stream.hip) is the faster one. It takes 16 columns a
+// workgroup over all of K and sums up by itself; the split GEMM (gemm_skinny.hip) takes 64
+// and shares K out, which a second launch folds, below 16384 columns, and all of K above.
+// So the first saves a launch, but it fills the chip in rounds of 256 workgroups that cost
+// 1.7 us each beside their loads, and every workgroup reads all of A: twice the bytes of
+// its W at 32 rows. us below: one launch, split.
+
+// A product with the norm of its rows, which the other form takes in a pass of its own
+// (4 to 5 us).
 static bool stream_rows(long M, long N, long K) {
   return M <= 16 || (M <= 32 && N * K <= (32L << 20));
+}
+
+// The unsplit form of the other one leaves CUs idle in its last round.
+static bool skinny_idles(long N) {
+  const long wgs = N / 64, rounds = (wgs + 255) / 256;
+  return N > 16384 && wgs * 10 < rounds * 256 * 7;
+}
+
+// A product alone, up to 32 rows.
+static bool stream_sums(long M, long N, long K) {
+  const long rounds = (N / 16 + 255) / 256;
+  const bool full = N * 5 >= rounds * 4096 * 4;
+  // One round: few columns leave it too little to hide a long chain over K, the more so the
+  // more rows. 1024 x 3072: 1 row 5.6, 7.3; 32 rows 7.3, 8.6. 4096 x 14336: 23.8, 28.7; 16
+  // rows 27.6, 28.8. 2048 x 8192: 1 row 11.2, 12.5; 16 rows 14.4, 13.3. 512 x 14336: 16.1,
+  // 15.4; 22.5, 16.2.
+  if (rounds == 1) return K * (192 * (M + 16) - N) <= 192L << 17;
+  // Beyond 16 rows two workgroups share a CU, and each reads twice as much of A. 8192 x 1024:
+  // 17 rows 6.5, 8.6. 8192 x 4096: 32 rows 20.5, 21.9. 5120 x 4096: 18.4, 17.3.
+  if (M > 16)
+    return (K <= 2048 && (rounds == 2 || (rounds == 3 && K >= 1024))) ||
+           (rounds == 2 && K <= 4096 && N >= 6144) || (skinny_idles(N) && K >= 2048);
+  // Two and three rounds, where K outweighs their start and few CUs sit the last one out.
+  // 5120 x 512: 1 row 4.8, 4.4. 8192 x 8192: 29.3, 31.4; 16 rows 33.1, 33.1. 4608 x 4096:
+  // 13.3, 14.6; 16.1, 16.0. 4608 x 14336: 37.0, 36.1; 46.7, 37.9.
+  if (rounds <= 3) {
+    if (K <= 2048) return K >= 1024;
+    if (full) return M <= (rounds == 3 || K > 8192 ? 12 : 16);
+    return K <= 6144 && K * M <= (rounds == 2 ? 1 << 16 : 1 << 15);
+  }
+  // Many columns: vocabularies and [gate | up], where the other form is one launch, too.
+  // 151936 x 1024: 1 row 96, 56; 16 rows 116, 64. 128256 x 4096: 190, 191; 243, 195. 18176 x
+  // 4096: 33.7, 40.1; 39.2, 42.4. 57344 x 8192: 161, 186; 192, 185.
+  return (skinny_idles(N) && K >= 2048) || (K >= 8192 && M <= 8);
+}
+
+// A gated product, which the other form does in one launch, too. This one's workgroups
+// take 8192 columns a round, the other's 16384: an odd number of rounds is less than the
+// other takes. 8192 x 4096: 1 row 15.7, 24.6; 32 rows 17.5, 25.6. 22016 x 4096: 36.1, 40.5;
+// 43.2, 45.7. 57344 x 8192: 158, 175; 186, 181. Even ones: 28672 x 4096 47.6, 48.6; 16 rows
+// 49.8, 47.4; 32 rows 56.5, 51.0. Short chains do not pay their start: 28672 x 512 10.0, 8.6.
+static bool stream_swiglu(long M, long N, long K) {
+  const long rounds = (N / 32 + 255) / 256;
+  return N <= 8192 || (K >= 1024 && (rounds % 2 == 1 || M <= 4));
+}
+
+// Queries, keys and values with their turns, 8192 columns a round: short chains, or one
+// round that is more than half full, or nearly two. 4096 x 1024: 1 row 5.3, 7.5; 32 rows
+// 7.4, 8.5. 6144 x 4096: 13.5, 15.4; 18.7, 18.1, where a step of 32 rows is 3 us a layer
+// faster with one launch less all the same. 10240 x 8192: 44.0, 41.7; 55.1, 46.4. 2048 x
+// 4096: 11.6, 8.9.
+static bool stream_rope(long M, long N, long K) {
+  if (M > 16) return K <= 1024 || (N >= 5120 && N <= 8192 && (K <= 4096 || N > 6144));
+  return K <= 2048 || (N <= 8192 && N >= (K <= 3072 ? 3072 : 5120)) || N >= 14336;
 }
 
 // A's rows go to LDS by 16-byte copies: a view that does not begin at 16 bytes is copied
@@ -909,7 +966,7 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   a.C = bf_ptr_mut(C);
   a.eps = eps;
   if (a.M == 0) return C;
-  if (!stream_rows(a.M, a.N, a.K)) {
+  if (!stream_swiglu(a.M, a.N, a.K)) {
     launch_skinny_fused<true>(a, a.K, 1, nullptr, nullptr);
     return C;
   }
@@ -971,7 +1028,7 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq
   a.start = start_pos.data_ptr<int>();
   a.k_pages = bf_ptr_mut(k_pages);
   a.v_pages = bf_ptr_mut(v_pages);
-  if (stream_rows(a.M, a.N, a.K)) {
+  if (stream_rope(a.M, a.N, a.K)) {
     by_rows(a.M, [&](auto mt, auto xn) {
       constexpr int MT = decltype(mt)::value;
       gemm_stream_kernel<EPI_ROPE, 2, MT, decltype(xn)::value, true, 4, 4 - MT>
@@ -1223,6 +1280,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);
   m.def("stream_rows", &stream_rows);
+  m.def("stream_sums", &stream_sums);
+  m.def("stream_swiglu", &stream_swiglu);
+  m.def("stream_rope", &stream_rope);
   m.def("attn_prefill", &attn_prefill);
   m.def("gemm_skinny", &gemm_skinny, py::arg("A"), py::arg("W"),
         py::arg("residual") = c10::nullopt, py::arg("bias") = c10::nullopt,

@@ -323,8 +323,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
             and K % 256 == 0 and N % 64 == 0):
         _require_ext()
         if (ss_in is None and ss_out is None
-                and (norm is None or norm[0] is None)
-                and hip_ops.stream_rows(M, N, K)):
+                and (hip_ops.stream_sums(M, N, K) if norm is None else
+                     norm[0] is None and hip_ops.stream_rows(M, N, K))):
             return hip_ops.gemm_stream(x.contiguous(), w, residual, bias,
                                        -1.0 if norm is None else float(norm[1]))
         if norm is not None or ss_out is not None:

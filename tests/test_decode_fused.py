@@ -225,3 +225,54 @@ def test_no_rows():
     for rows in (x, x.view(0, 1, 512), x.view(1, 0, 512)):
         assert ops.linear(rows, w).shape == (*rows.shape[:-1], 64)
         assert ops.linear_swiglu(rows, w, 1e-5).shape == (*rows.shape[:-1], 32)
+
+
+@pytest.mark.parametrize("N,K", [(512, 14336), (4096, 512), (4096, 14336), (4160, 512),
+                                 (4160, 1024), (4608, 4096), (8192, 4096), (8256, 3072),
+                                 (12288, 1024), (16384, 1024), (18176, 2048),
+                                 (32000, 1024)])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+def test_products_on_both_sides_of_their_rules(M, N, K):
+    """Rounds of workgroups full and nearly empty: whatever kernel takes a product, its
+    result is one rounding of a 32-bit sum."""
+    x, w, r = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5), draw(M, N, seed=3)
+    z = x.double() @ w.double().T
+    close(ops.linear(x, w), z)
+    close(ops.linear(x, w, residual=r), z + r.double())
+    n = rms(x, 1e-5) @ w.double().T
+    want = torch.nn.functional.silu(n[:, :N // 2]) * n[:, N // 2:]
+    close(ops.linear_swiglu(x, w, 1e-5), want)
+    if N % 192 == 0 or N == 8192:            # heads of 64, as many of each kind
+        H = N // 64
+        Hkv = 1 if N == 8192 else H // 3
+        Hq = H - 2 * Hkv
+        kp, vp = (torch.zeros(4, Hkv, *s, dtype=torch.bfloat16, device=DEV)
+                  for s in ((16, 64), (64, 16)))
+        table = torch.arange(4, device=DEV, dtype=torch.int32).view(1, 4)
+        start = torch.tensor([9], dtype=torch.int32, device=DEV)
+        cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(64, 128))
+        n = n.view(1, M, -1).float().cpu()
+        kw, vw = kp.float().cpu(), vp.float().cpu()
+        ops.rope_kv_write_(n, Hq, Hkv, cos.cpu(), sin.cpu(), None, kw, vw, table.cpu(),
+                           start.cpu())
+        got = ops.linear_rope_kv(x[None], w, 1e-5, Hq, Hkv, cos, sin, None, kp, vp, table,
+                                 start)
+        close(got[..., :Hq * 64].cpu(), n[..., :Hq * 64].double())
+        close(kp.cpu(), kw.double())
+        close(vp.cpu(), vw.double())
+
+
+def test_rules_of_decode_products():
+    """Both sides of each rule are reached by the sizes above."""
+    sums, glu, rope = (getattr(ops.hip_ops, "stream_" + n)
+                       for n in ("sums", "swiglu", "rope"))
+    assert sums(1, 4096, 14336) and not sums(32, 4096, 14336)
+    assert not sums(1, 4160, 512) and sums(1, 4160, 1024)
+    assert sums(16, 4608, 4096) and not sums(1, 4608, 6400)
+    assert sums(8, 9216, 4096) and not sums(9, 9216, 4096)
+    assert sums(16, 18176, 2048) and not sums(1, 32000, 1024)
+    assert sums(32, 8192, 4096) and not sums(32, 8256, 3072)
+    assert glu(32, 8192, 4096) and glu(4, 16384, 1024) and not glu(5, 16384, 1024)
+    assert glu(32, 18176, 2048) and not glu(16, 32000, 1024) and not glu(1, 18176, 512)
+    assert rope(17, 12288, 1024) and not rope(16, 4608, 4096)
+    assert rope(17, 8192, 4096) and not rope(17, 18176, 2048)
