@@ -291,7 +291,10 @@ static torch::Tensor attn_decode_core(
     alibi_ptr = alibi->data_ptr<float>();
   }
   int n_split = (int)n_split_req;
-  int share = n_split > 0 ? 1 : 128;   // least tokens of a split
+  // Least tokens of a split: the four waves of a workgroup take 32 tokens each, and
+  // shorter splits idle most of them. They share 32 where D = 512 (8 sequences of 300, 16
+  // heads on 8: 31.6 us with splits of 128, 18.7 so).
+  int share = n_split > 0 ? 1 : D == 512 ? 32 : 128;
   if (n_split <= 0) {
     // measured optimum (benchmarks/bench_kernels.py attn_decode): size the
     // grid for full residency — NT=1 runs 118 VGPRs -> 4 WGs/CU (1024 WGs),
@@ -317,8 +320,6 @@ static torch::Tensor attn_decode_core(
       share = 1024;
       n_split = (int)std::min(32L, (room + share - 1) / share);
     } else {
-      // a wave takes 32 tokens at a time, a workgroup 128: shorter splits idle
-      // most of its waves
       n_split = (int)std::max(1L, std::min({32L, target / units, room / share}));
     }
   }

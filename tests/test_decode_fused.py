@@ -276,3 +276,29 @@ def test_rules_of_decode_products():
     assert glu(32, 18176, 2048) and not glu(16, 32000, 1024) and not glu(1, 18176, 512)
     assert rope(17, 12288, 1024) and not rope(16, 4608, 4096)
     assert rope(17, 8192, 4096) and not rope(17, 18176, 2048)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,room,window", [
+    (1, 4, 2, 128, 4096, 300),                # splits ahead of the window
+    (2, 8, 4, 256, 4096, 1024),
+    (1, 8, 2, 64, 4096, 1),
+    (1, 8, 4, 512, 300, 0),                   # splits of 32 tokens
+    (2, 4, 1, 512, 4096, 700),
+    (3, 16, 1, 512, 96, 0),
+])
+def test_decode_attention_without_some_splits(B, Hq, Hkv, D, room, window):
+    """Splits ahead of a window or beyond a short context in a wide table hold nothing."""
+    lengths = [room, 33, 1][:B]
+    maxp = -(-room // 16)
+    kp, vp = draw(B * maxp, Hkv, 16, D, seed=1), draw(B * maxp, Hkv, D, 16, seed=2)
+    gen = torch.Generator().manual_seed(B)
+    table = torch.randperm(B * maxp, generator=gen).view(B, maxp).int().to(DEV)
+    q = draw(B, Hq, 1, D, seed=3)
+    start = torch.tensor([n - 1 for n in lengths], device=DEV)
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, start,
+                          sliding_window=window or None)
+    got = ops.attn_paged(q, kp, vp, table, start, window=window)
+    # weights enter the value product in bf16, 2^-9 of the largest value; so does the
+    # result
+    err = (got.float() - want).abs().max()
+    assert err <= 2 * 4.5 * 2.0 ** -9, err
