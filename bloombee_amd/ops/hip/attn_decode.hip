@@ -86,18 +86,20 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
   const float* pa = part_acc + ((long)bh * n_split * maxg + g) * D + col;
   for (int s0 = 0; s0 < n_split; s0 += WAVE) {
     const int s = s0 + lane;
-    float w = 0.f;
-    if (s < n_split) {
-      const float ls = ml[(long)s * maxg * 2 + 1];
-      // splits beyond the context have no sum; their values are zero
-      if (ls != 0.f) {
-        w = fast_exp2(ml[(long)s * maxg * 2] - m);
-        l += w * ls;
-      }
+    float w = 0.f, ls = 0.f;
+    if (s < n_split) ls = ml[(long)s * maxg * 2 + 1];
+    if (ls != 0.f) {
+      w = fast_exp2(ml[(long)s * maxg * 2] - m);
+      l += w * ls;
     }
-    const int n = min(WAVE, n_split - s0);
+    // splits beyond the context, or ahead of the window, have no sum: values are read
+    // from the first to the last that has one (a window of 1024 in 4096 tokens, 8 of 32
+    // splits of 256: 7.9 -> 4.9 us)
+    const unsigned long long live = __builtin_amdgcn_ballot_w64(ls != 0.f);
+    if (live == 0) continue;
+    const int end = WAVE - __builtin_clzll(live);
 #pragma unroll 8
-    for (int i = 0; i < n; ++i) {
+    for (int i = __builtin_ctzll(live); i < end; ++i) {
       const float wi = __shfl(w, i);
 #pragma unroll
       for (int j = 0; j < E; ++j)
