@@ -250,7 +250,17 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
         acc_o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[n], pfrag,
                                                            acc_o[n], 0, 0, 0);
     };
-    if (tbs < c1) {
+    if (tbs + TSTRIDE >= c1) {
+      // one tile of a short split: nothing to run ahead for (8 sequences of 1024, 64 heads
+      // on 8: 14.6 us with the loads of a second one, 14.0 without)
+      if (tbs < c1) {
+        Pages pa;
+        look_up(pa, tbs);
+        load_tile(vb0, kb0, tbs, pa);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_tile(vb0, kb0, tbs);
+      }
+    } else {
       Pages pa, pb;
       look_up(pa, tbs);
       look_up(pb, tbs + TSTRIDE);
