@@ -25,7 +25,7 @@
 // Measured, 32 heads on 8 of 128: four prompts of 4096 672 us (820 TF/s of the
 // visible half; 3808 us with 16-row tiles of one head each, staged through
 // registers, weights through LDS), one of 333 behind 1201 37 us (163), a tree of 25
-// behind 1500 20 us (168).
+// behind 1500 18.5 us (168).
 //
 // Numerics: fp32 softmax/accum; bf16 operands — matches reference tolerance
 // class (test_block_exact_match.py atol 1e-4 forward on fp32 inputs).
@@ -65,15 +65,24 @@ struct PrefillTile {
   }
 };
 
-// GENERAL: slopes, tree masks, scales that are not positive.
-// DIVIDE: pages that do not hold a power of two of keys; a form of its own, since even
-// the choice costs where pages are found by shifts (0.75 us of a tree's 20).
-template <int D, bool GENERAL, bool DIVIDE>
+// Where values beyond the last key come from: weights of zero meet them, which a value
+// that is not finite would turn into NaN.
+__device__ const unsigned short prefill_zeros[8] __attribute__((aligned(16))) = {};
+
+// GENERAL: slopes, scales that are not positive; TREE: these and tree masks, whose code
+// in between took slopes as long as it did trees (two tokens, 16 heads of 64: 7.4 us, 5.6
+// apart).
+// DIVIDE: TREE, and pages that do not hold a power of two of keys; a form of its own, since
+// even the choice costs where pages are found by shifts (0.75 us of a tree's 20).
+enum PrefillForm { PREFILL_PLAIN, PREFILL_GENERAL, PREFILL_TREE, PREFILL_DIVIDE };
+
+template <int D, int FORM>
 __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     PrefillArgs a) {
   using Tile = PrefillTile<D>;
   constexpr int KT = Tile::KT, RC = Tile::RC, NI = Tile::NI;
   constexpr int NKK = D / 16, ND = D / 32;
+  constexpr bool GENERAL = FORM != PREFILL_PLAIN, DIVIDE = FORM == PREFILL_DIVIDE;
   static_assert(NI >= 1, "tile smaller than the workgroup");
   extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
 
@@ -90,7 +99,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int lane = tid & (WAVE - 1);
   const int li = lane & 31, hi = lane >> 5;
   const int qs = a.q_start[b];
-  const bool tree = GENERAL && a.tree_mask != nullptr;
+  const bool tree = FORM >= PREFILL_TREE && a.tree_mask != nullptr;
   const int plog = a.p_log2, pmask = (1 << plog) - 1;
   auto page_of = [&](int pos) { return DIVIDE ? pos / a.P : pos >> plog; };
   auto slot_of = [&](int pos) { return DIVIDE ? pos % a.P : pos & pmask; };
@@ -159,10 +168,11 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int pos = slot_of(min(kb + vkey[i], (kend - 1) & ~7));
-      copy16_to_lds(a.v_pages +
-                        first_of(((long)vpage[i] * a.Hkv + g) * D + vrow[i]) + pos,
-                    buf + Tile::KB + (wave + i * 4) * 1024);
+      const unsigned short* src =
+          a.v_pages + first_of(((long)vpage[i] * a.Hkv + g) * D + vrow[i]) +
+          slot_of(kb + vkey[i]);
+      if (kb + vkey[i] >= kend) src = prefill_zeros;
+      copy16_to_lds(src, buf + Tile::KB + (wave + i * 4) * 1024);
     }
   };
 
@@ -174,6 +184,25 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int krow = li * (D * 2);
 
   auto compute = [&](int kb, const unsigned char* kt) {
+    // keys a tree's row does not see, element n * 16 + j of s below; ahead of the scores,
+    // whose registers the entries take meanwhile, and eight at a time, so that their loads
+    // overlap (25 tokens behind 1500: 19.8 us one by one, 18.5)
+    unsigned dead = 0;
+    if (tree && kb + KT - 1 > ihi) {
+      const int k0 = kb + hi * 8 - qs;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        unsigned char seen[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          seen[e] = mask[min(max(k0 + q * 16 + e, 0), a.Tq - 1)];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int k = k0 + q * 16 + e;
+          if (k >= a.Tq || (k >= 0 && !seen[e])) dead |= 1u << (q * 8 + e);
+        }
+      }
+    }
     f32x16 s[2];
     s[0] = s[1] = f32x16{};
 #pragma unroll
@@ -194,22 +223,22 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
                     slope2 * (float)(kb + n * 32 + (j & 8) * 2 + hi * 8 + (j & 7));
     }
     if (kb < ilo || kb + KT - 1 > ihi) {
-      const int d0 = qpos - kb - hi * 8;
+      if (tree) {
 #pragma unroll
-      for (int n = 0; n < 2; ++n)
+        for (int n = 0; n < 2; ++n)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int off = n * 32 + (j & 8) * 2 + (j & 7);
-          bool dead;
-          if (tree) {
-            const int k = kb + hi * 8 + off - qs;
-            dead = k >= a.Tq || (k >= 0 && !mask[k]);
-          } else {
-            const int dist = d0 - off;
-            dead = dist < 0 || dist >= sees;
+          for (int j = 0; j < 16; ++j)
+            if (dead >> (n * 16 + j) & 1) s[n][j] = NEG_BIG;
+      } else {
+        const int d0 = qpos - kb - hi * 8;
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            const int dist = d0 - (n * 32 + (j & 8) * 2 + (j & 7));
+            if (dist < 0 || dist >= sees) s[n][j] = NEG_BIG;
           }
-          if (dead) s[n][j] = NEG_BIG;
-        }
+      }
     }
     float mx = m;
 #pragma unroll
@@ -261,16 +290,6 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
       if (kb + KT < t1) {
         issue(kb + KT, prefill_lds + (buf ^ 1) * Tile::BYTES);
         look_up(kb + 2 * KT);
-      }
-      if (kb + KT > kend) {
-        // octets beyond the end repeat the last one: weights of zero meet them, but an
-        // infinite value takes no part twice
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-          if (kb + vkey[i] >= kend)
-            *reinterpret_cast<short8*>(prefill_lds + buf * Tile::BYTES + Tile::KB +
-                                       (wave + i * 4) * 1024 + lane * 16) = short8{};
-        __syncthreads();
       }
       if (kb <= wlast && kb + KT > wfirst)
         compute(kb, prefill_lds + buf * Tile::BYTES);

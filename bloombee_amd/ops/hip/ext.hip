@@ -394,7 +394,6 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   TORCH_CHECK(P > 0 && P % 8 == 0, "page size must be a multiple of eight");
   a.P = P;
   a.p_log2 = __builtin_ctz(P);
-  const bool divide = (P & (P - 1)) != 0;
   const long rows = (long)a.Tq * a.G, units = (long)a.B * a.Hkv;
   if (rows == 0 || units == 0) return;
   const long row_tiles = (rows + 127) / 128;
@@ -416,12 +415,10 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
     a.pacc = part.data_ptr<float>();
     a.pml = a.pacc + (long)a.n_split * units * rows * D;
   }
-  const bool general = divide || a.alibi || a.tree_mask || !(a.scale > 0.f);
   const dim3 grid(units * a.n_split, row_tiles);
-  auto launch = [&](auto d, auto gen, auto div) {
+  auto launch = [&](auto d, auto form) {
     constexpr int DD = decltype(d)::value;
-    auto kernel =
-        attn_prefill_kernel<DD, decltype(gen)::value, decltype(div)::value>;
+    auto kernel = attn_prefill_kernel<DD, decltype(form)::value>;
     constexpr int lds = 2 * PrefillTile<DD>::BYTES;
     if (lds > 64 * 1024)
       TORCH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -433,16 +430,18 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
       attn_prefill_fold_kernel<DD>
           <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
   };
-  auto by_dim = [&](auto gen, auto div) {
-    if (D == 128) launch(std::integral_constant<int, 128>{}, gen, div);
-    else if (D == 64) launch(std::integral_constant<int, 64>{}, gen, div);
-    else if (D == 256) launch(std::integral_constant<int, 256>{}, gen, div);
-    else if (D == 32) launch(std::integral_constant<int, 32>{}, gen, div);
+  auto by_dim = [&](auto form) {
+    if (D == 128) launch(std::integral_constant<int, 128>{}, form);
+    else if (D == 64) launch(std::integral_constant<int, 64>{}, form);
+    else if (D == 256) launch(std::integral_constant<int, 256>{}, form);
+    else if (D == 32) launch(std::integral_constant<int, 32>{}, form);
     else TORCH_CHECK(false, "unsupported head_dim ", D);
   };
-  if (divide) by_dim(std::true_type{}, std::true_type{});
-  else if (general) by_dim(std::true_type{}, std::false_type{});
-  else by_dim(std::false_type{}, std::false_type{});
+  if (P & (P - 1)) by_dim(std::integral_constant<int, PREFILL_DIVIDE>{});
+  else if (a.tree_mask) by_dim(std::integral_constant<int, PREFILL_TREE>{});
+  else if (a.alibi || !(a.scale > 0.f))
+    by_dim(std::integral_constant<int, PREFILL_GENERAL>{});
+  else by_dim(std::integral_constant<int, PREFILL_PLAIN>{});
 }
 
 // Pages go to LDS by 16-byte copies: a view that does not begin at 16 bytes is copied.
