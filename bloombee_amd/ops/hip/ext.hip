@@ -588,11 +588,15 @@ void rope_kv_write_(torch::Tensor qkv, long Hq_, long Hkv_, torch::Tensor cos_t,
     return;
   }
   dim3 grid(B * T, Hq + 2 * Hkv);
-  rope_kv_write_kernel<<<grid, 64, 0, cur_stream()>>>(
-      bf_ptr_mut(qkv), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), pos_ptr,
-      bf_ptr_mut(k_pages), bf_ptr_mut(v_pages), page_table.data_ptr<int>(),
-      start_pos.data_ptr<int>(), B, Hq, Hkv, T, D, P, maxp,
-      (int)cos_t.size(0), norms[0], norms[1], (float)eps);
+  auto launch = [&](auto norm) {
+    rope_kv_write_kernel<decltype(norm)::value><<<grid, 64, 0, cur_stream()>>>(
+        bf_ptr_mut(qkv), cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), pos_ptr,
+        bf_ptr_mut(k_pages), bf_ptr_mut(v_pages), page_table.data_ptr<int>(),
+        start_pos.data_ptr<int>(), B, Hq, Hkv, T, D, P, maxp, (int)cos_t.size(0),
+        norms[0], norms[1], (float)eps);
+  };
+  if (norms[0] || norms[1]) launch(std::true_type{});
+  else launch(std::false_type{});
 }
 
 
