@@ -31,30 +31,6 @@ DEVINL void load_bf16_e(const unsigned short* p, float* out) {
   }
 }
 
-template <int E>
-DEVINL void store_bf16_e(unsigned short* p, const float* in) {
-  if constexpr (E == 2) {
-    short2_v v;
-    v[0] = (short)f2bf(in[0]);
-    v[1] = (short)f2bf(in[1]);
-    *reinterpret_cast<short2_v*>(p) = v;
-  } else if constexpr (E == 4) {
-    short4_v v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(in[j]);
-    *reinterpret_cast<short4_v*>(p) = v;
-  } else {
-#pragma unroll
-    for (int c = 0; c < E / 8; ++c) {
-      short8 v;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = (short)f2bf(in[c * 8 + j]);
-      *reinterpret_cast<short8*>(p + c * 8) = v;
-    }
-  }
-}
-
-
 // Combine n_split partials: a wave a row (unit, head of the chunk), grid
 // ceil(units * maxg / 4). Lanes read the splits' maxima and sums at once and share
 // out the weights, so that the loads of the values do not wait for one another
