@@ -15,9 +15,11 @@ a flat MI355X-native block:
 Two forward paths (by design, mirroring the reference's split between
 iterate_rpc_inference and run_rpc_forward/backward):
   forward_inference — HIP kernels + paged KV, no autograd.
-  forward_train     — differentiable eager composition (fp32 softmax) used by
-                      the fine-tuning RPCs; gradients flow to inputs/prompts
-                      only (server weights frozen, ref backend.py:106-109).
+  forward_train     — differentiable steps of ops/training.py (fp32 softmax):
+                      kernels with their gradients for bf16 on the device, torch
+                      operations elsewhere. Used by the fine-tuning RPCs;
+                      gradients flow to inputs/prompts only (server weights
+                      frozen, ref backend.py:106-109).
 """
 from __future__ import annotations
 
@@ -123,8 +125,8 @@ class LlamaBlock(torch.nn.Module):
         one bf16 round), norm weights <- 1. rms_norm with unit weight is
         mathematically unchanged on EVERY path (train, prefill, CPU), and
         the decode GEMM then only applies the per-row 1/rms in its
-        epilogue (norm_mode 2) instead of per-element weight scaling
-        (profiles/r02 §13: the per-stage scale cost +4-8 us/GEMM)."""
+        epilogue, from the squares of the rows that it has at hand, instead
+        of per-element weight scaling, which cost 4 to 8 us a GEMM."""
         if getattr(self, "_norm_folded", False):
             return
         self._norm_fold_orig = (self.input_norm_w.detach().clone(),

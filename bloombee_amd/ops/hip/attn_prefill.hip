@@ -22,7 +22,7 @@
 // overlap); the chain of tiles bounds short ones, so there the keys are split over
 // workgroups and a second kernel folds the parts.
 //
-// Measured, 32 heads on 8 of 128: four prompts of 4096 672 us (820 TF/s of the
+// Measured, 32 heads on 8 of 128: four prompts of 4096 672 us alone (820 TF/s of the
 // visible half; 3808 us with 16-row tiles of one head each, staged through
 // registers, weights through LDS), one of 333 behind 1201 37 us (163), a tree of 25
 // behind 1500 18.5 us (168).

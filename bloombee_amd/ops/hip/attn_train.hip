@@ -21,7 +21,11 @@
 //
 // Weights and their gradients are 32-bit. They enter the second products as a sum of
 // two bf16 (the value and what its rounding lost); queries, keys, values and dO are
-// bf16 already. So a product loses no more than 2^-17 of a term.
+// bf16 already. So a product loses no more than 2^-17 of a term. Errors against 64 bits
+// over 12 sizes of 33 to 1999 tokens, inputs of scale 1 and 3, beside those of weights
+// kept in 32 bits (torch operations): results 0.0021 to 0.0077, the same; gradients of
+// queries 0.0027 to 0.0140 (0.0031 to 0.0141), keys 0.0028 to 0.0141 (0.0035 to 0.0143),
+// values 0.0022 to 0.0077 (0.0028 to 0.0079): a group's heads are summed in 32 bits here.
 //
 // The matrix cores bound all three: 3, 4 and 6 products of 32 x 32 x D a tile. Two
 // sequences of 1999, 32 heads on 8 of 128: 136, 166 and 401 us (721, 788 and 490

@@ -302,21 +302,20 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
            ss_in: Optional[torch.Tensor] = None,
            ss_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = (rmsnorm(x) if norm else x) @ w^T (+bias) (+residual).
-    Decode-shaped GEMMs (<=32 rows) on GPU go through the skinny-M MFMA
-    kernel (gemm_skinny.hip) — hipBLASLt leaves ~2x weight-stream bandwidth
-    on the table at M<=32; everything else uses hipBLASLt via F.linear.
-    norm=(weight, eps) folds the input rmsnorm into the kernel's A-operand
-    stage (launch-count reduction; the separate rms_norm launch + its
-    read/write disappear from the decode step). ss_in is the producing
-    GEMM's per-stripe row sum-of-squares (its ss_out) so the fused norm
-    skips re-streaming A; ss_out asks this GEMM's epilogue to emit the
-    same stats for ITS consumer (f32 (N/64, 32), overwritten — graph-safe)."""
+    Decode-shaped GEMMs (<=32 rows) on GPU go through the weight-streaming MFMA
+    kernels (gemm_stream.hip, gemm_skinny.hip) — hipBLASLt leaves ~2x weight-stream
+    bandwidth on the table at M<=32; everything else uses hipBLASLt via F.linear.
+    norm=(weight, eps): the input's rmsnorm is taken along; weight None: it is folded
+    into w. ss_in (f32, (stripes, 32)) are sums of squares of x's rows, the ss_out of
+    the product that made x, and spare a pass over x; ss_out (f32, (N/64, 32)) takes
+    those of the result. Blocks use neither: the products that take a norm along sum
+    up the squares themselves."""
     M = x.numel() // x.shape[-1]
     N, K = w.shape[0], x.shape[-1]
-    # All decode-shaped GEMMs route to the skinny kernel: although hipBLASLt
+    # All decode-shaped GEMMs route to these kernels: although hipBLASLt
     # wins the two MLP shapes in an isolated microbench, in the real decode
     # step it runs ~1.5x slower (cold L2 / per-stream heuristics, see
-    # profiles/), while gemm_skinny runs faster in-context AND fuses the
+    # profiles/), while these run faster in-context AND fuse the
     # residual/bias epilogue the blaslt path would re-emit as a separate
     # eager kernel.
     if (_on_gpu(x) and M <= 32 and x.dtype == torch.bfloat16
@@ -436,8 +435,11 @@ def routed_mlp(a: torch.Tensor, router_w: torch.Tensor, gate_up: torch.Tensor,
         a.reshape(-1, H).contiguous(),
         None if residual is None else residual.reshape(-1, H).contiguous(), w,
         router_w, top, eps)
-    # every step's results are bf16, as in a loop over the experts: the choices
-    # of later layers hang on near ties, and are to be the loop's
+    # gate and up are bf16 results, as where the experts' products are steps of their
+    # own: the choices of later layers hang on near ties, and fewer roundings move as
+    # many of them as other ones. An expert's weighted row is rounded once (a loop
+    # over the experts rounds it before the weight, too), and rows are summed in the
+    # order of the choices
     rows = ragged.moe_experts(y, gate_up.view(E, 2, I, H), down,
                               ragged.Routing(ids, wts, None), stepwise=True)
     return hip_ops.add_experts(None if residual is None else h, rows).view(a.shape)
