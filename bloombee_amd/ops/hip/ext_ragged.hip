@@ -802,6 +802,31 @@ void attn_ragged(Tensor q, Tensor kp, OptTensor vp, Tensor table,
 // routed experts
 // ---------------------------------------------------------------------------
 
+// Rows of a tile for experts of a rows on average: what takes the fewest padded rows,
+// with what a tile costs beside them, at counts that spread by sqrt(a). Two products of
+// eight experts, 4096 x 14336, us with tiles of 64 to 256 rows (the least bounds are
+// 540 of weights, 1.9 a row of an expert of operations at 1.5 PF):
+//   20 rows 484 with 64;  64: 630, 520 with 96, 525 with 128, 547 with 160
+//   96: 619, 651, 555, 573, 591 with 192;  125: 603 with 160, 620, 679 with 256
+//   225: 750 with 128, 889 with 160, 981, 750;  350: 1154 with 128, 1033 with 192, 1192
+//   425: 1286 with 128, 1320, 1516, 1196 with 256;  1000: 2824, 2825, 2799, 2671
+// Several tiles of 96 or 160 are slower than this makes them (300 rows: 1156, 1076,
+// two of 192 rows 1014).
+static int moe_rows(float a) {
+  const float s = sqrtf(a);
+  int best = 64;
+  float least = INFINITY;
+  for (int bm : {64, 96, 128, 160, 192, 256}) {
+    const float tiles = (ceilf((a - s) / bm) + ceilf(a / bm) + ceilf((a + s) / bm)) / 3;
+    if (tiles > 1 && (bm == 96 || bm == 160)) continue;
+    if (tiles * (bm + 48) < least) {
+      least = tiles * (bm + 48);
+      best = bm;
+    }
+  }
+  return best;
+}
+
 // h (N, K), up (E, planes, F, K), down (E, Wp, F), ids/wts (N, top)
 // -> y (N, top, Wp); rows of skipped choices are not written. Two planes:
 // gated activation (limit, slope, shift), one: relu(up)^2. win: the weight
@@ -827,6 +852,15 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
               E <= MOE_MAX_E && top >= 1);
   TORCH_CHECK(K % 64 == 0 && F % 64 == 0 && Wp % 64 == 0,
               "expert sizes must be padded to 64");
+  if (ta == at::kBFloat16 && (long)N * K >= 1L << 31) {
+    // a row's place in bytes has 32 bits
+    const int n = N / 2;
+    return torch::cat(
+        {moe_experts(h.slice(0, 0, n), up, down, ids.slice(0, 0, n),
+                     wts.slice(0, 0, n), win, limit, slope, shift, stepwise),
+         moe_experts(h.slice(0, n), up, down, ids.slice(0, n), wts.slice(0, n), win,
+                     limit, slope, shift, stepwise)});
+  }
   auto y = torch::empty({N, top, Wp}, h.options());
   if (N == 0) return y;
   auto act = torch::empty({S, F}, h.options());
@@ -862,7 +896,7 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     return y;
   }
 
-  const int BM = ta == at::kBFloat16 && S / E >= 96 ? 128 : 64;
+  const int BM = ta == at::kBFloat16 ? moe_rows(S / (float)E) : 64;
   const int max_tiles = S / BM + std::min(S, E);  // the count goes behind
   auto iopt = ids.options();
   auto off = torch::empty({E + 1}, iopt);
@@ -887,25 +921,40 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     check_launch();
     return y;
   }
-  auto tile = [&](auto bm) {
-    constexpr int B = decltype(bm)::value;
-    const int per = up.size(1) == 2 ? 128 : 256;
-    const int nu = (F + per - 1) / per, nd = (Wp + 255) / 256;
+  auto rows = [&](auto up_tile, auto down_tile) {
+    typedef decltype(up_tile) U;
+    typedef decltype(down_tile) D;
+    const int per = up.size(1) == 2 ? U::BN / 2 : U::BN;
+    const int nu = (F + per - 1) / per, nd = (Wp + D::BN - 1) / D::BN;
     by_planes([&](auto np) {
-      moe_tile_kernel<B, decltype(np)::value><<<nu * max_tiles, 256, 0, st>>>(
+      auto k = moe_rows_kernel<U, decltype(np)::value>;
+      allow_lds(k, U::LDS);
+      k<<<nu * max_tiles, U::THREADS, U::LDS, st>>>(
           (const bf16_bits*)h.data_ptr(), (const bf16_bits*)up.data_ptr(), offp,
           sp, tp, w1, (bf16_bits*)act.data_ptr(), max_tiles, nu, top, F, K, K,
           F, glu);
     });
     check_launch();
-    moe_tile_kernel<B, 0><<<nd * max_tiles, 256, 0, st>>>(
+    auto k = moe_rows_kernel<D, 0>;
+    allow_lds(k, D::LDS);
+    k<<<nd * max_tiles, D::THREADS, D::LDS, st>>>(
         (const bf16_bits*)act.data_ptr(), (const bf16_bits*)down.data_ptr(),
         offp, sp, tp, w2, (bf16_bits*)y.data_ptr(), max_tiles, nd, top, Wp, F,
         F, Wp, glu);
     check_launch();
   };
-  if (BM == 128) tile(std::integral_constant<int, 128>{});
-  else tile(std::integral_constant<int, 64>{});
+  // an expert's rows in one tile: its weights are streamed, more of them ahead;
+  // in several: wide tiles
+  const bool one = S / (float)E + sqrtf(S / (float)E) <= BM;
+  if (BM == 64) rows(RowsTile<64, 128, 2, 2, 1, 3, 2>{}, RowsTile<64, 128, 2, 2, 1, 3, 2>{});
+  else if (BM == 96) rows(RowsTile<96, 128, 2, 2, 1, 4, 1>{}, RowsTile<96, 128, 2, 2, 1, 4, 1>{});
+  else if (BM == 128 && one) rows(RowsTile<128, 256, 2, 4, 1, 3, 2>{}, RowsTile<128, 128, 2, 2, 1, 4, 1>{});
+  else if (BM == 128) rows(RowsTile<128, 256, 2, 4, 1, 3, 2>{}, RowsTile<128, 256, 2, 4, 1, 3, 2>{});
+  else if (BM == 160) rows(RowsTile<160, 256, 2, 2, 1, 3, 1>{}, RowsTile<160, 128, 2, 2, 1, 4, 1>{});
+  else if (BM == 192 && one) rows(RowsTile<192, 192, 2, 2, 1, 3, 1>{}, RowsTile<192, 192, 2, 2, 1, 3, 1>{});
+  else if (BM == 192) rows(RowsTile<192, 256, 2, 2, 1, 2, 1>{}, RowsTile<192, 256, 2, 2, 1, 2, 1>{});
+  else if (one) rows(RowsTile<256, 128, 2, 2, 1, 3, 1>{}, RowsTile<256, 128, 2, 2, 1, 3, 1>{});
+  else rows(RowsTile<256, 256, 2, 2, 1, 2, 1>{}, RowsTile<256, 256, 2, 2, 1, 2, 1>{});
   return y;
 }
 

@@ -1,0 +1,259 @@
+// A tile of rows times a tile of W's rows, C(BM,BN) = A(BM,K) @ W(BN,K)^T, for products
+// of some dozen rows to some thousand: the workgroups of moe_routed.hip.
+//
+// Stages of 64 columns of K (RB bytes a row, 16 B piece c of row r at c ^ (r & 7): what
+// the lanes read together covers all banks) come into LDS by DMA, ST of them on their
+// way or in use. Rows of 128 B, since half lines cost a whole one (27 B a clock and CU
+// of L2's 50 with 64 B). A wave holds BM / WM rows of BN / WN columns, the larger the
+// fewer bytes of LDS a product reads: 128 x 128 with one wave a SIMD and 256 sums a lane
+// in accumulation registers. While it multiplies one half of a stage, it reads the other
+// half's fragments, or the next stage's behind the one barrier a stage has, and asks for
+// the stage that takes the place of the one just read.
+//
+// Measured, 4096 columns, cold W: 256 x 256 with two stages 1326 TF at 2800 rows of 28672
+// columns (a stage 1.4 us: products alone 1.1, at the clock that power leaves them, DMA
+// alone 1.2). Where one round of workgroups streams W, three stages of smaller tiles hide
+// more of memory: 333 rows 73 us with 192 x 224, 87 with 192 x 256 and two stages, 94 with
+// 192 x 128 and four (W alone, walked by 128 B a row, takes 50).
+// What it writes goes through LDS by whole lines (8 B a lane straight from the sums: 78 us
+// for 73, 513 for 496).
+// Tried and left: 32 columns a stage with five stages, L2 touched a stage or two ahead,
+// all of a stage's DMA at the phase's start: no faster; eight waves of half the columns:
+// as fast at large sizes, 10% slower at 2800 rows.
+
+#pragma once
+#include "common.h"
+
+// 16 B a lane from memory to LDS, base and l the wave's. An asm block, since the
+// compiler lets every read of LDS behind the builtin wait for all such loads; the
+// waits are the caller's. Nothing else here uses m0.
+DEVINL void dma16(const void* base, unsigned ofs, unsigned l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(l), "v"(ofs), "s"(base));
+}
+
+// Until at most N loads of the wave are on their way and its reads of LDS are done.
+template <int N>
+DEVINL void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N) : "memory");
+}
+
+// A product whose sums stay where they are in the accumulation registers: with more
+// than 256 registers a wave the compiler moves them around between products (four
+// moves each). It knows nothing of the product's latency: settle() goes ahead of what
+// reads the sums.
+DEVINL void mfma_acc(f32x4& c, bf16x8 x, bf16x8 y) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
+}
+
+DEVINL void settle() { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
+
+DEVINL short4v pack4(f32x4 v) {
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+  return __builtin_bit_cast(short4v, __builtin_convertvector(v, bf16x4));
+}
+
+DEVINL f32x4 pick(bool c, f32x4 x, f32x4 y) {
+  f32x4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = c ? x[e] : y[e];
+  return r;
+}
+
+// WM x WN waves, times WK groups that take 64 columns each of a stage; ST stages; MINW
+// waves a SIMD.
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int ST_, int MINW_>
+struct RowsTile {
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, ST = ST_;
+  static constexpr int MINW = MINW_;
+  static constexpr int NW = WM * WN * WK, THREADS = NW * 64;
+  static constexpr int MI = BM / WM / 16, NI = BN / WN / 16;
+  static constexpr int BK = 64 * WK, RB = BK * 2, RPC = 1024 / RB;
+  static constexpr int STAGE = (BM + BN) * RB;
+  static constexpr int AJ = BM * RB / 1024 / NW, LPW = AJ + BN * RB / 1024 / NW;
+  static constexpr int EXCHANGE = WK > 1 ? BM * BN * 4 : 0;
+  static constexpr int OUT_RS = NI * 64 + 16;            // f32 row of the way out
+  static constexpr int OUT = NW * 16 * OUT_RS;
+  static constexpr int LDS0 = ST * STAGE > EXCHANGE ? ST * STAGE : EXCHANGE;
+  static constexpr int LDS = LDS0 > OUT ? LDS0 : OUT;
+  static_assert(AJ * NW * 1024 == BM * RB &&
+                (LPW - AJ) * NW * 1024 == BN * RB && LDS <= 160 * 1024, "chunks");
+
+  typedef f32x4 Acc[MI][NI];
+
+  // Row of the tile (of A for j < AJ, else of W) that load j of the thread is for, and
+  // the byte in the row.
+  static DEVINL int load_row(int j, int wave, int lane) {
+    return ((j < AJ ? j : j - AJ) * NW + wave) * RPC + lane / (RB / 16);
+  }
+  static DEVINL unsigned load_byte(int j, int wave, int lane) {
+    return ((lane % (RB / 16)) ^ (load_row(j, wave, lane) & 7)) * 16;
+  }
+
+  // Sums of `steps` stages. ofs: bytes from ap (j < AJ) or wp, which move on by a
+  // stage's columns; beyond(j): what the rows of a load lie behind wp, the wave's.
+  template <typename B>
+  static DEVINL void run(const unsigned (&ofs)[LPW], const unsigned short* ap,
+                         const unsigned short* wp, int steps, unsigned char* lds,
+                         Acc& acc, B beyond) {
+    const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
+    const unsigned base = (unsigned)(unsigned long)(lptr_t)lds;
+#pragma unroll
+    for (int m = 0; m < MI; ++m)
+#pragma unroll
+      for (int n = 0; n < NI; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (steps <= 0) return;
+
+    auto load = [&](int j, int buf) {
+      const unsigned to = base + buf * STAGE;
+      if (j < AJ)
+        dma16(ap, ofs[j], to + (j * NW + wave) * 1024);
+      else
+        dma16(wp + beyond(j), ofs[j], to + BM * RB + ((j - AJ) * NW + wave) * 1024);
+    };
+    // a lane's pieces of its rows
+    unsigned fa[2], fw[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const unsigned piece = ((wk * 8 + s * 4 + hi) ^ (li & 7)) * 16;
+      fa[s] = (wm * MI * 16 + li) * RB + piece;
+      fw[s] = BM * RB + (wn * NI * 16 + li) * RB + piece;
+    }
+    bf16x8 af[2][MI], wf[2][NI];
+    auto frag = [&](int i, int s, int buf) {
+      const unsigned char* stage = lds + buf * STAGE;
+      if (i < NI)
+        wf[s][i] = as_bf16x8(
+            *reinterpret_cast<const short8*>(stage + fw[s] + i * 16 * RB));
+      else
+        af[s][i - NI] = as_bf16x8(
+            *reinterpret_cast<const short8*>(stage + fa[s] + (i - NI) * 16 * RB));
+    };
+    // products of half s of a stage, with the other set's reads from buf and loads to
+    // `to` in between
+    auto phase = [&](int s, int buf, auto loads, int to) {
+      constexpr int FR = MI + NI, P = MI * NI;
+      int p = 0;
+#pragma unroll
+      for (int i = 0; i < FR; ++i) {
+        frag(i, s ^ 1, buf);
+        if constexpr (decltype(loads)::value) {
+#pragma unroll
+          for (int j = i * LPW / FR; j < (i + 1) * LPW / FR; ++j) load(j, to);
+        }
+#pragma unroll
+        for (; p < (i + 1) * P / FR; ++p) {
+          if constexpr (MINW == 1)
+            mfma_acc(acc[p % MI][p / MI], wf[s][p / MI], af[s][p % MI]);
+          else
+            acc[p % MI][p / MI] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                wf[s][p / MI], af[s][p % MI], acc[p % MI][p / MI], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto barrier = [&]() {
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    // until all but n stages have landed
+    auto wait = [&](int n) {
+      static_assert(ST <= 4, "stages");
+      if (n >= 3) wait_loads<3 * LPW>();
+      else if (n == 2) wait_loads<2 * LPW>();
+      else if (n == 1) wait_loads<LPW>();
+      else wait_loads<0>();
+    };
+
+#pragma unroll
+    for (int s = 0; s < ST; ++s)
+      if (s < steps) {
+#pragma unroll
+        for (int j = 0; j < LPW; ++j) load(j, s);
+        ap += BK;
+        wp += BK;
+      }
+    wait(min(ST, steps) - 1);
+    barrier();
+#pragma unroll
+    for (int i = 0; i < MI + NI; ++i) frag(i, 0, 0);
+    int buf = 0, t = 0;
+    for (; t + ST < steps; ++t) {
+      phase(0, buf, std::false_type{}, 0);
+      wait_loads<(ST - 2) * LPW>();
+      barrier();
+      const int next = buf + 1 == ST ? 0 : buf + 1;
+      phase(1, next, std::true_type{}, buf);
+      ap += BK;
+      wp += BK;
+      buf = next;
+      if (MINW == 1) settle();
+    }
+    for (; t < steps; ++t) {
+      phase(0, buf, std::false_type{}, 0);
+      wait(steps - 2 - t);
+      barrier();
+      buf = buf + 1 == ST ? 0 : buf + 1;
+      // behind the last stage these reads bring what nothing uses
+      phase(1, buf, std::false_type{}, 0);
+      if (MINW == 1) settle();
+    }
+
+    if constexpr (WK > 1) {
+      // a k group keeps half of the columns and hands the others' sums over
+      static_assert(WK == 2 && NI % 2 == 0, "halves");
+      constexpr int H = NI / 2;
+      __syncthreads();
+      f32x4* ex = reinterpret_cast<f32x4*>(lds) + (wm * WN + wn) * (MI * NI * 64);
+#pragma unroll
+      for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int n = 0; n < H; ++n)
+          ex[((wk ^ 1) * MI * H + m * H + n) * 64 + lane] =
+              pick(wk, acc[m][n], acc[m][n + H]);
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int n = 0; n < H; ++n)
+          acc[m][n] = pick(wk, acc[m][n + H], acc[m][n]) +
+                      ex[(wk * MI * H + m * H + n) * 64 + lane];
+    }
+    __syncthreads();   // the way out takes the place of the stages
+  }
+
+  // The wave's columns of the tile after run(): COLS of them from col0().
+  static constexpr int COLS = NI * 16 / WK;
+  static DEVINL int col0() {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    return wave / WK % WN * NI * 16 + wave % WK * COLS;
+  }
+  static DEVINL int row0() {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / (WK * WN) * MI * 16;
+  }
+
+  // Sixteen rows at a time, of `strips` strips of 16 columns, through LDS, so that
+  // whole lines are written: value(n) gives a lane's four of strip n, as f32 or bf16;
+  // put(row, column, eight values as they were).
+  template <int STRIPS, typename V, typename P>
+  static DEVINL void out16(unsigned char* lds, V value, P put) {
+    typedef decltype(value(0)) T4;
+    constexpr int E = sizeof(T4) / 4, RS = STRIPS * 16 * E + 16;
+    const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
+    unsigned char* mine = lds + threadIdx.x / WAVE * (16 * OUT_RS);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int n = 0; n < STRIPS; ++n)
+      *reinterpret_cast<T4*>(mine + li * RS + (n * 16 + hi * 4) * E) = value(n);
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < (STRIPS + 1) / 2; ++i) {
+      const int at = i * 64 + lane, r = at / (STRIPS * 2), c = at % (STRIPS * 2) * 8;
+      if (STRIPS % 2 && r >= 16) break;
+      struct alignas(16) T8 { T4 lo, hi; };
+      put(r, c, *reinterpret_cast<const T8*>(mine + r * RS + c * E));
+    }
+  }
+};

@@ -22,12 +22,13 @@
 //  * moe_skinny_kernel — up to 32 tokens: streams each chosen expert's weights
 //    once; a workgroup finds its expert's slots by scanning the ids itself, so
 //    a decode step needs no sort.
-//  * moe_sort_kernel + moe_tile_kernel — longer batches: expert-sorted slots,
-//    MFMA tiles of 64 or 128 rows staged through LDS.
+//  * moe_sort_kernel + moe_rows_kernel — longer batches: expert-sorted slots,
+//    tiles of 64 to 256 rows (gemm_rows.hip).
 //  * moe_simple_kernel — f32 arithmetic on f32 data.
 
 #pragma once
 #include "common.h"
+#include "gemm_rows.hip"
 #include "rows.hip"
 
 static constexpr int MOE_MAX_E = 1024;
@@ -262,168 +263,85 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// tile: grid of column tiles * row tiles; K % 64 == 0
+// tile: grid of column tiles * row tiles; K % 64 == 0, N % 8 == 0
 // ---------------------------------------------------------------------------
 
-// Place of 16 B piece c of a row of four: the lanes that read together (four rows each
-// of 0, 3 at one piece and 1, 2 at the next, by fours) cover all banks.
-DEVINL int moe_piece(int r, int c) {
-  const int g = (r >> 2) & 3;
-  return c ^ ((g & 1) << 1) ^ ((g >> 1) * 3);
-}
-
 // UP: A row = sorted slot / top, out row = sorted position, N = activations
-//     (two planes: 128 per tile, 128 gate rows and 128 up rows of W; one: 256).
-// else: A row = sorted position, out row = slot, 256 columns per tile.
+//     (two planes: half of a tile's rows of W are gates, half ups).
+// else: A row = sorted position, out row = slot.
 //
-// A BM x 256 tile per workgroup; each of the four waves holds all BM rows of
-// 64 columns, so a W fragment read from LDS feeds BM / 16 MFMAs. LDS rows are
-// 64 B (32 of K) in four 16 B pieces, piece c of row r at moe_piece(r, c).
+// A tile of gemm_rows.hip a workgroup: T::BM rows of one expert.
 //
 // Every expert's weights come from memory once at best; what bounds it is how often
 // they come again. Hence the order of the tiles below: an expert's row tiles take one
 // column after the other together and find W in their XCD's L2. Tiles of several
-// experts in a group of eight: 1430 us for both products at 1400 tokens, two of eight
-// experts, 4096 x 14336, now 1229 (5000 tokens: 4421, 4101).
-// Few rows an expert (BM 64) are a stream of weights: two of three buffers are on
-// their way while the third is computed with (64 tokens: 737 -> 615 us, 4.6 TB/s). At
-// BM 128 that much ahead costs more in L2 than it hides (1340 us for 1229), as does a
-// start of K that differs between columns; tiles of 32 x 32 are slower, too (1289).
-template <int BM, int UP>
-__global__ __launch_bounds__(256, 2) void moe_tile_kernel(
+// experts in a group of eight took 1430 us for both products at 1400 tokens, two of
+// eight experts, 4096 x 14336, in this order 1254 on tiles of 128 x 256 with 32 of K a
+// step, all rows a wave, and 1033 on these (160 tokens 637, 496; 700: 934, 715; 4000:
+// 3255, 2715).
+template <typename T, int UP>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
     const unsigned short* __restrict__ A, const unsigned short* __restrict__ W,
     const int* __restrict__ off, const int* __restrict__ sorted,
     const int* __restrict__ tiles, const float* __restrict__ wts,
     unsigned short* __restrict__ C, int max_tiles, int ntn, int top, int N,
     int K, int lda, int ldc, GluConst glu) {
-  constexpr int BK = 32, RB = BK * 2, BN = 256, HN = BN / 2;
-  constexpr int AI = BM * 4 / 256, BI = BN * 4 / 256;  // 16 B pieces per thread
-  constexpr int MT = BM / 16, NT = 4, NB = BM > 64 ? 2 : 3;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NB][(BM + BN) * RB];
-
-  // an expert's row tiles side by side, column after column: they read the same W
-  // within the time that L2 keeps it
-  const int nrt = tiles[4 * max_tiles];
-  const int total = nrt * ntn;
+  static_assert(T::WK == 1 && (UP < 2 || T::NI % 2 == 0), "pairs");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int nrt = tiles[4 * max_tiles], total = nrt * ntn;
   if ((int)blockIdx.x >= total) return;
   const int id = xcd_order(blockIdx.x, total);
   const int first = tiles[4 * (id / ntn) + 2], gsz = tiles[4 * (id / ntn) + 3];
   const int rt = first + (id - first * ntn) % gsz, nt = (id - first * ntn) / gsz;
-  const int e = tiles[4 * rt];
-  const int p0 = tiles[4 * rt + 1];
-  const int cnt = min(BM, off[e + 1] - p0);
-  const int n0 = nt * (UP == 2 ? HN : BN);
+  const int e = tiles[4 * rt], p0 = tiles[4 * rt + 1];
+  const int cnt = min(T::BM, off[e + 1] - p0);
+  constexpr int HALF = T::NI * 8;                    // a wave's gates, then its ups
+  const int n0 = nt * (UP == 2 ? T::BN / 2 : T::BN);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int li = lane & 15, hi = lane >> 4;
+  const int lane = threadIdx.x & (WAVE - 1), li = lane & 15;
 
-  const unsigned short* ap[AI];
-  const unsigned short* bp[BI];
+  unsigned ofs[T::LPW];
 #pragma unroll
-  for (int i = 0; i < AI; ++i) {
-    const int ch = (i * 4 + wave) * 64 + lane;
-    const int r = ch / 4, c = moe_piece(r, ch % 4);
-    const int p = p0 + min(r, cnt - 1);
-    ap[i] = A + (long)(UP ? sorted[p] / top : p) * lda + c * 8;
-  }
-#pragma unroll
-  for (int i = 0; i < BI; ++i) {
-    const int ch = (i * 4 + wave) * 64 + lane;
-    const int r = ch / 4, c = moe_piece(r, ch % 4);
-    const long wrow =
-        UP == 2 ? ((long)e * 2 + r / HN) * N + min(n0 + r % HN, N - 1)
-                : (long)e * N + min(n0 + r, N - 1);
-    bp[i] = W + wrow * K + c * 8;
-  }
-  auto issue = [&](int k, int buf) {
-#pragma unroll
-    for (int i = 0; i < AI; ++i)
-      copy16_to_lds(ap[i] + k, lds[buf] + (i * 4 + wave) * 1024);
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-      copy16_to_lds(bp[i] + k, lds[buf] + BM * RB + (i * 4 + wave) * 1024);
-  };
-  // W rows of this wave's four column tiles: two planes pair gate and up columns
-  int brow[NT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n)
-    brow[n] = (UP == 2 ? (n >> 1) * HN + wave * 32 + (n & 1) * 16
-                  : wave * 64 + n * 16) + li;
-
-  f32x4 acc[MT][NT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  issue(0, 0);
-  if (NB == 3) issue(BK, 1);  // K >= 64
-  int buf = 0, to = NB - 1;
-  for (int k = 0; k < K; k += BK) {
-    if (NB == 2) {
-      __syncthreads();
+  for (int j = 0; j < T::LPW; ++j) {
+    const int r = T::load_row(j, wave, lane);
+    unsigned row;
+    if (j < T::AJ) {
+      const int i = min(r, cnt - 1);
+      row = (unsigned)(UP ? sorted[p0 + i] / top : i) * (unsigned)lda;
     } else {
-      // this step's loads have landed, the next one's stay on their way
-      if (k + BK < K)
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(AI + BI) : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-      // and everyone's; the buffer of the last step is free
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
+      row = (unsigned)min(UP == 2 ? r / (2 * HALF) * HALF + r % HALF : r, N - 1 - n0) *
+            (unsigned)K;
     }
-    if (k + (NB - 1) * BK < K) issue(k + (NB - 1) * BK, to);
-    bf16x8 wf[NT];
-#pragma unroll
-    for (int n = 0; n < NT; ++n)
-      wf[n] = as_bf16x8(*reinterpret_cast<const short8*>(
-          lds[buf] + (BM + brow[n]) * RB + moe_piece(brow[n], hi) * 16));
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      const int r = m * 16 + li;
-      const bf16x8 af = as_bf16x8(*reinterpret_cast<const short8*>(
-          lds[buf] + r * RB + moe_piece(r, hi) * 16));
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], af,
-                                                            acc[m][n], 0, 0, 0);
-    }
-    buf = buf == NB - 1 ? 0 : buf + 1;
-    to = to == NB - 1 ? 0 : to + 1;
+    ofs[j] = row * 2 + T::load_byte(j, wave, lane);
   }
+  typename T::Acc acc;
+  T::run(ofs, UP ? A : A + (long)p0 * lda, W + ((long)e * (UP ? UP : 1) * N + n0) * K,
+         K / T::BK, lds, acc, [&](int j) {
+           // the eight rows of a load are of one plane
+           return UP == 2 ? (long)(T::load_row(j, wave, 0) / HALF % 2) * N * K : 0L;
+         });
 
-  // a lane holds columns hi*4..hi*4+3 of row li in every tile
+  const int r0 = T::row0(), c0 = n0 + (UP == 2 ? T::col0() / 2 : T::col0());
+  constexpr int S = UP == 2 ? T::NI / 2 : T::NI;
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int r = m * 16 + li;
-    if (r >= cnt) continue;
-    const int sl = sorted[p0 + r];
-    const float w = wts ? wts[sl] : 1.f;
-    if constexpr (UP == 2) {
+  for (int m = 0; m < T::MI; ++m) {
+    const int r = r0 + m * 16 + li;
+    const float w = wts && r < cnt ? wts[sorted[p0 + r]] : 1.f;
+    T::template out16<S>(lds, [&](int n) {
+      f32x4 v;
 #pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        const int col = n0 + wave * 32 + n * 16 + hi * 4;
-        if (col >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          v[j] = gated(glu, acc[m][n][j] * w, acc[m][n + 2][j] * w);
-        stv<4>(C + (long)(p0 + r) * ldc + col, v);
+      for (int j = 0; j < 4; ++j) {
+        v[j] = acc[m][n][j] * w;
+        if constexpr (UP == 2) v[j] = gated(glu, v[j], acc[m][n + S][j] * w);
+        if constexpr (UP == 1) v[j] = relu_sq(v[j]);
       }
-    } else {
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const int col = n0 + wave * 64 + n * 16 + hi * 4;
-        if (col >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          v[j] = acc[m][n][j] * w;
-          if constexpr (UP == 1) v[j] = relu_sq(v[j]);
-        }
-        stv<4>(C + (long)(UP ? p0 + r : sl) * ldc + col, v);
-      }
-    }
+      return pack4(v);
+    }, [&](int i, int c, auto v) {
+      const int at = r0 + m * 16 + i;
+      if (at >= cnt || c0 + c >= N) return;
+      const long row = UP ? p0 + at : sorted[p0 + at];
+      *reinterpret_cast<decltype(v)*>(C + row * ldc + c0 + c) = v;
+    });
   }
 }
 
