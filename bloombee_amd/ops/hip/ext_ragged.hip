@@ -802,29 +802,20 @@ void attn_ragged(Tensor q, Tensor kp, OptTensor vp, Tensor table,
 // routed experts
 // ---------------------------------------------------------------------------
 
-// Rows of a tile for experts of a rows on average: what takes the fewest padded rows,
-// with what a tile costs beside them, at counts that spread by sqrt(a). Two products of
-// eight experts, 4096 x 14336, us with tiles of 64 to 256 rows (the least bounds are
-// 540 of weights, 1.9 a row of an expert of operations at 1.5 PF):
+// Rows of a tile for experts of a rows on average, counts that spread by sqrt(a): the
+// lowest one that takes them at once, which streams weights with the most of them on
+// their way; beyond, several tiles of heights of their own (moe_rows_any_kernel). Two
+// products of eight experts, 4096 x 14336, us with tiles of 64 to 192 rows and those:
 //   20 rows 484 with 64;  64: 630, 520 with 96, 525 with 128, 547 with 160
-//   96: 619, 651, 555, 573, 591 with 192;  125: 603 with 160, 620, 679 with 256
-//   225: 750 with 128, 889 with 160, 981, 750;  350: 1154 with 128, 1033 with 192, 1192
-//   425: 1286 with 128, 1320, 1516, 1196 with 256;  1000: 2824, 2825, 2799, 2671
-// Several tiles of 96 or 160 are slower than this makes them (300 rows: 1156, 1076,
-// two of 192 rows 1014).
-static int moe_rows(float a) {
-  const float s = sqrtf(a);
-  int best = 64;
-  float least = INFINITY;
-  for (int bm : {64, 96, 128, 160, 192, 256}) {
-    const float tiles = (ceilf((a - s) / bm) + ceilf(a / bm) + ceilf((a + s) / bm)) / 3;
-    if (tiles > 1 && (bm == 96 || bm == 160)) continue;
-    if (tiles * (bm + 48) < least) {
-      least = tiles * (bm + 48);
-      best = bm;
-    }
-  }
-  return best;
+//   96: 695, 788, 553, 572, 614;  150: 644 with 192, 675;  175: 684, 722
+//   225: 809 with 128, 895, 1067, 768;  350: 1279 with 128, 1296, 1132, 1105
+//   1000: 3039 with 128, 2922, 2954, 2696
+// The least bounds are 540 of weights and 1.9 a row of operations at 1.5 PF.
+static int moe_height(float a) {
+  const float most = a + sqrtf(a);
+  for (int rows : {64, 96, 128, 160, 192})
+    if (most <= rows) return rows;
+  return 256;
 }
 
 // h (N, K), up (E, planes, F, K), down (E, Wp, F), ids/wts (N, top)
@@ -896,8 +887,8 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     return y;
   }
 
-  const int BM = ta == at::kBFloat16 ? moe_rows(S / (float)E) : 64;
-  const int max_tiles = S / BM + std::min(S, E);  // the count goes behind
+  const int BM = ta == at::kBFloat16 ? moe_height(S / (float)E) : 64;
+  const int max_tiles = S / (BM == 256 ? 128 : BM) + std::min(S, E);  // and the count
   auto iopt = ids.options();
   auto off = torch::empty({E + 1}, iopt);
   auto sorted = torch::empty({S}, iopt);
@@ -911,50 +902,55 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     by_planes([&](auto np) {
       moe_simple_kernel<decltype(np)::value>
           <<<dim3(F / 64, max_tiles), 256, 0, st>>>(
-              h.data_ptr<float>(), up.data_ptr<float>(), offp, sp, tp, w1,
+              h.data_ptr<float>(), up.data_ptr<float>(), sp, tp, w1,
               act.data_ptr<float>(), top, F, K, K, F, glu);
     });
     check_launch();
     moe_simple_kernel<0><<<dim3(Wp / 64, max_tiles), 256, 0, st>>>(
-        act.data_ptr<float>(), down.data_ptr<float>(), offp, sp, tp, w2,
+        act.data_ptr<float>(), down.data_ptr<float>(), sp, tp, w2,
         y.data_ptr<float>(), top, Wp, F, F, Wp, glu);
     check_launch();
     return y;
   }
+  auto product = [&](auto up_planes, auto kernel, int bn, int threads, int lds) {
+    constexpr int UP = decltype(up_planes)::value;
+    MoeArgs a{};
+    a.A = (const bf16_bits*)(UP ? h : act).data_ptr();
+    a.W = (const bf16_bits*)(UP ? up : down).data_ptr();
+    a.sorted = sp;
+    a.tiles = tp;
+    a.wts = UP ? w1 : w2;
+    a.C = (bf16_bits*)(UP ? act : y).data_ptr();
+    a.max_tiles = max_tiles;
+    a.top = top;
+    a.N = a.ldc = UP ? F : Wp;
+    a.K = a.lda = UP ? K : F;
+    a.glu = glu;
+    allow_lds(kernel, lds);
+    kernel<<<moe_columns<UP>(a.N, bn) * max_tiles, threads, lds, st>>>(a);
+    check_launch();
+  };
+  const std::integral_constant<int, 0> second{};
   auto rows = [&](auto up_tile, auto down_tile) {
     typedef decltype(up_tile) U;
     typedef decltype(down_tile) D;
-    const int per = up.size(1) == 2 ? U::BN / 2 : U::BN;
-    const int nu = (F + per - 1) / per, nd = (Wp + D::BN - 1) / D::BN;
     by_planes([&](auto np) {
-      auto k = moe_rows_kernel<U, decltype(np)::value>;
-      allow_lds(k, U::LDS);
-      k<<<nu * max_tiles, U::THREADS, U::LDS, st>>>(
-          (const bf16_bits*)h.data_ptr(), (const bf16_bits*)up.data_ptr(), offp,
-          sp, tp, w1, (bf16_bits*)act.data_ptr(), max_tiles, nu, top, F, K, K,
-          F, glu);
+      product(np, moe_rows_kernel<U, decltype(np)::value>, U::BN, U::THREADS, U::LDS);
     });
-    check_launch();
-    auto k = moe_rows_kernel<D, 0>;
-    allow_lds(k, D::LDS);
-    k<<<nd * max_tiles, D::THREADS, D::LDS, st>>>(
-        (const bf16_bits*)act.data_ptr(), (const bf16_bits*)down.data_ptr(),
-        offp, sp, tp, w2, (bf16_bits*)y.data_ptr(), max_tiles, nd, top, Wp, F,
-        F, Wp, glu);
-    check_launch();
+    product(second, moe_rows_kernel<D, 0>, D::BN, D::THREADS, D::LDS);
   };
-  // an expert's rows in one tile: its weights are streamed, more of them ahead;
-  // in several: wide tiles
-  const bool one = S / (float)E + sqrtf(S / (float)E) <= BM;
   if (BM == 64) rows(RowsTile<64, 128, 2, 2, 1, 3, 2>{}, RowsTile<64, 128, 2, 2, 1, 3, 2>{});
   else if (BM == 96) rows(RowsTile<96, 128, 2, 2, 1, 4, 1>{}, RowsTile<96, 128, 2, 2, 1, 4, 1>{});
-  else if (BM == 128 && one) rows(RowsTile<128, 256, 2, 4, 1, 3, 2>{}, RowsTile<128, 128, 2, 2, 1, 4, 1>{});
-  else if (BM == 128) rows(RowsTile<128, 256, 2, 4, 1, 3, 2>{}, RowsTile<128, 256, 2, 4, 1, 3, 2>{});
+  else if (BM == 128) rows(RowsTile<128, 256, 2, 4, 1, 3, 2>{}, RowsTile<128, 128, 2, 2, 1, 4, 1>{});
   else if (BM == 160) rows(RowsTile<160, 256, 2, 2, 1, 3, 1>{}, RowsTile<160, 128, 2, 2, 1, 4, 1>{});
-  else if (BM == 192 && one) rows(RowsTile<192, 192, 2, 2, 1, 3, 1>{}, RowsTile<192, 192, 2, 2, 1, 3, 1>{});
-  else if (BM == 192) rows(RowsTile<192, 256, 2, 2, 1, 2, 1>{}, RowsTile<192, 256, 2, 2, 1, 2, 1>{});
-  else if (one) rows(RowsTile<256, 128, 2, 2, 1, 3, 1>{}, RowsTile<256, 128, 2, 2, 1, 3, 1>{});
-  else rows(RowsTile<256, 256, 2, 2, 1, 2, 1>{}, RowsTile<256, 256, 2, 2, 1, 2, 1>{});
+  else if (BM == 192) rows(RowsTile<192, 192, 2, 2, 1, 3, 1>{}, RowsTile<192, 192, 2, 2, 1, 3, 1>{});
+  else {
+    constexpr int LDS = RowsTile<160, 256, 2, 2, 1, 3, 1>::LDS;   // the largest
+    by_planes([&](auto np) {
+      product(np, moe_rows_any_kernel<decltype(np)::value>, 128, 256, LDS);
+    });
+    product(second, moe_rows_any_kernel<0>, 128, 256, LDS);
+  }
   return y;
 }
 

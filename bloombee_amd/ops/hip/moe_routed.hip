@@ -61,9 +61,10 @@ DEVINL int xcd_order(int id, int n) {
 // sort: one workgroup of 1024
 // ---------------------------------------------------------------------------
 
-// off (E+1), sorted (S) slots, tiles (max_tiles + 1, 4): expert (-1 = unused), first
-// sorted position, group's first tile and number of tiles of every BM-row tile; then
-// the number of tiles. A group is a share of one expert's tiles, at most MOE_GROUP.
+// off (E+1), sorted (S) slots, tiles (max_tiles + 1, 4): expert and MOE_MAX_E * rows
+// (-1 = unused), first sorted position, group's first tile and number of tiles of every
+// tile; then the number of tiles. An expert's rows are shared out evenly to as few tiles
+// of up to BM as there can be (nearly), and its tiles to groups of at most MOE_GROUP.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     const int* __restrict__ ids, int* __restrict__ off,
     int* __restrict__ sorted, int* __restrict__ tiles, int S, int E, int BM,
@@ -77,7 +78,9 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  const int c = cnt[tid], nt = (c + BM - 1) / BM;
+  // two tiles read an expert's weights from one L2 faster than a high one takes them
+  // from memory (225 rows: 800 us for 915)
+  const int c = cnt[tid], nt = BM == 256 && c > 192 && c <= 256 ? 2 : (c + BM - 1) / BM;
   scan[tid] = c;
   tscan[tid] = nt;
   __syncthreads();
@@ -97,8 +100,9 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
     for (int k = 0; k < nt; ++k) {
       const int at = t0 + k, g = k / per * per;
       if (at < max_tiles) {
-        tiles[4 * at] = tid;
-        tiles[4 * at + 1] = first + k * BM;
+        const int from = (long)c * k / nt, to = (long)c * (k + 1) / nt;
+        tiles[4 * at] = tid + MOE_MAX_E * (to - from);
+        tiles[4 * at + 1] = first + from;
         tiles[4 * at + 2] = t0 + g;
         tiles[4 * at + 3] = min(per, min(nt, max_tiles - t0) - g);
       }
@@ -277,26 +281,51 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(
 // column after the other together and find W in their XCD's L2. Tiles of several
 // experts in a group of eight took 1430 us for both products at 1400 tokens, two of
 // eight experts, 4096 x 14336, in this order 1254 on tiles of 128 x 256 with 32 of K a
-// step, all rows a wave, and 1033 on these (160 tokens 637, 496; 700: 934, 715; 4000:
-// 3255, 2715).
-template <typename T, int UP>
-__global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
-    const unsigned short* __restrict__ A, const unsigned short* __restrict__ W,
-    const int* __restrict__ off, const int* __restrict__ sorted,
-    const int* __restrict__ tiles, const float* __restrict__ wts,
-    unsigned short* __restrict__ C, int max_tiles, int ntn, int top, int N,
-    int K, int lda, int ldc, GluConst glu) {
-  static_assert(T::WK == 1 && (UP < 2 || T::NI % 2 == 0), "pairs");
-  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  const int nrt = tiles[4 * max_tiles], total = nrt * ntn;
-  if ((int)blockIdx.x >= total) return;
+// step, all rows a wave, and 1105 on these (160 tokens 637, 495; 700: 934, 684; 4000:
+// 3255, 2696).
+struct MoeArgs {
+  const unsigned short* A;   // rows of lda
+  const unsigned short* W;   // (E, UP or 1, N, K)
+  const int* sorted;
+  const int* tiles;
+  const float* wts;          // or null
+  unsigned short* C;         // rows of ldc
+  int max_tiles, top, N, K, lda, ldc;
+  GluConst glu;
+};
+
+struct MoeTile {
+  int e, p0, cnt, nt;        // expert, first sorted position, rows, column tile
+};
+
+// The workgroup's tile; false: none.
+DEVINL bool moe_tile(const MoeArgs& a, int ntn, MoeTile& t) {
+  const int total = a.tiles[4 * a.max_tiles] * ntn;
+  if ((int)blockIdx.x >= total) return false;
   const int id = xcd_order(blockIdx.x, total);
-  const int first = tiles[4 * (id / ntn) + 2], gsz = tiles[4 * (id / ntn) + 3];
-  const int rt = first + (id - first * ntn) % gsz, nt = (id - first * ntn) / gsz;
-  const int e = tiles[4 * rt], p0 = tiles[4 * rt + 1];
-  const int cnt = min(T::BM, off[e + 1] - p0);
+  const int* group = a.tiles + 4 * (id / ntn);
+  const int first = group[2], gsz = group[3];
+  const int rt = first + (id - first * ntn) % gsz;
+  t.nt = (id - first * ntn) / gsz;
+  t.e = a.tiles[4 * rt] % MOE_MAX_E;
+  t.cnt = a.tiles[4 * rt] / MOE_MAX_E;
+  t.p0 = a.tiles[4 * rt + 1];
+  return true;
+}
+
+// Column tiles of BN.
+template <int UP>
+__host__ DEVINL int moe_columns(int N, int BN) {
+  const int per = UP == 2 ? BN / 2 : BN;
+  return (N + per - 1) / per;
+}
+
+template <typename T, int UP>
+DEVINL void moe_rows(const MoeArgs& a, const MoeTile& t, unsigned char* lds) {
+  static_assert(T::WK == 1 && (UP < 2 || T::NI % 2 == 0), "pairs");
+  const int p0 = t.p0, cnt = t.cnt, N = a.N, K = a.K;
   constexpr int HALF = T::NI * 8;                    // a wave's gates, then its ups
-  const int n0 = nt * (UP == 2 ? T::BN / 2 : T::BN);
+  const int n0 = t.nt * (UP == 2 ? T::BN / 2 : T::BN);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x & (WAVE - 1), li = lane & 15;
 
@@ -307,7 +336,7 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
     unsigned row;
     if (j < T::AJ) {
       const int i = min(r, cnt - 1);
-      row = (unsigned)(UP ? sorted[p0 + i] / top : i) * (unsigned)lda;
+      row = (unsigned)(UP ? a.sorted[p0 + i] / a.top : i) * (unsigned)a.lda;
     } else {
       row = (unsigned)min(UP == 2 ? r / (2 * HALF) * HALF + r % HALF : r, N - 1 - n0) *
             (unsigned)K;
@@ -315,7 +344,8 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
     ofs[j] = row * 2 + T::load_byte(j, wave, lane);
   }
   typename T::Acc acc;
-  T::run(ofs, UP ? A : A + (long)p0 * lda, W + ((long)e * (UP ? UP : 1) * N + n0) * K,
+  T::run(ofs, UP ? a.A : a.A + (long)p0 * a.lda,
+         a.W + ((long)t.e * (UP ? UP : 1) * N + n0) * K,
          K / T::BK, lds, acc, [&](int j) {
            // the eight rows of a load are of one plane
            return UP == 2 ? (long)(T::load_row(j, wave, 0) / HALF % 2) * N * K : 0L;
@@ -326,22 +356,53 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
 #pragma unroll
   for (int m = 0; m < T::MI; ++m) {
     const int r = r0 + m * 16 + li;
-    const float w = wts && r < cnt ? wts[sorted[p0 + r]] : 1.f;
+    const float w = a.wts && r < cnt ? a.wts[a.sorted[p0 + r]] : 1.f;
     T::template out16<S>(lds, [&](int n) {
       f32x4 v;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         v[j] = acc[m][n][j] * w;
-        if constexpr (UP == 2) v[j] = gated(glu, v[j], acc[m][n + S][j] * w);
+        if constexpr (UP == 2) v[j] = gated(a.glu, v[j], acc[m][n + S][j] * w);
         if constexpr (UP == 1) v[j] = relu_sq(v[j]);
       }
       return pack4(v);
     }, [&](int i, int c, auto v) {
       const int at = r0 + m * 16 + i;
       if (at >= cnt || c0 + c >= N) return;
-      const long row = UP ? p0 + at : sorted[p0 + at];
-      *reinterpret_cast<decltype(v)*>(C + row * ldc + c0 + c) = v;
+      const long row = UP ? p0 + at : a.sorted[p0 + at];
+      *reinterpret_cast<decltype(v)*>(a.C + row * a.ldc + c0 + c) = v;
     });
+  }
+}
+
+template <typename T, int UP>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(MoeArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  MoeTile t;
+  if (moe_tile(a, moe_columns<UP>(a.N, T::BN), t)) moe_rows<T, UP>(a, t, lds);
+}
+
+// Tiles of up to 256 rows on the height that fits, since experts' counts differ. They are
+// 256 columns wide, but where those leave CUs idle in their last round half as wide ones
+// end sooner: a stage of 64 columns takes 1.14 us there, 0.66 here (19 tiles of 4096
+// columns: two rounds for three).
+template <int UP>
+__global__ __launch_bounds__(256, 1) void moe_rows_any_kernel(MoeArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int tiles = a.tiles[4 * a.max_tiles];
+  const int wide = moe_columns<UP>(a.N, 256), half = moe_columns<UP>(a.N, 128);
+  MoeTile t;
+  if ((tiles * wide + 255) / 256 * 12 <= (tiles * half + 255) / 256 * 7) {
+    if (!moe_tile(a, wide, t)) return;
+    if (t.cnt > 192) moe_rows<RowsTile<256, 256, 2, 2, 1, 2, 1>, UP>(a, t, lds);
+    else if (t.cnt > 160) moe_rows<RowsTile<192, 256, 2, 2, 1, 2, 1>, UP>(a, t, lds);
+    else if (t.cnt > 128) moe_rows<RowsTile<160, 256, 2, 2, 1, 3, 1>, UP>(a, t, lds);
+    else moe_rows<RowsTile<128, 256, 2, 2, 1, 3, 1>, UP>(a, t, lds);
+  } else {
+    if (!moe_tile(a, half, t)) return;
+    if (t.cnt > 192) moe_rows<RowsTile<256, 128, 2, 2, 1, 3, 1>, UP>(a, t, lds);
+    else if (t.cnt > 128) moe_rows<RowsTile<192, 128, 2, 2, 1, 3, 1>, UP>(a, t, lds);
+    else moe_rows<RowsTile<128, 128, 2, 2, 1, 4, 1>, UP>(a, t, lds);
   }
 }
 
@@ -352,16 +413,16 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void moe_rows_kernel(
 template <int UP>
 __global__ __launch_bounds__(256) void moe_simple_kernel(
     const float* __restrict__ A, const float* __restrict__ W,
-    const int* __restrict__ off, const int* __restrict__ sorted,
+    const int* __restrict__ sorted,
     const int* __restrict__ tiles, const float* __restrict__ wts,
     float* __restrict__ C, int top, int N, int K, int lda, int ldc,
     GluConst glu) {
   constexpr int NW = UP ? UP : 1, BK = 16;
   __shared__ float al[BK][64 + 4], wl[NW][BK][64 + 4];
-  const int e = tiles[4 * blockIdx.y];
-  if (e < 0) return;
+  if (tiles[4 * blockIdx.y] < 0) return;
+  const int e = tiles[4 * blockIdx.y] % MOE_MAX_E;
+  const int cnt = tiles[4 * blockIdx.y] / MOE_MAX_E;
   const int p0 = tiles[4 * blockIdx.y + 1];
-  const int cnt = min(64, off[e + 1] - p0);
   const int n0 = blockIdx.x * 64;
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
   float acc[NW][4][4] = {};

@@ -97,16 +97,17 @@ def test_routed_mlp(N, E, top, H, I):
     ([40, 0, 1, 64, 65], 64, 64, 320),               # tiles of 64 rows, two steps each
     ([129, 1, 300, 0, 127], 192, 192, 64),           # tiles of 128
     ([0, 1030, 128, 2, 2400], 128, 320, 64),         # groups of 5 and 4, of 7, 6 and 6
-    # tiles of every height, of one an expert and of several, with fewer steps than
-    # buffers and more, columns that end within a tile
+    # tiles of every height, with fewer steps than buffers and more, columns that end
+    # within a tile
     ([57, 97, 38], 320, 192, 320),                   # 96 rows
     ([87, 1, 200], 448, 320, 192),                   # 128
     ([118, 161, 75], 64, 64, 64),                    # 160
     ([148, 193, 103], 128, 448, 320),                # 192
-    ([179, 257, 101], 448, 128, 448),                # 256
-    ([193, 385, 300], 320, 448, 64),                 # 192, two
-    ([513, 770, 1], 192, 320, 320),                  # 256, two and more
-    ([580, 640, 511], 448, 192, 192),                # 128, five
+    ([179, 257, 101], 448, 128, 448),                # 101 to 179 rows, half as wide
+    ([193, 385, 300, 513], 320, 448, 64),            # 97 to 193
+    ([513, 770, 1], 64, 320, 320),
+    # 40 tiles or more, 256 columns wide: 97, 128, 150, 171, 192, 200 and 256 rows
+    ([193, 256, 300, 342, 384, 400, 512] * 4, 192, 832, 1600),
 ])
 @pytest.mark.parametrize("planes", [1, 2])
 def test_order_of_tiles(counts, K, F, W, planes):
