@@ -196,6 +196,13 @@ class LlamaBlock(torch.nn.Module):
                 y = y + d
         return y
 
+    def _gated(self, y):
+        """The gated product of gate_up's result."""
+        if (getattr(self, "_w4", None) is None
+                and getattr(self, "lora_delta", None) is None):
+            return ops.linear_gated(y, self.gate_up_w)
+        return ops.swiglu(self._lin(y, self.gate_up_w, "gate_up_w"))
+
     # ------------------------------------------------------------------
     # inference path (HIP kernels, paged KV)
     # ------------------------------------------------------------------
@@ -266,8 +273,7 @@ class LlamaBlock(torch.nn.Module):
         # h2 = hidden + a fused into the post-attention norm
         h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
         # residual add fused into the down-projection epilogue
-        return self._lin(ops.swiglu(self._lin(y, self.gate_up_w, "gate_up_w")),
-                         self.down_w, "down_w", residual=h2)
+        return self._lin(self._gated(y), self.down_w, "down_w", residual=h2)
 
     # ------------------------------------------------------------------
     # training path (differentiable; full sequence, no KV cache)

@@ -75,8 +75,7 @@ class Qwen3Block(LlamaBlock):
             return self._fused_tail(hidden, attn)
         a = self._lin(attn, self.o_w, "o_w")
         h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
-        return self._lin(ops.swiglu(self._lin(y, self.gate_up_w, "gate_up_w")),
-                         self.down_w, "down_w", residual=h2)
+        return self._lin(self._gated(y), self.down_w, "down_w", residual=h2)
 
     def forward_train(self, hidden: torch.Tensor, start_pos: int = 0) -> torch.Tensor:
         B, T, H = hidden.shape

@@ -19,6 +19,7 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     kv_write,
     layer_norm,
     linear,
+    linear_gated,
     linear_rope_kv,
     linear_swiglu,
     linear_w4,

@@ -91,7 +91,7 @@ DEVINL void copy16_to_lds(const unsigned short* g, unsigned char* l) {
   __builtin_amdgcn_global_load_lds((gptr_t)g, (lptr_t)l, 16, 0, 0);
 }
 
-DEVINL long ldiv_up(long a, long b) { return (a + b - 1) / b; }
+__host__ DEVINL long ldiv_up(long a, long b) { return (a + b - 1) / b; }
 
 #define HIP_OK(expr)                                                         \
   do {                                                                       \

@@ -18,6 +18,7 @@
 #include "attn_prefill.hip"
 #include "gemm_skinny.hip"
 #include "gemm_stream.hip"
+#include "gemm_rows.hip"
 #include "moe_gemm.hip"
 #include "moe_route.hip"
 #include "w4_gemm.hip"
@@ -1260,6 +1261,191 @@ torch::Tensor mfma_selftest(torch::Tensor A, torch::Tensor B) {
   return C;
 }
 
+// ---------------------------------------------------------------------------
+// products of some dozen rows to a thousand (gemm_rows.hip)
+// ---------------------------------------------------------------------------
+
+// A tile, what a round of its workgroups costs beside its stages and what a stage of 64
+// columns costs, us: fitted to 288 products, 33 to 2000 rows (a round is 256 workgroups).
+#define ROWS_TILES(X)                                                                 \
+  X(0, 256, 256, 2, 2, 1, 2, 1, 7.3f, 1.136f) X(1, 160, 256, 2, 2, 1, 3, 1, 5.2f, .752f) \
+  X(2, 192, 224, 2, 2, 1, 3, 1, 6.0f, .776f) X(3, 256, 160, 2, 2, 1, 3, 1, 6.4f, .757f) \
+  X(4, 256, 128, 2, 2, 1, 3, 1, 4.9f, .663f) X(5, 192, 128, 2, 2, 1, 3, 1, 3.7f, .565f) \
+  X(6, 128, 128, 2, 2, 1, 4, 1, 2.4f, .462f) X(7, 96, 128, 2, 2, 1, 4, 1, 2.2f, .378f) \
+  X(8, 64, 128, 2, 2, 1, 3, 2, 1.1f, .340f) X(9, 96, 64, 2, 1, 2, 3, 1, 2.4f, .265f)
+
+struct RowsPlan {
+  int tile = -1, splits = 1;
+  float us = INFINITY;
+};
+
+// The tile and the splits of K that take least by the figures above: small results are
+// split so that all CUs take part, which a fold pays for. Over those products the choice
+// takes 2.4% more than the best of 19 tiles and up to 16 splits.
+static RowsPlan rows_plan(long M, long N, long K, bool swiglu) {
+  static const struct { int bm, bn, wk; float round, stage; } tiles[] = {
+#define X(i, bm, bn, wm, wn, wk, st, mw, round, stage) {bm, bn, wk, round, stage},
+      ROWS_TILES(X)
+#undef X
+  };
+  RowsPlan best;
+  for (int i = 0; i < 10; ++i) {
+    const auto& t = tiles[i];
+    if (K % (64 * t.wk) || (swiglu && t.wk > 1)) continue;
+    const long wgs = ldiv_up(M, t.bm) * ldiv_up(N, t.bn), all = K / (64 * t.wk);
+    for (int s = 1; s <= (swiglu ? 1 : 16); ++s) {
+      if (s > 1 && (wgs * s > 300 || all / s < 6)) break;
+      const float us = ldiv_up(wgs * s, 256) * (t.round + ldiv_up(all, s) * t.wk * t.stage) +
+                       (s > 1 ? 3.f + s * (M * N) * 1.6e-6f : 0.f);
+      if (us < best.us) best = {i, s, us};
+    }
+  }
+  best.us += (N + M) * K / 9.8e6f;   // memory, a quarter of it not hidden
+  return best;
+}
+
+// Whether these are the faster form. The library's kernels are at 1.1 to 1.6 PF where
+// their tiles fill the chip, which takes many rows or columns; below, and where K is
+// long, they leave CUs idle. us, library and these, N x K:
+//   28672 x 4096: 97 rows 55, 55; 333 76, 72; 450 89, 101; 1000 172, 189
+//   4096 x 14336: 97 46, 29; 333 74, 52; 617 109, 73; 1400 150, 139; 2000 184, 185
+//   6144 x 4096: 97 23, 18; 333 34, 29; 512 35, 36; 768 46, 41; 2000 78, 93
+//   4096 x 4096: 97 21, 14; 333 23, 21; 617 33, 29; 768 32, 33; 1400 46, 43
+//   8192 x 28672: 97 195, 98; 450 301, 210; 617 248, 269; 57344 x 8192: 200 194, 242
+//   1024 x 3072: any 20 (the host's time), 9 to 19
+static bool rows_wins(long M, long N, long K) {
+  if (M <= 32 || N % 8 || K % 64 || K < 256) return false;
+  return M * N <= (M <= 384 ? 11200000 : 6000000) && (K <= 16384 || M <= 512);
+}
+
+// The same for the gated product in one launch: the other way goes over the projection
+// once more. 28672 x 4096: 333 rows 73 us (72 + 7), 617 127 (126 + 10).
+static bool rows_swiglu_wins(long M, long N, long K) {
+  if (M <= 32 || M > 1024 || N % 16 || K % 64 || K < 256) return false;
+  const double library = std::max(2e-6 * M * N * K / 1.2e3, (N + M) * K * 2 / 4.7e6);
+  return rows_plan(M, N, K, true).us * 1.07 < library + M * N * 3 / 5e6 + 3;
+}
+
+template <typename F>
+static void rows_tile(int tile, F f) {
+  switch (tile) {
+#define X(i, bm, bn, wm, wn, wk, st, mw, round, stage) \
+  case i:                                              \
+    f(RowsTile<bm, bn, wm, wn, wk, st, mw>{});         \
+    break;
+    ROWS_TILES(X)
+#undef X
+    default:
+      TORCH_CHECK(false, "no tile");
+  }
+}
+
+template <typename K>
+static void rows_launch(K kernel, long grid, int threads, int lds, const RowsArgs& a) {
+  HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  kernel<<<grid, threads, lds, cur_stream()>>>(a);
+  HIP_OK(hipGetLastError());
+}
+
+// Both operands come by 16-byte copies: a view that does not begin at 16 bytes is copied
+// first.
+static RowsArgs rows_args(torch::Tensor& A, torch::Tensor& W) {
+  CHECK_DEV(A); CHECK_BF16(A); CHECK_CONTIG(A);
+  CHECK_DEV(W); CHECK_BF16(W); CHECK_CONTIG(W);
+  if ((size_t)A.data_ptr() % 16) A = A.clone();
+  if ((size_t)W.data_ptr() % 16) W = W.clone();
+  RowsArgs a{};
+  const long K = A.size(-1);
+  TORCH_CHECK(W.dim() == 2 && W.size(1) == K && K > 0 && K % 64 == 0 && K < 1 << 20,
+              "A/W K mismatch");
+  TORCH_CHECK(A.numel() / K < 1 << 24 && W.size(0) < 1 << 24 && W.size(0) > 0);
+  a.M = A.numel() / K;
+  a.N = W.size(0);
+  a.K = K;
+  a.splits = 1;
+  a.A = bf_ptr(A);
+  a.W = bf_ptr(W);
+  return a;
+}
+
+static void rows_product(RowsArgs& a, const RowsPlan& plan) {
+  rows_tile(plan.tile, [&](auto tile) {
+    typedef decltype(tile) T;
+    rows_launch(gemm_rows_kernel<T>,
+                ldiv_up(a.M, T::BM) * ldiv_up(a.N, T::BN) * a.splits, T::THREADS, T::LDS,
+                a);
+  });
+}
+
+// C(M,N) = A @ W^T [+ bias] [+ residual].
+torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
+                        c10::optional<torch::Tensor> residual,
+                        c10::optional<torch::Tensor> bias) {
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(a.N % 8 == 0, "N % 8 != 0");
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N;
+  auto C = torch::empty(sizes, A.options());
+  auto operand = [&](c10::optional<torch::Tensor>& t, long n) -> const unsigned short* {
+    if (!t.has_value()) return nullptr;
+    CHECK_DEV((*t)); CHECK_BF16((*t)); CHECK_CONTIG((*t));
+    TORCH_CHECK(t->numel() == n, "size of residual or bias");
+    if ((size_t)t->data_ptr() % 16) t = t->clone();
+    return bf_ptr(*t);
+  };
+  a.R = operand(residual, (long)a.M * a.N);
+  a.bias = operand(bias, a.N);
+  if (a.M == 0) return C;
+  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
+  a.splits = plan.splits;
+  a.C = plan.splits > 1 ? nullptr : bf_ptr_mut(C);
+  torch::Tensor part;
+  if (plan.splits > 1) {
+    part = torch::empty({plan.splits, a.M, a.N}, A.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+  }
+  rows_product(a, plan);
+  if (plan.splits > 1) {
+    a.C = bf_ptr_mut(C);
+    gemm_rows_fold_kernel<<<ldiv_up((long)a.M * a.N, 2048), 256, 0, cur_stream()>>>(a);
+    HIP_OK(hipGetLastError());
+  }
+  return C;
+}
+
+// A (M, K) @ W^T as (splits, M, N): f32 sums of splits, or one part in bf16.
+torch::Tensor gemm_rows_parts(torch::Tensor A, torch::Tensor W) {
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(A.dim() == 2 && a.N % 8 == 0 && a.M > 0, "A (M, K), N % 8 == 0");
+  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
+  a.splits = plan.splits;
+  auto C = torch::empty({plan.splits, a.M, a.N},
+                        A.options().dtype(plan.splits > 1 ? at::kFloat : at::kBFloat16));
+  if (plan.splits > 1) a.part = C.data_ptr<float>();
+  else a.C = bf_ptr_mut(C);
+  rows_product(a, plan);
+  return C;
+}
+
+// swiglu(A @ W^T) of a fused [gate | up] W: (..., N / 2).
+torch::Tensor gemm_rows_swiglu(torch::Tensor A, torch::Tensor W) {
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(a.N % 16 == 0, "N % 16 != 0");
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N / 2;
+  auto C = torch::empty(sizes, A.options());
+  if (a.M == 0) return C;
+  a.C = bf_ptr_mut(C);
+  rows_tile(rows_plan(a.M, a.N, a.K, true).tile, [&](auto tile) {
+    typedef decltype(tile) T;
+    if constexpr (T::WK == 1)
+      rows_launch(gemm_rows_swiglu_kernel<T>,
+                  ldiv_up(a.M, T::BM) * ldiv_up(a.N / 2, T::BN / 2), T::THREADS, T::LDS, a);
+  });
+  return C;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm);
   m.def("rms_norm_residual", &rms_norm_residual);
@@ -1281,6 +1467,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_route", &norm_route);
   m.def("add_experts", &add_experts);
   m.def("gemm_stream", &gemm_stream);
+  m.def("rows_wins", &rows_wins);
+  m.def("rows_swiglu_wins", &rows_swiglu_wins);
+  m.def("rows_plan", [](long M, long N, long K, bool swiglu) {
+    const RowsPlan p = rows_plan(M, N, K, swiglu);
+    return py::make_tuple(p.tile, p.splits);
+  });
+  m.def("gemm_rows", &gemm_rows);
+  m.def("gemm_rows_parts", &gemm_rows_parts);
+  m.def("gemm_rows_swiglu", &gemm_rows_swiglu);
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);
   m.def("stream_rows", &stream_rows);

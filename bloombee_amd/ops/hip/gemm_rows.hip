@@ -234,10 +234,10 @@ struct RowsTile {
     return __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) / (WK * WN) * MI * 16;
   }
 
-  // Sixteen rows at a time, of `strips` strips of 16 columns, through LDS, so that
-  // whole lines are written: value(n) gives a lane's four of strip n, as f32 or bf16;
-  // put(row, column, eight values as they were).
-  template <int STRIPS, typename V, typename P>
+  // Sixteen rows at a time, of STRIPS strips of 16 columns (the first PIECES * 8 of
+  // them), through LDS, so that whole lines are written: value(n) gives a lane's four of
+  // strip n, as f32 or bf16; put(row, column, eight values as they were).
+  template <int STRIPS, int PIECES = STRIPS * 2, typename V, typename P>
   static DEVINL void out16(unsigned char* lds, V value, P put) {
     typedef decltype(value(0)) T4;
     constexpr int E = sizeof(T4) / 4, RS = STRIPS * 16 * E + 16;
@@ -249,11 +249,181 @@ struct RowsTile {
       *reinterpret_cast<T4*>(mine + li * RS + (n * 16 + hi * 4) * E) = value(n);
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int i = 0; i < (STRIPS + 1) / 2; ++i) {
-      const int at = i * 64 + lane, r = at / (STRIPS * 2), c = at % (STRIPS * 2) * 8;
-      if (STRIPS % 2 && r >= 16) break;
+    for (int i = 0; i < (PIECES + 3) / 4; ++i) {
+      const int at = i * 64 + lane, r = at / PIECES, c = at % PIECES * 8;
+      if (PIECES % 4 && r >= 16) break;
       struct alignas(16) T8 { T4 lo, hi; };
       put(r, c, *reinterpret_cast<const T8*>(mine + r * RS + c * E));
     }
   }
 };
+
+struct RowsArgs {
+  const unsigned short* A;     // (M, K)
+  const unsigned short* W;     // (N, K)
+  const unsigned short* R;     // (M, N) residual or null
+  const unsigned short* bias;  // (N,) or null
+  unsigned short* C;           // (M, N), or null:
+  float* part;                 // (splits, M, N)
+  int M, N, K, splits;
+};
+
+// The chip's order of tiles: the row tiles of a column tile side by side on one XCD, which
+// share W there.
+template <typename T>
+DEVINL void rows_place(int M, int n_tiles, int& m0, int& nt, int& split) {
+  const int mt = (M + T::BM - 1) / T::BM;
+  const int n = gridDim.x, q = n / 8, r = n % 8, x = blockIdx.x % 8;
+  const int id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + blockIdx.x / 8;
+  m0 = id % mt * T::BM;
+  nt = id / mt % n_tiles;
+  split = id / mt / n_tiles;
+}
+
+// grid: row tiles * column tiles * splits; K % BK == 0, N % 8 == 0
+template <typename T>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_kernel(RowsArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  int m0, nt, split;
+  rows_place<T>(a.M, (a.N + T::BN - 1) / T::BN, m0, nt, split);
+  const int n0 = nt * T::BN;
+  const int all = a.K / T::BK, per = (all + a.splits - 1) / a.splits;
+  const int first = split * per;
+
+  unsigned ofs[T::LPW];
+#pragma unroll
+  for (int j = 0; j < T::LPW; ++j) {
+    const int r = T::load_row(j, wave, lane);
+    const int row = j < T::AJ ? min(r, a.M - 1 - m0) : min(r, a.N - 1 - n0);
+    ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
+  }
+  typename T::Acc acc;
+  T::run(ofs, a.A + (long)m0 * a.K + (long)first * T::BK,
+         a.W + (long)n0 * a.K + (long)first * T::BK, min(all, first + per) - first, lds,
+         acc, [](int) { return 0L; });
+
+  const int c0 = n0 + T::col0(), r0 = m0 + T::row0();
+  constexpr int S = T::COLS / 16;
+#pragma unroll
+  for (int m = 0; m < T::MI; ++m) {
+    const int row0 = r0 + m * 16;
+    if (!a.C) {
+      float* part = a.part + ((long)split * a.M + row0) * a.N + c0;
+      T::template out16<S>(lds, [&](int n) { return acc[m][n]; },
+                           [&](int r, int c, auto v) {
+        if (row0 + r >= a.M || c0 + c >= a.N) return;
+        *reinterpret_cast<f32x4*>(part + (long)r * a.N + c) = v.lo;
+        *reinterpret_cast<f32x4*>(part + (long)r * a.N + c + 4) = v.hi;
+      });
+    } else if (a.R || a.bias) {
+      T::template out16<S>(lds, [&](int n) { return acc[m][n]; },
+                           [&](int r, int c, auto v) {
+        if (row0 + r >= a.M || c0 + c >= a.N) return;
+        const long at = (long)(row0 + r) * a.N + c0 + c;
+        float y[8], x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = e < 4 ? v.lo[e & 3] : v.hi[e & 3];
+        if (a.bias) {
+          load_bf16x8(a.bias + c0 + c, x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] += x[e];
+        }
+        if (a.R) {
+          load_bf16x8(a.R + at, x);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) y[e] += x[e];
+        }
+        store_bf16x8(a.C + at, y);
+      });
+    } else {
+      T::template out16<S>(lds, [&](int n) { return pack4(acc[m][n]); },
+                           [&](int r, int c, auto v) {
+        if (row0 + r < a.M && c0 + c < a.N)
+          *reinterpret_cast<decltype(v)*>(a.C + (long)(row0 + r) * a.N + c0 + c) = v;
+      });
+    }
+  }
+}
+
+// silu(gate) * up of a fused [gate | up] W, C (M, N / 2), unsplit. A strip of 16 rows of
+// the tile is eight gates and their eight ups: half of a lane's sums change places with
+// those of the lane 32 on, and every lane has both.
+// grid: row tiles * tiles of BN / 2 activations; N % 16 == 0
+template <typename T>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_swiglu_kernel(RowsArgs a) {
+  static_assert(T::WK == 1 && T::RPC == 8, "eight rows a load");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int F = a.N / 2;
+  int m0, nt, split;
+  rows_place<T>(a.M, (F + T::BN / 2 - 1) / (T::BN / 2), m0, nt, split);
+  const int n0 = nt * (T::BN / 2);
+
+  unsigned ofs[T::LPW];
+#pragma unroll
+  for (int j = 0; j < T::LPW; ++j) {
+    const int r = T::load_row(j, wave, lane);
+    const int row = j < T::AJ ? min(r, a.M - 1 - m0)
+                              : min(r / 16 * 8 + r % 8, F - 1 - n0);
+    ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
+  }
+  typename T::Acc acc;
+  T::run(ofs, a.A + (long)m0 * a.K, a.W + (long)n0 * a.K, a.K / T::BK, lds, acc,
+         [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * F * a.K; });
+
+  const int c0 = n0 + T::col0() / 2, r0 = m0 + T::row0();
+  constexpr int S = (T::NI + 1) / 2;
+#pragma unroll
+  for (int m = 0; m < T::MI; ++m) {
+    const int row0 = r0 + m * 16;
+    T::template out16<S, T::NI>(lds, [&](int n) {
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = acc[m][2 * n][e];
+        const float y = 2 * n + 1 < T::NI ? acc[m][2 * n + 1 < T::NI ? 2 * n + 1 : 0][e] : 0.f;
+        const auto s = __builtin_amdgcn_permlane32_swap(
+            __builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y), false, false);
+        const float g = __builtin_bit_cast(float, (unsigned)s[0]);
+        v[e] = g / (1.f + fast_expf(-g)) * __builtin_bit_cast(float, (unsigned)s[1]);
+      }
+      return pack4(v);
+    }, [&](int r, int c, auto v) {
+      if (row0 + r < a.M && c0 + c < F)
+        *reinterpret_cast<decltype(v)*>(a.C + (long)(row0 + r) * F + c0 + c) = v;
+    });
+  }
+}
+
+// Folds the splits, eight columns a thread; grid M * N / 8 / 256.
+__global__ __launch_bounds__(256) void gemm_rows_fold_kernel(RowsArgs a) {
+  const long n = (long)a.M * a.N;
+  const long at = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (at >= n) return;
+  float v[8] = {};
+#pragma unroll 4
+  for (int s = 0; s < a.splits; ++s) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(a.part + s * n + at);
+    const f32x4 y = *reinterpret_cast<const f32x4*>(a.part + s * n + at + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] += x[j];
+      v[j + 4] += y[j];
+    }
+  }
+  float x[8];
+  if (a.bias) {
+    load_bf16x8(a.bias + at % a.N, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += x[j];
+  }
+  if (a.R) {
+    load_bf16x8(a.R + at, x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += x[j];
+  }
+  store_bf16x8(a.C + at, v);
+}

@@ -13,6 +13,7 @@ import os
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 from bloombee_amd.ops import reference as ref
 from bloombee_amd.ops.reference import alibi_slopes as alibi_slopes_for  # noqa: F401
@@ -41,6 +42,40 @@ def _require_ext():
 
 def _on_gpu(t: torch.Tensor) -> bool:
     return t.is_cuda
+
+
+def _plain(t: torch.Tensor) -> bool:
+    """A tensor that a kernel can read, not a wrapper around some."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter)
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and not torch._C._functorch.is_legacy_batchedtensor(t))
+
+
+def _no_function_mode() -> bool:
+    """No mode sees torch's functions but that of a default device, which places
+    what factories make."""
+    return (torch._C._len_torch_function_stack() == 0
+            or all(type(m) is DeviceContext
+                   for m in torch.overrides._get_current_function_mode_stack()))
+
+
+def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """The kernels take these: weights are frozen. They are launched on the current
+    device's stream: tensors of another device are left to torch, which switches."""
+    return (x.is_cuda and x.numel() > 0
+            and x.device.index == torch.cuda.current_device()
+            and all(t.dtype == torch.bfloat16 and _plain(t)
+                    for t in (x, *weights))
+            and all(w.device == x.device and not w.requires_grad
+                    for w in weights)
+            and not torch.is_autocast_enabled("cuda")
+            and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and _no_function_mode()
+            and torch._C._functorch.peek_interpreter_stack() is None
+            and all(torch.autograd.forward_ad.unpack_dual(t).tangent is None
+                    for t in (x, *weights)))
 
 
 # ---------------------------------------------------------------------------
@@ -304,7 +339,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
     """y = (rmsnorm(x) if norm else x) @ w^T (+bias) (+residual).
     Decode-shaped GEMMs (<=32 rows) on GPU go through the weight-streaming MFMA
     kernels (gemm_stream.hip, gemm_skinny.hip) — hipBLASLt leaves ~2x weight-stream
-    bandwidth on the table at M<=32; everything else uses hipBLASLt via F.linear.
+    bandwidth on the table at M<=32; up to some hundred rows, or a thousand of few
+    columns, where it leaves CUs idle, through the tiles of gemm_rows.hip; everything
+    else uses hipBLASLt via F.linear.
     norm=(weight, eps): the input's rmsnorm is taken along; weight None: it is folded
     into w. ss_in (f32, (stripes, 32)) are sums of squares of x's rows, the ss_out of
     the product that made x, and spare a pass over x; ss_out (f32, (N/64, 32)) takes
@@ -345,6 +382,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
         if nw is None:
             nw = torch.ones(x.shape[-1], dtype=x.dtype, device=x.device)
         x = rms_norm(x, nw, norm[1])
+    if ss_out is None and rows_ok(x, w) and all(
+            t is None or (t.dtype == torch.bfloat16 and t.device == x.device
+                          and not t.requires_grad and _plain(t) and t.numel() == n)
+            for t, n in ((bias, N), (residual, M * N))):
+        return hip_ops.gemm_rows(
+            x.contiguous(), w,
+            None if residual is None else residual.contiguous(),
+            None if bias is None else bias.contiguous())
     y = torch.nn.functional.linear(x, w, bias)
     if residual is not None:
         y = y + residual.view_as(y)
@@ -352,6 +397,28 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
         raise RuntimeError("ss_out requires the GPU skinny-GEMM path "
                            "(callers gate on fuse_norm_linear_ok)")
     return y
+
+
+def _rows_take(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """gemm_rows.hip reads these, and nobody records or watches the product."""
+    return (HAVE_HIP_OPS and x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+            and w.dim() == 2 and x.dim() >= 2 and x.shape[-1] == w.shape[1]
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and _fused(x, w))
+
+
+def rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """x @ w^T of tensors without gradients is faster on the tiles of gemm_rows.hip."""
+    return (_rows_take(x, w) and not (x.requires_grad and torch.is_grad_enabled())
+            and hip_ops.rows_wins(x.numel() // x.shape[-1], *w.shape))
+
+
+def linear_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """swiglu(x @ w^T) of a fused [gate | up] projection, in one launch where that is
+    the faster form; gate and up are then not rounded ahead of the product."""
+    if (_rows_take(x, w) and not (x.requires_grad and torch.is_grad_enabled())
+            and hip_ops.rows_swiglu_wins(x.numel() // x.shape[-1], *w.shape)):
+        return hip_ops.gemm_rows_swiglu(x.contiguous(), w)
+    return swiglu(linear(x, w))
 
 
 _FUSE_NORM = os.environ.get("BBAMD_FUSE_NORM", "1") != "0"

@@ -32,6 +32,7 @@ from typing import Optional, Tuple
 import torch
 import torch.nn.functional as F
 
+from bloombee_amd.ops import interface
 from bloombee_amd.ops import reference as ref
 
 _hip_ragged = None   # loaded by the first device call
@@ -286,11 +287,17 @@ def embed_rows(ids: torch.Tensor, positions: torch.Tensor,
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x (M, K) @ w (N, K)^T as (splits, M, N): f32 partials of the split-K
-    weight-stream kernel for up to 32 bf16 rows, else one part in x's type
-    from the vendor GEMM."""
+    weight-stream kernel for up to 32 bf16 rows, else one part in x's type, from
+    the tiles of gemm_rows.hip or the vendor GEMM."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= SKINNY_ROWS):
         return _ext().gemm_parts(x, w, 0)
-    return F.linear(x, w).unsqueeze(0)
+    return _linear(x, w).unsqueeze(0)
+
+
+def _linear(x, w):
+    if interface.rows_ok(x, w):
+        return interface.hip_ops.gemm_rows(x.contiguous(), w, None, None)
+    return F.linear(x, w)
 
 
 def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -369,7 +376,7 @@ def input_projection(h: torch.Tensor, w: torch.Tensor, spec,
     if r < 0:
         return linear_parts(h, w), None, 0
     if not h.is_cuda or (h.dtype == torch.bfloat16 and h.shape[0] > SKINNY_ROWS):
-        return (F.linear(h, w[:r]).unsqueeze(0),
+        return (_linear(h, w[:r]).unsqueeze(0),
                 router_logits(h, w[r:], spec.router_n), 0)
     parts = linear_parts(h, w)      # f32 either way
     return parts, parts, r

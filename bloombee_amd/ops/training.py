@@ -16,9 +16,9 @@ from typing import Tuple
 
 import torch
 import torch.nn.functional as F
-from torch.utils._device import DeviceContext
 
 from bloombee_amd.ops import interface
+from bloombee_amd.ops.interface import _fused, _plain
 
 _module = None
 
@@ -35,40 +35,6 @@ def _ext():
                 "Run `python setup.py hip` (PYTORCH_ROCM_ARCH=gfx950). "
                 f"Import error was: {e}") from e
     return _module
-
-
-def _plain(t: torch.Tensor) -> bool:
-    """A tensor that a kernel can read, not a wrapper around some."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter)
-            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and not torch._C._functorch.is_legacy_batchedtensor(t))
-
-
-def _no_function_mode() -> bool:
-    """No mode sees torch's functions but that of a default device, which places
-    what factories make."""
-    return (torch._C._len_torch_function_stack() == 0
-            or all(type(m) is DeviceContext
-                   for m in torch.overrides._get_current_function_mode_stack()))
-
-
-def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
-    """The kernels take these: weights are frozen. They are launched on the current
-    device's stream: tensors of another device are left to torch, which switches."""
-    return (x.is_cuda and x.numel() > 0
-            and x.device.index == torch.cuda.current_device()
-            and all(t.dtype == torch.bfloat16 and _plain(t)
-                    for t in (x, *weights))
-            and all(w.device == x.device and not w.requires_grad
-                    for w in weights)
-            and not torch.is_autocast_enabled("cuda")
-            and not torch.jit.is_tracing()
-            and not torch.compiler.is_compiling()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and _no_function_mode()
-            and torch._C._functorch.peek_interpreter_stack() is None
-            and all(torch.autograd.forward_ad.unpack_dual(t).tangent is None
-                    for t in (x, *weights)))
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -287,7 +253,7 @@ class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w):
         ctx.save_for_backward(w)
-        return F.linear(x, w)
+        return interface.linear(x, w)
 
     @staticmethod
     def backward(ctx, g):
@@ -301,13 +267,30 @@ class _Linear(torch.autograd.Function):
         return dx.view(*g.shape[:-1], w.shape[1]), None
 
 
+class _Product(torch.autograd.Function):
+    """Where only the product itself is faster than the library's."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(w)
+        return interface.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, g):
+        w, = ctx.saved_tensors
+        return g.matmul(w), None
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T; w is frozen where the gradient kernel is to take part."""
     if (torch.is_grad_enabled() and x.requires_grad and _fused(x, w)
             and w.dim() == 2 and x.dim() >= 2 and x.shape[-1] == w.shape[1]
-            and w.is_contiguous()
-            and _few_rows(x.numel() // x.shape[-1], *w.shape)):
-        return _Linear.apply(x, w)
+            and w.is_contiguous()):
+        M = x.numel() // x.shape[-1]
+        if _few_rows(M, *w.shape):
+            return _Linear.apply(x, w)
+        if interface.hip_ops.rows_wins(M, *w.shape) and w.data_ptr() % 16 == 0:
+            return _Product.apply(x, w)
     return F.linear(x, w)
 
 

@@ -1,0 +1,125 @@
+"""Products of some dozen rows to a thousand on the tiles of gemm_rows.hip."""
+import pytest
+import torch
+
+from bloombee_amd import ops
+from bloombee_amd.ops import training
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def draw(*shape, seed, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).bfloat16()
+
+
+def close(got, want, terms):
+    """The result's rounding, 2^-9, and 32-bit sums of `terms` (the sum of the
+    products' magnitudes) in any order."""
+    return bool(((got.double() - want).abs()
+                 <= 2.0 ** -8 * want.abs() + 2.0 ** -20 * terms + 1e-30).all())
+
+
+# (rows, columns, K): every tile, unsplit and split; one row, strip or column short of a
+# tile or past it; fewer steps than buffers, as many, more
+SIZES = [(33, 8, 256), (65, 136, 320), (97, 248, 448), (129, 4096, 1024),
+         (192, 1032, 704), (193, 28672, 256), (200, 6144, 1088), (256, 10240, 512),
+         (333, 4096, 4096), (450, 4096, 5120), (512, 8192, 1536), (617, 6208, 576),
+         (768, 6144, 1536), (1000, 1024, 3072), (1025, 4104, 448), (1400, 4096, 1024),
+         (193, 42568, 256), (138, 33360, 256), (167, 33064, 320), (203, 32960, 256),
+         (333, 28672, 512), (1891, 8, 7168), (1650, 8, 7104), (300, 33000, 704)]
+
+
+GATED = [(33, 8, 256), (97, 1000, 320), (200, 14336, 256), (333, 14336, 448),
+         (450, 56, 4096), (617, 4096, 384), (1000, 8192, 512), (64, 120, 576),
+         (164, 29456, 256), (155, 17032, 256), (171, 19000, 256), (222, 16880, 256),
+         (226, 13024, 256), (131, 11224, 256), (109, 8312, 256), (65, 8912, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_product(M, N, K):
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    r, b = draw(M, N, seed=3), draw(N, seed=4)
+    assert ops.hip_ops.rows_wins(M, N, K)
+    want = x.double() @ w.double().T
+    terms = x.double().abs() @ w.double().abs().T
+    assert close(ops.linear(x, w), want, terms)
+    more = want + r.double() + b.double()
+    assert close(ops.linear(x, w, residual=r, bias=b), more,
+                 terms + r.double().abs() + b.double().abs())
+    parts = ops.hip_ops.gemm_rows_parts(x, w)
+    assert close(parts.float().sum(0), want, terms)
+
+
+def test_tiles_are_reached():
+    plans = {ops.hip_ops.rows_plan(M, N, K, False) for M, N, K in SIZES}
+    assert {t for t, _ in plans} == set(range(10)) and len({s for _, s in plans}) >= 3
+    plans = {ops.hip_ops.rows_plan(M, 2 * F, K, True) for M, F, K in GATED}
+    assert plans == {(t, 1) for t in range(9)}
+
+
+@pytest.mark.parametrize("M,F,K", GATED)
+def test_gated(M, F, K):
+    x, w = draw(M, K, seed=1), draw(2 * F, K, seed=2, scale=K ** -0.5)
+    g, u = (x.double() @ w.double().T).chunk(2, -1)
+    want = torch.nn.functional.silu(g) * u
+    got = ops.hip_ops.gemm_rows_swiglu(x, w)
+    # sums of 32 bits within 2^-20 of their terms, hardware exponential and reciprocal
+    tol = (x.double().abs() @ w.double().abs().T).chunk(2, -1)
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -19 * (tol[0] * u.abs() + tol[1] * g.abs()) + 1e-30).all())
+    y = ops.linear_gated(x, w)
+    # where it is two steps, gate and up are rounded, 2^-9 of each
+    assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -8 * (g.abs() + 1) * u.abs() + 1e-6).all())
+
+
+def test_not_finite():
+    """Infinities and NaN stay in their rows and columns."""
+    M, N, K = 100, 640, 512
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2)
+    x[7, 3], x[99, 511], w[5, 0] = float("inf"), float("nan"), float("-inf")
+    want = x.float() @ w.float().T
+    got = ops.linear(x, w).float()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+    some = want.isfinite()
+    assert torch.allclose(got[some], want[some], rtol=2.0 ** -7, atol=1e-3)
+
+
+def test_views():
+    """Rows at any address and of any stride, weights that do not begin at 16 bytes."""
+    M, N, K = 64, 256, 320
+    flat = draw(M * K + 1, seed=1)
+    w = draw(N, K, seed=2)
+    for x in (flat[1:].view(M, K), draw(M, 2 * K, seed=3)[:, :K],
+              draw(K, M, seed=4).T, draw(2, M // 2, K, seed=5)):
+        want = x.double() @ w.double().T
+        terms = x.double().abs() @ w.double().abs().T
+        assert close(ops.linear(x, w), want, terms)
+    odd = draw(N * K + 1, seed=6)[1:].view(N, K)
+    x = draw(M, K, seed=7)
+    assert close(ops.linear(x, odd), x.double() @ odd.double().T,
+                 x.double().abs() @ odd.double().abs().T)
+
+
+def test_recorded_and_replayed():
+    """Gradients reach x through linear; a captured product gives the eager one's bits
+    on every replay."""
+    M, N, K = 100, 1024, 1024
+    x, w = draw(M, K, seed=1).requires_grad_(True), draw(N, K, seed=2)
+    g = draw(M, N, seed=3)
+    for f in (ops.linear, training.linear):
+        dx, = torch.autograd.grad(f(x, w), x, g)
+        assert close(dx, g.double() @ w.double(), g.double().abs() @ w.double().abs())
+    at = x.detach().clone()
+    ops.linear(at, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.linear(at, w)
+    for seed in (4, 5, 6):
+        at.copy_(draw(M, K, seed=seed))
+        graph.replay()
+        assert torch.equal(out, ops.linear(at, w))
