@@ -18,7 +18,7 @@
 #include "attn_prefill.hip"
 #include "gemm_skinny.hip"
 #include "gemm_stream.hip"
-#include "gemm_rows.hip"
+#include "gemm_rows_host.h"
 #include "moe_gemm.hip"
 #include "moe_route.hip"
 #include "w4_gemm.hip"
@@ -1274,34 +1274,13 @@ torch::Tensor mfma_selftest(torch::Tensor A, torch::Tensor B) {
   X(6, 128, 128, 2, 2, 1, 4, 1, 2.4f, .462f) X(7, 96, 128, 2, 2, 1, 4, 1, 2.2f, .378f) \
   X(8, 64, 128, 2, 2, 1, 3, 2, 1.1f, .340f) X(9, 96, 64, 2, 1, 2, 3, 1, 2.4f, .265f)
 
-struct RowsPlan {
-  int tile = -1, splits = 1;
-  float us = INFINITY;
-};
-
-// The tile and the splits of K that take least by the figures above: small results are
-// split so that all CUs take part, which a fold pays for. Over those products the choice
-// takes 2.4% more than the best of 19 tiles and up to 16 splits.
 static RowsPlan rows_plan(long M, long N, long K, bool swiglu) {
-  static const struct { int bm, bn, wk; float round, stage; } tiles[] = {
+  static const RowsCost tiles[] = {
 #define X(i, bm, bn, wm, wn, wk, st, mw, round, stage) {bm, bn, wk, round, stage},
       ROWS_TILES(X)
 #undef X
   };
-  RowsPlan best;
-  for (int i = 0; i < 10; ++i) {
-    const auto& t = tiles[i];
-    if (K % (64 * t.wk) || (swiglu && t.wk > 1)) continue;
-    const long wgs = ldiv_up(M, t.bm) * ldiv_up(N, t.bn), all = K / (64 * t.wk);
-    for (int s = 1; s <= (swiglu ? 1 : 16); ++s) {
-      if (s > 1 && (wgs * s > 300 || all / s < 6)) break;
-      const float us = ldiv_up(wgs * s, 256) * (t.round + ldiv_up(all, s) * t.wk * t.stage) +
-                       (s > 1 ? 3.f + s * (M * N) * 1.6e-6f : 0.f);
-      if (us < best.us) best = {i, s, us};
-    }
-  }
-  best.us += (N + M) * K / 9.8e6f;   // memory, a quarter of it not hidden
-  return best;
+  return rows_best(tiles, 10, M, N, K, swiglu);
 }
 
 // Whether these are the faster form. The library's kernels are at 1.1 to 1.6 PF where
@@ -1340,14 +1319,6 @@ static void rows_tile(int tile, F f) {
   }
 }
 
-template <typename K>
-static void rows_launch(K kernel, long grid, int threads, int lds, const RowsArgs& a) {
-  HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  kernel<<<grid, threads, lds, cur_stream()>>>(a);
-  HIP_OK(hipGetLastError());
-}
-
 // Both operands come by 16-byte copies: a view that does not begin at 16 bytes is copied
 // first.
 static RowsArgs rows_args(torch::Tensor& A, torch::Tensor& W) {
@@ -1374,7 +1345,7 @@ static void rows_product(RowsArgs& a, const RowsPlan& plan) {
     typedef decltype(tile) T;
     rows_launch(gemm_rows_kernel<T>,
                 ldiv_up(a.M, T::BM) * ldiv_up(a.N, T::BN) * a.splits, T::THREADS, T::LDS,
-                a);
+                cur_stream(), a);
   });
 }
 
@@ -1441,7 +1412,8 @@ torch::Tensor gemm_rows_swiglu(torch::Tensor A, torch::Tensor W) {
     typedef decltype(tile) T;
     if constexpr (T::WK == 1)
       rows_launch(gemm_rows_swiglu_kernel<T>,
-                  ldiv_up(a.M, T::BM) * ldiv_up(a.N / 2, T::BN / 2), T::THREADS, T::LDS, a);
+                  ldiv_up(a.M, T::BM) * ldiv_up(a.N / 2, T::BN / 2), T::THREADS, T::LDS,
+                  cur_stream(), a);
   });
   return C;
 }

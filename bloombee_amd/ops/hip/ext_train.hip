@@ -6,6 +6,7 @@
 
 #include "attn_train.hip"
 #include "gemm_grad.hip"
+#include "gemm_rows_host.h"
 #include "train_rows.hip"
 
 using torch::Tensor;
@@ -179,6 +180,36 @@ Tensor swiglu_grad(Tensor gu, Tensor gm) {
   return dgu;
 }
 
+// Tiles of gemm_rows.hip whose sums run over rows of w, and what their rounds and stages
+// cost: fitted to 192 products, 33 to 2000 rows, where the choice takes 2.5% more than
+// the best of eleven tiles and up to 16 splits.
+#define GRAD_TILES(X)                                                                     \
+  X(0, 256, 256, 2, 2, 2, 1, 8.4f, 1.271f) X(1, 160, 256, 2, 2, 3, 1, 6.7f, .854f)         \
+  X(2, 128, 256, 2, 4, 3, 2, 3.3f, .664f) X(3, 192, 128, 2, 2, 3, 1, 5.1f, .587f)          \
+  X(4, 128, 128, 2, 2, 4, 1, 4.2f, .476f) X(5, 96, 128, 2, 2, 4, 1, 3.8f, .406f)           \
+  X(6, 64, 128, 2, 2, 3, 2, 2.6f, .340f)
+
+static RowsPlan grad_plan(long M, long N, long K) {
+  static const RowsCost tiles[] = {
+#define X(i, bm, bn, wm, wn, st, mw, round, stage) {bm, bn, 1, round, stage},
+      GRAD_TILES(X)
+#undef X
+  };
+  return rows_best(tiles, 7, M, K, N, false);
+}
+
+// Whether linear_grad beats the library's GEMM, which leaves CUs idle where the result
+// has few tiles. us, library and here, rows of w x columns:
+//   28672 x 4096: 33 rows 160, 45; 128 142, 52; 450 283, 112; 900 307, 195; 1400 302, 308
+//   4096 x 14336: 33 35, 25; 450 65, 56; 768 87, 88; 1700 163, 181
+//   6144 x 4096: 33 29, 14; 450 52, 37; 1400 72, 69; 2000 92, 83
+//   4096 x 4096: 450 38, 29; 2000 64, 57.  8192 x 28672: 333 159, 189; 900 382, 390
+//   57344 x 8192: 128 297, 170; 450 538, 402; 617 528, 535; 900 695, 738
+static bool linear_grad_wins(long M, long N, long K) {
+  return N % 64 == 0 && K % 256 == 0 && M * K <= 8500000 &&
+         (M <= 512 || M * K * N <= 150000000000L);
+}
+
 // g (M, N) @ w (N, K) -> (M, K); splits <= 0: as many as the sizes want.
 Tensor linear_grad(Tensor g, Tensor w, long splits) {
   CHECK_ROWS(g);
@@ -187,25 +218,56 @@ Tensor linear_grad(Tensor g, Tensor w, long splits) {
                   g.size(0) < (1L << 30) && w.size(0) % 32 == 0 &&
                   w.size(1) % 256 == 0 && w.numel() > 0 && w.numel() < (1L << 40),
               "need (M, N) @ (N, K), N % 32 == 0, K % 256 == 0");
+  const long M = g.size(0), N = w.size(0), K = w.size(1);
+  Tensor c = torch::empty({M, K}, g.options());
+  if (M == 0) return c;
+  Tensor part;
+  auto parts = [&](long n) {
+    part = torch::empty({n, M, K}, g.options().dtype(at::kFloat));
+    return part.data_ptr<float>();
+  };
+  // a stage's rows of w lie within 32 bits of bytes
+  if (N % 64 == 0 && K < (1L << 24) && N < (1L << 24)) {
+    RowsPlan plan = grad_plan(M, N, K);
+    if (splits > 0) plan.splits = (int)std::min<long>(splits, N / 64);
+    RowsArgs a{};
+    a.A = in(g);
+    a.W = in(w);
+    a.M = M;
+    a.N = K;
+    a.K = N;
+    a.splits = plan.splits;
+    if (a.splits > 1) a.part = parts(a.splits);
+    else a.C = out(c);
+    switch (plan.tile) {
+#define X(i, bm, bn, wm, wn, st, mw, round, stage)                                      \
+  case i: {                                                                             \
+    typedef RowsTile<bm, bn, wm, wn, 1, st, mw, true> T;                                \
+    rows_launch(gemm_rows_kernel<T>, ldiv_up(M, bm) * ldiv_up(K, bn) * a.splits,        \
+                T::THREADS, T::LDS, stream(), a);                                       \
+    break;                                                                              \
+  }
+      GRAD_TILES(X)
+#undef X
+    }
+    if (a.splits > 1) {
+      a.C = out(c);
+      gemm_rows_fold_kernel<<<ldiv_up(M * K, 2048), 256, 0, stream()>>>(a);
+      check_launch();
+    }
+    return c;
+  }
   GemmGradArgs a{};
   a.A = in(g);
   a.W = in(w);
-  a.M = g.size(0);
-  a.N = w.size(0);
-  a.K = w.size(1);
-  Tensor c = torch::empty({g.size(0), w.size(1)}, g.options());
-  if (a.M == 0) return c;
+  a.M = M;
+  a.N = N;
+  a.K = K;
   const long tiles = ((a.M + 127) / 128) * (a.K / 256);
   if (splits <= 0) splits = std::min<long>(32, 512 / std::max<long>(1, tiles));
   a.splits = (int)std::max<long>(1, std::min<long>(splits, a.N / 256));
-  Tensor part;
-  if (a.splits > 1) {
-    part = torch::empty({a.splits, g.size(0), w.size(1)},
-                        g.options().dtype(at::kFloat));
-    a.part = part.data_ptr<float>();
-  } else {
-    a.C = out(c);
-  }
+  if (a.splits > 1) a.part = parts(a.splits);
+  else a.C = out(c);
   gemm_grad_kernel<<<tiles * a.splits, 256, 0, stream()>>>(a);
   check_launch();
   if (a.splits > 1) {
@@ -218,6 +280,11 @@ Tensor linear_grad(Tensor g, Tensor w, long splits) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("linear_grad", &linear_grad);
+  m.def("linear_grad_wins", &linear_grad_wins);
+  m.def("linear_grad_plan", [](long M, long N, long K) {
+    const RowsPlan p = grad_plan(M, N, K);
+    return py::make_tuple(p.tile, p.splits);
+  });
   m.def("rope_attention", &rope_attention);
   m.def("rope_attention_grad", &rope_attention_grad);
   m.def("rms_norm_grad", &rms_norm_grad);

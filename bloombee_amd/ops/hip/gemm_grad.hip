@@ -2,14 +2,13 @@
 // projection has it: sums run over rows of W, whose fragments are read from LDS by
 // columns (transposing reads).
 //
-// Short texts leave few tiles of C, and the sum along N is long (28672 for a fused
-// [gate | up]): it is split over workgroups so that two run on every CU, each leaving
-// f32 sums that a second kernel folds. 28672 x 4096: 33 rows 53 us, 4.4 TB/s of weights
-// (the library's GEMM, unsplit: 164), 450 rows 156, 680 TF/s (279). Reads of LDS, of A
-// by all four waves, bound large ones, as they do the tiles of routed experts.
+// Rows of W that come in 64s take the tiles of gemm_rows.hip, TURNED (28672 x 4096: 33
+// rows 45 us, 450 112, where this takes 53 and 157); this is for the others, N % 32 == 0.
 //
 // A 128 x 256 tile a workgroup, 32 of N a step, two buffers filled by DMA; a wave holds
-// all rows of 64 columns.
+// all rows of 64 columns. The sum along N is split over workgroups so that two run on
+// every CU, each leaving f32 sums that a second kernel folds. Reads of LDS, of A by all
+// four waves, bound large ones.
 
 #pragma once
 #include "attn_train.hip"

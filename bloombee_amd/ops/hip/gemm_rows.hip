@@ -61,9 +61,13 @@ DEVINL f32x4 pick(bool c, f32x4 x, f32x4 y) {
 }
 
 // WM x WN waves, times WK groups that take 64 columns each of a stage; ST stages; MINW
-// waves a SIMD.
-template <int BM_, int BN_, int WM_, int WN_, int WK_, int ST_, int MINW_>
+// waves a SIMD. TURNED: sums run over rows of W instead, C(BM,BN) = A(BM,K) @ W(K,BN):
+// 64 rows of it are a stage, by 128 columns, 16 B piece c of row r at c ^ turn(r), and
+// fragments come by transposing reads.
+template <int BM_, int BN_, int WM_, int WN_, int WK_, int ST_, int MINW_,
+          bool TURNED_ = false>
 struct RowsTile {
+  static constexpr bool TURNED = TURNED_;
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, ST = ST_;
   static constexpr int MINW = MINW_;
   static constexpr int NW = WM * WN * WK, THREADS = NW * 64;
@@ -81,21 +85,29 @@ struct RowsTile {
 
   typedef f32x4 Acc[MI][NI];
 
+  static DEVINL int turn(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+
   // Row of the tile (of A for j < AJ, else of W) that load j of the thread is for, and
   // the byte in the row.
   static DEVINL int load_row(int j, int wave, int lane) {
-    return ((j < AJ ? j : j - AJ) * NW + wave) * RPC + lane / (RB / 16);
+    const int chunk = (j < AJ ? j : j - AJ) * NW + wave;
+    if (TURNED && j >= AJ) return chunk % 16 * 4 + lane / 16;
+    return chunk * RPC + lane / (RB / 16);
   }
   static DEVINL unsigned load_byte(int j, int wave, int lane) {
-    return ((lane % (RB / 16)) ^ (load_row(j, wave, lane) & 7)) * 16;
+    const int r = load_row(j, wave, lane);
+    if (TURNED && j >= AJ)
+      return ((j - AJ) * NW + wave) / 16 * 256 + ((lane % 16) ^ turn(r)) * 16;
+    return ((lane % (RB / 16)) ^ (r & 7)) * 16;
   }
 
   // Sums of `steps` stages. ofs: bytes from ap (j < AJ) or wp, which move on by a
-  // stage's columns; beyond(j): what the rows of a load lie behind wp, the wave's.
+  // stage's columns (wp by w_step); beyond(j): what the rows of a load lie behind wp, the
+  // wave's.
   template <typename B>
   static DEVINL void run(const unsigned (&ofs)[LPW], const unsigned short* ap,
                          const unsigned short* wp, int steps, unsigned char* lds,
-                         Acc& acc, B beyond) {
+                         Acc& acc, B beyond, long w_step = BK) {
     const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
@@ -121,10 +133,35 @@ struct RowsTile {
       fa[s] = (wm * MI * 16 + li) * RB + piece;
       fw[s] = BM * RB + (wn * NI * 16 + li) * RB + piece;
     }
+    unsigned turned[NI][2];
+    if constexpr (TURNED) {
+      static_assert(WK == 1 && BN % 128 == 0, "stages by 128 columns");
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int c = (wn * NI + i) * 16, r = hi * 8 + q * 4 + (li >> 2);
+          const int piece = c % 128 / 8 + ((li >> 1) & 1);
+          turned[i][q] = BM * RB + c / 128 * 16384 + r * 256 + ((piece ^ turn(r)) << 4) +
+                         (li & 1) * 8;
+        }
+    }
     bf16x8 af[2][MI], wf[2][NI];
     auto frag = [&](int i, int s, int buf) {
       const unsigned char* stage = lds + buf * STAGE;
-      if (i < NI)
+      if (TURNED && i < NI) {
+        // column li of rows s * 32 + hi * 8 .. +7
+        typedef __attribute__((address_space(3))) short4v lds4;
+        short8 v;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const short4v c = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds4*)(stage + turned[i][q] + s * 8192));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[q * 4 + e] = c[e];
+        }
+        wf[s][i] = as_bf16x8(v);
+      } else if (i < NI)
         wf[s][i] = as_bf16x8(
             *reinterpret_cast<const short8*>(stage + fw[s] + i * 16 * RB));
       else
@@ -173,7 +210,7 @@ struct RowsTile {
 #pragma unroll
         for (int j = 0; j < LPW; ++j) load(j, s);
         ap += BK;
-        wp += BK;
+        wp += w_step;
       }
     wait(min(ST, steps) - 1);
     barrier();
@@ -187,7 +224,7 @@ struct RowsTile {
       const int next = buf + 1 == ST ? 0 : buf + 1;
       phase(1, next, std::true_type{}, buf);
       ap += BK;
-      wp += BK;
+      wp += w_step;
       buf = next;
       if (MINW == 1) settle();
     }
@@ -260,7 +297,7 @@ struct RowsTile {
 
 struct RowsArgs {
   const unsigned short* A;     // (M, K)
-  const unsigned short* W;     // (N, K)
+  const unsigned short* W;     // (N, K); turned: (K, N)
   const unsigned short* R;     // (M, N) residual or null
   const unsigned short* bias;  // (N,) or null
   unsigned short* C;           // (M, N), or null:
@@ -296,13 +333,19 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_kernel(RowsArgs
 #pragma unroll
   for (int j = 0; j < T::LPW; ++j) {
     const int r = T::load_row(j, wave, lane);
-    const int row = j < T::AJ ? min(r, a.M - 1 - m0) : min(r, a.N - 1 - n0);
-    ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
+    const unsigned byte = T::load_byte(j, wave, lane);
+    if (T::TURNED && j >= T::AJ) {
+      ofs[j] = (unsigned)r * (unsigned)(a.N * 2) + min(byte, (a.N - n0) * 2 - 16u);
+    } else {
+      const int row = j < T::AJ ? min(r, a.M - 1 - m0) : min(r, a.N - 1 - n0);
+      ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + byte;
+    }
   }
   typename T::Acc acc;
+  const long w_step = T::TURNED ? 64L * a.N : T::BK;
   T::run(ofs, a.A + (long)m0 * a.K + (long)first * T::BK,
-         a.W + (long)n0 * a.K + (long)first * T::BK, min(all, first + per) - first, lds,
-         acc, [](int) { return 0L; });
+         a.W + (T::TURNED ? (long)n0 : (long)n0 * a.K) + first * w_step,
+         min(all, first + per) - first, lds, acc, [](int) { return 0L; }, w_step);
 
   const int c0 = n0 + T::col0(), r0 = m0 + T::row0();
   constexpr int S = T::COLS / 16;

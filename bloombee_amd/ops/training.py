@@ -233,9 +233,9 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
 # ---------------------------------------------------------------------------
 
 def _few_rows(M: int, N: int, K: int) -> bool:
-    """Whether a split sum along N beats the library's GEMM for the gradient,
-    (M, N) @ (N, K): that one leaves most of the chip idle where the result has
-    few tiles. us, split and library, N x K:
+    """Whether the split sum along N, (M, N) @ (N, K), beats the library's GEMM also
+    for N in 32s, which leaves most of the chip idle where the result has few tiles.
+    us, split and library, N x K:
     28672 x 4096: 33 rows 53, 164; 128 67, 145; 450 156, 279; 1024 296, 360;
         2000 554, 414
     20480 x 5120: 300 rows 127, 137; 900 277, 268 (160 tiles)
@@ -249,6 +249,10 @@ def _few_rows(M: int, N: int, K: int) -> bool:
             or M <= 1024 and N >= 4 * K and K <= 5120 and tiles <= 128)
 
 
+def _split_gradient(M: int, N: int, K: int) -> bool:
+    return _ext().linear_grad_wins(M, N, K) or _few_rows(M, N, K)
+
+
 class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w):
@@ -258,7 +262,8 @@ class _Linear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         w, = ctx.saved_tensors
-        if _again(g) or not _plain(w):
+        if (_again(g) or not _plain(w)
+                or not _split_gradient(g.numel() // g.shape[-1], *w.shape)):
             return g.matmul(w), None
         rows, w = g.reshape(-1, g.shape[-1]).contiguous(), w.contiguous()
         if rows.data_ptr() % 16 or w.data_ptr() % 16:
@@ -267,18 +272,8 @@ class _Linear(torch.autograd.Function):
         return dx.view(*g.shape[:-1], w.shape[1]), None
 
 
-class _Product(torch.autograd.Function):
-    """Where only the product itself is faster than the library's."""
-
-    @staticmethod
-    def forward(ctx, x, w):
-        ctx.save_for_backward(w)
-        return interface.linear(x, w)
-
-    @staticmethod
-    def backward(ctx, g):
-        w, = ctx.saved_tensors
-        return g.matmul(w), None
+class _Product(_Linear):
+    """The same beyond the sizes that _few_rows names."""
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -289,7 +284,8 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         M = x.numel() // x.shape[-1]
         if _few_rows(M, *w.shape):
             return _Linear.apply(x, w)
-        if interface.hip_ops.rows_wins(M, *w.shape) and w.data_ptr() % 16 == 0:
+        if (interface.hip_ops.rows_wins(M, *w.shape)
+                or _ext().linear_grad_wins(M, *w.shape)):
             return _Product.apply(x, w)
     return F.linear(x, w)
 

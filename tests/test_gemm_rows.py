@@ -75,6 +75,29 @@ def test_gated(M, F, K):
                  + 2.0 ** -8 * (g.abs() + 1) * u.abs() + 1e-6).all())
 
 
+# (rows, rows of w, columns): every tile, one row short of it or past it, fewer steps
+# than buffers and more
+GRADS = [(1, 64, 256), (63, 128, 512), (65, 448, 4096), (134, 128, 11520),
+         (202, 320, 11520), (284, 1728, 11520), (643, 64, 11264), (450, 4096, 14336),
+         (193, 15168, 11008), (450, 6144, 4096), (333, 28672, 1024), (1999, 4096, 4096)]
+
+
+@pytest.mark.parametrize("M,N,K", GRADS)
+@pytest.mark.parametrize("splits", [0, 1, 5])
+def test_gradient(M, N, K, splits):
+    g, w = draw(M, N, seed=1), draw(N, K, seed=2, scale=N ** -0.5)
+    got = training._ext().linear_grad(g, w, splits)
+    # in blocks: the magnitudes in 64 bits are large
+    for r in range(0, M, 500):
+        a = g[r:r + 500].double()
+        assert close(got[r:r + 500], a @ w.double(), a.abs() @ w.double().abs())
+
+
+def test_gradient_tiles_are_reached():
+    plans = {training._ext().linear_grad_plan(*s) for s in GRADS}
+    assert {t for t, _ in plans} == set(range(7)) and len({s for _, s in plans}) >= 3
+
+
 def test_not_finite():
     """Infinities and NaN stay in their rows and columns."""
     M, N, K = 100, 640, 512
