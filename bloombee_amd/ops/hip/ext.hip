@@ -1268,15 +1268,15 @@ torch::Tensor mfma_selftest(torch::Tensor A, torch::Tensor B) {
 // A tile, what a round of its workgroups costs beside its stages and what a stage of 64
 // columns costs, us: fitted to 288 products, 33 to 2000 rows (a round is 256 workgroups).
 #define ROWS_TILES(X)                                                                 \
-  X(0, 256, 256, 2, 2, 1, 2, 1, 7.3f, 1.136f) X(1, 160, 256, 2, 2, 1, 3, 1, 5.2f, .752f) \
-  X(2, 192, 224, 2, 2, 1, 3, 1, 6.0f, .776f) X(3, 256, 160, 2, 2, 1, 3, 1, 6.4f, .757f) \
-  X(4, 256, 128, 2, 2, 1, 3, 1, 4.9f, .663f) X(5, 192, 128, 2, 2, 1, 3, 1, 3.7f, .565f) \
-  X(6, 128, 128, 2, 2, 1, 4, 1, 2.4f, .462f) X(7, 96, 128, 2, 2, 1, 4, 1, 2.2f, .378f) \
-  X(8, 64, 128, 2, 2, 1, 3, 2, 1.1f, .340f) X(9, 96, 64, 2, 1, 2, 3, 1, 2.4f, .265f)
+  X(0, 256, 256, 2, 4, 1, 2, 2, 2, 6.0f, 1.08f) X(1, 160, 256, 2, 2, 1, 3, 1, 0, 5.2f, .752f) \
+  X(2, 192, 224, 2, 2, 1, 3, 1, 0, 6.0f, .776f) X(3, 256, 160, 2, 2, 1, 3, 1, 0, 6.4f, .757f) \
+  X(4, 256, 128, 2, 2, 1, 3, 1, 0, 4.9f, .663f) X(5, 192, 128, 2, 2, 1, 3, 1, 0, 3.7f, .565f) \
+  X(6, 128, 128, 2, 2, 1, 4, 1, 0, 2.4f, .462f) X(7, 96, 128, 2, 2, 1, 4, 1, 0, 2.2f, .378f) \
+  X(8, 64, 128, 2, 2, 1, 3, 2, 0, 1.1f, .340f) X(9, 96, 64, 2, 1, 2, 3, 1, 0, 2.4f, .265f)
 
 static RowsPlan rows_plan(long M, long N, long K, bool swiglu) {
   static const RowsCost tiles[] = {
-#define X(i, bm, bn, wm, wn, wk, st, mw, round, stage) {bm, bn, wk, round, stage},
+#define X(i, bm, bn, wm, wn, wk, st, mw, more, round, stage) {bm, bn, wk, round, stage},
       ROWS_TILES(X)
 #undef X
   };
@@ -1298,9 +1298,10 @@ static bool rows_wins(long M, long N, long K) {
 }
 
 // The same for the gated product in one launch: the other way goes over the projection
-// once more. 28672 x 4096: 333 rows 73 us (72 + 7), 617 127 (126 + 10).
+// once more, which counts the more the shorter K is. 28672 x 4096: 333 rows 73 us (72 +
+// 7), 450 116 (106), 768 159 (185), 1400 288 (294), 2800 483 (607), 16384 2674 (2891).
 static bool rows_swiglu_wins(long M, long N, long K) {
-  if (M <= 32 || M > 1024 || N % 16 || K % 64 || K < 256) return false;
+  if (M <= 32 || N % 16 || K % 64 || K < 256 || (M > 1024 && K > 5120)) return false;
   const double library = std::max(2e-6 * M * N * K / 1.2e3, (N + M) * K * 2 / 4.7e6);
   return rows_plan(M, N, K, true).us * 1.07 < library + M * N * 3 / 5e6 + 3;
 }
@@ -1308,9 +1309,9 @@ static bool rows_swiglu_wins(long M, long N, long K) {
 template <typename F>
 static void rows_tile(int tile, F f) {
   switch (tile) {
-#define X(i, bm, bn, wm, wn, wk, st, mw, round, stage) \
+#define X(i, bm, bn, wm, wn, wk, st, mw, more, round, stage) \
   case i:                                              \
-    f(RowsTile<bm, bn, wm, wn, wk, st, mw>{});         \
+    f(RowsTile<bm, bn, wm, wn, wk, st, mw, false, more>{});         \
     break;
     ROWS_TILES(X)
 #undef X

@@ -808,8 +808,8 @@ void attn_ragged(Tensor q, Tensor kp, OptTensor vp, Tensor table,
 // products of eight experts, 4096 x 14336, us with tiles of 64 to 192 rows and those:
 //   20 rows 484 with 64;  64: 630, 520 with 96, 525 with 128, 547 with 160
 //   96: 695, 788, 553, 572, 614;  150: 644 with 192, 675;  175: 684, 722
-//   225: 809 with 128, 895, 1067, 768;  350: 1279 with 128, 1296, 1132, 1105
-//   1000: 3039 with 128, 2922, 2954, 2696
+//   225: 809 with 128, 895, 1067, 759;  350: 1279 with 128, 1296, 1132, 1036
+//   1000: 3039 with 128, 2922, 2954, 2573
 // The least bounds are 540 of weights and 1.9 a row of operations at 1.5 PF.
 static int moe_height(float a) {
   const float most = a + sqrtf(a);
@@ -945,11 +945,11 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
   else if (BM == 160) rows(RowsTile<160, 256, 2, 2, 1, 3, 1>{}, RowsTile<160, 128, 2, 2, 1, 4, 1>{});
   else if (BM == 192) rows(RowsTile<192, 192, 2, 2, 1, 3, 1>{}, RowsTile<192, 192, 2, 2, 1, 3, 1>{});
   else {
-    constexpr int LDS = RowsTile<160, 256, 2, 2, 1, 3, 1>::LDS;   // the largest
+    constexpr int LDS = RowsTile<256, 256, 2, 4, 1, 2, 2, false, 2>::LDS;   // the largest
     by_planes([&](auto np) {
-      product(np, moe_rows_any_kernel<decltype(np)::value>, 128, 256, LDS);
+      product(np, moe_rows_any_kernel<decltype(np)::value>, 128, 512, LDS);
     });
-    product(second, moe_rows_any_kernel<0>, 128, 256, LDS);
+    product(second, moe_rows_any_kernel<0>, 128, 512, LDS);
   }
   return y;
 }

@@ -184,14 +184,14 @@ Tensor swiglu_grad(Tensor gu, Tensor gm) {
 // cost: fitted to 192 products, 33 to 2000 rows, where the choice takes 2.5% more than
 // the best of eleven tiles and up to 16 splits.
 #define GRAD_TILES(X)                                                                     \
-  X(0, 256, 256, 2, 2, 2, 1, 8.4f, 1.271f) X(1, 160, 256, 2, 2, 3, 1, 6.7f, .854f)         \
-  X(2, 128, 256, 2, 4, 3, 2, 3.3f, .664f) X(3, 192, 128, 2, 2, 3, 1, 5.1f, .587f)          \
-  X(4, 128, 128, 2, 2, 4, 1, 4.2f, .476f) X(5, 96, 128, 2, 2, 4, 1, 3.8f, .406f)           \
-  X(6, 64, 128, 2, 2, 3, 2, 2.6f, .340f)
+  X(0, 256, 256, 2, 4, 2, 2, 2, 6.0f, 1.15f) X(1, 160, 256, 2, 2, 3, 1, 0, 6.7f, .854f)         \
+  X(2, 128, 256, 2, 4, 3, 2, 0, 3.3f, .664f) X(3, 192, 128, 2, 2, 3, 1, 0, 5.1f, .587f)          \
+  X(4, 128, 128, 2, 2, 4, 1, 0, 4.2f, .476f) X(5, 96, 128, 2, 2, 4, 1, 0, 3.8f, .406f)           \
+  X(6, 64, 128, 2, 2, 3, 2, 0, 2.6f, .340f)
 
 static RowsPlan grad_plan(long M, long N, long K) {
   static const RowsCost tiles[] = {
-#define X(i, bm, bn, wm, wn, st, mw, round, stage) {bm, bn, 1, round, stage},
+#define X(i, bm, bn, wm, wn, st, mw, more, round, stage) {bm, bn, 1, round, stage},
       GRAD_TILES(X)
 #undef X
   };
@@ -205,9 +205,13 @@ static RowsPlan grad_plan(long M, long N, long K) {
 //   6144 x 4096: 33 29, 14; 450 52, 37; 1400 72, 69; 2000 92, 83
 //   4096 x 4096: 450 38, 29; 2000 64, 57.  8192 x 28672: 333 159, 189; 900 382, 390
 //   57344 x 8192: 128 297, 170; 450 538, 402; 617 528, 535; 900 695, 738
+// Its form for rows of w to sum over is 4 to 8% slower than that for columns, these are
+// not: 28672 x 4096, 3998 rows 706, 674; 16384 2842, 2818. 4096 x 14336: 3998 393, 376;
+// 16384 1485, 1388. 6144 x 4096: 159, 150; 625, 591. 4096 x 4096: 112, 103; 425, 400.
 static bool linear_grad_wins(long M, long N, long K) {
-  return N % 64 == 0 && K % 256 == 0 && M * K <= 8500000 &&
-         (M <= 512 || M * K * N <= 150000000000L);
+  return N % 64 == 0 && K % 256 == 0 &&
+         (M >= 3000 ||
+          (M * K <= 8500000 && (M <= 512 || M * K * N <= 150000000000L)));
 }
 
 // g (M, N) @ w (N, K) -> (M, K); splits <= 0: as many as the sizes want.
@@ -240,9 +244,9 @@ Tensor linear_grad(Tensor g, Tensor w, long splits) {
     if (a.splits > 1) a.part = parts(a.splits);
     else a.C = out(c);
     switch (plan.tile) {
-#define X(i, bm, bn, wm, wn, st, mw, round, stage)                                      \
+#define X(i, bm, bn, wm, wn, st, mw, more, round, stage)                                      \
   case i: {                                                                             \
-    typedef RowsTile<bm, bn, wm, wn, 1, st, mw, true> T;                                \
+    typedef RowsTile<bm, bn, wm, wn, 1, st, mw, true, more> T;                                \
     rows_launch(gemm_rows_kernel<T>, ldiv_up(M, bm) * ldiv_up(K, bn) * a.splits,        \
                 T::THREADS, T::LDS, stream(), a);                                       \
     break;                                                                              \

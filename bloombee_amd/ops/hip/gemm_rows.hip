@@ -10,16 +10,19 @@
 // half's fragments, or the next stage's behind the one barrier a stage has, and asks for
 // the stage that takes the place of the one just read.
 //
-// Measured, 4096 columns, cold W: 256 x 256 with two stages 1326 TF at 2800 rows of 28672
-// columns (a stage 1.4 us: products alone 1.1, at the clock that power leaves them, DMA
-// alone 1.2). Where one round of workgroups streams W, three stages of smaller tiles hide
-// more of memory: 333 rows 73 us with 192 x 224, 87 with 192 x 256 and two stages, 94 with
+// Measured, 4096 columns, cold W. Large sizes want 256 x 256, on which power and the way
+// from L2 bound it together (a stage 1.4 us: products alone 1.1 at the clock that power
+// leaves them, DMA alone 1.2): four waves and two buffers 1326 TF at 2800 rows of 28672
+// columns, eight waves of half the columns, with a third buffer for W in what LDS is left,
+// 1450 to 1510 from 4096 rows on (a third one for A: 1440; the library's 1525 to 1640).
+// Where one round of workgroups streams W, three stages of smaller tiles hide more of
+// memory: 333 rows 73 us with 192 x 224, 87 with 192 x 256 and two stages, 94 with
 // 192 x 128 and four (W alone, walked by 128 B a row, takes 50).
 // What it writes goes through LDS by whole lines (8 B a lane straight from the sums: 78 us
 // for 73, 513 for 496).
 // Tried and left: 32 columns a stage with five stages, L2 touched a stage or two ahead,
-// all of a stage's DMA at the phase's start: no faster; eight waves of half the columns:
-// as fast at large sizes, 10% slower at 2800 rows.
+// all of a stage's DMA at the phase's start (1347 us for 1320, 8192 rows), the compiler's
+// own order of reads and products in a phase (1430), priorities (1340).
 
 #pragma once
 #include "common.h"
@@ -63,11 +66,13 @@ DEVINL f32x4 pick(bool c, f32x4 x, f32x4 y) {
 // WM x WN waves, times WK groups that take 64 columns each of a stage; ST stages; MINW
 // waves a SIMD. TURNED: sums run over rows of W instead, C(BM,BN) = A(BM,K) @ W(K,BN):
 // 64 rows of it are a stage, by 128 columns, 16 B piece c of row r at c ^ turn(r), and
-// fragments come by transposing reads.
+// fragments come by transposing reads. MORE: one more buffer for A (1) or for W (2), whose
+// loads then come behind the other's.
 template <int BM_, int BN_, int WM_, int WN_, int WK_, int ST_, int MINW_,
-          bool TURNED_ = false>
+          bool TURNED_ = false, int MORE_ = 0>
 struct RowsTile {
   static constexpr bool TURNED = TURNED_;
+  static constexpr int MORE = MORE_;
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, ST = ST_;
   static constexpr int MINW = MINW_;
   static constexpr int NW = WM * WN * WK, THREADS = NW * 64;
@@ -78,7 +83,11 @@ struct RowsTile {
   static constexpr int EXCHANGE = WK > 1 ? BM * BN * 4 : 0;
   static constexpr int OUT_RS = NI * 64 + 16;            // f32 row of the way out
   static constexpr int OUT = NW * 16 * OUT_RS;
-  static constexpr int LDS0 = ST * STAGE > EXCHANGE ? ST * STAGE : EXCHANGE;
+  // buffers of A and of W; loads of the operand that has one more
+  static constexpr int SA = ST + (MORE == 1), SW = ST + (MORE == 2);
+  static constexpr int EX = MORE == 1 ? AJ : MORE == 2 ? LPW - AJ : 0;
+  static constexpr int WBASE = SA * BM * RB, STAGES = WBASE + SW * BN * RB;
+  static constexpr int LDS0 = STAGES > EXCHANGE ? STAGES : EXCHANGE;
   static constexpr int LDS = LDS0 > OUT ? LDS0 : OUT;
   static_assert(AJ * NW * 1024 == BM * RB &&
                 (LPW - AJ) * NW * 1024 == BN * RB && LDS <= 160 * 1024, "chunks");
@@ -118,20 +127,22 @@ struct RowsTile {
       for (int n = 0; n < NI; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
     if (steps <= 0) return;
 
-    auto load = [&](int j, int buf) {
-      const unsigned to = base + buf * STAGE;
+    auto load = [&](int j, int slot_a, int slot_w) {
       if (j < AJ)
-        dma16(ap, ofs[j], to + (j * NW + wave) * 1024);
+        dma16(ap, ofs[j], base + slot_a * (BM * RB) + (j * NW + wave) * 1024);
       else
-        dma16(wp + beyond(j), ofs[j], to + BM * RB + ((j - AJ) * NW + wave) * 1024);
+        dma16(wp + beyond(j), ofs[j],
+              base + WBASE + slot_w * (BN * RB) + ((j - AJ) * NW + wave) * 1024);
     };
+    // load i of an iteration: of the operand with fewer buffers first
+    auto turn_of = [](int i) { return MORE == 1 ? (i + AJ) % LPW : i; };
     // a lane's pieces of its rows
     unsigned fa[2], fw[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const unsigned piece = ((wk * 8 + s * 4 + hi) ^ (li & 7)) * 16;
       fa[s] = (wm * MI * 16 + li) * RB + piece;
-      fw[s] = BM * RB + (wn * NI * 16 + li) * RB + piece;
+      fw[s] = WBASE + (wn * NI * 16 + li) * RB + piece;
     }
     unsigned turned[NI][2];
     if constexpr (TURNED) {
@@ -142,13 +153,13 @@ struct RowsTile {
         for (int q = 0; q < 2; ++q) {
           const int c = (wn * NI + i) * 16, r = hi * 8 + q * 4 + (li >> 2);
           const int piece = c % 128 / 8 + ((li >> 1) & 1);
-          turned[i][q] = BM * RB + c / 128 * 16384 + r * 256 + ((piece ^ turn(r)) << 4) +
+          turned[i][q] = WBASE + c / 128 * 16384 + r * 256 + ((piece ^ turn(r)) << 4) +
                          (li & 1) * 8;
         }
     }
     bf16x8 af[2][MI], wf[2][NI];
-    auto frag = [&](int i, int s, int buf) {
-      const unsigned char* stage = lds + buf * STAGE;
+    auto frag = [&](int i, int s, int slot_a, int slot_w) {
+      const unsigned char* stage = lds + (i < NI ? slot_w * (BN * RB) : slot_a * (BM * RB));
       if (TURNED && i < NI) {
         // column li of rows s * 32 + hi * 8 .. +7
         typedef __attribute__((address_space(3))) short4v lds4;
@@ -168,17 +179,18 @@ struct RowsTile {
         af[s][i - NI] = as_bf16x8(
             *reinterpret_cast<const short8*>(stage + fa[s] + (i - NI) * 16 * RB));
     };
-    // products of half s of a stage, with the other set's reads from buf and loads to
-    // `to` in between
-    auto phase = [&](int s, int buf, auto loads, int to) {
+    // products of half s of a stage, with the other set's reads from slots a, w and, with
+    // loads, those to slots to_a, to_w in between
+    auto phase = [&](int s, int a, int w, auto loads, int to_a, int to_w) {
       constexpr int FR = MI + NI, P = MI * NI;
       int p = 0;
 #pragma unroll
       for (int i = 0; i < FR; ++i) {
-        frag(i, s ^ 1, buf);
+        frag(i, s ^ 1, a, w);
         if constexpr (decltype(loads)::value) {
 #pragma unroll
-          for (int j = i * LPW / FR; j < (i + 1) * LPW / FR; ++j) load(j, to);
+          for (int j = i * LPW / FR; j < (i + 1) * LPW / FR; ++j)
+            load(turn_of(j), to_a, to_w);
         }
 #pragma unroll
         for (; p < (i + 1) * P / FR; ++p) {
@@ -204,37 +216,56 @@ struct RowsTile {
       else wait_loads<0>();
     };
 
+    // ap and wp stand behind what was asked for, the operand with one more buffer ahead
 #pragma unroll
     for (int s = 0; s < ST; ++s)
       if (s < steps) {
 #pragma unroll
-        for (int j = 0; j < LPW; ++j) load(j, s);
+        for (int j = 0; j < LPW; ++j) load(j, s, s);
         ap += BK;
         wp += w_step;
       }
-    wait(min(ST, steps) - 1);
+    if (MORE && ST < steps) {
+#pragma unroll
+      for (int j = 0; j < LPW; ++j)
+        if ((j < AJ) == (MORE == 1)) load(j, ST, ST);
+      if (MORE == 1) ap += BK;
+      else wp += w_step;
+      wait_loads<(ST - 1) * LPW + EX>();
+    } else {
+      wait(min(ST, steps) - 1);
+    }
     barrier();
 #pragma unroll
-    for (int i = 0; i < MI + NI; ++i) frag(i, 0, 0);
-    int buf = 0, t = 0;
-    for (; t + ST < steps; ++t) {
-      phase(0, buf, std::false_type{}, 0);
-      wait_loads<(ST - 2) * LPW>();
+    for (int i = 0; i < MI + NI; ++i) frag(i, 0, 0, 0);
+    int a = 0, w = 0, t = 0;
+    for (; t + ST + (MORE > 0) < steps; ++t) {
+      phase(0, a, w, std::false_type{}, 0, 0);
+      wait_loads<(ST - 2) * LPW + EX>();
       barrier();
-      const int next = buf + 1 == ST ? 0 : buf + 1;
-      phase(1, next, std::true_type{}, buf);
+      const int na = a + 1 == SA ? 0 : a + 1, nw = w + 1 == SW ? 0 : w + 1;
+      phase(1, na, nw, std::true_type{}, a, w);
       ap += BK;
       wp += w_step;
-      buf = next;
+      a = na;
+      w = nw;
       if (MINW == 1) settle();
     }
     for (; t < steps; ++t) {
-      phase(0, buf, std::false_type{}, 0);
-      wait(steps - 2 - t);
+      phase(0, a, w, std::false_type{}, 0, 0);
+      if (MORE) wait_loads<0>();
+      else wait(steps - 2 - t);
       barrier();
-      buf = buf + 1 == ST ? 0 : buf + 1;
+      if (MORE && t + ST < steps) {
+        // the last stage of the operand with fewer buffers
+#pragma unroll
+        for (int j = 0; j < LPW; ++j)
+          if ((j < AJ) != (MORE == 1)) load(j, a, w);
+      }
+      a = a + 1 == SA ? 0 : a + 1;
+      w = w + 1 == SW ? 0 : w + 1;
       // behind the last stage these reads bring what nothing uses
-      phase(1, buf, std::false_type{}, 0);
+      phase(1, a, w, std::false_type{}, 0, 0);
       if (MINW == 1) settle();
     }
 
@@ -305,16 +336,21 @@ struct RowsArgs {
   int M, N, K, splits;
 };
 
-// The chip's order of tiles: the row tiles of a column tile side by side on one XCD, which
-// share W there.
+// The chip's order of tiles: up to eight row tiles of a column tile side by side on one
+// XCD, which share W there, column after column, then the next rows: 32 workgroups at a
+// time read 12 tiles' operands from beyond L2 (64 row tiles side by side, 33 of them: 3338
+// us for 2745, 16384 rows of 28672 columns).
 template <typename T>
 DEVINL void rows_place(int M, int n_tiles, int& m0, int& nt, int& split) {
   const int mt = (M + T::BM - 1) / T::BM;
   const int n = gridDim.x, q = n / 8, r = n % 8, x = blockIdx.x % 8;
-  const int id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + blockIdx.x / 8;
-  m0 = id % mt * T::BM;
-  nt = id / mt % n_tiles;
-  split = id / mt / n_tiles;
+  int id = (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + blockIdx.x / 8;
+  split = id / (mt * n_tiles);
+  id -= split * (mt * n_tiles);
+  const int first = id / (8 * n_tiles) * 8, rows = min(8, mt - first);
+  id -= first * n_tiles;
+  m0 = (first + id % rows) * T::BM;
+  nt = id / rows;
 }
 
 // grid: row tiles * column tiles * splits; K % BK == 0, N % 8 == 0

@@ -33,7 +33,7 @@ SIZES = [(33, 8, 256), (65, 136, 320), (97, 248, 448), (129, 4096, 1024),
 
 GATED = [(33, 8, 256), (97, 1000, 320), (200, 14336, 256), (333, 14336, 448),
          (450, 56, 4096), (617, 4096, 384), (1000, 8192, 512), (64, 120, 576),
-         (164, 29456, 256), (155, 17032, 256), (171, 19000, 256), (222, 16880, 256),
+         (194, 21360, 256), (194, 21360, 320), (155, 17032, 256), (171, 19000, 256), (222, 16880, 256),
          (226, 13024, 256), (131, 11224, 256), (109, 8312, 256), (65, 8912, 256)]
 
 
@@ -78,7 +78,8 @@ def test_gated(M, F, K):
 # (rows, rows of w, columns): every tile, one row short of it or past it, fewer steps
 # than buffers and more
 GRADS = [(1, 64, 256), (63, 128, 512), (65, 448, 4096), (134, 128, 11520),
-         (202, 320, 11520), (284, 1728, 11520), (643, 64, 11264), (450, 4096, 14336),
+         (202, 320, 11520), (284, 1728, 11520), (643, 64, 11264), (643, 128, 11264),
+         (643, 192, 11264), (643, 256, 11264), (520, 192, 13312), (450, 4096, 14336),
          (193, 15168, 11008), (450, 6144, 4096), (333, 28672, 1024), (1999, 4096, 4096)]
 
 

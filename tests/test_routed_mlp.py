@@ -108,6 +108,7 @@ def test_routed_mlp(N, E, top, H, I):
     ([513, 770, 1], 64, 320, 320),
     # 40 tiles or more, 256 columns wide: 97, 128, 150, 171, 192, 200 and 256 rows
     ([193, 256, 300, 342, 384, 400, 512] * 4, 192, 832, 1600),
+    ([400, 130] * 12, 128, 896, 1600),
 ])
 @pytest.mark.parametrize("planes", [1, 2])
 def test_order_of_tiles(counts, K, F, W, planes):
