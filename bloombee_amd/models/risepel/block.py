@@ -251,10 +251,9 @@ class RisepelBlock(torch.nn.Module):
         y = self._gla(h, batch) if self.is_gla else self._latent(h, batch)
         h = add(ragged.linear_parts(y, self.out_w), None, self.norm1_w)
         if self.mlp is not None:
-            a = ragged.clamped_glu(
-                ragged.linear_parts(h, self.mlp_w), 0, self.up_off, self.ff,
-                self.gate_b, self.up_b, self.limit, GLU_SLOPE,
-                self.down_w.shape[1], dt)
+            a = ragged.linear_glu(h, self.mlp_w, self.up_off, self.ff, self.gate_b,
+                                  self.up_b, self.limit, GLU_SLOPE,
+                                  self.down_w.shape[1], dt)
             h = add(ragged.linear_parts(a, self.down_w), self.down_b,
                     self.norm2_w)
         return Carried(h)

@@ -1400,6 +1400,17 @@ torch::Tensor gemm_rows_parts(torch::Tensor A, torch::Tensor W) {
   return C;
 }
 
+template <bool CLAMPED>
+static void rows_glu(RowsArgs& a, const RowsGlu& glu) {
+  rows_tile(rows_plan(a.M, 2L * glu.F, a.K, true).tile, [&](auto tile) {
+    typedef decltype(tile) T;
+    if constexpr (T::WK == 1)
+      rows_launch(gemm_rows_glu_kernel<T, CLAMPED>,
+                  ldiv_up(a.M, T::BM) * ldiv_up(glu.ldc, T::BN / 2), T::THREADS, T::LDS,
+                  cur_stream(), a, glu);
+  });
+}
+
 // swiglu(A @ W^T) of a fused [gate | up] W: (..., N / 2).
 torch::Tensor gemm_rows_swiglu(torch::Tensor A, torch::Tensor W) {
   RowsArgs a = rows_args(A, W);
@@ -1409,13 +1420,31 @@ torch::Tensor gemm_rows_swiglu(torch::Tensor A, torch::Tensor W) {
   auto C = torch::empty(sizes, A.options());
   if (a.M == 0) return C;
   a.C = bf_ptr_mut(C);
-  rows_tile(rows_plan(a.M, a.N, a.K, true).tile, [&](auto tile) {
-    typedef decltype(tile) T;
-    if constexpr (T::WK == 1)
-      rows_launch(gemm_rows_swiglu_kernel<T>,
-                  ldiv_up(a.M, T::BM) * ldiv_up(a.N / 2, T::BN / 2), T::THREADS, T::LDS,
-                  cur_stream(), a);
-  });
+  rows_glu<false>(a, RowsGlu{a.N / 2, a.N / 2, a.N / 2});
+  return C;
+}
+
+// The clamped gated product of rows 0 .. F - 1 of W, gates, and up .. up + F - 1:
+// (M, cols) with zeros behind F.
+torch::Tensor gemm_rows_glu(torch::Tensor A, torch::Tensor W, long up, long F, long cols,
+                            c10::optional<torch::Tensor> gate_b,
+                            c10::optional<torch::Tensor> up_b, double limit,
+                            double slope) {
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(A.dim() == 2 && F > 0 && F % 8 == 0 && cols % 8 == 0 && cols >= F &&
+              up >= 0 && up + F <= a.N && cols < 1 << 24, "bad gated product");
+  auto bias = [&](const c10::optional<torch::Tensor>& t) -> const float* {
+    if (!t.has_value()) return nullptr;
+    TORCH_CHECK(t->is_cuda() && t->scalar_type() == at::kFloat && t->is_contiguous() &&
+                t->numel() >= F, "bad bias");
+    return t->data_ptr<float>();
+  };
+  RowsGlu glu{(int)up, (int)F, (int)cols, bias(gate_b), bias(up_b), (float)limit,
+              (float)slope};
+  auto C = torch::empty({a.M, cols}, A.options());
+  if (a.M == 0) return C;
+  a.C = bf_ptr_mut(C);
+  rows_glu<true>(a, glu);
   return C;
 }
 
@@ -1449,6 +1478,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rows", &gemm_rows);
   m.def("gemm_rows_parts", &gemm_rows_parts);
   m.def("gemm_rows_swiglu", &gemm_rows_swiglu);
+  m.def("gemm_rows_glu", &gemm_rows_glu);
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);
   m.def("stream_rows", &stream_rows);

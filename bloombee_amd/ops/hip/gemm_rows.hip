@@ -426,39 +426,59 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_kernel(RowsArgs
   }
 }
 
-// silu(gate) * up of a fused [gate | up] W, C (M, N / 2), unsplit. A strip of 16 rows of
-// the tile is eight gates and their eight ups: half of a lane's sums change places with
-// those of the lane 32 on, and every lane has both.
-// grid: row tiles * tiles of BN / 2 activations; N % 16 == 0
-template <typename T>
-__global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_swiglu_kernel(RowsArgs a) {
+struct RowsGlu {
+  int up, F, ldc;            // rows of W from a gate to its up, activations, C's columns
+  const float* gate_b;       // CLAMPED: (F,) biases or null
+  const float* up_b;
+  float limit, slope;
+};
+
+// The gated product of a fused [gate | up] W, C (M, ldc) with zeros behind F, unsplit:
+// silu(gate) * up, or with CLAMPED g = min(gate, limit), u = clamp(up, -limit, limit), g *
+// sigmoid(slope * g) * (u + 1). A strip of 16 rows of the tile is eight gates and their
+// eight ups: half of a lane's sums change places with those of the lane 32 on, and every
+// lane has both. grid: row tiles * tiles of BN / 2 of C's columns; F, ldc % 8 == 0
+template <typename T, bool CLAMPED>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(RowsArgs a,
+                                                                            RowsGlu glu) {
   static_assert(T::WK == 1 && T::RPC == 8, "eight rows a load");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  const int lane = threadIdx.x & (WAVE - 1);
+  const int lane = threadIdx.x & (WAVE - 1), hi = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int F = a.N / 2;
   int m0, nt, split;
-  rows_place<T>(a.M, (F + T::BN / 2 - 1) / (T::BN / 2), m0, nt, split);
-  const int n0 = nt * (T::BN / 2);
+  rows_place<T>(a.M, (glu.ldc + T::BN / 2 - 1) / (T::BN / 2), m0, nt, split);
+  const int n0 = nt * (T::BN / 2), w0 = min(n0, glu.F - 1);
 
   unsigned ofs[T::LPW];
 #pragma unroll
   for (int j = 0; j < T::LPW; ++j) {
     const int r = T::load_row(j, wave, lane);
     const int row = j < T::AJ ? min(r, a.M - 1 - m0)
-                              : min(r / 16 * 8 + r % 8, F - 1 - n0);
+                              : min(r / 16 * 8 + r % 8, glu.F - 1 - w0);
     ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
   }
   typename T::Acc acc;
-  T::run(ofs, a.A + (long)m0 * a.K, a.W + (long)n0 * a.K, a.K / T::BK, lds, acc,
-         [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * F * a.K; });
+  T::run(ofs, a.A + (long)m0 * a.K, a.W + (long)w0 * a.K, a.K / T::BK, lds, acc,
+         [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * glu.up * a.K; });
 
   const int c0 = n0 + T::col0() / 2, r0 = m0 + T::row0();
   constexpr int S = (T::NI + 1) / 2;
+  f32x4 gb[S], ub[S];
+  if constexpr (CLAMPED) {
+#pragma unroll
+    for (int n = 0; n < S; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int at = min(c0 + n * 16 + hi * 4 + e, glu.F - 1);
+        gb[n][e] = glu.gate_b ? glu.gate_b[at] : 0.f;
+        ub[n][e] = glu.up_b ? glu.up_b[at] : 0.f;
+      }
+  }
 #pragma unroll
   for (int m = 0; m < T::MI; ++m) {
     const int row0 = r0 + m * 16;
     T::template out16<S, T::NI>(lds, [&](int n) {
+      const int col = c0 + n * 16 + hi * 4;
       f32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -466,13 +486,21 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_swiglu_kernel(R
         const float y = 2 * n + 1 < T::NI ? acc[m][2 * n + 1 < T::NI ? 2 * n + 1 : 0][e] : 0.f;
         const auto s = __builtin_amdgcn_permlane32_swap(
             __builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y), false, false);
-        const float g = __builtin_bit_cast(float, (unsigned)s[0]);
-        v[e] = g / (1.f + fast_expf(-g)) * __builtin_bit_cast(float, (unsigned)s[1]);
+        float g = __builtin_bit_cast(float, (unsigned)s[0]);
+        float u = __builtin_bit_cast(float, (unsigned)s[1]);
+        if constexpr (CLAMPED) {
+          g = fminf(g + gb[n][e], glu.limit);
+          u = fminf(fmaxf(u + ub[n][e], -glu.limit), glu.limit);
+          v[e] = g / (1.f + fast_expf(-glu.slope * g)) * (u + 1.f);
+        } else {
+          v[e] = g / (1.f + fast_expf(-g)) * u;
+        }
+        if (col >= glu.F) v[e] = 0.f;
       }
       return pack4(v);
     }, [&](int r, int c, auto v) {
-      if (row0 + r < a.M && c0 + c < F)
-        *reinterpret_cast<decltype(v)*>(a.C + (long)(row0 + r) * F + c0 + c) = v;
+      if (row0 + r < a.M && c0 + c < glu.ldc)
+        *reinterpret_cast<decltype(v)*>(a.C + (long)(row0 + r) * glu.ldc + c0 + c) = v;
     });
   }
 }

@@ -37,11 +37,11 @@ static RowsPlan rows_best(const RowsCost* tiles, int n, long M, long N, long K,
   return best;
 }
 
-template <typename K>
+template <typename K, typename... Args>
 static void rows_launch(K kernel, long grid, int threads, int lds, hipStream_t stream,
-                        const RowsArgs& a) {
+                        const Args&... a) {
   HIP_OK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-  kernel<<<grid, threads, lds, stream>>>(a);
+  kernel<<<grid, threads, lds, stream>>>(a...);
   HIP_OK(hipGetLastError());
 }

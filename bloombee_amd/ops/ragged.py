@@ -216,6 +216,20 @@ def clamped_glu(parts: torch.Tensor, g_off: int, u_off: int, ff: int,
     return F.pad(a.to(dtype), (0, cols - ff))
 
 
+def linear_glu(x: torch.Tensor, w: torch.Tensor, u_off: int, ff: int,
+               gate_b: Optional[torch.Tensor], up_b: Optional[torch.Tensor],
+               limit: float, slope: float, cols: int,
+               dtype: torch.dtype) -> torch.Tensor:
+    """clamped_glu of x (M, K) @ w^T, gates from row 0 and ups from row u_off of w: in
+    one launch where that is the faster form (sums are then not rounded between)."""
+    if (x.dtype == dtype and ff % 8 == 0 and cols % 8 == 0
+            and interface.rows_glu_ok(x, w, ff)):
+        return interface.hip_ops.gemm_rows_glu(x.contiguous(), w, u_off, ff, cols,
+                                               gate_b, up_b, limit, slope)
+    return clamped_glu(linear_parts(x, w), 0, u_off, ff, gate_b, up_b, limit, slope,
+                       cols, dtype)
+
+
 def softcap_(z: torch.Tensor, cap: float) -> torch.Tensor:
     """z <- cap * tanh(z / cap), f32, in place."""
     if z.is_cuda:

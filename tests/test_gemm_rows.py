@@ -75,6 +75,33 @@ def test_gated(M, F, K):
                  + 2.0 ** -8 * (g.abs() + 1) * u.abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("M,F,up,cols,K", [
+    (33, 8, 8, 64, 256), (65, 1000, 1024, 1088, 320), (200, 4096, 4100, 4096, 256),
+    (333, 712, 715, 768, 576), (617, 1400, 1400, 1408, 384), (194, 21360, 21376, 21504, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_clamped(M, F, up, cols, K, bias):
+    """Activations that end within a tile, columns of zeros behind them."""
+    from bloombee_amd.ops import ragged
+    x, w = draw(M, K, seed=1), draw(up + F, K, seed=2, scale=K ** -0.5)
+    b = ((torch.randn(F, device=DEV), torch.randn(F, device=DEV)) if bias
+         else (None, None))
+    g, u = (x.double() @ w[o:o + F].double().T + (0 if v is None else v.double())
+            for o, v in zip((0, up), b))
+    g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+    want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    got = ops.hip_ops.gemm_rows_glu(x, w, up, F, cols, *b, 1.5, 1.702)
+    # a sum is off by 2^-20 of its terms, their product by as much of both
+    tol = (x.double().abs() @ w[:F].double().abs().T,
+           x.double().abs() @ w[up:].double().abs().T)
+    assert bool(((got[:, :F].double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -18 * (tol[0] * 2.5 + tol[1] * g.abs() + 1)).all())
+    assert got.shape == (M, cols) and not got[:, F:].any()
+    y = ragged.linear_glu(x, w, up, F, *b, 1.5, 1.702, cols, torch.bfloat16)
+    # where it is two steps, gate and up are rounded, 2^-9 of each
+    assert bool(((y[:, :F].double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -7 * (g.abs() + 1) * 2.5).all()) and not y[:, F:].any()
+
+
 # (rows, rows of w, columns): every tile, one row short of it or past it, fewer steps
 # than buffers and more
 GRADS = [(1, 64, 256), (63, 128, 512), (65, 448, 4096), (134, 128, 11520),
