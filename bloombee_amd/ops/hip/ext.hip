@@ -961,6 +961,60 @@ static void launch_skinny_fused(const StreamArgs& a, int kchunk, int ksplit,
   else launch(std::integral_constant<int, 2>{});
 }
 
+// ---------------------------------------------------------------------------
+// decode products on a tile of gemm_rows.hip
+// ---------------------------------------------------------------------------
+
+// 32 rows by 64 columns, two groups of waves over K, two workgroups a CU: W comes by whole
+// lines and by DMA, up to 48 KB ahead a workgroup, and its rows of A once for 64 columns.
+typedef RowsTile<32, 64, 2, 1, 2, 3, 2> FewRows;
+
+// Splits of K that let all CUs take part, one or two workgroups each.
+static int few_splits(long N, long K) {
+  const long wgs = ldiv_up(N, 64);
+  int best = 1;
+  float most = 0.f;
+  for (int s = 1; s <= 16 && (s == 1 || (wgs * s <= 512 && K / s >= 512)); ++s) {
+    const float fill = wgs * s / (256.f * ldiv_up(wgs * s, 256));
+    if (fill > most + .02f) {
+      most = fill;
+      best = s;
+    }
+    if (fill >= .9f) break;
+  }
+  return best;
+}
+
+// Whether it beats the gated products of gemm_stream.hip and gemm_skinny.hip: where its
+// workgroups fill the chip's rounds. Up to 16 rows are left to those, which are 2 us faster
+// in a step than alone, this is not. us alone, those and this: 28672 x 4096: 1 row 45.3,
+// 45.0; 16 rows 46.9, 44.7; 32 50.4, 47.2. 27648 x 5120, 32 rows: 63.3, 55.0; 12288 x 1536
+// 12.8, 10.5; 57344 x 8192 188.2, 167.7; 128256 x 4096 206.3, 196.2. Half empty, 17 rows:
+// 22016 x 4096 39.8, 41.2; 36864 x 4096 62.3, 63.7; 6144 x 4096 14.2, 17.2.
+static bool few_swiglu(long M, long N, long K) {
+  const long wgs = ldiv_up(N, 64);
+  if (K % 128 || K < 1024 || M <= 16 || M > 32) return false;
+  if (wgs <= 256) return wgs >= 190;
+  if (wgs <= 512) return wgs >= 410;
+  return wgs * 20 >= ldiv_up(wgs, 512) * 512 * 17;
+}
+
+// Whether it beats their sums: wherever those want the split form (whose waves take W by
+// 64 B of a row), and from some rows on where the one-launch form reads all of A for every
+// 16 columns. us in a graph, those and this: 4096 x 14336: 8 rows 25.1, 25.7; 16 30.0,
+// 25.7; 32 31.5, 25.2. 5120 x 13824: 1 row 35.3, 29.5; 32 39.4, 30.6. 28672 x 4096: 44.2,
+// 43.6; 16 48.4, 44.5. 512 x 14336: 13.3, 8.2. 8192 x 28672: 32 rows 99.2, 91.5. 151936 x
+// 1024: 16 rows 64.3, 60.6. One launch: 6144 x 4096: 4 rows 14.4, 14.4; 16 16.5, 15.0; 32
+// 19.4, 15.9. 20480 x 5120: 4 44.1, 47.0; 16 58.1, 49.2. 4096 x 4096: 16 10.3, 11.4; 18176 x
+// 4096, 284 workgroups: 17 rows 36.3, 39.6. 1024 x 3072: any 5.6 to 7.2, 6.8 to 7.6.
+static bool few_sums(long M, long N, long K) {
+  if (M <= 0 || M > 32 || K % 128 || K < 1024 || N % 8) return false;
+  if (!stream_sums(M, N, K)) return true;
+  const long wgs = ldiv_up(N, 64) * few_splits(N, K);
+  return M > 8 && N * K >= 24L << 20 && K >= 3072 &&
+         wgs * 10 >= ldiv_up(wgs, 256) * 256 * 6;
+}
+
 // silu(gate) * up of [gate | up] = rms(A) @ W^T, norm weight folded into W.
 torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   StreamArgs a = stream_args(A, W);
@@ -971,6 +1025,21 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   a.C = bf_ptr_mut(C);
   a.eps = eps;
   if (a.M == 0) return C;
+  if ((size_t)W.data_ptr() % 16 == 0 && few_swiglu(a.M, a.N, a.K)) {
+    RowsArgs r{};
+    r.A = a.A;
+    r.W = a.W;
+    r.C = a.C;
+    r.M = a.M;
+    r.N = a.N;
+    r.K = a.K;
+    r.splits = 1;
+    RowsGlu glu{a.N / 2, a.N / 2, a.N / 2};
+    glu.eps = a.eps;
+    rows_launch(gemm_rows_glu_kernel<FewRows, false, true>, ldiv_up(a.N, FewRows::BN),
+                FewRows::THREADS, FewRows::LDS, cur_stream(), r, glu);
+    return C;
+  }
   if (!stream_swiglu(a.M, a.N, a.K)) {
     launch_skinny_fused<true>(a, a.K, 1, nullptr, nullptr);
     return C;
@@ -1369,7 +1438,9 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
   a.R = operand(residual, (long)a.M * a.N);
   a.bias = operand(bias, a.N);
   if (a.M == 0) return C;
-  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
+  const bool few = few_sums(a.M, a.N, a.K);
+  const RowsPlan plan =
+      few ? RowsPlan{-1, few_splits(a.N, a.K)} : rows_plan(a.M, a.N, a.K, false);
   a.splits = plan.splits;
   a.C = plan.splits > 1 ? nullptr : bf_ptr_mut(C);
   torch::Tensor part;
@@ -1377,7 +1448,11 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
     part = torch::empty({plan.splits, a.M, a.N}, A.options().dtype(at::kFloat));
     a.part = part.data_ptr<float>();
   }
-  rows_product(a, plan);
+  if (few)
+    rows_launch(gemm_rows_kernel<FewRows>, ldiv_up(a.N, FewRows::BN) * a.splits,
+                FewRows::THREADS, FewRows::LDS, cur_stream(), a);
+  else
+    rows_product(a, plan);
   if (plan.splits > 1) {
     a.C = bf_ptr_mut(C);
     gemm_rows_fold_kernel<<<ldiv_up((long)a.M * a.N, 2048), 256, 0, cur_stream()>>>(a);
@@ -1469,6 +1544,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("norm_route", &norm_route);
   m.def("add_experts", &add_experts);
   m.def("gemm_stream", &gemm_stream);
+  m.def("few_sums", &few_sums);
+  m.def("few_swiglu", &few_swiglu);
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {

@@ -112,11 +112,12 @@ struct RowsTile {
 
   // Sums of `steps` stages. ofs: bytes from ap (j < AJ) or wp, which move on by a
   // stage's columns (wp by w_step); beyond(j): what the rows of a load lie behind wp, the
-  // wave's.
-  template <typename B>
+  // wave's. NORM: rows of A are divided by their root mean square, columns of K; a row's
+  // sum of squares is the diagonal of A A^T, made from the fragments at hand.
+  template <bool NORM = false, typename B>
   static DEVINL void run(const unsigned (&ofs)[LPW], const unsigned short* ap,
                          const unsigned short* wp, int steps, unsigned char* lds,
-                         Acc& acc, B beyond, long w_step = BK) {
+                         Acc& acc, B beyond, long w_step = BK, float eps = 0.f) {
     const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
@@ -157,6 +158,9 @@ struct RowsTile {
                          (li & 1) * 8;
         }
     }
+    f32x4 sq[MI];
+#pragma unroll
+    for (int m = 0; m < MI; ++m) sq[m] = (f32x4){0.f, 0.f, 0.f, 0.f};
     bf16x8 af[2][MI], wf[2][NI];
     auto frag = [&](int i, int s, int slot_a, int slot_w) {
       const unsigned char* stage = lds + (i < NI ? slot_w * (BN * RB) : slot_a * (BM * RB));
@@ -202,6 +206,11 @@ struct RowsTile {
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (NORM)
+#pragma unroll
+        for (int m = 0; m < MI; ++m)
+          sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[s][m], af[s][m], sq[m], 0, 0,
+                                                          0);
     };
     auto barrier = [&]() {
       __builtin_amdgcn_s_barrier();
@@ -288,6 +297,26 @@ struct RowsTile {
         for (int n = 0; n < H; ++n)
           acc[m][n] = pick(wk, acc[m][n + H], acc[m][n]) +
                       ex[(wk * MI * H + m * H + n) * 64 + lane];
+    }
+    if constexpr (NORM) {
+      static_assert(MINW > 1 && WK * BM * 4 + EXCHANGE <= STAGES, "squares");
+      if (WK == 1) __syncthreads();
+      float* squares = reinterpret_cast<float*>(lds + EXCHANGE);
+#pragma unroll
+      for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (hi * 4 + e == li) squares[wk * BM + (wm * MI + m) * 16 + li] = sq[m][e];
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < MI; ++m) {
+        float all = 0.f;
+#pragma unroll
+        for (int g = 0; g < WK; ++g) all += squares[g * BM + (wm * MI + m) * 16 + li];
+        const float r = rsqrtf(all / (float)(steps * BK) + eps);
+#pragma unroll
+        for (int n = 0; n < NI / WK; ++n) acc[m][n] *= r;
+      }
     }
     __syncthreads();   // the way out takes the place of the stages
   }
@@ -431,6 +460,7 @@ struct RowsGlu {
   const float* gate_b;       // CLAMPED: (F,) biases or null
   const float* up_b;
   float limit, slope;
+  float eps;                 // NORM
 };
 
 // The gated product of a fused [gate | up] W, C (M, ldc) with zeros behind F, unsplit:
@@ -438,10 +468,11 @@ struct RowsGlu {
 // sigmoid(slope * g) * (u + 1). A strip of 16 rows of the tile is eight gates and their
 // eight ups: half of a lane's sums change places with those of the lane 32 on, and every
 // lane has both. grid: row tiles * tiles of BN / 2 of C's columns; F, ldc % 8 == 0
-template <typename T, bool CLAMPED>
+// NORM: of the rows of A, their norm's weight folded into W.
+template <typename T, bool CLAMPED, bool NORM = false>
 __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(RowsArgs a,
                                                                             RowsGlu glu) {
-  static_assert(T::WK == 1 && T::RPC == 8, "eight rows a load");
+  static_assert(8 % T::RPC == 0, "rows of a load are of one kind");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & (WAVE - 1), hi = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -458,11 +489,13 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(Rows
     ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
   }
   typename T::Acc acc;
-  T::run(ofs, a.A + (long)m0 * a.K, a.W + (long)w0 * a.K, a.K / T::BK, lds, acc,
-         [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * glu.up * a.K; });
+  T::template run<NORM>(
+      ofs, a.A + (long)m0 * a.K, a.W + (long)w0 * a.K, a.K / T::BK, lds, acc,
+      [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * glu.up * a.K; }, T::BK,
+      glu.eps);
 
   const int c0 = n0 + T::col0() / 2, r0 = m0 + T::row0();
-  constexpr int S = (T::NI + 1) / 2;
+  constexpr int NO = T::COLS / 16, S = (NO + 1) / 2;
   f32x4 gb[S], ub[S];
   if constexpr (CLAMPED) {
 #pragma unroll
@@ -477,13 +510,13 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(Rows
 #pragma unroll
   for (int m = 0; m < T::MI; ++m) {
     const int row0 = r0 + m * 16;
-    T::template out16<S, T::NI>(lds, [&](int n) {
+    T::template out16<S, NO>(lds, [&](int n) {
       const int col = c0 + n * 16 + hi * 4;
       f32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float x = acc[m][2 * n][e];
-        const float y = 2 * n + 1 < T::NI ? acc[m][2 * n + 1 < T::NI ? 2 * n + 1 : 0][e] : 0.f;
+        const float y = 2 * n + 1 < NO ? acc[m][2 * n + 1 < NO ? 2 * n + 1 : 0][e] : 0.f;
         const auto s = __builtin_amdgcn_permlane32_swap(
             __builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y), false, false);
         float g = __builtin_bit_cast(float, (unsigned)s[0]);

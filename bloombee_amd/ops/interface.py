@@ -358,6 +358,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
     if (_on_gpu(x) and M <= 32 and x.dtype == torch.bfloat16
             and K % 256 == 0 and N % 64 == 0):
         _require_ext()
+        if (norm is None and ss_in is None and ss_out is None
+                and w.data_ptr() % 16 == 0 and hip_ops.few_sums(M, N, K)):
+            return hip_ops.gemm_rows(x.contiguous(), w, residual, bias)
         if (ss_in is None and ss_out is None
                 and (hip_ops.stream_sums(M, N, K) if norm is None else
                      norm[0] is None and hip_ops.stream_rows(M, N, K))):

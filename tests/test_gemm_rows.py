@@ -75,6 +75,40 @@ def test_gated(M, F, K):
                  + 2.0 ** -8 * (g.abs() + 1) * u.abs() + 1e-6).all())
 
 
+FEW = [(1, 28672, 1024), (9, 5120, 13824), (16, 4096, 14336), (17, 28672, 1280),
+       (31, 576, 9216), (32, 8192, 8192), (32, 6144, 4096), (5, 192, 14336)]
+
+
+@pytest.mark.parametrize("M,N,K", FEW)
+def test_few_rows(M, N, K):
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    r, b = draw(M, N, seed=3), draw(N, seed=4)
+    want = x.double() @ w.double().T
+    terms = x.double().abs() @ w.double().abs().T
+    assert ops.hip_ops.few_sums(M, N, K)
+    assert close(ops.linear(x, w), want, terms)
+    assert close(ops.linear(x, w, residual=r, bias=b), want + r.double() + b.double(),
+                 terms + r.double().abs() + b.double().abs())
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 26304, 1024), (18, 12288, 1280), (25, 28672, 4096),
+                                   (32, 27648, 1280), (17, 57344, 1024), (31, 98304, 1024)])
+def test_few_rows_gated(M, N, K):
+    """The rows' norm, folded into w, rides along."""
+    x, w = draw(M, K, seed=1, scale=3.0), draw(N, K, seed=2, scale=K ** -0.5)
+    x[0] *= 1e-3      # where eps counts
+    assert ops.hip_ops.few_swiglu(M, N, K)
+    y = x.double()
+    r = (y.square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+    g, u = ((y @ w.double().T) * r).chunk(2, -1)
+    want = torch.nn.functional.silu(g) * u
+    got = ops.linear_swiglu(x, w, 1e-5)
+    tol = ((y.abs() @ w.double().abs().T) * r).chunk(2, -1)
+    # sums and root within 2^-20 of their terms, hardware exponential and reciprocal
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -18 * (tol[0] * (u.abs() + 1) + tol[1] * (g.abs() + 1))).all())
+
+
 @pytest.mark.parametrize("M,F,up,cols,K", [
     (33, 8, 8, 64, 256), (65, 1000, 1024, 1088, 320), (200, 4096, 4100, 4096, 256),
     (333, 712, 715, 768, 576), (617, 1400, 1400, 1408, 384), (194, 21360, 21376, 21504, 256)])
