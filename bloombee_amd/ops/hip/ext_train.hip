@@ -230,8 +230,8 @@ Tensor linear_grad(Tensor g, Tensor w, long splits) {
     part = torch::empty({n, M, K}, g.options().dtype(at::kFloat));
     return part.data_ptr<float>();
   };
-  // a stage's rows of w lie within 32 bits of bytes
-  if (N % 64 == 0 && K < (1L << 24) && N < (1L << 24)) {
+  // a tile's 256 rows of g and a stage's 64 of w lie within 32 bits of bytes
+  if (N % 64 == 0 && K < (1L << 24) && N < (1L << 23)) {
     RowsPlan plan = grad_plan(M, N, K);
     if (splits > 0) plan.splits = (int)std::min<long>(splits, N / 64);
     RowsArgs a{};

@@ -189,6 +189,14 @@ def test_views():
                  x.double().abs() @ odd.double().abs().T)
 
 
+def test_places_of_32_bits():
+    """Rows too long for a tile's places are left to the kernels that had them."""
+    assert ops.hip_ops.few_sums(1, 64, (1 << 20) - 128)
+    assert not ops.hip_ops.few_sums(1, 64, 1 << 20)
+    assert not ops.hip_ops.rows_wins(33, 64, 1 << 20)
+    assert not ops.hip_ops.rows_swiglu_wins(33, 64, 1 << 20)
+
+
 def test_recorded_and_replayed():
     """Gradients reach x through linear; a captured product gives the eager one's bits
     on every replay."""
