@@ -909,6 +909,19 @@ static void by_rows(int M, F f) {
   else f(std::integral_constant<int, 2>{}, std::integral_constant<int, 8>{});
 }
 
+// How many parts of K a product of few rows and columns is taken in at once
+// (gemm_stream_parts_kernel), 0: none, workgroups of 16 rows of W. Parts pay where these
+// leave half of the chip or more idle and theirs fit one round, the more of them the
+// longer K. us in a graph, with 0, 2, 4 parts: 1024 x 1024: 1 row 3.6, 3.7, 3.9; x 2048:
+// 4.6, 3.7, 4.0; 8 rows 5.1, 4.4; x 3072: 1 row 5.6, 4.8, 4.0; 4 rows 5.7, 5.6, 4.7; 8 rows
+// 6.4, 6.2; x 8192: 1 row 10.7, 7.1, 5.3. 2048 x 1024: 3.7, 3.9, 5.0; x 2048: 4.7, 4.0,
+// 5.1; x 4096: 6.7, 5.3, 5.3; 4 rows 6.8, 5.8, 6.5; 8 rows 7.5, 6.4. Two rounds: 2560 x
+// 2048: 4.8, 5.0, 6.2; 4096 x 4096: 7.9, 7.8, 7.6; 4 rows 7.9, 8.8, 10.1.
+static int stream_parts(long M, long N, long K) {
+  if (M > 8 || N > 2048 || K <= 1024) return 0;
+  return M <= 4 && N <= 1024 && K > 2048 ? 4 : 2;
+}
+
 // C(M,N) = A @ W^T [* 1/rms of A's rows] [+ bias] [+ residual], M <= 32; eps < 0: no
 // norm.
 torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
@@ -933,6 +946,15 @@ torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
     a.bias = bf_ptr(*bias);
   }
   if (a.M == 0) return C;
+  const int parts = eps < 0 ? stream_parts(a.M, a.N, a.K) : 0;
+  if (parts) {
+    if (parts == 4)
+      gemm_stream_parts_kernel<4, 8><<<a.N / 4, 512, 0, cur_stream()>>>(a);
+    else
+      gemm_stream_parts_kernel<2, 8><<<a.N / 8, 512, 0, cur_stream()>>>(a);
+    HIP_OK(hipGetLastError());
+    return C;
+  }
   by_rows(a.M, [&](auto mt, auto xn) {
     constexpr int MT = decltype(mt)::value, XN = decltype(xn)::value;
     constexpr int DP = MT == 1 ? 4 : 1;
@@ -1562,6 +1584,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_rope_kv", &gemm_rope_kv);
   m.def("stream_rows", &stream_rows);
   m.def("stream_sums", &stream_sums);
+  m.def("stream_parts", &stream_parts);
   m.def("stream_swiglu", &stream_swiglu);
   m.def("stream_rope", &stream_rope);
   m.def("attn_prefill", &attn_prefill);

@@ -269,3 +269,58 @@ __global__ __launch_bounds__(NW * 64, NW / 4) void gemm_stream_kernel(StreamArgs
     rope_kv_store(a, row0[0] / a.D, row0[0] % a.D + n, m, v, u);
   }
 }
+
+// EPI_SUM of up to RW = 16 / PARTS rows without a norm, where W has too few rows for
+// workgroups of 16 to fill the chip: a workgroup owns RW rows of W, and what would be
+// sixteen rows of an operand are RW of each in PARTS parts of K. Products of unequal
+// parts are nobody's; those of part p are where p = li / RW = hi * 4 / RW. A wave takes 32
+// * PARTS columns at a time, whole lines of each row, four such pieces on their way; A
+// comes to registers, bias and residual ahead of it all.
+// What a CU takes in bounds small products: with 64 of them at work 1024 x 3072 takes 5.6
+// us, with all 256, each a quarter of the bytes, 4.0, of which 3 are the launch.
+template <int PARTS, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_stream_parts_kernel(StreamArgs a) {
+  constexpr int DP = 4, RW = 16 / PARTS, STEP = 32 * PARTS, GROUPS = 64 / (RW * RW);
+  __shared__ __attribute__((aligned(16))) float sums[NW * PARTS * RW * RW];
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int li = lane & 15, hi = lane >> 4, part = li / RW;
+  const int row0 = blockIdx.x * RW, count = a.K / STEP;
+  const int m = lane % (RW * RW) / RW, n = row0 + lane % RW;   // of the way out
+  const bool mine = wave == 0 && lane < RW * RW && m < a.M;
+  unsigned short bias = 0, res = 0;
+  if (mine && a.bias) bias = a.bias[n];
+  if (mine && a.R) res = a.R[(long)m * a.N + n];
+  const unsigned short* w = a.W + (long)(row0 + li % RW) * a.K + part * 32 + hi * 8;
+  const unsigned short* x = a.A + (long)min(li % RW, a.M - 1) * a.K + part * 32 + hi * 8;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int i = wave; i < count; i += NW * DP) {
+    short8 wf[DP], xf[DP];
+#pragma unroll
+    for (int d = 0; d < DP; ++d) {
+      const int k = min(i + d * NW, count - 1) * STEP;
+      wf[d] = *reinterpret_cast<const short8*>(w + k);
+      xf[d] = *reinterpret_cast<const short8*>(x + k);
+    }
+#pragma unroll
+    for (int d = 0; d < DP; ++d) {
+      if (i + d * NW >= count) wf[d] = xf[d] = short8{};
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(wf[d]), as_bf16x8(xf[d]),
+                                                    acc, 0, 0, 0);
+    }
+  }
+  // [wave and part][row of A][row of W]
+  if (hi * 4 / RW == part)
+    *reinterpret_cast<f32x4*>(
+        &sums[((wave * PARTS + part) * RW + li % RW) * RW + hi * 4 % RW]) = acc;
+  __syncthreads();
+  if (wave) return;
+  float v = 0.f;
+#pragma unroll
+  for (int i = 0; i < NW * PARTS / GROUPS; ++i)
+    v += sums[(lane / (RW * RW) * (NW * PARTS / GROUPS) + i) * (RW * RW) +
+              lane % (RW * RW)];
+#pragma unroll
+  for (int o = RW * RW; o < 64; o *= 2) v += __shfl_xor(v, o);
+  if (mine) a.C[(long)m * a.N + n] = f2bf(v + bf2f(bias) + bf2f(res));
+}

@@ -42,6 +42,28 @@ def test_stream(M, N, K):
           rms(x, 1e-5) @ w.double().T + r.double())
 
 
+# (columns, K, parts of K up to 4 rows and up to 8): ends of the rule; a wave's pieces
+# fewer than four, four and more, some waves without any
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 7, 8, 9])
+@pytest.mark.parametrize("N,K,few,more", [
+    (16, 1024, 0, 0), (16, 1152, 2, 2), (1024, 2048, 2, 2), (1024, 2176, 4, 2),
+    (1040, 3072, 2, 2), (2048, 1152, 2, 2), (2064, 2048, 0, 0), (32, 4096, 4, 2),
+    (48, 4224, 4, 2)])
+def test_stream_in_parts(M, N, K, few, more):
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    b, r = draw(N, seed=3), draw(M, N, seed=4)
+    assert ops.hip_ops.stream_parts(M, N, K) == (few if M <= 4 else more if M <= 8
+                                                 else 0)
+    want = x.double() @ w.double().T
+    close(ops.hip_ops.gemm_stream(x, w, None, None, -1.0), want)
+    close(ops.hip_ops.gemm_stream(x, w, r, b, -1.0), want + b.double() + r.double())
+    # what is not finite stays in its row of x or of w
+    x[M - 1, K - 1], w[5, 0] = float("inf"), float("nan")
+    got, want = ops.hip_ops.gemm_stream(x, w, None, None, -1.0), x.float() @ w.float().T
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf())
+
+
 def test_stream_refuses_what_it_cannot_do():
     for M, N, K in ((33, 16, 128), (1, 24, 128), (1, 16, 192)):
         with pytest.raises(RuntimeError):
