@@ -63,8 +63,9 @@ DEVINL float quad16_reduce_sum(float x) {
 // every tile's loads were waited for ahead of the one before it. 32 contexts of 2048
 // 54.5 -> 50.1 us, of 8000 184 -> 172 (6.1 TB/s), 97 of 64 to 4000 182 -> 157.
 // Costs ~96 VGPRs of double buffers.
-template <int D, int MAXG, int NT, int PIPE = 0>
-__global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
+// NW: waves a workgroup, which share its split's tiles.
+template <int D, int MAXG, int NT, int PIPE = 0, int NW = 4>
+__global__ __launch_bounds__(NW * 64, 2) void attn_decode_mfma_kernel(
     const unsigned short* __restrict__ q,        // strided, see q_sb/q_sh
     const unsigned short* __restrict__ k_pages,  // (np, Hkv, P, D)
     const unsigned short* __restrict__ v_pages,  // (np, Hkv, D, P) d-major
@@ -108,10 +109,11 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
   const float sc2 = scale * LOG2E;
 
   // per-wave LDS: P^T tile (C->B relayout, head-major rows) + merge scratch
+  constexpr int SLOTS = MAXG == 4 ? NW : NW - 1;   // of waves' results
   __shared__ __attribute__((aligned(16))) unsigned char lds[
-      4 * 16 * PROW_B + 3 * (MAXG * (D + 2) * 4)];
+      NW * 16 * PROW_B + SLOTS * (MAXG * (D + 2) * 4)];
   unsigned char* p_lds = lds + wave * 16 * PROW_B;
-  float* merge_lds = (float*)(lds + 4 * 16 * PROW_B);
+  float* merge_lds = (float*)(lds + NW * 16 * PROW_B);
 
   // Q fragments: B[k=d][col=head]; col = li (cols >= Gl harmless garbage)
   const int qh = g0 + ((li < Gl) ? li : Gl - 1);
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
   // with compile-time indices, and sched_barrier pins each prefetch above
   // the compute phase it overlaps (the scheduler otherwise sinks loads to
   // their uses and the pipeline degenerates to the serial form).
-  constexpr int TSTRIDE = 4 * NT * DKVBLK;
+  constexpr int TSTRIDE = NW * NT * DKVBLK;
   const int tbs = c0 + (tile0 + wave * NT) * DKVBLK;
 
   if constexpr (PIPE) {
@@ -398,14 +400,14 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
   }
   }
 
-  // ---- merge the 4 waves ----
+  // ---- merge the waves ----
   // C col li holds chunk-local head g = li (valid for g < Gl); C row
   // hi*4 + reg of tile n is dimension d = 16n + hi*4 + reg. (m, l) are
   // replicated across the 4 hi subgroups — hi == 0 publishes them.
   auto wave_slot = [&](int slot) { return merge_lds + slot * MAXG * (D + 2); };
   __syncthreads();
-  if (wave > 0) {
-    float* dst = wave_slot(wave - 1);
+  if (SLOTS == NW || wave > 0) {
+    float* dst = wave_slot(SLOTS == NW ? wave : wave - 1);
     if (li < Gl) {
 #pragma unroll
       for (int n = 0; n < NDT; ++n)
@@ -419,8 +421,40 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma_kernel(
     }
   }
   __syncthreads();
+  if constexpr (SLOTS == NW) {
+    // few heads: every thread folds dimensions of its own (one wave alone, the others'
+    // results one after the other, took 1.2 us longer, 7.5 for 6.3: 1 sequence of 170)
+    for (int i = tid; i < Gl * D; i += NW * 64) {
+      const int g = i / D, d = i % D;
+      const float* src = merge_lds + g * (D + 2);
+      float mw[NW], mx = NEG_BIG, lt = 0.f, v = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        mw[w] = src[w * MAXG * (D + 2) + D];
+        mx = fmaxf(mx, mw[w]);
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float c = fast_exp2(mw[w] - mx);
+        lt += src[w * MAXG * (D + 2) + D + 1] * c;
+        v += src[w * MAXG * (D + 2) + d] * c;
+      }
+      if (n_split == 1) {
+        out[(long)b * out_sb + (long)(kvh * G + g0 + g) * out_sh + d] =
+            f2bf(lt > 0.f ? v * (1.f / lt) : 0.f);
+        continue;
+      }
+      const long at = ((long)bh * n_split + split) * MAXG + g;
+      part_acc[at * D + d] = v;
+      if (d == 0) {
+        part_ml[at * 2] = mx;
+        part_ml[at * 2 + 1] = lt;
+      }
+    }
+    return;
+  }
   if (wave != 0) return;
-  for (int slot = 0; slot < 3; ++slot) {
+  for (int slot = 0; slot < NW - 1; ++slot) {
     const float* src = wave_slot(slot);
     if (li < Gl) {
       const float mo = src[li * (D + 2) + D];

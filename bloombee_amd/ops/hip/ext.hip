@@ -207,7 +207,7 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
                                int Hkv, int G, int nch, int P, int maxp,
                                int n_split, int window, float scale, long q_off,
                                long q_sb, long q_sh, long out_sb, long out_sh,
-                               int ctx_add, int share) {
+                               int ctx_add, int share, bool wide) {
   dim3 grid(B * Hkv * nch, n_split);
   const int maxg = (G <= 4 && nch == 1) ? 4 : 16;
   // paired-tile variant (NT=2): 2x KV bytes in flight per wave — the
@@ -238,13 +238,20 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
               maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
               share);
     } else if (D <= 128 && pf) {
-      attn_decode_mfma_kernel<D, decltype(mg)::value, 1, 1>
-          <<<grid, 256, 0, cur_stream()>>>(
-              bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
-              ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
-              pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
-              maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
-              share);
+      auto go = [&](auto waves) {
+        constexpr int NW = decltype(waves)::value;
+        attn_decode_mfma_kernel<D, decltype(mg)::value, 1, 1, NW>
+            <<<grid, NW * 64, 0, cur_stream()>>>(
+                bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(),
+                ctx.data_ptr<int>(), alibi_ptr, bf_ptr_mut(out),
+                pml.data_ptr<float>(), pacc.data_ptr<float>(), B, Hkv, G, nch, P,
+                maxp, n_split, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add,
+                share);
+      };
+      if constexpr (decltype(mg)::value == 4) {
+        if (wide) return go(std::integral_constant<int, 8>{});
+      }
+      go(std::integral_constant<int, 4>{});
     } else if (D <= 128 && nt2) {
       attn_decode_mfma_kernel<D, decltype(mg)::value, 2>
           <<<grid, 256, 0, cur_stream()>>>(
@@ -296,6 +303,7 @@ static torch::Tensor attn_decode_core(
   // shorter splits idle most of them. They share 32 where D = 512 (8 sequences of 300, 16
   // heads on 8: 31.6 us with splits of 128, 18.7 so).
   int share = n_split > 0 ? 1 : D == 512 ? 32 : 128;
+  bool wide = false;
   if (n_split <= 0) {
     // measured optimum (benchmarks/bench_kernels.py attn_decode): size the
     // grid for full residency — NT=1 runs 118 VGPRs -> 4 WGs/CU (1024 WGs),
@@ -313,7 +321,19 @@ static torch::Tensor attn_decode_core(
     const long target = (pf_env0 && D <= 128) ? 512
                         : (nt_env0 >= 2 && D <= 128) ? 768 : 1024;
     const long units = std::max(1, B * Hkv * nch), room = (long)maxp * P;
-    if (units > target) {
+    // Workgroups of eight waves with twice the tokens halve the splits to fold. They pay
+    // where those still fill the chip as well, or where one does without any fold. us in
+    // a graph, four waves and eight, heads of 128, 8 of keys: 1 sequence of 300 tokens 9.3,
+    // 7.9; 500 8.6, 10.7; 4 of 1000 12.1, 13.1; 2000 16.7, 14.4; 2 of 2000 12.8, 13.2; 4000
+    // 17.2, 15.0; 8 of 1000 14.9, 14.0; 8000 52.1, 48.5; 16 of 300 11.0, 9.0; 500 13.3, 12.9;
+    // 2000 28.8, 28.3; 32 of 300 14.1, 10.5; 2000 48.2, 45.1.
+    wide = pf_env0 && D <= 128 && G <= 4 && units <= 256 &&
+           ((room >= 256 && room <= 352) ||
+            (units * room >= 60000 && 256 / units * 2 >= target / units));
+    if (wide) {
+      share = 256;
+      n_split = (int)std::max(1L, std::min({32L, 256 / units, room / share}));
+    } else if (units > target) {
       // More units than fit at once: contexts of a large batch differ, and a
       // workgroup with a long one outlasts the rest. Shares of 1024 tokens even it
       // out (97 sequences of 64 to 4000 tokens, 8 heads of 128: 168 us unsplit,
@@ -338,7 +358,7 @@ static torch::Tensor attn_decode_core(
     attn_decode_launch<decltype(d)::value>(
         q, k_pages, v_pages, page_table, ctx_lens, alibi_ptr, out, pml, pacc,
         B, Hkv, G, nch, P, maxp, n_split, (int)window, (float)scale, q_off,
-        q_sb, q_sh, out_sb, out_sh, ctx_add, share);
+        q_sb, q_sh, out_sb, out_sh, ctx_add, share, wide);
   };
   if (D == 128) go(std::integral_constant<int, 128>{});
   else if (D == 64) go(std::integral_constant<int, 64>{});

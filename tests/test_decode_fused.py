@@ -194,6 +194,12 @@ def test_octets_of_tokens(B, T, Hq, Hkv, D, P, norms):
     (2, 8, 2, 128, 4096, [5, 4096]),          # a short context in a wide table
     (1, 71, 1, 64, 2000, [777]),              # a group in five chunks
     (65, 8, 8, 64, 2100, None),               # more units than fit: even shares
+    (3, 16, 8, 128, 264, [264, 1, 257]),      # eight waves: one split
+    (3, 8, 8, 64, 336, [330, 31, 256]),
+    (16, 32, 8, 128, 480, None),              # a split of two that is not there
+    (2, 16, 8, 128, 4000, [4000, 511]),       # one of many
+    (32, 8, 8, 32, 240, None), (32, 32, 8, 64, 1000, None),
+    (24, 8, 8, 128, 600, None), (17, 8, 8, 128, 600, None),   # two tiles and more a wave
 ])
 @pytest.mark.parametrize("P", [8, 16, 24])        # 24: pages found by division
 def test_decode_attention_splits(B, Hq, Hkv, D, room, lengths, P):
