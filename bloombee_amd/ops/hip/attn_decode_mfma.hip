@@ -21,9 +21,9 @@
 // LDS is only used for the P^T C->B relayout (tiny) and the final 4-wave
 // merge, so occupancy is VGPR-limited, not LDS-limited.
 //
-// Work decomposition: grid = (B*Hkv*nch, n_split) flash-decode splits, 4
-// waves per workgroup; wave w owns KV tiles (32 positions) w, w+4, w+8, ...
-// of its split, with a final 4-way LDS merge of (m, l, acc). V fragment
+// Work decomposition: grid = (B*Hkv*nch, n_split) flash-decode splits, NW = 4
+// or 8 waves per workgroup; wave w owns KV tiles (32 positions) w, w+NW, ...
+// of its split, with a final merge of the waves' (m, l, acc) in LDS. V fragment
 // loads are issued BEFORE the QK^T/softmax phase so their HBM latency is
 // covered (measured: moving them later costs ~35%).
 

@@ -861,7 +861,8 @@ static bool stream_sums(long M, long N, long K) {
   const long rounds = (N / 16 + 255) / 256;
   const bool full = N * 5 >= rounds * 4096 * 4;
   // One round: few columns leave it too little to hide a long chain over K, the more so the
-  // more rows. 1024 x 3072: 1 row 5.6, 7.3; 32 rows 7.3, 8.6. 4096 x 14336: 23.8, 28.7; 16
+  // more rows (up to 8 of few columns have another form, stream_parts, not in these figures).
+  // 1024 x 3072: 1 row 5.6, 7.3; 32 rows 7.3, 8.6. 4096 x 14336: 23.8, 28.7; 16
   // rows 27.6, 28.8. 2048 x 8192: 1 row 11.2, 12.5; 16 rows 14.4, 13.3. 512 x 14336: 16.1,
   // 15.4; 22.5, 16.2.
   if (rounds == 1) return K * (192 * (M + 16) - N) <= 192L << 17;
