@@ -385,13 +385,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
         if nw is None:
             nw = torch.ones(x.shape[-1], dtype=x.dtype, device=x.device)
         x = rms_norm(x, nw, norm[1])
-    if ss_out is None and rows_ok(x, w) and all(
-            t is None or (t.dtype == torch.bfloat16 and t.device == x.device
-                          and not t.requires_grad and _plain(t) and t.numel() == n)
-            for t, n in ((bias, N), (residual, M * N))):
+    if (ss_out is None and rows_ok(x, w)
+            and (bias is None or bias.dim() == 1 and _addend(bias, x, N))
+            and (residual is None or _addend(residual, x, M * N))):
         return hip_ops.gemm_rows(
             x.contiguous(), w,
-            None if residual is None else residual.contiguous(),
+            None if residual is None else
+            residual.view(*x.shape[:-1], N).contiguous(),
             None if bias is None else bias.contiguous())
     y = torch.nn.functional.linear(x, w, bias)
     if residual is not None:
@@ -400,6 +400,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
         raise RuntimeError("ss_out requires the GPU skinny-GEMM path "
                            "(callers gate on fuse_norm_linear_ok)")
     return y
+
+
+def _addend(t: torch.Tensor, x: torch.Tensor, n: int) -> bool:
+    """gemm_rows.hip adds these n values to a product of x; no tangent is lost."""
+    return (t.dtype == torch.bfloat16 and t.device == x.device
+            and not t.requires_grad and _plain(t) and t.numel() == n
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
 
 
 def _rows_take(x: torch.Tensor, w: torch.Tensor) -> bool:

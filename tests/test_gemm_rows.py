@@ -173,6 +173,33 @@ def test_not_finite():
     assert torch.allclose(got[some], want[some], rtol=2.0 ** -7, atol=1e-3)
 
 
+def test_addends_are_torchs():
+    """What is added keeps its tangent and broadcasts, or is refused, as torch has it."""
+    import torch.autograd.forward_ad as fwd
+    M, N, K = 64, 64, 256
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    r, t = draw(M, N, seed=3), draw(M, N, seed=4)
+    assert ops.hip_ops.rows_wins(M, N, K)
+    with fwd.dual_level():
+        y = fwd.unpack_dual(ops.linear(x, w, residual=fwd.make_dual(r, t)))
+        assert torch.equal(y.tangent, t)
+        y = fwd.unpack_dual(ops.linear(x, w, bias=fwd.make_dual(r[0], t[0])))
+        assert torch.equal(y.tangent, t[0].expand(M, N))
+    rows = draw(M, 1, seed=5)                # one value a row
+    assert close(ops.linear(x, w, bias=rows), x.double() @ w.double().T + rows.double(),
+                 x.double().abs() @ w.double().abs().T + rows.double().abs())
+    apart = draw(2, M, N // 2, seed=6).transpose(0, 1)   # no view of (M, N)
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w, residual=apart)
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w[:32], bias=rows[:32])
+    # any other layout of the right shape, and any shape of the right values
+    for res in (draw(N, M, seed=8).T, draw(M * N, seed=9), draw(M, 2 * N, seed=9)[:, N:]):
+        assert close(ops.linear(x, w, residual=res),
+                     x.double() @ w.double().T + res.reshape(M, N).double(),
+                     x.double().abs() @ w.double().abs().T + res.reshape(M, N).double().abs())
+
+
 def test_views():
     """Rows at any address and of any stride, weights that do not begin at 16 bytes."""
     M, N, K = 64, 256, 320
