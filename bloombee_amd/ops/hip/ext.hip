@@ -966,7 +966,7 @@ torch::Tensor gemm_stream(torch::Tensor A, torch::Tensor W,
                 bias->is_contiguous() && bias->numel() == a.N, "bad bias");
     a.bias = bf_ptr(*bias);
   }
-  if (a.M == 0) return C;
+  if (a.M == 0 || a.N == 0) return C;
   const int parts = eps < 0 ? stream_parts(a.M, a.N, a.K) : 0;
   if (parts) {
     if (parts == 4)
@@ -1051,7 +1051,7 @@ static bool few_swiglu(long M, long N, long K) {
 // 19.4, 15.9. 20480 x 5120: 4 44.1, 47.0; 16 58.1, 49.2. 4096 x 4096: 16 10.3, 11.4; 18176 x
 // 4096, 284 workgroups: 17 rows 36.3, 39.6. 1024 x 3072: any 5.6 to 7.2, 6.8 to 7.6.
 static bool few_sums(long M, long N, long K) {
-  if (M <= 0 || M > 32 || K % 128 || K < 1024 || N % 8) return false;
+  if (M <= 0 || M > 32 || K % 128 || K < 1024 || N <= 0 || N % 8) return false;
   if (K >= 1 << 20 || N >= 1 << 24) return false;   // rows_args
   if (!stream_sums(M, N, K)) return true;
   const long wgs = ldiv_up(N, 64) * few_splits(N, K);
@@ -1406,7 +1406,7 @@ static RowsPlan rows_plan(long M, long N, long K, bool swiglu) {
 //   8192 x 28672: 97 195, 98; 450 301, 210; 617 248, 269; 57344 x 8192: 200 194, 242
 //   1024 x 3072: any 20 (the host's time), 9 to 19
 static bool rows_wins(long M, long N, long K) {
-  if (M <= 32 || N % 8 || K % 64 || K < 256 || K >= 1 << 20) return false;
+  if (M <= 32 || N <= 0 || N % 8 || K % 64 || K < 256 || K >= 1 << 20) return false;
   return M * N <= (M <= 384 ? 11200000 : 6000000) && (K <= 16384 || M <= 512);
 }
 
@@ -1414,7 +1414,8 @@ static bool rows_wins(long M, long N, long K) {
 // once more, which counts the more the shorter K is. 28672 x 4096: 333 rows 73 us (72 +
 // 7), 450 116 (106), 768 159 (185), 1400 288 (294), 2800 483 (607), 16384 2674 (2891).
 static bool rows_swiglu_wins(long M, long N, long K) {
-  if (M <= 32 || N % 16 || K % 64 || K < 256 || (M > 1024 && K > 5120)) return false;
+  if (M <= 32 || N <= 0 || N % 16 || K % 64 || K < 256 || (M > 1024 && K > 5120))
+    return false;
   if (K >= 1 << 20 || M >= 1 << 24 || N >= 1 << 24) return false;   // rows_args
   const double library = std::max(2e-6 * M * N * K / 1.2e3, (N + M) * K * 2 / 4.7e6);
   return rows_plan(M, N, K, true).us * 1.07 < library + M * N * 3 / 5e6 + 3;

@@ -209,7 +209,7 @@ static RowsPlan grad_plan(long M, long N, long K) {
 // not: 28672 x 4096, 3998 rows 706, 674; 16384 2842, 2818. 4096 x 14336: 3998 393, 376;
 // 16384 1485, 1388. 6144 x 4096: 159, 150; 625, 591. 4096 x 4096: 112, 103; 425, 400.
 static bool linear_grad_wins(long M, long N, long K) {
-  return N % 64 == 0 && K % 256 == 0 &&
+  return N > 0 && N % 64 == 0 && K > 0 && K % 256 == 0 &&
          (M >= 3000 ||
           (M * K <= 8500000 && (M <= 512 || M * K * N <= 150000000000L)));
 }

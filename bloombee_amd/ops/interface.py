@@ -356,7 +356,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
     # residual/bias epilogue the blaslt path would re-emit as a separate
     # eager kernel.
     if (_on_gpu(x) and M <= 32 and x.dtype == torch.bfloat16
-            and K % 256 == 0 and N % 64 == 0):
+            and K % 256 == 0 and N % 64 == 0 and N > 0):
         _require_ext()
         if (norm is None and ss_in is None and ss_out is None
                 and w.data_ptr() % 16 == 0 and hip_ops.few_sums(M, N, K)):

@@ -200,6 +200,19 @@ def test_addends_are_torchs():
                      x.double().abs() @ w.double().abs().T + res.reshape(M, N).double().abs())
 
 
+@pytest.mark.parametrize("M", [1, 8, 20, 64])
+@pytest.mark.parametrize("K", [256, 2048])
+def test_weights_without_rows(M, K):
+    x, w = draw(M, K, seed=1), draw(0, K, seed=2)
+    assert ops.linear(x, w).shape == (M, 0)
+    assert ops.hip_ops.gemm_stream(x[:32], w, None, None, -1.0).shape == (min(M, 32), 0)
+    x.requires_grad_(True)
+    dx, = torch.autograd.grad(training.linear(x, w).sum(), x)
+    assert dx.shape == x.shape and not dx.any()
+    torch.cuda.synchronize()
+    assert not draw(M, K, seed=1).isnan().any()     # no error is left for the next call
+
+
 def test_views():
     """Rows at any address and of any stride, weights that do not begin at 16 bytes."""
     M, N, K = 64, 256, 320
