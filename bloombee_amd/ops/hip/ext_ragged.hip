@@ -846,10 +846,11 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
   if (ta == at::kBFloat16 && (long)N * K >= 1L << 31) {
     // a row's place in bytes has 32 bits
     const int n = N / 2;
+    const Tensor wt = wts.view({N, top});
     return torch::cat(
         {moe_experts(h.slice(0, 0, n), up, down, ids.slice(0, 0, n),
-                     wts.slice(0, 0, n), win, limit, slope, shift, stepwise),
-         moe_experts(h.slice(0, n), up, down, ids.slice(0, n), wts.slice(0, n), win,
+                     wt.slice(0, 0, n), win, limit, slope, shift, stepwise),
+         moe_experts(h.slice(0, n), up, down, ids.slice(0, n), wt.slice(0, n), win,
                      limit, slope, shift, stepwise)});
   }
   auto y = torch::empty({N, top, Wp}, h.options());

@@ -175,3 +175,31 @@ def test_order_of_unusual_logits(bits):
     _, _, ids, wts = ops.hip_ops.norm_route(a, None, None, router, 5, 0.0)
     assert ids[0].tolist() == [0, 1, 3, 2, 4]
     assert bool(((wts - 0.2).abs() <= 2.0 ** -10).all())
+
+
+@pytest.mark.parametrize("flat", [False, True])
+def test_more_rows_than_32_bits_of_bytes_reach(flat):
+    """Batches of 2^32 bytes are taken in parts, weights laid out (N, top) or not."""
+    N, K, top = 1 << 15, 1 << 16, 2
+    h = torch.zeros(N, K, dtype=torch.bfloat16, device=DEV)
+    at = torch.tensor([0, 1, N // 2 - 1, N // 2, N - 2, N - 1], device=DEV)
+    h[at] = draw(len(at), K, seed=1)
+    up = draw(2, 1, 64, K, seed=2, scale=K ** -0.5)
+    down = draw(2, 64, 64, seed=3, scale=0.125)
+    gen = torch.Generator().manual_seed(4)
+    ids = torch.rand(N, 2, generator=gen).argsort(1).int().to(DEV)
+    wts = torch.rand(N, top, generator=gen).to(DEV)
+    got = ragged._ext().moe_experts(h, up, down, ids, wts.flatten() if flat else wts,
+                                    False, 0.0, 1.0, 0.0, False)
+    x, e = h[at].double(), ids[at].long()
+    act = torch.relu(torch.einsum("nk,etk->net", x, up[:, 0].double())).square()
+    act = act[torch.arange(len(at), device=DEV)[:, None], e]         # (n, top, 64)
+    back = down.double()[e]                                          # (n, top, 64, 64)
+    w = wts[at].double()[..., None]
+    want = w * (back * act[:, :, None]).sum(-1)
+    # an activation and its row are rounded to 16 bits, 2^-9 of each
+    tol = 2.0 ** -8 * (want.abs() + w * (back.abs() * act[:, :, None]).sum(-1))
+    assert bool(((got[at].double() - want).abs() <= tol + 1e-6).all())
+    zero = torch.ones(N, dtype=torch.bool, device=DEV)
+    zero[at] = False
+    assert not got[zero].any()
