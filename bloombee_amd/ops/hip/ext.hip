@@ -1012,12 +1012,16 @@ static void launch_skinny_fused(const StreamArgs& a, int kchunk, int ksplit,
 // lines and by DMA, up to 48 KB ahead a workgroup, and its rows of A once for 64 columns.
 typedef RowsTile<32, 64, 2, 1, 2, 3, 2> FewRows;
 
-// Splits of K that let all CUs take part, one or two workgroups each.
+// Splits of K that let all CUs take part, one or two workgroups each, and do not meet in
+// the channels of memory (two splits of up to 8192 do no harm: 8192 x 8192, 32 rows 32.8
+// with 2, 34.4 with 3).
 static int few_splits(long N, long K) {
   const long wgs = ldiv_up(N, 64);
   int best = 1;
   float most = 0.f;
   for (int s = 1; s <= 16 && (s == 1 || (wgs * s <= 512 && K / s >= 512)); ++s) {
+    if (s > 1 && (K > 8192 || s > 2) && same_channels(K, ldiv_up(K / 128, s) * 128))
+      continue;
     const float fill = wgs * s / (256.f * ldiv_up(wgs * s, 256));
     if (fill > most + .02f) {
       most = fill;
@@ -1044,18 +1048,20 @@ static bool few_swiglu(long M, long N, long K) {
 
 // Whether it beats their sums: wherever those want the split form (whose waves take W by
 // 64 B of a row), and from some rows on where the one-launch form reads all of A for every
-// 16 columns. us in a graph, those and this: 4096 x 14336: 8 rows 25.1, 25.7; 16 30.0,
-// 25.7; 32 31.5, 25.2. 5120 x 13824: 1 row 35.3, 29.5; 32 39.4, 30.6. 28672 x 4096: 44.2,
-// 43.6; 16 48.4, 44.5. 512 x 14336: 13.3, 8.2. 8192 x 28672: 32 rows 99.2, 91.5. 151936 x
-// 1024: 16 rows 64.3, 60.6. One launch: 6144 x 4096: 4 rows 14.4, 14.4; 16 16.5, 15.0; 32
-// 19.4, 15.9. 20480 x 5120: 4 44.1, 47.0; 16 58.1, 49.2. 4096 x 4096: 16 10.3, 11.4; 18176 x
-// 4096, 284 workgroups: 17 rows 36.3, 39.6. 1024 x 3072: any 5.6 to 7.2, 6.8 to 7.6.
+// 16 columns. us in a graph, W from memory, those and this: 4096 x 14336: 9 rows 25.4, 25.7;
+// 16 28.4, 25.8; 32 30.9, 26.1. 5120 x 13824: 1 row 36.0, 29.9; 32 40.1, 31.1. 28672 x 4096:
+// 44.2, 43.6; 16 48.4, 44.5. 512 x 14336: 15.1, 9.3. 8192 x 28672: 17 rows 99.7, 84.8; 32
+// 104.6, 86.4. 151936 x 1024: 16 rows 64.3, 60.6. One launch: 6144 x 4096: 4 rows 14.4, 14.4;
+// 16 16.5, 15.0; 32 19.4, 15.9. 20480 x 5120: 4 44.1, 47.0; 16 58.1, 49.2. 4096 x 4096: 16
+// 10.3, 11.4; 18176 x 4096, 284 workgroups: 17 rows 36.3, 39.6. 1024 x 3072: any 5.6 to 7.2,
+// 6.8 to 7.6. Up to 12 rows of few columns or long K that form keeps up: 9 rows, 4096 x 8192
+// 15.5, 17.2; x 16384 30.2, 32.4; 12288 x 16384 76.4, 89.3; but 10240 x 8192 40.4, 37.9.
 static bool few_sums(long M, long N, long K) {
   if (M <= 0 || M > 32 || K % 128 || K < 1024 || N <= 0 || N % 8) return false;
   if (K >= 1 << 20 || N >= 1 << 24) return false;   // rows_args
   if (!stream_sums(M, N, K)) return true;
   const long wgs = ldiv_up(N, 64) * few_splits(N, K);
-  return M > 8 && N * K >= 24L << 20 && K >= 3072 &&
+  return M > 8 && (M > 12 || (N > 4096 && K <= 8192)) && N * K >= 24L << 20 && K >= 3072 &&
          wgs * 10 >= ldiv_up(wgs, 256) * 256 * 6;
 }
 
@@ -1591,6 +1597,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("add_experts", &add_experts);
   m.def("gemm_stream", &gemm_stream);
   m.def("few_sums", &few_sums);
+  m.def("few_splits", &few_splits);
   m.def("few_swiglu", &few_swiglu);
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);

@@ -195,7 +195,7 @@ static RowsPlan grad_plan(long M, long N, long K) {
       GRAD_TILES(X)
 #undef X
   };
-  return rows_best(tiles, 7, M, K, N, false);
+  return rows_best(tiles, 7, M, K, N, false, true);
 }
 
 // Whether linear_grad beats the library's GEMM, which leaves CUs idle where the result

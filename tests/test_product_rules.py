@@ -17,3 +17,30 @@ def test_weights_without_rows_stay_torchs(M, K):
     h = ops.hip_ops
     assert not (h.rows_wins(M, 0, K) or h.rows_swiglu_wins(M, 0, K)
                 or h.few_sums(M, 0, K) or grad_wins(M, 0, K))
+
+
+@pytest.mark.parametrize("N,K,splits", [
+    (8192, 28672, 4), (7168, 28672, 4), (8192, 16384, 3), (4096, 8192, 8),
+    (4096, 14336, 4), (8192, 8192, 2), (5120, 13824, 3), (512, 14336, 16), (16384, 4096, 1)])
+def test_splits_begin_in_channels_of_their_own(N, K, splits):
+    """Up to 32 rows: splits fill the chip, but do not begin a multiple of 4 KiB apart
+    where rows of W do (two of up to 8192 columns may)."""
+    assert ops.hip_ops.few_splits(N, K) == splits
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 8192, 8192), (64, 8192, 8192), (80, 8192, 8192),
+                                   (128, 8192, 8192), (33, 14336, 4096), (64, 16384, 4096),
+                                   (48, 12288, 12288), (112, 8192, 4096)])
+def test_tiles_begin_in_channels_of_their_own(M, N, K):
+    tile, splits = ops.hip_ops.rows_plan(M, N, K, False)
+    stages = K // (128 if tile == 9 else 64)     # the last tile takes twice the columns
+    columns = -(-stages // splits) * K // stages
+    assert splits == 1 or columns % 2048
+
+
+@pytest.mark.parametrize("M,N,K,tiles", [
+    (9, 4096, 8192, False), (12, 4096, 14336, False), (13, 4096, 14336, True),
+    (9, 12288, 16384, False), (12, 8192, 28672, False), (17, 8192, 28672, True),
+    (9, 10240, 8192, True), (8, 10240, 8192, False), (1, 5120, 13824, True)])
+def test_some_rows_with_long_sums(M, N, K, tiles):
+    assert ops.hip_ops.few_sums(M, N, K) == tiles
