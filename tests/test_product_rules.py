@@ -44,3 +44,11 @@ def test_tiles_begin_in_channels_of_their_own(M, N, K):
     (9, 10240, 8192, True), (8, 10240, 8192, False), (1, 5120, 13824, True)])
 def test_some_rows_with_long_sums(M, N, K, tiles):
     assert ops.hip_ops.few_sums(M, N, K) == tiles
+
+
+@pytest.mark.parametrize("M,N,K,plan", [
+    (193, 6144, 4096, (6, 2)), (300, 4672, 4544, (6, 2)), (288, 18176, 4544, (1, 1)),
+    (617, 1024, 2048, (9, 1))])
+def test_low_tiles_cost_what_they_take_from_memory(M, N, K, plan):
+    """Where the two lowest tiles looked the cheapest and were not."""
+    assert ops.hip_ops.rows_plan(M, N, K, False) == plan
