@@ -59,7 +59,17 @@ def _no_function_mode() -> bool:
                    for m in torch.overrides._get_current_function_mode_stack()))
 
 
-def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+def _unwatched() -> bool:
+    """Nothing traces torch's operations, replaces them or runs them in other types."""
+    return (not torch.is_autocast_enabled("cuda")
+            and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0
+            and _no_function_mode()
+            and torch._C._functorch.peek_interpreter_stack() is None)
+
+
+def _readable(x: torch.Tensor, *weights: torch.Tensor) -> bool:
     """The kernels take these: weights are frozen. They are launched on the current
     device's stream: tensors of another device are left to torch, which switches."""
     return (x.is_cuda and x.numel() > 0
@@ -68,14 +78,12 @@ def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
                     for t in (x, *weights))
             and all(w.device == x.device and not w.requires_grad
                     for w in weights)
-            and not torch.is_autocast_enabled("cuda")
-            and not torch.jit.is_tracing()
-            and not torch.compiler.is_compiling()
-            and torch._C._len_torch_dispatch_stack() == 0
-            and _no_function_mode()
-            and torch._C._functorch.peek_interpreter_stack() is None
             and all(torch.autograd.forward_ad.unpack_dual(t).tangent is None
                     for t in (x, *weights)))
+
+
+def _fused(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    return _unwatched() and _readable(x, *weights)
 
 
 # ---------------------------------------------------------------------------
@@ -409,23 +417,26 @@ def _addend(t: torch.Tensor, x: torch.Tensor, n: int) -> bool:
             and torch.autograd.forward_ad.unpack_dual(t).tangent is None)
 
 
-def _rows_take(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """gemm_rows.hip reads these, and nobody records or watches the product."""
-    return (HAVE_HIP_OPS and x.is_cuda and x.dtype == w.dtype == torch.bfloat16
+def _rows_take(x: torch.Tensor, w: torch.Tensor, wins, n: int) -> bool:
+    """gemm_rows.hip reads these, nobody records or watches the product, and the rule
+    says that n columns are faster so. What rules out most calls is asked first: the
+    rule takes 0.5 us of the host, the tensors 3."""
+    return (x.is_cuda and x.dtype == w.dtype == torch.bfloat16
             and w.dim() == 2 and x.dim() >= 2 and x.shape[-1] == w.shape[1]
-            and w.is_contiguous() and w.data_ptr() % 16 == 0 and _fused(x, w))
+            and x.numel() > 32 * w.shape[1] and _unwatched()
+            and wins(x.numel() // w.shape[1], n, w.shape[1])
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and _readable(x, w)
+            and not (x.requires_grad and torch.is_grad_enabled()))
 
 
 def rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """x @ w^T of tensors without gradients is faster on the tiles of gemm_rows.hip."""
-    return (_rows_take(x, w) and not (x.requires_grad and torch.is_grad_enabled())
-            and hip_ops.rows_wins(x.numel() // x.shape[-1], *w.shape))
+    return HAVE_HIP_OPS and _rows_take(x, w, hip_ops.rows_wins, w.shape[0])
 
 
 def rows_glu_ok(x: torch.Tensor, w: torch.Tensor, ff: int) -> bool:
     """A gated product of ff activations of x @ w^T is faster in one launch."""
-    return (_rows_take(x, w) and not (x.requires_grad and torch.is_grad_enabled())
-            and hip_ops.rows_swiglu_wins(x.numel() // x.shape[-1], 2 * ff, w.shape[1]))
+    return HAVE_HIP_OPS and _rows_take(x, w, hip_ops.rows_swiglu_wins, 2 * ff)
 
 
 def linear_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

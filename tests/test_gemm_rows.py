@@ -213,6 +213,25 @@ def test_weights_without_rows(M, K):
     assert not draw(M, K, seed=1).isnan().any()     # no error is left for the next call
 
 
+def test_sizes_are_asked_first(monkeypatch):
+    """Products that the rules leave to others do not pay for a look at their tensors."""
+    from bloombee_amd.ops import interface, ragged
+
+    def look(*tensors):
+        raise AssertionError("looked at")
+    monkeypatch.setattr(interface, "_readable", look)
+    b = torch.zeros(1024, device=DEV)
+    for M in (1, 8, 32):       # a decode step's rows
+        x, w = draw(M, 256, seed=1), draw(2048, 256, seed=2)
+        ragged.linear_glu(x, w, 1024, 1024, b, b, 1.5, 1.702, 1024, torch.bfloat16)
+        ops.linear_gated(x, w)
+        ops.linear(x, w)
+    x, w = draw(64, 264, seed=1), draw(2048, 264, seed=2)     # K % 64
+    ops.linear_gated(x, w)
+    with pytest.raises(AssertionError):
+        ops.linear(draw(64, 256, seed=1), draw(2048, 256, seed=2))
+
+
 def test_views():
     """Rows at any address and of any stride, weights that do not begin at 16 bytes."""
     M, N, K = 64, 256, 320
