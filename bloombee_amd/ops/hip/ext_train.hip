@@ -199,18 +199,21 @@ static RowsPlan grad_plan(long M, long N, long K) {
 }
 
 // Whether linear_grad beats the library's GEMM, which leaves CUs idle where the result
-// has few tiles. us, library and here, rows of w x columns:
-//   28672 x 4096: 33 rows 160, 45; 128 142, 52; 450 283, 112; 900 307, 195; 1400 302, 308
-//   4096 x 14336: 33 35, 25; 450 65, 56; 768 87, 88; 1700 163, 181
-//   6144 x 4096: 33 29, 14; 450 52, 37; 1400 72, 69; 2000 92, 83
-//   4096 x 4096: 450 38, 29; 2000 64, 57.  8192 x 28672: 333 159, 189; 900 382, 390
-//   57344 x 8192: 128 297, 170; 450 538, 402; 617 528, 535; 900 695, 738
+// has few tiles. us in a graph, w from memory, library and here, rows of w x columns:
+//   28672 x 4096: 1 row 146, 47; 33 160, 48; 128 143, 57; 450 276, 110; 1024 344, 186; 1400
+//   305, 330;  38400 x 4096: 1024 460, 247;  57344 x 4096: 1024 532, 351
+//   4096 x 14336: 1 29, 26; 33 37, 27; 450 67, 59; 768 87, 81; 1700 165, 174
+//   6144 x 4096: 1 34, 14; 33 29, 15; 450 54, 38; 1400 73, 70; 2000 95, 84; 2500 107, 111
+//   4096 x 4096: 450 39, 30; 2000 67, 58; 2500 75, 78;  1024 x 2048: 1 6, 8; 64 9, 8
+//   8192 x 28672: 200 143, 129; 333 161, 178; 900 369, 349
+//   57344 x 8192: 128 298, 172; 333 351, 369; 450 543, 362; 513 501, 515; 900 742, 685
 // Its form for rows of w to sum over is 4 to 8% slower than that for columns, these are
-// not: 28672 x 4096, 3998 rows 706, 674; 16384 2842, 2818. 4096 x 14336: 3998 393, 376;
-// 16384 1485, 1388. 6144 x 4096: 159, 150; 625, 591. 4096 x 4096: 112, 103; 425, 400.
+// not, but take tiles of 256 x 256, and 3000 rows of few columns leave a quarter of the
+// chip idle: 28672 x 4096, 3000 rows 550, 600; 4000 700, 660; 8000 1392, 1337. 4096 x 14336:
+// 3000 315, 284; 8000 737, 682. 6144 x 4096: 3000 125, 128; 4000 158, 149; 8000 305, 287.
 static bool linear_grad_wins(long M, long N, long K) {
   return N > 0 && N % 64 == 0 && K > 0 && K % 256 == 0 &&
-         (M >= 3000 ||
+         (M >= 3000 || (M <= 1024 && N >= 4 * K && K <= 5120) ||
           (M * K <= 8500000 && (M <= 512 || M * K * N <= 150000000000L)));
 }
 

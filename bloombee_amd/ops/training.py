@@ -232,17 +232,16 @@ def swiglu(gu: torch.Tensor) -> torch.Tensor:
 # frozen projections
 # ---------------------------------------------------------------------------
 
-def _few_rows(M: int, N: int, K: int) -> bool:
-    """Whether the split sum along N, (M, N) @ (N, K), beats the library's GEMM also
-    for N in 32s, which leaves most of the chip idle where the result has few tiles.
-    us, split and library, N x K:
-    28672 x 4096: 33 rows 53, 164; 128 67, 145; 450 156, 279; 1024 296, 360;
-        2000 554, 414
-    20480 x 5120: 300 rows 127, 137; 900 277, 268 (160 tiles)
-    57344 x 8192: 128 rows 192, 298; 300 481, 398
-    6144 x 4096:  33 rows 21, 25; 128 31, 46; 450 50, 48
-    4096 x 4096:  33 rows 17, 22; 128 24, 34; 200 32, 26"""
-    if N % 32 or K % 256:
+def _half_steps(M: int, N: int, K: int) -> bool:
+    """Whether the split sum along N, (M, N) @ (N, K), beats the library's GEMM for
+    rows of w that come in 32s and not in 64s (gemm_grad.hip). us, split and library,
+    N x K:
+    28704 x 4096: 1 row 52, 146; 33 57, 163; 128 73, 155; 450 161, 297; 1000 285, 371;
+        1200 385, 374
+    6176 x 2048: 33 rows 20, 33; 128 25, 33; 200 31, 34
+    4128 x 1024: 33 rows 15, 15; 128 20, 19; 300 24, 23
+    2080 x 512: any 12 to 24, 9 to 16, where a call is 20 us of the host's time"""
+    if N % 64 != 32 or K % 256:
         return False
     tiles = -(-M // 128) * (K // 256)
     return (M <= 128 and N >= K
@@ -250,7 +249,7 @@ def _few_rows(M: int, N: int, K: int) -> bool:
 
 
 def _split_gradient(M: int, N: int, K: int) -> bool:
-    return _ext().linear_grad_wins(M, N, K) or _few_rows(M, N, K)
+    return _ext().linear_grad_wins(M, N, K) or _half_steps(M, N, K)
 
 
 class _Linear(torch.autograd.Function):
@@ -272,21 +271,15 @@ class _Linear(torch.autograd.Function):
         return dx.view(*g.shape[:-1], w.shape[1]), None
 
 
-class _Product(_Linear):
-    """The same beyond the sizes that _few_rows names."""
-
-
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x @ w^T; w is frozen where the gradient kernel is to take part."""
     if (torch.is_grad_enabled() and x.requires_grad and _fused(x, w)
             and w.dim() == 2 and x.dim() >= 2 and x.shape[-1] == w.shape[1]
             and w.is_contiguous()):
         M = x.numel() // x.shape[-1]
-        if _few_rows(M, *w.shape):
-            return _Linear.apply(x, w)
         if (interface.hip_ops.rows_wins(M, *w.shape)
-                or _ext().linear_grad_wins(M, *w.shape)):
-            return _Product.apply(x, w)
+                or _split_gradient(M, *w.shape)):
+            return _Linear.apply(x, w)
     return F.linear(x, w)
 
 

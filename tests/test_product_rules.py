@@ -52,3 +52,33 @@ def test_some_rows_with_long_sums(M, N, K, tiles):
 def test_low_tiles_cost_what_they_take_from_memory(M, N, K, plan):
     """Where the two lowest tiles looked the cheapest and were not."""
     assert ops.hip_ops.rows_plan(M, N, K, False) == plan
+
+
+@pytest.mark.parametrize("M,N,K,wins", [
+    (1, 64, 256, True), (1, 96, 256, False), (1, 64, 320, False),       # N % 64, K % 256
+    (512, 4096, 16384, True), (513, 4096, 16384, True), (519, 4096, 16384, False),
+    (512, 28672, 8192, True), (513, 57344, 8192, False), (638, 28672, 8192, True),
+    (639, 28672, 8192, False),                                          # M * K * N
+    (1024, 57344, 4096, True), (1025, 57344, 4096, False), (1024, 16384, 4096, True),
+    (2999, 4096, 4096, False), (3000, 4096, 4096, True),
+    (3000, 12288, 4096, True)])
+def test_gradients_at_the_rule(M, N, K, wins):
+    assert grad_wins(M, N, K) == wins
+
+
+@pytest.mark.parametrize("M,N,K,wins", [
+    (128, 288, 256, True), (129, 288, 256, False), (128, 256, 256, False),
+    (1024, 28704, 4096, True), (1025, 28704, 4096, False), (1024, 28704, 5120, False),
+    (128, 224, 256, False), (129, 1056, 256, True), (64, 96, 320, False)])
+def test_gradients_of_32_rows_at_the_rule(M, N, K, wins):
+    from bloombee_amd.ops import training
+    assert training._half_steps(M, N, K) == wins
+
+
+@pytest.mark.parametrize("M,N,K,wins", [
+    (32, 256, 256, False), (33, 256, 256, True), (64, 252, 256, False),
+    (64, 256, 192, False), (64, 256, 288, False), (384, 29160, 4096, True),
+    (384, 29168, 4096, False), (385, 15576, 4096, True), (385, 15592, 4096, False),
+    (512, 64, 16448, True), (513, 64, 16448, False), (513, 64, 16384, True)])
+def test_products_at_the_rule(M, N, K, wins):
+    assert ops.hip_ops.rows_wins(M, N, K) == wins

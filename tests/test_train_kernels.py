@@ -157,13 +157,21 @@ def test_gradient_of_a_projection(M, N, K, splits):
 
 
 def test_projections_at_the_rule():
-    for M, N, K in ((128, 256, 256), (129, 256, 256), (130, 1024, 256),
-                    (1025, 1024, 256), (64, 256, 512), (64, 264, 256)):
+    """Sizes that a kernel takes forward, backward or both ways, and sizes left to torch."""
+    for M, N, K, forward, backward in (
+            (128, 256, 256, True, True), (129, 256, 256, True, True),
+            (64, 264, 256, True, False), (64, 256, 320, True, False),
+            (130, 1056, 256, True, True), (129, 288, 256, True, False),
+            (32, 256, 256, False, True), (8, 264, 256, False, False),
+            (64, 256, 264, False, False), (1, 2080, 512, False, True),
+            (1025, 1024, 256, True, True)):
+        assert ops.hip_ops.rows_wins(M, N, K) == forward
+        assert training._split_gradient(M, N, K) == backward
         x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
         g = draw(M, N, seed=3)
         taken = "_Linear" in type(training.linear(x.requires_grad_(True), w).grad_fn
                                   ).__name__
-        assert taken == ((M <= 128 or (M == 130)) and N >= K and N % 32 == 0)
+        assert taken == (forward or backward)
         f, p, e = (grads(fn, [x], [g], dt) for fn, dt in (
             (lambda t: training.linear(t, w), None),
             (lambda t: torch.nn.functional.linear(t, w), None),
