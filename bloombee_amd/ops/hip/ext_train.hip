@@ -213,7 +213,7 @@ static RowsPlan grad_plan(long M, long N, long K) {
 // 3000 315, 284; 8000 737, 682. 6144 x 4096: 3000 125, 128; 4000 158, 149; 8000 305, 287.
 static bool linear_grad_wins(long M, long N, long K) {
   return N > 0 && N % 64 == 0 && K > 0 && K % 256 == 0 &&
-         (M >= 3000 || (M <= 1024 && N >= 4 * K && K <= 5120) ||
+         (M >= (N >= 3 * K ? 3600 : 3000) || (M <= 1024 && N >= 4 * K && K <= 5120) ||
           (M * K <= 8500000 && (M <= 512 || M * K * N <= 150000000000L)));
 }
 

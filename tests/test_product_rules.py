@@ -61,7 +61,7 @@ def test_low_tiles_cost_what_they_take_from_memory(M, N, K, plan):
     (639, 28672, 8192, False),                                          # M * K * N
     (1024, 57344, 4096, True), (1025, 57344, 4096, False), (1024, 16384, 4096, True),
     (2999, 4096, 4096, False), (3000, 4096, 4096, True),
-    (3000, 12288, 4096, True)])
+    (3599, 12288, 4096, False), (3600, 12288, 4096, True)])
 def test_gradients_at_the_rule(M, N, K, wins):
     assert grad_wins(M, N, K) == wins
 
