@@ -1525,20 +1525,6 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
   return C;
 }
 
-// A (M, K) @ W^T as (splits, M, N): f32 sums of splits, or one part in bf16.
-torch::Tensor gemm_rows_parts(torch::Tensor A, torch::Tensor W) {
-  RowsArgs a = rows_args(A, W);
-  TORCH_CHECK(A.dim() == 2 && a.N % 8 == 0 && a.M > 0, "A (M, K), N % 8 == 0");
-  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
-  a.splits = plan.splits;
-  auto C = torch::empty({plan.splits, a.M, a.N},
-                        A.options().dtype(plan.splits > 1 ? at::kFloat : at::kBFloat16));
-  if (plan.splits > 1) a.part = C.data_ptr<float>();
-  else a.C = bf_ptr_mut(C);
-  rows_product(a, plan);
-  return C;
-}
-
 template <bool CLAMPED>
 static void rows_glu(RowsArgs& a, const RowsGlu& glu) {
   rows_tile(rows_plan(a.M, 2L * glu.F, a.K, true).tile, [&](auto tile) {
@@ -1618,7 +1604,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return py::make_tuple(p.tile, p.splits);
   });
   m.def("gemm_rows", &gemm_rows);
-  m.def("gemm_rows_parts", &gemm_rows_parts);
   m.def("gemm_rows_swiglu", &gemm_rows_swiglu);
   m.def("gemm_rows_glu", &gemm_rows_glu);
   m.def("gemm_swiglu", &gemm_swiglu);

@@ -891,13 +891,11 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
   const int BM = ta == at::kBFloat16 ? moe_height(S / (float)E) : 64;
   const int max_tiles = S / (BM == 256 ? 128 : BM) + std::min(S, E);  // and the count
   auto iopt = ids.options();
-  auto off = torch::empty({E + 1}, iopt);
   auto sorted = torch::empty({S}, iopt);
   auto tiles = torch::empty({max_tiles + 1, 4}, iopt);
-  int* offp = off.data_ptr<int>();
   int* sp = sorted.data_ptr<int>();
   int* tp = tiles.data_ptr<int>();
-  moe_sort_kernel<<<1, 1024, 0, st>>>(idp, offp, sp, tp, S, E, BM, max_tiles);
+  moe_sort_kernel<<<1, 1024, 0, st>>>(idp, sp, tp, S, E, BM, max_tiles);
   check_launch();
   if (ta == at::kFloat) {
     by_planes([&](auto np) {

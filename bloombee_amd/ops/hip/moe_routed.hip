@@ -61,14 +61,13 @@ DEVINL int xcd_order(int id, int n) {
 // sort: one workgroup of 1024
 // ---------------------------------------------------------------------------
 
-// off (E+1), sorted (S) slots, tiles (max_tiles + 1, 4): expert and MOE_MAX_E * rows
-// (-1 = unused), first sorted position, group's first tile and number of tiles of every
-// tile; then the number of tiles. An expert's rows are shared out evenly to as few tiles
+// sorted (S) slots, tiles (max_tiles + 1, 4): expert and MOE_MAX_E * rows (-1 = unused),
+// first sorted position, group's first tile and number of tiles of every tile; then the
+// number of tiles. An expert's rows are shared out evenly to as few tiles
 // of up to BM as there can be (nearly), and its tiles to groups of at most MOE_GROUP.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
-    const int* __restrict__ ids, int* __restrict__ off,
-    int* __restrict__ sorted, int* __restrict__ tiles, int S, int E, int BM,
-    int max_tiles) {
+    const int* __restrict__ ids, int* __restrict__ sorted, int* __restrict__ tiles,
+    int S, int E, int BM, int max_tiles) {
   __shared__ int cnt[MOE_MAX_E], scan[MOE_MAX_E], tscan[MOE_MAX_E];
   const int tid = threadIdx.x;
   cnt[tid] = 0;
@@ -94,7 +93,6 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
   }
   const int first = scan[tid] - c;
   if (tid < E) {
-    off[tid] = first;
     const int t0 = tscan[tid] - nt, groups = (nt + MOE_GROUP - 1) / MOE_GROUP;
     const int per = nt ? (nt + groups - 1) / groups : 1;
     for (int k = 0; k < nt; ++k) {
@@ -108,7 +106,6 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
       }
     }
   }
-  if (tid == E - 1) off[E] = scan[tid];
   if (tid == 0) tiles[4 * max_tiles] = min(tscan[MOE_MAX_E - 1], max_tiles);
   for (int i = tscan[MOE_MAX_E - 1] + tid; i < max_tiles; i += 1024)
     tiles[4 * i] = -1;
