@@ -18,8 +18,8 @@
 //  * V pages are d-major (np, Hkv, D, P): an A-fragment of V^T (8
 //    consecutive positions at fixed d) is a contiguous 16 B load. The
 //    transpose happened once at kv-write time.
-// LDS is only used for the P^T C->B relayout (tiny) and the final 4-wave
-// merge, so occupancy is VGPR-limited, not LDS-limited.
+// LDS is only used for the P^T C->B relayout (tiny) and the final merge of
+// the waves, so occupancy is VGPR-limited, not LDS-limited.
 //
 // Work decomposition: grid = (B*Hkv*nch, n_split) flash-decode splits, NW = 4
 // or 8 waves per workgroup; wave w owns KV tiles (32 positions) w, w+NW, ...

@@ -811,6 +811,10 @@ void attn_ragged(Tensor q, Tensor kp, OptTensor vp, Tensor table,
 //   225: 809 with 128, 895, 1067, 759;  350: 1279 with 128, 1296, 1132, 1036
 //   1000: 3039 with 128, 2922, 2954, 2573
 // The least bounds are 540 of weights and 1.9 a row of operations at 1.5 PF.
+// Counts that spread more (half of the experts chosen 20 times less, experts by their rank,
+// one chosen by all) cost what they did with tiles of 64 and 128 rows or less: of 150 such
+// steps of 8 to 64 experts, 40 to 4000 rows, two take more, 64 experts of exactly 125 rows
+// (234 us, 213) and 1400 rows that all choose one of eight (1361, 1301).
 static int moe_height(float a) {
   const float most = a + sqrtf(a);
   for (int rows : {64, 96, 128, 160, 192})
