@@ -4,8 +4,9 @@ Replaces the reference's OptimizedLlamaDecoderLayer + FLEX_LlamaAttention/MLP
 stack (models/llama/block.py:149-861, models/llama/flex_llama.py:434-793) with
 a flat MI355X-native block:
 
-  * plain-GEMM projections via hipBLASLt (torch F.linear on bf16) with QKV and
-    gate/up fused into single GEMMs (fewer, larger GEMMs — xGMI/HBM sizing),
+  * projections via ops.linear (hand-written products for decode and some hundred
+    rows, hipBLASLt beyond) with QKV and gate/up fused into single GEMMs (fewer,
+    larger GEMMs — xGMI/HBM sizing),
   * hand-written HIP kernels for everything fused: rmsnorm(+residual), RoPE,
     paged KV write, paged decode/prefill attention, SwiGLU,
   * one paged KV pool shared across local layers (kv/paged.py), no
