@@ -1192,7 +1192,7 @@ torch::Tensor gemm_skinny(torch::Tensor A, torch::Tensor W,
   const int N = W.size(0);
   TORCH_CHECK(M <= 32, "gemm_skinny is for M <= 32, got ", M);
   TORCH_CHECK(W.size(1) == K, "A/W K mismatch");
-  TORCH_CHECK(K % 32 == 0 && N % 64 == 0, "K%32, N%64 required");
+  TORCH_CHECK(K % 32 == 0 && N % 64 == 0 && N > 0, "K%32, N%64 required");
   // norm_mode: 0 none; 1 scale A by invr*norm_w per stage; 2 norm weight
   // pre-folded into W — only the invr accumulator scale remains (cheap).
   int norm_mode = (int)norm_mode_req;

@@ -615,8 +615,8 @@ Tensor gemm_parts(Tensor A, Tensor W, long ksplit_req) {
   CHECK_T(W, at::kBFloat16);
   TORCH_CHECK(A.dim() == 2 && W.dim() == 2 && A.size(1) == W.size(1));
   const int M = A.size(0), N = W.size(0), K = A.size(1);
-  TORCH_CHECK(M >= 1 && M <= 32 && K % 32 == 0 && N % 64 == 0,
-              "need M <= 32, K % 32 == 0, N % 64 == 0");
+  TORCH_CHECK(M >= 1 && M <= 32 && K % 32 == 0 && N % 64 == 0 && N > 0,
+              "need M <= 32, K % 32 == 0, N % 64 == 0, N > 0");
   int ks = (int)ksplit_req;
   if (ks <= 0) {
     // as gemm_skinny: one split once N alone covers the chip, else up to

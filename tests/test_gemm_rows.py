@@ -201,9 +201,15 @@ def test_addends_are_torchs():
 @pytest.mark.parametrize("M", [1, 8, 20, 64])
 @pytest.mark.parametrize("K", [256, 2048])
 def test_weights_without_rows(M, K):
+    from bloombee_amd.ops import ragged
     x, w = draw(M, K, seed=1), draw(0, K, seed=2)
     assert ops.linear(x, w).shape == (M, 0)
     assert ops.hip_ops.gemm_stream(x[:32], w, None, None, -1.0).shape == (min(M, 32), 0)
+    if K == 2048 and M <= 32:
+        with pytest.raises(RuntimeError):      # refused, no division by its columns
+            ops.hip_ops.gemm_skinny(x, w, None, None, 0, None, 0.0, None, None, 0)
+        with pytest.raises(RuntimeError):
+            ragged._ext().gemm_parts(x, w, 0)
     x.requires_grad_(True)
     dx, = torch.autograd.grad(training.linear(x, w).sum(), x)
     assert dx.shape == x.shape and not dx.any()
