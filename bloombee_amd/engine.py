@@ -29,6 +29,7 @@ from bloombee_amd.models.llama.block import RopeTables
 from bloombee_amd.utils.logging import get_logger
 from bloombee_amd import ops
 from bloombee_amd.ops import ragged, training
+from bloombee_amd.ops.span import decode_span
 
 logger = get_logger(__name__)
 
@@ -122,6 +123,10 @@ class BlockStack(torch.nn.Module):
                     x.view(B, T, C)[:, :n_over, :dp.shape[-1]] += dp
             self.forward_batch(x, lockstep_batch(kv, start_pos, B, T), hook)
             return x.view(B, T, C)
+        if tree_mask is None and n_over <= 0:
+            out = self._decode_span(hidden, kv, start_pos, position_ids)
+            if out is not None:
+                return out
         for i, blk in enumerate(self.blocks):
             if n_over > 0:
                 dp = deep_prompts[i, sp0:sp0 + n_over].to(hidden.dtype)
@@ -132,6 +137,40 @@ class BlockStack(torch.nn.Module):
             else:
                 hidden = blk.forward_inference(hidden, kv, start_pos, position_ids)
         return hidden
+
+    def _decode_span(self, hidden: torch.Tensor, kv: SessionHandle,
+                     start_pos: torch.Tensor,
+                     position_ids: Optional[torch.Tensor]
+                     ) -> Optional[torch.Tensor]:
+        """All blocks in one launch, where there is one for them (ops/span.py). It
+        wins from two blocks on (1024 columns: 0.67 to 0.88 of the time, 4096: 0.86 to
+        0.97); of a single one 3 to 4 sequences take 1 to 2% longer than block by
+        block, fewer 1 to 24% less."""
+        if (len(self.blocks) < 2 or hidden.shape[1] != 1 or hidden.shape[0] > 4
+                or not hidden.is_cuda):
+            return None
+        weights = []
+        first = self.blocks[0]
+        for blk in self.blocks:
+            norms = getattr(blk, "span_norms", None)
+            norms = norms() if norms is not None else None
+            if (norms is None or "forward_inference" in blk.__dict__
+                    or blk.rope is not first.rope
+                    or not blk._fuse_norm_gate(hidden)
+                    or (hasattr(kv, "host_prefix")
+                        and kv.host_prefix(blk.layer_index) is not None)):
+                return None
+            weights += [blk.qkv_w, blk.o_w, blk.gate_up_w, blk.down_w, *norms,
+                        kv.k_pages(blk.layer_index), kv.v_pages(blk.layer_index)]
+        off = getattr(kv, "pos_offset", 0)
+        if off and position_ids is None:
+            position_ids = (start_pos.view(-1, 1) + off).int()
+        for blk in self.blocks:
+            blk.fold_norm_weights()
+        cos, sin = first.rope.get(hidden.device)
+        return decode_span(hidden, weights, first.Hq, cos, sin, position_ids,
+                           start_pos, kv.page_table(), first.config.rms_norm_eps,
+                           first.scale)
 
     @torch.no_grad()
     def forward_batch(self, hidden: torch.Tensor, batch: TokenBatch,

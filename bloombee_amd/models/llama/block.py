@@ -119,6 +119,14 @@ class LlamaBlock(torch.nn.Module):
         m = ops.linear_swiglu(h2, self.gate_up_w, self.config.rms_norm_eps)
         return ops.linear(m, self.down_w, residual=h2)
 
+    def span_norms(self):
+        """Norm weights of q and k heads for a span's launch, empty without any; None
+        where a block does more than such a launch."""
+        if type(self).forward_inference is not _LLAMA_STEP:
+            return None
+        none = self.qkv_w.new_empty(0)
+        return none, none
+
     @torch.no_grad()
     def fold_norm_weights(self):
         """Reparameterize for the fused-norm decode path: qkv_w <- qkv_w *
@@ -304,3 +312,7 @@ class LlamaBlock(torch.nn.Module):
 
     def forward(self, *args, **kw):
         return self.forward_inference(*args, **kw)
+
+
+# the step that a span's launch stands for
+_LLAMA_STEP = LlamaBlock.forward_inference

@@ -26,6 +26,11 @@ class Qwen3Block(LlamaBlock):
         self.k_norm_w = torch.nn.Parameter(torch.empty(D, dtype=dt),
                                            requires_grad=False)
 
+    def span_norms(self):
+        if type(self).forward_inference is not _QWEN3_STEP:
+            return None
+        return self.q_norm_w, self.k_norm_w
+
     @torch.no_grad()
     def forward_inference(self, hidden: torch.Tensor, kv: SessionHandle,
                           start_pos: torch.Tensor,
@@ -113,3 +118,7 @@ class Qwen3Block(LlamaBlock):
         m = torch.nn.functional.linear(
             torch.nn.functional.silu(g.float()).to(u.dtype) * u, self.down_w)
         return h2 + m
+
+
+# the step that a span's launch stands for
+_QWEN3_STEP = Qwen3Block.forward_inference

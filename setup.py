@@ -21,13 +21,14 @@ OPS_DIR = ROOT / "bloombee_amd" / "ops"
 # _hip_mixers latent attention and gated linear attention, _hip_recurrent the
 # matrix memory and the gated linear recurrent unit, _hip_differential differential
 # attention, _hip_hgrn gated linear attention that writes what it forgets,
-# _hip_train attention and row steps with their gradients.
+# _hip_train attention and row steps with their gradients, _hip_span a decode step of
+# whole layers in one launch.
 MODULES = {"_hip_ops": "ext.hip", "_hip_ragged": "ext_ragged.hip",
            "_hip_mixers": "ext_mixers.hip",
            "_hip_recurrent": "ext_recurrent.hip",
            "_hip_differential": "ext_differential.hip",
            "_hip_hgrn": "ext_hgrn.hip",
-           "_hip_train": "ext_train.hip"}
+           "_hip_train": "ext_train.hip", "_hip_span": "ext_span.hip"}
 ARCH = os.environ.get("PYTORCH_ROCM_ARCH", "gfx950")
 
 
