@@ -22,10 +22,12 @@
 // overlap); the chain of tiles bounds short ones, so there the keys are split over
 // workgroups and a second kernel folds the parts.
 //
-// Measured, 32 heads on 8 of 128: four prompts of 4096 672 us alone (820 TF/s of the
-// visible half; 3808 us with 16-row tiles of one head each, staged through
-// registers, weights through LDS), one of 333 behind 1201 37 us (163), a tree of 25
-// behind 1500 18.5 us (168).
+// Measured, 32 heads on 8 of 128: four prompts of 4096 625 us alone (880 TF/s of the
+// visible half; 675 with an address a lane, 3808 us with 16-row tiles of one head each,
+// staged through registers, weights through LDS), 2000 tokens behind 6000 270 us (299 with
+// an address a lane), one of 333 behind 1201 37 us (163), a tree of 25 behind 1500 18.5 us
+// (168). The loads alone take 293 us of the 625: what is left overlaps by half. Scores a
+// tile ahead of the weights within a wave took 686, 256 rows a workgroup 641 (loads 172).
 //
 // Numerics: fp32 softmax/accum; bf16 operands — matches reference tolerance
 // class (test_block_exact_match.py atol 1e-4 forward on fp32 inputs).
@@ -72,17 +74,22 @@ __device__ const unsigned short prefill_zeros[8] __attribute__((aligned(16))) = 
 // GENERAL: slopes, scales that are not positive; TREE: these and tree masks, whose code
 // in between took slopes as long as it did trees (two tokens, 16 heads of 64: 7.4 us, 5.6
 // apart).
-// DIVIDE: TREE, and pages that do not hold a power of two of keys; a form of its own, since
-// even the choice costs where pages are found by shifts (0.75 us of a tree's 20).
-enum PrefillForm { PREFILL_PLAIN, PREFILL_GENERAL, PREFILL_TREE, PREFILL_DIVIDE };
+enum PrefillForm { PREFILL_PLAIN, PREFILL_GENERAL, PREFILL_TREE };
 
-template <int D, int FORM>
+// A load brings keys (values) of one group of sixteen. GROUPS: pages hold a power of two of
+// keys, 16 or more, so that a load's page is the wave's. EIGHTS: of 8, which a lane looks up
+// for itself; MIXED: not a power of two. Forms of their own, since even the choice costs
+// where a lane finds pages by shifts (0.75 us of a tree's 20).
+enum PrefillPages { PREFILL_GROUPS, PREFILL_EIGHTS, PREFILL_MIXED };
+
+template <int D, int FORM, int PAGES>
 __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     PrefillArgs a) {
   using Tile = PrefillTile<D>;
   constexpr int KT = Tile::KT, RC = Tile::RC, NI = Tile::NI;
   constexpr int NKK = D / 16, ND = D / 32;
-  constexpr bool GENERAL = FORM != PREFILL_PLAIN, DIVIDE = FORM == PREFILL_DIVIDE;
+  constexpr bool GENERAL = FORM != PREFILL_PLAIN, DIVIDE = PAGES == PREFILL_MIXED;
+  constexpr bool LANES = PAGES != PREFILL_GROUPS;
   static_assert(NI >= 1, "tile smaller than the workgroup");
   extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
 
@@ -99,8 +106,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int lane = tid & (WAVE - 1);
   const int li = lane & 31, hi = lane >> 5;
   const int qs = a.q_start[b];
-  const bool tree = FORM >= PREFILL_TREE && a.tree_mask != nullptr;
-  const int plog = a.p_log2, pmask = (1 << plog) - 1;
+  const bool tree = FORM == PREFILL_TREE && a.tree_mask != nullptr;
+  const int plog = PAGES == PREFILL_EIGHTS ? 3 : a.p_log2, pmask = (1 << plog) - 1;
   auto page_of = [&](int pos) { return DIVIDE ? pos / a.P : pos >> plog; };
   auto slot_of = [&](int pos) { return DIVIDE ? pos % a.P : pos & pmask; };
   auto first_of = [&](long page) { return DIVIDE ? page * a.P : page << plog; };
@@ -139,7 +146,10 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int t0 = kbeg + split * per * KT;
   const int t1 = min(kend, t0 + per * KT);
 
-  // where this lane's pieces come from
+  // Where this lane's pieces come from. Load i of a wave brings pieces of keys (values) of
+  // group group_of(i) of sixteen: of the wave's page, at offsets that are the same in every
+  // tile. (An address a lane took 139 vector instructions a tile, some of them four times
+  // as long as others; the softmax takes 105.)
   int kkey[NI], kcol[NI], vkey[NI], vrow[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
@@ -150,29 +160,64 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     vkey[i] = at / (2 * D) * 16 + (at & 1) * 8;   // groups of 16 keys, (d, octet)
     vrow[i] = at % (2 * D) / 2;
   }
-  int kpage[NI], vpage[NI];
+  static_assert(64 / RC <= 16 && 2 * D >= 64, "a load is of one group");
+  auto group_of = [&](int i) { return (wave + i * 4) * 32 / D * 16; };
+  constexpr int OFS = 256 / RC % 16 ? 2 : 1;      // loads of different offsets
+  static_assert(OFS == (256 % (2 * D) ? 2 : 1), "values as keys");
+  unsigned kofs[OFS], vofs[OFS];
+#pragma unroll
+  for (int i = 0; i < OFS; ++i) {
+    kofs[i] = (unsigned)((kkey[i] & 15) * D + kcol[i]) * 2;
+    vofs[i] = (unsigned)(vrow[i] * a.P + (lane & 1) * 8) * 2;
+  }
+  // nothing writes the table meanwhile: scalar loads
+  const auto* pages = (const __attribute__((address_space(4))) int*)table;
+  int kpage[NI], vpage[NI];      // of the tile that is asked for next
   auto look_up = [&](int kb) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      kpage[i] = table[page_of(min(kb + kkey[i], kend - 1))];
-      vpage[i] = table[page_of(min(kb + vkey[i], kend - 1))];
+      if constexpr (LANES) {
+        kpage[i] = table[page_of(min(kb + kkey[i], kend - 1))];
+        vpage[i] = table[page_of(min(kb + vkey[i], kend - 1))];
+      } else {
+        kpage[i] = vpage[i] = pages[page_of(min(kb + group_of(i), kend - 1))];
+      }
     }
   };
   auto issue = [&](int kb, unsigned char* buf) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int pos = slot_of(min(kb + kkey[i], kend - 1));
-      copy16_to_lds(a.k_pages +
-                        (first_of((long)kpage[i] * a.Hkv + g) + pos) * D + kcol[i],
-                    buf + (wave + i * 4) * 1024);
+      unsigned char* to = buf + (wave + i * 4) * 1024;
+      if constexpr (LANES) {
+        const int pos = slot_of(min(kb + kkey[i], kend - 1));
+        copy16_to_lds(a.k_pages + (first_of((long)kpage[i] * a.Hkv + g) + pos) * D +
+                          kcol[i],
+                      to);
+      } else {
+        // keys behind the last one are masked
+        const int at = (kb + group_of(i)) & pmask;
+        dma16(a.k_pages + (first_of((long)kpage[i] * a.Hkv + g) + at) * D, kofs[i % OFS],
+              (unsigned)(unsigned long)(lptr_t)to);
+      }
     }
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const unsigned short* src =
-          a.v_pages + first_of(((long)vpage[i] * a.Hkv + g) * D + vrow[i]) +
-          slot_of(kb + vkey[i]);
-      if (kb + vkey[i] >= kend) src = prefill_zeros;
-      copy16_to_lds(src, buf + Tile::KB + (wave + i * 4) * 1024);
+      unsigned char* to = buf + Tile::KB + (wave + i * 4) * 1024;
+      const unsigned short* head = a.v_pages + first_of(((long)vpage[i] * a.Hkv + g) * D);
+      if constexpr (LANES) {
+        const unsigned short* src = head + first_of(vrow[i]) + slot_of(kb + vkey[i]);
+        if (kb + vkey[i] >= kend) src = prefill_zeros;
+        copy16_to_lds(src, to);
+      } else {
+        head += (kb + group_of(i)) & pmask;
+        if (kb + KT > kend) {
+          const unsigned short* src = head + vofs[i % OFS] / 2;
+          if (kb + group_of(i) + (lane & 1) * 8 >= kend) src = prefill_zeros;
+          dma16_to_lds(src, to);
+        } else {
+          dma16(head, vofs[i % OFS], (unsigned)(unsigned long)(lptr_t)to);
+        }
+      }
     }
   };
 
@@ -284,6 +329,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
     look_up(t0);
     issue(t0, prefill_lds);
     look_up(t0 + KT);
+    if (!LANES) landed();
     __syncthreads();
     int buf = 0;
     for (int kb = t0; kb < t1; kb += KT) {
@@ -293,6 +339,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
       }
       if (kb <= wlast && kb + KT > wfirst)
         compute(kb, prefill_lds + buf * Tile::BYTES);
+      if (!LANES) landed();
       __syncthreads();
       buf ^= 1;
     }

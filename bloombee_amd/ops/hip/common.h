@@ -91,6 +91,22 @@ DEVINL void copy16_to_lds(const unsigned short* g, unsigned char* l) {
   __builtin_amdgcn_global_load_lds((gptr_t)g, (lptr_t)l, 16, 0, 0);
 }
 
+// The same in assembly: the compiler lets every read of LDS behind the builtin wait for
+// all such loads, also for those into another buffer. The wait for these is the caller's,
+// landed() or a count, ahead of a barrier.
+DEVINL void dma16_to_lds(const void* g, unsigned char* l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"((unsigned)(unsigned long)(lptr_t)l), "v"(g) : "m0", "memory");
+}
+
+// From base + ofs bytes, base and l the wave's: nothing to calculate but ofs.
+DEVINL void dma16(const void* base, unsigned ofs, unsigned l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(l), "v"(ofs), "s"(base) : "m0");
+}
+
+DEVINL void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 __host__ DEVINL long ldiv_up(long a, long b) { return (a + b - 1) / b; }
 
 #define HIP_OK(expr)                                                         \

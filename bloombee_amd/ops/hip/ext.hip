@@ -439,9 +439,10 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
     a.pml = a.pacc + (long)a.n_split * units * rows * D;
   }
   const dim3 grid(units * a.n_split, row_tiles);
-  auto launch = [&](auto d, auto form) {
+  auto launch = [&](auto d, auto form, auto pages) {
     constexpr int DD = decltype(d)::value;
-    auto kernel = attn_prefill_kernel<DD, decltype(form)::value>;
+    auto kernel =
+        attn_prefill_kernel<DD, decltype(form)::value, decltype(pages)::value>;
     constexpr int lds = 2 * PrefillTile<DD>::BYTES;
     if (lds > 64 * 1024)
       TORCH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -453,18 +454,25 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
       attn_prefill_fold_kernel<DD>
           <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
   };
-  auto by_dim = [&](auto form) {
-    if (D == 128) launch(std::integral_constant<int, 128>{}, form);
-    else if (D == 64) launch(std::integral_constant<int, 64>{}, form);
-    else if (D == 256) launch(std::integral_constant<int, 256>{}, form);
-    else if (D == 32) launch(std::integral_constant<int, 32>{}, form);
+  auto by_dim = [&](auto form, auto pages) {
+    if (D == 128) launch(std::integral_constant<int, 128>{}, form, pages);
+    else if (D == 64) launch(std::integral_constant<int, 64>{}, form, pages);
+    else if (D == 256) launch(std::integral_constant<int, 256>{}, form, pages);
+    else if (D == 32) launch(std::integral_constant<int, 32>{}, form, pages);
     else TORCH_CHECK(false, "unsupported head_dim ", D);
   };
-  if (P & (P - 1)) by_dim(std::integral_constant<int, PREFILL_DIVIDE>{});
-  else if (a.tree_mask) by_dim(std::integral_constant<int, PREFILL_TREE>{});
-  else if (a.alibi || !(a.scale > 0.f))
-    by_dim(std::integral_constant<int, PREFILL_GENERAL>{});
-  else by_dim(std::integral_constant<int, PREFILL_PLAIN>{});
+  constexpr std::integral_constant<int, PREFILL_TREE> tree;
+  auto by_form = [&](auto pages) {
+    if (a.tree_mask) by_dim(tree, pages);
+    else if (a.alibi || !(a.scale > 0.f))
+      by_dim(std::integral_constant<int, PREFILL_GENERAL>{}, pages);
+    else by_dim(std::integral_constant<int, PREFILL_PLAIN>{}, pages);
+  };
+  // beyond 2^20 keys a page's offsets would leave 32 bits
+  if ((P & (P - 1)) || P > 1 << 20)
+    by_dim(tree, std::integral_constant<int, PREFILL_MIXED>{});
+  else if (P < 16) by_form(std::integral_constant<int, PREFILL_EIGHTS>{});
+  else by_form(std::integral_constant<int, PREFILL_GROUPS>{});
 }
 
 // Pages go to LDS by 16-byte copies: a view that does not begin at 16 bytes is copied.

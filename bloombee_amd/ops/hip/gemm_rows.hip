@@ -27,14 +27,6 @@
 #pragma once
 #include "common.h"
 
-// 16 B a lane from memory to LDS, base and l the wave's. An asm block, since the
-// compiler lets every read of LDS behind the builtin wait for all such loads; the
-// waits are the caller's.
-DEVINL void dma16(const void* base, unsigned ofs, unsigned l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(l), "v"(ofs), "s"(base) : "m0");
-}
-
 // Until at most N loads of the wave are on their way and its reads of LDS are done.
 template <int N>
 DEVINL void wait_loads() {

@@ -198,3 +198,21 @@ def test_infinite_values_of_the_last_key(Hkv, D, room, tokens, start):
     assert torch.equal(got.float().isinf(), want.isinf())
     seen = want.isfinite()
     close(got[seen], want[seen])
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("P", [8, 16, 32, 128, 48])
+@pytest.mark.parametrize("length", [63, 65, 200])
+def test_pages_behind_the_last_key(D, P, length):
+    """Every head size with pages that a wave or a lane looks up, tiles that end within a
+    page and before it; keys that are not numbers behind the last one do no harm."""
+    B, Hq, Hkv, T = 2, 4, 2, 37
+    starts = (length - T, 1)
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], 256, seed=P)
+    kp[kp == 50.0] = float("nan")
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    want = ref.attn_paged(q.float(), kp.float().nan_to_num(0), vp.float(), table,
+                          qs.long())
+    close(ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)]), want)
