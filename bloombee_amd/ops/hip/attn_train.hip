@@ -27,10 +27,11 @@
 // queries 0.0027 to 0.0140 (0.0031 to 0.0141), keys 0.0028 to 0.0141 (0.0035 to 0.0143),
 // values 0.0022 to 0.0077 (0.0028 to 0.0079): a group's heads are summed in 32 bits here.
 //
-// The matrix cores bound all three: 3, 4 and 6 products of 32 x 32 x D a tile. Two
-// sequences of 1999, 32 heads on 8 of 128: 136, 166 and 401 us (721, 788 and 490
-// TF/s of the visible half); as float32 torch operations a layer's attention took
-// 9.2 ms both ways.
+// 3, 4 and 6 products of 32 x 32 x D a tile. Two sequences of 1999, 32 heads on 8 of 128:
+// 136, 168 and 252 us (721, 779 and 780 TF/s of the visible half); as float32 torch
+// operations a layer's attention took 9.2 ms both ways. The first two keep the matrix cores
+// busy for 37 and 39% of that, and the vector units, which weigh and split, for as much; the
+// third is described where it stands.
 
 #pragma once
 #include "common.h"
@@ -120,9 +121,42 @@ DEVINL void stage_rows(const RowMap& m, int r0, int last, unsigned char* tile,
   for (int i = 0; i < Tile::NI; ++i) {
     const int at = (wave + i * 4) * 64 + lane;
     const int r = at / Tile::RC, c = (at % Tile::RC) ^ Tile::swizzle(r);
-    copy16_to_lds(m.at(min(r0 + r, last), D) + c * 8, tile + (wave + i * 4) * 1024);
+    dma16_to_lds(m.at(min(r0 + r, last), D) + c * 8, tile + (wave + i * 4) * 1024);
   }
 }
+
+// The same for tiles that begin at multiples of 64. Where the heads of a group divide 64
+// and no row is beyond `last`, a lane's offsets from the tile's first row are those of any
+// tile, and nothing is calculated (a division and a 64-bit product a load otherwise).
+template <int D>
+struct RowStage {
+  using Tile = TrainTile<D>;
+  RowMap m;
+  long step;               // from a tile's first row to the next one's
+  int last, wave, lane;
+  unsigned ofs[Tile::NI];
+  DEVINL RowStage(const RowMap& rows, int last_, int wave_, int lane_)
+      : m(rows), step(64 % rows.G ? 0 : 64 / rows.G * rows.ld), last(last_),
+        wave(wave_), lane(lane_) {
+#pragma unroll
+    for (int i = 0; i < Tile::NI; ++i) {
+      const int at = (wave + i * 4) * 64 + lane;
+      const int r = at / Tile::RC, c = (at % Tile::RC) ^ Tile::swizzle(r);
+      ofs[i] = (unsigned)((r / m.G * m.ld + r % m.G * D + c * 8) * 2);
+    }
+  }
+  DEVINL void operator()(int r0, unsigned char* tile) const {
+    if (step == 0 || r0 + 63 > last) {
+      stage_rows<D>(m, r0, last, tile, wave, lane);
+      return;
+    }
+    const unsigned short* base = m.base + (r0 >> 6) * step;
+#pragma unroll
+    for (int i = 0; i < Tile::NI; ++i)
+      dma16(base, ofs[i],
+            (unsigned)(unsigned long)(lptr_t)(tile + (wave + i * 4) * 1024));
+  }
+};
 
 // grid: ceil(B * T * (Hq + Hkv) * D / 16 / 256); a thread turns eight pairs
 __global__ __launch_bounds__(256) void rope_rows_kernel(
@@ -190,6 +224,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_kernel(TrainAttnArgs a) {
 
   stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
   stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
+  landed();
   __syncthreads();
   int buf = 0;
   for (int kb = 0; kb < kend; kb += KT) {
@@ -254,6 +289,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_kernel(TrainAttnArgs a) {
           }
         }
     }
+    landed();
     __syncthreads();
     buf ^= 1;
   }
@@ -328,6 +364,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) 
 
   stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
   stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
+  landed();
   __syncthreads();
   int buf = 0;
   for (int kb = 0; kb < kend; kb += KT) {
@@ -371,6 +408,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) 
         }
       }
     }
+    landed();
     __syncthreads();
     buf ^= 1;
   }
@@ -399,16 +437,45 @@ __global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) 
     }
 }
 
+DEVINL void dma4(const void* base, unsigned ofs, unsigned l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :: "s"(l), "v"(ofs), "s"(base) : "m0");
+}
+
+template <int N>
+DEVINL void landed_but() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+
+// Where the tiles of 64 rows wait: one is worked on, the next one's rows are read as well,
+// two are on their way.
+template <int D>
+struct TrainRing {
+  static constexpr int DEPTH = 4;
+  static constexpr int SLOT = 2 * TrainTile<D>::BYTES + 1024;
+  static constexpr int LOADS = 2 * TrainTile<D>::NI + 1;   // of a wave and tile
+  static constexpr int BYTES = DEPTH * SLOT;
+};
+
 // grid (B * Hkv, tiles of 64 keys); waves 0 and 1 own 32 keys each, waves 2 and 3 the
 // same keys: the two pairs take the two halves of a tile of 64 rows and add up at the
 // end. 192 accumulator and operand registers leave room for one wave a SIMD; tiles of
 // 64 keys and not 128 make twice as many workgroups with half as long a chain.
+//
+// With one wave a SIMD nothing overlaps but what the wave's own order lets: the products
+// of a tile run beside the vector work and the LDS reads of its neighbours. 16 products of
+// the last tile's second half hide the reads of this one's numbers and the next one's rows,
+// the next one's 16 score products half of the weights (about ten instructions an element)
+// and the reads of columns, 16 products of the first half the rest. Two sequences of 1999,
+// 32 heads on 8 of 128: products and vector work one after the other, every read waited
+// for, 410 us; reads at once, addresses of constant offsets 291; tiles three ahead 288; the
+// order above 262; sums exchanged both ways at the end, rotation tables read at once 252.
+// 600 tokens: 103 us, now 60. What is left: a tile's 48 products take 770 ns of 1900, its
+// LDS traffic (160 KB a workgroup) about 600.
 template <int D>
 __global__ __launch_bounds__(256, 1) void attn_train_dkv_kernel(TrainAttnArgs a) {
   using Tile = TrainTile<D>;
   constexpr int NKK = D / 16, ND = D / 32;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[4 * Tile::BYTES];
-  __shared__ __attribute__((aligned(16))) float stat[2][2][64];
+  using Ring = TrainRing<D>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char train_lds[];
   const int b = blockIdx.x / a.Hkv, g = blockIdx.x % a.Hkv;
   const int G = a.G, R = a.T * G, Hq = a.Hkv * G;
   const int k0 = blockIdx.y * 64;                // early keys are seen most
@@ -442,111 +509,213 @@ __global__ __launch_bounds__(256, 1) void attn_train_dkv_kernel(TrainAttnArgs a)
 
   f32x16 dk[ND], dv[ND];
 #pragma unroll
-  for (int n = 0; n < ND; ++n) dk[n] = dv[n] = f32x16{};
-
-  const int r0 = (k0 * G) & ~63;
-  float mine = 0.f;
-  auto fetch = [&](int rb) {
-    if (tid < 64) mine = lse[min(rb + tid, R - 1)];
-    else if (tid < 128) mine = delta[min(rb + tid - 64, R - 1)];
-  };
-  auto keep = [&](int bf) {
-    if (tid < 128) stat[bf][tid >> 6][tid & 63] = mine;
-  };
-  stage_rows<D>(rows, r0, R - 1, lds, wave, lane);
-  stage_rows<D>(outs, r0, R - 1, lds + Tile::BYTES, wave, lane);
-  fetch(r0);
-  keep(0);
-  __syncthreads();
-  int buf = 0;
-  for (int rb = r0; rb < R; rb += 64) {
-    const bool more = rb + 64 < R;
-    if (more) {
-      unsigned char* next = lds + (buf ^ 1) * 2 * Tile::BYTES;
-      stage_rows<D>(rows, rb + 64, R - 1, next, wave, lane);
-      stage_rows<D>(outs, rb + 64, R - 1, next + Tile::BYTES, wave, lane);
-      fetch(rb + 64);
-    }
-    const unsigned char* qt = lds + buf * 2 * Tile::BYTES;
-    const unsigned char* ot = qt + Tile::BYTES;
-    const int w0 = rb + half;
-    if (w0 < R && w0 + 31 >= (k0 + (wave & 1) * 32) * G) {
-      f32x16 s = f32x16{}, dp = f32x16{};
-#pragma unroll
-      for (int kk = 0; kk < NKK; ++kk) {
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(qt, qrow, kk, hi),
-                                                    kf[kk], s, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(ot, qrow, kk, hi),
-                                                     vf[kk], dp, 0, 0, 0);
-      }
-      // element j of a lane is row w0 + (j & 8) * 2 + hi * 8 + (j & 7)
-      const bool edge = w0 < full || w0 + 31 >= R;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        float p[8], ds[8];
-        const int rr = half + j * 16 + hi * 8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          p[e] = fast_exp2(fmaf(s[j * 8 + e], sc2, -stat[buf][0][rr + e]));
-          const int q = rb + rr + e;
-          if (edge && (q < first || q >= R)) p[e] = 0.f;
-          ds[e] = p[e] * (dp[j * 8 + e] - stat[buf][1][rr + e]);
-        }
-        bf16x8 ph, pl, dh, dl;
-        split_pair(p, ph, pl);
-        split_pair(ds, dh, dl);
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const bf16x8 oc = col_frag<D>(ot, half + j * 16, d, lane);
-          const bf16x8 qc = col_frag<D>(qt, half + j * 16, d, lane);
-          dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ph, oc, dv[d], 0, 0, 0);
-          dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dh, qc, dk[d], 0, 0, 0);
-          dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pl, oc, dv[d], 0, 0, 0);
-          dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dl, qc, dk[d], 0, 0, 0);
-        }
-      }
-    }
-    if (more) keep(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
+  for (int n = 0; n < ND; ++n) {
+    dk[n] = dv[n] = f32x16{};
+    // known zeros would be carried through the loop as 16 numbers each, and copied
+    asm volatile("" : "+a"(dk[n]), "+a"(dv[n]));
   }
 
-  // the second pair's sums go through LDS, values and keys one after the other
-  float* sums = reinterpret_cast<float*>(lds) + (wave & 1) * 32 * D;
-  auto join = [&](f32x16 (&x)[ND]) {
-    if (wave >> 1) {
-#pragma unroll
-      for (int n = 0; n < ND; ++n)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) sums[(n * 16 + j) * 64 + lane] = x[n][j];
-    }
-    __syncthreads();
-    if (!(wave >> 1)) {
-#pragma unroll
-      for (int n = 0; n < ND; ++n)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) x[n][j] += sums[(n * 16 + j) * 64 + lane];
-    }
-    __syncthreads();
+  const int r0 = (k0 * G) & ~63;
+  const RowStage<D> row_tile(rows, R - 1, wave, lane);
+  const RowStage<D> out_tile(outs, R - 1, wave, lane);
+  // a tile's rows, and of each wave its log-sums (waves 0 and 2) or sums of dO * O
+  auto ask = [&](int t) {
+    unsigned char* to = train_lds + t % Ring::DEPTH * Ring::SLOT;
+    const int rb = r0 + t * 64;
+    row_tile(rb, to);
+    out_tile(rb, to + Tile::BYTES);
+    dma4(wave & 1 ? delta : lse, (unsigned)min(rb + lane, R - 1) * 4,
+         (unsigned)(unsigned long)(lptr_t)(to + 2 * Tile::BYTES + wave * 256));
   };
-  join(dv);
-  join(dk);
-  if (wave >> 1) return;
+  const int tiles = (R - r0 + 63) / 64;
+  for (int t = 0; t < min(tiles, Ring::DEPTH - 1); ++t) ask(t);
+  // these have arrived: what is waited for from here on are the tiles alone
+#pragma unroll
+  for (int kk = 0; kk < NKK; ++kk) asm volatile("" : "+v"(kf[kk]), "+v"(vf[kk]));
+  // tiles of which this wave's half sees keys of its own
+  const int seen = max(0, (k0 + (wave & 1) * 32) * G - half - 31 - r0 + 63) / 64;
+  const int rest = (R - half - r0 + 63) / 64;
+
+  // of a tile: the scores and dO V^T, ahead of the rest by one tile
+  f32x16 s, dp, s1, dp1;
+  bf16x8 qa[NKK], oa[NKK], oc[2][ND], qc[2][ND], ph[2], pl[2], dh[2], dl[2];
+  f32x4 ls[4], de[4];
+  float p[8], ds[8];
+  auto weigh = [&](int e) {      // element e, of the one before it as well the splits
+    const int j = e >> 3, i = e & 7;
+    p[i] = fast_exp2(fmaf(s[e], sc2, -ls[e >> 2][e & 3]));
+    ds[i] = p[i] * (dp[e] - de[e >> 2][e & 3]);
+    if (i & 1) {
+#pragma unroll
+      for (int c = i - 1; c <= i; ++c) {
+        ph[j][c] = (__bf16)p[c];
+        dh[j][c] = (__bf16)ds[c];
+        pl[j][c] = (__bf16)(p[c] - (float)ph[j][c]);
+        dl[j][c] = (__bf16)(ds[c] - (float)dh[j][c]);
+      }
+    }
+  };
+  auto add = [&](int j, int d) {
+    dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ph[j], oc[j][d], dv[d], 0, 0, 0);
+    dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dh[j], qc[j][d], dk[d], 0, 0, 0);
+    dv[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pl[j], oc[j][d], dv[d], 0, 0, 0);
+    dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dl[j], qc[j][d], dk[d], 0, 0, 0);
+  };
+  auto turn = [&](int t) {
+    if (tiles - t > 2) landed_but<Ring::LOADS>();
+    else landed();
+    // everybody's loads of this tile and the next, and everybody is done with the one
+    // before, whose place another takes
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (t + Ring::DEPTH - 1 < tiles) ask(t + Ring::DEPTH - 1);
+  };
+#pragma unroll
+  for (int d = 0; d < ND; ++d) {
+    oc[1][d] = qc[1][d] = bf16x8{};
+    asm volatile("" : "+v"(oc[1][d]), "+v"(qc[1][d]));
+  }
+  ph[1] = pl[1] = dh[1] = dl[1] = bf16x8{};
+  asm volatile("" : "+v"(ph[1]), "+v"(pl[1]), "+v"(dh[1]), "+v"(dl[1]));
+  int t = 0;
+  for (; t < min(seen, tiles); ++t) turn(t);
+  if (t < rest) {
+    turn(t);
+    const unsigned char* qt = train_lds + t % Ring::DEPTH * Ring::SLOT;
+    s = dp = f32x16{};
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(qt, qrow, kk, hi), kf[kk],
+                                                  s, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          row_frag<D>(qt + Tile::BYTES, qrow, kk, hi), vf[kk], dp, 0, 0, 0);
+    }
+  }
+  while (t < rest) {
+    const unsigned char* qt = train_lds + t % Ring::DEPTH * Ring::SLOT;
+    const unsigned char* ot = qt + Tile::BYTES;
+    const unsigned char* qn = train_lds + (t + 1) % Ring::DEPTH * Ring::SLOT;
+    const unsigned char* on = qn + Tile::BYTES;
+    const float* stat =
+        reinterpret_cast<const float*>(qt + 2 * Tile::BYTES) + (wave & 2) * 64;
+    __builtin_amdgcn_sched_barrier(0);
+    auto numbers = [&](int j) {
+      const int rr = half + (j >> 1) * 16 + hi * 8 + (j & 1) * 4;
+      ls[j] = *reinterpret_cast<const f32x4*>(stat + rr);
+      de[j] = *reinterpret_cast<const f32x4*>(stat + 64 + rr);
+    };
+    auto next_rows = [&](int kk) {
+      qa[kk] = row_frag<D>(qn, qrow, kk, hi);
+      oa[kk] = row_frag<D>(on, qrow, kk, hi);
+    };
+    // what is left of the tile before; meanwhile this one's numbers and the next's rows
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      add(1, d);
+#pragma unroll
+      for (int j = d * 4 / ND; j < (d + 1) * 4 / ND; ++j) numbers(j);
+      next_rows(d * 2);
+      next_rows(d * 2 + 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // element j of a lane is row w0 + (j & 8) * 2 + hi * 8 + (j & 7); rows that do not see
+    // the key get weights of zero, whatever their log-sum
+    const int w0 = r0 + t * 64 + half;
+    if (w0 < full || w0 + 31 >= R) {
+      const int q0 = w0 + hi * 8;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int q = q0 + (j & 8) * 2 + (j & 7);
+        if (q < first || q >= R) {
+          s[j] = 0.f;
+          ls[j >> 2][j & 3] = __builtin_inff();
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the next tile's scores; meanwhile half of this one's weights
+    s1 = dp1 = f32x16{};
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+      s1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[kk], kf[kk], s1, 0, 0, 0);
+      dp1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(oa[kk], vf[kk], dp1, 0, 0, 0);
+      if (kk & 1) qc[0][kk >> 1] = col_frag<D>(qt, half, kk >> 1, lane);
+      else oc[0][kk >> 1] = col_frag<D>(ot, half, kk >> 1, lane);
+#pragma unroll
+      for (int e = kk * 8 / NKK; e < (kk + 1) * 8 / NKK; ++e) weigh(e);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the products of this half; meanwhile the other half
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      add(0, d);
+      oc[1][d] = col_frag<D>(ot, half + 16, d, lane);
+      qc[1][d] = col_frag<D>(qt, half + 16, d, lane);
+#pragma unroll
+      for (int e = d * 8 / ND; e < (d + 1) * 8 / ND; ++e) weigh(8 + e);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    s = s1;
+    dp = dp1;
+    if (++t < rest) turn(t);
+  }
+  for (; t < tiles; ++t) turn(t);
+#pragma unroll
+  for (int d = 0; d < ND; ++d) add(1, d);
+  __syncthreads();
+
+  // waves 0 and 1 finish the keys, 2 and 3 the values: each pair hands the other what it
+  // has of these, through LDS
+  auto place = [&](int w) { return reinterpret_cast<float*>(train_lds) + w * 32 * D; };
+  auto hand = [&](const f32x16 (&x)[ND]) {
+    float* to = place(wave ^ 2);
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) to[(n * 16 + j) * 64 + lane] = x[n][j];
+  };
+  if (wave >> 1) hand(dk);
+  else hand(dv);
+  __syncthreads();
+  const float* other = place(wave);
+  // element j of a lane is key j % 4 + j / 4 * 8 + hi * 4
+  const int t0 = k0 + (wave & 1) * 32 + hi * 4;
+  unsigned short* kx = a.dqkv + ((long)b * a.T + t0) * ldx + (long)(Hq + g) * D + li;
+  if (wave >> 1) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int d = (j & 3) + (j >> 2) * 8;
+      if (t0 + d >= a.T) continue;
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+        kx[(long)a.Hkv * D + d * ldx + n * 32] =
+            f2bf(other[(n * 16 + j) * 64 + lane] + dv[n][j]);
+    }
+    return;
+  }
+  float cs[16][ND / 2], sn[16][ND / 2];   // all at once: one latency
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
-    const int t = k0 + (wave & 1) * 32 + (j & 3) + (j >> 2) * 8 + hi * 4;
-    if (t >= a.T) continue;
-    unsigned short* kx = a.dqkv + ((long)b * a.T + t) * ldx + (long)(Hq + g) * D + li;
-    unsigned short* vx = kx + (long)a.Hkv * D;
-    const long p = (long)(a.start + t) * (D / 2) + li;
-#pragma unroll
-    for (int n = 0; n < ND; ++n) vx[n * 32] = f2bf(dv[n][j]);
+    const int t = min(t0 + (j & 3) + (j >> 2) * 8, a.T - 1);
+    const long at = (long)(a.start + t) * (D / 2) + li;
 #pragma unroll
     for (int n = 0; n < ND / 2; ++n) {
-      const float cs = a.cos_t[p + n * 32], sn = a.sin_t[p + n * 32];
-      const float u = dk[n][j] * a.scale, v = dk[n + ND / 2][j] * a.scale;
-      kx[n * 32] = f2bf(u * cs + v * sn);
-      kx[D / 2 + n * 32] = f2bf(v * cs - u * sn);
+      cs[j][n] = a.cos_t[at + n * 32];
+      sn[j][n] = a.sin_t[at + n * 32];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int d = (j & 3) + (j >> 2) * 8;
+    if (t0 + d >= a.T) continue;
+#pragma unroll
+    for (int n = 0; n < ND / 2; ++n) {
+      const int m = n + ND / 2;
+      const float u = (dk[n][j] + other[(n * 16 + j) * 64 + lane]) * a.scale;
+      const float v = (dk[m][j] + other[(m * 16 + j) * 64 + lane]) * a.scale;
+      kx[d * ldx + n * 32] = f2bf(u * cs[j][n] + v * sn[j][n]);
+      kx[d * ldx + D / 2 + n * 32] = f2bf(v * cs[j][n] - u * sn[j][n]);
     }
   }
 }

@@ -130,8 +130,13 @@ Tensor rope_attention_grad(Tensor gout, Tensor qkv, Tensor qk, Tensor o32,
     constexpr int DD = decltype(d)::value;
     attn_train_dq_kernel<DD>
         <<<dim3(B * Hkv, (T * a.G + 127) / 128), 256, 0, stream()>>>(a);
+    constexpr int lds = TrainRing<DD>::BYTES;
+    TORCH_CHECK(hipFuncSetAttribute(
+                    reinterpret_cast<const void*>(attn_train_dkv_kernel<DD>),
+                    hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess,
+                "cannot reserve ", lds, " bytes of LDS");
     attn_train_dkv_kernel<DD>
-        <<<dim3(B * Hkv, (T + 63) / 64), 256, 0, stream()>>>(a);
+        <<<dim3(B * Hkv, (T + 63) / 64), 256, lds, stream()>>>(a);
   });
   check_launch();
   return dqkv;

@@ -82,6 +82,29 @@ def test_attention(case):
         assert torch.equal(fused(x), fused(x.clone().requires_grad_(True)))
 
 
+@pytest.mark.parametrize("case", [
+    # tiles of 64 rows on their way three ahead, heads that divide 64 and others: less
+    # than the ring holds, its size, more; waves that join late and leave early
+    (1, 6, 2, 128, 150, 0), (1, 14, 2, 64, 100, 3), (1, 64, 1, 64, 9, 0),
+    (1, 71, 1, 128, 40, 0), (1, 128, 1, 64, 70, 0), (2, 4, 4, 128, 191, 0),
+    (1, 4, 4, 64, 193, 0), (1, 8, 4, 128, 257, 0), (1, 10, 2, 128, 97, 0),
+], ids=lambda c: "-".join(map(str, c)))
+def test_gradients_of_keys_and_values(case):
+    """Every head, also where a row's gradient or log-sum is not a number: keys it does not
+    see, of other tiles than its own, keep what they have."""
+    B, Hq, Hkv, D, T, start = case
+    x = draw(B, T, (Hq + 2 * Hkv) * D, seed=T)
+    g = draw(B, T, Hq * D, seed=T + 1)
+    fused, plain, exact = attention(Hq, Hkv, D, T, start)
+    want = grads(fused, [x], [g])
+    check(want, grads(plain, [x], [g]), grads(exact, [x], [g], torch.float64))
+    g[0, 0, 0] = float("nan")                 # the first token sees the first key alone
+    got = grads(fused, [x], [g])[1].view(B, T, Hq + 2 * Hkv, D)
+    want = want[1].view(B, T, Hq + 2 * Hkv, D)
+    assert bool(got[0, 0].isnan().any())
+    assert torch.equal(got[0, 64:], want[0, 64:]) and torch.equal(got[1:], want[1:])
+
+
 @pytest.mark.parametrize("shape", [(1, 8), (3, 5, 256), (7, 2056), (2, 3, 4096),
                                    (5, 16384)], ids=str)
 def test_norms(shape):
