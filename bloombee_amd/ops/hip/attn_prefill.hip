@@ -19,14 +19,15 @@
 //
 // The matrix cores bound long prompts (a tile is 32 products of 32 clocks a wave,
 // and its softmax about as many clocks on the vector units, which two waves a SIMD
-// overlap); the chain of tiles bounds short ones, so there the keys are split over
-// workgroups and a second kernel folds the parts.
+// overlap); the chain of tiles bounds short ones, so there the keys are shared out to two
+// groups of waves of a workgroup, whose sums meet in LDS, and split over workgroups, whose
+// parts a second kernel folds.
 //
 // Measured, 32 heads on 8 of 128: four prompts of 4096 625 us alone (880 TF/s of the
 // visible half; 675 with an address a lane, 3808 us with 16-row tiles of one head each,
 // staged through registers, weights through LDS), 2000 tokens behind 6000 270 us (299 with
-// an address a lane), one of 333 behind 1201 37 us (163), a tree of 25 behind 1500 18.5 us
-// (168). The loads alone take 293 us of the 625: what is left overlaps by half. Scores a
+// an address a lane), one of 333 behind 1201 38 us (41 with one group a workgroup), a tree
+// of 25 behind 1500 23.5 us. The loads alone take 293 us of the 625: what is left overlaps by half. Scores a
 // tile ahead of the weights within a wave took 686, 256 rows a workgroup 641 (loads 172).
 //
 // Numerics: fp32 softmax/accum; bf16 operands — matches reference tolerance
@@ -82,8 +83,10 @@ enum PrefillForm { PREFILL_PLAIN, PREFILL_GENERAL, PREFILL_TREE };
 // where a lane finds pages by shifts (0.75 us of a tree's 20).
 enum PrefillPages { PREFILL_GROUPS, PREFILL_EIGHTS, PREFILL_MIXED };
 
-template <int D, int FORM, int PAGES>
-__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
+// KG groups of four waves share out the keys of a workgroup; what each of two has found
+// meets in LDS.
+template <int D, int FORM, int PAGES, int KG>
+__global__ __launch_bounds__(256 * KG, D > 128 ? 1 : 2) void attn_prefill_kernel(
     PrefillArgs a) {
   using Tile = PrefillTile<D>;
   constexpr int KT = Tile::KT, RC = Tile::RC, NI = Tile::NI;
@@ -102,7 +105,9 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
   const int G = a.G, R = a.Tq * G;
   const int base = (int)(gridDim.y - 1 - blockIdx.y) * 128;
   const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int any = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int wave = KG > 1 ? any % 4 : any, group = KG > 1 ? any / 4 : 0;
+  unsigned char* const lds = prefill_lds + group * (2 * Tile::BYTES);
   const int lane = tid & (WAVE - 1);
   const int li = lane & 31, hi = lane >> 5;
   const int qs = a.q_start[b];
@@ -143,8 +148,10 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
 
   const int tiles = (kend - kbeg + KT - 1) / KT;
   const int per = (tiles + a.n_split - 1) / a.n_split;
-  const int t0 = kbeg + split * per * KT;
-  const int t1 = min(kend, t0 + per * KT);
+  const int turns = (per + KG - 1) / KG;         // tiles of a group
+  const int u0 = kbeg + split * per * KT, u1 = min(kend, u0 + per * KT);
+  const int t0 = u0 + group * turns * KT;
+  const int t1 = KG == 1 ? u1 : min(u1, t0 + turns * KT);
 
   // Where this lane's pieces come from. Load i of a wave brings pieces of keys (values) of
   // group group_of(i) of sixteen: of the wave's page, at offsets that are the same in every
@@ -324,25 +331,54 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void attn_prefill_kernel(
       }
   };
 
-  if (t0 < t1) {
+  // every group takes as many turns as the first one, which has most tiles
+  const int stop = KG == 1 ? t1 : t0 + min(u1 - u0, turns * KT);
+  if (u0 < u1) {
     // page numbers are looked up a tile ahead of the loads that need them
-    look_up(t0);
-    issue(t0, prefill_lds);
-    look_up(t0 + KT);
+    if (KG == 1 || t0 < t1) {
+      look_up(t0);
+      issue(t0, lds);
+      look_up(t0 + KT);
+    }
     if (!LANES) landed();
     __syncthreads();
     int buf = 0;
-    for (int kb = t0; kb < t1; kb += KT) {
+    for (int kb = t0; kb < stop; kb += KT) {
       if (kb + KT < t1) {
-        issue(kb + KT, prefill_lds + (buf ^ 1) * Tile::BYTES);
+        issue(kb + KT, lds + (buf ^ 1) * Tile::BYTES);
         look_up(kb + 2 * KT);
       }
-      if (kb <= wlast && kb + KT > wfirst)
-        compute(kb, prefill_lds + buf * Tile::BYTES);
+      if ((KG == 1 || kb < t1) && kb <= wlast && kb + KT > wfirst)
+        compute(kb, lds + buf * Tile::BYTES);
       if (!LANES) landed();
       __syncthreads();
       buf ^= 1;
     }
+  }
+  if constexpr (KG == 2) {
+    // what the second group has found goes to the first
+    static_assert(4 * (ND * 16 + 2) * 256 <= 4 * Tile::BYTES, "place");
+    float* at = reinterpret_cast<float*>(prefill_lds) + wave * (ND * 16 + 2) * 64 + lane;
+    if (group) {
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) at[(n * 16 + j) * 64] = acc[n][j];
+      at[ND * 16 * 64] = m;
+      at[(ND * 16 + 1) * 64] = l;
+    }
+    __syncthreads();
+    if (group) return;
+    const float m2 = at[ND * 16 * 64], l2 = at[(ND * 16 + 1) * 64];
+    const float f = GENERAL ? 1.f : sc2, mx = fmaxf(m, m2);
+    const float c = fast_exp2((m - mx) * f), c2 = fast_exp2((m2 - mx) * f);
+    l = l * c + l2 * c2;
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        acc[n][j] = acc[n][j] * c + at[(n * 16 + j) * 64] * c2;
+    m = mx;
   }
 
   // a row's values are spread over the two lanes of its column

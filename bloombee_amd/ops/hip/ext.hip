@@ -429,9 +429,35 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   // 38 / 195 / 51, 333 behind 1201 37 / 42 / 39, 500 behind 7000 (four splits)
   // 95 / 184 / 106, 1000 behind 4000 (two) 114 / 127 / 125.
   const long base = row_tiles * units, room = (long)a.maxp * P;
+  // beyond 2^20 keys a page's offsets would leave 32 bits
+  const bool powers = (P & (P - 1)) == 0 && P <= 1 << 20, grouped = powers && P >= 16;
   long splits = std::max<long>(1, 256 / base);
   if (room > splits * 24 * 64) splits = std::max<long>(1, 512 / base);
   a.n_split = (int)std::max<long>(1, std::min({splits, room / 128, 32L}));
+  // Two groups of waves that share out a workgroup's keys halve its chain for 4.5 us, where
+  // another split takes 4 and its sums' way through memory and back, 45 ns a workgroup; a
+  // tile takes 2.4 us. Measured, us with the splits above and one group / as chosen here:
+  // 333 behind 1201 45 / 39, behind 300 31 / 24, behind 8000 (one) 82; 2 x 333 behind 1201
+  // 54 / 41; 480 behind 100 35 / 25; 1000 behind 4000 114 / 105; 64 behind 2000 28.5 /
+  // 26.5; 1024 behind 1024 65 / 50. Chains of a tile or two keep one group, and large trees
+  // as many workgroups as they can have, for the bytes of their masks (600 tokens of 16
+  // heads of 64: 36 / 42).
+  bool two = false;
+  if (grouped && D <= 128 && base <= 256 && (!a.tree_mask || a.Tq <= 128)) {
+    const long tiles = (room + 63) / 64;
+    auto cost = [&](long s, long groups) {
+      return 2.4 * ((tiles + groups * s - 1) / (groups * s)) +
+             (s > 1 ? 4 + 0.045 * base * s : 0.) + (groups > 1 ? 4.5 : 0);
+    };
+    double least = cost(a.n_split, 1);
+    const long most = std::max<long>(1, std::min({256 / base, room / 128, 32L}));
+    for (long s = 1; s <= most; ++s)
+      if (cost(s, 2) < least) {
+        least = cost(s, 2);
+        a.n_split = (int)s;
+        two = true;
+      }
+  }
   torch::Tensor part;
   if (a.n_split > 1) {
     part = torch::empty({(long)a.n_split * units * rows * (D + 2)}, f32);
@@ -439,20 +465,25 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
     a.pml = a.pacc + (long)a.n_split * units * rows * D;
   }
   const dim3 grid(units * a.n_split, row_tiles);
-  auto launch = [&](auto d, auto form, auto pages) {
-    constexpr int DD = decltype(d)::value;
+  auto start = [&](auto d, auto form, auto pages, auto groups) {
+    constexpr int DD = decltype(d)::value, KG = decltype(groups)::value;
     auto kernel =
-        attn_prefill_kernel<DD, decltype(form)::value, decltype(pages)::value>;
-    constexpr int lds = 2 * PrefillTile<DD>::BYTES;
+        attn_prefill_kernel<DD, decltype(form)::value, decltype(pages)::value, KG>;
+    constexpr int lds = KG * 2 * PrefillTile<DD>::BYTES;
     if (lds > 64 * 1024)
       TORCH_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       lds) == hipSuccess,
                   "cannot reserve ", lds, " bytes of LDS");
-    kernel<<<grid, 256, lds, cur_stream()>>>(a);
+    kernel<<<grid, 256 * KG, lds, cur_stream()>>>(a);
     if (a.n_split > 1)
       attn_prefill_fold_kernel<DD>
           <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
+  };
+  auto launch = [&](auto d, auto form, auto pages) {
+    if constexpr (decltype(pages)::value == PREFILL_GROUPS && decltype(d)::value <= 128)
+      if (two) return start(d, form, pages, std::integral_constant<int, 2>{});
+    start(d, form, pages, std::integral_constant<int, 1>{});
   };
   auto by_dim = [&](auto form, auto pages) {
     if (D == 128) launch(std::integral_constant<int, 128>{}, form, pages);
@@ -468,10 +499,8 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
       by_dim(std::integral_constant<int, PREFILL_GENERAL>{}, pages);
     else by_dim(std::integral_constant<int, PREFILL_PLAIN>{}, pages);
   };
-  // beyond 2^20 keys a page's offsets would leave 32 bits
-  if ((P & (P - 1)) || P > 1 << 20)
-    by_dim(tree, std::integral_constant<int, PREFILL_MIXED>{});
-  else if (P < 16) by_form(std::integral_constant<int, PREFILL_EIGHTS>{});
+  if (!powers) by_dim(tree, std::integral_constant<int, PREFILL_MIXED>{});
+  else if (!grouped) by_form(std::integral_constant<int, PREFILL_EIGHTS>{});
   else by_form(std::integral_constant<int, PREFILL_GROUPS>{});
 }
 

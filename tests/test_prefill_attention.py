@@ -216,3 +216,45 @@ def test_pages_behind_the_last_key(D, P, length):
     want = ref.attn_paged(q.float(), kp.float().nan_to_num(0), vp.float(), table,
                           qs.long())
     close(ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)]), want)
+
+
+GROUPED = [
+    # sizes at which two groups of waves share out a workgroup's keys: unsplit and split,
+    # an odd number of tiles, nothing left for the second group, rows of both sides
+    (1, 32, 8, 128, 300, (0,), 320, 0),
+    (2, 32, 8, 128, 200, (500, 3), 704, 0),
+    (1, 8, 2, 64, 128, (1000,), 4096, 0),
+    (1, 8, 2, 128, 100, (0,), 2048, 0),
+    (2, 32, 8, 32, 97, (411, 900), 1024, 0),
+    (1, 32, 8, 128, 333, (400,), 752, 150),
+]
+
+
+@pytest.mark.parametrize("case", GROUPED, ids=lambda c: "-".join(map(str, c[:6])))
+@pytest.mark.parametrize("form", ["plain", "alibi", "tree", "nan"])
+def test_two_groups_of_waves(case, form):
+    B, Hq, Hkv, D, T, starts, room, window = case
+    if form == "tree" and (window or T > 128):
+        pytest.skip("large trees have one group, and no window")
+    P = 16
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=T)
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    slopes = ops.alibi_slopes_for(Hq) if form == "alibi" else None
+    tree = None
+    if form == "tree":
+        tree = torch.rand(B, T, T, generator=gen) < 0.3
+        tree |= torch.eye(T, dtype=torch.bool)
+    if form == "nan":             # a key of each half, each of another head's
+        for head, pos in ((0, starts[0] + 9), (1, starts[0] + T - 20)):
+            kp[int(table[0, pos // P]), head, pos % P, 5] = float("nan")
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long(),
+                          sliding_window=window or None, alibi_slopes=slopes,
+                          tree_mask=tree)
+    got = ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)], window=window,
+                         alibi_slopes=slopes,
+                         tree_mask=None if tree is None else tree.to(DEV)).cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert bool(want.isnan().any()) == (form == "nan")
+    close(got.nan_to_num(0), want.nan_to_num(0))
