@@ -175,6 +175,8 @@ void residual_norm(Tensor x, OptTensor parts, OptTensor routed, OptTensor ids,
   }
   if (N == 0) return;
   const size_t lds = 4 * (((W + 3) & ~3) + (size_t)a.groups + 32);
+  const bool plain = vec && a.nw && a.groups == 1 && !a.routed && !a.idw && !a.bias &&
+                     !a.bw && !a.other && W >= 4;
   by_type(tp, [&](auto p) {
     by_type(ta, [&](auto t) {
       by_bool(vec, [&](auto v) {
@@ -185,6 +187,25 @@ void residual_norm(Tensor x, OptTensor parts, OptTensor routed, OptTensor ids,
           allow_lds(k, lds);
           k<<<N, decltype(blk)::value, lds, cur_stream()>>>(a);
         };
+        // whether the row fits in R pieces a thread
+        auto held = [&](auto blk, auto pieces) {
+          constexpr int B = decltype(blk)::value, R = decltype(pieces)::value;
+          if (!plain || W > B * 4 * R) return false;
+          residual_norm_plain_kernel<decltype(p), decltype(t), B, R>
+              <<<N, B, 0, cur_stream()>>>(a);
+          return true;
+        };
+        if constexpr (V == 4) {
+          const std::integral_constant<int, 1024> many{};
+          const std::integral_constant<int, 256> few{};
+          const std::integral_constant<int, 1> one{};
+          const std::integral_constant<int, 4> four{};
+          const std::integral_constant<int, 8> eight{};
+          if (W > 2048 && N <= 256
+                  ? held(many, one) || held(many, four)
+                  : held(few, one) || held(few, four) || held(few, eight))
+            return;
+        }
         // few rows: more waves on each; many: more rows at a time
         if (W > 2048 && N <= 256) go(std::integral_constant<int, 1024>{});
         else go(std::integral_constant<int, 256>{});

@@ -42,6 +42,32 @@ def test_plain_residual_sum(N, W, cols, dt, groups, shift):
     assert torch.equal(h2[:, :W], x2.bfloat16()) and bool((h2[:, W:] == 0).all())
 
 
+@pytest.mark.parametrize("N", [3, 257])
+@pytest.mark.parametrize("W,cols", [(8, 8), (1024, 1024), (1028, 6016), (8192, 8192),
+                                    (8196, 8256), (16384, 16384), (16388, 20480)])
+@pytest.mark.parametrize("splits", [0, 1, 3])
+def test_norms_of_rows_in_registers(N, W, cols, splits):
+    """Rows that fill a thread's pieces and one vector more; without parts the residual
+    stays as it is."""
+    x, w = draw(N, W, seed=1), draw(W, seed=3)
+    x[-1, W // 2] = float("inf")                  # its row is not a number there
+    parts = draw(max(splits, 1), N, W, seed=2).bfloat16()
+    got, pending = x.clone(), ragged.Pending(parts, keep=0.5) if splits else None
+    h = ragged.residual_norm(got, pending, w, 1, 1e-5, cols)
+    want = 0.5 * x.double() + parts.double().sum(0) if splits else x.double()
+    if splits:
+        # a rounding of 32 bits a part
+        bound = 2.0 ** -22 * (x.double().abs() + parts.double().abs().sum(0))
+        assert bool((((got.double() - want).abs() <= bound) | want.isinf()).all())
+    else:
+        assert torch.equal(got, x)
+    n = want * torch.rsqrt(want.pow(2).mean(-1, keepdim=True) + 1e-5) * w.double()
+    # one rounding to bf16 behind 32-bit sums, whose terms may cancel
+    near = (h[:, :W].double() - n).abs() <= 2.01 * 2.0 ** -9 * n.abs() + 1e-5
+    assert bool((near | n.isnan()).all())
+    assert torch.equal(h[:, :W].isnan(), n.isnan()) and bool((h[:, W:] == 0).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 32), (16, 16, 96), (17, 17, 256),
                                    (33, 80, 288), (15, 15, 4128)])
 def test_router_tiles(M, N, K):
