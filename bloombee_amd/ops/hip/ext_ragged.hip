@@ -175,8 +175,8 @@ void residual_norm(Tensor x, OptTensor parts, OptTensor routed, OptTensor ids,
   }
   if (N == 0) return;
   const size_t lds = 4 * (((W + 3) & ~3) + (size_t)a.groups + 32);
-  const bool plain = vec && a.nw && a.groups == 1 && !a.routed && !a.idw && !a.bias &&
-                     !a.bw && !a.other && W >= 4;
+  const bool plain = vec && a.nw && a.groups == 1 && !a.routed && !a.idw && !a.bw &&
+                     !a.other && W >= 4;
   by_type(tp, [&](auto p) {
     by_type(ta, [&](auto t) {
       by_bool(vec, [&](auto v) {

@@ -376,7 +376,7 @@ __global__ __launch_bounds__(BLOCK) void residual_norm_kernel(ResidualArgs a) {
   }
 }
 
-// The same for one norm over a sum of parts alone: the row stays in registers, R pieces of
+// The same for one norm over a sum of parts and a bias: the row stays in registers, R pieces of
 // four a thread, every load is asked for at once and one barrier is all there is to wait
 // for: latencies, not bytes, bound a row. us in a graph, here and by the kernel above: 24
 // rows of 4096 2.7, 5.0; four parts 3.1, 5.2; 617 rows 5.8, 7.8; 1400 10.2, 12.1; 16 of 1024
@@ -389,15 +389,16 @@ __global__ __launch_bounds__(BLOCK) void residual_norm_plain_kernel(ResidualArgs
   const int W = a.W, i0 = threadIdx.x * V;
   float* xr = a.x + t * a.ldx;
   const TP* pr = (const TP*)a.parts + t * a.ldp;
-  float v[R][V], w[R][V], d[R][V];
+  float v[R][V], w[R][V], d[R][V], b[R][V];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int i = min(i0 + r * BLOCK * V, W - V);
     ldv<V>(xr + i, v[r]);
     ldv<V>(a.nw + i, w[r]);
 #pragma unroll
-    for (int j = 0; j < V; ++j) d[r][j] = 0.f;
+    for (int j = 0; j < V; ++j) d[r][j] = b[r][j] = 0.f;
     if (a.parts) ldv<V>(pr + i, d[r]);
+    if (a.bias) ldv<V>(a.bias + i, b[r]);
   }
   for (int s = 1; s < (a.parts ? a.ks : 1); ++s) {
     float u[R][V];
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(BLOCK) void residual_norm_plain_kernel(ResidualArgs
     const int i = i0 + r * BLOCK * V;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      v[r][j] = v[r][j] * a.alpha + d[r][j];
+      v[r][j] = v[r][j] * a.alpha + (a.bias ? d[r][j] + b[r][j] : d[r][j]);
       if (i < W) ss += v[r][j] * v[r][j];
     }
     if (a.parts && !a.post && i < W) stv<V>(xr + i, v[r]);

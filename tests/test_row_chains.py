@@ -45,19 +45,23 @@ def test_plain_residual_sum(N, W, cols, dt, groups, shift):
 @pytest.mark.parametrize("N", [3, 257])
 @pytest.mark.parametrize("W,cols", [(8, 8), (1024, 1024), (1028, 6016), (8192, 8192),
                                     (8196, 8256), (16384, 16384), (16388, 20480)])
-@pytest.mark.parametrize("splits", [0, 1, 3])
-def test_norms_of_rows_in_registers(N, W, cols, splits):
+@pytest.mark.parametrize("splits,biased", [(0, False), (1, False), (1, True), (3, True)])
+def test_norms_of_rows_in_registers(N, W, cols, splits, biased):
     """Rows that fill a thread's pieces and one vector more; without parts the residual
     stays as it is."""
     x, w = draw(N, W, seed=1), draw(W, seed=3)
     x[-1, W // 2] = float("inf")                  # its row is not a number there
     parts = draw(max(splits, 1), N, W, seed=2).bfloat16()
-    got, pending = x.clone(), ragged.Pending(parts, keep=0.5) if splits else None
+    bias = draw(W, seed=4) if biased else None
+    pending = ragged.Pending(parts, keep=0.5, bias=bias) if splits else None
+    got = x.clone()
     h = ragged.residual_norm(got, pending, w, 1, 1e-5, cols)
     want = 0.5 * x.double() + parts.double().sum(0) if splits else x.double()
     if splits:
-        # a rounding of 32 bits a part
-        bound = 2.0 ** -22 * (x.double().abs() + parts.double().abs().sum(0))
+        more = bias.double() if biased else torch.zeros_like(w).double()
+        want = want + more
+        # a rounding of 32 bits a term
+        bound = 2.0 ** -22 * (x.double().abs() + parts.double().abs().sum(0) + more.abs())
         assert bool((((got.double() - want).abs() <= bound) | want.isinf()).all())
     else:
         assert torch.equal(got, x)
