@@ -340,7 +340,7 @@ __global__ __launch_bounds__(256 * KG, D > 128 ? 1 : 2) void attn_prefill_kernel
       issue(t0, lds);
       look_up(t0 + KT);
     }
-    if (!LANES) landed();
+    if (!LANES) wait_loads<0>();
     __syncthreads();
     int buf = 0;
     for (int kb = t0; kb < stop; kb += KT) {
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256 * KG, D > 128 ? 1 : 2) void attn_prefill_kernel
       }
       if ((KG == 1 || kb < t1) && kb <= wlast && kb + KT > wfirst)
         compute(kb, lds + buf * Tile::BYTES);
-      if (!LANES) landed();
+      if (!LANES) wait_loads<0>();
       __syncthreads();
       buf ^= 1;
     }

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_kernel(TrainAttnArgs a) {
 
   stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
   stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
-  landed();
+  wait_loads<0>();
   __syncthreads();
   int buf = 0;
   for (int kb = 0; kb < kend; kb += KT) {
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_kernel(TrainAttnArgs a) {
           }
         }
     }
-    landed();
+    wait_loads<0>();
     __syncthreads();
     buf ^= 1;
   }
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) 
 
   stage_rows<D>(keys, 0, kend - 1, lds, wave, lane);
   stage_rows<D>(vals, 0, kend - 1, lds + Tile::BYTES, wave, lane);
-  landed();
+  wait_loads<0>();
   __syncthreads();
   int buf = 0;
   for (int kb = 0; kb < kend; kb += KT) {
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256, 2) void attn_train_dq_kernel(TrainAttnArgs a) 
         }
       }
     }
-    landed();
+    wait_loads<0>();
     __syncthreads();
     buf ^= 1;
   }
@@ -441,9 +441,6 @@ DEVINL void dma4(const void* base, unsigned ofs, unsigned l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :: "s"(l), "v"(ofs), "s"(base) : "m0");
 }
-
-template <int N>
-DEVINL void landed_but() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
 
 // Where the tiles of 64 rows wait: one is worked on, the next one's rows are read as well,
 // two are on their way.
@@ -562,8 +559,8 @@ __global__ __launch_bounds__(256, 1) void attn_train_dkv_kernel(TrainAttnArgs a)
     dk[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(dl[j], qc[j][d], dk[d], 0, 0, 0);
   };
   auto turn = [&](int t) {
-    if (tiles - t > 2) landed_but<Ring::LOADS>();
-    else landed();
+    if (tiles - t > 2) wait_loads<Ring::LOADS>();
+    else wait_loads<0>();
     // everybody's loads of this tile and the next, and everybody is done with the one
     // before, whose place another takes
     __builtin_amdgcn_s_barrier();

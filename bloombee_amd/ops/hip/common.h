@@ -93,7 +93,7 @@ DEVINL void copy16_to_lds(const unsigned short* g, unsigned char* l) {
 
 // The same in assembly: the compiler lets every read of LDS behind the builtin wait for
 // all such loads, also for those into another buffer. The wait for these is the caller's,
-// landed() or a count, ahead of a barrier.
+// wait_loads() ahead of a barrier.
 DEVINL void dma16_to_lds(const void* g, unsigned char* l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                :: "s"((unsigned)(unsigned long)(lptr_t)l), "v"(g) : "m0", "memory");
@@ -105,7 +105,12 @@ DEVINL void dma16(const void* base, unsigned ofs, unsigned l) {
                :: "s"(l), "v"(ofs), "s"(base) : "m0");
 }
 
-DEVINL void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Until at most N loads of the wave are on their way and its reads of LDS are done: behind
+// the next barrier loads of others may replace what it has read.
+template <int N>
+DEVINL void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N) : "memory");
+}
 
 __host__ DEVINL long ldiv_up(long a, long b) { return (a + b - 1) / b; }
 

@@ -27,12 +27,6 @@
 #pragma once
 #include "common.h"
 
-// Until at most N loads of the wave are on their way and its reads of LDS are done.
-template <int N>
-DEVINL void wait_loads() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(N) : "memory");
-}
-
 // A product whose sums stay where they are in the accumulation registers: with more
 // than 256 registers a wave the compiler moves them around between products (four
 // moves each). It knows nothing of the product's latency: settle() goes ahead of what
