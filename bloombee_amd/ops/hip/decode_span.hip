@@ -919,15 +919,17 @@ struct Worker {
       const unsigned* src = part_of(l, s, g);
       float* to = reinterpret_cast<float*>(wide());
       fetch(src, wide(), s.parts * HEAD);
-      if (wave == NW - 1) {
-        const u64* ml = reinterpret_cast<const u64*>(src + a.parts * HEAD) +
-                        min(lane, s.parts - 1);
+      // up to three key heads may have more splits than a wave has lanes
+      for (int i0 = 0; wave == NW - 1 && i0 < s.parts; i0 += WAVE) {
+        const int i = i0 + lane;
+        const u64* ml =
+            reinterpret_cast<const u64*>(src + a.parts * HEAD) + min(i, s.parts - 1);
         u64 got;
         int polls = 0;
         do got = peek(ml);
         while (__builtin_amdgcn_ballot_w64(!there(got)) && ++polls < PATIENCE);
         if (!there(got)) ctl->late[flag] = 1;
-        if (lane < s.parts) reinterpret_cast<u64*>(to + s.parts * HEAD)[lane] = got;
+        if (i < s.parts) reinterpret_cast<u64*>(to + s.parts * HEAD)[i] = got;
       }
       meet();
       if (late()) return false;

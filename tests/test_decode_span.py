@@ -141,6 +141,28 @@ def test_against_64_bits(sizes, norms, lengths, monkeypatch):
     assert torch.equal(s.forward_inference(x, kv, start), got)
 
 
+# more splits of a sequence than a wave has lanes, of a small model's slots for attention
+# alone, of all slots, of a wide model; the values behind the 64th are unlike the others
+@gpu
+@pytest.mark.parametrize("sizes,lengths", [
+    (SMALL, [16700]), (SMALL, [70001]), ((1536, 4352, 16, 2), [17001]),
+    ((1024, 4096, 8, 1), [300, 20000])])
+def test_many_splits(sizes, lengths, monkeypatch):
+    cfg, s = stack(*sizes, 2, False)
+    pool, kv, start = session(s, lengths)
+    weights = [{n: w.detach().clone() for n, w in b.named_parameters()}
+               for b in s.blocks]
+    table = kv.page_table().long()
+    for i in range(2):
+        pool.v_pages(i)[table[len(lengths) - 1, 64 * 256 // 16:]] += 8
+    x = torch.randn(len(lengths), 1, sizes[0], device=DEV).bfloat16()
+    want, _ = exact(cfg, weights, x, pool, kv, start, start.clamp(max=8191))
+    taken = in_one_launch(s, monkeypatch)
+    got = s.forward_inference(x, kv, start)
+    assert taken == [True]
+    assert relative(got[:, 0], want) < 2.0 ** -9 * math.sqrt(10 * 2)
+
+
 @gpu
 @pytest.mark.parametrize("page", [8, 32])
 def test_pages_and_positions(page, monkeypatch):
