@@ -52,6 +52,16 @@ class _SeqState:
     slot: int = -1    # row of the recurrent states, -1 = no recurrent layers
 
 
+def context_bound(kv, tokens: int) -> int:
+    """Tokens of the longest sequence of a session (or a view of one), those of the
+    present step of `tokens` a sequence among them, for kernels that share out their
+    work by it: the page table is as wide as the sequences may become. 0 for single
+    tokens, whose kernels look at each sequence's length, and where it is not known."""
+    if tokens == 1:
+        return 0
+    return max((s.l_spec for s in getattr(kv, "seqs", ())), default=0)
+
+
 class PagedKVCache:
     """Device-resident paged KV pool for a contiguous range of layers."""
 

@@ -11,7 +11,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 
 
@@ -74,7 +74,8 @@ class BloomBlock(torch.nn.Module):
         pt = kv.page_table()
         ops.kv_write(k, v, kp, vp, pt, start_pos)
         out = ops.attn_paged(q, kp, vp, pt, start_pos.long(), self.scale,
-                             alibi_slopes=self.alibi)
+                             alibi_slopes=self.alibi,
+                             longest=context_bound(kv, T))
         out = out.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
         return ops.linear(out, self.dense_w, bias=self.dense_b)
 

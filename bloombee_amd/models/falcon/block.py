@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.models.llama.block import RopeTables
 
@@ -75,7 +75,8 @@ class FalconBlock(torch.nn.Module):
         ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
                            start_pos)
         attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos,
-                                  self.scale)
+                                  self.scale,
+                                  longest=context_bound(kv, T))
         a = ops.linear(attn, self.o_w)
         # parallel branches: both read the SAME layernorm output
         m = ops.linear(ops.gelu_tanh(ops.linear(x, self.up_w)), self.down_w)

@@ -10,7 +10,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.gemma4.config import Gemma4Config
 from bloombee_amd.ops.reference import rope_cos_sin
 
@@ -156,7 +156,8 @@ class Gemma4Block(torch.nn.Module):
 
         attn = ops.attn_paged(q, kv.k_pages(kv_layer), kv.v_pages(kv_layer),
                               kv.page_table(), start_pos.long(), scale=1.0,
-                              window=self.window)
+                              window=self.window,
+                              longest=context_bound(kv, T))
         attn = attn.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
         a = ops.linear(attn, self.o_w)
         a = _rms1p(a, self.post_attn_norm_w, eps)

@@ -30,7 +30,7 @@ from typing import Optional, Tuple
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.ops import training
 
@@ -274,7 +274,8 @@ class LlamaBlock(torch.nn.Module):
         else:
             # tree_mask: tree-structured verify step (spec decoding)
             attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos,
-                                      self.scale, tree_mask=tree_mask)
+                                      self.scale, tree_mask=tree_mask,
+                                      longest=context_bound(kv, T))
         if fuse_norm:
             return self._fused_tail(hidden, attn)
         a = self._lin(attn, self.o_w, "o_w")

@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.models.llama.block import RopeTables
 
@@ -112,7 +112,8 @@ class MixtralBlock(torch.nn.Module):
         qkv = ops.linear(x, self.qkv_w)
         ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
                            start_pos)
-        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale)
+        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale,
+                                  longest=context_bound(kv, T))
         a = ops.linear(attn, self.o_w)
         if self._grouped(hidden):
             return ops.routed_mlp(a, self.router_w, self.expert_gate_up_w,

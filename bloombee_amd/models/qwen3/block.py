@@ -10,7 +10,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.models.llama.block import LlamaBlock, RopeTables
 
@@ -75,7 +75,7 @@ class Qwen3Block(LlamaBlock):
             attn = attn.permute(0, 2, 1, 3).reshape(B, T, Hq * D)
         else:
             attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos,
-                                      self.scale)
+                                      self.scale, longest=context_bound(kv, T))
         if fuse_norm:
             return self._fused_tail(hidden, attn)
         a = self._lin(attn, self.o_w, "o_w")

@@ -44,7 +44,7 @@ from typing import Optional
 import torch
 
 from bloombee_amd import ops
-from bloombee_amd.kv.paged import SessionHandle
+from bloombee_amd.kv.paged import SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.models.llama.block import RopeTables
 
@@ -116,7 +116,8 @@ class {{ Family }}Block(torch.nn.Module):
         k = qkv[..., Hq * D:(Hq + Hkv) * D].view(B, T, Hkv, D).permute(0, 2, 1, 3).contiguous()
         v = qkv[..., (Hq + Hkv) * D:].view(B, T, Hkv, D).permute(0, 2, 1, 3).contiguous()
         ops.kv_write(k, v, kp, vp, pt, start_pos)
-{% endif %}        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale)
+{% endif %}        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale,
+                                  longest=context_bound(kv, T))
         a = ops.linear(attn, self.o_w)
         h = hidden + a
         y = self._norm(h, self.post_norm_w{% if norm == "layernorm" %}, self.post_norm_b{% endif %})

@@ -355,7 +355,9 @@ __global__ __launch_bounds__(256 * KG, D > 128 ? 1 : 2) void attn_prefill_kernel
       buf ^= 1;
     }
   }
-  if constexpr (KG == 2) {
+  if (KG == 2 && u0 + turns * KT >= u1) {
+    if (group) return;      // it had no keys
+  } else if constexpr (KG == 2) {
     // what the second group has found goes to the first
     static_assert(4 * (ND * 16 + 2) * 256 <= 4 * Tile::BYTES, "place");
     float* at = reinterpret_cast<float*>(prefill_lds) + wave * (ND * 16 + 2) * 64 + lane;

@@ -410,30 +410,32 @@ torch::Tensor attn_decode_qkv(torch::Tensor qkv, long Hq, torch::Tensor k_pages,
       .view({B, 1, Hq * D});
 }
 
-// Launches attention of a.Tq tokens a sequence; a's tensors and strides are set.
-static void launch_attn_prefill(PrefillArgs a, int D, int P,
-                                const torch::TensorOptions& f32) {
-  // eight values of a page's row are read at once
-  TORCH_CHECK(P > 0 && P % 8 == 0, "page size must be a multiple of eight");
-  a.P = P;
-  a.p_log2 = __builtin_ctz(P);
-  const long rows = (long)a.Tq * a.G, units = (long)a.B * a.Hkv;
-  if (rows == 0 || units == 0) return;
-  const long row_tiles = (rows + 127) / 128;
+// beyond 2^20 keys a page's offsets would leave 32 bits
+static PrefillPages prefill_pages(int P) {
+  if ((P & (P - 1)) != 0 || P > 1 << 20) return PREFILL_MIXED;
+  return P >= 16 ? PREFILL_GROUPS : PREFILL_EIGHTS;
+}
+
+struct PrefillPlan { int splits; bool two; };
+
+// How the keys of attn_prefill are shared out: splits, and whether two groups of waves
+// share those of a workgroup. keys: that a row may see, at most (333 tokens behind 3000
+// with windows of 512 take 19.9 us by their windows, 29.8 by the context).
+static PrefillPlan prefill_plan(long units, int G, int Tq, int D, int P, long keys,
+                                bool tree, int window) {
+  const long base = ((long)Tq * G + 127) / 128 * units;   // workgroups without splits
+  // a workgroup's rows are 128 / G tokens, whose windows begin within a tile
+  if (window > 0) keys = std::min(keys, (long)window + 128 / G + 64);
   // A workgroup walks its keys in a chain of tiles, about 1.7 us each at D = 128
   // when it has the CU to itself. Where row tiles alone leave CUs idle the keys are
   // split until every CU has a workgroup, and until it has two where the chains
-  // stay long; no split is shorter than two tiles of the longest context the table
-  // can name. Measured with 32 heads on 8, splits as written against none / against
+  // stay long; no split is shorter than two tiles of the longest context. Measured with 32 heads on 8, splits as written against none / against
   // twice as many: 25 tokens behind 1500 20 / 41 / 20 us, 64 behind 8000
   // 38 / 195 / 51, 333 behind 1201 37 / 42 / 39, 500 behind 7000 (four splits)
   // 95 / 184 / 106, 1000 behind 4000 (two) 114 / 127 / 125.
-  const long base = row_tiles * units, room = (long)a.maxp * P;
-  // beyond 2^20 keys a page's offsets would leave 32 bits
-  const bool powers = (P & (P - 1)) == 0 && P <= 1 << 20, grouped = powers && P >= 16;
   long splits = std::max<long>(1, 256 / base);
-  if (room > splits * 24 * 64) splits = std::max<long>(1, 512 / base);
-  a.n_split = (int)std::max<long>(1, std::min({splits, room / 128, 32L}));
+  if (keys > splits * 24 * 64) splits = std::max<long>(1, 512 / base);
+  PrefillPlan plan{(int)std::max<long>(1, std::min({splits, keys / 128, 32L})), false};
   // Two groups of waves that share out a workgroup's keys halve its chain for 4.5 us, where
   // another split takes 4 and its sums' way through memory and back, 45 ns a workgroup; a
   // tile takes 2.4 us. Measured, us with the splits above and one group / as chosen here:
@@ -442,24 +444,55 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   // 26.5; 1024 behind 1024 65 / 50. Chains of a tile or two keep one group, and large trees
   // as many workgroups as they can have, for the bytes of their masks (600 tokens of 16
   // heads of 64: 36 / 42).
-  bool two = false;
-  if (grouped && D <= 128 && base <= 256 && (!a.tree_mask || a.Tq <= 128)) {
-    const long tiles = (room + 63) / 64;
+  if (prefill_pages(P) == PREFILL_GROUPS && D <= 128 && base <= 256 &&
+      (!tree || Tq <= 128)) {
+    const long tiles = (keys + 63) / 64;
     auto cost = [&](long s, long groups) {
       return 2.4 * ((tiles + groups * s - 1) / (groups * s)) +
              (s > 1 ? 4 + 0.045 * base * s : 0.) + (groups > 1 ? 4.5 : 0);
     };
     // these costs are no closer than 8% (two trees of 40 nodes behind 2000 gain 5% by them
     // and lost 4)
-    double least = cost(a.n_split, 1) / 1.08;
-    const long most = std::max<long>(1, std::min({256 / base, room / 128, 32L}));
+    double least = cost(plan.splits, 1) / 1.08;
+    const long most = std::max<long>(1, std::min({256 / base, keys / 128, 32L}));
     for (long s = 1; s <= most; ++s)
       if (cost(s, 2) < least) {
         least = cost(s, 2);
-        a.n_split = (int)s;
-        two = true;
+        plan = {(int)s, true};
       }
   }
+  return plan;
+}
+
+// Whether the launches to come are replayed later, with contexts of any length; also where
+// the stream does not tell.
+static bool captured() {
+  hipStreamCaptureStatus status;
+  if (hipStreamIsCapturing(cur_stream(), &status) == hipSuccess)
+    return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// Launches attention of a.Tq tokens a sequence; a's tensors and strides are set. longest:
+// no sequence has more tokens, these among them, as far as the caller knows; 0: unknown.
+static void launch_attn_prefill(PrefillArgs a, int D, int P,
+                                const torch::TensorOptions& f32, long longest) {
+  // eight values of a page's row are read at once
+  TORCH_CHECK(P > 0 && P % 8 == 0, "page size must be a multiple of eight");
+  a.P = P;
+  a.p_log2 = __builtin_ctz(P);
+  const long rows = (long)a.Tq * a.G, units = (long)a.B * a.Hkv;
+  if (rows == 0 || units == 0) return;
+  const long row_tiles = (rows + 127) / 128;
+  // A table is as wide as a session may become. By its width, 64 tokens that begin one of
+  // 8192 took 16 splits of two groups for their single tile: 13.5 us, 6.8 by their number.
+  long keys = (long)a.maxp * P;
+  if (longest > 0 && !captured())
+    keys = std::min(keys, ldiv_up(std::max<long>(longest, a.Tq), P) * P);
+  const PrefillPlan plan =
+      prefill_plan(units, a.G, a.Tq, D, P, keys, a.tree_mask != nullptr, a.window);
+  a.n_split = plan.splits;
   torch::Tensor part;
   if (a.n_split > 1) {
     part = torch::empty({(long)a.n_split * units * rows * (D + 2)}, f32);
@@ -484,7 +517,7 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
   };
   auto launch = [&](auto d, auto form, auto pages) {
     if constexpr (decltype(pages)::value == PREFILL_GROUPS && decltype(d)::value <= 128)
-      if (two) return start(d, form, pages, std::integral_constant<int, 2>{});
+      if (plan.two) return start(d, form, pages, std::integral_constant<int, 2>{});
     start(d, form, pages, std::integral_constant<int, 1>{});
   };
   auto by_dim = [&](auto form, auto pages) {
@@ -501,8 +534,10 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
       by_dim(std::integral_constant<int, PREFILL_GENERAL>{}, pages);
     else by_dim(std::integral_constant<int, PREFILL_PLAIN>{}, pages);
   };
-  if (!powers) by_dim(tree, std::integral_constant<int, PREFILL_MIXED>{});
-  else if (!grouped) by_form(std::integral_constant<int, PREFILL_EIGHTS>{});
+  const PrefillPages kind = prefill_pages(P);
+  if (kind == PREFILL_MIXED) by_dim(tree, std::integral_constant<int, PREFILL_MIXED>{});
+  else if (kind == PREFILL_EIGHTS)
+    by_form(std::integral_constant<int, PREFILL_EIGHTS>{});
   else by_form(std::integral_constant<int, PREFILL_GROUPS>{});
 }
 
@@ -530,7 +565,7 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
                            torch::Tensor v_pages, torch::Tensor page_table,
                            torch::Tensor q_start, double scale, long window,
                            c10::optional<torch::Tensor> alibi,
-                           c10::optional<torch::Tensor> tree_mask) {
+                           c10::optional<torch::Tensor> tree_mask, long longest) {
   CHECK_DEV(q); CHECK_BF16(q); CHECK_CONTIG(q);
   CHECK_DEV_ALL3(k_pages, page_table, q_start);
   if (alibi.has_value()) CHECK_DEV((*alibi));
@@ -555,7 +590,7 @@ torch::Tensor attn_prefill(torch::Tensor q, torch::Tensor k_pages,
   a.q_sb = a.o_sb = (long)Hq * Tq * D;
   a.q_st = a.o_st = D;
   a.q_sh = a.o_sh = (long)Tq * D;
-  launch_attn_prefill(a, D, P, q.options().dtype(at::kFloat));
+  launch_attn_prefill(a, D, P, q.options().dtype(at::kFloat), longest);
   return out;
 }
 
@@ -565,7 +600,7 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
                                torch::Tensor k_pages, torch::Tensor v_pages,
                                torch::Tensor page_table, torch::Tensor q_start,
                                double scale, long window,
-                               c10::optional<torch::Tensor> tree_mask) {
+                               c10::optional<torch::Tensor> tree_mask, long longest) {
   CHECK_DEV(qkv); CHECK_BF16(qkv); CHECK_CONTIG(qkv);
   CHECK_DEV_ALL3(k_pages, page_table, q_start);
   const int Hkv = k_pages.size(1), P = k_pages.size(2), D = k_pages.size(3);
@@ -590,7 +625,7 @@ torch::Tensor attn_prefill_qkv(torch::Tensor qkv, long Hq_,
   a.q_sh = a.o_sh = D;
   a.o_sb = (long)Tq * Hq * D;
   a.o_st = (long)Hq * D;
-  launch_attn_prefill(a, D, P, qkv.options().dtype(at::kFloat));
+  launch_attn_prefill(a, D, P, qkv.options().dtype(at::kFloat), longest);
   return out;
 }
 
@@ -1632,7 +1667,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wire_inflate_mt", &wire_inflate_mt);
   m.def("attn_decode", &attn_decode);
   m.def("attn_decode_qkv", &attn_decode_qkv);
-  m.def("attn_prefill_qkv", &attn_prefill_qkv);
+  m.def("attn_prefill_qkv", &attn_prefill_qkv, py::arg("qkv"), py::arg("Hq"),
+        py::arg("k_pages"), py::arg("v_pages"), py::arg("page_table"),
+        py::arg("q_start"), py::arg("scale"), py::arg("window"), py::arg("tree_mask"),
+        py::arg("longest") = 0);
   m.def("rope_kv_write_", &rope_kv_write_);
   m.def("norm_route", &norm_route);
   m.def("add_experts", &add_experts);
@@ -1656,7 +1694,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("stream_parts", &stream_parts);
   m.def("stream_swiglu", &stream_swiglu);
   m.def("stream_rope", &stream_rope);
-  m.def("attn_prefill", &attn_prefill);
+  m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("k_pages"),
+        py::arg("v_pages"), py::arg("page_table"), py::arg("q_start"), py::arg("scale"),
+        py::arg("window"), py::arg("alibi"), py::arg("tree_mask"),
+        py::arg("longest") = 0);
+  m.def("prefill_plan", [](long B, int Hq, int Hkv, int Tq, int D, int P, long keys,
+                           bool tree, int window) {
+    const PrefillPlan p = prefill_plan(B * Hkv, Hq / Hkv, Tq, D, P, keys, tree, window);
+    return py::make_tuple(p.splits, p.two ? 2 : 1);
+  });
   m.def("gemm_skinny", &gemm_skinny, py::arg("A"), py::arg("W"),
         py::arg("residual") = c10::nullopt, py::arg("bias") = c10::nullopt,
         py::arg("ksplit") = 0, py::arg("norm_w") = c10::nullopt,

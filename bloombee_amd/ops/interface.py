@@ -214,10 +214,12 @@ def attn_decode(
 
 def attn_prefill(
     q, k_pages, v_pages, page_table, q_start, scale: Optional[float] = None,
-    window: int = 0, alibi_slopes=None,
+    window: int = 0, alibi_slopes=None, longest: int = 0,
 ) -> torch.Tensor:
     """Multi-token causal paged attention. q: (B, Hq, Tq, D); the new tokens'
-    K/V must already be in the pages (kv_write first)."""
+    K/V must already be in the pages (kv_write first). longest: tokens of the longest
+    sequence, these among them, where the host knows (kv.paged.context_bound): the
+    kernel shares out its work by it, and by the width of the table otherwise."""
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])
     if _on_gpu(q):
@@ -230,7 +232,7 @@ def attn_prefill(
         al = (alibi_slopes.float().to(q.device).contiguous()
               if alibi_slopes is not None else None)
         return hip_ops.attn_prefill(q.contiguous(), k_pages, v_pages, page_table,
-                                    q_start.int(), scale, window, al, None)
+                                    q_start.int(), scale, window, al, None, longest)
     return ref.attn_paged(q, k_pages, v_pages, page_table, q_start, scale,
                           sliding_window=window if window > 0 else None,
                           alibi_slopes=alibi_slopes)
@@ -269,12 +271,13 @@ def rope_kv_write_(qkv, Hq: int, Hkv: int, cos, sin, position_ids,
 
 
 def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
-                   q_start, scale=None, window: int = 0, tree_mask=None):
+                   q_start, scale=None, window: int = 0, tree_mask=None,
+                   longest: int = 0):
     """Attention reading q straight from the fused QKV buffer.
 
     qkv: (B, T, (Hq+2Hkv)*D) with the q section already roped and the new
     tokens' K/V already in the pages (rope_kv_write_ first). tree_mask: as in
-    attn_paged.
+    attn_paged; longest: as in attn_prefill.
     Returns (B, T, Hq*D) — the O-projection GEMM input, no transposes.
     """
     B, T, _ = qkv.shape
@@ -292,7 +295,7 @@ def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
                 tree_mask = tree_mask.to(qkv.device).contiguous().bool()
             return hip_ops.attn_prefill_qkv(qkv, Hq, k_pages, v_pages,
                                             page_table, q_start.int(), scale,
-                                            window, tree_mask)
+                                            window, tree_mask, longest)
     q = qkv[..., : Hq * D].view(B, T, Hq, D).permute(0, 2, 1, 3).contiguous()
     if tree_mask is not None:
         out = attn_paged(q, k_pages, v_pages, page_table, q_start.long(), scale,
@@ -305,8 +308,9 @@ def attn_paged_qkv(qkv, Hq: int, Hkv: int, k_pages, v_pages, page_table,
 
 
 def attn_paged(q, k_pages, v_pages, page_table, q_start, scale=None, window: int = 0,
-               tree_mask=None, alibi_slopes=None):
-    """Unified entry: picks decode vs prefill kernel by Tq."""
+               tree_mask=None, alibi_slopes=None, longest: int = 0):
+    """Unified entry: picks decode vs prefill kernel by Tq. longest: as in
+    attn_prefill."""
     Tq = q.shape[2]
     if alibi_slopes is not None and not _on_gpu(q):
         if scale is None:
@@ -325,7 +329,7 @@ def attn_paged(q, k_pages, v_pages, page_table, q_start, scale=None, window: int
             tm = tree_mask.to(q.device).contiguous().bool()
             return hip_ops.attn_prefill(q.contiguous(), k_pages, v_pages,
                                         page_table, q_start.int(), scale, 0,
-                                        None, tm)
+                                        None, tm, longest)
         # tree-attention (spec decode verify): device-agnostic torch
         # composition (ref.attn_paged runs on GPU tensors directly)
         return ref.attn_paged(q, k_pages, v_pages, page_table,
@@ -336,7 +340,7 @@ def attn_paged(q, k_pages, v_pages, page_table, q_start, scale=None, window: int
         return attn_decode(q, k_pages, v_pages, page_table, ctx_lens, scale,
                            window, alibi_slopes=alibi_slopes)
     return attn_prefill(q, k_pages, v_pages, page_table, q_start, scale, window,
-                        alibi_slopes=alibi_slopes)
+                        alibi_slopes=alibi_slopes, longest=longest)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = None,

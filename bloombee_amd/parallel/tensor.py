@@ -26,7 +26,7 @@ import torch.distributed as dist
 
 from bloombee_amd import ops
 from bloombee_amd.engine import BlockStack
-from bloombee_amd.kv.paged import PagedKVCache, SessionHandle
+from bloombee_amd.kv.paged import PagedKVCache, SessionHandle, context_bound
 from bloombee_amd.models.base import ModelConfig
 from bloombee_amd.models.llama.block import LlamaBlock
 from bloombee_amd.utils.logging import get_logger
@@ -99,7 +99,8 @@ class TPShardedLlamaBlock(torch.nn.Module):
         pt = kv.page_table()
         ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp, pt,
                            start_pos)
-        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale)
+        attn = ops.attn_paged_qkv(qkv, Hq, Hkv, kp, vp, pt, start_pos, self.scale,
+                                  longest=context_bound(kv, T))
         a = ops.linear(attn, self.o_w)
         a = _all_reduce(a, self.group)            # RCCL all-reduce #1
         h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
