@@ -29,7 +29,7 @@ from bloombee_amd.models.llama.block import RopeTables
 from bloombee_amd.utils.logging import get_logger
 from bloombee_amd import ops
 from bloombee_amd.ops import ragged, training
-from bloombee_amd.ops.span import decode_span
+from bloombee_amd.ops.span import decode_span, span_fits
 
 logger = get_logger(__name__)
 
@@ -155,6 +155,8 @@ class BlockStack(torch.nn.Module):
             norms = getattr(blk, "span_norms", None)
             norms = norms() if norms is not None else None
             if (norms is None or "forward_inference" in blk.__dict__
+                    or blk is first and not span_fits(hidden, blk.I, blk.Hq,
+                                                      kv.k_pages(blk.layer_index))
                     or blk.rope is not first.rope
                     or not blk._fuse_norm_gate(hidden)
                     or (hasattr(kv, "host_prefix")

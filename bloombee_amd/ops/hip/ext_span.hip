@@ -80,7 +80,7 @@ bool plain(const Tensor& t, at::ScalarType type, const Tensor& like) {
 }  // namespace
 
 // Whether decode_span takes these; the same arguments.
-bool span_takes(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_t,
+static bool span_takes(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_t,
                 Tensor sin_t, OptTensor pos, Tensor start, Tensor table) {
   if (!plain(hidden, at::kBFloat16, hidden) || hidden.dim() != 3 || hidden.size(1) != 1 ||
       weights.empty() || weights.size() % 8 || weights[6].dim() != 4 ||
@@ -119,13 +119,12 @@ bool span_takes(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_
 // A decoded token of each sequence through a span of layers: hidden (M, 1, H). weights:
 // eight tensors a layer: qkv, o, gate_up, down, q norm, k norm (both empty: none), k pages,
 // v pages; the norms of the rows are folded into them. Columns of table are how far the
-// sequences may reach. groups: workgroups, each a slot's; fewer take several.
-Tensor decode_span(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_t,
-                   Tensor sin_t, OptTensor pos, Tensor start, Tensor table, double eps,
-                   double scale, long groups) {
-  TORCH_CHECK(groups >= 1 && groups <= span::SLOTS, "workgroups of a span");
-  TORCH_CHECK(span_takes(hidden, weights, Hq, cos_t, sin_t, pos, start, table),
-              "decode_span: sizes, types or layouts that the kernel does not take");
+// sequences may reach. groups: workgroups, each a slot's; fewer take several. span_takes()
+// has said yes.
+static Tensor run_span(Tensor hidden, const std::vector<Tensor>& weights, long Hq,
+                       const Tensor& cos_t, const Tensor& sin_t, const OptTensor& pos,
+                       const Tensor& start, const Tensor& table, double eps, double scale,
+                       long groups) {
   const int M = hidden.size(0), H = hidden.size(2), I = weights[3].size(1);
   const int Hkv = weights[6].size(1), P = weights[6].size(2);
   const int layers = (int)(weights.size() / 8);
@@ -184,11 +183,31 @@ Tensor decode_span(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor c
   return hidden;
 }
 
+Tensor decode_span(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_t,
+                   Tensor sin_t, OptTensor pos, Tensor start, Tensor table, double eps,
+                   double scale, long groups) {
+  TORCH_CHECK(groups >= 1 && groups <= span::SLOTS, "workgroups of a span");
+  TORCH_CHECK(span_takes(hidden, weights, Hq, cos_t, sin_t, pos, start, table),
+              "decode_span: sizes, types or layouts that the kernel does not take");
+  return run_span(hidden, weights, Hq, cos_t, sin_t, pos, start, table, eps, scale,
+                  groups);
+}
+
+// None where decode_span would raise.
+OptTensor decode_span_if(Tensor hidden, std::vector<Tensor> weights, long Hq, Tensor cos_t,
+                         Tensor sin_t, OptTensor pos, Tensor start, Tensor table,
+                         double eps, double scale) {
+  if (!span_takes(hidden, weights, Hq, cos_t, sin_t, pos, start, table))
+    return c10::nullopt;
+  return run_span(hidden, weights, Hq, cos_t, sin_t, pos, start, table, eps, scale,
+                  span::SLOTS);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("decode_span", &decode_span, py::arg("hidden"), py::arg("weights"), py::arg("Hq"),
         py::arg("cos_t"), py::arg("sin_t"), py::arg("pos"), py::arg("start"),
         py::arg("table"), py::arg("eps"), py::arg("scale"),
         py::arg("groups") = span::SLOTS);
-  m.def("span_takes", &span_takes);
+  m.def("decode_span_if", &decode_span_if);
   m.def("span_fits", &span_fits);
 }

@@ -27,23 +27,31 @@ def _whole_device(index: int) -> bool:
     return torch.cuda.get_device_properties(index).multi_processor_count >= 256
 
 
+@functools.lru_cache(256)
+def _fits(*sizes: int) -> bool:
+    return _ext().span_fits(*sizes)
+
+
+def span_fits(hidden: torch.Tensor, I: int, Hq: int, k_pages: torch.Tensor) -> bool:
+    """Whether layers of these sizes may be run in one launch: what rules out most steps,
+    to be asked ahead of every layer's tensors (22 layers that do not fit: 66 of an eager
+    step's 954 us of the host where they were walked first)."""
+    B, T, H = hidden.shape
+    return (T == 1 and hidden.is_cuda and hidden.dtype == torch.bfloat16
+            and hidden.device.index == torch.cuda.current_device()
+            and _whole_device(hidden.device.index) and k_pages.dim() == 4
+            and _fits(B, H, I, Hq, k_pages.shape[1], k_pages.shape[3],
+                      k_pages.shape[2]))
+
+
 def decode_span(hidden: torch.Tensor, weights: List[torch.Tensor], Hq: int, cos, sin,
                 position_ids: Optional[torch.Tensor], start_pos: torch.Tensor,
                 page_table: torch.Tensor, eps: float,
                 scale: float) -> Optional[torch.Tensor]:
     """hidden (B, 1, H) through layers of eight tensors each in weights: qkv, o, gate_up
     and down projections, q and k head norms (both empty: none), pages of keys and of
-    values. The new tokens' keys and values are in the pages afterwards. None where the
-    layers are to be run one by one."""
-    B, T, H = hidden.shape
-    if (T != 1 or not hidden.is_cuda or hidden.dtype != torch.bfloat16
-            or hidden.device.index != torch.cuda.current_device()
-            or not _whole_device(hidden.device.index)):
-        return None
+    values. The new tokens' keys and values are in the pages afterwards. Callers have
+    asked span_fits; None where the tensors are others than these sizes' after all."""
     pos = position_ids.int().contiguous() if position_ids is not None else None
-    args = (hidden.contiguous(), weights, Hq, cos, sin, pos, start_pos.int().contiguous(),
-            page_table)
-    ext = _ext()
-    if not ext.span_takes(*args):
-        return None
-    return ext.decode_span(*args, eps, scale)
+    return _ext().decode_span_if(hidden.contiguous(), weights, Hq, cos, sin, pos,
+                                 start_pos.int().contiguous(), page_table, eps, scale)

@@ -298,6 +298,24 @@ def test_left_to_the_blocks(monkeypatch):
     assert step() == 0
 
 
+@gpu
+def test_sizes_are_asked_ahead_of_the_layers(monkeypatch):
+    """Layers that no launch takes are not walked for it at each step."""
+    cfg = LlamaConfig(hidden_size=512, intermediate_size=1024, num_attention_heads=8,
+                      num_key_value_heads=2, head_dim=64, num_hidden_layers=6,
+                      vocab_size=64, max_position_embeddings=64)
+    s = BlockStack(cfg, 0, 6, device=DEV)
+    taken = in_one_launch(s, monkeypatch)
+    kv = s.make_kv(64).allocate(1, 32)
+    kv.extend(9)
+    asked = []
+    pages = kv.k_pages
+    monkeypatch.setattr(kv, "k_pages", lambda i: asked.append(i) or pages(i))
+    s.forward_inference(torch.randn(1, 1, 512, device=DEV).bfloat16(), kv,
+                        torch.tensor([8], dtype=torch.int32, device=DEV))
+    assert not taken and asked == [0, 0, 1, 2, 3, 4, 5]
+
+
 @pytest.mark.parametrize("change,fits", [
     ({}, True), (dict(M=4), True), (dict(M=5), False), (dict(M=0), False),
     (dict(D=64), False), (dict(P=16), True), (dict(P=4), False), (dict(P=12), False),
