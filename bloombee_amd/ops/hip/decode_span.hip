@@ -22,10 +22,17 @@
 //
 // Slots. The work of every step is cut in slots of equal size, one a CU; a workgroup owns a
 // slot for the whole launch. Nothing here needs all workgroups to be resident: one that has
-// waited long looks for slots that nobody has begun and works on those as well, from the
-// first step on (results stay where they are for the whole launch). A slot that waits
-// waits for earlier steps of slots that someone runs, so the earliest step always goes
-// on, with any number of workgroups and whatever else the device is doing.
+// waited long looks for slots that nobody has begun, and stands in for one until its own
+// workgroup comes, from the first step on (results stay where they are for the whole
+// launch; whoever runs a step stores the same bits). A slot that waits waits for earlier
+// steps of slots that someone runs, so the earliest step always goes on, with any number of
+// workgroups and whatever else the device is doing. Where another launch holds a CU for all
+// of the time, who stands in does the work of two slots, and everybody waits for it: the
+// drafter 930 us (391 alone, 800 layer by layer), four layers of 4096 columns 655 (370,
+// 400); when all who waited left their straight way for catch_up(), 1170 and 922. Beside
+// copies that fill the chip for 200 us each, the drafter 740 (1490 layer by layer; 2240 when
+// a workgroup that came late found its slot taken). Several such launches at once take as
+// long as one after the other: three drafters 1140 us, 1090 layer by layer.
 // Attention's keys and values are many times what another slot has to load: where up to
 // half the slots do for it they have nothing else (MOST_SPARED), and the others wait for
 // it with all other weights of the layer in registers.
@@ -38,7 +45,9 @@
 // Between exchanges a step is one chain of latencies, some 0.8 to 1.2 us of it. Measured on
 // the way: waits for loads that are still on their way (flat loads, registers that a branch
 // joins, loads under conditions) cost 1 to 1.5 us each; LDS reads waited for one by one 0.5;
-// ds_bpermute in place of DPP 0.1 each.
+// ds_bpermute in place of DPP 0.1 each. Registers are short all the same: SmallSizes takes
+// 256 and spills 72 more where a slot has attention and products, and both sizes keep some
+// 700 scalar registers' worth in lanes.
 
 #pragma once
 #include "common.h"
@@ -60,8 +69,12 @@ constexpr int MOST_SPARED = 128;
 // From a step's results to the first look at the others', in 64 cycles. 12: 383 us, 22 and
 // 26: 375, 30: 380; between two looks 0 or 1, 4: 390.
 constexpr int FIRST_POLL = 22;
-constexpr int PATIENCE = 200;       // looks until a workgroup looks for idle slots
-constexpr int GIVE_UP = 1 << 16;    // times that many, some ten seconds
+// Looks, of a quarter of a microsecond, until one for idle slots; such looks until a
+// workgroup steps back though there are none; times it does so, some ten seconds.
+constexpr int PATIENCE = 256, TRIES = 64, GIVE_UP = 1 << 12;
+// A slot's flag: not begun, run by its own workgroup, or by another one, which adds the steps
+// that it has done.
+constexpr int IDLE = 0, OWN = 1, STAND_IN = 2;
 
 typedef unsigned long long u64;
 typedef unsigned short u16;
@@ -119,7 +132,7 @@ static inline long fill_places(Places& p, long M, long H, long I, long Hq, long 
 
 struct Control {
   int late[2];          // of this step and of the one before
-  int got, count, more, rounds, fail;
+  int got, count, rounds, fail;
   short slot[SLOTS];
   int next[SLOTS];
   // of the launch's arguments, which are far away and not cached for long
@@ -190,35 +203,6 @@ DEVINL float sum_of_wave(float v) {
 DEVINL float sum_of_four(float v) {
   v += lane_of<XOR1>(v);
   return v + lane_of<XOR2>(v);
-}
-
-// Rows of 64 words of 8 bytes to LDS; false if some were not there for long. Waves take
-// rows in turns, without masks.
-template <int DELAY>
-DEVINL bool gather(const u64* src, unsigned char* lds, int rows, int wave, int lane) {
-  constexpr int J = 4;
-  const u64* from = src + lane;
-  u64* to = reinterpret_cast<u64*>(lds) + lane;
-  int polls = 0;
-  if (DELAY && wave < rows) __builtin_amdgcn_s_sleep(DELAY);
-  for (int r = wave; r < rows; r += NW * J) {
-    u64 v[J];
-    while (true) {
-      bool missing = false;
-#pragma unroll
-      for (int j = 0; j < J; ++j)
-        if (r + j * NW < rows) v[j] = peek(from + (r + j * NW) * 64);
-#pragma unroll
-      for (int j = 0; j < J; ++j)
-        if (r + j * NW < rows) missing |= !there(v[j]);
-      if (!__builtin_amdgcn_ballot_w64(missing)) break;
-      if (++polls == PATIENCE) return false;
-    }
-#pragma unroll
-    for (int j = 0; j < J; ++j)
-      if (r + j * NW < rows) to[(r + j * NW) * 64] = v[j];
-  }
-  return true;
 }
 
 // A slot's rows of W in one step: units [first, first + units), pairs of units where gate
@@ -376,13 +360,16 @@ struct Stream {
 
 // What differs with the size of a model: units and pieces in registers of each product.
 // Small: all that a slot has of a layer of 1024 columns, also where half of them are spared;
-// what a slot does not have is not loaded. Large: pieces follow each other.
+// what a slot does not have is not loaded. Large: pieces follow each other. Any: whatever
+// slot, a step at a time; its units divide the others', whose partial sums have room.
 struct SmallSizes {
   static constexpr bool EARLY = true, SPARES = true;
   typedef Stream<8, 1, false, true> Qkv;
   typedef Stream<2, 2, false, true> O;
   typedef Stream<12, 1, true, true> Glu;
   typedef Stream<2, 3, false, true> Down;
+  typedef Stream<2, 2, false, false> AnyRows;
+  typedef Stream<2, 2, true, false> AnyPairs;
 };
 struct LargeSizes {
   static constexpr bool EARLY = false, SPARES = false;
@@ -390,9 +377,9 @@ struct LargeSizes {
   typedef Stream<4, 2, false, false> O;
   typedef Stream<4, 2, true, false> Glu;
   typedef Stream<4, 2, false, false> Down;
+  typedef Stream<2, 4, false, false> AnyRows;
+  typedef Stream<4, 2, true, false> AnyPairs;
 };
-typedef Stream<1, 1, false, false> AnyRows;
-typedef Stream<2, 1, true, false> AnyPairs;
 
 template <class Sizes>
 struct Worker {
@@ -403,6 +390,7 @@ struct Worker {
   int flag;             // which of the two late ones is this step's
   int parts, grain;     // attention splits of the longest sequence, tokens of one
   int spared;           // slots that have attention only, no rows of the products
+  int patience;         // the other slots' is longer: who has attention only stands in first
 
   DEVINL Worker(const Args& args, unsigned char* l) : a(args), lds(l) {
     ctl = reinterpret_cast<Control*>(lds + a.lds_control);
@@ -424,6 +412,7 @@ struct Worker {
       }
     }
     parts = parts_of(longest);
+    patience = (int)blockIdx.x < spared || !spared ? PATIENCE : 8 * PATIENCE;
   }
   DEVINL int parts_of(int ctx) { return min(a.parts, (ctx + grain - 1) / grain); }
   DEVINL Layer layer_of(int l) {
@@ -468,35 +457,93 @@ struct Worker {
   // ---- waiting. Who waited in vain says so; after the next barrier all know, and take up
   // a slot that nobody has begun, if there is one.
   DEVINL bool late() { return __builtin_amdgcn_readfirstlane(ctl->late[flag]); }
-  // true: there is another slot to catch up with, or the launch has failed
-  DEVINL bool claim_idle() {
-    int* flags = reinterpret_cast<int*>(a.work);
+  DEVINL int* flags() { return reinterpret_cast<int*>(a.work); }
+  DEVINL bool idle(int slot) {
+    return __hip_atomic_load(flags() + slot, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT) == IDLE;
+  }
+  // Whether to look again after a look in vain. Only who could take up a slot leaves the
+  // straight way for it: results are late where others load long contexts, too.
+  DEVINL bool patient(int& looks) {
+    if (++looks % PATIENCE || looks % patience) return true;
+    bool any = looks == PATIENCE * TRIES;
+#pragma unroll
+    for (int k = 0; k < SLOTS; k += WAVE) any |= idle(k + lane);
+    return !__builtin_amdgcn_ballot_w64(any);
+  }
+  // Everybody begins to look at another place, so that they find different ones.
+  DEVINL void claim_idle() {
     if (tid == 0) ctl->got = SLOTS;
     meet();
-    if (ctl->more && tid < SLOTS &&
-        __hip_atomic_load(flags + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-      atomicMin(&ctl->got, tid);
+    const int own = __builtin_amdgcn_readfirstlane(ctl->slot[0]);
+    if (tid < SLOTS && idle(tid)) atomicMin(&ctl->got, (tid - own) & (SLOTS - 1));
     meet();
     if (tid == 0) {
-      const int s = ctl->got;
+      const int s = (own + ctl->got) & (SLOTS - 1);
+      int nobody = IDLE;
       ctl->late[0] = ctl->late[1] = 0;
       ctl->fail = ++ctl->rounds > GIVE_UP;
-      if (s == SLOTS) {
-        ctl->more = 0;
-      } else if (__hip_atomic_exchange(flags + s, 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT)) {
-        ctl->got = SLOTS;
-      } else {
+      if (ctl->got < SLOTS &&
+          __hip_atomic_compare_exchange_strong(flags() + s, &nobody, STAND_IN,
+                                               __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT)) {
         ctl->slot[ctl->count] = (short)s;
         ctl->next[ctl->count++] = 0;
       }
     }
     meet();
-    return __builtin_amdgcn_readfirstlane((ctl->got < SLOTS) | ctl->fail);
+  }
+  // Whether a slot's own workgroup has come, so that nobody need stand in any more; it is told
+  // how far that has got.
+  DEVINL bool relieved(int slot, int done) {
+    int seen = __hip_atomic_load(flags() + slot, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+    return seen == OWN || !__hip_atomic_compare_exchange_strong(
+                              flags() + slot, &seen, STAND_IN + done, __ATOMIC_RELAXED,
+                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // Whether this workgroup runs its own slot: not if another one has done half of it.
+  DEVINL bool begins(int slot) {
+    int seen = __hip_atomic_load(flags() + slot, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+    while (seen < STAND_IN + a.layers * STEPS / 2)
+      if (__hip_atomic_compare_exchange_strong(flags() + slot, &seen, OWN,
+                                               __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT))
+        return true;
+    return false;
+  }
+  // Rows of 64 words of 8 bytes to LDS; false if some were not there for long. Waves take
+  // rows in turns, without masks.
+  template <int DELAY>
+  DEVINL bool gather(const u64* src, unsigned char* dst, int rows) {
+    constexpr int J = 4;
+    const u64* from = src + lane;
+    u64* to = reinterpret_cast<u64*>(dst) + lane;
+    int looks = 0;
+    if (DELAY && wave < rows) __builtin_amdgcn_s_sleep(DELAY);
+    for (int r = wave; r < rows; r += NW * J) {
+      u64 v[J];
+      while (true) {
+        bool missing = false;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          if (r + j * NW < rows) v[j] = peek(from + (r + j * NW) * 64);
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          if (r + j * NW < rows) missing |= !there(v[j]);
+        if (!__builtin_amdgcn_ballot_w64(missing)) break;
+        if (!patient(looks)) return false;
+      }
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (r + j * NW < rows) to[(r + j * NW) * 64] = v[j];
+    }
+    return true;
   }
   template <int DELAY = 0>
   DEVINL void fetch(const unsigned* src, unsigned char* dst, int words) {
-    if (!gather<DELAY>(reinterpret_cast<const u64*>(src), dst, words / 128, wave, lane))
+    if (!gather<DELAY>(reinterpret_cast<const u64*>(src), dst, words / 128))
       ctl->late[flag] = 1;
   }
   // a slot's copy of what all read
@@ -723,9 +770,9 @@ struct Worker {
       const u64* src = reinterpret_cast<const u64*>(
                            exchange(l) + a.at.qkv + s.b * qkv_rows() + from * HEAD) + lane;
       u64 got;
-      int polls = 0;
+      int looks = 0;
       do got = peek(src);
-      while (__builtin_amdgcn_ballot_w64(!there(got)) && ++polls < PATIENCE);
+      while (__builtin_amdgcn_ballot_w64(!there(got)) && patient(looks));
       if (!there(got)) ctl->late[flag] = 1;
       float x = as_float((unsigned)got), y = as_float((unsigned)(got >> 32));
       if (h <= G) {
@@ -925,9 +972,9 @@ struct Worker {
         const u64* ml =
             reinterpret_cast<const u64*>(src + a.parts * HEAD) + min(i, s.parts - 1);
         u64 got;
-        int polls = 0;
+        int looks = 0;
         do got = peek(ml);
-        while (__builtin_amdgcn_ballot_w64(!there(got)) && ++polls < PATIENCE);
+        while (__builtin_amdgcn_ballot_w64(!there(got)) && patient(looks));
         if (!there(got)) ctl->late[flag] = 1;
         if (i < s.parts) reinterpret_cast<u64*>(to + s.parts * HEAD)[i] = got;
       }
@@ -951,25 +998,38 @@ struct Worker {
 
   // ---- all slots of the list, step by step; those behind come first
   DEVINL void catch_up() {
+    typedef typename Sizes::AnyRows Rows;
+    typedef typename Sizes::AnyPairs Pairs;
+    static_assert(Sizes::Qkv::UNITS % Rows::UNITS == 0 && Sizes::O::UNITS % Rows::UNITS == 0 &&
+                      Sizes::Down::UNITS % Rows::UNITS == 0 &&
+                      Sizes::Glu::UNITS % Pairs::UNITS == 0,
+                  "partial sums");
+    const int end = a.layers * STEPS;
     while (!__builtin_amdgcn_readfirstlane(ctl->fail)) {
       const int n = __builtin_amdgcn_readfirstlane(ctl->count);
-      int p = a.layers * STEPS;
+      int p = end;
       for (int i = 0; i < n; ++i)
         p = min(p, __builtin_amdgcn_readfirstlane(ctl->next[i]));
-      if (p == a.layers * STEPS) return;
+      if (p == end) return;
       const int l = p / STEPS, step = p % STEPS;
       const Layer w = layer_of(l);
-      bool ok = true;
+      bool ok = true, fetched = false;
       for (int i = 0; i < n && ok; ++i) {
         if (__builtin_amdgcn_readfirstlane(ctl->next[i]) != p) continue;
         const int slot = __builtin_amdgcn_readfirstlane(ctl->slot[i]);
+        // without work in this step: what would be looked up for it takes microseconds
+        if (step == 1 || step == 2
+                ? slot >= a.M * a.Hkv * parts || (step == 2 && parts == 1)
+                : slot < spared)
+          continue;
         meet();      // the LDS of the slot before is free
         fresh();
-        AnyRows rows;
-        AnyPairs pairs;
+        Rows rows;
+        Pairs pairs;
+        // what one slot has fetched of a product's rows is there for the others
         if (step == 0) {
           rows.begin(qkv_job(w, slot), wave, lane);
-          fetch_hidden(l, slot);
+          if (!fetched) fetch_hidden(l, slot);
           ok = run_qkv(l, qkv_job(w, slot), rows);
         } else if (step == 1 || step == 2) {
           const Split s = split_of(slot);
@@ -984,33 +1044,41 @@ struct Worker {
           }
         } else if (step == 3) {
           rows.begin(o_job(w, slot), wave, lane);
-          fetch_hidden(l, slot);      // the residual
-          fetch_attention(l, slot);
+          if (!fetched) {
+            fetch_hidden(l, slot);      // the residual
+            fetch_attention(l, slot);
+          }
           ok = run_o(l, o_job(w, slot), rows);
         } else if (step == 4) {
           pairs.begin(glu_job(w, slot), wave, lane);
-          fetch_h2(l, slot);
+          if (!fetched) fetch_h2(l, slot);
           ok = run_glu(l, glu_job(w, slot), pairs);
         } else {
           rows.begin(down_job(w, slot), wave, lane);
-          fetch_h2(l, slot);
-          fetch_mid(l, slot);
+          if (!fetched) {
+            fetch_h2(l, slot);
+            fetch_mid(l, slot);
+          }
           ok = run_down(l, down_job(w, slot), rows);
         }
+        fetched = true;
       }
       if (!ok) {
         claim_idle();
         continue;
       }
       meet();
-      if (tid < n && ctl->next[tid] == p) ctl->next[tid] = p + 1;
+      if (tid < n && ctl->next[tid] == p)
+        ctl->next[tid] =
+            tid && step == STEPS - 1 && relieved(ctl->slot[tid], p + 1) ? end : p + 1;
       meet();
     }
   }
 
   // ---- one slot, to the end. False: something was late (or the launch has failed), after
   // that many steps; what has to be done from there on is done by catch_up(). To do a step
-  // again here would cost every step: loads in flight are counted only on straight ways.
+  // again here would cost every step: loads in flight are counted only on straight ways. To
+  // come back here for the next layer takes registers (drafter 407 us for 390).
   // EARLY: the weights of a layer's other products are asked for behind the first one's
   // results, to come while attention is waited for, those of the next layer's first one
   // behind the others' results, no more at a time than an exchange takes. Otherwise those
@@ -1105,17 +1173,16 @@ __global__ __launch_bounds__(NT, 2) void decode_span_kernel(const Args a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   Worker<Sizes> w(a, lds);
   if (w.tid == 0) {
-    w.ctl->got = __hip_atomic_exchange(reinterpret_cast<int*>(a.work) + blockIdx.x, 1,
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    w.ctl->got = w.begins(blockIdx.x);
     w.ctl->late[0] = w.ctl->late[1] = w.ctl->rounds = w.ctl->fail = 0;
-    w.ctl->more = w.ctl->count = 1;
+    w.ctl->count = 1;
     w.ctl->slot[0] = (short)blockIdx.x;
   }
   for (int i = w.tid; i < a.layers * (int)sizeof(Layer) / 16; i += NT)
     reinterpret_cast<uint4v*>(w.ctl->layer)[i] =
         reinterpret_cast<const uint4v*>(a.layer)[i];
   meet();
-  if (__builtin_amdgcn_readfirstlane(w.ctl->got)) return;   // another workgroup's by now
+  if (!__builtin_amdgcn_readfirstlane(w.ctl->got)) return;
   int done = 0;
   const int slot = blockIdx.x;
   const bool attends = w.split_of(slot).any;

@@ -233,6 +233,28 @@ def test_beside_another_launch():
 
 
 @gpu
+@pytest.mark.parametrize("sizes", [QWEN, WIDE], ids=["small", "wide"])
+@pytest.mark.parametrize("cycles", [10 ** 5, 4 * 10 ** 5, 10 ** 6, 10 ** 7])
+def test_beside_a_launch_that_stays(sizes, cycles):
+    """A compute unit is held as long as a few layers, half of them, all: its slot's own
+    workgroup comes to relieve who stands in, or too late."""
+    from bloombee_amd.ops import span
+    _, s = stack(*sizes, 12, True)
+    _, kv, start = session(s, [40, 300])
+    args = arguments(s, torch.randn(2, 1, sizes[0], device=DEV).bfloat16(), kv, start)
+    want = span._ext().decode_span(*args)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(3):
+        with torch.cuda.stream(other):
+            torch.cuda._sleep(cycles)
+        got.append(span._ext().decode_span(*args))
+    torch.cuda.synchronize()
+    assert all(torch.equal(g, want) for g in got)
+
+
+@gpu
 def test_replayed():
     """A captured step at other positions, eager steps in between."""
     _, s = stack(*QWEN, 3, True)
