@@ -229,8 +229,19 @@ GROUPED = [
     (1, 32, 8, 128, 333, (400,), 752, 150),
 ]
 
+# and those at which the rule takes two for certain, trees among them: every head size,
+# unsplit and split, the second group with and without keys, a window
+TWO_GROUPS = [
+    (1, 16, 16, 128, 20, (300,), 320, 0),
+    (1, 16, 16, 32, 33, (2001,), 2064, 0),
+    (2, 16, 16, 64, 33, (1007, 3), 1040, 0),
+    (2, 32, 8, 128, 60, (3, 980), 1040, 0),
+    (1, 32, 8, 128, 333, (400,), 752, 400),
+]
 
-@pytest.mark.parametrize("case", GROUPED, ids=lambda c: "-".join(map(str, c[:6])))
+
+@pytest.mark.parametrize("case", GROUPED + TWO_GROUPS,
+                         ids=lambda c: "-".join(map(str, c[:6])))
 @pytest.mark.parametrize("form", ["plain", "alibi", "tree", "nan"])
 def test_two_groups_of_waves(case, form):
     B, Hq, Hkv, D, T, starts, room, window = case

@@ -9,6 +9,8 @@ from bloombee_amd.kv.paged import context_bound
 from bloombee_amd.kv.views import SessionView
 from bloombee_amd.models.base import resolve_config
 
+from tests.test_prefill_attention import TWO_GROUPS
+
 
 @pytest.mark.skipif(not ops.HAVE_HIP_OPS, reason="extension not built")
 @pytest.mark.parametrize("tokens,keys,window,plan", [
@@ -19,6 +21,17 @@ from bloombee_amd.models.base import resolve_config
     (4096, 8192, 64, (1, 1))])
 def test_plan(tokens, keys, window, plan):
     assert ops.hip_ops.prefill_plan(1, 32, 8, tokens, 128, 16, keys, False, window) == plan
+
+
+@pytest.mark.skipif(not ops.HAVE_HIP_OPS, reason="extension not built")
+@pytest.mark.parametrize("case", TWO_GROUPS, ids=str)
+def test_sizes_of_two_groups(case):
+    """What the device tests hold for two groups of waves has two."""
+    B, Hq, Hkv, D, T, starts, room, window = case
+    for tree in (False, True):
+        if not (tree and (window or T > 128)):
+            plan = ops.hip_ops.prefill_plan(B, Hq, Hkv, T, D, 16, room, tree, window)
+            assert plan[1] == 2
 
 
 def spy(monkeypatch):
