@@ -23,12 +23,14 @@
 // groups of waves of a workgroup, whose sums meet in LDS, and split over workgroups, whose
 // parts a second kernel folds.
 //
-// Measured, 32 heads on 8 of 128: four prompts of 4096 625 us alone (880 TF/s of the
-// visible half; 675 with an address a lane, 3808 us with 16-row tiles of one head each,
-// staged through registers, weights through LDS), 2000 tokens behind 6000 270 us (299 with
-// an address a lane), one of 333 behind 1201 38 us (41 with one group a workgroup), a tree
-// of 25 behind 1500 23.5 us. The loads alone take 293 us of the 625: what is left overlaps by half. Scores a
-// tile ahead of the weights within a wave took 686, 256 rows a workgroup 641 (loads 172).
+// Measured, 32 heads on 8 of 128, a call of several in a graph: four prompts of 4096 592 us
+// (930 TF/s of the visible half; 642 with an address a lane, 3808 with 16-row tiles of one
+// head each, staged through registers, weights through LDS; 674 in a step, whose products
+// leave less power), 2000 tokens behind 6000 250 us (277 with an address a lane), one of 333
+// behind 1201 33 us (36 with an address a lane and one group a workgroup), a tree of 25
+// behind 1500 18.2 us. Of 625 us for the first in another session the loads alone took 293:
+// what is left overlaps by half. Scores a tile ahead of the weights within a wave took 686
+// there, 256 rows a workgroup 641 (loads 172).
 //
 // Numerics: fp32 softmax/accum; bf16 operands — matches reference tolerance
 // class (test_block_exact_match.py atol 1e-4 forward on fp32 inputs).
@@ -80,7 +82,7 @@ enum PrefillForm { PREFILL_PLAIN, PREFILL_GENERAL, PREFILL_TREE };
 // A load brings keys (values) of one group of sixteen. GROUPS: pages hold a power of two of
 // keys, 16 or more, so that a load's page is the wave's. EIGHTS: of 8, which a lane looks up
 // for itself; MIXED: not a power of two. Forms of their own, since even the choice costs
-// where a lane finds pages by shifts (0.75 us of a tree's 20).
+// where a lane finds pages by shifts (0.75 us of a tree's 18).
 enum PrefillPages { PREFILL_GROUPS, PREFILL_EIGHTS, PREFILL_MIXED };
 
 // KG groups of four waves share out the keys of a workgroup; what each of two has found
@@ -238,7 +240,7 @@ __global__ __launch_bounds__(256 * KG, D > 128 ? 1 : 2) void attn_prefill_kernel
   auto compute = [&](int kb, const unsigned char* kt) {
     // keys a tree's row does not see, element n * 16 + j of s below; ahead of the scores,
     // whose registers the entries take meanwhile, and eight at a time, so that their loads
-    // overlap (25 tokens behind 1500: 19.8 us one by one, 18.5)
+    // overlap (25 tokens behind 1500: 1.3 us longer one by one)
     unsigned dead = 0;
     if (tree && kb + KT - 1 > ihi) {
       const int k0 = kb + hi * 8 - qs;

@@ -28,7 +28,7 @@
 // values 0.0022 to 0.0077 (0.0028 to 0.0079): a group's heads are summed in 32 bits here.
 //
 // 3, 4 and 6 products of 32 x 32 x D a tile. Two sequences of 1999, 32 heads on 8 of 128:
-// 136, 168 and 252 us (721, 779 and 780 TF/s of the visible half); as float32 torch
+// 132, 167 and 234 us (743, 784 and 840 TF/s of the visible half); as float32 torch
 // operations a layer's attention took 9.2 ms both ways. The first two keep the matrix cores
 // busy for 37 and 39% of that, and the vector units, which weigh and split, for as much; the
 // third is described where it stands.
@@ -464,9 +464,10 @@ struct TrainRing {
 // and the reads of columns, 16 products of the first half the rest. Two sequences of 1999,
 // 32 heads on 8 of 128: products and vector work one after the other, every read waited
 // for, 410 us; reads at once, addresses of constant offsets 291; tiles three ahead 288; the
-// order above 262; sums exchanged both ways at the end, rotation tables read at once 252.
-// 600 tokens: 103 us, now 60. What is left: a tile's 48 products take 770 ns of 1900, its
-// LDS traffic (160 KB a workgroup) about 600.
+// order above 262; sums exchanged both ways at the end, rotation tables read at once 252, all
+// in one session (234 in later ones; the wait for reads of LDS ahead of the barrier costs
+// nothing). 600 tokens: 103 us, now 60. What is left: a tile's 48 products take 770 ns of
+// 1900, its LDS traffic (160 KB a workgroup) about 600.
 template <int D>
 __global__ __launch_bounds__(256, 1) void attn_train_dkv_kernel(TrainAttnArgs a) {
   using Tile = TrainTile<D>;

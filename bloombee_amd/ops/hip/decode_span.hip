@@ -5,9 +5,9 @@
 // A launch costs 3 to 5 us whatever it does, and a small model's layer has little else:
 // its weights are 6 us of memory, its six launches took 28. Here what one step makes and
 // all workgroups need for the next goes through memory in a few KB, past the L2s, and
-// nobody waits for a launch. 28 layers of 1024 columns, one sequence of 170 tokens: 798 us
-// before, 375 here (and 3 for the launch ahead that clears the exchange); four layers of
-// 4096 columns, one of 1024 tokens: 405 and 355.
+// nobody waits for a launch. 28 layers of 1024 columns, one sequence of 170 tokens: 795 us
+// layer by layer, 392 here, 5 of them the launch ahead that clears the exchange; four layers
+// of 4096 columns, one of 1024 tokens: 404 and 358.
 //
 // Exchange. The words of a step's result (pairs of bf16, or an f32) are stored once each to
 // memory that was filled with ones in all bits, which no result has, so that a word is its
@@ -59,15 +59,15 @@ constexpr int MAX_ROWS = 4, MAX_LAYERS = 48;
 constexpr int STEPS = 6;            // of a layer
 constexpr int PITCH = 144;          // floats of a unit's partial sums, 32 x 4 and padding
 // Cached tokens of an attention split: a tile a wave. Twice that where it keeps attention
-// to slots of its own: 4 sequences of 2000 tokens 636 us, 824 with 256; 1 of 300 435, 417
-// with 256 and a merge of two splits.
+// to slots of its own: 4 sequences of 2000 tokens 646 us, 834 with 256; 1 of 300 would take
+// 4% longer unsplit.
 constexpr int MIN_PART = 256;
 constexpr int PART_FLOATS = HEAD + 2;
-// Slots for attention alone, at most: 4 sequences of 500 tokens 462 us, 623 where 32 was
+// Slots for attention alone, at most: 4 sequences of 500 tokens 473 us, 548 where 32 was
 // the most and all slots had rows of products; short contexts the same within 2%.
 constexpr int MOST_SPARED = 128;
-// From a step's results to the first look at the others', in 64 cycles. 12: 383 us, 22 and
-// 26: 375, 30: 380; between two looks 0 or 1, 4: 390.
+// From a step's results to the first look at the others', in 64 cycles. 12: 398 us, 22: 392,
+// 26: 396, 30: 401; 4 of them between two looks: 395.
 constexpr int FIRST_POLL = 22;
 // Looks, of a quarter of a microsecond, until one for idle slots; such looks until a
 // workgroup steps back though there are none; times it does so, some ten seconds.

@@ -429,21 +429,23 @@ static PrefillPlan prefill_plan(long units, int G, int Tq, int D, int P, long ke
   // A workgroup walks its keys in a chain of tiles, about 1.7 us each at D = 128
   // when it has the CU to itself. Where row tiles alone leave CUs idle the keys are
   // split until every CU has a workgroup, and until it has two where the chains
-  // stay long; no split is shorter than two tiles of the longest context. Measured with 32 heads on 8, splits as written against none / against
-  // twice as many: 25 tokens behind 1500 20 / 41 / 20 us, 64 behind 8000
-  // 38 / 195 / 51, 333 behind 1201 37 / 42 / 39, 500 behind 7000 (four splits)
-  // 95 / 184 / 106, 1000 behind 4000 (two) 114 / 127 / 125.
+  // stay long; no split is shorter than two tiles of the longest context. Measured with 32
+  // heads on 8 and one group of waves (an address a lane, alone in a graph: some 4 us more
+  // than in a row), splits as written against none / against twice as many: 25 tokens behind
+  // 1500 20 / 41 / 20 us, 64 behind 8000 38 / 195 / 51, 333 behind 1201 37 / 42 / 39, 500
+  // behind 7000 (four splits) 95 / 184 / 106, 1000 behind 4000 (two) 114 / 127 / 125.
   long splits = std::max<long>(1, 256 / base);
   if (keys > splits * 24 * 64) splits = std::max<long>(1, 512 / base);
   PrefillPlan plan{(int)std::max<long>(1, std::min({splits, keys / 128, 32L})), false};
   // Two groups of waves that share out a workgroup's keys halve its chain for 4.5 us, where
   // another split takes 4 and its sums' way through memory and back, 45 ns a workgroup; a
-  // tile takes 2.4 us. Measured, us with the splits above and one group / as chosen here:
-  // 333 behind 1201 45 / 39, behind 300 31 / 24, behind 8000 (one) 82; 2 x 333 behind 1201
-  // 54 / 41; 480 behind 100 35 / 25; 1000 behind 4000 114 / 105; 64 behind 2000 28.5 /
-  // 26.5; 1024 behind 1024 65 / 50. Chains of a tile or two keep one group, and large trees
-  // as many workgroups as they can have, for the bytes of their masks (600 tokens of 16
-  // heads of 64: 36 / 42).
+  // tile takes 2.4 us. Measured, a call of several in a graph, us with the splits above and
+  // one group, an address a lane / as chosen here: 333 behind none 21 / 14, behind 300
+  // 25 / 19, behind 1201 36 / 33, behind 8000 (one group) 78 / 72; 2 x 333 behind 1201
+  // 43 / 35; 480 behind 100 28.5 / 19.5; 1000 behind 4000 111 / 97; 64 behind 2000
+  // 22.5 / 21; 1024 behind 1024 57 / 45.5. Chains of a tile or two keep one group, and large
+  // trees as many workgroups as they can have, for the bytes of their masks (600 tokens of
+  // 16 heads of 64: 31; two groups take a sixth more).
   if (prefill_pages(P) == PREFILL_GROUPS && D <= 128 && base <= 256 &&
       (!tree || Tq <= 128)) {
     const long tiles = (keys + 63) / 64;
