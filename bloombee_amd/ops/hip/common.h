@@ -99,10 +99,18 @@ DEVINL void dma16_to_lds(const void* g, unsigned char* l) {
                :: "s"((unsigned)(unsigned long)(lptr_t)l), "v"(g) : "m0", "memory");
 }
 
-// From base + ofs bytes, base and l the wave's: nothing to calculate but ofs.
+// From base + ofs bytes, base and l the wave's: nothing to calculate but ofs. ONCE: what
+// no other workgroup reads goes through the caches without a stay (whole lines only: the
+// other half of one would be read again). 235 MB of random bits, 256 workgroups that have
+// 32 KB each on their way: 6.2 TB/s, 6.7 with it.
+template <bool ONCE = false>
 DEVINL void dma16(const void* base, unsigned ofs, unsigned l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(l), "v"(ofs), "s"(base) : "m0");
+  if constexpr (ONCE)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :: "s"(l), "v"(ofs), "s"(base) : "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :: "s"(l), "v"(ofs), "s"(base) : "m0");
 }
 
 // Until at most N loads of the wave are on their way and its reads of LDS are done: behind

@@ -1164,7 +1164,7 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
     r.splits = 1;
     RowsGlu glu{a.N / 2, a.N / 2, a.N / 2};
     glu.eps = a.eps;
-    rows_launch(gemm_rows_glu_kernel<FewRows, false, true>, ldiv_up(a.N, FewRows::BN),
+    rows_launch(gemm_rows_glu_kernel<FewRows, false, true, true>, ldiv_up(a.N, FewRows::BN),
                 FewRows::THREADS, FewRows::LDS, cur_stream(), r, glu);
     return C;
   }
@@ -1557,7 +1557,7 @@ static RowsArgs rows_args(torch::Tensor& A, torch::Tensor& W) {
 static void rows_product(RowsArgs& a, const RowsPlan& plan) {
   rows_tile(plan.tile, [&](auto tile) {
     typedef decltype(tile) T;
-    rows_launch(gemm_rows_kernel<T>,
+    rows_launch(a.M <= T::BM ? gemm_rows_kernel<T, true> : gemm_rows_kernel<T>,
                 ldiv_up(a.M, T::BM) * ldiv_up(a.N, T::BN) * a.splits, T::THREADS, T::LDS,
                 cur_stream(), a);
   });
@@ -1593,7 +1593,7 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
     a.part = part.data_ptr<float>();
   }
   if (few)
-    rows_launch(gemm_rows_kernel<FewRows>, ldiv_up(a.N, FewRows::BN) * a.splits,
+    rows_launch(gemm_rows_kernel<FewRows, true>, ldiv_up(a.N, FewRows::BN) * a.splits,
                 FewRows::THREADS, FewRows::LDS, cur_stream(), a);
   else
     rows_product(a, plan);
@@ -1610,7 +1610,8 @@ static void rows_glu(RowsArgs& a, const RowsGlu& glu) {
   rows_tile(rows_plan(a.M, 2L * glu.F, a.K, true).tile, [&](auto tile) {
     typedef decltype(tile) T;
     if constexpr (T::WK == 1)
-      rows_launch(gemm_rows_glu_kernel<T, CLAMPED>,
+      rows_launch(a.M <= T::BM ? gemm_rows_glu_kernel<T, CLAMPED, false, true>
+                               : gemm_rows_glu_kernel<T, CLAMPED>,
                   ldiv_up(a.M, T::BM) * ldiv_up(glu.ldc, T::BN / 2), T::THREADS, T::LDS,
                   cur_stream(), a, glu);
   });

@@ -99,11 +99,13 @@ struct RowsTile {
   // Sums of `steps` stages. ofs: bytes from ap (j < AJ) or wp, which move on by a
   // stage's columns (wp by w_step); beyond(j): what the rows of a load lie behind wp, the
   // wave's. NORM: rows of A are divided by their root mean square, columns of K; a row's
-  // sum of squares is the diagonal of A A^T, made from the fragments at hand.
-  template <bool NORM = false, typename B>
+  // sum of squares is the diagonal of A A^T, made from the fragments at hand. ONCE: nobody
+  // else reads these rows of W, and stage `begin` comes first, number 0 behind the last.
+  template <bool NORM = false, bool ONCE = false, typename B>
   static DEVINL void run(const unsigned (&ofs)[LPW], const unsigned short* ap,
                          const unsigned short* wp, int steps, unsigned char* lds,
-                         Acc& acc, B beyond, long w_step = BK, float eps = 0.f) {
+                         Acc& acc, B beyond, long w_step = BK, float eps = 0.f,
+                         int begin = 0) {
     const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int wk = wave % WK, wn = wave / WK % WN, wm = wave / (WK * WN);
@@ -114,11 +116,30 @@ struct RowsTile {
       for (int n = 0; n < NI; ++n) acc[m][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
     if (steps <= 0) return;
 
+    int a_left = steps - begin, w_left = a_left;
+    if constexpr (ONCE) {
+      ap += (long)begin * BK;
+      wp += begin * w_step;
+    }
+    auto next_a = [&]() {
+      ap += BK;
+      if (ONCE && --a_left == 0) {
+        ap -= (long)steps * BK;
+        a_left = steps;
+      }
+    };
+    auto next_w = [&]() {
+      wp += w_step;
+      if (ONCE && --w_left == 0) {
+        wp -= steps * w_step;
+        w_left = steps;
+      }
+    };
     auto load = [&](int j, int slot_a, int slot_w) {
       if (j < AJ)
         dma16(ap, ofs[j], base + slot_a * (BM * RB) + (j * NW + wave) * 1024);
       else
-        dma16(wp + beyond(j), ofs[j],
+        dma16<ONCE>(wp + beyond(j), ofs[j],
               base + WBASE + slot_w * (BN * RB) + ((j - AJ) * NW + wave) * 1024);
     };
     // load i of an iteration: of the operand with fewer buffers first
@@ -217,15 +238,15 @@ struct RowsTile {
       if (s < steps) {
 #pragma unroll
         for (int j = 0; j < LPW; ++j) load(j, s, s);
-        ap += BK;
-        wp += w_step;
+        next_a();
+        next_w();
       }
     if (MORE && ST < steps) {
 #pragma unroll
       for (int j = 0; j < LPW; ++j)
         if ((j < AJ) == (MORE == 1)) load(j, ST, ST);
-      if (MORE == 1) ap += BK;
-      else wp += w_step;
+      if (MORE == 1) next_a();
+      else next_w();
       wait_loads<(ST - 1) * LPW + EX>();
     } else {
       wait(min(ST, steps) - 1);
@@ -240,8 +261,8 @@ struct RowsTile {
       barrier();
       const int na = a + 1 == SA ? 0 : a + 1, nw = w + 1 == SW ? 0 : w + 1;
       phase(1, na, nw, std::true_type{}, a, w);
-      ap += BK;
-      wp += w_step;
+      next_a();
+      next_w();
       a = na;
       w = nw;
       if (MINW == 1) settle();
@@ -368,8 +389,17 @@ DEVINL void rows_place(int M, int n_tiles, int& m0, int& nt, int& split) {
   nt = id / rows;
 }
 
-// grid: row tiles * column tiles * splits; K % BK == 0, N % 8 == 0
-template <typename T>
+// Where a workgroup begins with K: rows of W are often a multiple of 4 KiB apart, so that
+// workgroups in step read from a part of memory's channels at a time; an eighth of K apart
+// by XCD, they read from all. us, W from memory, without, with, and with ONCE: 64 rows of
+// 28672 x 4096 gated 51.2, 42.1, 38.9; 97 rows 54.3, 49.4, 46.2; 8192 x 8192, W alone 63.0,
+// 48.4. Rows of 10 KiB have no such difference, splits begin apart as it is (same_channels;
+// 4096 x 14336 in 8, 40 rows 23.6, 27.6), and where more row tiles share W, their products
+// bound it: 333 rows 83.0, 83.5; 4096 rows 715, 713.
+DEVINL int rows_begin(int steps) { return (int)(blockIdx.x % 8) * steps / 8; }
+
+// grid: row tiles * column tiles * splits; K % BK == 0, N % 8 == 0. ONCE: one row tile.
+template <typename T, bool ONCE = false>
 __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_kernel(RowsArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & (WAVE - 1);
@@ -394,9 +424,12 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_kernel(RowsArgs
   }
   typename T::Acc acc;
   const long w_step = T::TURNED ? 64L * a.N : T::BK;
-  T::run(ofs, a.A + (long)m0 * a.K + (long)first * T::BK,
-         a.W + (T::TURNED ? (long)n0 : (long)n0 * a.K) + first * w_step,
-         min(all, first + per) - first, lds, acc, [](int) { return 0L; }, w_step);
+  const int steps = min(all, first + per) - first;
+  T::template run<false, ONCE>(
+      ofs, a.A + (long)m0 * a.K + (long)first * T::BK,
+      a.W + (T::TURNED ? (long)n0 : (long)n0 * a.K) + first * w_step, steps, lds, acc,
+      [](int) { return 0L; }, w_step, 0.f,
+      ONCE && !T::TURNED && a.splits == 1 ? rows_begin(steps) : 0);
 
   const int c0 = n0 + T::col0(), r0 = m0 + T::row0();
   constexpr int S = T::COLS / 16;
@@ -455,7 +488,7 @@ struct RowsGlu {
 // eight ups: half of a lane's sums change places with those of the lane 32 on, and every
 // lane has both. grid: row tiles * tiles of BN / 2 of C's columns; F, ldc % 8 == 0
 // NORM: of the rows of A, their norm's weight folded into W.
-template <typename T, bool CLAMPED, bool NORM = false>
+template <typename T, bool CLAMPED, bool NORM = false, bool ONCE = false>
 __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(RowsArgs a,
                                                                             RowsGlu glu) {
   static_assert(8 % T::RPC == 0, "rows of a load are of one kind");
@@ -475,10 +508,10 @@ __global__ __launch_bounds__(T::THREADS, T::MINW) void gemm_rows_glu_kernel(Rows
     ofs[j] = (unsigned)row * (unsigned)(a.K * 2) + T::load_byte(j, wave, lane);
   }
   typename T::Acc acc;
-  T::template run<NORM>(
+  T::template run<NORM, ONCE>(
       ofs, a.A + (long)m0 * a.K, a.W + (long)w0 * a.K, a.K / T::BK, lds, acc,
       [&](int j) { return (long)(T::load_row(j, wave, 0) / 8 % 2) * glu.up * a.K; }, T::BK,
-      glu.eps);
+      glu.eps, ONCE ? rows_begin(a.K / T::BK) : 0);
 
   const int c0 = n0 + T::col0() / 2, r0 = m0 + T::row0();
   constexpr int NO = T::COLS / 16, S = (NO + 1) / 2;

@@ -107,6 +107,24 @@ def test_few_rows_gated(M, N, K):
                  + 2.0 ** -18 * (tol[0] * (u.abs() + 1) + tol[1] * (g.abs() + 1))).all())
 
 
+@pytest.mark.parametrize("K", [256, 320, 448, 512, 576, 4096])
+@pytest.mark.parametrize("M", [40, 64])
+def test_one_row_tile(M, K):
+    """Each XCD begins with another stage of K, of fewer than eight too."""
+    N = 8192
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    assert ops.hip_ops.rows_plan(M, N, K, False)[1] == 1 or K == 4096
+    want = x.double() @ w.double().T
+    terms = x.double().abs() @ w.double().abs().T
+    assert close(ops.hip_ops.gemm_rows(x, w, None, None), want, terms)
+    g, u = want.chunk(2, -1)
+    tol = terms.chunk(2, -1)
+    got = ops.hip_ops.gemm_rows_swiglu(x, w)
+    want = torch.nn.functional.silu(g) * u
+    assert bool(((got.double() - want).abs() <= 2.0 ** -8 * want.abs()
+                 + 2.0 ** -19 * (tol[0] * u.abs() + tol[1] * g.abs()) + 1e-30).all())
+
+
 @pytest.mark.parametrize("M,F,up,cols,K", [
     (33, 8, 8, 64, 256), (65, 1000, 1024, 1088, 320), (200, 4096, 4100, 4096, 256),
     (333, 712, 715, 768, 576), (617, 1400, 1400, 1408, 384), (194, 21360, 21376, 21504, 256)])
