@@ -246,8 +246,8 @@ struct Stream {
       const int unit = min(j.first + g * PER + (PAIRED ? u / 2 : u), j.last);
       const unsigned at = (unsigned)(unit * 4 * j.K + s * 128) * 2 +
                           (PAIRED && (u & 1) ? j.up : 0) + lane_ofs;
-      w[d][u] = *reinterpret_cast<const IN_MEMORY short8*>(
-          reinterpret_cast<const IN_MEMORY char*>(j.W) + at);
+      w[d][u] = __builtin_nontemporal_load(reinterpret_cast<const IN_MEMORY short8*>(
+          reinterpret_cast<const IN_MEMORY char*>(j.W) + at));
     }
   }
   DEVINL static unsigned place(int K, int lane) {
