@@ -6,8 +6,9 @@
 // its weights are 6 us of memory, its six launches took 28. Here what one step makes and
 // all workgroups need for the next goes through memory in a few KB, past the L2s, and
 // nobody waits for a launch. 28 layers of 1024 columns, one sequence of 170 tokens: 795 us
-// layer by layer, 392 here, 5 of them the launch ahead that clears the exchange; four layers
-// of 4096 columns, one of 1024 tokens: 404 and 358.
+// layer by layer, 385 here, 5 of them the launch ahead that clears the exchange; four layers
+// of 4096 columns, one of 1024 tokens: 404 and 328 (358 where weights took their place in
+// the caches, 333 with two pieces of the down projection on their way for four).
 //
 // Exchange. The words of a step's result (pairs of bf16, or an f32) are stored once each to
 // memory that was filled with ones in all bits, which no result has, so that a word is its
@@ -376,7 +377,7 @@ struct LargeSizes {
   typedef Stream<6, 2, false, false> Qkv;
   typedef Stream<4, 2, false, false> O;
   typedef Stream<4, 2, true, false> Glu;
-  typedef Stream<4, 2, false, false> Down;
+  typedef Stream<4, 4, false, false> Down;
   typedef Stream<2, 4, false, false> AnyRows;
   typedef Stream<4, 2, true, false> AnyPairs;
 };
