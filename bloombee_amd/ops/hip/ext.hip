@@ -1110,18 +1110,46 @@ static int few_splits(long N, long K) {
   return best;
 }
 
-// Whether it beats the gated products of gemm_stream.hip and gemm_skinny.hip: where its
-// workgroups fill the chip's rounds. Up to 16 rows are left to those, which are 2 us faster
-// in a step than alone, this is not. us alone, those and this: 28672 x 4096: 1 row 45.3,
-// 45.0; 16 rows 46.9, 44.7; 32 50.4, 47.2. 27648 x 5120, 32 rows: 63.3, 55.0; 12288 x 1536
-// 12.8, 10.5; 57344 x 8192 188.2, 167.7; 128256 x 4096 206.3, 196.2. Half empty, 17 rows:
-// 22016 x 4096 39.8, 41.2; 36864 x 4096 62.3, 63.7; 6144 x 4096 14.2, 17.2.
+// The same 32 to 160 columns wide, unsplit. What a CU reads bounds them where memory does
+// not: W's columns, A again for every workgroup, 45 B a ns. So the width is the one that
+// leaves a CU the fewest columns, and of those the widest, whose workgroups read A the
+// least. 32 rows, gated, us for 32, 64, 96, 128 and 160: 28672 x 4096 45.7, 41.6, 50.4, 36.4,
+// 38.4; 24576 x 4096 35.0, 36.6, 32.4, 33.7, 36.8; 36864 x 4096 57.0, 57.4, 56.5, 63.5, 46.6;
+// 16384 x 4096 24.2, 22.1, 25.3, 28.5, 33.6; 8192 x 4096 14.0, 18.7, 22.8, 26.9, 31.4; 8 rows
+// of 28672 x 4096 41.1, 38.6, 47.0, 36.3, 36.8.
+static int few_width(long N) {
+  int best = 0;
+  long least = 0;
+  for (int bn : {160, 128, 96, 64, 32}) {
+    const long columns = ldiv_up(ldiv_up(N, bn), 256) * bn;
+    if (!best || columns < least) {
+      best = bn;
+      least = columns;
+    }
+  }
+  return best;
+}
+
+template <typename F>
+static void few_tile(int width, F f) {
+  switch (width) {
+    case 32: f(RowsTile<32, 32, 2, 1, 2, 4, 2>{}); break;
+    case 64: f(FewRows{}); break;
+    case 96: f(RowsTile<32, 96, 2, 2, 1, 4, 2>{}); break;
+    case 128: f(RowsTile<32, 128, 2, 2, 1, 4, 2>{}); break;
+    default: f(RowsTile<32, 160, 2, 2, 1, 4, 2>{}); break;
+  }
+}
+
+// Whether it beats the gated products of gemm_stream.hip and gemm_skinny.hip, which the
+// smallest are left to and those whose W does not begin at 16 bytes. us in a graph, W from
+// memory, the faster of those and this: 28672 x 4096: 1 row 45.9, 36.8; 32 rows 46.9, 36.8.
+// 57344 x 8192: 161, 146; 183, 162. 36864 x 4096 60.3, 49.5; 72.7, 47.6. 20480 x 5120 46.7,
+// 35.4; 57.9, 40.7. 12288 x 1536 11.5, 9.1; 10.8, 9.8. 8192 x 4096 14.5, 12.5; 17.0, 13.9.
+// 6144 x 1024 5.6, 5.7; 6.8, 5.7. 22528 x 768 10.6, 8.8; 13.2, 9.4. 1536 x 512 3.8, 3.8; 4.5,
+// 4.2. 512 x 256 3.0, 3.3; 8 rows 3.2, 3.4; 32 rows 3.7, 3.5.
 static bool few_swiglu(long M, long N, long K) {
-  const long wgs = ldiv_up(N, 64);
-  if (K % 128 || K < 1024 || M <= 16 || M > 32) return false;
-  if (wgs <= 256) return wgs >= 190;
-  if (wgs <= 512) return wgs >= 410;
-  return wgs * 20 >= ldiv_up(wgs, 512) * 512 * 17;
+  return M > 0 && M <= 32 && K % 128 == 0 && (M > 8 || K > 256 || N > 2048);
 }
 
 // Whether it beats their sums: wherever those want the split form (whose waves take W by
@@ -1164,8 +1192,11 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
     r.splits = 1;
     RowsGlu glu{a.N / 2, a.N / 2, a.N / 2};
     glu.eps = a.eps;
-    rows_launch(gemm_rows_glu_kernel<FewRows, false, true, true>, ldiv_up(a.N, FewRows::BN),
-                FewRows::THREADS, FewRows::LDS, cur_stream(), r, glu);
+    few_tile(few_width(a.N), [&](auto tile) {
+      typedef decltype(tile) T;
+      rows_launch(gemm_rows_glu_kernel<T, false, true, true>, ldiv_up(a.N, T::BN),
+                  T::THREADS, T::LDS, cur_stream(), r, glu);
+    });
     return C;
   }
   if (!stream_swiglu(a.M, a.N, a.K)) {
@@ -1681,6 +1712,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_sums", &few_sums);
   m.def("few_splits", &few_splits);
   m.def("few_swiglu", &few_swiglu);
+  m.def("few_width", &few_width);
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {
@@ -1693,9 +1725,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm_swiglu", &gemm_swiglu);
   m.def("gemm_rope_kv", &gemm_rope_kv);
   m.def("stream_rows", &stream_rows);
+  m.def("stream_swiglu", &stream_swiglu);
   m.def("stream_sums", &stream_sums);
   m.def("stream_parts", &stream_parts);
-  m.def("stream_swiglu", &stream_swiglu);
   m.def("stream_rope", &stream_rope);
   m.def("attn_prefill", &attn_prefill, py::arg("q"), py::arg("k_pages"),
         py::arg("v_pages"), py::arg("page_table"), py::arg("q_start"), py::arg("scale"),

@@ -107,6 +107,18 @@ def test_few_rows_gated(M, N, K):
                  + 2.0 ** -18 * (tol[0] * (u.abs() + 1) + tol[1] * (g.abs() + 1))).all())
 
 
+@pytest.mark.parametrize("N,K,width", [
+    (64, 512, 32), (8192, 256, 32), (8256, 512, 64), (16384, 768, 64), (16448, 256, 96),
+    (24576, 1024, 96), (24640, 512, 128), (32768, 256, 128), (32832, 512, 160),
+    (40960, 256, 160), (41024, 256, 96)])
+@pytest.mark.parametrize("M", [1, 9, 32])
+def test_widths_of_few_rows(M, N, K, width):
+    """One tile and strip short of a round of workgroups, or past it; fewer stages than
+    buffers."""
+    test_few_rows_gated(M, N, K)
+    assert ops.hip_ops.few_width(N) == width
+
+
 @pytest.mark.parametrize("K", [256, 320, 448, 512, 576, 4096])
 @pytest.mark.parametrize("M", [40, 64])
 def test_one_row_tile(M, K):
