@@ -19,6 +19,7 @@
 #include "gemm_skinny.hip"
 #include "gemm_stream.hip"
 #include "gemm_rows_host.h"
+#include "gemm_rows_rope.hip"
 #include "moe_gemm.hip"
 #include "moe_route.hip"
 #include "w4_gemm.hip"
@@ -1152,6 +1153,17 @@ static bool few_swiglu(long M, long N, long K) {
   return M > 0 && M <= 32 && K % 128 == 0 && (M > 8 || K > 256 || N > 2048);
 }
 
+// Whether it beats the turned projections of gemm_stream.hip and gemm_skinny.hip (a second
+// launch folds its splits): few columns leave it too few workgroups for a long K, and the
+// smallest are left to the former. us in a graph, W from memory, the faster of those and
+// this: 6144 x 4096: 1 row 13.8, 13.5; 8 rows 15.2, 13.5; 32 rows 20.2, 16.2. 4096 x 1024:
+// 5.6, 5.5; 6.0, 5.9; 8.2, 7.1. 24576 x 8192 78.6, 70.7; 85.9, 71.8; 106, 74.0. 12288 x 4096
+// 25.3, 20.9; 26.4, 21.2; 29.7, 24.9. 2048 x 2048 7.5, 7.0; 7.9, 7.2; 10.1, 8.6. 2048 x 4096
+// 8.9, 11.0; 9.4, 11.2; 10.5, 13.0. 1024 x 512 3.8, 4.2; 4.0, 4.3; 5.3, 4.8.
+static bool few_rope(long M, long N, long K) {
+  return M > 0 && M <= 32 && (K <= 2048 || N >= 4096) && (M > 16 || K >= 1024);
+}
+
 // Whether it beats their sums: wherever those want the split form (whose waves take W by
 // 64 B of a row), and from some rows on where the one-launch form reads all of A for every
 // 16 columns. us in a graph, W from memory, those and this: 4096 x 14336: 9 rows 25.4, 25.7;
@@ -1261,6 +1273,14 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq
   a.start = start_pos.data_ptr<int>();
   a.k_pages = bf_ptr_mut(k_pages);
   a.v_pages = bf_ptr_mut(v_pages);
+  if ((size_t)W.data_ptr() % 16 == 0 && few_rope(a.M, a.N, a.K)) {
+    few_tile(few_width(a.N), [&](auto tile) {
+      typedef decltype(tile) T;
+      rows_launch(gemm_rows_rope_kernel<T>, ldiv_up(a.N, T::BN), T::THREADS, T::LDS,
+                  cur_stream(), a);
+    });
+    return C;
+  }
   if (stream_rope(a.M, a.N, a.K)) {
     by_rows(a.M, [&](auto mt, auto xn) {
       constexpr int MT = decltype(mt)::value;
@@ -1713,6 +1733,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_splits", &few_splits);
   m.def("few_swiglu", &few_swiglu);
   m.def("few_width", &few_width);
+  m.def("few_rope", &few_rope);
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {

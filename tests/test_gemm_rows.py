@@ -119,6 +119,35 @@ def test_widths_of_few_rows(M, N, K, width):
     assert ops.hip_ops.few_width(N) == width
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,K,width", [
+    (4, 2, 32, 1024, 32), (61, 1, 128, 1024, 32), (28, 6, 256, 1024, 64),
+    (200, 28, 96, 1024, 96), (1000, 10, 32, 1024, 128), (260, 2, 128, 1280, 160)])
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 3), (32, 1), (2, 11)])
+@pytest.mark.parametrize("placed", [False, True])
+def test_turned_projections(Hq, Hkv, D, K, width, B, T, placed):
+    """Tiles that end within a head or take several; rows short of a strip."""
+    N = (Hq + 2 * Hkv) * D
+    assert ops.hip_ops.few_rope(B * T, N, K) and ops.hip_ops.few_width(N) == width
+    x, w = draw(B, T, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    P, start = 16, torch.arange(B, device=DEV, dtype=torch.int32) * 7 + 13
+    maxp = (7 * B + 13 + T) // P + 1
+    table = torch.randperm(B * maxp, device=DEV).int().view(B, maxp)
+    kp = draw(B * maxp, Hkv, P, D, seed=3)
+    vp = draw(B * maxp, Hkv, D, P, seed=4)
+    pos = torch.randint(0, 400, (B, T), device=DEV).int() if placed else None
+    cos, sin = (t.to(DEV) for t in ops.rope_cos_sin(D, 512))
+    y = x.double()
+    z = (y * (y.square().mean(-1, keepdim=True) + 1e-5).rsqrt()) @ w.double().T
+    want, kw, vw = z.float().cpu(), kp.float().cpu(), vp.float().cpu()
+    ops.rope_kv_write_(want, Hq, Hkv, cos.cpu(), sin.cpu(),
+                       None if pos is None else pos.cpu(), kw, vw, table.cpu(),
+                       start.cpu())
+    got = ops.linear_rope_kv(x, w, 1e-5, Hq, Hkv, cos, sin, pos, kp, vp, table, start)
+    # one rounding of 32-bit sums, 2^-9 of a value; turns and root within 2^-18 of terms
+    for a, b in ((got[..., :Hq * D], want[..., :Hq * D]), (kp, kw), (vp, vw)):
+        assert bool(((a.float().cpu() - b).abs() <= 2.0 ** -8 * b.abs() + 1e-4).all())
+
+
 @pytest.mark.parametrize("K", [256, 320, 448, 512, 576, 4096])
 @pytest.mark.parametrize("M", [40, 64])
 def test_one_row_tile(M, K):
