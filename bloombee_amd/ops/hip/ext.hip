@@ -1142,6 +1142,23 @@ static void few_tile(int width, F f) {
   }
 }
 
+// A sum's width and splits of K: what a CU reads at 45 B a ns, memory at 6.6 TB/s, 2 us of a
+// launch, 4 of the fold. 32 rows, us for 32 columns unsplit and 64 in few_splits: 6144 x 4096
+// 13.3, 15.5; 8192 x 8192 23.0, 30.8; 8192 x 1024 5.9, 7.0; 4096 x 14336 36, 23.9.
+static RowsPlan few_plan(long M, long N, long K) {
+  RowsPlan best;
+  auto look = [&](int width, int splits) {
+    const float cu = ldiv_up(ldiv_up(N, width) * splits, 256) * (width + 32.f) * 2.f *
+                     ldiv_up(K / 128, splits) * 128 / 45000.f;
+    const float us = std::max(cu, N * K * 2 / 6.6e6f) +
+                     (splits > 1 ? 6.f + splits * M * N * 1.6e-6f : 2.f);
+    if (us < best.us) best = {width, splits, us};
+  };
+  look(few_width(N), 1);
+  look(64, few_splits(N, K));
+  return best;
+}
+
 // Whether it beats the gated products of gemm_stream.hip and gemm_skinny.hip, which the
 // smallest are left to and those whose W does not begin at 16 bytes. us in a graph, W from
 // memory, the faster of those and this: 28672 x 4096: 1 row 45.9, 36.8; 32 rows 46.9, 36.8.
@@ -1181,6 +1198,22 @@ static bool few_sums(long M, long N, long K) {
   const long wgs = ldiv_up(N, 64) * few_splits(N, K);
   return M > 8 && (M > 12 || (N > 4096 && K <= 8192)) && N * K >= 24L << 20 && K >= 3072 &&
          wgs * 10 >= ldiv_up(wgs, 256) * 256 * 6;
+}
+
+// Whether a sum goes to few_plan's tiles. Beside few_sums, where 64 columns did with W kept
+// in the caches: more than one round of 16-row workgroups, and long K, the earlier the more
+// rows. us in a graph, W from memory, the faster of gemm_stream.hip and gemm_skinny.hip, and
+// this: 8192 x 8192: 1 row 31.1, 25.1; 8 rows 34.1, 25.0. 6144 x 4096 14.6, 13.2; 15.7, 13.2.
+// 8192 x 2048 10.4, 8.5; 32 rows 13.2, 9.0. 8192 x 28672 86.8, 78.3; 12 rows 101, 79. 4352 x
+// 1024 6.2, 5.3. 4160 x 512 4.2, 4.1; 16384 x 512 5.7, 6.0. One round: 4096 x 11008, 8 rows
+// 23.7, 21.0; 3584 x 18944, 1 row 28.2, 29.3, 8 rows 32.4, 30.0; 4096 x 5120, 13 rows 13.2,
+// 12.3; 4096 x 4096, 16 rows 10.3, 10.9, 32 rows 12.6, 11.4; 4096 x 3072, 32 rows 9.5, 9.9.
+static bool few_wins(long M, long N, long K) {
+  if (few_sums(M, N, K)) return true;
+  if (M <= 0 || M > 32 || K % 128 || K < 512 || N <= 0 || N % 8) return false;
+  if (K >= 1 << 20 || N >= 1 << 24) return false;   // rows_args
+  return (N > 4096 && (K >= 1024 || N <= 8192)) || (M >= 8 && K > 8192) ||
+         (M >= 13 && K >= 4864) || (M > 16 && K >= 4096);
 }
 
 // silu(gate) * up of [gate | up] = rms(A) @ W^T, norm weight folded into W.
@@ -1633,9 +1666,9 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
   a.R = operand(residual, (long)a.M * a.N);
   a.bias = operand(bias, a.N);
   if (a.M == 0) return C;
-  const bool few = few_sums(a.M, a.N, a.K);
+  const bool few = a.M <= 32 && a.K % 128 == 0;
   const RowsPlan plan =
-      few ? RowsPlan{-1, few_splits(a.N, a.K)} : rows_plan(a.M, a.N, a.K, false);
+      few ? few_plan(a.M, a.N, a.K) : rows_plan(a.M, a.N, a.K, false);
   a.splits = plan.splits;
   a.C = plan.splits > 1 ? nullptr : bf_ptr_mut(C);
   torch::Tensor part;
@@ -1644,8 +1677,11 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
     a.part = part.data_ptr<float>();
   }
   if (few)
-    rows_launch(gemm_rows_kernel<FewRows, true>, ldiv_up(a.N, FewRows::BN) * a.splits,
-                FewRows::THREADS, FewRows::LDS, cur_stream(), a);
+    few_tile(plan.tile, [&](auto tile) {
+      typedef decltype(tile) T;
+      rows_launch(gemm_rows_kernel<T, true>, ldiv_up(a.N, T::BN) * a.splits, T::THREADS,
+                  T::LDS, cur_stream(), a);
+    });
   else
     rows_product(a, plan);
   if (plan.splits > 1) {
@@ -1730,10 +1766,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("add_experts", &add_experts);
   m.def("gemm_stream", &gemm_stream);
   m.def("few_sums", &few_sums);
+  m.def("few_wins", &few_wins);
   m.def("few_splits", &few_splits);
   m.def("few_swiglu", &few_swiglu);
   m.def("few_width", &few_width);
   m.def("few_rope", &few_rope);
+  m.def("few_plan", [](long M, long N, long K) {
+    const RowsPlan p = few_plan(M, N, K);
+    return std::make_pair(p.tile, p.splits);
+  });
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {

@@ -371,7 +371,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
             and K % 256 == 0 and N % 64 == 0 and N > 0):
         _require_ext()
         if (norm is None and ss_in is None and ss_out is None
-                and w.data_ptr() % 16 == 0 and hip_ops.few_sums(M, N, K)):
+                and w.data_ptr() % 16 == 0 and hip_ops.few_wins(M, N, K)):
             return hip_ops.gemm_rows(x.contiguous(), w, residual, bias)
         if (ss_in is None and ss_out is None
                 and (hip_ops.stream_sums(M, N, K) if norm is None else

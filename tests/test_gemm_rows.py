@@ -166,6 +166,23 @@ def test_one_row_tile(M, K):
                  + 2.0 ** -19 * (tol[0] * u.abs() + tol[1] * g.abs()) + 1e-30).all())
 
 
+@pytest.mark.parametrize("M,N,K,plan", [
+    (1, 4160, 512, (32, 1)), (3, 8192, 512, (32, 1)), (7, 16320, 1024, (64, 1)),
+    (1, 20480, 1024, (96, 1)), (5, 28672, 1024, (128, 1)), (9, 36864, 1024, (160, 1)),
+    (8, 2560, 8448, (64, 6)), (13, 1024, 4864, (64, 9)), (17, 2048, 4096, (64, 8)),
+    (32, 6144, 4096, (32, 1))])
+def test_few_rows_by_their_plan(M, N, K, plan):
+    """Every width unsplit, and the splits of few columns."""
+    assert ops.hip_ops.few_wins(M, N, K) and ops.hip_ops.few_plan(M, N, K) == plan
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    r, b = draw(M, N, seed=3), draw(N, seed=4)
+    want = x.double() @ w.double().T
+    terms = x.double().abs() @ w.double().abs().T
+    assert close(ops.linear(x, w), want, terms)
+    assert close(ops.linear(x, w, residual=r, bias=b), want + r.double() + b.double(),
+                 terms + r.double().abs() + b.double().abs())
+
+
 @pytest.mark.parametrize("M,F,up,cols,K", [
     (33, 8, 8, 64, 256), (65, 1000, 1024, 1088, 320), (200, 4096, 4100, 4096, 256),
     (333, 712, 715, 768, 576), (617, 1400, 1400, 1408, 384), (194, 21360, 21376, 21504, 256)])
