@@ -843,6 +843,20 @@ static int moe_height(float a) {
   return 256;
 }
 
+// f(tile) for the products of 1 to 32 rows of up to `experts` experts: the width of W that
+// leaves a CU the fewest columns if as many are chosen, of those the widest.
+template <int UP, typename F>
+static void few_experts(int N, int experts, F f) {
+  auto columns = [&](int bn) {
+    return ((long)moe_columns<UP>(N, bn) * experts + 255) / 256 * bn;
+  };
+  typedef RowsTile<32, 64, 2, 2, 1, 4, 2> Half;
+  if (columns(128) <= columns(64)) f(RowsTile<32, 128, 2, 2, 1, 3, 2>{});
+  else if constexpr (UP == 2) f(Half{});
+  else if (columns(64) <= columns(32)) f(Half{});
+  else f(RowsTile<32, 32, 2, 2, 1, 6, 2>{});
+}
+
 // h (N, K), up (E, planes, F, K), down (E, Wp, F), ids/wts (N, top)
 // -> y (N, top, Wp); rows of skipped choices are not written. Two planes:
 // gated activation (limit, slope, shift), one: relu(up)^2. win: the weight
@@ -878,6 +892,11 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
          moe_experts(h.slice(0, n), up, down, ids.slice(0, n), wt.slice(0, n), win,
                      limit, slope, shift, stepwise)});
   }
+  if (ta == at::kBFloat16) {
+    // rows come by 16-byte copies: a view that does not begin at 16 bytes is copied first
+    for (Tensor* t : {&h, &up, &down})
+      if ((size_t)t->data_ptr() % 16) *t = t->clone();
+  }
   auto y = torch::empty({N, top, Wp}, h.options());
   if (N == 0) return y;
   auto act = torch::empty({S, F}, h.options());
@@ -891,25 +910,23 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     else f(std::integral_constant<int, 1>{});
   };
 
-  if (ta == at::kBFloat16 && N <= 32) {
-    const bf16_bits* hp = (const bf16_bits*)h.data_ptr();
-    bf16_bits* actp = (bf16_bits*)act.data_ptr();
-    by_bool(K % 256 == 0, [&](auto full) {
-      by_planes([&](auto np) {
-        moe_skinny_kernel<decltype(np)::value, decltype(full)::value>
-            <<<dim3(F / 64, E), 256, 0, st>>>(
-                hp, (const bf16_bits*)up.data_ptr(), idp, w1, actp, S, top, F,
-                K, K, F, glu);
+  // a row's place in bytes has 32 bits
+  if (ta == at::kBFloat16 && N <= 32 && (long)S * std::max(K, F) < 1L << 31) {
+    auto product = [&](auto up_planes, const Tensor& a, const Tensor& w, const float* wt,
+                       Tensor& c, int n, int k) {
+      constexpr int UP = decltype(up_planes)::value;
+      few_experts<UP>(n, std::min(S, E), [&](auto tile) {
+        typedef decltype(tile) T;
+        auto kernel = moe_few_kernel<T, UP>;
+        allow_lds(kernel, T::LDS);
+        kernel<<<dim3(moe_columns<UP>(n, T::BN), E), T::THREADS, T::LDS, st>>>(
+            (const bf16_bits*)a.data_ptr(), (const bf16_bits*)w.data_ptr(), idp, wt,
+            (bf16_bits*)c.data_ptr(), S, top, n, k, k, n, glu);
       });
-    });
-    check_launch();
-    by_bool(F % 256 == 0, [&](auto full) {
-      moe_skinny_kernel<0, decltype(full)::value>
-          <<<dim3(Wp / 64, E), 256, 0, st>>>(
-              actp, (const bf16_bits*)down.data_ptr(), idp, w2,
-              (bf16_bits*)y.data_ptr(), S, top, Wp, F, F, Wp, glu);
-    });
-    check_launch();
+      check_launch();
+    };
+    by_planes([&](auto np) { product(np, h, up, w1, act, F, K); });
+    product(std::integral_constant<int, 0>{}, act, down, w2, y, Wp, F);
     return y;
   }
 

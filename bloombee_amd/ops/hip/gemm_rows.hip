@@ -225,8 +225,10 @@ struct RowsTile {
     };
     // until all but n stages have landed
     auto wait = [&](int n) {
-      static_assert(ST <= 4, "stages");
-      if (n >= 3) wait_loads<3 * LPW>();
+      static_assert(ST <= 6 && (ST - 1) * LPW < 64, "stages");
+      if (ST > 5 && n >= 5) wait_loads<(ST > 5 ? 5 : 0) * LPW>();
+      else if (ST > 4 && n >= 4) wait_loads<(ST > 4 ? 4 : 0) * LPW>();
+      else if (n >= 3) wait_loads<3 * LPW>();
       else if (n == 2) wait_loads<2 * LPW>();
       else if (n == 1) wait_loads<LPW>();
       else wait_loads<0>();

@@ -19,7 +19,7 @@
 // Kernels take UP, the planes of the first product, 0 for the second, and wts,
 // the weights to apply or null.
 //
-//  * moe_skinny_kernel — up to 32 tokens: streams each chosen expert's weights
+//  * moe_few_kernel — up to 32 tokens: streams each chosen expert's weights
 //    once; a workgroup finds its expert's slots by scanning the ids itself, so
 //    a decode step needs no sort.
 //  * moe_sort_kernel + moe_rows_kernel — longer batches: expert-sorted slots,
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// skinny: grid (N / 64, E), at most 32 tokens
+// few rows: grid (column tiles, E), at most 32 tokens
 // ---------------------------------------------------------------------------
 
 DEVINL float relu_sq(float z) {
@@ -126,28 +126,35 @@ DEVINL float relu_sq(float z) {
   return r * r;
 }
 
-// UP: A row = slot / top (the token), out row = slot, activation.
+// UP: A row = slot / top (the token), out row = slot, activation (of two planes half of a
+// tile's rows of W are gates, half ups).
 // else: A row = slot, out row = slot.
-template <int UP, bool FULL>  // FULL: K % 256 == 0
-__global__ __launch_bounds__(256) void moe_skinny_kernel(
+//
+// A tile of gemm_rows.hip with an expert's 1 to 32 rows. Its weights are read once, by whole
+// lines past the caches, and bound it. us for both products by half lines of 16 rows a wave
+// and here: eight experts, 4096 x 14336, two a token: 1 token 220, 126; 16 tokens 490, 381
+// (6.6 TB/s); 64 experts, 2048 x 1024, eight a token: 55, 34; 141, 116. K % 64 == 0
+template <typename T, int UP>
+__global__ __launch_bounds__(T::THREADS, T::MINW) void moe_few_kernel(
     const unsigned short* __restrict__ A, const unsigned short* __restrict__ W,
     const int* __restrict__ ids, const float* __restrict__ wts,
     unsigned short* __restrict__ C, int S, int top, int N, int K, int lda,
     int ldc, GluConst glu) {
-  constexpr int NW = UP ? UP : 1, U = 4, KSTEP = 256, RS = KSTEP + 8;
-  __shared__ __attribute__((aligned(16))) unsigned short at[32 * RS];
+  static_assert(T::WK == 1 && (UP < 2 || T::NI % 2 == 0), "pairs");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   __shared__ int slots[32];
   __shared__ int n_slots;
+  constexpr int HALF = T::NI * 8;                    // a wave's gates, then its ups
   const int e = blockIdx.y;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
-  const int li = lane & 15, hi = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x & (WAVE - 1), li = lane & 15;
   if (wave == 0) {
     int n = 0;
     for (int b = 0; b < S; b += WAVE) {
       const bool mine = b + lane < S && ids[b + lane] == e;
       const unsigned long long m = __builtin_amdgcn_ballot_w64(mine);
-      const int at_ = n + __popcll(m & ((1ull << lane) - 1));
-      if (mine && at_ < 32) slots[at_] = b + lane;
+      const int at = n + __popcll(m & ((1ull << lane) - 1));
+      if (mine && at < 32) slots[at] = b + lane;
       n += __popcll(m);
     }
     if (lane == 0) n_slots = min(n, 32);  // choices of a token are distinct
@@ -155,112 +162,51 @@ __global__ __launch_bounds__(256) void moe_skinny_kernel(
   __syncthreads();
   const int cnt = n_slots;
   if (cnt == 0) return;
-  const int mt = cnt > 16 ? 2 : 1;
-  const int n0 = xcd_order(blockIdx.x, gridDim.x) * 64 + wave * 16;
-  const unsigned short* wr[NW];
-#pragma unroll
-  for (int w = 0; w < NW; ++w)
-    wr[w] = W + (((long)e * NW + w) * N + n0 + li) * K + hi * 8;
+  const int n0 = xcd_order(blockIdx.x, gridDim.x) * (UP == 2 ? T::BN / 2 : T::BN);
 
-  f32x4 acc[NW][2];
+  unsigned ofs[T::LPW];
 #pragma unroll
-  for (int w = 0; w < NW; ++w)
-#pragma unroll
-    for (int t = 0; t < 2; ++t) acc[w][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  const unsigned short* arow[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int flat = threadIdx.x + j * 256;
-    const int sl = slots[min(flat / 32, cnt - 1)];
-    arow[j] = A + (long)(UP ? sl / top : sl) * lda + (flat % 32) * 8;
+  for (int j = 0; j < T::LPW; ++j) {
+    const int r = T::load_row(j, wave, lane);
+    unsigned row;
+    if (j < T::AJ) {
+      const int sl = slots[min(r, cnt - 1)];
+      row = (unsigned)(UP ? sl / top : sl) * (unsigned)lda;
+    } else {
+      row = (unsigned)min(UP == 2 ? r / (2 * HALF) * HALF + r % HALF : r, N - 1 - n0) *
+            (unsigned)K;
+    }
+    ofs[j] = row * 2 + T::load_byte(j, wave, lane);
   }
-  short8 areg[4];
-  auto load_a = [&](int k) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j >= 2 * mt) break;
-      areg[j] = short8{};
-      if (FULL || k + (int)(threadIdx.x % 32) * 8 < K)
-        areg[j] = *reinterpret_cast<const short8*>(arow[j] + k);
-    }
-  };
-  auto store_a = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (j >= 2 * mt) break;
-      const int flat = threadIdx.x + j * 256;
-      *reinterpret_cast<short8*>(at + (flat / 32) * RS + (flat % 32) * 8) = areg[j];
-    }
-  };
-  bf16x8 b0[NW][U], b1[NW][U];
-  auto load_w = [&](bf16x8 (&b)[NW][U], int k) {
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if constexpr (FULL) {
-          b[w][u] = as_bf16x8(
-              *reinterpret_cast<const short8*>(wr[w] + k + u * 32));
-        } else {
-          b[w][u] = as_bf16x8(short8{});
-          if (k + u * 32 < K)
-            b[w][u] = as_bf16x8(
-                *reinterpret_cast<const short8*>(wr[w] + k + u * 32));
-        }
-      }
-  };
-  auto mma = [&](const bf16x8 (&b)[NW][U], int half) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (t >= mt) break;
-        const bf16x8 af = as_bf16x8(*reinterpret_cast<const short8*>(
-            at + (t * 16 + li) * RS + half * 128 + u * 32 + hi * 8));
-#pragma unroll
-        for (int w = 0; w < NW; ++w)
-          acc[w][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, b[w][u],
-                                                              acc[w][t], 0, 0, 0);
-      }
-  };
+  typename T::Acc acc;
+  T::template run<false, true>(
+      ofs, A, W + ((long)e * (UP ? UP : 1) * N + n0) * K, K / T::BK, lds, acc,
+      [&](int j) {
+        // the eight rows of a load are of one plane
+        return UP == 2 ? (long)(T::load_row(j, wave, 0) / HALF % 2) * N * K : 0L;
+      }, T::BK, 0.f, rows_begin(K / T::BK));
 
-  load_a(0);
-  load_w(b0, 0);
-  store_a();
-  __syncthreads();
-  auto stage = [&](int k, auto more) {
-    if constexpr (decltype(more)::value) load_a(k + KSTEP);
-    load_w(b1, k + 128);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(b0, 0);
-    if constexpr (decltype(more)::value) load_w(b0, k + KSTEP);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(b1, 1);
-    if constexpr (decltype(more)::value) {
-      __syncthreads();
-      store_a();
-      __syncthreads();
-    }
-  };
-  // the last stage apart: a wait behind loads under a condition has to assume that
-  // they were not issued, and drains them
-  int k = 0;
-  for (; k + KSTEP < K; k += KSTEP) stage(k, std::true_type{});
-  stage(k, std::false_type{});
+  const int r0 = T::row0(), c0 = n0 + (UP == 2 ? T::col0() / 2 : T::col0());
+  constexpr int STRIPS = UP == 2 ? T::NI / 2 : T::NI;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int m = 0; m < T::MI; ++m) {
+    const int r = r0 + m * 16 + li;
+    const float w = wts && r < cnt ? wts[slots[r]] : 1.f;
+    T::template out16<STRIPS>(lds, [&](int n) {
+      f32x4 v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = t * 16 + hi * 4 + r;
-      if (m >= cnt) continue;
-      const int sl = slots[m];
-      const float w = wts ? wts[sl] : 1.f;
-      float v = acc[0][t][r] * w;
-      if constexpr (UP == 2) v = gated(glu, v, acc[NW - 1][t][r] * w);
-      if constexpr (UP == 1) v = relu_sq(v);
-      C[(long)sl * ldc + n0 + li] = f2bf(v);
-    }
+      for (int j = 0; j < 4; ++j) {
+        v[j] = acc[m][n][j] * w;
+        if constexpr (UP == 2) v[j] = gated(glu, v[j], acc[m][n + STRIPS][j] * w);
+        if constexpr (UP == 1) v[j] = relu_sq(v[j]);
+      }
+      return pack4(v);
+    }, [&](int i, int c, auto v) {
+      const int at = r0 + m * 16 + i;
+      if (at < cnt && c0 + c < N)
+        *reinterpret_cast<decltype(v)*>(C + (long)slots[at] * ldc + c0 + c) = v;
+    });
+  }
 }
 
 // ---------------------------------------------------------------------------

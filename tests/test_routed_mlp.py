@@ -203,3 +203,36 @@ def test_more_rows_than_32_bits_of_bytes_reach(flat):
     zero = torch.ones(N, dtype=torch.bool, device=DEV)
     zero[at] = False
     assert not got[zero].any()
+
+
+@pytest.mark.parametrize("N,E,top,planes,K,F,Wp", [
+    (1, 4, 2, 2, 64, 64, 64),                # one row, one stage of K
+    (32, 1, 1, 2, 192, 192, 320),            # all rows of one expert
+    (17, 2, 1, 1, 320, 192, 4160),           # a tile's last columns
+    (16, 8, 2, 2, 128, 4096, 8192),          # enough columns for wide tiles
+    (9, 64, 6, 1, 576, 1088, 64), (31, 300, 3, 2, 64, 128, 192)])
+@pytest.mark.parametrize("win", [False, True])
+def test_few_tokens(N, E, top, planes, K, F, Wp, win):
+    h = draw(N, K, seed=1)
+    up = draw(E, planes, F, K, seed=2, scale=K ** -0.5)
+    down = draw(E, Wp, F, seed=3, scale=F ** -0.5)
+    gen = torch.Generator().manual_seed(4)
+    ids = torch.rand(N, E, generator=gen).argsort(1)[:, :top].int()
+    wts = torch.rand(N, top, generator=gen) + 0.5
+    skipped = torch.rand(N, top, generator=gen) < 0.2
+    got = ragged._ext().moe_experts(h, up, down, ids.masked_fill(skipped, -1).to(DEV),
+                                    wts.to(DEV), win, float("inf"), 1.0, 0.0, False)
+    x, up, down = (t.double().cpu() for t in (h, up, down))
+    for n in range(N):
+        for c in range(top):
+            if skipped[n, c]:
+                continue
+            e, w = int(ids[n, c]), float(wts[n, c])
+            z = up[e] @ x[n] * (w if win else 1.0)
+            act = (torch.nn.functional.silu(z[0]) * z[1] if planes == 2 else
+                   torch.relu(z[0]).square())
+            want = down[e] @ act * (1.0 if win else w)
+            # an activation and its row are rounded to 16 bits, 2^-9 of each
+            tol = 2.0 ** -8 * (want.abs() + (1.0 if win else w)
+                               * (down[e].abs() @ act.abs()))
+            assert bool(((got[n, c].double().cpu() - want).abs() <= tol + 1e-6).all())
