@@ -967,6 +967,7 @@ Tensor moe_experts(Tensor h, Tensor up, Tensor down, Tensor ids, Tensor wts,
     a.N = a.ldc = UP ? F : Wp;
     a.K = a.lda = UP ? K : F;
     a.glu = glu;
+    a.large = (up.numel() + down.numel()) * 2 > 32L << 20;
     allow_lds(kernel, lds);
     kernel<<<moe_columns<UP>(a.N, bn) * max_tiles, threads, lds, st>>>(a);
     check_launch();
