@@ -1569,6 +1569,24 @@ static RowsPlan rows_plan(long M, long N, long K, bool swiglu) {
   return rows_best(tiles, 10, M, N, K, swiglu);
 }
 
+// The gated product on a tile of its own, unsplit, with what it takes: one wave a SIMD with
+// 280 sums a lane reads the least of L2 and of LDS a product, and its height is between
+// those whose workgroups leave a round half empty. us, the tile of rows_plan and this: 28672 x
+// 4096: 560 rows 135.5, 113.8; 617 134, 112; 640 139, 116; 1200 264, 212; 1900 352, 333. 36864
+// x 3072: 300 rows 108, 84. 57344 x 4096: 617 269, 230; 900 365, 333. 14336 x 4096: 1200 135,
+// 112. Full rounds of 256 x 256 are faster: 4096 rows of 28672 x 4096 665, 725. Of 224 sizes
+// the rule takes 37, all of them faster, by 2 to 25%.
+typedef RowsTile<320, 224, 2, 2, 1, 2, 1> TallRows;
+
+static float tall_us(long M, long N, long K) {
+  return ldiv_up(ldiv_up(M, TallRows::BM) * ldiv_up(N, TallRows::BN), 256) *
+             (6.f + K / 64 * 1.28f) + (N + M) * K / 9.8e6f;
+}
+
+static bool rows_tall(long M, long N, long K) {
+  return tall_us(M, N, K) < .97f * rows_plan(M, N, K, true).us;
+}
+
 // Whether these are the faster form. The library's kernels are at 1.1 to 1.6 PF where
 // their tiles fill the chip, which takes many rows or columns; below, and where K is
 // long, they leave CUs idle. us in a graph, W from memory, library and these, N x K:
@@ -1600,7 +1618,8 @@ static bool rows_swiglu_wins(long M, long N, long K) {
     return false;
   if (K >= 1 << 20 || M >= 1 << 24 || N >= 1 << 24) return false;   // rows_args
   const double library = std::max(2e-6 * M * N * K / 1.2e3, (N + M) * K * 2 / 4.7e6);
-  return rows_plan(M, N, K, true).us * 1.04 < library + M * N * 3 / 5e6 + 3;
+  return std::min(rows_plan(M, N, K, true).us, tall_us(M, N, K)) * 1.04 <
+         library + M * N * 3 / 5e6 + 3;
 }
 
 template <typename F>
@@ -1694,14 +1713,16 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
 
 template <bool CLAMPED>
 static void rows_glu(RowsArgs& a, const RowsGlu& glu) {
-  rows_tile(rows_plan(a.M, 2L * glu.F, a.K, true).tile, [&](auto tile) {
+  auto launch = [&](auto tile) {
     typedef decltype(tile) T;
     if constexpr (T::WK == 1)
       rows_launch(a.M <= T::BM ? gemm_rows_glu_kernel<T, CLAMPED, false, true>
                                : gemm_rows_glu_kernel<T, CLAMPED>,
                   ldiv_up(a.M, T::BM) * ldiv_up(glu.ldc, T::BN / 2), T::THREADS, T::LDS,
                   cur_stream(), a, glu);
-  });
+  };
+  if (rows_tall(a.M, 2L * glu.F, a.K)) launch(TallRows{});
+  else rows_tile(rows_plan(a.M, 2L * glu.F, a.K, true).tile, launch);
 }
 
 // swiglu(A @ W^T) of a fused [gate | up] W: (..., N / 2).
@@ -1777,6 +1798,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
+  m.def("rows_tall", &rows_tall);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {
     const RowsPlan p = rows_plan(M, N, K, swiglu);
     return py::make_tuple(p.tile, p.splits);

@@ -31,8 +31,13 @@
 // than 256 registers a wave the compiler moves them around between products (four
 // moves each). It knows nothing of the product's latency: settle() goes ahead of what
 // reads the sums.
+// Accumulation registers hold 64 such sums a lane; IN_VECTOR: one beyond them.
+template <bool IN_VECTOR = false>
 DEVINL void mfma_acc(f32x4& c, bf16x8 x, bf16x8 y) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
+  if constexpr (IN_VECTOR)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(x), "v"(y));
+  else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(x), "v"(y));
 }
 
 DEVINL void settle() { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
@@ -205,8 +210,12 @@ struct RowsTile {
         }
 #pragma unroll
         for (; p < (i + 1) * P / FR; ++p) {
-          if constexpr (MINW == 1)
-            mfma_acc(acc[p % MI][p / MI], wf[s][p / MI], af[s][p % MI]);
+          if constexpr (MINW == 1) {
+            if (P > 64 && p >= 58)
+              mfma_acc<true>(acc[p % MI][p / MI], wf[s][p / MI], af[s][p % MI]);
+            else
+              mfma_acc(acc[p % MI][p / MI], wf[s][p / MI], af[s][p % MI]);
+          }
           else
             acc[p % MI][p / MI] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 wf[s][p / MI], af[s][p % MI], acc[p % MI][p / MI], 0, 0, 0);

@@ -73,6 +73,14 @@ def test_gated(M, F, K):
                  + 2.0 ** -8 * (g.abs() + 1) * u.abs() + 1e-6).all())
 
 
+@pytest.mark.parametrize("M,F,K", [(257, 20480, 256), (300, 28672, 320), (320, 18432, 448),
+                                   (617, 11088, 1024), (640, 14336, 256), (601, 28000, 576)])
+def test_gated_on_the_tall_tile(M, F, K):
+    """One row tile, whose W passes the caches, and two."""
+    assert ops.hip_ops.rows_tall(M, 2 * F, K)
+    test_gated(M, F, K)
+
+
 FEW = [(1, 28672, 1024), (9, 5120, 13824), (16, 4096, 14336), (17, 28672, 1280),
        (31, 576, 9216), (32, 8192, 8192), (32, 6144, 4096), (5, 192, 14336)]
 
