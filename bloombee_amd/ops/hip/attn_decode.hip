@@ -35,11 +35,12 @@ DEVINL void load_bf16_e(const unsigned short* p, float* out) {
 // ceil(units * maxg / 4). Lanes read the splits' maxima and sums at once and share
 // out the weights, so that the loads of the values do not wait for one another
 // (32 splits: 15 us in a decode step when they did, about 5 now, which is a launch).
+// cuts: of equal shares (attn_decode_even_kernel), a context's first one and how many.
 template <int D>
 __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
     const float* __restrict__ part_ml, const float* __restrict__ part_acc,
     unsigned short* __restrict__ out, int units, int Hkv, int G, int nch, int maxg,
-    int n_split, long out_sb, long out_sh) {
+    int n_split, const int2* __restrict__ cuts, long out_sb, long out_sh) {
   constexpr int E = D >= 128 ? D / 64 : 1;   // columns of a lane
   const int row = blockIdx.x * 4 + threadIdx.x / WAVE;
   const int lane = threadIdx.x & (WAVE - 1);
@@ -50,22 +51,30 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
   const int kvh = rem / nch;
   const int g0 = (rem % nch) * maxg;
   if (g0 + g >= G) return;
-  const float* ml = part_ml + ((long)bh * n_split * maxg + g) * 2;
+  long first = (long)bh * n_split;   // the unit's rows, `step` apart
+  int step = maxg;
+  if (cuts) {
+    first = (long)(cuts[b].x + b) * (Hkv * nch) + rem;
+    n_split = cuts[b].y;
+    step = Hkv * nch * maxg;
+    if (n_split == 1) return;        // is in `out`
+  }
+  const float* ml = part_ml + (first * maxg + g) * 2;
   float m = NEG_BIG;
   for (int s = lane; s < n_split; s += WAVE)
-    if (ml[(long)s * maxg * 2 + 1] != 0.f) m = fmaxf(m, ml[(long)s * maxg * 2]);
+    if (ml[(long)s * step * 2 + 1] != 0.f) m = fmaxf(m, ml[(long)s * step * 2]);
   m = wave_reduce_max(m);
   float l = 0.f, acc[E];
 #pragma unroll
   for (int j = 0; j < E; ++j) acc[j] = 0.f;
   const int col = min(lane * E, D - E);
-  const float* pa = part_acc + ((long)bh * n_split * maxg + g) * D + col;
+  const float* pa = part_acc + (first * maxg + g) * D + col;
   for (int s0 = 0; s0 < n_split; s0 += WAVE) {
     const int s = s0 + lane;
     float w = 0.f, ls = 0.f;
-    if (s < n_split) ls = ml[(long)s * maxg * 2 + 1];
+    if (s < n_split) ls = ml[(long)s * step * 2 + 1];
     if (ls != 0.f) {
-      w = fast_exp2(ml[(long)s * maxg * 2] - m);
+      w = fast_exp2(ml[(long)s * step * 2] - m);
       l += w * ls;
     }
     // splits beyond the context, or ahead of the window, have no sum: values are read
@@ -79,7 +88,7 @@ __global__ __launch_bounds__(256) void attn_decode_combine_kernel(
       const float wi = __shfl(w, i);
 #pragma unroll
       for (int j = 0; j < E; ++j)
-        acc[j] += wi * pa[(long)(s0 + i) * maxg * D + j];
+        acc[j] += wi * pa[(long)(s0 + i) * step * D + j];
     }
   }
   l = wave_reduce_sum(l);

@@ -502,6 +502,329 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_decode_mfma_kernel(
   }
 }
 
+// Tiles of 32 positions that a step reads of a context, at least one.
+DEVINL int decode_tiles(int ctx, int window) {
+  return max(1, (ctx + DKVBLK - 1) / DKVBLK - (window > 0 ? max(0, ctx - window) : 0) / DKVBLK);
+}
+
+// A batch of contexts of any lengths in equal shares: their tiles in a row, `shares` times
+// as many workgroups as heads, each of which has as many tiles of its head as any other, to
+// one. A share goes on from context to context, a wave with every NW-th of its tiles, the
+// next one's loads on their way (as under PIPE) also where the context ends: there the waves
+// put together what they have of it, `out` where that is all of it, else row (share +
+// context) * heads + head of the partial results; cuts (B, 2): a context's first share and
+// how many have a part. Bound by memory; a workgroup to a piece of one context left CUs
+// idle behind the longest ones and drained its loads at every end. 97 contexts of 64 to 4000
+// tokens, 8 heads of 128 (850 MB): 159 us (5.4 TB/s), 143 (6.0) with the fold; draining at a
+// context's end 166, shares of single waves 152 (more parts to fold), loads again of whole
+// tiles behind the last one 147.
+// grid: shares * heads; B * tiles of a context < 2^31
+template <int D, int MAXG, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void attn_decode_even_kernel(
+    const unsigned short* __restrict__ q, const unsigned short* __restrict__ k_pages,
+    const unsigned short* __restrict__ v_pages, const int* __restrict__ page_table,
+    const int* __restrict__ ctx_lens, const float* __restrict__ alibi,
+    unsigned short* __restrict__ out, float* __restrict__ part_ml,
+    float* __restrict__ part_acc, int2* __restrict__ cuts, int B, int Hkv, int G, int nch,
+    int P, int maxp, int window, float scale, long q_sb, long q_sh, long out_sb, long out_sh,
+    int ctx_add, int shares) {
+  constexpr int NKK = D / 32;   // QK^T k-slices
+  constexpr int NDT = D / 16;   // PV d-tiles
+  constexpr int NPT = DKVBLK / 16;  // position tiles per KV tile
+  constexpr int PROW_B = DKVBLK * 2 + 16;  // P^T LDS row pitch
+  __shared__ __attribute__((aligned(16))) unsigned char lds[
+      NW * 16 * PROW_B + NW * MAXG * (D + 2) * 4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int heads = Hkv * nch, share = blockIdx.x / heads, head = blockIdx.x % heads;
+  const int kvh = head / nch, g0 = head % nch * MAXG;
+  const int lane = threadIdx.x & (WAVE - 1), li = lane & 15, hi = lane >> 4;
+  const float sc2 = scale * LOG2E;
+  unsigned char* p_lds = lds + wave * 16 * PROW_B;
+  float* merge_lds = reinterpret_cast<float*>(lds + NW * 16 * PROW_B);
+
+  auto tiles = [&](int b) {
+    return b < B ? decode_tiles(ctx_lens[b] + ctx_add, window) : 0;
+  };
+  int all = 0;
+  for (int b = lane; b < B; b += WAVE) all += tiles(b);
+#pragma unroll
+  for (int o = 32; o; o >>= 1) all += __shfl_xor(all, o);
+  all = __builtin_amdgcn_readfirstlane(all);
+  const int per = max(NW, (all + shares - 1) / shares);
+  const int at = share * per;
+  const int n_tiles = min(all, at + per) - at;
+  if (n_tiles <= 0) return;
+  // the context of the first tile, tiles ahead of it
+  int b0 = 0, before = 0;
+  for (int base = 0; base < B; base += WAVE) {
+    const int n = tiles(base + lane);
+    int upto = n;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const int x = __shfl_up(upto, o);
+      if (lane >= o) upto += x;
+    }
+    const unsigned long long hit = __builtin_amdgcn_ballot_w64(before + upto > at);
+    if (hit) {
+      const int l = __builtin_ctzll(hit);
+      b0 = base + l;
+      before += __builtin_amdgcn_readlane(upto - n, l);
+      break;
+    }
+    before += __builtin_amdgcn_readlane(upto, WAVE - 1);
+  }
+
+  // a tile: its context, the context's length, the first position
+  struct Place { int b, ctx, tb; };
+  auto enter = [&](Place& p, int b) {
+    p.b = b;
+    p.ctx = max(0, __builtin_amdgcn_readfirstlane(ctx_lens[b]) + ctx_add);
+    p.tb = (window > 0 ? max(0, p.ctx - window) : 0) / DKVBLK * DKVBLK;
+  };
+  auto advance = [&](Place& p, int by) {
+    p.tb += by * DKVBLK;
+    while (true) {
+      const int over = p.tb - max(DKVBLK, (p.ctx + DKVBLK - 1) / DKVBLK * DKVBLK);
+      if (over < 0) break;
+      enter(p, p.b + 1);
+      p.tb += over;
+    }
+  };
+  // what the share has of a context: `got` of its `own` tiles, behind `skipped`
+  Place piece;
+  enter(piece, b0);
+  int skipped = at - before, left = n_tiles, own = decode_tiles(piece.ctx, window);
+  int got = min(own - skipped, left);
+  Place now = piece, ahead;
+  int now_i = wave, ahead_i = wave;     // tiles of the share, the wave's: every NW-th
+  if (wave < n_tiles) advance(now, skipped + wave);
+  else now.b = -1;
+  ahead = now;
+  if (wave >= n_tiles) {
+    ahead = piece;
+    ahead.tb = ahead.ctx;
+  }
+
+  const bool pow2 = (P & (P - 1)) == 0;
+  const int plog = 31 - __builtin_clz(P);
+  auto page_of = [&](int pos) { return pow2 ? pos >> plog : pos / P; };
+  // a tile on its way: of which the last position is, the first one, pages
+  struct Tile { int last, tb, v, k[NPT]; };
+  // the next tile; behind the last one its context's last position again
+  auto look_up = [&](Tile& t) {
+    const bool some = ahead.ctx > 0;
+    t.last = max(0, ahead.ctx - 1);
+    t.tb = ahead.tb;
+    const int* table = page_table + (long)ahead.b * maxp;
+    t.v = table[page_of(min(t.tb + hi * 8, t.last & ~7))];
+#pragma unroll
+    for (int n = 0; n < NPT; ++n)
+      t.k[n] = table[page_of(min(t.tb + li + 16 * n, t.last))];
+    if (!some) {
+      t.v = 0;
+#pragma unroll
+      for (int n = 0; n < NPT; ++n) t.k[n] = 0;
+    }
+    if (ahead_i + NW < n_tiles) {
+      ahead_i += NW;
+      advance(ahead, NW);
+    } else {
+      ahead.tb = ahead.ctx;
+    }
+  };
+  auto load_tile = [&](bf16x8 (&vb)[NDT], bf16x8 (&kb)[NPT][NKK], const Tile& t) {
+    const int vpos = min(t.tb + hi * 8, t.last & ~7);
+    const unsigned short* vrow = v_pages + ((long)t.v * Hkv + kvh) * D * P +
+                                 (long)li * P + (vpos - page_of(vpos) * P);
+#pragma unroll
+    for (int n = 0; n < NDT; ++n)
+      vb[n] = as_bf16x8(__builtin_nontemporal_load(
+          reinterpret_cast<const short8*>(vrow + 16 * n * P)));
+#pragma unroll
+    for (int n = 0; n < NPT; ++n) {
+      const int pos = min(t.tb + li + 16 * n, t.last);
+      const unsigned short* krow = k_pages + ((long)t.k[n] * Hkv + kvh) * P * D +
+                                   (long)(pos - page_of(pos) * P) * D;
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk)
+        kb[n][kk] = as_bf16x8(__builtin_nontemporal_load(
+            reinterpret_cast<const short8*>(krow + hi * 8 + 32 * kk)));
+    }
+  };
+
+  const int qh = kvh * G + min(g0 + li, min(G, g0 + MAXG) - 1);
+  const float aslope = alibi != nullptr ? alibi[qh] * LOG2E : 0.f;
+  bf16x8 qfrag[NKK];
+  auto load_q = [&]() {
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk)
+      qfrag[kk] = as_bf16x8(*reinterpret_cast<const short8*>(
+          q + (long)piece.b * q_sb + (long)qh * q_sh + hi * 8 + 32 * kk));
+  };
+  float m2 = NEG_BIG, l = 0.f;
+  f32x4 acc_o[NDT];  // O^T: rows = d (hi*4+reg + 16n), cols = head (li)
+  auto clear = [&]() {
+    m2 = NEG_BIG;
+    l = 0.f;
+#pragma unroll
+    for (int n = 0; n < NDT; ++n) acc_o[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  };
+  auto compute_tile = [&](bf16x8 (&vb)[NDT], const bf16x8 (&kb)[NPT][NKK], int tb) {
+    const int c1 = piece.ctx, lo = window > 0 ? max(0, c1 - window) : 0;
+    f32x4 st[NPT];
+#pragma unroll
+    for (int n = 0; n < NPT; ++n) {
+      st[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < NKK; ++kk)
+        st[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[n][kk], qfrag[kk], st[n], 0, 0, 0);
+    }
+    float p[NPT][4];
+    float rm = NEG_BIG;
+#pragma unroll
+    for (int n = 0; n < NPT; ++n)
+#pragma unroll
+      for (int reg = 0; reg < 4; ++reg) {
+        const int kpos = tb + 16 * n + hi * 4 + reg;
+        float sv = st[n][reg] * sc2 + aslope * (float)kpos;
+        const bool dead = (kpos >= c1) | (kpos < lo);
+        sv = dead ? NEG_BIG : sv;
+        p[n][reg] = sv;
+        rm = fmaxf(rm, sv);
+      }
+    rm = quad16_reduce_max(rm);
+    const float mn = fmaxf(m2, rm);
+    const float corr = fast_exp2(m2 - mn);
+    float psum = 0.f;
+#pragma unroll
+    for (int n = 0; n < NPT; ++n)
+#pragma unroll
+      for (int reg = 0; reg < 4; ++reg) {
+        p[n][reg] = fast_exp2(p[n][reg] - mn);
+        psum += p[n][reg];
+      }
+    psum = quad16_reduce_sum(psum);
+    l = l * corr + psum;
+    m2 = mn;
+    if (__builtin_amdgcn_ballot_w64(corr < 0.9999f)) {
+#pragma unroll
+      for (int n = 0; n < NDT; ++n)
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg) acc_o[n][reg] *= corr;
+    }
+#pragma unroll
+    for (int n = 0; n < NPT; ++n)
+#pragma unroll
+      for (int reg = 0; reg < 4; ++reg)
+        *(unsigned short*)(p_lds + li * PROW_B + (16 * n + hi * 4 + reg) * 2) =
+            f2bf(p[n][reg]);
+    bf16x8 pfrag = as_bf16x8(*reinterpret_cast<const short8*>(p_lds + li * PROW_B + hi * 16));
+    if (tb + DKVBLK > c1) {
+#pragma unroll
+      for (int n = 0; n < NDT; ++n)
+        if (tb + hi * 8 >= c1) vb[n] = as_bf16x8(short8{});
+    }
+#pragma unroll
+    for (int n = 0; n < NDT; ++n)
+      acc_o[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vb[n], pfrag, acc_o[n], 0, 0, 0);
+  };
+  // LDS only: loads from memory stay on their way
+  auto barrier = [&]() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // the waves' results of a piece together
+  auto merge = [&]() {
+    const int Gl = min(G - g0, MAXG);
+    barrier();
+    float* dst = merge_lds + (wave * MAXG + li) * (D + 2);
+    if (li < Gl) {
+#pragma unroll
+      for (int n = 0; n < NDT; ++n)
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg) dst[16 * n + hi * 4 + reg] = acc_o[n][reg];
+      if (hi == 0) {
+        dst[D] = m2;
+        dst[D + 1] = l;
+      }
+    }
+    barrier();
+    if (skipped == 0 && head == 0 && threadIdx.x == 0)
+      cuts[piece.b] = make_int2(share, 1 + (own - got + per - 1) / per);
+    for (int i = threadIdx.x; i < Gl * D; i += NW * 64) {
+      const int g = i / D, d = i % D;
+      const float* src = merge_lds + g * (D + 2);
+      float mw[NW], mx = NEG_BIG, lt = 0.f, v = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        mw[w] = src[w * MAXG * (D + 2) + D];
+        mx = fmaxf(mx, mw[w]);
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float c = fast_exp2(mw[w] - mx);
+        lt += src[w * MAXG * (D + 2) + D + 1] * c;
+        v += src[w * MAXG * (D + 2) + d] * c;
+      }
+      if (got == own) {
+        out[(long)piece.b * out_sb + (long)(kvh * G + g0 + g) * out_sh + d] =
+            f2bf(lt > 0.f ? v * (1.f / lt) : 0.f);
+      } else {
+        const long row = ((long)(share + piece.b) * heads + head) * MAXG + g;
+        part_acc[row * D + d] = v;
+        if (d == 0) {
+          part_ml[row * 2] = mx;
+          part_ml[row * 2 + 1] = lt;
+        }
+      }
+    }
+  };
+
+  bf16x8 vb0[NDT], vb1[NDT];
+  bf16x8 kb0[NPT][NKK], kb1[NPT][NKK];
+  Tile ta, tb;
+  look_up(ta);
+  look_up(tb);
+  load_tile(vb0, kb0, ta);
+  load_q();
+  clear();
+  // to the wave's next tile; false: there is none
+  auto meet = [&]() {
+    while (now.b != piece.b) {
+      merge();
+      left -= got;
+      if (left == 0) return false;
+      enter(piece, piece.b + 1);
+      skipped = 0;
+      own = decode_tiles(piece.ctx, window);
+      got = min(own, left);
+      load_q();
+      clear();
+    }
+    return true;
+  };
+  auto next = [&]() {
+    now_i += NW;
+    if (now_i < n_tiles) advance(now, NW);
+    else now.b = -1;
+    return meet();
+  };
+  if (!meet()) return;
+  while (true) {
+    look_up(ta);
+    load_tile(vb1, kb1, tb);
+    __builtin_amdgcn_sched_barrier(0);
+    compute_tile(vb0, kb0, now.tb);
+    if (!next()) break;
+    look_up(tb);
+    load_tile(vb0, kb0, ta);
+    __builtin_amdgcn_sched_barrier(0);
+    compute_tile(vb1, kb1, now.tb);
+    if (!next()) break;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Wide-head decode attention (D = 512: gemma-4 global layers).
 //

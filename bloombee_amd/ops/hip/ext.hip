@@ -278,8 +278,47 @@ static void attn_decode_launch(const torch::Tensor& q, const torch::Tensor& kp,
     attn_decode_combine_kernel<D>
         <<<(units * maxg + 3) / 4, 256, 0, cur_stream()>>>(
             pml.data_ptr<float>(), pacc.data_ptr<float>(), bf_ptr_mut(out),
-            units, Hkv, G, nch, maxg, n_split, out_sb, out_sh);
+            units, Hkv, G, nch, maxg, n_split, nullptr, out_sb, out_sh);
   }
+}
+
+// The same in equal shares of the batch's tiles, then the parts of the cut contexts.
+template <int D, int MAXG>
+static void attn_decode_even_launch(
+    const torch::Tensor& q, const torch::Tensor& kp, const torch::Tensor& vp,
+    const torch::Tensor& pt, const torch::Tensor& ctx, const float* alibi_ptr,
+    torch::Tensor& out, int B, int Hkv, int G, int nch, int P, int maxp, int window,
+    float scale, long q_off, long q_sb, long q_sh, long out_sb, long out_sh, int ctx_add) {
+  // two workgroups a CU: 222 registers
+  const int heads = Hkv * nch, shares = std::max(1, 512 / heads);
+  const long rows = (long)(B + shares) * heads;
+  auto fopt = torch::TensorOptions().device(q.device()).dtype(at::kFloat);
+  auto cuts = torch::empty({B, 2}, fopt.dtype(at::kInt));
+  auto pml = torch::empty({rows, MAXG, 2}, fopt);
+  auto pacc = torch::empty({rows, MAXG, D}, fopt);
+  int2* cp = reinterpret_cast<int2*>(cuts.data_ptr<int>());
+  attn_decode_even_kernel<D, MAXG, 4><<<shares * heads, 256, 0, cur_stream()>>>(
+      bf_ptr(q) + q_off, bf_ptr(kp), bf_ptr(vp), pt.data_ptr<int>(), ctx.data_ptr<int>(),
+      alibi_ptr, bf_ptr_mut(out), pml.data_ptr<float>(), pacc.data_ptr<float>(), cp, B, Hkv, G,
+      nch, P, maxp, window, scale, q_sb, q_sh, out_sb, out_sh, ctx_add, shares);
+  attn_decode_combine_kernel<D><<<(B * heads * MAXG + 3) / 4, 256, 0, cur_stream()>>>(
+      pml.data_ptr<float>(), pacc.data_ptr<float>(), bf_ptr_mut(out), B * heads, Hkv, G, nch,
+      MAXG, 0, cp, out_sb, out_sh);
+}
+
+// Whether a batch goes in equal shares, by the room of its contexts; their lengths are on
+// the device. From more than one context a CU on, one workgroup has all of one or pieces
+// of 1024 and the longest outlast the rest; what the shares cost is their folds, a launch.
+// us in a graph, pieces and shares, 8 heads of keys, tokens: 33 contexts of 64 to 4000 63.2,
+// 55.6; 40 115, 62; 64 127, 93; 64 of 64 to 8000 245, 172; 70 223, 190; 97 of 64 to 4000 159,
+// 143; 200 of 64 to 2000 178, 158; 36 of 64 to 1000 33.9, 26.4; 256 119, 108; of one length:
+// 40 of 1000 39.8, 37.5; 97 of 2000 142, 131; 300 of 2048 428, 395; 56 of 2000 81.0, 81.6; 64
+// of 2000 86.0, 89.2. Shorter ones lose: 64 of 1000 34.8, 37.0, 100 of 150 18.5, 23.6; and
+// those that leave CUs idle are split evenly as it is (32 of 2048 45.3, 50.9).
+static bool decode_even(long B, long heads, long room) {
+  const long units = B * heads;
+  return units > 256 && room >= (units > 512 ? 1024 : 1536) && heads <= 64 && B <= 1024 &&
+         B * room < 1L << 34;
 }
 
 static torch::Tensor attn_decode_core(
@@ -330,6 +369,22 @@ static torch::Tensor attn_decode_core(
     // 2000 28.8, 28.3; 32 of 300 14.1, 10.5; 2000 48.2, 45.1. Heads of 32, 64 and 128, 1 to 32
     // of keys, 1 to 64 sequences of 100 to 8000 tokens, 4572 steps: none is slower by more than
     // 5% (0.5 us) than with one wave's fold and four waves throughout.
+    if (pf_env0 && D <= 128 && decode_even(B, Hkv * nch, room)) {
+      auto even = [&](auto d, auto g) {
+        attn_decode_even_launch<decltype(d)::value, decltype(g)::value>(
+            q, k_pages, v_pages, page_table, ctx_lens, alibi_ptr, out, B, Hkv, G, nch, P, maxp,
+            (int)window, (float)scale, q_off, q_sb, q_sh, out_sb, out_sh, ctx_add);
+      };
+      auto of = [&](auto d) {
+        if (G <= 4 && nch == 1) even(d, std::integral_constant<int, 4>{});
+        else even(d, std::integral_constant<int, 16>{});
+      };
+      if (D == 128) of(std::integral_constant<int, 128>{});
+      else if (D == 64) of(std::integral_constant<int, 64>{});
+      else if (D == 32) of(std::integral_constant<int, 32>{});
+      else TORCH_CHECK(false, "unsupported head_dim ", D);
+      return out;
+    }
     wide = pf_env0 && D <= 128 && G <= 4 && units <= 256 &&
            ((room >= 256 && room <= 352) ||
             (units * room >= 60000 && 256 / units * 2 >= target / units));
@@ -338,9 +393,8 @@ static torch::Tensor attn_decode_core(
       n_split = (int)std::max(1L, std::min({32L, 256 / units, room / share}));
     } else if (units > target) {
       // More units than fit at once: contexts of a large batch differ, and a
-      // workgroup with a long one outlasts the rest. Shares of 1024 tokens even it
-      // out (97 sequences of 64 to 4000 tokens, 8 heads of 128: 168 us unsplit,
-      // 157 us so).
+      // workgroup with a long one outlasts the rest. Pieces of 1024 tokens even it
+      // out, where equal shares don't (heads wider than 128, or more than 64).
       share = 1024;
       n_split = (int)std::min(32L, (room + share - 1) / share);
     } else {
@@ -1799,6 +1853,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rows_wins", &rows_wins);
   m.def("rows_swiglu_wins", &rows_swiglu_wins);
   m.def("rows_tall", &rows_tall);
+  m.def("decode_even", &decode_even);
   m.def("rows_plan", [](long M, long N, long K, bool swiglu) {
     const RowsPlan p = rows_plan(M, N, K, swiglu);
     return py::make_tuple(p.tile, p.splits);
