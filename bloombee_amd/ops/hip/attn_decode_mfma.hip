@@ -502,6 +502,17 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_decode_mfma_kernel(
   }
 }
 
+// Sums over the lanes up to each.
+DEVINL int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31
+  return x;
+}
+
 // Tiles of 32 positions that a step reads of a context, at least one.
 DEVINL int decode_tiles(int ctx, int window) {
   return max(1, (ctx + DKVBLK - 1) / DKVBLK - (window > 0 ? max(0, ctx - window) : 0) / DKVBLK);
@@ -515,7 +526,7 @@ DEVINL int decode_tiles(int ctx, int window) {
 // context) * heads + head of the partial results; cuts (B, 2): a context's first share and
 // how many have a part. Bound by memory; a workgroup to a piece of one context left CUs
 // idle behind the longest ones and drained its loads at every end. 97 contexts of 64 to 4000
-// tokens, 8 heads of 128 (850 MB): 159 us (5.4 TB/s), 143 (6.0) with the fold; draining at a
+// tokens, 8 heads of 128 (850 MB): 159 us (5.4 TB/s), 142 (6.0) with the fold; draining at a
 // context's end 166, shares of single waves 152 (more parts to fold), loads again of whole
 // tiles behind the last one 147.
 // grid: shares * heads; B * tiles of a context < 2^31
@@ -542,44 +553,38 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_decode_even_kernel(
   unsigned char* p_lds = lds + wave * 16 * PROW_B;
   float* merge_lds = reinterpret_cast<float*>(lds + NW * 16 * PROW_B);
 
-  auto tiles = [&](int b) {
-    return b < B ? decode_tiles(ctx_lens[b] + ctx_add, window) : 0;
-  };
-  int all = 0;
-  for (int b = lane; b < B; b += WAVE) all += tiles(b);
-#pragma unroll
-  for (int o = 32; o; o >>= 1) all += __shfl_xor(all, o);
-  all = __builtin_amdgcn_readfirstlane(all);
+  auto length = [&](int b) { return b < B ? max(0, ctx_lens[b] + ctx_add) : -1; };
+  auto tiles = [&](int ctx) { return ctx < 0 ? 0 : decode_tiles(ctx, window); };
+  // 64 contexts at a time: most batches are read once
+  const int len0 = length(lane), upto0 = wave_scan(tiles(len0));
+  int all = __builtin_amdgcn_readlane(upto0, WAVE - 1);
+  for (int base = WAVE; base < B; base += WAVE)
+    all += __builtin_amdgcn_readlane(wave_scan(tiles(length(base + lane))), WAVE - 1);
   const int per = max(NW, (all + shares - 1) / shares);
   const int at = share * per;
   const int n_tiles = min(all, at + per) - at;
   if (n_tiles <= 0) return;
   // the context of the first tile, tiles ahead of it
-  int b0 = 0, before = 0;
-  for (int base = 0; base < B; base += WAVE) {
-    const int n = tiles(base + lane);
-    int upto = n;
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-      const int x = __shfl_up(upto, o);
-      if (lane >= o) upto += x;
-    }
-    const unsigned long long hit = __builtin_amdgcn_ballot_w64(before + upto > at);
-    if (hit) {
-      const int l = __builtin_ctzll(hit);
-      b0 = base + l;
-      before += __builtin_amdgcn_readlane(upto - n, l);
-      break;
-    }
+  int len = len0, upto = upto0, base = 0, before = 0;
+  unsigned long long hit;
+  while (!(hit = __builtin_amdgcn_ballot_w64(before + upto > at))) {
     before += __builtin_amdgcn_readlane(upto, WAVE - 1);
+    base += WAVE;
+    len = length(base + lane);
+    upto = wave_scan(tiles(len));
   }
+  const int l0 = __builtin_ctzll(hit);
+  before += __builtin_amdgcn_readlane(upto - tiles(len), l0);
 
   // a tile: its context, the context's length, the first position
   struct Place { int b, ctx, tb; };
-  auto enter = [&](Place& p, int b) {
+  auto put = [&](Place& p, int b, int ctx) {
     p.b = b;
-    p.ctx = max(0, __builtin_amdgcn_readfirstlane(ctx_lens[b]) + ctx_add);
-    p.tb = (window > 0 ? max(0, p.ctx - window) : 0) / DKVBLK * DKVBLK;
+    p.ctx = ctx;
+    p.tb = (window > 0 ? max(0, ctx - window) : 0) / DKVBLK * DKVBLK;
+  };
+  auto enter = [&](Place& p, int b) {
+    put(p, b, max(0, __builtin_amdgcn_readfirstlane(ctx_lens[b]) + ctx_add));
   };
   auto advance = [&](Place& p, int by) {
     p.tb += by * DKVBLK;
@@ -592,7 +597,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_decode_even_kernel(
   };
   // what the share has of a context: `got` of its `own` tiles, behind `skipped`
   Place piece;
-  enter(piece, b0);
+  put(piece, base + l0, __builtin_amdgcn_readlane(len, l0));
   int skipped = at - before, left = n_tiles, own = decode_tiles(piece.ctx, window);
   int got = min(own - skipped, left);
   Place now = piece, ahead;

@@ -307,18 +307,21 @@ static void attn_decode_even_launch(
 }
 
 // Whether a batch goes in equal shares, by the room of its contexts; their lengths are on
-// the device. From more than one context a CU on, one workgroup has all of one or pieces
-// of 1024 and the longest outlast the rest; what the shares cost is their folds, a launch.
-// us in a graph, pieces and shares, 8 heads of keys, tokens: 33 contexts of 64 to 4000 63.2,
-// 55.6; 40 115, 62; 64 127, 93; 64 of 64 to 8000 245, 172; 70 223, 190; 97 of 64 to 4000 159,
-// 143; 200 of 64 to 2000 178, 158; 36 of 64 to 1000 33.9, 26.4; 256 119, 108; of one length:
-// 40 of 1000 39.8, 37.5; 97 of 2000 142, 131; 300 of 2048 428, 395; 56 of 2000 81.0, 81.6; 64
-// of 2000 86.0, 89.2. Shorter ones lose: 64 of 1000 34.8, 37.0, 100 of 150 18.5, 23.6; and
-// those that leave CUs idle are split evenly as it is (32 of 2048 45.3, 50.9).
+// the device. Where contexts and heads don't split evenly over the chip, a workgroup has all
+// of one or an equal part of each, and the longest outlast the rest; what the shares cost is
+// their folds, a launch, and finding them. us in a graph, without and with, 8 heads of keys,
+// tokens of a context: 16 of 500 to 4000 42.6, 36.0; 24 of 100 to 2000 35.7, 26.8; 33 of 64
+// to 4000 63.2, 55; 40 115, 61; 64 127, 92; 64 of 64 to 8000 245, 171; 70 223, 189; 97 of 64
+// to 4000 159, 142; 200 of 64 to 2000 178, 157; 256 of 100 to 1000 119, 108; all of one
+// length: 16 of 2000 29.1, 30.3; 24 41.2, 40.1; 28 43.0, 44.9; 40 of 1000 39.8, 37; 97 of
+// 2000 142, 130; 300 of 2048 428, 394; 64 of 2000 87.4, 89.0. Shorter ones lose (16 of 1000
+// 18.3, 19.1; 64 of 100 to 1000 34.8, 36; 100 of 150 18.3, 22.8), as do fewer (8 of 2000
+// 19.1, 20.6) and those of which each CU has one (32 of 2048 46.7, 50.7; of 100 to 2000
+// 37.7, 33.8).
 static bool decode_even(long B, long heads, long room) {
   const long units = B * heads;
-  return units > 256 && room >= (units > 512 ? 1024 : 1536) && heads <= 64 && B <= 1024 &&
-         B * room < 1L << 34;
+  return units >= 128 && (units <= 240 || units > 256) && room >= (units > 512 ? 1024 : 1536) &&
+         heads <= 64 && B <= 1024 && B * room < 1L << 34;
 }
 
 static torch::Tensor attn_decode_core(

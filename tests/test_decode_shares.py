@@ -54,6 +54,8 @@ def _lens(kind, B, room, seed):
     (33, 8, 4, 64, 8, 1600, "same", 0),
     (70, 8, 3, 32, 32, 1100, "mixed", 100),
     (33, 8, 8, 128, 32, 1600, "mixed", 0),
+    (16, 8, 4, 128, 32, 6000, "empty", 0),
+    (130, 1, 4, 128, 32, 1600, "mixed", 0),
     (52, 5, 4, 128, 32, 1600, "mixed", 777),
     (60, 1, 71, 64, 32, 1600, "mixed", 0),
     (9, 32, 1, 128, 32, 1600, "mixed", 0),
@@ -107,10 +109,11 @@ def test_shares(B, Hkv, G, D, P, room, kind, window):
 
 
 def test_which_batches():
-    """More than a context a CU, with room for long ones."""
+    """Contexts with room for long ones that the chip has no even split of."""
     from bloombee_amd.ops import hip_ops
     even = hip_ops.decode_even
     assert not even(32, 8, 8192) and even(33, 8, 1536) and not even(33, 8, 1535)
+    assert even(16, 8, 1536) and even(30, 8, 8192) and not even(15, 8, 8192)
     assert even(65, 8, 1024) and not even(65, 8, 1023)
     assert not even(65, 65, 4096) and not even(1025, 8, 4096)
     assert not even(1024, 8, 1 << 24)
