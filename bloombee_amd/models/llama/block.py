@@ -205,10 +205,22 @@ class LlamaBlock(torch.nn.Module):
                 y = y + d
         return y
 
+    def _plain_weights(self) -> bool:
+        """Projections are products with the weights as they are, nothing else."""
+        return (getattr(self, "_w4", None) is None
+                and getattr(self, "lora_delta", None) is None)
+
+    def _attended(self, attn, hidden):
+        """h2 = hidden + o(attn) and its post-attention norm."""
+        eps = self.config.rms_norm_eps
+        if self._plain_weights():
+            return ops.linear_norm(attn, self.o_w, hidden, self.post_norm_w, eps)
+        return ops.rms_norm_residual(self._lin(attn, self.o_w, "o_w"), hidden,
+                                     self.post_norm_w, eps)
+
     def _gated(self, y):
         """The gated product of gate_up's result."""
-        if (getattr(self, "_w4", None) is None
-                and getattr(self, "lora_delta", None) is None):
+        if self._plain_weights():
             return ops.linear_gated(y, self.gate_up_w)
         return ops.swiglu(self._lin(y, self.gate_up_w, "gate_up_w"))
 
@@ -256,9 +268,13 @@ class LlamaBlock(torch.nn.Module):
                                      start_pos)
         else:
             x = ops.rms_norm(hidden, self.input_norm_w, cfg.rms_norm_eps)
-            qkv = self._lin(x, self.qkv_w, "qkv_w")    # (B, T, (Hq+2Hkv)D)
-            ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp,
-                               pt, start_pos)
+            if self._plain_weights():
+                qkv = ops.linear_rope_kv_rows(x, self.qkv_w, Hq, Hkv, cos, sin,
+                                              position_ids, kp, vp, pt, start_pos)
+            else:
+                qkv = self._lin(x, self.qkv_w, "qkv_w")    # (B, T, (Hq+2Hkv)D)
+                ops.rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, kp, vp,
+                                   pt, start_pos)
         hp = (kv.host_prefix(self.layer_index)
               if hasattr(kv, "host_prefix") else None)
         if hp is not None:
@@ -278,10 +294,7 @@ class LlamaBlock(torch.nn.Module):
                                       longest=context_bound(kv, T))
         if fuse_norm:
             return self._fused_tail(hidden, attn)
-        a = self._lin(attn, self.o_w, "o_w")
-
-        # h2 = hidden + a fused into the post-attention norm
-        h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
+        h2, y = self._attended(attn, hidden)
         # residual add fused into the down-projection epilogue
         return self._lin(self._gated(y), self.down_w, "down_w", residual=h2)
 

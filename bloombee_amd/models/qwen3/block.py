@@ -78,8 +78,7 @@ class Qwen3Block(LlamaBlock):
                                       self.scale, longest=context_bound(kv, T))
         if fuse_norm:
             return self._fused_tail(hidden, attn)
-        a = self._lin(attn, self.o_w, "o_w")
-        h2, y = ops.rms_norm_residual(a, hidden, self.post_norm_w, cfg.rms_norm_eps)
+        h2, y = self._attended(attn, hidden)
         return self._lin(self._gated(y), self.down_w, "down_w", residual=h2)
 
     def forward_train(self, hidden: torch.Tensor, start_pos: int = 0) -> torch.Tensor:

@@ -20,6 +20,8 @@ from bloombee_amd.ops.interface import (  # noqa: F401
     layer_norm,
     linear,
     linear_gated,
+    linear_norm,
+    linear_rope_kv_rows,
     linear_rope_kv,
     linear_swiglu,
     linear_w4,

@@ -1313,17 +1313,12 @@ torch::Tensor gemm_swiglu(torch::Tensor A, torch::Tensor W, double eps) {
   return C;
 }
 
-// [q | k | v] = rms(A) @ W^T with q turned in the result and k, v in their page slots
-// (their columns of the result stay unwritten). A (B, T, K), norm weight folded in.
-torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq,
-                           long Hkv,
-                           torch::Tensor cos_t, torch::Tensor sin_t,
-                           c10::optional<torch::Tensor> pos, torch::Tensor k_pages,
-                           torch::Tensor v_pages, torch::Tensor page_table,
-                           torch::Tensor start_pos) {
-  StreamArgs a = stream_args(A, W);
-  TORCH_CHECK(A.dim() == 3 && a.K % 256 == 0 && a.N % 64 == 0,
-              "(B, T, K) rows, K%256, N%64 required");
+// Where the rotated rows of a fused projection go.
+static void rope_args(StreamArgs& a, const torch::Tensor& A, long Hq, long Hkv,
+                      const torch::Tensor& cos_t, const torch::Tensor& sin_t,
+                      const c10::optional<torch::Tensor>& pos, torch::Tensor& k_pages,
+                      torch::Tensor& v_pages, const torch::Tensor& page_table,
+                      const torch::Tensor& start_pos) {
   CHECK_DEV_ALL3(k_pages, v_pages, page_table);
   CHECK_DEV_ALL3(cos_t, sin_t, start_pos);
   CHECK_BF16(k_pages); CHECK_BF16(v_pages);
@@ -1350,12 +1345,6 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq
                 pos->numel() == a.M, "bad position ids");
     a.pos = pos->data_ptr<int>();
   }
-  auto sizes = A.sizes().vec();
-  sizes.back() = a.N;
-  auto C = torch::empty(sizes, A.options());
-  a.C = bf_ptr_mut(C);
-  if (a.M == 0) return C;
-  a.eps = eps;
   a.cos_t = cos_t.data_ptr<float>();
   a.sin_t = sin_t.data_ptr<float>();
   a.max_pos = cos_t.size(0);
@@ -1363,6 +1352,26 @@ torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq
   a.start = start_pos.data_ptr<int>();
   a.k_pages = bf_ptr_mut(k_pages);
   a.v_pages = bf_ptr_mut(v_pages);
+}
+
+// [q | k | v] = rms(A) @ W^T with q turned in the result and k, v in their page slots
+// (their columns of the result stay unwritten). A (B, T, K), norm weight folded in.
+torch::Tensor gemm_rope_kv(torch::Tensor A, torch::Tensor W, double eps, long Hq,
+                           long Hkv,
+                           torch::Tensor cos_t, torch::Tensor sin_t,
+                           c10::optional<torch::Tensor> pos, torch::Tensor k_pages,
+                           torch::Tensor v_pages, torch::Tensor page_table,
+                           torch::Tensor start_pos) {
+  StreamArgs a = stream_args(A, W);
+  TORCH_CHECK(A.dim() == 3 && a.K % 256 == 0 && a.N % 64 == 0,
+              "(B, T, K) rows, K%256, N%64 required");
+  rope_args(a, A, Hq, Hkv, cos_t, sin_t, pos, k_pages, v_pages, page_table, start_pos);
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N;
+  auto C = torch::empty(sizes, A.options());
+  a.C = bf_ptr_mut(C);
+  if (a.M == 0) return C;
+  a.eps = eps;
   if ((size_t)W.data_ptr() % 16 == 0 && few_rope(a.M, a.N, a.K)) {
     few_tile(few_width(a.N), [&](auto tile) {
       typedef decltype(tile) T;
@@ -1768,6 +1777,91 @@ torch::Tensor gemm_rows(torch::Tensor A, torch::Tensor W,
   return C;
 }
 
+// h = A @ W^T + residual and its RMS norm, (h, y). Where the product is split, its fold makes
+// both.
+std::vector<torch::Tensor> gemm_rows_norm(torch::Tensor A, torch::Tensor W,
+                                          torch::Tensor residual, torch::Tensor weight,
+                                          double eps) {
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(a.N % 8 == 0, "N % 8 != 0");
+  auto operand = [&](torch::Tensor& t, long n) {
+    CHECK_DEV(t); CHECK_BF16(t); CHECK_CONTIG(t);
+    TORCH_CHECK(t.numel() == n, "size of residual or weight");
+    if ((size_t)t.data_ptr() % 16) t = t.clone();
+    return bf_ptr(t);
+  };
+  const unsigned short* w = operand(weight, a.N);
+  const unsigned short* r = operand(residual, (long)a.M * a.N);
+  TORCH_CHECK(a.N <= 16384, "columns");
+  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
+  if (a.M == 0 || plan.splits == 1)
+    return rms_norm_residual(gemm_rows(A, W, c10::nullopt, c10::nullopt), residual, weight, eps);
+  auto sizes = A.sizes().vec();
+  sizes.back() = a.N;
+  auto h = torch::empty(sizes, A.options()), y = torch::empty(sizes, A.options());
+  auto part = torch::empty({plan.splits, a.M, a.N}, A.options().dtype(at::kFloat));
+  a.splits = plan.splits;
+  a.part = part.data_ptr<float>();
+  rows_product(a, plan);
+  a.C = bf_ptr_mut(h);
+  a.R = r;
+  auto fold = [&](auto iters) {
+    gemm_rows_fold_norm_kernel<decltype(iters)::value>
+        <<<a.M, 512, 0, cur_stream()>>>(a, w, bf_ptr_mut(y), (float)eps);
+  };
+  if (a.N <= 4096) fold(std::integral_constant<int, 1>{});
+  else if (a.N <= 8192) fold(std::integral_constant<int, 2>{});
+  else fold(std::integral_constant<int, 4>{});
+  HIP_OK(hipGetLastError());
+  return {h, y};
+}
+
+// rope_kv_write_ of A @ W^T: (B, T, (Hq + 2 Hkv) * D) with the turned queries; keys and
+// values are in the pages. Where the product is split and a sequence has a few tokens (its
+// values go to their pages one by one), its fold does it.
+torch::Tensor gemm_rows_rope_kv(torch::Tensor A, torch::Tensor W, long Hq, long Hkv,
+                                torch::Tensor cos_t, torch::Tensor sin_t,
+                                c10::optional<torch::Tensor> pos, torch::Tensor k_pages,
+                                torch::Tensor v_pages, torch::Tensor page_table,
+                                torch::Tensor start_pos) {
+  TORCH_CHECK(A.dim() == 3, "(B, T, K) rows");
+  RowsArgs a = rows_args(A, W);
+  TORCH_CHECK(a.N % 8 == 0, "N % 8 != 0");
+  StreamArgs r{};
+  r.M = a.M;
+  r.N = a.N;
+  rope_args(r, A, Hq, Hkv, cos_t, sin_t, pos, k_pages, v_pages, page_table, start_pos);
+  auto C = torch::empty({A.size(0), A.size(1), a.N}, A.options());
+  if (a.M == 0) return C;
+  const RowsPlan plan = rows_plan(a.M, a.N, a.K, false);
+  a.splits = plan.splits;
+  const bool fold = plan.splits > 1 && r.T <= 4 && r.D <= 256 && (r.D & (r.D - 1)) == 0 &&
+                    (size_t)k_pages.data_ptr() % 16 == 0;
+  torch::Tensor part;
+  if (plan.splits > 1) {
+    part = torch::empty({plan.splits, a.M, a.N}, A.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+  } else {
+    a.C = bf_ptr_mut(C);
+  }
+  rows_product(a, plan);
+  if (fold) {
+    a.C = r.C = bf_ptr_mut(C);
+    const long items = (long)a.M * (a.N / 16);
+    gemm_rows_fold_rope_kernel<<<ldiv_up(items, 256), 256, 0, cur_stream()>>>(a, r);
+    HIP_OK(hipGetLastError());
+    return C;
+  }
+  if (plan.splits > 1) {
+    a.C = bf_ptr_mut(C);
+    gemm_rows_fold_kernel<<<ldiv_up((long)a.M * a.N, 2048), 256, 0, cur_stream()>>>(a);
+    HIP_OK(hipGetLastError());
+  }
+  rope_kv_write_(C, Hq, Hkv, cos_t, sin_t, pos, k_pages, v_pages, page_table, start_pos,
+                 c10::nullopt, c10::nullopt, 0.0);
+  return C;
+}
+
 template <bool CLAMPED>
 static void rows_glu(RowsArgs& a, const RowsGlu& glu) {
   auto launch = [&](auto tile) {
@@ -1862,6 +1956,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return py::make_tuple(p.tile, p.splits);
   });
   m.def("gemm_rows", &gemm_rows);
+  m.def("gemm_rows_norm", &gemm_rows_norm);
+  m.def("gemm_rows_rope_kv", &gemm_rows_rope_kv);
   m.def("gemm_rows_swiglu", &gemm_rows_swiglu);
   m.def("gemm_rows_glu", &gemm_rows_glu);
   m.def("gemm_swiglu", &gemm_swiglu);

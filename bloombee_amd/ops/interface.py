@@ -451,6 +451,38 @@ def linear_gated(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return swiglu(linear(x, w))
 
 
+def linear_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+                weight: torch.Tensor, eps: float) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(h, rmsnorm(h) * weight) of h = x @ w^T + residual. On the tiles of gemm_rows.hip the
+    sums are not rounded ahead of the residual, and the fold of a split product makes both."""
+    N = w.shape[0]
+    if (rows_ok(x, w) and N <= 16384 and _addend(weight.detach(), x, N)
+            and _addend(residual, x, x.numel() // x.shape[-1] * N)):
+        return tuple(hip_ops.gemm_rows_norm(
+            x.contiguous(), w, residual.contiguous(), weight.detach().contiguous(), eps))
+    return rms_norm_residual(linear(x, w), residual, weight, eps)
+
+
+def linear_rope_kv_rows(x: torch.Tensor, w: torch.Tensor, Hq: int, Hkv: int, cos, sin,
+                        position_ids, k_pages, v_pages, page_table,
+                        start_pos) -> torch.Tensor:
+    """rope_kv_write_ of x @ w^T: (B, T, (Hq+2Hkv)*D) with the turned queries; of keys and
+    values only the pages are sure to have them. The fold of a split product does it."""
+    if (x.dim() == 3 and rows_ok(x, w) and k_pages.is_contiguous()
+            and v_pages.is_contiguous() and page_table.is_contiguous()
+            and k_pages.shape[3] % 32 == 0
+            and (position_ids is None
+                 or position_ids.numel() == x.shape[0] * x.shape[1])):
+        return hip_ops.gemm_rows_rope_kv(
+            x.contiguous(), w, Hq, Hkv, cos, sin,
+            position_ids.int().contiguous() if position_ids is not None else None,
+            k_pages, v_pages, page_table, start_pos.int())
+    qkv = linear(x, w)
+    rope_kv_write_(qkv, Hq, Hkv, cos, sin, position_ids, k_pages, v_pages, page_table,
+                   start_pos)
+    return qkv
+
+
 _FUSE_NORM = os.environ.get("BBAMD_FUSE_NORM", "1") != "0"
 
 

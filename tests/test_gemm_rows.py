@@ -363,3 +363,64 @@ def test_recorded_and_replayed():
         at.copy_(draw(M, K, seed=seed))
         graph.replay()
         assert torch.equal(out, ops.linear(at, w))
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 4096, 4096), (64, 512, 1024), (97, 4096, 1536),
+                                   (250, 5120, 4096), (40, 8192, 8192), (33, 16384, 1024),
+                                   (512, 1024, 512), (33, 1032, 2048)])
+def test_fold_with_norm(M, N, K):
+    """The fold of a split product that makes a row's norm too, and products unsplit."""
+    x, w = draw(M, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    r, nw = draw(M, N, seed=3), draw(N, seed=4)
+    h, y = ops.hip_ops.gemm_rows_norm(x, w, r, nw, 1e-5)
+    xd, wd = x.double(), w.double()
+    want = xd @ wd.t() + r.double()
+    # unsplit, the product is rounded ahead of the residual
+    assert close(h, want, xd.abs() @ wd.abs().t()
+                 + 2.0 ** 12 * (want - r.double()).abs())
+    hd = h.double()
+    norm = hd * torch.rsqrt(hd.pow(2).mean(-1, keepdim=True) + 1e-5) * nw.double()
+    assert close(y, norm, norm.abs() * 2.0 ** 6)
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,D,P,K,pos", [
+    (33, 1, 16, 4, 128, 32, 2048, False), (97, 1, 32, 8, 128, 32, 4096, True),
+    (20, 4, 8, 8, 64, 16, 1024, False), (40, 1, 4, 1, 256, 8, 2048, True),
+    (35, 2, 6, 3, 32, 32, 4096, False), (12, 5, 16, 4, 128, 32, 2048, False),
+    (300, 1, 8, 2, 96, 16, 2048, False), (700, 1, 8, 2, 64, 32, 512, False)])
+def test_fold_with_rotation(B, T, Hq, Hkv, D, P, K, pos):
+    """The fold of a split product that turns queries and keys and fills the pages, and
+    the steps apart where it does not."""
+    M, N, half, maxp = B * T, (Hq + 2 * Hkv) * D, D // 2, 4
+    x, w = draw(B, T, K, seed=1), draw(N, K, seed=2, scale=K ** -0.5)
+    angle = torch.arange(200, device=DEV)[:, None] * torch.rand(half, device=DEV)
+    cos, sin = angle.cos(), angle.sin()
+    start = (torch.arange(B, device=DEV) * 7 % (P * maxp - T)).int()
+    table = torch.randperm(B * maxp, device=DEV).int().view(B, maxp)
+    at = start[:, None].long() + torch.arange(T, device=DEV)
+    ids = (at * 3 % 150).int() if pos else None
+    kp = draw(B * maxp, Hkv, P, D, seed=5)
+    vp = draw(B * maxp, Hkv, D, P, seed=6)
+    kept_k, kept_v = kp.clone(), vp.clone()
+    got = ops.linear_rope_kv_rows(x, w, Hq, Hkv, cos, sin, ids, kp, vp, table, start)
+    xd, wd = x.view(M, K).double(), w.double()
+    flat, terms = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    # apart, the product is rounded ahead of the rotation
+    terms = (terms + 2.0 ** 12 * flat.abs()).view(B, T, -1, D)
+    y = flat.view(B, T, -1, D)
+    where = (ids if pos else at).long()
+    c, s = cos.double()[where][:, :, None], sin.double()[where][:, :, None]
+    turned = torch.cat([y[..., :half] * c - y[..., half:] * s,
+                        y[..., half:] * c + y[..., :half] * s], -1)
+    both = terms[..., :half] + terms[..., half:]
+    both = torch.cat([both, both], -1)
+    q = got.view(B, T, -1, D)[:, :, :Hq]
+    assert close(q, turned[:, :, :Hq], both[:, :, :Hq])
+    page = table.long().gather(1, at // P)
+    k = kp[page, :, at % P]
+    assert close(k, turned[:, :, Hq:Hq + Hkv], both[:, :, Hq:Hq + Hkv])
+    v = vp[page, :, :, at % P]
+    assert close(v, y[:, :, Hq + Hkv:], terms[:, :, Hq + Hkv:])
+    kept_k[page, :, at % P] = k
+    kept_v[page, :, :, at % P] = v
+    assert torch.equal(kp, kept_k) and torch.equal(vp, kept_v)
