@@ -571,9 +571,13 @@ static void launch_attn_prefill(PrefillArgs a, int D, int P,
                                       lds) == hipSuccess,
                   "cannot reserve ", lds, " bytes of LDS");
     kernel<<<grid, 256 * KG, lds, cur_stream()>>>(a);
-    if (a.n_split > 1)
-      attn_prefill_fold_kernel<DD>
-          <<<(units * rows + 3) / 4, 256, 0, cur_stream()>>>(a);
+    auto fold = [&](auto c) {
+      attn_prefill_fold_kernel<DD, decltype(c)::value>
+          <<<ldiv_up((long)units * rows * (DD / 4), 256), 256, 0, cur_stream()>>>(a);
+    };
+    if (a.n_split > 4) fold(std::integral_constant<int, 8>{});
+    else if (a.n_split > 2) fold(std::integral_constant<int, 4>{});
+    else if (a.n_split > 1) fold(std::integral_constant<int, 2>{});
   };
   auto launch = [&](auto d, auto form, auto pages) {
     if constexpr (decltype(pages)::value == PREFILL_GROUPS && decltype(d)::value <= 128)

@@ -269,3 +269,21 @@ def test_two_groups_of_waves(case, form):
     assert torch.equal(got.isnan(), want.isnan())
     assert bool(want.isnan().any()) == (form == "nan")
     close(got.nan_to_num(0), want.nan_to_num(0))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("splits,starts", [(2, (254, 0)), (3, (382, 60)), (4, (510, 3)),
+                                           (5, (638, 300)), (8, (1022, 100)),
+                                           (9, (1150, 0)), (16, (2046, 700))])
+def test_folds_of_any_number_of_splits(D, splits, starts):
+    """One chunk of the fold, a chunk and a split, several; a context that leaves splits
+    without keys."""
+    B, Hq, Hkv, T, P, room = 2, 8, 2, 2, 16, starts[0] + 2
+    assert ops.hip_ops.prefill_plan(B, Hq, Hkv, T, D, P, room, False, 0)[0] == splits
+    kp, vp, table = paged(B, Hkv, D, P, [s + T for s in starts], room, seed=splits)
+    gen = torch.Generator().manual_seed(3)
+    q = torch.randn(B, Hq, T, D, generator=gen).bfloat16()
+    qs = torch.tensor(starts, dtype=torch.int32)
+    want = ref.attn_paged(q.float(), kp.float(), vp.float(), table, qs.long())
+    got = ops.attn_paged(*[t.to(DEV) for t in (q, kp, vp, table, qs)])
+    close(got, want)
