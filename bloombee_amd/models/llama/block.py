@@ -241,7 +241,7 @@ class LlamaBlock(torch.nn.Module):
         cfg = self.config
 
         # Decode-shaped GPU steps fold both per-layer rmsnorms into the
-        # skinny GEMMs, the rotation with the K/V write into the first one and
+        # decode GEMMs, the rotation with the K/V write into the first one and
         # the gated product into the third: a launch there costs more than
         # most of these steps do. W4/LoRA blocks and prefill keep the separate
         # steps.

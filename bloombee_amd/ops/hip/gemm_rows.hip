@@ -17,7 +17,9 @@
 // 1450 to 1510 from 4096 rows on (a third one for A: 1440; the library's 1525 to 1640).
 // Where one round of workgroups streams W, three stages of smaller tiles hide more of
 // memory: 333 rows 73 us with 192 x 224, 87 with 192 x 256 and two stages, 94 with
-// 192 x 128 and four (W alone, walked by 128 B a row, takes 50).
+// 192 x 128 and four (W alone takes 50 in step, 37 with its K begun apart, rows_begin: no
+// more than 1 us of it is left here, nor does K begun apart by column tile for the L2's
+// channels gain anything, 1 to 5 us slower).
 // What it writes goes through LDS by whole lines (8 B a lane straight from the sums: 78 us
 // for 73, 513 for 496).
 // Tried and left: 32 columns a stage with five stages, L2 touched a stage or two ahead,

@@ -16,7 +16,9 @@
 // many bytes as of W at 16 rows: it comes from L2 to a piece of LDS of the wave's own,
 // in whole lines and without registers on the way (fragments straight from L2 took
 // 51 us where this takes 35: 32 rows, 14336 x 4096).
-// Loads of W as nontemporal cost 15% (29.5 us for 25.6: one row, 14336 x 4096).
+// Loads of W as nontemporal cost 15% (29.5 us for 25.6: one row, 14336 x 4096): these are
+// half lines. By whole ones past the caches the tiles of gemm_rows.hip are faster, and take
+// what they are built for.
 //
 // A row's sum of squares for the norm is the diagonal of A A^T, made by the matrix
 // cores from the fragments at hand.

@@ -349,11 +349,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, residual: Optional[torch.Tensor] = 
            ss_in: Optional[torch.Tensor] = None,
            ss_out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = (rmsnorm(x) if norm else x) @ w^T (+bias) (+residual).
-    Decode-shaped GEMMs (<=32 rows) on GPU go through the weight-streaming MFMA
-    kernels (gemm_stream.hip, gemm_skinny.hip) — hipBLASLt leaves ~2x weight-stream
-    bandwidth on the table at M<=32; up to some hundred rows, or a thousand of few
-    columns, where it leaves CUs idle, through the tiles of gemm_rows.hip; everything
-    else uses hipBLASLt via F.linear.
+    Decode-shaped GEMMs (<=32 rows) on GPU go through the tiles of gemm_rows.hip where
+    few_wins says so and the weight-streaming MFMA kernels (gemm_stream.hip,
+    gemm_skinny.hip) elsewhere — hipBLASLt leaves ~2x weight-stream bandwidth on the
+    table at M<=32; up to some hundred rows, or a thousand of few columns, where it
+    leaves CUs idle, through the tiles as well; everything else uses hipBLASLt via
+    F.linear.
     norm=(weight, eps): the input's rmsnorm is taken along; weight None: it is folded
     into w. ss_in (f32, (stripes, 32)) are sums of squares of x's rows, the ss_out of
     the product that made x, and spare a pass over x; ss_out (f32, (N/64, 32)) takes
@@ -552,8 +553,8 @@ def routed_mlp(a: torch.Tensor, router_w: torch.Tensor, gate_up: torch.Tensor,
     """Sum of the chosen experts of the rows a: the top router logits choose, a
     softmax over them weighs. With a residual and norm=(weight, eps): h +
     experts(rmsnorm(h)), h = a + residual. Norm and routing are one launch, the
-    experts two weight streams up to 32 rows and a sort with two tiled GEMMs
-    beyond (moe_routed.hip); nothing waits for the host. Callers gate on
+    experts two launches that find their rows themselves up to 32 of them and a sort
+    with two tiled GEMMs beyond (moe_routed.hip); nothing waits for the host. Callers gate on
     routed_mlp_ok."""
     _require_ext()
     from bloombee_amd.ops import ragged
