@@ -11,6 +11,7 @@
 #include "attn_ragged.hip"
 #include "moe_routed.hip"
 #include "gemm_skinny.hip"
+#include "gemm_rows_host.h"
 
 // pair: [buckets, mul_prev, mul_cur] with prev and pair_table
 Tensor embed_rows(Tensor ids, Tensor pos, Tensor table, OptTensor pos_table,
@@ -630,6 +631,39 @@ Tensor router_gemm(Tensor A, Tensor W) {
   return C;
 }
 
+// f(tile) for up to 32 rows on tiles of `width` columns.
+template <typename F>
+static void parts_tile(int width, F f) {
+  switch (width) {
+    case 32: f(RowsTile<32, 32, 2, 1, 2, 4, 2>{}); break;
+    case 64: f(RowsTile<32, 64, 2, 1, 2, 3, 2>{}); break;
+    case 96: f(RowsTile<32, 96, 2, 2, 1, 4, 2>{}); break;
+    case 128: f(RowsTile<32, 128, 2, 2, 1, 4, 2>{}); break;
+    default: f(RowsTile<32, 160, 2, 2, 1, 4, 2>{}); break;
+  }
+}
+
+// Their width and splits of K, most of `most`: what a CU takes in at 45 B a ns, memory at
+// 6.6 TB/s, the sums' way out and in again.
+static std::pair<int, int> parts_plan(long M, long N, long K, int most) {
+  std::pair<int, int> best{0, 0};
+  float least = INFINITY;
+  for (int width : {160, 128, 96, 64, 32})
+    for (int splits = 1; splits <= most && K / 128 / splits >= (splits > 1 ? 3 : 1); ++splits) {
+      const long per = ldiv_up(K / 128, splits);
+      const float cu = ldiv_up(ldiv_up(N, width) * splits, 256) * (width + 32.f) * 2.f * per *
+                       128 / 45000.f;
+      float us = std::max(cu, N * K * 2 / 6.6e6f);
+      if (splits > 1 && same_channels(K, per * 128)) us *= 1.3f;
+      us += splits * M * N * 1.4e-6f;
+      if (us < least) {
+        least = us;
+        best = {width, (int)ldiv_up(K / 128, per)};
+      }
+    }
+  return best;
+}
+
 // (ksplit, M, N) f32 partials of A @ W^T, M <= 32.
 Tensor gemm_parts(Tensor A, Tensor W, long ksplit_req) {
   CHECK_T(A, at::kBFloat16);
@@ -639,6 +673,30 @@ Tensor gemm_parts(Tensor A, Tensor W, long ksplit_req) {
   TORCH_CHECK(M >= 1 && M <= 32 && K % 32 == 0 && N % 64 == 0 && N > 0,
               "need M <= 32, K % 32 == 0, N % 64 == 0, N > 0");
   int ks = (int)ksplit_req;
+  // On tiles, W by whole lines past the caches where the split form takes it by 64 B of a
+  // row. us in a graph, W from memory, that and this, 1 and 32 rows: 28672 x 4096 50.3, 41.2;
+  // 54.9, 43.0. 4096 x 14336 24.9, 22.1; 28.2, 22.7. 8256 x 4096 16.5, 14.0; 18.9, 15.2. 4096
+  // x 4096 8.6, 8.4; 10.3, 8.9. 12288 x 1536 11.0, 9.3; 13.1, 10.5. 128256 x 4096 192, 186;
+  // 213, 198. 576 x 4096 4.7, 3.9; 64 x 512 3.3, 3.1. Shorter K is left: 768 x 256 2.6, 3.1.
+  if (K % 128 == 0 && K >= 512 && K < 1 << 20 && (size_t)A.data_ptr() % 16 == 0 &&
+      (size_t)W.data_ptr() % 16 == 0) {
+    const auto [width, splits] = parts_plan(M, N, K, ks > 0 ? ks : 8);
+    auto part = torch::empty({splits, M, N}, A.options().dtype(at::kFloat));
+    RowsArgs r{};
+    r.A = (const unsigned short*)A.data_ptr();
+    r.W = (const unsigned short*)W.data_ptr();
+    r.part = part.data_ptr<float>();
+    r.M = M;
+    r.N = N;
+    r.K = K;
+    r.splits = splits;
+    parts_tile(width, [&](auto tile) {
+      typedef decltype(tile) T;
+      rows_launch(gemm_rows_kernel<T, true>, ldiv_up(N, T::BN) * r.splits, T::THREADS, T::LDS,
+                  cur_stream(), r);
+    });
+    return part;
+  }
   if (ks <= 0) {
     // as gemm_skinny: one split once N alone covers the chip, else up to
     // eight so that narrow outputs still fill it

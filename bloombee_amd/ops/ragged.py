@@ -300,8 +300,8 @@ def embed_rows(ids: torch.Tensor, positions: torch.Tensor,
 
 
 def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x (M, K) @ w (N, K)^T as (splits, M, N): f32 partials of the split-K
-    weight-stream kernel for up to 32 bf16 rows, else one part in x's type, from
+    """x (M, K) @ w (N, K)^T as (splits, M, N): f32 partials, of tiles of
+    gemm_rows.hip or the split-K weight-stream kernel, for up to 32 bf16 rows, else one part in x's type, from
     the tiles of gemm_rows.hip or the vendor GEMM."""
     if (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[0] <= SKINNY_ROWS):
         return _ext().gemm_parts(x, w, 0)

@@ -424,3 +424,24 @@ def test_fold_with_rotation(B, T, Hq, Hkv, D, P, K, pos):
     kept_k[page, :, at % P] = k
     kept_v[page, :, :, at % P] = v
     assert torch.equal(kp, kept_k) and torch.equal(vp, kept_v)
+
+
+@pytest.mark.parametrize("N,K", [(64, 512), (576, 4096), (8256, 2048), (4096, 4096),
+                                 (40960, 1024), (28672, 640), (192, 16384), (33024, 512)])
+def test_parts_of_few_rows(N, K):
+    """Partial sums in 32 bits of any width and number of splits; W that does not begin
+    at 16 bytes."""
+    from bloombee_amd.ops import ragged
+    w = draw(N, K, seed=2, scale=K ** -0.5)
+    off = torch.empty(N * K + 1, dtype=torch.bfloat16, device=DEV)[1:].view(N, K)
+    off.copy_(w)
+    for M in (1, 15, 17, 32):
+        x = draw(M, K, seed=M)
+        want, terms = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        for splits in (0, 1):
+            p = ragged._ext().gemm_parts(x, w, splits)
+            assert p.dtype == torch.float32 and (not splits or p.shape[0] == 1)
+            assert bool(((p.double().sum(0) - want).abs() <= 2.0 ** -20 * terms).all())
+    if K % 256 == 0:
+        p = ragged._ext().gemm_parts(x, off, 0)
+        assert bool(((p.double().sum(0) - want).abs() <= 2.0 ** -20 * terms).all())
